@@ -1137,8 +1137,12 @@ def knn_topk(x: Tensor, y: Tensor, K: int) -> Tuple[Tensor, Tensor]:
         raise RuntimeError(f'{what}: feature dimensions differ')
     dist2 = torch.empty((N, K), dtype=torch.float32, device=x.device)
     index = torch.empty((N, K), dtype=torch.int64, device=x.device)
+    lib = _lib()
+    nbytes = lib.fsgs_knn_topk_workspace_bytes(N, M, D, K)
+    ws = _workspace(nbytes, x.device) if nbytes else None
     with _timed('knn_topk'):
-        rc = _lib().fsgs_knn_topk(N, M, D, K, L.ptr(x), L.ptr(y), L.ptr(dist2), L.ptr(index), L.current_stream())
+        rc = lib.fsgs_knn_topk_ws(N, M, D, K, L.ptr(x), L.ptr(y), L.ptr(dist2), L.ptr(index), L.ptr(ws), nbytes,
+                                  L.current_stream())
     L.check(rc, what)
     return dist2, index
 

@@ -1,0 +1,593 @@
+// K nearest control points of many 3D queries through candidate lists per grid cell, for gfx950.
+//
+// Same result as knn_topk_kernel (point_ops.hip), bit for bit: squared distances dx*dx + dy*dy + dz*dz in single
+// precision without contraction, ascending, equal distances by lower index. What bounds the search over all M control
+// points is its vector work, 18 to 23 instructions for each of the N * M pairs; all but a few dozen control points can be
+// ruled out for a whole cell of a grid over the control points at once:
+//   1. knn_cell_lists_kernel: the cells of a G x G x G grid. U = a bound on the K-th nearest distance of ANY point of the
+//      cell (the K-th smallest of 64 far-corner distances); the cell's list holds the control points whose nearest-corner
+//      distance does not exceed U, in ascending index order. A block builds the list of one of 8 x 8 x 8 coarse cells and
+//      refines it for the (G / 8)^3 cells inside.
+//   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 35 entries for 2048 control
+//      points and G = 32). The walk only keeps the K + 1 smallest keys -- the distance's bits with the low seven replaced
+//      by the list position -- in a sorted register list, one v_med3_u32 per slot; the K exact distances and indices are
+//      looked up afterwards. Queries whose keys cannot separate two neighbours (distances equal in their upper 25 bits),
+//      whose cell has more than 128 candidates, or that lie outside the grid are taken by the whole wavefront one at a
+//      time (64 control points per step), or all together by the search over all control points when they are many.
+// The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.30 ms this way (lists
+// 0.048, queries 0.248; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by the address path
+// of the vector memory (busy 0.7 of the time: every lane reads its own list lines), vector issue is 0.6.
+// 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
+#include <algorithm>
+
+#include "common.hpp"
+
+namespace fsgs {
+namespace {
+
+constexpr int kListCap   = 128;   // candidates per cell: seven position bits
+constexpr int kCoarse    = 8;     // coarse cells per axis
+constexpr int kMaxPoints = 2560;  // control points a block keeps in LDS, 16 bytes each (55 KB in the list kernel)
+constexpr int kMaxK      = 8;
+constexpr int kOctantCap = 1024;  // candidates of an octant of a coarse cell
+constexpr int kAhead = 4;
+// list entries are byte offsets of the control points in a block's LDS copy
+constexpr int kEntryScale = 16;
+static_assert((kMaxPoints + 8) * kEntryScale < 65536, "an entry has 16 bits");
+constexpr int kBuildThreads = 512, kQueryThreads = 512;
+constexpr uint16_t kLongList = 0xffff;
+constexpr int kFewQueries = 16384;
+
+enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
+
+// Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
+// alone) and N * M / 4e12 s when they fill the chip; a wavefront per query 0.8 (M = 512) to 2.0 ns (M = 2048) a query;
+// building the lists 10 us (G = 16, 512 control points) to 48 us (G = 32, 2048). With G = 16 the lists of more than 640
+// control points outgrow their 128 entries; below that the finer grid pays from a million queries on.
+Scheme knn_scheme(int N, int M, int D, int K) {
+  if (D != 3 || K > kMaxK || M > kMaxPoints || M < 96) return kAllPairs;
+  if (N <= kFewQueries) return kAlone;
+  if (M < 192) return kAllPairs;
+  return M > 640 || N >= 1000000 ? kGrid32 : kGrid16;
+}
+
+struct GridLayout {
+  int G;
+  size_t planes, lengths, lists, bytes;
+};
+GridLayout grid_layout(Scheme scheme) {
+  GridLayout l{scheme == kGrid32 ? 32 : scheme == kGrid16 ? 16 : 0, 0, 0, 0, 0};
+  if (l.G == 0) return l;
+  const size_t cells = (size_t) l.G * l.G * l.G;
+  l.planes  = 0;
+  l.lengths = align_up(3 * (size_t) (l.G + 1) * 4, 256);
+  l.lists   = align_up(l.lengths + cells * 2, 256);
+  l.bytes   = l.lists + cells * kListCap * 2;
+  return l;
+}
+
+__device__ __forceinline__ float distance2(float qx, float qy, float qz, const float4& p) {
+#pragma clang fp contract(off)
+  const float dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
+  return (dx * dx + dy * dy) + dz * dz;
+}
+
+// Upper bound on the K-th smallest of the 64 lanes' non-negative values: the value's upper bits by bisection on lane masks
+// (scalar work), the lower `kDrop` bits rounded up (19: at most 1/16 above the value; 0: the value itself). Infinity when
+// fewer than K lanes hold a finite value.
+template <int kDrop = 19>
+__device__ __forceinline__ float wave_kth_bound(float v, int K) {
+  const uint32_t bits = __float_as_uint(v);  // NaN compares above every finite value
+  uint32_t low = 0;
+#pragma unroll
+  for (int b = 30; b >= kDrop; --b) {
+    const uint32_t trial = low | (1u << b);
+    if ((int) __popcll(wave_ballot(bits < trial)) < K) low = trial;
+  }
+  return low >= 0x7f800000u ? __builtin_inff() : __uint_as_float(low | ((1u << kDrop) - 1u));
+}
+
+// Squared distance of a point to the farthest / nearest point of a box.
+__device__ __forceinline__ float box_far2(const float4& p, const float* lo, const float* hi) {
+  const float x = fmaxf(fabsf(p.x - lo[0]), fabsf(p.x - hi[0])), y = fmaxf(fabsf(p.y - lo[1]), fabsf(p.y - hi[1])),
+              z = fmaxf(fabsf(p.z - lo[2]), fabsf(p.z - hi[2]));
+  return x * x + y * y + z * z;
+}
+__device__ __forceinline__ float box_near2(const float4& p, const float* lo, const float* hi) {
+  const float x = fmaxf(fmaxf(lo[0] - p.x, p.x - hi[0]), 0.0f), y = fmaxf(fmaxf(lo[1] - p.y, p.y - hi[1]), 0.0f),
+              z = fmaxf(fmaxf(lo[2] - p.z, p.z - hi[2]), 0.0f);
+  return x * x + y * y + z * z;
+}
+// What a nearest-corner distance may reach at most: the bound widened by far more than the rounding of either side (and,
+// near the underflow threshold, by an absolute amount), so that a point left out is strictly farther in single precision
+// than K points of the list, whatever the query.
+__device__ __forceinline__ float widened(float bound2) { return bound2 * 1.00002f + 1e-36f; }
+
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {
+  return (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) mask, 0u));
+}
+
+// Order-preserving 32-bit image of a float (NaN on top), and back.
+__device__ __forceinline__ uint32_t ordered_bits(float v) {
+  v = v == v ? fminf(fmaxf(v, -3e38f), 3e38f) : 3e38f;
+  const uint32_t b = __float_as_uint(v);
+  return (b & 0x80000000u) ? ~b : b | 0x80000000u;
+}
+__device__ __forceinline__ float from_ordered_bits(uint32_t b) {
+  return __uint_as_float((b & 0x80000000u) ? b & 0x7fffffffu : ~b);
+}
+
+template <int kG>
+struct PlaneLds {
+  static constexpr int kSamples = 8 * kG;
+  uint32_t key[3][kSamples];
+  float sorted[3][kSamples], along[3][kSamples];
+  float plane[3][kG + 1];
+};
+
+// The grid planes, from 8 G sampled control points per axis: sorted by counting ranks, inner planes at equal steps of the
+// accumulated square root of the gaps (cells shrink with density, but slower than quantiles would), one plane a tenth of
+// the extent beyond the sample on either side. Every block computes them for itself (3 us) instead of waiting for another launch.
+template <int kG>
+__device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<kG>& s) {
+  constexpr int S = PlaneLds<kG>::kSamples;
+  const int t = threadIdx.x;
+  for (int e = t; e < 3 * S; e += kBuildThreads) {
+    const int a = e / S, j = e - a * S;
+    const float4 p = s_y[(int) ((int64_t) j * M / S)];
+    s.key[a][j] = (ordered_bits(a == 0 ? p.x : a == 1 ? p.y : p.z) & ~(uint32_t) (S - 1)) | (uint32_t) j;
+  }
+  __syncthreads();
+  for (int e = t; e < 3 * S; e += kBuildThreads) {
+    const int a = e / S, j = e - a * S;
+    const uint32_t mine = s.key[a][j];
+    int rank = 0;
+#pragma unroll 4
+    for (int i = 0; i < S; i += 4) {
+      const uint4 k = *(const uint4*) &s.key[a][i];
+      rank += (k.x < mine) + (k.y < mine) + (k.z < mine) + (k.w < mine);
+    }
+    s.sorted[a][rank] = from_ordered_bits(mine & ~(uint32_t) (S - 1));
+  }
+  __syncthreads();
+  const int a = t >> 6, lane = t & 63;  // a wavefront per axis
+  if (a < 3) {
+    constexpr int kPer = S / 64;
+    float part[kPer], sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int j = lane * kPer + i;
+      sum += j > 0 ? sqrtf(fmaxf(s.sorted[a][j] - s.sorted[a][j - 1], 0.0f)) : 0.0f;
+      part[i] = sum;
+    }
+    float inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const float up = __shfl_up(inc, d, kWave);
+      if (lane >= d) inc += up;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) s.along[a][lane * kPer + i] = (inc - sum) + part[i];
+  }
+  __syncthreads();
+  if (a < 3) {
+    const float lo = s.sorted[a][0], hi = s.sorted[a][S - 1], ext = hi - lo;
+    float v = -3e38f;
+    if (lane <= kG) {
+      const int i = lane;
+      if (i == 0) v = lo - 0.1f * ext;
+      else if (i == kG) v = hi + 0.1f * ext;
+      else {
+        const float target = s.along[a][S - 1] * ((float) (i - 1) / (float) (kG - 2));
+        int j = 0;  // last sample whose accumulated step does not exceed the target
+#pragma unroll
+        for (int step = S / 2; step >= 1; step >>= 1)
+          if (s.along[a][j + step] <= target) j += step;
+        const int n = min(j + 1, S - 1);
+        const float w = s.along[a][n] - s.along[a][j];
+        v = s.sorted[a][j] + (s.sorted[a][n] - s.sorted[a][j]) * (w > 0.0f ? (target - s.along[a][j]) / w : 0.0f);
+      }
+    }
+    // ascending whatever the roundings did
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const float up = __shfl_up(v, d, kWave);
+      if (lane >= d) v = fmaxf(v, up);
+    }
+    if (lane <= kG) s.plane[a][lane] = v;
+  }
+  __syncthreads();
+}
+
+// The members of `sub` within `limit` of a box, appended to `out` (times `scale`) in index order by one wavefront; stops
+// once there are more than `cap`. Returns how many there are, or a number above cap.
+__device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* sub, int n_sub, const float* lo,
+                                            const float* hi, float limit, int cap, int scale, uint16_t* out) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int i0 = 0; i0 < n_sub && n <= cap; i0 += kAhead * kWave) {  // the LDS reads of kAhead steps are in flight together
+    int i[kAhead];
+    bool in[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) i[u] = sub[min(i0 + u * kWave + lane, n_sub - 1)];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      in[u] = (int) (box_near2(s_y[i[u]], lo, hi) <= limit) & (int) (i0 + u * kWave + lane < n_sub);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const unsigned long long m = wave_ballot(in[u]);
+      const int pos = n + lanes_below(m);
+      if (in[u] && pos < cap) out[pos] = (uint16_t) (i[u] * scale);
+      n += (int) __popcll(m);
+    }
+  }
+  return n;
+}
+
+// One block per coarse cell, one wavefront per octant of it: with G = 16 an octant is a cell, with G = 32 it is narrowed
+// down once more for its eight cells. 26 M vector instructions (98 us) when the cells were taken from the coarse list
+// directly: the coarse lists at the rim of the cloud hold nearly everything.
+template <int kG>
+__global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
+    float* __restrict__ planes, uint16_t* __restrict__ lengths, uint16_t* __restrict__ lists) {
+  constexpr int kWaves = kBuildThreads / kWave;
+  static_assert(kWaves == 8, "a wavefront per octant");
+  __shared__ float4 s_y[kMaxPoints];
+  __shared__ uint16_t s_sub[kMaxPoints];  // the coarse cell's list
+  __shared__ uint16_t s_octant[kG > 16 ? kWaves : 1][kG > 16 ? kOctantCap : 1];
+  __shared__ PlaneLds<kG> s;
+  __shared__ float s_bound[kWaves];
+  __shared__ int s_count[kWaves];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  for (int i = t; i < M; i += kBuildThreads) s_y[i] = make_float4(y[3 * i], y[3 * i + 1], y[3 * i + 2], 0.0f);
+  __syncthreads();
+  make_planes<kG>(s_y, M, s);
+  if (blockIdx.x == 0)
+    for (int e = t; e < 3 * (kG + 1); e += kBuildThreads) planes[e] = (&s.plane[0][0])[e];
+
+  constexpr int kSub = kG / kCoarse;  // cells per axis inside a coarse cell
+  const int cc[3] = {(int) blockIdx.x % kCoarse, (int) blockIdx.x / kCoarse % kCoarse, (int) blockIdx.x / (kCoarse * kCoarse)};
+  float lo[3], hi[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][cc[a] * kSub], hi[a] = s.plane[a][(cc[a] + 1) * kSub];
+  // coarse list: every wavefront bounds the K-th distance from the control points it looks at, the best bound counts
+  float least = __builtin_inff();
+  for (int i = t; i < M; i += kBuildThreads) least = fminf(least, box_far2(s_y[i], lo, hi));
+  const float bound = wave_kth_bound(least, K);
+  if (lane == 0) s_bound[wave] = bound;
+  __syncthreads();
+  float limit = s_bound[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) limit = fminf(limit, s_bound[w]);
+  limit = widened(limit);
+  const int per = ((M + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;  // a contiguous share per wavefront: index order
+  const int first = wave * per, last = min(M, first + per);
+  int n_mine = 0;
+  for (int i0 = first; i0 < last; i0 += kWave)
+    n_mine += __popcll(wave_ballot(i0 + lane < last && box_near2(s_y[min(i0 + lane, M - 1)], lo, hi) <= limit));
+  if (lane == 0) s_count[wave] = n_mine;
+  __syncthreads();
+  int at = 0, n_sub = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) at += s_count[w];
+    n_sub += s_count[w];
+  }
+  for (int i0 = first; i0 < last; i0 += kWave) {
+    const bool in = i0 + lane < last && box_near2(s_y[min(i0 + lane, M - 1)], lo, hi) <= limit;
+    const unsigned long long m = wave_ballot(in);
+    if (in) s_sub[at + lanes_below(m)] = (uint16_t) (i0 + lane);
+    at += __popcll(m);
+  }
+  __syncthreads();
+
+  constexpr int kIn = kSub / 2;  // cells per axis inside an octant
+  const int corner[3] = {cc[0] * kSub + (wave & 1) * kIn, cc[1] * kSub + ((wave >> 1) & 1) * kIn,
+                         cc[2] * kSub + (wave >> 2) * kIn};
+  auto bound_of = [&](const uint16_t* sub, int n) {
+    float nearest = __builtin_inff();
+    for (int i0 = lane; i0 < n; i0 += kAhead * kWave) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int i    = i0 + u * kWave;
+        const float d2 = box_far2(s_y[sub[min(i, n - 1)]], lo, hi);
+        nearest        = fminf(nearest, i < n ? d2 : __builtin_inff());
+      }
+    }
+    return widened(wave_kth_bound(nearest, K));
+  };
+  const uint16_t* from = s_sub;
+  int n_from = n_sub;
+  if constexpr (kG > 16) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][corner[a]], hi[a] = s.plane[a][corner[a] + kIn];
+    uint16_t* mine = s_octant[wave];
+    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, bound_of(s_sub, n_sub), kOctantCap, 1, mine);
+    from   = mine;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  for (int c = 0; c < kIn * kIn * kIn; ++c) {
+    const int g[3] = {corner[0] + c % kIn, corner[1] + c / kIn % kIn, corner[2] + c / (kIn * kIn)};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][g[a]], hi[a] = s.plane[a][g[a] + 1];
+    const int cell = (g[2] * kG + g[1]) * kG + g[0];
+    uint16_t* list = lists + (size_t) cell * kListCap;
+    int n = kListCap + 1;  // an octant with too many candidates: its cells have long lists too
+    if (kG == 16 || n_from <= kOctantCap)
+      n = collect_near(s_y, from, n_from, lo, hi, bound_of(from, n_from), kListCap, kEntryScale, list);
+    // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
+    if (n <= kListCap && lane < 8 && n + lane < (n + 7) / 8 * 8) list[n + lane] = (uint16_t) (M * kEntryScale);
+    if (lane == 0) lengths[cell] = n <= kListCap ? (uint16_t) n : kLongList;
+  }
+}
+
+__device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+__device__ __forceinline__ uint32_t and_or_b32(uint32_t a, uint32_t mask, uint32_t b) {
+  uint32_t r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(mask), "s"(b));
+  return r;
+}
+
+template <int kK>
+__device__ __forceinline__ void store_result(float* __restrict__ dist2, int64_t* __restrict__ index, int n,
+                                             const float (&d)[kK], const int (&i)[kK]) {
+  float* od   = dist2 + (size_t) n * kK;
+  int64_t* oi = index + (size_t) n * kK;
+  if constexpr (kK % 4 == 0) {
+#pragma unroll
+    for (int k = 0; k < kK; k += 4) *(float4*) (od + k) = make_float4(d[k], d[k + 1], d[k + 2], d[k + 3]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < kK; ++k) od[k] = d[k];
+  }
+  if constexpr (kK % 2 == 0) {
+#pragma unroll
+    for (int k = 0; k < kK; k += 2) *(longlong2*) (oi + k) = make_longlong2(i[k], i[k + 1]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < kK; ++k) oi[k] = i[k];
+  }
+}
+
+// kG == 0: no grid, a wavefront per query.
+template <int kK, int kG>
+__global__ void __launch_bounds__(kQueryThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
+knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
+    const float* __restrict__ y, const float* __restrict__ planes, const uint16_t* __restrict__ lengths,
+    const uint16_t* __restrict__ lists, float* __restrict__ dist2, int64_t* __restrict__ index) {
+  // a query alone costs a wavefront about 20 M / 64 + 300 instructions, the all-pairs walk about 20 M for all 64
+  const int max_alone = 20 * M / (20 * M / 64 + 300);
+  constexpr int kWaves = kQueryThreads / kWave;
+  extern __shared__ __attribute__((aligned(16))) char s_dyn[];
+  float4* s_y = (float4*) s_dyn;  // [M + 8], the last eight at infinity
+  __shared__ float s_plane[3][kG + 1];
+  __shared__ float s_cand_d[kWaves][kWave];
+  __shared__ int s_cand_i[kWaves][kWave];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  for (int i = t; i < M; i += kQueryThreads) s_y[i] = make_float4(y[3 * i], y[3 * i + 1], y[3 * i + 2], 0.0f);
+  if (t < 8) s_y[M + t] = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
+  if (kG > 0)
+    for (int e = t; e < 3 * (kG + 1); e += kQueryThreads) (&s_plane[0][0])[e] = planes[e];
+  __syncthreads();
+
+  // The whole wavefront on one query: a bound on the K-th distance from the lanes' nearest control points, the control
+  // points within it collected in index order, ranked against each other. False when more than 64 are within the bound.
+  auto alone = [&](int n, float qx, float qy, float qz) -> bool {
+    float least = __builtin_inff();
+    for (int i = lane; i < M; i += kWave) least = fminf(least, distance2(qx, qy, qz, s_y[i]));
+    auto collect = [&](float bound) {
+      int count = 0;
+      for (int i0 = 0; i0 < M; i0 += kWave) {
+        const int i   = min(i0 + lane, M);
+        const float d = distance2(qx, qy, qz, s_y[i]);
+        const unsigned long long m = wave_ballot(i < M) & wave_ballot(d <= bound) & wave_ballot(d < __builtin_inff());
+        const int pos = count + lanes_below(m);
+        if (((m >> lane) & 1ull) && pos < kWave) s_cand_d[wave][pos] = d, s_cand_i[wave][pos] = i;
+        count += (int) __popcll(m);
+      }
+      return count;
+    };
+    int count = collect(wave_kth_bound(least, kK));
+    if (count > kWave) count = collect(wave_kth_bound<0>(least, kK));  // a far query: nearly everything at one distance
+    if (count > kWave) return false;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float d = lane < count ? s_cand_d[wave][lane] : __builtin_inff();
+    const int i   = lane < count ? s_cand_i[wave][lane] : -1;
+    int rank = 0;
+    for (int c = 0; c < count; ++c) {
+      const float o = s_cand_d[wave][c];
+      rank += (int) (o < d) | ((int) (o == d) & (int) (c < lane));
+    }
+    if (lane >= count) rank = lane;  // slots nobody fills
+    if (rank < kK) {
+      dist2[(size_t) n * kK + rank] = lane < count ? d : -1.0f;
+      index[(size_t) n * kK + rank] = i;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return true;
+  };
+  // Every lane on its own query, over all control points in index order.
+  auto all_pairs = [&](float qx, float qy, float qz, float (&bd)[kK], int (&bi)[kK]) {
+#pragma unroll
+    for (int k = 0; k < kK; ++k) bd[k] = __builtin_inff(), bi[k] = -1;
+    for (int m0 = 0; m0 < M; m0 += 8) {
+      float d[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) d[u] = distance2(qx, qy, qz, s_y[m0 + u]);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (d[u] < bd[kK - 1]) {
+          bool before[kK];
+#pragma unroll
+          for (int k = 0; k < kK; ++k) before[k] = d[u] < bd[k];
+#pragma unroll
+          for (int k = kK - 1; k >= 1; --k) {
+            bd[k] = __builtin_amdgcn_fmed3f(bd[k - 1], d[u], bd[k]);
+            const int stay = before[k] ? m0 + u : bi[k];
+            bi[k] = before[k - 1] ? bi[k - 1] : stay;
+          }
+          bd[0] = before[0] ? d[u] : bd[0], bi[0] = before[0] ? m0 + u : bi[0];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kK; ++k)
+      if (bi[k] < 0) bd[k] = -1.0f;
+  };
+
+  if constexpr (kG == 0) {
+    for (int n = blockIdx.x * kWaves + wave; n < N; n += gridDim.x * kWaves) {
+      const float qx = x[3 * (size_t) n], qy = x[3 * (size_t) n + 1], qz = x[3 * (size_t) n + 2];
+      if (!alone(n, qx, qy, qz)) {
+        float bd[kK];
+        int bi[kK];
+        all_pairs(qx, qy, qz, bd, bi);
+        if (lane == 0) store_result<kK>(dist2, index, n, bd, bi);
+      }
+    }
+  } else {
+    for (int n0 = (blockIdx.x * kWaves + wave) * kWave; n0 < N; n0 += gridDim.x * kQueryThreads) {
+      const int n     = n0 + lane;
+      const bool live = n < N;
+      const size_t at = 3 * (size_t) (live ? n : N - 1);
+      const float q[3] = {x[at], x[at + 1], x[at + 2]};
+      bool inside = live;
+      int cell = 0;
+#pragma unroll
+      for (int a = 2; a >= 0; --a) {
+        int i = 0;
+#pragma unroll
+        for (int step = kG / 2; step >= 1; step >>= 1)
+          if (s_plane[a][i + step] <= q[a]) i += step;
+        inside = inside && q[a] >= s_plane[a][0] && q[a] < s_plane[a][kG];  // false for NaN
+        cell   = cell * kG + i;
+      }
+      const int len   = inside ? (int) lengths[cell] : (int) kLongList;
+      bool slow       = live && len == (int) kLongList;
+      const int n_list = len == (int) kLongList ? 0 : len;
+      const uint16_t* list = lists + (size_t) cell * kListCap;
+      const uint32_t key_mask = ~(uint32_t) (kListCap - 1);
+      uint32_t key[kK + 1];
+#pragma unroll
+      for (int k = 0; k <= kK; ++k) key[k] = 0xffffffffu;
+      uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
+      for (int c = 0; c < n_list; c += 8) {  // c is the same in every lane still in the loop
+        const uint4 now = next;
+        if (c + 8 < n_list) next = *(const uint4*) (list + c + 8);
+        const uint32_t w[4] = {now.x, now.y, now.z, now.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t i = (j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu);
+          const float d = distance2(q[0], q[1], q[2], *(const float4*) (s_dyn + i));
+          const uint32_t nk = and_or_b32(__float_as_uint(d), key_mask, (uint32_t) (c + j));
+#pragma unroll
+          for (int k = kK; k >= 1; --k) key[k] = med3_u32(key[k - 1], nk, key[k]);
+          key[0] = min(key[0], nk);
+        }
+      }
+      // neighbours that agree in all the bits a key keeps are not in a known order
+      constexpr uint32_t kInfinite = 0x7f800000u;
+#pragma unroll
+      for (int k = 0; k < kK; ++k)
+        if (key[k] < kInfinite && (key[k] ^ key[k + 1]) < (uint32_t) kListCap) slow = live;
+      float bd[kK];
+      int bi[kK];
+#pragma unroll
+      for (int k = 0; k < kK; ++k) {
+        const bool found = !slow && key[k] < kInfinite;
+        bi[k] = found ? (int) list[key[k] & (uint32_t) (kListCap - 1)] / kEntryScale : M;
+        bd[k] = distance2(q[0], q[1], q[2], s_y[bi[k]]);
+        if (!found) bi[k] = -1, bd[k] = -1.0f;
+      }
+      if (live && !slow) store_result<kK>(dist2, index, n, bd, bi);
+
+      unsigned long long rest = wave_ballot(slow), together = 0ull;
+      if (__popcll(rest) > max_alone) together = rest, rest = 0ull;
+      while (rest) {
+        const int l = __builtin_ctzll(rest);
+        rest &= rest - 1;
+        if (!alone(n0 + l, __shfl(q[0], l, kWave), __shfl(q[1], l, kWave), __shfl(q[2], l, kWave))) together |= 1ull << l;
+      }
+      if (together) {
+        all_pairs(q[0], q[1], q[2], bd, bi);
+        if ((together >> lane) & 1ull) store_result<kK>(dist2, index, n, bd, bi);
+      }
+    }
+  }
+}
+
+template <int kK, int kG>
+void launch_query(int N, int M, const float* x, const float* y, const GridLayout& l, char* ws, float* dist2,
+                  int64_t* index, hipStream_t s) {
+  const size_t lds = 16 * (size_t) (M + 8);
+  // blocks take the queries in strides, so that the control points are staged once for many; two rounds of the four
+  // blocks that fit on a compute unit (one round 259 us, two 248, four and more 248 at 3M x 2048)
+  const int per_block = kG > 0 ? kQueryThreads : kQueryThreads / kWave;
+  const int blocks = std::min(div_up(N, per_block), 256 * 8);
+  hipLaunchKernelGGL((knn_cell_query_kernel<kK, kG>), dim3(blocks), dim3(kQueryThreads), lds, s, N, M, x, y,
+                     (const float*) (ws + l.planes), (const uint16_t*) (ws + l.lengths), (const uint16_t*) (ws + l.lists),
+                     dist2, index);
+}
+
+template <int kK>
+int launch_grid_knn(Scheme scheme, int N, int M, const float* x, const float* y, float* dist2, int64_t* index, char* ws,
+                    hipStream_t s) {
+  const GridLayout l = grid_layout(scheme);
+  if (scheme == kAlone) {
+    launch_query<kK, 0>(N, M, x, y, l, ws, dist2, index, s);
+  } else if (scheme == kGrid16) {
+    hipLaunchKernelGGL(knn_cell_lists_kernel<16>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
+                       (float*) (ws + l.planes), (uint16_t*) (ws + l.lengths), (uint16_t*) (ws + l.lists));
+    launch_query<kK, 16>(N, M, x, y, l, ws, dist2, index, s);
+  } else {
+    hipLaunchKernelGGL(knn_cell_lists_kernel<32>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
+                       (float*) (ws + l.planes), (uint16_t*) (ws + l.lengths), (uint16_t*) (ws + l.lists));
+    launch_query<kK, 32>(N, M, x, y, l, ws, dist2, index, s);
+  }
+  return check_launch("knn_topk");
+}
+
+}  // namespace
+}  // namespace fsgs
+
+using namespace fsgs;
+
+FSGS_API int fsgs_knn_topk(int N, int M, int D, int K, const float* x, const float* y, float* dist2, int64_t* index,
+                           void* stream);
+
+FSGS_API size_t fsgs_knn_topk_workspace_bytes(int N, int M, int D, int K) {
+  return N > 0 && M > 0 ? grid_layout(knn_scheme(N, M, D, K)).bytes : 0;
+}
+
+FSGS_API int fsgs_knn_topk_ws(int N, int M, int D, int K, const float* x, const float* y, float* dist2, int64_t* index,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  FSGS_REQUIRE(N >= 0 && M > 0 && D > 0 && K > 0 && x && y && dist2 && index, "knn_topk: bad arguments");
+  const Scheme scheme = knn_scheme(N, M, D, K);
+  const bool aligned  = (((uintptr_t) dist2 | (uintptr_t) index) & 15) == 0;  // rows are stored in 16-byte pieces
+  if (N == 0 || scheme == kAllPairs || !aligned) return fsgs_knn_topk(N, M, D, K, x, y, dist2, index, stream);
+  if (workspace_bytes < grid_layout(scheme).bytes || (grid_layout(scheme).bytes > 0 && !workspace))
+    return fail(kWorkspaceSmall, "knn_topk: workspace %zu < %zu bytes", workspace_bytes, grid_layout(scheme).bytes);
+  char* ws = (char*) workspace;
+  hipStream_t s = (hipStream_t) stream;
+  switch (K) {
+    case 1: return launch_grid_knn<1>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 2: return launch_grid_knn<2>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 3: return launch_grid_knn<3>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 4: return launch_grid_knn<4>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 5: return launch_grid_knn<5>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 6: return launch_grid_knn<6>(scheme, N, M, x, y, dist2, index, ws, s);
+    case 7: return launch_grid_knn<7>(scheme, N, M, x, y, dist2, index, ws, s);
+    default: return launch_grid_knn<8>(scheme, N, M, x, y, dist2, index, ws, s);
+  }
+}

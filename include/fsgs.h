@@ -350,6 +350,11 @@ int fsgs_cdist_top_backward_typed(int dtype, int B, int N, int M, int D, const v
  * pytorch3d.ops.knn_points(points[None], sp_points[None], K=K) at fast_2d_gs/network.py:504. */
 int fsgs_knn_topk(int N, int M, int D, int K, const float* x, const float* y, float* dist2, int64_t* index,
                   void* stream);
+/* The same result with a workspace of fsgs_knn_topk_workspace_bytes(N, M, D, K) bytes (256-byte aligned; may be 0), which
+ * lets large 3D searches rule out most control points per grid cell instead of forming all N * M distances. */
+size_t fsgs_knn_topk_workspace_bytes(int N, int M, int D, int K);
+int fsgs_knn_topk_ws(int N, int M, int D, int K, const float* x, const float* y, float* dist2, int64_t* index,
+                     void* workspace, size_t workspace_bytes, void* stream);
 
 /* The superpoint warp of fast_2d_gs/network.py:498-573 in one call: neighbour weights (calc_LBS_weight, :507-517) and
  * the blend (warp, :545-573) over the K neighbours index[N,K] (int64, from fsgs_knn_topk; slots outside [0, M) get

@@ -232,6 +232,37 @@ def test_knn_and_lbs(device, oracle_mod, c1):
     assert np.array_equal(npy(idx), ri) and np.array_equal(npy(d2), rd)
 
 
+# the searches by candidate lists: a wavefront per query up to 16384 queries, a 16^3 grid up to 640 control points, a 32^3
+# grid above (at most 2560), all pairs below 192 (96 for few queries) and for K > 8; kinds with ties, degenerate extents,
+# outliers and non-finite coordinates end in the wavefront-per-query and all-pairs fallbacks
+@pytest.mark.parametrize('N,M,K', [(1, 96, 1), (63, 640, 8), (16384, 96, 3), (16385, 191, 2), (16385, 192, 2), (17000, 640, 7),
+                                   (17001, 641, 5), (17003, 2560, 8), (16500, 2561, 4), (17005, 513, 9)])
+@pytest.mark.parametrize('kind', ['normal', 'lattice', 'same', 'outliers', 'nonfinite'])
+def test_knn_candidate_lists(N, M, K, kind, device, oracle_mod):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N + M + K)
+    pts, ctrl = torch.randn(N, 3, generator=g), torch.randn(M, 3, generator=g)
+    if kind == 'lattice':  # many equal distances: the lower index comes first
+        pts, ctrl = (pts * 2).round(), (ctrl * 2).round()
+    elif kind == 'same':
+        ctrl[:] = ctrl[0]
+    elif kind == 'outliers':
+        pts[::50] *= 40
+        ctrl[::40] *= 40
+    elif kind == 'nonfinite':
+        pts[::7, 0], pts[::11, 1], ctrl[::13, 2], ctrl[::17, 0] = float('nan'), float('inf'), float('-inf'), float('nan')
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    if kind == 'nonfinite':  # the all-pairs kernel defines what happens to distances that are not finite
+        from fast_sp_gs_amd import lib as L
+        x, y, want_d, want_i = pts.to(device), ctrl.to(device), torch.empty_like(d2), torch.empty_like(idx)
+        L.check(L.load().fsgs_knn_topk(N, M, 3, K, L.ptr(x), L.ptr(y), L.ptr(want_d), L.ptr(want_i), L.current_stream()), 'knn')
+        assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+        return
+    rd, ri = np.zeros((N, K), np.float32), np.zeros((N, K), np.int64)
+    oracle_mod.call("knn_topk_f32", N, M, 3, K, npy(pts), npy(ctrl), rd, ri)
+    assert np.array_equal(npy(idx), ri) and np.array_equal(npy(d2), rd)
+
+
 LBS_CASES = [  # (warp method with a local rotation | None without one, weight method)
     (None, 'weighted_kernel'),   # the reference's default configuration: translations only, kernel weights
     (None, 'dist'), ('LBS', 'dist'), ('LBS_c', 'dist'), ('LBS_c', 'weighted_kernel'), ('LBS', 'kernel'),
