@@ -19,6 +19,7 @@
 
 #include "binning.hpp"
 #include "blend.hpp"
+#include "instance_slots.hpp"
 
 namespace fsgs {
 namespace {
@@ -334,8 +335,10 @@ inline BinsLayout bins_layout(int P, int T) {
 template <int kMode>
 __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, int gx, int gy,
     const float2* __restrict__ means2D, const int32_t* __restrict__ radii, WalkInputs in,
-    uint32_t* __restrict__ hist) {
+    uint32_t* __restrict__ hist, SlotPublish publish) {
   __shared__ unsigned s_count[kMaxLdsTiles];
+  // first of all, so that the instance count reaches the host while the rest of the counting is still running
+  if (publish.counters && blockIdx.x == 0 && threadIdx.x < kWave) publish_slot_regions(publish);
   const int T = gx * gy;
   for (int t = threadIdx.x; t < T; t += blockDim.x) s_count[t] = 0u;
   __syncthreads();
@@ -785,6 +788,8 @@ __global__ void __launch_bounds__(kSortThreads) sort_scatter_kernel(int64_t R, i
   }
 }
 
+__global__ void __launch_bounds__(kWave) publish_slots_kernel(SlotPublish publish) { publish_slot_regions(publish); }
+
 // ---- ranges -----------------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) fill_zero_i64_kernel(int64_t n, int64_t* __restrict__ p) {
   const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -905,10 +910,10 @@ int fast_bucket_fill(int P, int W, int H, const float* means2D, const float* inv
   const WalkInputs in{inverse_m, opacities, keep_masks};
   if (keep_masks)
     hipLaunchKernelGGL(tile_hist_kernel<kWalkCornerMask>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                       (const float2*) means2D, radii, in, hist);
+                       (const float2*) means2D, radii, in, hist, SlotPublish{});
   else
     hipLaunchKernelGGL(tile_hist_kernel<kWalkCorner>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                       (const float2*) means2D, radii, in, hist);
+                       (const float2*) means2D, radii, in, hist, SlotPublish{});
   hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
                      bl.blocks, hist, rng);
   hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
@@ -1012,7 +1017,7 @@ namespace {
 // keep_masks (optional): the per-surfel keep masks of cull_mask_kernel; with them an instance is only counted (and
 // later scattered) when its bit is set.
 int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const uint32_t* keep_masks,
-               int64_t* ranges, void* bins, hipStream_t s) {
+               int64_t* ranges, void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
@@ -1022,10 +1027,10 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
     uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
     if (keep_masks)
       hipLaunchKernelGGL(tile_hist_kernel<kWalkMask>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, keep_masks}, hist);
+                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, keep_masks}, hist, publish);
     else
       hipLaunchKernelGGL(tile_hist_kernel<kWalkAll>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, nullptr}, hist);
+                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, nullptr}, hist, publish);
     hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
                        bl.blocks, hist, rng);
     hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
@@ -1033,6 +1038,7 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
     // sorts) is built from them by an extra block of the scatter, in the second part.
   } else {
     // no room for one LDS counter per tile (or no surfels): count straight into ranges[t].y, then scan to (start, start)
+    if (publish.counters) hipLaunchKernelGGL(publish_slots_kernel, dim3(1), dim3(kWave), 0, s, publish);
     hipLaunchKernelGGL(fill_zero_i64_kernel, dim3(div_up(2 * (int64_t) T, 256)), dim3(256), 0, s, 2 * (int64_t) T,
                        ranges);
     if (P > 0)
@@ -1177,6 +1183,37 @@ FSGS_API int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const floa
                 fsgs_gs_prepare_bins_bytes(P, W, H));
   return fill_sort(P, W, H, means2D, depths, radii, culling_enabled() ? masks : nullptr, R, ranges,
                    point_list, sorted_keys_out, workspace, bins, (hipStream_t) stream);
+}
+
+// The counting part for views whose preprocess handed out the record slots (instance_slots.hpp).
+FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii,
+                                const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
+                                int64_t* num_rendered_host, int64_t* ranges, void* bins, size_t bins_bytes,
+                                void* stream) {
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins, "gs_view_count: bad arguments");
+  FSGS_REQUIRE(means2D && radii && slot_counters && num_rendered_host, "gs_view_count: null pointer");
+  if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
+    return fail(kWorkspaceSmall, "gs_view_count: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+  tile_order_invalidate((hipStream_t) stream);
+  __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  return fill_count(P, W, H, means2D, radii, culling_enabled() ? keep_masks : nullptr, ranges, bins,
+                    (hipStream_t) stream, SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
+}
+
+// Waits until the count has been written. Reading the word is all it takes as long as the stream works; a stream that
+// has run dry, or failed, without writing it is an error.
+FSGS_API int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream) {
+  FSGS_REQUIRE(num_rendered_host, "gs_view_wait: null pointer");
+  for (unsigned spins = 1;; ++spins) {
+    if (__atomic_load_n(num_rendered_host, __ATOMIC_ACQUIRE) >= 0) return kOk;
+    if (spins % 65536 == 0) {
+      const hipError_t e = hipStreamQuery((hipStream_t) stream);
+      if (e == hipErrorNotReady) continue;
+      if (__atomic_load_n(num_rendered_host, __ATOMIC_ACQUIRE) >= 0) return kOk;
+      return fail(kLaunchFailure, "gs_view_wait: %s", e == hipSuccess ? "the stream ended without an instance count" : hipGetErrorString(e));
+    }
+    __builtin_ia32_pause();
+  }
 }
 
 FSGS_API int fsgs_gs_prepare_fill(int P, int W, int H, const float* means2D, const float* depths,

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "blend.hpp"
+#include "instance_slots.hpp"
 #include "pair_queue.hpp"
 
 namespace fsgs {
@@ -56,9 +57,14 @@ blend_backward_kernel(
     const float2* __restrict__ out_flow, const float* __restrict__ dL_dpix, const float* __restrict__ dL_dextras,
     const float* __restrict__ dL_dopacity, const float2* __restrict__ dL_dflow, float* __restrict__ g_means2D,
     float* __restrict__ g_normal_opacity, float* __restrict__ g_colors, float* __restrict__ g_trans,
-    const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii, float* __restrict__ slot_grads,
+    SlotSource slots, const int32_t* __restrict__ radii, float* __restrict__ slot_grads,
     const float4* __restrict__ records) {
   constexpr bool kQueue = kBwdQueue && !kFlow;
+  // First record slot of a surfel; `stored` is what its packed record says (-1: packed before the offsets were known).
+  auto first_slot = [&](int id, int64_t stored) -> int64_t {
+    if (slots.region) return (stored >= 0 ? stored : (int64_t) slots.offset[id]) + slots.region[slot_region(id)];
+    return stored >= 0 ? stored : (id == 0 ? 0 : slots.scan[id - 1]);
+  };
   __shared__ SplatHot s_hot[kBwdBatch];
   __shared__ SplatCold s_cold[kBwdBatch];
   // Each wavefront's sums over its 64 pixels, one row per staged surfel; the flush adds the four rows in wavefront
@@ -108,12 +114,11 @@ blend_backward_kernel(
       int64_t off;
       if (records) {
         const float4 q2 = records[5 * (size_t) id + 2], q4 = records[5 * (size_t) id + 4];
-        cx = q2.y, cy = q2.z, rad = __float_as_int(q4.z), off = (int64_t) __float_as_int(q4.w);
-        if (rad < 0) rad = radii[id];  // a record packed without radii / offsets holds -1 there
-        if (off < 0) off = id == 0 ? 0 : point_offsets[id - 1];
+        cx = q2.y, cy = q2.z, rad = __float_as_int(q4.z), off = first_slot(id, (int64_t) __float_as_int(q4.w));
+        if (rad < 0) rad = radii[id];  // a record packed without radii holds -1 there
       } else {
         const float2 c = means2D[id];
-        cx = c.x, cy = c.y, rad = radii[id], off = id == 0 ? 0 : point_offsets[id - 1];
+        cx = c.x, cy = c.y, rad = radii[id], off = first_slot(id, -1);
       }
       const TileRect r = tile_rect(cx, cy, rad, gx, gy);
       const int64_t slot = off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0);
@@ -181,7 +186,7 @@ blend_backward_kernel(
       // a record carries the surfel's radius (-1 if it was packed without radii) and, once the binning's scan has
       // stored it, its offset (-1 until then)
       next_radius = records && ex.radius >= 0 ? ex.radius : radii[next.cold.id];
-      next_off    = records && ex.offset >= 0 ? ex.offset : (next.cold.id == 0 ? 0 : point_offsets[next.cold.id - 1]);
+      next_off    = first_slot(next.cold.id, records ? ex.offset : -1);
     }
   }
 
@@ -214,7 +219,7 @@ blend_backward_kernel(
         for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
       if (kSlots) {
         next_radius = records && ex.radius >= 0 ? ex.radius : radii[next.cold.id];
-        next_off    = records && ex.offset >= 0 ? ex.offset : (next.cold.id == 0 ? 0 : point_offsets[next.cold.id - 1]);
+        next_off    = first_slot(next.cold.id, records ? ex.offset : -1);
       }
     }
 
@@ -524,7 +529,7 @@ blend_backward_kernel(
 // ends. A surfel's records are fetched eight at a time (past its last record the last one is read again and not added),
 // so most surfels need one round trip to memory; the sum itself runs in instance order. Every row of the four outputs
 // is written (zeros for surfels without instances): no initialisation, no atomics, and the sum order is fixed.
-__global__ void __launch_bounds__(256) slot_reduce_kernel(int P, const int64_t* __restrict__ point_offsets,
+__global__ void __launch_bounds__(256) slot_reduce_kernel(int P, SlotSource slots,
     const float* __restrict__ slot_grads, float* __restrict__ g_colors, float* __restrict__ g_means2D,
     float* __restrict__ g_trans, float* __restrict__ g_normal_opacity) {
   constexpr int kPerWave = 7, kLanes = 9;  // 63 of 64 lanes busy
@@ -534,8 +539,11 @@ __global__ void __launch_bounds__(256) slot_reduce_kernel(int P, const int64_t* 
   const int sub = lane / kLanes, k = lane - sub * kLanes;
   const int i = wave * kPerWave + sub;
   if (sub >= kPerWave || i >= P) return;
-  // A surfel without instances (not rendered) has equal scan offsets, so the visibility need not be read.
-  const int64_t e0 = i > 0 ? point_offsets[i - 1] : 0, e1 = point_offsets[i];
+  // A surfel without instances (not rendered) has an empty span, so the visibility need not be read.
+  int64_t e0;
+  int count;
+  slot_span(slots, i, e0, count);
+  const int64_t e1 = e0 + count;
   const float2* src = (const float2*) slot_grads + k;
   float2 acc = make_float2(0.0f, 0.0f);
   for (int64_t base = e0; base < e1; base += kDepth) {
@@ -563,7 +571,7 @@ __global__ void __launch_bounds__(256) slot_reduce_kernel(int P, const int64_t* 
 // The same sum over lists built by the culled binning (fsgs_gs_prepare_*_culled): the positions of a surfel's span
 // whose bit is clear in its keep mask belong to no list, were never written and are not read. Nine positions of the
 // span per step, row-major over the surfel's rectangle, the records of the kept ones requested together.
-__global__ void __launch_bounds__(256) slot_reduce_culled_kernel(int P, const int64_t* __restrict__ point_offsets,
+__global__ void __launch_bounds__(256) slot_reduce_culled_kernel(int P, SlotSource slots,
     const uint32_t* __restrict__ masks, const float* __restrict__ slot_grads, float* __restrict__ g_colors,
     float* __restrict__ g_means2D, float* __restrict__ g_trans, float* __restrict__ g_normal_opacity) {
   constexpr int kPerWave = 7, kLanes = 9;
@@ -572,8 +580,9 @@ __global__ void __launch_bounds__(256) slot_reduce_culled_kernel(int P, const in
   const int sub = lane / kLanes, k = lane - sub * kLanes;
   const int i = wave * kPerWave + sub;
   if (sub >= kPerWave || i >= P) return;
-  const int64_t e0 = i > 0 ? point_offsets[i - 1] : 0, e1 = point_offsets[i];
-  const int count = (int) (e1 - e0);
+  int64_t e0;
+  int count;
+  slot_span(slots, i, e0, count);
   // rectangles above kCullMaskTiles tiles are kept whole
   const uint32_t mask = count > kCullMaskTiles ? 0xffffffffu : masks[i];
   const float2* src = (const float2*) slot_grads + (size_t) e0 * kLanes + k;
@@ -614,7 +623,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
     const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
     const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
     const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
-    float* g_normal_opacity, int64_t R, const int64_t* point_offsets, const int32_t* radii, void* workspace,
+    float* g_normal_opacity, int64_t R, const SlotSource& source, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const float* records, const uint32_t* keep_masks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_render_backward: bad sizes");
   if (P == 0) return kOk;
@@ -626,7 +635,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
   FSGS_REQUIRE(!flow || (trans_mat_t2 && out_flow && aux),
                "GS_2D_render_backward: flow gradients need trans_mat_t2, out_flow and the auxiliary maps");
   FSGS_REQUIRE(((uintptr_t) records & 15) == 0, "GS_2D_render_backward: records must be 16-byte aligned");
-  const bool slots = point_offsets != nullptr;
+  const bool slots = source.scan || source.region;
   if (slots) {
     FSGS_REQUIRE(radii && workspace && R >= 0 && R < (int64_t) 0x7fffffff,
                  "GS_2D_render_backward: the ordered-sum path needs radii, a workspace and the instance count R");
@@ -645,7 +654,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
                      (float) far_n, ranges, point_list, n_contrib, (const float2*) means2D,                          \
                      (const float4*) normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity, out_extras,       \
                      (const float2*) out_flow, dL_dpix, dL_dextras, dL_dopacity, (const float2*) dL_dflow,           \
-                     g_means2D, g_normal_opacity, g_colors, g_trans, point_offsets, radii, slot_grads,               \
+                     g_means2D, g_normal_opacity, g_colors, g_trans, source, radii, slot_grads,               \
                      (const float4*) records)
   if (slots) {
     if (aux && flow) FSGS_LAUNCH_BWD(true, true, true);
@@ -654,9 +663,9 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
     const int waves = div_up(P, 7);  // kPerWave surfels per wavefront
     if (keep_masks && culling_enabled())
       hipLaunchKernelGGL(slot_reduce_culled_kernel, dim3(div_up((int64_t) waves * 64, 256)), dim3(256), 0, s, P,
-                         point_offsets, keep_masks, slot_grads, g_colors, g_means2D, g_trans, g_normal_opacity);
+                         source, keep_masks, slot_grads, g_colors, g_means2D, g_trans, g_normal_opacity);
     else
-      hipLaunchKernelGGL(slot_reduce_kernel, dim3(div_up((int64_t) waves * 64, 256)), dim3(256), 0, s, P, point_offsets,
+      hipLaunchKernelGGL(slot_reduce_kernel, dim3(div_up((int64_t) waves * 64, 256)), dim3(256), 0, s, P, source,
                          slot_grads, g_colors, g_means2D, g_trans, g_normal_opacity);
   } else {
     if (aux && flow) FSGS_LAUNCH_BWD(true, true, false);
@@ -677,7 +686,7 @@ FSGS_API int fsgs_gs_2d_render_backward(int P, int W, int H, double near_n, doub
     size_t workspace_bytes, const float* records, void* stream) {
   return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
-                         g_colors, g_means2D, g_trans, g_normal_opacity, R, point_offsets, radii, workspace,
+                         g_colors, g_means2D, g_trans, g_normal_opacity, R, SlotSource{point_offsets}, radii, workspace,
                          workspace_bytes, records, nullptr, stream);
 }
 
@@ -692,6 +701,24 @@ FSGS_API int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_
                "GS_2D_render_backward_culled: the ordered-sum path over culled lists needs the keep masks");
   return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
-                         g_colors, g_means2D, g_trans, g_normal_opacity, R, point_offsets, radii, workspace,
+                         g_colors, g_means2D, g_trans, g_normal_opacity, R, SlotSource{point_offsets}, radii, workspace,
+                         workspace_bytes, records, keep_masks, stream);
+}
+
+// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp).
+FSGS_API int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
+    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
+    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
+    const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
+    float* g_normal_opacity, int64_t R, const int32_t* slot_offsets, const int32_t* slot_regions,
+    const int32_t* tiles_touched, const int32_t* radii, void* workspace, size_t workspace_bytes, const float* records,
+    const uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && records),
+               "gs_2d_view_backward: record slots and packed records are required");
+  return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
+                         out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
+                         g_colors, g_means2D, g_trans, g_normal_opacity, R,
+                         SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
                          workspace_bytes, records, keep_masks, stream);
 }

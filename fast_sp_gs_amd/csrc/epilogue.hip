@@ -155,7 +155,8 @@ __global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, fl
     const float* __restrict__ opacity, const float* __restrict__ background, const float* __restrict__ g_normals,
     const float* __restrict__ g_depths, const float* __restrict__ g_surf_depth,
     const float* __restrict__ g_surf_normal, const float* __restrict__ g_distortion,
-    const float* __restrict__ g_composited, float* __restrict__ g_extras, float* __restrict__ g_opacity) {
+    const float* __restrict__ g_composited, const float* __restrict__ g_opacity_in, float* __restrict__ g_extras,
+    float* __restrict__ g_opacity) {
   __shared__ PixelRays s_rays;
   if (threadIdx.x == 0 && threadIdx.y == 0) pixel_rays(W, H, Tw2v, Tv2c, s_rays);
   __syncthreads();
@@ -208,7 +209,7 @@ __global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, fl
     if (g_composited)
 #pragma unroll
       for (int c = 0; c < 3; ++c) s += g_composited[c * HW + p] * background[c];
-    g_opacity[p] = -s;
+    g_opacity[p] = g_opacity_in ? g_opacity_in[p] - s : -s;
   }
 }
 
@@ -231,10 +232,10 @@ FSGS_API int fsgs_gs_2d_epilogue_forward(int W, int H, double depth_ratio, const
   return check_launch("gs_2d_epilogue_forward");
 }
 
-FSGS_API int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
+FSGS_API int fsgs_gs_2d_view_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
-    float* g_extras, float* g_opacity, void* stream) {
+    const float* g_opacity_in, float* g_extras, float* g_opacity, void* stream) {
   FSGS_REQUIRE(W >= 0 && H >= 0, "gs_2d_epilogue_backward: bad size");
   if ((size_t) W * H == 0) return kOk;
   FSGS_REQUIRE(Tw2v && Tv2c && extras && opacity && g_extras, "gs_2d_epilogue_backward: null pointer");
@@ -243,6 +244,15 @@ FSGS_API int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, cons
   const dim3 grid(div_up(W, 32), div_up(H, 8)), block(32, 8);
   hipLaunchKernelGGL(epilogue_backward_kernel, grid, block, 0, (hipStream_t) stream, W, H, (float) depth_ratio, Tw2v,
                      Tv2c, extras, opacity, background, g_normals, g_depths, g_surf_depth, g_surf_normal, g_distortion,
-                     g_composited, g_extras, g_opacity);
+                     g_composited, g_opacity_in, g_extras, g_opacity);
   return check_launch("gs_2d_epilogue_backward");
+}
+
+FSGS_API int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
+    const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
+    const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
+    float* g_extras, float* g_opacity, void* stream) {
+  return fsgs_gs_2d_view_epilogue_backward(W, H, depth_ratio, Tw2v, Tv2c, extras, opacity, background, g_normals, g_depths,
+                                           g_surf_depth, g_surf_normal, g_distortion, g_composited, nullptr, g_extras,
+                                           g_opacity, stream);
 }

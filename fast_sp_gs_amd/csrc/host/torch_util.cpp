@@ -1,0 +1,75 @@
+#include "torch_util.hpp"
+
+#include <map>
+
+namespace fsgs_host {
+
+std::string shape_text(at::IntArrayRef shape) {
+  std::string s = "(";
+  for (size_t i = 0; i < shape.size(); ++i) s += (i ? ", " : "") + std::to_string(shape[i]);
+  return s + (shape.size() == 1 ? ",)" : ")");
+}
+
+std::string dtype_text(at::ScalarType type) {
+  switch (type) {
+    case at::kFloat: return "torch.float32";
+    case at::kDouble: return "torch.float64";
+    case at::kHalf: return "torch.float16";
+    case at::kBFloat16: return "torch.bfloat16";
+    case at::kInt: return "torch.int32";
+    case at::kLong: return "torch.int64";
+    case at::kBool: return "torch.bool";
+    case at::kByte: return "torch.uint8";
+    default: return c10::toString(type);
+  }
+}
+
+void require(const char* what, const char* name, const Tensor& t, at::ScalarType type) {
+  if (!t.is_cuda()) fail(std::string(what) + ": " + name + " must be a CUDA tensor");
+  if (!t.is_contiguous()) fail(std::string(what) + ": " + name + " must be contiguous");
+  if (t.scalar_type() != type)
+    fail(std::string(what) + ": " + name + " must have dtype " + dtype_text(type) + ", got " + dtype_text(t.scalar_type()));
+}
+
+void require_shape(const char* what, const char* name, const Tensor& t, at::IntArrayRef shape) {
+  if (t.sizes() != shape)
+    fail(std::string(what) + ": " + name + " must have shape " + shape_text(shape) + ", got " + shape_text(t.sizes()));
+}
+
+int64_t* pinned_count() {
+  static thread_local Tensor word;
+  if (!word.defined()) word = at::zeros({8}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  return word.data_ptr<int64_t>();
+}
+
+namespace {
+constexpr size_t kMostCounters = 64;  // kept in all, over streams and devices
+std::mutex g_counters_mu;
+std::map<std::pair<int, void*>, std::vector<Tensor>>& free_counters() {
+  static auto* m = new std::map<std::pair<int, void*>, std::vector<Tensor>>;  // outlives the allocator's own end
+  return *m;
+}
+size_t g_counters_kept = 0;
+}  // namespace
+
+SlotCounters::SlotCounters(const Tensor& like) : key_((int) like.device().index(), stream_of(like)) {
+  {
+    std::lock_guard<std::mutex> lock(g_counters_mu);
+    auto it = free_counters().find(key_);
+    if (it != free_counters().end() && !it->second.empty()) {
+      memory_ = std::move(it->second.back());
+      it->second.pop_back();
+      --g_counters_kept;
+    }
+  }
+  if (!memory_.defined()) memory_ = at::zeros({kSlotRegions}, like.options().dtype(at::kLong));
+}
+
+void SlotCounters::give_back() {
+  std::lock_guard<std::mutex> lock(g_counters_mu);
+  if (g_counters_kept >= kMostCounters) return;  // the allocator takes them back
+  free_counters()[key_].push_back(std::move(memory_));
+  ++g_counters_kept;
+}
+
+}  // namespace fsgs_host

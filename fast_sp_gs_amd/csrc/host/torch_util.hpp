@@ -1,0 +1,98 @@
+// Shared pieces of the native host layer: argument checks with the operators' error texts, output allocation, and the two
+// small resources a view needs besides its tensors (a pinned word for the instance count, zeroed slot counters).
+//
+// This layer does in C++ what the Python operators do for one whole render call: check, allocate, launch, record one
+// autograd node. A render of 10k surfels keeps the GPU busy for 0.08 ms and its backward for 0.09 ms; marshalling its 13 to
+// 20 launches through Python took 0.14 and 0.4 ms.
+#pragma once
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+
+#include <mutex>
+#include <stdexcept>
+#include <string>
+#include <unordered_map>
+#include <vector>
+
+#include "../../../include/fsgs.h"
+
+namespace fsgs_host {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+constexpr int kTile = 16, kSlotRegions = 64;
+
+[[noreturn]] inline void fail(const std::string& text) { throw std::runtime_error(text); }
+
+inline void check(int rc, const char* what) {
+  if (rc == 0) return;
+  const char* text = fsgs_last_error();
+  fail(std::string(what) + ": " + (text && *text ? text : "error") + " (status " + std::to_string(rc) + ")");
+}
+
+std::string shape_text(at::IntArrayRef shape);
+std::string dtype_text(at::ScalarType type);
+
+// A device tensor, contiguous, of the given type (the operators' CHECK_INPUT).
+void require(const char* what, const char* name, const Tensor& t, at::ScalarType type);
+void require_shape(const char* what, const char* name, const Tensor& t, at::IntArrayRef shape);
+inline bool has(const OptTensor& t) { return t.has_value() && t->defined(); }
+inline Tensor opt(const OptTensor& t) { return has(t) ? *t : Tensor(); }
+
+template <typename T>
+T* data(const Tensor& t) {
+  return t.defined() ? (T*) t.data_ptr() : nullptr;
+}
+inline float* f32(const Tensor& t) { return data<float>(t); }
+inline int32_t* i32(const Tensor& t) { return data<int32_t>(t); }
+inline int64_t* i64(const Tensor& t) { return data<int64_t>(t); }
+
+inline Tensor empty(at::IntArrayRef shape, const Tensor& like, at::ScalarType type = at::kFloat) {
+  return at::empty(shape, like.options().dtype(type));
+}
+inline Tensor contiguous(const Tensor& t) { return t.defined() ? t.contiguous() : t; }
+
+inline void* stream_of(const Tensor& t) { return (void*) c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// One uninitialised allocation handed out in 256-byte aligned pieces: a view's scratch, or what only its backward reads.
+class Slab {
+ public:
+  size_t reserve(size_t bytes) {
+    const size_t at = size_;
+    size_ = (size_ + bytes + 255) / 256 * 256;
+    return at;
+  }
+  void allocate(const Tensor& like) { memory_ = empty({(int64_t) (size_ ? size_ : 1)}, like, at::kByte); }
+  template <typename T>
+  T* at(size_t offset) const {
+    return (T*) ((char*) memory_.data_ptr() + offset);
+  }
+  const Tensor& memory() const { return memory_; }
+
+ private:
+  size_t size_ = 0;
+  Tensor memory_;
+};
+
+// Page-locked word the instance count of a view is stored to; one per host thread (a thread waits for its count before
+// it starts the next view).
+int64_t* pinned_count();
+
+// 64 zeroed counters on the tensor's device for one view on its current stream. They go back to a list of that stream
+// once the kernel that zeroes them again is queued; a view that fails in between drops them.
+class SlotCounters {
+ public:
+  explicit SlotCounters(const Tensor& like);
+  uint64_t* data() const { return (uint64_t*) memory_.data_ptr(); }
+  void give_back();
+
+ private:
+  Tensor memory_;
+  std::pair<int, void*> key_;
+};
+
+}  // namespace fsgs_host

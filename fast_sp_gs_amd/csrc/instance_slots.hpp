@@ -1,0 +1,86 @@
+// Where the gradient records of a (surfel, tile) instance go, and how many instances a view has.
+//
+// A surfel's instances take consecutive record slots in the order of the tiles of its rectangle. Two ways of handing the
+// slots out:
+//  * the inclusive prefix scan of tiles_touched (the reference's point_offsets), two kernels of their own;
+//  * by regions: the preprocess kernel's block b (256 surfels) takes its slots from region b % 64 with one atomic on that
+//    region's counter, so a surfel's offset inside its region is known while its record is written, and no scan, no copy
+//    of the count and no second pass over the records is needed (15 us at 300k surfels, 110 us at 3M: the scan's kernel
+//    that stored 3M offsets into 80-byte records alone took 91). The regions' first slots follow from the 64 counters
+//    afterwards (publish_slot_regions, run by a block of the next kernel), which also hands the instance count to the
+//    host. Which block comes first inside a region varies from run to run, the sums do not: a surfel's records are always
+//    its own, added in tile order.
+// 64 counters keep the atomics on one address few (5 at 300k surfels, 180 at 3M); they are served one after the other.
+#pragma once
+#include "common.hpp"
+
+namespace fsgs {
+
+constexpr int kSlotRegions = 64;
+constexpr int kSlotBlockBits = 8;  // the preprocess kernels' block: 256 surfels
+
+struct SlotSource {
+  const int64_t* scan = nullptr;     // [P] inclusive prefix scan, or
+  const int32_t* offset = nullptr;   // [P] offset inside the surfel's region,
+  const int32_t* region = nullptr;   // [64] first slot of each region,
+  const int32_t* tiles = nullptr;    // [P] instances of the surfel
+};
+
+__device__ __forceinline__ int slot_region(int i) { return (i >> kSlotBlockBits) & (kSlotRegions - 1); }
+
+__device__ __forceinline__ void slot_span(const SlotSource& s, int i, int64_t& first, int& count) {
+  if (s.region) {
+    first = (int64_t) s.offset[i] + s.region[slot_region(i)];
+    count = s.tiles[i];
+  } else {
+    first = i > 0 ? s.scan[i - 1] : 0;
+    count = (int) (s.scan[i] - first);
+  }
+}
+
+// First part, one call by all 256 lanes of the block: lane-ordered prefix of `count` over the block. `s_wave`: four words
+// of LDS. Holds a barrier.
+__device__ __forceinline__ int slots_in_block(int count, int* s_wave, int& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int inc = count;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int up = __shfl_up(inc, d, kWave);
+    if (lane >= d) inc += up;
+  }
+  if (lane == kWave - 1) s_wave[wave] = inc;
+  __syncthreads();
+  int before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int v = s_wave[w];
+    if (w < wave) before += v;
+    total += v;
+  }
+  return before + inc - count;
+}
+
+// What the kernel behind the preprocess hands on: see above. `counters` nullptr: nothing to do.
+struct SlotPublish {
+  unsigned long long* counters = nullptr;  // [64], zeroed again
+  int32_t* region = nullptr;               // [64] or nullptr
+  int64_t* host_count = nullptr;           // pinned host memory
+};
+
+// One wavefront.
+__device__ __forceinline__ void publish_slot_regions(const SlotPublish& p) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long mine = p.counters[lane];
+  unsigned long long inc = mine;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const unsigned long long up = __shfl_up(inc, d, kWave);
+    if (lane >= d) inc += up;
+  }
+  if (p.region) p.region[lane] = (int32_t) (inc - mine);
+  p.counters[lane] = 0ull;
+  if (lane == kWave - 1) __hip_atomic_store(p.host_count, (int64_t) inc, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace fsgs

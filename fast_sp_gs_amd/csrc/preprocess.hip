@@ -7,6 +7,7 @@
 // against a plain IEEE evaluation of the same expressions.
 #include "common.hpp"
 #include "cull_bound.hpp"
+#include "instance_slots.hpp"
 #include "sh.hpp"
 #include "sh_stage.hpp"
 #include "surfel_geom.hpp"
@@ -81,6 +82,14 @@ __device__ __forceinline__ void transmat(int W, int H, const float* p, float sx,
   nrm[2] = Tw2v[8] * t0 + Tw2v[9] * t1 + Tw2v[10] * t2;
 }
 
+// What a view through the native host path asks for on top (all optional): the surfel's first record slot inside its
+// block's region (instance_slots.hpp), the region counters, and the visibility as a byte.
+struct ViewOutputs {
+  unsigned long long* counters = nullptr;
+  int32_t* slot_offsets = nullptr;
+  uint8_t* visible = nullptr;
+};
+
 // kWave: complete degree-3 rows in one 16-byte aligned [P,16,3] tensor, moved by each wavefront on its own.
 template <int kSh, bool kWave>
 __global__ void __launch_bounds__(256) preprocess_forward_kernel(
@@ -90,11 +99,14 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     const float* __restrict__ campos, const float* __restrict__ trans_precomp, const uint8_t* __restrict__ culling,
     int means2D_preserve, float2* __restrict__ means2D, float* __restrict__ colors, float* __restrict__ trans_mat,
     float4* __restrict__ normal_opacity, float* __restrict__ depths, int32_t* __restrict__ radii,
-    int32_t* __restrict__ tiles_touched, float4* __restrict__ records, uint32_t* __restrict__ keep_masks) {
+    int32_t* __restrict__ tiles_touched, float4* __restrict__ records, uint32_t* __restrict__ keep_masks,
+    ViewOutputs view) {
   constexpr bool kStage = kSh == 16;  // degree <= 3: SH rows travel through LDS, read from HBM line by line
   __shared__ float s_Tw2v[16], s_Tw2c[16];
   __shared__ float s_rows[kStage ? kShStageRows * kShStageStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
+  __shared__ int s_wave_slots[4];
+  __shared__ int s_block_slot;
   load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
@@ -149,6 +161,14 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     ok    = true;
   } while (false);
 
+  // the block's record slots: the atomic is on its way while the colours are formed
+  int slot = 0;
+  unsigned long long block_slot = 0;
+  if (view.counters) {
+    int total;
+    slot = slots_in_block(ok ? area : 0, s_wave_slots, total);
+    if (threadIdx.x == 0) block_slot = atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+  }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
     if (kWave) {
@@ -171,8 +191,15 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
     }
   }
+  if (view.slot_offsets) {
+    if (threadIdx.x == 0) s_block_slot = (int) block_slot;
+    __syncthreads();
+    slot += s_block_slot;
+  }
   if (!valid) return;
 
+  if (view.slot_offsets) view.slot_offsets[i] = slot;
+  if (view.visible) view.visible[i] = ok && f2i_sat(radius) > 0;
   if (trans_precomp == nullptr) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) trans_mat[9 * (size_t) i + k] = ok ? M[k] : 0.0f;
@@ -196,7 +223,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       r[1] = make_float4(M[4], M[5], M[6], M[7]);
       r[2] = make_float4(M[8], c2[0], c2[1], op);
       r[3] = make_float4(nrm[0], nrm[1], nrm[2], col[0]);
-      r[4] = make_float4(col[1], col[2], __int_as_float(f2i_sat(radius)), __int_as_float(-1));  // offset: not known yet
+      r[4] = make_float4(col[1], col[2], __int_as_float(f2i_sat(radius)), __int_as_float(view.slot_offsets ? slot : -1));  // -1: not known yet
     } else {
 #pragma unroll
       for (int k = 0; k < 5; ++k) r[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -452,11 +479,12 @@ __global__ void __launch_bounds__(256) transmat_backward_kernel(int P, int W, in
 
 using namespace fsgs;
 
-FSGS_API int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+namespace {
+int preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2c, const float* campos, const float* trans_precomp, const uint8_t* culling,
     int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* normal_opacity, float* depths,
-    int32_t* radii, int32_t* tiles_touched, float* records, uint32_t* keep_masks, void* stream) {
+    int32_t* radii, int32_t* tiles_touched, float* records, uint32_t* keep_masks, const ViewOutputs& view, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_preprocess_forward: bad sizes P=%d W=%d H=%d", P, W, H);
   FSGS_REQUIRE(((uintptr_t) records & 15) == 0, "gs_2d_preprocess_forward: records must be 16-byte aligned");
   FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_2d_preprocess_forward: sh_degree %d > %d not supported", sh_degree,
@@ -474,8 +502,31 @@ FSGS_API int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, i
                               : (wave_rows ? preprocess_forward_kernel<16, true> : preprocess_forward_kernel<16, false>);
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, opacities, shs,
                      sh_rest, Tw2v, Tv2c, campos, trans_precomp, culling, means2D_preserve, (float2*) means2D, colors,
-                     trans_mat, (float4*) normal_opacity, depths, radii, tiles_touched, (float4*) records, keep_masks);
+                     trans_mat, (float4*) normal_opacity, depths, radii, tiles_touched, (float4*) records, keep_masks, view);
   return check_launch("gs_2d_preprocess_forward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, const float* trans_precomp, const uint8_t* culling,
+    int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* normal_opacity, float* depths,
+    int32_t* radii, int32_t* tiles_touched, float* records, uint32_t* keep_masks, void* stream) {
+  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                            campos, trans_precomp, culling, means2D_preserve, means2D, colors, trans_mat, normal_opacity,
+                            depths, radii, tiles_touched, records, keep_masks, ViewOutputs{}, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
+  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
+                            tiles_touched, records, keep_masks,
+                            ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,

@@ -5,6 +5,7 @@ The product path has no CPU fallback: if the shared object is missing, loading f
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import re
 from pathlib import Path
 from typing import Dict, List, Tuple
@@ -69,6 +70,18 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def _host_layer():
+    """The native host layer (csrc/host): whole render calls, from argument checks to the autograd node, in C++."""
+    load()
+    path = PKG_DIR / "_host.so"
+    if not path.exists():
+        raise RuntimeError(f"{path} is missing: build it first (python -m fast_sp_gs_amd.build)")
+    spec = importlib.util.spec_from_file_location("fast_sp_gs_amd._host", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
 def ptr(t):
     """Device (or host) address of a tensor, NULL for None."""
     if t is None:
@@ -110,3 +123,6 @@ def require_shape(what: str, name: str, t: torch.Tensor, *shape) -> None:
 def require_dtype(what: str, name: str, t: torch.Tensor, dtype) -> None:
     if t.dtype != dtype:
         raise RuntimeError(f"{what}: {name} must have dtype {dtype}, got {t.dtype}")
+
+
+surfel_render = _host_layer().surfel_render

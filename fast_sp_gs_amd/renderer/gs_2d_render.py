@@ -1,6 +1,7 @@
 """Host side of the 2DGS surfel renderer: the autograd wiring and the PyTorch epilogue of the reference's
-`fast_2d_gs/renderer/gs_2d_render.py` (`_GS_2D_Render` :473-547, `GS_2D_render` :550-633, `depth_to_normal` :438-470),
-calling the HIP operators through the operator boundary by name, exactly as the reference's wrappers do.
+`fast_2d_gs/renderer/gs_2d_render.py` (`_GS_2D_Render` :473-547, `GS_2D_render` :550-633, `depth_to_normal` :438-470).
+`GS_2D_render` is one call into the native host layer (csrc/host/surfel.cpp); the other classes call the HIP operators
+through the operator boundary by name, as the reference's wrappers do.
 """
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
+from fast_sp_gs_amd.lib import surfel_render
 
 __all__ = ['GS_2D_render', 'RasterizeBuffer', 'GS_2D_topk_weights', 'GS_prepare', 'render_step']
 
@@ -60,6 +62,8 @@ def depth_to_normal(Tw2v: Tensor, Tv2c: Tensor, size, depth: Tensor) -> Tensor:
 
 
 class _GS_2D_Render(torch.autograd.Function):
+    """The view on the operators, one call each (the reference's class of this name, gs_2d_render.py:473-547).
+    `GS_2D_render` makes the same launches through the native host layer."""
     _preprocess_forward = get_C_function('gs_2d_preprocess_forward')
     _preprocess_backward = get_C_function('gs_2d_preprocess_backward')
     _render_forward = get_C_function('GS_2D_render_forward')
@@ -127,34 +131,6 @@ class _GS_2D_Render(torch.autograd.Function):
         return tuple(grad_inputs)
 
 
-class _GS_2D_Epilogue(torch.autograd.Function):
-    """normals to world space, nan_to_num of the depth maps, surf_depth, depth_to_normal * opacity.detach() and the
-    optional background composite (gs_2d_render.py:608-617, network.py:725-726) through the fused kernels."""
-    _forward = get_C_function('gs_2d_epilogue_forward')
-    _backward = get_C_function('gs_2d_epilogue_backward')
-
-    @staticmethod
-    def forward(ctx, extras, opacity, images, background, Tw2v, Tv2c, depth_ratio, W, H):
-        extras, opacity = extras.contiguous(), opacity.contiguous()
-        bg = None if background is None else background.detach().reshape(3).contiguous()
-        normals, depths, surf_depth, surf_normal, comp = _GS_2D_Epilogue._forward(
-            W, H, depth_ratio, Tw2v, Tv2c, extras, opacity, None if images is None else images.contiguous(), bg)
-        ctx.save_for_backward(extras, opacity, Tw2v, Tv2c, bg)
-        ctx._info = (W, H, depth_ratio)
-        ctx.set_materialize_grads(False)
-        return normals, depths, surf_depth, surf_normal, comp
-
-    @staticmethod
-    def backward(ctx, g_normals, g_depths, g_surf_depth, g_surf_normal, g_comp):
-        extras, opacity, Tw2v, Tv2c, bg = ctx.saved_tensors
-        W, H, depth_ratio = ctx._info
-        c = lambda t: None if t is None else t.contiguous()
-        g_extras, g_opacity = _GS_2D_Epilogue._backward(W, H, depth_ratio, Tw2v, Tv2c, extras, opacity, bg,
-                                                        c(g_normals), c(g_depths), c(g_surf_depth), c(g_surf_normal),
-                                                        None, c(g_comp))
-        return g_extras, g_opacity, g_comp, None, None, None, None, None, None
-
-
 def GS_2D_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity: Tensor,
                  size: Union[Tuple[int, int], Tensor], Tw2v: Tensor, Tv2c: Tensor, campos: Tensor = None,
                  focals: Tensor = None, FoV: Tensor = None, is_opengl=False, near=0.2, far=100, sh_degree=0,
@@ -165,18 +141,27 @@ def GS_2D_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity: Ten
     """Same inputs, outputs and dict keys as the reference's GS_2D_render (gs_2d_render.py:550-633). The per-pixel tail
     (:608-617) runs as one fused kernel each way. `background` ([3], optional, not in the reference's signature) also
     folds the caller's composite `images + (1 - opacity) * background` (network.py:725-726) into that kernel."""
-    means2D = points.new_zeros(points.shape[0], 2, requires_grad=True)
-    W, H = size
+    # the preprocess kernel writes every row (zeros for surfels that are not rendered)
+    means2D = torch.empty((points.shape[0], 2), dtype=torch.float32, device=points.device, requires_grad=True)
+    W, H = int(size[0]), int(size[1])
     if campos is None:
         campos = Tw2v.inverse()[:3, 3].contiguous()
-    images, opacities, out_extras, flow, n_contrib, radii, buffer = _GS_2D_Render.apply(
-        points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest,
-        Tw2v.contiguous(), Tv2c.contiguous(), campos.contiguous(), size, sh_degree if colors is None else -1,
-        is_opengl, near, far, False, None, means2D, trans_mat_t2, culling, accum_max_count, accum_weights_p,
-        accum_weights_count)
-    distortion = out_extras[5:6]
-    if Tw2v.requires_grad or Tv2c.requires_grad:
-        # camera optimisation: the fused epilogue produces no camera gradients, take the reference's torch ops
+    # camera optimisation: the fused epilogue produces no camera gradients, take the reference's torch ops
+    fused = not (Tw2v.requires_grad or Tv2c.requires_grad)
+    near, far, depth_ratio = float(near), float(far), float(depth_ratio)
+    maps, n_contrib, radii, visible, tile_range, point_list, normal_opacity, trans_mat = surfel_render(
+        points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest, means2D,
+        Tw2v.contiguous(), Tv2c.contiguous(), campos.contiguous(),
+        background.detach().reshape(3).contiguous() if fused and background is not None else None, trans_mat_t2, culling,
+        accum_max_count, accum_weights_p, accum_weights_count, W, H, int(sh_degree) if colors is None else -1, near, far,
+        depth_ratio, fused, bool(CULL_LISTS))
+    buffer = RasterizeBuffer(W, H, points.shape[0], point_list.shape[0], near, far, tile_range, point_list, n_contrib,
+                             means2D, normal_opacity, trans_mat)
+    if fused:
+        images, opacities, normals, median_depths, surf_depth, surf_normal, distortion, *flow = maps
+    else:
+        images, opacities, out_extras, *flow = maps
+        distortion = out_extras[5:6]
         if background is not None:
             images = images + (1.0 - opacities) * background.view(3, 1, 1)
         depths, normals, median_depths, _, _ = out_extras.split([1, 3, 1, 1, 3], dim=0)
@@ -186,19 +171,13 @@ def GS_2D_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity: Ten
         surf_depth = depths * (1 - depth_ratio) + depth_ratio * median_depths
         surf_normal = depth_to_normal(Tw2v, Tv2c, (W, H), surf_depth).permute(2, 0, 1)
         surf_normal = surf_normal * opacities.detach()
-    else:
-        normals, median_depths, surf_depth, surf_normal, composited = _GS_2D_Epilogue.apply(
-            out_extras, opacities, images if background is not None else None, background, Tw2v.contiguous(),
-            Tv2c.contiguous(), float(depth_ratio), W, H)
-        if background is not None:
-            images = composited
     outputs = {
         'images': images, 'depths': median_depths, 'normals': normals, 'opacity': opacities,
         'distortion': distortion, 'surf_depth': surf_depth, 'surf_normal': surf_normal, 'radii': radii,
-        'viewspace_points': means2D, 'visibility_filter': radii > 0, 'buffer': buffer,
+        'viewspace_points': means2D, 'visibility_filter': visible, 'buffer': buffer,
     }
-    if flow is not None:
-        outputs['flow'] = flow
+    if flow:
+        outputs['flow'] = flow[0]
     return outputs
 
 

@@ -49,6 +49,16 @@ int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, 
     int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* normal_opacity, float* depths,
     int32_t* radii, int32_t* tiles_touched, float* records, uint32_t* keep_masks, void* stream);
 
+/* A whole view without a prefix scan (no counterpart in the reference): the preprocess hands out the gradient records'
+ * slots itself. slot_counters[64] are zero before the call and again after fsgs_gs_view_count; a surfel's slots start at
+ * slot_offsets[i] + slot_regions[(i / 256) % 64] and are tiles_touched[i] many. visible[P] (0 / 1), slot_offsets, records
+ * and keep_masks are optional. Every row of the outputs is written. */
+int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
+    const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
+    float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream);
+
 /* gs_2d_preprocess_backward -- gs_2d_preprocess.cu:423-499 (kernel :268-329). Every row of g_* is ASSIGNED: the
  * gradient for surfels with radii > 0, zeros for the others and for SH coefficients above the active degree (the
  * reference relies on its caller's zero-fill for those), so the outputs need no initialisation. grad_mean2D[P,2] is
@@ -130,6 +140,15 @@ int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const float* means2
                                         int32_t* point_list, int64_t* sorted_keys_out, void* bins, size_t bins_bytes,
                                         void* workspace, size_t workspace_bytes, void* stream);
 
+/* The counting part of the binning (as fsgs_gs_prepare_count, or _culled with keep_masks) for a view preprocessed by
+ * fsgs_gs_*_view_preprocess; P > 0. Its first block writes slot_regions[64] (optional), zeroes slot_counters and stores
+ * the instance count to num_rendered_host (pinned memory, set to -1 here); fsgs_gs_view_wait returns once it is there.
+ * fsgs_gs_prepare_fill_counted(_culled) follows. */
+int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii, const uint32_t* keep_masks,
+                       uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges,
+                       void* bins, size_t bins_bytes, void* stream);
+int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream);
+
 /* ---- per-tile alpha blend ------------------------------------------------------------------------------------- */
 
 /* Optional accelerator without a counterpart in the reference: packs what the blend kernels gather per surfel
@@ -181,6 +200,16 @@ int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_n, double
     const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
     float* g_normal_opacity, int64_t R, const int64_t* point_offsets, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const float* records, const uint32_t* keep_masks, void* stream);
+
+/* The same with the record slots of fsgs_gs_2d_view_preprocess; keep_masks nullptr for full lists. */
+int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
+    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
+    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
+    const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
+    float* g_normal_opacity, int64_t R, const int32_t* slot_offsets, const int32_t* slot_regions,
+    const int32_t* tiles_touched, const int32_t* radii, void* workspace, size_t workspace_bytes, const float* records,
+    const uint32_t* keep_masks, void* stream);
 
 /* ---- "fast" surfel path: transform through camera intrinsics Tv2s[3,3], adjugate-based intersection, fused
  * corner-test binning. Optical flow (trans_mat_t2) is carried by the two blend entry points below. ---- */
@@ -555,6 +584,11 @@ int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, const float* 
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
     float* g_extras, float* g_opacity, void* stream);
+/* The same, with the gradient the opacity map has from elsewhere added into g_opacity (g_opacity_in[H,W], optional). */
+int fsgs_gs_2d_view_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
+    const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
+    const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
+    const float* g_opacity_in, float* g_extras, float* g_opacity, void* stream);
 
 /* simple_knn -- fast_2d_gs/_C/src/other/knn.cu:180-205 (kernels :57-178). points[P,3] -> mean_dist2[P]: the mean of
  * the three smallest squared distances from each point to the other points (exact search; with fewer than four

@@ -1,0 +1,106 @@
+"""Views through the native host layer (one C++ call and one autograd node per render, record slots handed out by regions
+of 256-surfel blocks instead of a prefix scan) against the same view on the operators: equal maps, equal gradients.
+Sizes: one, around a block, around one turn of the 64 regions (16 384 surfels), ragged images."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(P, W, H, seed, scale=-4.2):
+    from fast_sp_gs_amd import scenes
+    g = torch.Generator().manual_seed(seed)
+    s = scenes._surfels(g, P, 'cube', scale, 0.7, 0.0, 1.5)
+    return s, scenes.pinhole(W, H, 50.0, torch.tensor([0.3, 0.2, 4.0])), g
+
+
+def _leaves(device, *tensors):
+    return [t.to(device).requires_grad_(True) for t in tensors]
+
+
+@pytest.mark.parametrize('P,W,H,mode', [(1, 16, 16, 'sh'), (255, 49, 31, 'split'), (256, 49, 31, 'colors'),
+                                        (257, 64, 48, 'culling'), (16_384, 161, 99, 'sh'), (16_385, 161, 99, 'flow'),
+                                        (40_000, 250, 130, 'accum')])
+def test_surfel_view_equals_operators(P, W, H, mode, device):
+    from fast_sp_gs_amd.renderer import gs_2d_render as m
+    s, cam_h, g = _scene(P, W, H, P + 1)
+    cam = cam_h.to(device)
+    params = _leaves(device, s.means3D, s.scales, s.rotations, s.opacities)
+    rest = None
+    if mode == 'split':
+        sh, rest = _leaves(device, s.shs[:, :1].contiguous(), s.shs[:, 1:].contiguous())
+    elif mode == 'colors':
+        sh, = _leaves(device, s.shs[:, 0].contiguous())
+    else:
+        sh, = _leaves(device, s.shs)
+    culling = (torch.rand(P, generator=g) < 0.3).to(device) if mode == 'culling' else None
+    t2 = torch.randn(P, 3, 3, generator=g).to(device) if mode == 'flow' else None
+    accum = lambda: ([torch.zeros(P, dtype=torch.int32, device=device), torch.zeros(P, device=device),
+                      torch.zeros(P, dtype=torch.int32, device=device)] if mode == 'accum' else [None] * 3)
+    a1, a2 = accum(), accum()
+    out = m.GS_2D_render(*params, (W, H), cam.Tw2v, cam.Tv2c, campos=cam.campos, sh_degree=3, near=0.2, far=100.0,
+                         colors=sh if mode == 'colors' else None, sh_features=None if mode == 'colors' else sh,
+                         sh_features_rest=rest, culling=culling, trans_mat_t2=t2, accum_max_count=a1[0],
+                         accum_weights_p=a1[1], accum_weights_count=a1[2])
+    m2 = torch.zeros(P, 2, device=device, requires_grad=True)
+    img, opac, extras, flow, n_contrib, radii, buf = m._GS_2D_Render.apply(
+        *params, sh, rest, cam.Tw2v, cam.Tv2c, cam.campos, (W, H), -1 if mode == 'colors' else 3, False, 0.2, 100.0, False,
+        None, m2, t2, culling, *a2)
+    same = lambda a, b: a.shape == b.shape and torch.equal(a, b)
+    assert same(out['images'], img) and same(out['opacity'], opac) and same(out['distortion'], extras[5:6])
+    assert same(out['radii'], radii) and same(out['visibility_filter'], radii > 0)
+    assert same(out['depths'], torch.nan_to_num(extras[4:5], 0, 0))
+    assert same(out['viewspace_points'], m2) and same(out['buffer'].n_contribed, n_contrib)
+    assert same(out['buffer'].tile_ranges, buf.tile_ranges) and out['buffer'].R == buf.R
+    used = int((buf.tile_ranges[:, 1] - buf.tile_ranges[:, 0]).sum())
+    assert torch.equal(out['buffer'].point_list[:used], buf.point_list[:used])
+    for x, y in zip(a1[::2], a2[::2]):
+        assert x is None or torch.equal(x, y)
+    g_img, g_op, g_dist = (torch.randn(t.shape, generator=g).to(device) for t in (img, opac, extras[5:6]))
+    wrt = params + [sh] + ([rest] if rest is not None else [])
+    maps, ups = [out['images'], out['opacity'], out['distortion']], [g_img, g_op, g_dist]
+    o_maps = [img, opac, extras[5:6]]
+    if mode == 'flow':
+        assert same(out['flow'], flow)
+        g_flow = torch.randn(flow.shape, generator=g).to(device) * (flow.abs() < 1e3)
+        maps, o_maps, ups = maps + [out['flow']], o_maps + [flow], ups + [g_flow]
+    got = torch.autograd.grad(maps, wrt + [out['viewspace_points']], ups, allow_unused=True)
+    want = torch.autograd.grad(o_maps, wrt + [m2], ups, allow_unused=True)
+    for x, y in zip(got, want):
+        assert (x is None) == (y is None) and (x is None or torch.equal(torch.nan_to_num(x), torch.nan_to_num(y)))
+
+
+def test_surfel_views_on_two_streams_and_threads(device):
+    """Views of two host threads on two streams at once give what they give alone (counters are per stream and call)."""
+    import threading
+
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    jobs = []
+    for k, P in enumerate((3_000, 9_000)):
+        s, cam_h, _ = _scene(P, 200, 120, k)
+        jobs.append((s.to(device), cam_h.to(device)))
+
+    def view(job):
+        s, cam = job
+        with torch.no_grad():
+            return GS_2D_render(s.means3D, s.scales, s.rotations, s.opacities, (cam.W, cam.H), cam.Tw2v, cam.Tv2c,
+                                campos=cam.campos, sh_degree=3, sh_features=s.shs)['images']
+
+    want = [view(j) for j in jobs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def loop(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                if not torch.equal(view(jobs[k]), want[k]):
+                    bad.append(k)
+            torch.cuda.current_stream().synchronize()
+
+    threads = [threading.Thread(target=loop, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
