@@ -134,56 +134,7 @@ static_assert(kCoopThreshold == kCullMaskTiles, "a lane's serial walk covers exa
 // Empty tiles get (0, 0) as the reference's zero-initialised ranges have. Tile grids above kMaxLdsTiles tiles (no room
 // for one LDS counter per tile) count and scatter with 64-bit global atomics on ranges[t].y instead (tile_emit_kernel).
 
-// Visits every (surfel, tile) pair; kScatter = false counts, true scatters. `masks` (optional): a surfel's keep mask,
-// the cleared bits of a rectangle of at most kCoopThreshold tiles are passed over.
-template <bool kScatter>
-__global__ void __launch_bounds__(256) tile_emit_kernel(int P, int gx, int gy, int64_t R,
-    const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
-    const uint32_t* __restrict__ masks, unsigned long long* __restrict__ ranges, uint64_t* __restrict__ entries) {
-  const int i    = blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = __lane_id();
-  int x0 = 0, y0 = 0, w = 0, h = 0;
-  uint32_t dbits = 0;
-  if (i < P && radii[i] > 0) {
-    const float2 c   = means2D[i];
-    const TileRect r = tile_rect(c.x, c.y, radii[i], gx, gy);
-    x0 = r.x0, y0 = r.y0, w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
-    if (kScatter) dbits = __float_as_uint(depths[i]);
-  }
-  auto visit = [&](int tile, uint32_t bits, int id) {
-    unsigned long long* slot = ranges + 2 * (size_t) tile + 1;
-    if (kScatter) {
-      const unsigned long long pos = atomicAdd(slot, 1ull);
-      if ((int64_t) pos < R) entries[pos] = ((uint64_t) bits << 32) | (uint32_t) id;
-    } else {
-      atomicAdd(slot, 1ull);
-    }
-  };
-  const int count = w * h;
-  if (count > 0 && count <= kCoopThreshold) {
-    uint32_t keep = masks ? masks[i] : 0xffffffffu;
-    for (int y = 0; y < h; ++y)
-      for (int x = 0; x < w; ++x, keep >>= 1)
-        if (keep & 1u) visit((y0 + y) * gx + (x0 + x), dbits, i);
-  }
-  unsigned long long big = __ballot(count > kCoopThreshold);
-  while (big) {
-    const int src = __ffsll((long long) big) - 1;
-    big &= big - 1;
-    const int sx0 = __shfl(x0, src, kWave), sy0 = __shfl(y0, src, kWave), sw = __shfl(w, src, kWave);
-    const int scount = __shfl(count, src, kWave), sid = __shfl(i, src, kWave);
-    const uint32_t sbits = __shfl(dbits, src, kWave);
-    for (int e = lane; e < scount; e += kWave) {
-      const int y = e / sw, x = e - y * sw;
-      visit((sy0 + y) * gx + (sx0 + x), sbits, sid);
-    }
-  }
-}
-
-// The same traversal with the counters in LDS, one per tile (tile grids up to kMaxLdsTiles tiles): blocks of 1024 lanes
-// walk a slice of the surfels each; what they do with an instance is up to the caller (tile_hist_kernel,
-// tile_scatter_kernel).
-constexpr int kMaxLdsTiles = 16384;
+constexpr int kMaxLdsTiles = 16384;  // one counter per tile in LDS
 
 // Which tiles of a surfel's rectangle are visited: all of them (the reference's lists), those that pass the fast path's
 // corner test (CornerTest, from the surfel's adjugate and opacity), or those whose bit is set in the surfel's keep mask
@@ -200,7 +151,14 @@ struct WalkInputs {
   const float* inverse_m;
   const float* opacities;
   const uint32_t* keep_masks;
+
+  WalkMode mode() const {
+    if (inverse_m) return keep_masks ? kWalkCornerMask : kWalkCorner;
+    return keep_masks ? kWalkMask : kWalkAll;
+  }
 };
+
+// Visits the kept (surfel, tile) pairs of surfel i (P: none); all lanes of a wavefront call it together.
 
 template <int kMode, typename Visit>
 __device__ __forceinline__ void for_each_instance(int i, int P, int gx, int gy, const float2* __restrict__ means2D,
@@ -256,6 +214,17 @@ __device__ __forceinline__ void for_each_instance(int i, int P, int gx, int gy, 
       if (!kCorner || ct.tile(sx0 + x, sy0 + y)) visit((sy0 + y) * gx + (sx0 + x), sid);
     }
   }
+}
+
+// Counting (kScatter = false) and scattering with global atomics, for tile grids beyond kMaxLdsTiles.
+template <int kMode, bool kScatter>
+__global__ void __launch_bounds__(256) tile_emit_kernel(int P, int gx, int gy, int64_t R,
+    const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
+    WalkInputs in, unsigned long long* __restrict__ ranges, uint64_t* __restrict__ entries) {
+  for_each_instance<kMode>(blockIdx.x * blockDim.x + threadIdx.x, P, gx, gy, means2D, radii, in, [&](int tile, int id) {
+    const unsigned long long pos = atomicAdd(ranges + 2 * (size_t) tile + 1, 1ull);
+    if (kScatter && (int64_t) pos < R) entries[pos] = ((uint64_t) __float_as_uint(depths[id]) << 32) | (uint32_t) id;
+  });
 }
 
 // One lane per 3D Gaussian: the keep mask of its rectangle from its projected mean, conic and opacity.
@@ -895,47 +864,92 @@ size_t fast_bucket_bins_bytes(int P, int W, int H) {
   return bl.blocks > 0 ? bl.bytes : 0;
 }
 
-int fast_bucket_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
-                     const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R,
-                     int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace, void* bins,
-                     hipStream_t s) {
+namespace {
+#define FSGS_BY_WALK_MODE(IN, CALL)                                     \
+  do {                                                                  \
+    switch ((IN).mode()) {                                              \
+      case kWalkAll: { constexpr int kMode = kWalkAll; CALL; break; }   \
+      case kWalkCorner: { constexpr int kMode = kWalkCorner; CALL; break; } \
+      case kWalkMask: { constexpr int kMode = kWalkMask; CALL; break; } \
+      case kWalkCornerMask: { constexpr int kMode = kWalkCornerMask; CALL; break; } \
+    }                                                                   \
+  } while (0)
+
+// First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
+// (start, end); the header of `bins` is set (length of the long-segment queue: 0 | instances in all tiles).
+int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in, int64_t* ranges,
+               void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
-  const BinsLayout bl = bins_layout(P, T);
   unsigned long long* rng = (unsigned long long*) ranges;
-  int* header      = (int*) bins;  // [0] length of the long-segment queue, [1] instances kept by the corner test
-  uint32_t* hist   = (uint32_t*) ((char*) bins + kBinsHeader);
-  uint64_t* entries = sort_keys_in(R, workspace);
-  int* large_list   = (int*) ((char*) workspace + sort_layout(R).keys1);
-  const WalkInputs in{inverse_m, opacities, keep_masks};
-  if (keep_masks)
-    hipLaunchKernelGGL(tile_hist_kernel<kWalkCornerMask>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                       (const float2*) means2D, radii, in, hist, SlotPublish{});
-  else
-    hipLaunchKernelGGL(tile_hist_kernel<kWalkCorner>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                       (const float2*) means2D, radii, in, hist, SlotPublish{});
-  hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
-                     bl.blocks, hist, rng);
-  hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
-  // the schedule the blend kernels of this view find under `ranges`, built by an extra block of the scatter
+  int* header = (int*) bins;
+  const BinsLayout bl = bins_layout(P, T);
+  if (bl.blocks > 0) {
+    uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
+    FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_hist_kernel<kMode>), dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block,
+                                             gx, gy, (const float2*) means2D, radii, in, hist, publish));
+    hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
+                       bl.blocks, hist, rng);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
+    // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
+    // sorts) is built from them by an extra block of the scatter, in the second part.
+  } else {
+    // no room for one LDS counter per tile (or no surfels): count straight into ranges[t].y, then scan to (start, start)
+    if (publish.counters) hipLaunchKernelGGL(publish_slots_kernel, dim3(1), dim3(kWave), 0, s, publish);
+    launch_zero_ranges(T, ranges, s);
+    if (P > 0)
+      FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, false>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx,
+                                               gy, (int64_t) 0, (const float2*) means2D, (const float*) nullptr, radii, in,
+                                               rng, (uint64_t*) nullptr));
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, false);
+  }
+  return check_launch("gs_prepare_count");
+}
+
+// Second part: scatter (depth bits << 32 | surfel) into the tile segments and sort every segment. pad: the list positions
+// behind the kept instances get the fast path's padding entries.
+int fill_sort(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
+              int64_t R, int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace, void* bins,
+              bool pad, hipStream_t s) {
+  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
+  const int T  = gx * gy;
+  unsigned long long* rng = (unsigned long long*) ranges;
+  int* header             = (int*) bins;
+  uint64_t* entries       = sort_keys_in(R, workspace);
+  // queue of long segments: at most R / kSmallSegment tiles, kept behind the entries in the workspace
+  int* large_list = (int*) ((char*) workspace + sort_layout(R).keys1);
+  const BinsLayout bl = bins_layout(P, T);
+  // The schedule table: built by one extra block of the scatter (the ranges are final since the counting part), or by a
+  // launch of its own on the global-atomic path, whose ranges only become final with the scatter.
   const int* order = nullptr;
-  int* build       = nullptr;
-  (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
-  if (keep_masks)
-    hipLaunchKernelGGL(tile_scatter_kernel<kWalkCornerMask>, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), 0, s, P,
-                       bl.per_block, gx, gy, R, (const float2*) means2D, depths, radii, in, (const uint32_t*) hist, rng,
-                       entries, build);
-  else
-    hipLaunchKernelGGL(tile_scatter_kernel<kWalkCorner>, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), 0, s, P,
-                       bl.per_block, gx, gy, R, (const float2*) means2D, depths, radii, in, (const uint32_t*) hist, rng,
-                       entries, build);
-  // 256 blocks more than tiles: they write the padding entries behind the kept instances
-  hipLaunchKernelGGL(tile_sort_small_kernel, dim3(T + 256), dim3(256), 0, s, ranges, entries, point_list,
+  if (bl.blocks > 0) {
+    int* build = nullptr;
+    (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
+    FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_scatter_kernel<kMode>), dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), 0, s,
+                                             P, bl.per_block, gx, gy, R, (const float2*) means2D, depths, radii, in,
+                                             (const uint32_t*) ((const char*) bins + kBinsHeader), rng, entries, build));
+  } else {
+    FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, true>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy,
+                                             R, (const float2*) means2D, depths, radii, in, rng, entries));
+    (void) launch_tile_order(gx, gy, ranges, s, &order);
+  }
+  // with padding, 256 blocks more than tiles: they write the entries behind the kept instances
+  hipLaunchKernelGGL(tile_sort_small_kernel, dim3(T + (pad ? 256 : 0)), dim3(256), 0, s, ranges, entries, point_list,
                      sorted_keys_out, header, large_list, order, T, R, (const int*) (header + 1),
                      (uint64_t) (uint32_t) T << 32);
   hipLaunchKernelGGL(tile_sort_large_kernel, dim3(256), dim3(1024), 0, s, ranges, entries, point_list, sorted_keys_out,
                      header, large_list);
-  return check_launch("gs_2d_fast_prepare_fill");
+  return check_launch("gs_prepare_fill");
+}
+}  // namespace
+
+int fast_bucket_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                     const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R,
+                     int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace, void* bins,
+                     hipStream_t s) {
+  const WalkInputs in{inverse_m, opacities, keep_masks};
+  if (int rc = fill_count(P, W, H, means2D, radii, in, ranges, bins, s)) return rc;
+  return fill_sort(P, W, H, means2D, depths, radii, in, R, ranges, point_list, sorted_keys_out, workspace, bins, true, s);
 }
 
 }  // namespace fsgs
@@ -1011,83 +1025,6 @@ FSGS_API int fsgs_gs_prepare_sort_bits(int W, int H) {
   return 32 + (int) higher_msb((uint32_t) (gx * gy));
 }
 
-namespace {
-// First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
-// (start, end); the long-segment queue's counter (first word of `bins`) is reset.
-// keep_masks (optional): the per-surfel keep masks of cull_mask_kernel; with them an instance is only counted (and
-// later scattered) when its bit is set.
-int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const uint32_t* keep_masks,
-               int64_t* ranges, void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
-  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
-  const int T  = gx * gy;
-  unsigned long long* rng = (unsigned long long*) ranges;
-  int* header = (int*) bins;
-  const BinsLayout bl = bins_layout(P, T);
-  if (bl.blocks > 0) {
-    uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
-    if (keep_masks)
-      hipLaunchKernelGGL(tile_hist_kernel<kWalkMask>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, keep_masks}, hist, publish);
-    else
-      hipLaunchKernelGGL(tile_hist_kernel<kWalkAll>, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy,
-                         (const float2*) means2D, radii, WalkInputs{nullptr, nullptr, nullptr}, hist, publish);
-    hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
-                       bl.blocks, hist, rng);
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
-    // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
-    // sorts) is built from them by an extra block of the scatter, in the second part.
-  } else {
-    // no room for one LDS counter per tile (or no surfels): count straight into ranges[t].y, then scan to (start, start)
-    if (publish.counters) hipLaunchKernelGGL(publish_slots_kernel, dim3(1), dim3(kWave), 0, s, publish);
-    hipLaunchKernelGGL(fill_zero_i64_kernel, dim3(div_up(2 * (int64_t) T, 256)), dim3(256), 0, s, 2 * (int64_t) T,
-                       ranges);
-    if (P > 0)
-      hipLaunchKernelGGL(tile_emit_kernel<false>, dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy, (int64_t) 0,
-                         (const float2*) means2D, (const float*) nullptr, radii, keep_masks, rng, (uint64_t*) nullptr);
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, false);
-  }
-  return check_launch("gs_prepare_count");
-}
-
-// Second part: scatter (depth bits << 32 | surfel) into the tile segments and sort every segment.
-int fill_sort(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii,
-              const uint32_t* keep_masks, int64_t R, int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out,
-              void* workspace, void* bins, hipStream_t s) {
-  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
-  const int T  = gx * gy;
-  unsigned long long* rng = (unsigned long long*) ranges;
-  uint64_t* entries       = sort_keys_in(R, workspace);
-  int* large_count        = (int*) bins;
-  // queue of long segments: at most R / kSmallSegment tiles, kept behind the entries in the workspace
-  int* large_list = (int*) ((char*) workspace + sort_layout(R).keys1);
-  const BinsLayout bl = bins_layout(P, T);
-  // The schedule table: built by one extra block of the scatter (the ranges are final since the counting part), or by a
-  // launch of its own on the global-atomic path, whose ranges only become final with the scatter.
-  const int* order = nullptr;
-  int* build       = nullptr;
-  if (bl.blocks > 0) (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
-  const dim3 scatter_grid(bl.blocks + (build ? 1 : 0));
-  if (bl.blocks > 0 && keep_masks)
-    hipLaunchKernelGGL(tile_scatter_kernel<kWalkMask>, scatter_grid, dim3(1024), 0, s, P, bl.per_block, gx, gy, R,
-                       (const float2*) means2D, depths, radii, WalkInputs{nullptr, nullptr, keep_masks},
-                       (const uint32_t*) ((const char*) bins + kBinsHeader), rng, entries, build);
-  else if (bl.blocks > 0)
-    hipLaunchKernelGGL(tile_scatter_kernel<kWalkAll>, scatter_grid, dim3(1024), 0, s, P, bl.per_block, gx, gy, R,
-                       (const float2*) means2D, depths, radii, WalkInputs{nullptr, nullptr, nullptr},
-                       (const uint32_t*) ((const char*) bins + kBinsHeader), rng, entries, build);
-  else {
-    hipLaunchKernelGGL(tile_emit_kernel<true>, dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy, R,
-                       (const float2*) means2D, depths, radii, keep_masks, rng, entries);
-    (void) launch_tile_order(gx, gy, ranges, s, &order);
-  }
-  hipLaunchKernelGGL(tile_sort_small_kernel, dim3(T), dim3(256), 0, s, ranges, entries, point_list, sorted_keys_out,
-                     large_count, large_list, order, T, (int64_t) 0, (const int*) nullptr, (uint64_t) 0);
-  hipLaunchKernelGGL(tile_sort_large_kernel, dim3(256), dim3(1024), 0, s, ranges, entries, point_list, sorted_keys_out,
-                     large_count, large_list);
-  return check_launch("gs_prepare_fill");
-}
-}  // namespace
-
 FSGS_API size_t fsgs_gs_prepare_bins_bytes(int P, int W, int H) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   return bins_layout(P, gx * gy).bytes;
@@ -1101,7 +1038,7 @@ FSGS_API int fsgs_gs_prepare_count(int P, int W, int H, const float* means2D, co
     return fail(kWorkspaceSmall, "gs_prepare_count: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
   tile_order_invalidate((hipStream_t) stream);  // the ranges are rewritten: the blend schedule of this stream is stale
-  return fill_count(P, W, H, means2D, radii, nullptr, ranges, bins, (hipStream_t) stream);
+  return fill_count(P, W, H, means2D, radii, WalkInputs{}, ranges, bins, (hipStream_t) stream);
 }
 
 FSGS_API int fsgs_gs_prepare_fill_counted(int P, int W, int H, const float* means2D, const float* depths,
@@ -1118,8 +1055,8 @@ FSGS_API int fsgs_gs_prepare_fill_counted(int P, int W, int H, const float* mean
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_prepare_fill: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, nullptr, R, ranges, point_list, sorted_keys_out, workspace, bins,
-                   (hipStream_t) stream);
+  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
+                   false, (hipStream_t) stream);
 }
 
 // Keep masks for the culled binning: a bit per tile of a surfel's rectangle (row-major, rectangles of at most 32 tiles;
@@ -1162,7 +1099,7 @@ FSGS_API int fsgs_gs_prepare_count_culled(int P, int W, int H, const float* mean
     return fail(kWorkspaceSmall, "gs_prepare_count_culled: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
   tile_order_invalidate((hipStream_t) stream);
-  return fill_count(P, W, H, means2D, radii, culling_enabled() ? masks : nullptr, ranges, bins,
+  return fill_count(P, W, H, means2D, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? masks : nullptr}, ranges, bins,
                     (hipStream_t) stream);
 }
 
@@ -1181,23 +1118,58 @@ FSGS_API int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const floa
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_prepare_fill_culled: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, culling_enabled() ? masks : nullptr, R, ranges,
-                   point_list, sorted_keys_out, workspace, bins, (hipStream_t) stream);
+  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? masks : nullptr}, R,
+                   ranges, point_list, sorted_keys_out, workspace, bins, false, (hipStream_t) stream);
 }
 
 // The counting part for views whose preprocess handed out the record slots (instance_slots.hpp).
-FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii,
-                                const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
-                                int64_t* num_rendered_host, int64_t* ranges, void* bins, size_t bins_bytes,
-                                void* stream) {
+namespace {
+int view_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in,
+               uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges, void* bins,
+               size_t bins_bytes, void* stream) {
   FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins, "gs_view_count: bad arguments");
   FSGS_REQUIRE(means2D && radii && slot_counters && num_rendered_host, "gs_view_count: null pointer");
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_view_count: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
   tile_order_invalidate((hipStream_t) stream);
   __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
-  return fill_count(P, W, H, means2D, radii, culling_enabled() ? keep_masks : nullptr, ranges, bins,
-                    (hipStream_t) stream, SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
+  return fill_count(P, W, H, means2D, radii, in, ranges, bins, (hipStream_t) stream,
+                    SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii,
+                                const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
+                                int64_t* num_rendered_host, int64_t* ranges, void* bins, size_t bins_bytes,
+                                void* stream) {
+  return view_count(P, W, H, means2D, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? keep_masks : nullptr},
+                    slot_counters, slot_regions, num_rendered_host, ranges, bins, bins_bytes, stream);
+}
+
+FSGS_API int fsgs_gs_2d_fast_view_count(int P, int W, int H, const float* means2D, const float* inverse_m,
+                                        const float* opacities, const int32_t* radii, const uint32_t* keep_masks,
+                                        uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host,
+                                        int64_t* ranges, void* bins, size_t bins_bytes, void* stream) {
+  FSGS_REQUIRE(inverse_m && opacities && keep_masks, "gs_2d_fast_view_count: null pointer");
+  return view_count(P, W, H, means2D, radii, WalkInputs{inverse_m, opacities, keep_masks}, slot_counters, slot_regions,
+                    num_rendered_host, ranges, bins, bins_bytes, stream);
+}
+
+FSGS_API int fsgs_gs_2d_fast_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m,
+                                       const float* depths, const float* opacities, const int32_t* radii,
+                                       const uint32_t* keep_masks, int64_t R, int64_t* ranges, int32_t* point_list,
+                                       void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && R >= 0 && ranges && bins, "gs_2d_fast_view_fill: bad arguments");
+  FSGS_REQUIRE(R < (int64_t) 0x7fffffff, "gs_2d_fast_view_fill: %lld instances exceed the 2^31-1 limit", (long long) R);
+  if (R == 0) return kOk;
+  FSGS_REQUIRE(means2D && inverse_m && depths && opacities && radii && keep_masks && point_list && workspace,
+               "gs_2d_fast_view_fill: null pointer");
+  if (workspace_bytes < sort_workspace_bytes(R) || bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
+    return fail(kWorkspaceSmall, "gs_2d_fast_view_fill: workspace %zu < %zu or bins %zu < %zu bytes", workspace_bytes,
+                sort_workspace_bytes(R), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{inverse_m, opacities, keep_masks}, R, ranges, point_list,
+                   nullptr, workspace, bins, false, (hipStream_t) stream);
 }
 
 // Waits until the count has been written. Reading the word is all it takes as long as the stream works; a stream that
@@ -1238,6 +1210,7 @@ FSGS_API int fsgs_gs_prepare_fill(int P, int W, int H, const float* means2D, con
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_prepare_fill: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
-  if (int rc = fill_count(P, W, H, means2D, radii, nullptr, ranges, bins, s)) return rc;
-  return fill_sort(P, W, H, means2D, depths, radii, nullptr, R, ranges, point_list, sorted_keys_out, workspace, bins, s);
+  if (int rc = fill_count(P, W, H, means2D, radii, WalkInputs{}, ranges, bins, s)) return rc;
+  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
+                   false, s);
 }

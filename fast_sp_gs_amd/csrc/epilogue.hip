@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(256) epilogue_forward_kernel(int W, int H, flo
   const float n0 = extras[HW + p], n1 = extras[2 * HW + p], n2 = extras[3 * HW + p];
 #pragma unroll
   for (int j = 0; j < 3; ++j) normals[j * HW + p] = n0 * Tw2v[j] + n1 * Tw2v[4 + j] + n2 * Tw2v[8 + j];
-  depths[p]     = nan0(maps.median[p]);
+  if (depths) depths[p] = nan0(maps.median[p]);
   surf_depth[p] = maps.surf(x, y);
   Vec3 n = {0.0f, 0.0f, 0.0f};
   if (x >= 1 && y >= 1 && x <= W - 2 && y <= H - 2) {
@@ -150,7 +150,7 @@ __device__ __forceinline__ void normal_backward(const PixelRays& r, const DepthM
   gb = cross3(gc, a);
 }
 
-__global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, float ratio,
+__global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, int channels, float ratio,
     const float* __restrict__ Tw2v, const float* __restrict__ Tv2c, const float* __restrict__ extras,
     const float* __restrict__ opacity, const float* __restrict__ background, const float* __restrict__ g_normals,
     const float* __restrict__ g_depths, const float* __restrict__ g_surf_depth,
@@ -202,8 +202,7 @@ __global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, fl
 #pragma unroll
   for (int i = 0; i < 3; ++i) g_extras[(1 + i) * HW + p] = gn[i];
   g_extras[5 * HW + p] = g_distortion ? g_distortion[p] : 0.0f;
-#pragma unroll
-  for (int c = 6; c < 9; ++c) g_extras[c * HW + p] = 0.0f;
+  for (int c = 6; c < channels; ++c) g_extras[c * HW + p] = 0.0f;
   if (g_opacity) {
     float s = 0.0f;
     if (g_composited)
@@ -223,7 +222,7 @@ FSGS_API int fsgs_gs_2d_epilogue_forward(int W, int H, double depth_ratio, const
     float* depths, float* surf_depth, float* surf_normal, float* composited, void* stream) {
   FSGS_REQUIRE(W >= 0 && H >= 0, "gs_2d_epilogue_forward: bad size");
   if ((size_t) W * H == 0) return kOk;
-  FSGS_REQUIRE(Tw2v && Tv2c && extras && opacity && normals && depths && surf_depth && surf_normal,
+  FSGS_REQUIRE(Tw2v && Tv2c && extras && opacity && normals && surf_depth && surf_normal,
                "gs_2d_epilogue_forward: null pointer");
   FSGS_REQUIRE(!composited || (images && background), "gs_2d_epilogue_forward: composite needs images and background");
   const dim3 grid(div_up(W, 32), div_up(H, 8)), block(32, 8);
@@ -232,17 +231,17 @@ FSGS_API int fsgs_gs_2d_epilogue_forward(int W, int H, double depth_ratio, const
   return check_launch("gs_2d_epilogue_forward");
 }
 
-FSGS_API int fsgs_gs_2d_view_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
+FSGS_API int fsgs_gs_2d_view_epilogue_backward(int W, int H, int channels, double depth_ratio, const float* Tw2v, const float* Tv2c,
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
     const float* g_opacity_in, float* g_extras, float* g_opacity, void* stream) {
-  FSGS_REQUIRE(W >= 0 && H >= 0, "gs_2d_epilogue_backward: bad size");
+  FSGS_REQUIRE(W >= 0 && H >= 0 && channels >= 6, "gs_2d_epilogue_backward: bad size");
   if ((size_t) W * H == 0) return kOk;
   FSGS_REQUIRE(Tw2v && Tv2c && extras && opacity && g_extras, "gs_2d_epilogue_backward: null pointer");
   FSGS_REQUIRE(!g_composited || (background && g_opacity),
                "gs_2d_epilogue_backward: the composite gradient needs the background and g_opacity");
   const dim3 grid(div_up(W, 32), div_up(H, 8)), block(32, 8);
-  hipLaunchKernelGGL(epilogue_backward_kernel, grid, block, 0, (hipStream_t) stream, W, H, (float) depth_ratio, Tw2v,
+  hipLaunchKernelGGL(epilogue_backward_kernel, grid, block, 0, (hipStream_t) stream, W, H, channels, (float) depth_ratio, Tw2v,
                      Tv2c, extras, opacity, background, g_normals, g_depths, g_surf_depth, g_surf_normal, g_distortion,
                      g_composited, g_opacity_in, g_extras, g_opacity);
   return check_launch("gs_2d_epilogue_backward");
@@ -252,7 +251,7 @@ FSGS_API int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, cons
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
     float* g_extras, float* g_opacity, void* stream) {
-  return fsgs_gs_2d_view_epilogue_backward(W, H, depth_ratio, Tw2v, Tv2c, extras, opacity, background, g_normals, g_depths,
+  return fsgs_gs_2d_view_epilogue_backward(W, H, 9, depth_ratio, Tw2v, Tv2c, extras, opacity, background, g_normals, g_depths,
                                            g_surf_depth, g_surf_normal, g_distortion, g_composited, nullptr, g_extras,
                                            g_opacity, stream);
 }

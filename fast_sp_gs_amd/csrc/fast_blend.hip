@@ -20,6 +20,7 @@
 // (pair_queue.hpp).
 #include "binning.hpp"
 #include "blend.hpp"
+#include "instance_slots.hpp"
 #include "ordered_sums.hpp"
 #include "pair_queue.hpp"
 
@@ -384,7 +385,7 @@ struct FastScatter {
 // in the span; a wavefront none of whose surfels has a larger rectangle then reads neither the adjugates nor the opacity
 // and does not set the test up.
 __global__ void __launch_bounds__(256) fast_slot_sum_kernel(int P, int gx, int gy,
-    const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii, const float2* __restrict__ means2D,
+    const SlotSource slots, const int32_t* __restrict__ radii, const float2* __restrict__ means2D,
     const float* __restrict__ inverse_m, const float4* __restrict__ normal_opacity,
     const uint32_t* __restrict__ keep_masks, const float* __restrict__ records, FastScatter out) {
   constexpr int kLanes = kFastRecordSlots / 2, kPerWave = 64 / kLanes;
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(256) fast_slot_sum_kernel(int P, int gx, int g
     h = max(r.y1 - r.y0, 1), count = max(r.x1 - r.x0, 0) * max(r.y1 - r.y0, 0), x0 = r.x0, y0 = r.y0;
     masked = keep_masks != nullptr && count <= 32;
     if (masked) mask = keep_masks[i];
-    src += (size_t) (i > 0 ? point_offsets[i - 1] : 0) * kLanes + k;
+    src += (size_t) slot_first(slots, i) * kLanes + k;
   }
   const bool tested     = radius > 0 && !masked;
   const bool any_tested = wave_ballot(tested) != 0ull;  // wave-uniform
@@ -455,7 +456,7 @@ __global__ void __launch_bounds__(kBlendThreads)
     const float* __restrict__ dL_dpix, const float* __restrict__ dL_dextras, const float* __restrict__ dL_dopacity,
     const float2* __restrict__ dL_dflow,
     float* __restrict__ g_means2D, float* __restrict__ g_normal_opacity, float* __restrict__ g_colors,
-    float* __restrict__ g_trans, float* __restrict__ g_inv, const int64_t* __restrict__ point_offsets,
+    float* __restrict__ g_trans, float* __restrict__ g_inv, const SlotSource slots,
     const int32_t* __restrict__ radii, float* __restrict__ slot_records) {
   constexpr int kB = 64;  // surfels staged per round
   static_assert(kB == kWave, "one ballot covers a round, and a queued pair names its entry in a byte");
@@ -505,7 +506,7 @@ __global__ void __launch_bounds__(kBlendThreads)
       const int id = point_list[r0 + e];
       const float2 c = means2D[id];
       const TileRect r = tile_rect(c.x, c.y, radii[id], gx, gy);
-      const int64_t at = (id == 0 ? 0 : point_offsets[id - 1]) + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) + (tile_y - r.y0);
+      const int64_t at = slot_first(slots, id) + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) + (tile_y - r.y0);
       float2* dst = (float2*) (slot_records + (size_t) at * kFastRecordSlots);
 #pragma unroll
       for (int c2 = 0; c2 < kFastRecordSlots / 2; ++c2) dst[c2] = make_float2(0.0f, 0.0f);
@@ -564,7 +565,7 @@ __global__ void __launch_bounds__(kBlendThreads)
 #pragma unroll
       for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) id + k];
     }
-    if (kSlots) next_radius = radii[id], next_off = id == 0 ? 0 : point_offsets[id - 1];
+    if (kSlots) next_radius = radii[id], next_off = slot_first(slots, id);
   };
   if ((int) threadIdx.x < min(n_todo, kB)) gather(n_todo - 1 - (int) threadIdx.x);
 
@@ -856,7 +857,7 @@ __global__ void __launch_bounds__(64) fast_bucket_backward_kernel(int W, int H, 
     const float* __restrict__ sampled_acc, const float* __restrict__ sampled_aux, const float* __restrict__ dL_dpix,
     const float* __restrict__ dL_dextras, const float* __restrict__ dL_dopacity, float* __restrict__ g_means2D,
     float* __restrict__ g_normal_opacity, float* __restrict__ g_colors, float* __restrict__ g_trans,
-    float* __restrict__ g_inv, const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii,
+    float* __restrict__ g_inv, const SlotSource slots, const int32_t* __restrict__ radii,
     float* __restrict__ slot_records) {
   __shared__ float4 s_up[256];                // dL/d(r, g, b) | dL/ddepth
   __shared__ float4 s_up2[kAux ? 256 : 1];    // dL/dnormal | dL/dM1
@@ -883,7 +884,7 @@ __global__ void __launch_bounds__(64) fast_bucket_backward_kernel(int W, int H, 
     hot = g.hot, cold = g.cold;
     if (kSlots) {
       const TileRect r = tile_rect(hot.cx, hot.cy, radii[cold.id], gx, gy);
-      slot = (size_t) ((cold.id == 0 ? 0 : point_offsets[cold.id - 1]) + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) +
+      slot = (size_t) (slot_first(slots, cold.id) + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) +
                        (tile_y - r.y0));
     }
   }
@@ -1007,13 +1008,13 @@ __global__ void __launch_bounds__(64) fast_bucket_backward_kernel(int W, int H, 
   }
 }
 
-void launch_fast_slot_sum(int P, int gx, int gy, const int64_t* point_offsets, const int32_t* radii,
+void launch_fast_slot_sum(int P, int gx, int gy, const SlotSource& slots, const int32_t* radii,
                           const float* means2D, const float* inverse_m, const float* normal_opacity,
                           const uint32_t* keep_masks, const SlotWorkspace& ws, FastScatter out, hipStream_t s) {
   constexpr int kPerWave = 64 / (kFastRecordSlots / 2);
   const int64_t waves = div_up(P, kPerWave);
   hipLaunchKernelGGL(fast_slot_sum_kernel, dim3((unsigned) div_up(waves * 64, 256)), dim3(256), 0, s, P, gx, gy,
-                     point_offsets, radii, (const float2*) means2D, inverse_m, (const float4*) normal_opacity,
+                     slots, radii, (const float2*) means2D, inverse_m, (const float4*) normal_opacity,
                      keep_masks, ws.records, out);
 }
 
@@ -1068,13 +1069,14 @@ FSGS_API size_t fsgs_gs_2d_fast_render_backward_workspace_bytes(int64_t R) {
   return slot_workspace_bytes(R, kFastRecordSlots);
 }
 
-FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n, double far_n, int per_splat_form,
+namespace {
+int fast_render_backward(int P, int W, int H, double near_n, double far_n, int per_splat_form,
     const float* means2D, const float* normal_opacity, const float* colors, const float* trans_mat,
     const float* inverse_m, const float* trans_mat_t2, const float* out_opacity, const float* out_extras,
     const float* out_flow, const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras,
     const float* dL_dflow, const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib,
     float* g_colors, float* g_means2D, float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R,
-    const int64_t* point_offsets, const int32_t* radii, void* workspace, size_t workspace_bytes,
+    const SlotSource& source, const int32_t* radii, void* workspace, size_t workspace_bytes,
     const uint32_t* keep_masks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_fast_render_backward: bad sizes");
   if (P == 0) return kOk;
@@ -1085,7 +1087,7 @@ FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n,
   const bool flow = dL_dflow != nullptr;
   FSGS_REQUIRE(!flow || (aux && trans_mat_t2 && out_flow),
                "GS_2D_fast_render_backward: flow gradients need trans_mat2, out_flows and the auxiliary maps");
-  const bool slots = point_offsets != nullptr;
+  const bool slots = source.scan || source.region;
   SlotWorkspace ws{nullptr};
   if (slots) {
     FSGS_REQUIRE(radii && workspace && R >= 0 && R < (int64_t) 0x7fffffff,
@@ -1106,7 +1108,7 @@ FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n,
                      (float) near_n, (float) far_n, ranges, point_list, n_contrib, (const float2*) means2D,          \
                      (const float4*) normal_opacity, colors, trans_mat, inverse_m, trans_mat_t2, out_opacity,        \
                      out_extras, (const float2*) out_flow, dL_dpix, dL_dextras, dL_dopacity,                         \
-                     (const float2*) dL_dflow, g_means2D, g_normal_opacity, g_colors, g_trans, g_inv, point_offsets, \
+                     (const float2*) dL_dflow, g_means2D, g_normal_opacity, g_colors, g_trans, g_inv, source,        \
                      radii, ws.records)
 #define FSGS_LAUNCH_BWD(AUX, SPLAT, FLOW) \
   do { if (slots) FSGS_LAUNCH_BWD_S(AUX, SPLAT, FLOW, true); else FSGS_LAUNCH_BWD_S(AUX, SPLAT, FLOW, false); } while (0)
@@ -1119,9 +1121,42 @@ FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n,
 #undef FSGS_LAUNCH_BWD
 #undef FSGS_LAUNCH_BWD_S
   if (slots)
-    launch_fast_slot_sum(P, gx, gy, point_offsets, radii, means2D, inverse_m, normal_opacity, keep_masks, ws,
+    launch_fast_slot_sum(P, gx, gy, source, radii, means2D, inverse_m, normal_opacity, keep_masks, ws,
                          FastScatter{g_means2D, g_normal_opacity, g_colors, g_trans, g_inv}, s);
   return check_launch("GS_2D_fast_render_backward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n, double far_n, int per_splat_form,
+    const float* means2D, const float* normal_opacity, const float* colors, const float* trans_mat,
+    const float* inverse_m, const float* trans_mat_t2, const float* out_opacity, const float* out_extras,
+    const float* out_flow, const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras,
+    const float* dL_dflow, const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib,
+    float* g_colors, float* g_means2D, float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R,
+    const int64_t* point_offsets, const int32_t* radii, void* workspace, size_t workspace_bytes,
+    const uint32_t* keep_masks, void* stream) {
+  return fast_render_backward(P, W, H, near_n, far_n, per_splat_form, means2D, normal_opacity, colors, trans_mat, inverse_m,
+                              trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
+                              ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
+                              SlotSource{point_offsets}, radii, workspace, workspace_bytes, keep_masks, stream);
+}
+
+// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp).
+FSGS_API int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
+    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
+    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
+    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
+    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched),
+               "gs_2d_fast_view_backward: record slots are required");
+  return fast_render_backward(P, W, H, near_n, far_n, 0, means2D, normal_opacity, colors, trans_mat, inverse_m,
+                              trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
+                              ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
+                              SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
+                              workspace_bytes, keep_masks, stream);
 }
 
 // The per-splat decomposition itself (fast_bucket_backward_kernel), for callers that want the reference's second
@@ -1162,7 +1197,7 @@ FSGS_API int fsgs_gs_2d_fast_render_bucket_backward(int P, int W, int H, double 
                      (float) far_n, ranges, point_list, (const float2*) means2D, (const float4*) normal_opacity,      \
                      colors, trans_mat, inverse_m, images, out_opacity, out_extras, n_contrib, max_contrib,           \
                      bucket_offset, bucket_to_tile, sampled_T, sampled_acc, sampled_aux, dL_dpix, dL_dextras,         \
-                     dL_dopacity, g_means2D, g_normal_opacity, g_colors, g_trans, g_inv, point_offsets, radii,        \
+                     dL_dopacity, g_means2D, g_normal_opacity, g_colors, g_trans, g_inv, SlotSource{point_offsets}, radii, \
                      ws.records)
   if (B > 0) {
     if (aux && slots) FSGS_FAST_BKT(true, true);
@@ -1172,7 +1207,7 @@ FSGS_API int fsgs_gs_2d_fast_render_bucket_backward(int P, int W, int H, double 
   }
 #undef FSGS_FAST_BKT
   if (slots)
-    launch_fast_slot_sum(P, (W + kTile - 1) / kTile, (H + kTile - 1) / kTile, point_offsets, radii, means2D, inverse_m,
+    launch_fast_slot_sum(P, (W + kTile - 1) / kTile, (H + kTile - 1) / kTile, SlotSource{point_offsets}, radii, means2D, inverse_m,
                          normal_opacity, keep_masks, ws,
                          FastScatter{g_means2D, g_normal_opacity, g_colors, g_trans, g_inv}, s);
   return check_launch("GS_2D_fast_render_bucket_backward");

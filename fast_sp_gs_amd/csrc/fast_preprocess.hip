@@ -11,6 +11,7 @@
 // Geometry and the corner test are compiled with contraction off in the reference's operation order, so radii, tile
 // counts, keys, ranges and point lists are reproducible bit for bit against a plain IEEE evaluation.
 #include "binning.hpp"
+#include "instance_slots.hpp"
 #include "sh.hpp"
 #include "sh_stage.hpp"
 #include "surfel_geom.hpp"
@@ -107,11 +108,13 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     const float* __restrict__ campos, const float* __restrict__ trans_precomp, const uint8_t* __restrict__ culling,
     int means2D_preserve, float2* __restrict__ means2D, float* __restrict__ colors, float* __restrict__ trans_mat,
     float* __restrict__ inverse_m, float4* __restrict__ normal_opacity, float* __restrict__ depths,
-    int32_t* __restrict__ radii, int32_t* __restrict__ tiles_touched, uint32_t* __restrict__ keep_masks) {
+    int32_t* __restrict__ radii, int32_t* __restrict__ tiles_touched, uint32_t* __restrict__ keep_masks,
+    ViewOutputs view) {
   __shared__ float s_rows[kWave ? kShStageRows * kShStageStride : 1];
   const int i0     = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i0 < P;
-  if (!kWave && !valid) return;
+  __shared__ int s_wave_slots[4];
+  __shared__ int s_block_slot;
   const int i = valid ? i0 : P - 1;  // lanes past the end stay for the wavefront's row movement and write nothing
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   float Tw2v[16], Tv2s[9];
@@ -165,6 +168,14 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     ok    = true;
   } while (false);
 
+  // the block's record slots: the atomic is on its way while the colours are formed
+  int slot = 0;
+  unsigned long long block_slot = 0;
+  if (view.counters) {
+    int total;
+    slot = slots_in_block(ok ? area : 0, s_wave_slots, total);
+    if (threadIdx.x == 0) block_slot = atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+  }
   if (kWave) {
     if (wanted) wave_rows_to_lds(sh_regs, s_wave_rows);
     wave_lds_sync();
@@ -180,7 +191,14 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
     rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
   }
+  if (view.slot_offsets) {
+    if (threadIdx.x == 0) s_block_slot = (int) block_slot;
+    __syncthreads();
+    slot += s_block_slot;
+  }
   if (!valid) return;
+  if (view.slot_offsets) view.slot_offsets[i] = slot;
+  if (view.visible) view.visible[i] = ok && f2i_sat(radius) > 0;
   float adj[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) adj[k] = 0.0f;
@@ -427,12 +445,17 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     const float* c0 = kWave ? my_row : shs + (size_t) i * m1 * 3;
     const float* cr = kWave ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
     float* o0  = kWave ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
-    float* orr = kWave ? my_row : (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : o0);
+    float* orr = kWave ? my_row
+                       : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
     if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
     tl[0] = 0.0f;
     for (int l = 1; l < n; ++l) {
       tl[l] = g[0] * cr[3 * l] + g[1] * cr[3 * l + 1] + g[2] * cr[3 * l + 2];
-      if (o0) orr[3 * l] = g[0] * Y[l], orr[3 * l + 1] = g[1] * Y[l], orr[3 * l + 2] = g[2] * Y[l];
+      if (orr) orr[3 * l] = g[0] * Y[l], orr[3 * l + 1] = g[1] * Y[l], orr[3 * l + 2] = g[2] * Y[l];
+    }
+    if (!kWave && orr) {  // coefficients above the active degree
+      for (int l = n; l < (sh_rest ? n_sh + 1 : n_sh); ++l)
+        orr[3 * l] = 0.0f, orr[3 * l + 1] = 0.0f, orr[3 * l + 2] = 0.0f;
     }
     float dx = 0, dy = 0, dz = 0;
     sh_grad_accumulate(sh_degree, x, y, z, tl, dx, dy, dz);
@@ -500,11 +523,13 @@ __global__ void __launch_bounds__(256) fast_transmat_backward_kernel(int P, cons
 
 using namespace fsgs;
 
-FSGS_API int fsgs_gs_2d_fast_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+namespace {
+int fast_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2s, const float* campos, const float* trans_precomp, const uint8_t* culling,
     int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* inverse_m, float* normal_opacity,
-    float* depths, int32_t* radii, int32_t* tiles_touched, uint32_t* keep_masks, void* stream) {
+    float* depths, int32_t* radii, int32_t* tiles_touched, uint32_t* keep_masks,
+    const ViewOutputs& view, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_fast_preprocess_forward: bad sizes");
   FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_2d_fast_preprocess_forward: sh_degree %d not supported", sh_degree);
   if (sh_degree >= 0)
@@ -522,8 +547,31 @@ FSGS_API int fsgs_gs_2d_fast_preprocess_forward(int P, int W, int H, int sh_degr
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh,
                      means3D, (const float2*) scales, (const float4*) rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
                      campos, trans_precomp, culling, means2D_preserve, (float2*) means2D, colors, trans_mat, inverse_m,
-                     (float4*) normal_opacity, depths, radii, tiles_touched, keep_masks);
+                     (float4*) normal_opacity, depths, radii, tiles_touched, keep_masks, view);
   return check_launch("gs_2d_fast_preprocess_forward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_2d_fast_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2s, const float* campos, const float* trans_precomp, const uint8_t* culling,
+    int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* inverse_m, float* normal_opacity,
+    float* depths, int32_t* radii, int32_t* tiles_touched, uint32_t* keep_masks, void* stream) {
+  return fast_preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
+                                 campos, trans_precomp, culling, means2D_preserve, means2D, colors, trans_mat, inverse_m,
+                                 normal_opacity, depths, radii, tiles_touched, keep_masks, ViewOutputs{}, stream);
+}
+
+FSGS_API int fsgs_gs_2d_fast_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
+    int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_2d_fast_view_preprocess: slot_counters are required");
+  return fast_preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
+                                 campos, nullptr, culling, 0, means2D, colors, trans_mat, inverse_m, normal_opacity, depths,
+                                 radii, tiles_touched, keep_masks,
+                                 ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_fast_prepare_sort_bits(int W, int H) {

@@ -1,6 +1,7 @@
 // Python entry points of the native host layer (fast_sp_gs_amd._host).
 #include <torch/csrc/utils/pybind.h>
 
+#include "fast_surfel.hpp"
 #include "surfel.hpp"
 
 namespace py = pybind11;
@@ -27,8 +28,23 @@ py::tuple surfel_render_py(const Tensor& points, const Tensor& scales, const Ten
   return py::make_tuple(r.maps, r.n_contrib, r.radii, r.visible, r.ranges, r.point_list, r.normal_opacity, r.trans_mat);
 }
 
+py::tuple fast_surfel_render_py(const Tensor& points, const Tensor& scales, const Tensor& rotations,
+                                const Tensor& opacities, const Tensor& shs, const OptTensor& sh_rest,
+                                const Tensor& means2D, const Tensor& Tw2v, const Tensor& Tv2c, const Tensor& Tv2s,
+                                const Tensor& campos, const OptTensor& trans_mat_t2, const OptTensor& culling,
+                                const OptTensor& accum_max_count, const OptTensor& accum_weights_p,
+                                const OptTensor& accum_weights_count, int W, int H, int sh_degree, double near_n,
+                                double far_n, double depth_ratio, bool epilogue) {
+  const FastSurfelView v{points, scales, rotations, opacities, shs, sh_rest, means2D, Tw2v, Tv2c, Tv2s, campos, trans_mat_t2,
+                         culling, accum_max_count, accum_weights_p, accum_weights_count, W, H, sh_degree, near_n, far_n,
+                         depth_ratio, epilogue};
+  const FastSurfelResult r = without_gil([&] { return fast_surfel_render(v); });
+  return py::make_tuple(r.maps, r.radii, r.visible);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
   m.def("surfel_render", &surfel_render_py);
+  m.def("fast_surfel_render", &fast_surfel_render_py);
 }

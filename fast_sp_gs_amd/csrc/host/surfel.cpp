@@ -21,23 +21,6 @@ struct Buffers {
   Saved saved;
 };
 
-int sh_coefficients(const char* what, const SurfelView& v, int64_t P) {
-  const int64_t need = (int64_t) (1 + v.sh_degree) * (1 + v.sh_degree);
-  if (has(v.sh_rest) && v.sh_rest->numel() > 0) {
-    require(what, "sh_rest", *v.sh_rest, at::kFloat);
-    const auto s = v.sh_rest->sizes();
-    if (!(s.size() == 3 && s[0] == P && s[1] >= need - 1 && s[2] == 3)) fail("Error shape for sh features");
-    return (int) s[1];
-  }
-  if (v.sh_degree < 0) {
-    require_shape(what, "shs", v.shs, {P, 3});
-    return 0;
-  }
-  const auto s = v.shs.sizes();
-  if (!(s.size() == 3 && s[0] == P && s[1] >= need && s[2] == 3)) fail("Error shape for sh features");
-  return (int) s[1];
-}
-
 Buffers forward_view(const SurfelView& v, bool train) {
   const char* what = "gs_2d_preprocess_forward";
   require(what, "means3D", v.points, at::kFloat), require(what, "scales", v.scales, at::kFloat);
@@ -46,11 +29,8 @@ Buffers forward_view(const SurfelView& v, bool train) {
   require(what, "Tv2c", v.Tv2c, at::kFloat), require(what, "cam_pos", v.campos, at::kFloat);
   if (v.points.dim() != 2 || v.points.size(-1) != 3) fail("Error shape for means3D");
   const int64_t P = v.points.size(0);
-  const int M = sh_coefficients(what, v, P);
-  if (has(v.culling)) {
-    require(what, "culling", *v.culling, at::kBool);
-    require_shape(what, "culling", *v.culling, {P});
-  }
+  const int M = sh_coefficients(what, v.shs, v.sh_rest, v.sh_degree, P);
+  require_point_mask(what, v.culling, P);
   require_shape(what, "scales", v.scales, {P, 2}), require_shape(what, "rotations", v.rotations, {P, 4});
   require_shape(what, "opacities", v.opacities, {P, 1});
   require_shape(what, "Tw2v", v.Tw2v, {4, 4}), require_shape(what, "Tv2c", v.Tv2c, {4, 4});
@@ -61,18 +41,7 @@ Buffers forward_view(const SurfelView& v, bool train) {
     require(blend, "trans_mat_t2", *v.trans_mat_t2, at::kFloat);
     require_shape(blend, "trans_mat_t2", *v.trans_mat_t2, {P, 3, 3});
   }
-  if (has(v.accum_max_count)) {
-    require(blend, "accum_max_count", *v.accum_max_count, at::kInt);
-    require_shape(blend, "accum_max_count", *v.accum_max_count, {P});
-  }
-  if (has(v.accum_weights_count)) {
-    require(blend, "accum_weights_count", *v.accum_weights_count, at::kInt);
-    require_shape(blend, "accum_weights_count", *v.accum_weights_count, {P});
-  }
-  if (has(v.accum_weights_p)) {
-    require(blend, "accum_weights_p", *v.accum_weights_p, at::kFloat);
-    require_shape(blend, "accum_weights_p", *v.accum_weights_p, {P});
-  }
+  require_accumulators(blend, v.accum_max_count, v.accum_weights_p, v.accum_weights_count, P);
   if (has(v.background)) {
     require("gs_2d_epilogue_forward", "background", *v.background, at::kFloat);
     if (v.background->numel() != 3) fail("gs_2d_epilogue_forward: background must have 3 elements");
@@ -232,7 +201,7 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
           g_dist.defined()) {
         g_extras = empty({9, H, W}, points);
         Tensor g_total = composite || !g_opacity.defined() ? empty({H, W}, points) : Tensor();
-        check(fsgs_gs_2d_view_epilogue_backward(W, H, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
+        check(fsgs_gs_2d_view_epilogue_backward(W, H, 9, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
                                                 f32(background), f32(g_normals), f32(g_depths), f32(g_surf_depth),
                                                 f32(g_surf_normal), f32(g_dist), composite ? f32(g_image) : nullptr,
                                                 f32(g_opacity), f32(g_extras), f32(g_total), stream),

@@ -36,6 +36,41 @@ void require_shape(const char* what, const char* name, const Tensor& t, at::IntA
     fail(std::string(what) + ": " + name + " must have shape " + shape_text(shape) + ", got " + shape_text(t.sizes()));
 }
 
+int sh_coefficients(const char* what, const Tensor& shs, const OptTensor& sh_rest, int sh_degree, int64_t P) {
+  const int64_t need = (int64_t) (1 + sh_degree) * (1 + sh_degree);
+  if (has(sh_rest) && sh_rest->numel() > 0) {
+    require(what, "sh_rest", *sh_rest, at::kFloat);
+    const auto s = sh_rest->sizes();
+    if (!(s.size() == 3 && s[0] == P && s[1] >= need - 1 && s[2] == 3)) fail("Error shape for sh features");
+    return (int) s[1];
+  }
+  if (sh_degree < 0) {
+    require_shape(what, "shs", shs, {P, 3});
+    return 0;
+  }
+  const auto s = shs.sizes();
+  if (!(s.size() == 3 && s[0] == P && s[1] >= need && s[2] == 3)) fail("Error shape for sh features");
+  return (int) s[1];
+}
+
+void require_point_mask(const char* what, const OptTensor& culling, int64_t P) {
+  if (!has(culling)) return;
+  require(what, "culling", *culling, at::kBool);
+  require_shape(what, "culling", *culling, {P});
+}
+
+void require_accumulators(const char* what, const OptTensor& max_count, const OptTensor& weights_p,
+                          const OptTensor& weights_count, int64_t P) {
+  auto one = [&](const char* name, const OptTensor& t, at::ScalarType type) {
+    if (!has(t)) return;
+    require(what, name, *t, type);
+    require_shape(what, name, *t, {P});
+  };
+  one("accum_max_count", max_count, at::kInt);
+  one("accum_weights_count", weights_count, at::kInt);
+  one("accum_weights_p", weights_p, at::kFloat);
+}
+
 int64_t* pinned_count() {
   static thread_local Tensor word;
   if (!word.defined()) word = at::zeros({8}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));

@@ -43,6 +43,13 @@ void require_shape(const char* what, const char* name, const Tensor& t, at::IntA
 inline bool has(const OptTensor& t) { return t.has_value() && t->defined(); }
 inline Tensor opt(const OptTensor& t) { return has(t) ? *t : Tensor(); }
 
+// Stored SH coefficients per point beside the split-off first one: checks [P,M,3] (or [P,1,3] + [P,M,3], or colours [P,3]
+// for degree < 0) and returns M.
+int sh_coefficients(const char* what, const Tensor& shs, const OptTensor& sh_rest, int sh_degree, int64_t P);
+void require_point_mask(const char* what, const OptTensor& culling, int64_t P);
+void require_accumulators(const char* what, const OptTensor& max_count, const OptTensor& weights_p,
+                          const OptTensor& weights_count, int64_t P);
+
 template <typename T>
 T* data(const Tensor& t) {
   return t.defined() ? (T*) t.data_ptr() : nullptr;

@@ -28,6 +28,12 @@ struct SlotSource {
 
 __device__ __forceinline__ int slot_region(int i) { return (i >> kSlotBlockBits) & (kSlotRegions - 1); }
 
+// First record slot of a surfel.
+__device__ __forceinline__ int64_t slot_first(const SlotSource& s, int i) {
+  if (s.region) return (int64_t) s.offset[i] + s.region[slot_region(i)];
+  return i > 0 ? s.scan[i - 1] : 0;
+}
+
 __device__ __forceinline__ void slot_span(const SlotSource& s, int i, int64_t& first, int& count) {
   if (s.region) {
     first = (int64_t) s.offset[i] + s.region[slot_region(i)];
@@ -60,6 +66,14 @@ __device__ __forceinline__ int slots_in_block(int count, int* s_wave, int& total
   }
   return before + inc - count;
 }
+
+// What a view through the native host path asks of a preprocess kernel on top (all optional): the region counters, the
+// surfel's first record slot inside its block's region, and the visibility as a byte.
+struct ViewOutputs {
+  unsigned long long* counters = nullptr;
+  int32_t* slot_offsets = nullptr;
+  uint8_t* visible = nullptr;
+};
 
 // What the kernel behind the preprocess hands on: see above. `counters` nullptr: nothing to do.
 struct SlotPublish {

@@ -82,14 +82,6 @@ __device__ __forceinline__ void transmat(int W, int H, const float* p, float sx,
   nrm[2] = Tw2v[8] * t0 + Tw2v[9] * t1 + Tw2v[10] * t2;
 }
 
-// What a view through the native host path asks for on top (all optional): the surfel's first record slot inside its
-// block's region (instance_slots.hpp), the region counters, and the visibility as a byte.
-struct ViewOutputs {
-  unsigned long long* counters = nullptr;
-  int32_t* slot_offsets = nullptr;
-  uint8_t* visible = nullptr;
-};
-
 // kWave: complete degree-3 rows in one 16-byte aligned [P,16,3] tensor, moved by each wavefront on its own.
 template <int kSh, bool kWave>
 __global__ void __launch_bounds__(256) preprocess_forward_kernel(

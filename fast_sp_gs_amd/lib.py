@@ -125,4 +125,6 @@ def require_dtype(what: str, name: str, t: torch.Tensor, dtype) -> None:
         raise RuntimeError(f"{what}: {name} must have dtype {dtype}, got {t.dtype}")
 
 
-surfel_render = _host_layer().surfel_render
+_host = _host_layer()
+surfel_render = _host.surfel_render
+fast_surfel_render = _host.fast_surfel_render

@@ -9,6 +9,7 @@ import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
+from fast_sp_gs_amd.lib import fast_surfel_render
 from .gs_2d_render import depth_to_normal
 
 __all__ = ['GS_2D_fast_render', 'GS_2D_fast_preprocess', 'GS_2D_fast_rasterize', 'GS_2D_fast_rasterize_v2',
@@ -181,6 +182,8 @@ def GS_2D_fast_rasterize_v2(W: int, H: int, mean2D: Tensor, colors: Tensor, norm
 
 
 class _Fast_Render(torch.autograd.Function):
+    """The view on the operators, one call each (the reference's class of this name, gs_2d_fast_render.py:592-667).
+    `GS_2D_fast_render` makes the same launches through the native host layer."""
     _preprocess_forward = get_C_function('gs_2d_fast_preprocess_forward')
     _preprocess_backward = get_C_function('gs_2d_fast_preprocess_backward')
     _render_forward = get_C_function('GS_2D_fast_render_forward')
@@ -249,26 +252,34 @@ def GS_2D_fast_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity
                       sh_features: Tensor = None, sh_features_rest: Tensor = None, depth_ratio=1.,
                       culling: Tensor = None, accum_max_count: Tensor = None, accum_weights_p: Tensor = None,
                       accum_weights_count: Tensor = None, trans_mat_t2: Tensor = None, **kwargs):
-    means2D = points.new_zeros(points.shape[0], 2, requires_grad=True)
-    W, H = size
+    # the preprocess kernel writes every row (zeros for surfels that are not rendered)
+    means2D = torch.empty((points.shape[0], 2), dtype=torch.float32, device=points.device, requires_grad=True)
+    W, H = int(size[0]), int(size[1])
     if campos is None:
         campos = Tw2v.inverse()[:3, 3].contiguous()
-    images, opacities, out_extras, flows, n_contrib, radii = _Fast_Render.apply(
-        points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest,
-        Tw2v.contiguous(), Tv2c.contiguous(), Tv2s.contiguous(), campos.contiguous(), size,
-        sh_degree if colors is None else -1, is_opengl, near, far, False, None, means2D, trans_mat_t2, culling,
-        accum_max_count, accum_weights_p, accum_weights_count)
-    depths, normals, median_depths, distortion, _ = out_extras.split([1, 3, 1, 1, 2], dim=0)
-    normals = (normals.permute(1, 2, 0) @ Tw2v[:3, :3]).permute(2, 0, 1)
-    median_depths = torch.nan_to_num(median_depths, 0, 0)
-    depths = torch.nan_to_num(depths, 0, 0)
-    surf_depth = depths * (1 - depth_ratio) + depth_ratio * median_depths
-    surf_normal = depth_to_normal(Tw2v, Tv2c, (W, H), surf_depth).permute(2, 0, 1)
-    surf_normal = surf_normal * opacities.detach()
+    # camera optimisation: the fused epilogue produces no camera gradients, take the reference's torch ops
+    fused = not (Tw2v.requires_grad or Tv2c.requires_grad)
+    depth_ratio = float(depth_ratio)
+    maps, radii, visible = fast_surfel_render(
+        points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest, means2D,
+        Tw2v.contiguous(), Tv2c.contiguous(), Tv2s.contiguous(), campos.contiguous(), trans_mat_t2, culling,
+        accum_max_count, accum_weights_p, accum_weights_count, W, H, int(sh_degree) if colors is None else -1,
+        float(near), float(far), depth_ratio, fused)
+    if fused:
+        images, opacities, normals, surf_depth, surf_normal, distortion, *flow = maps
+    else:
+        images, opacities, out_extras, *flow = maps
+        depths, normals, median_depths, distortion, _ = out_extras.split([1, 3, 1, 1, 2], dim=0)
+        normals = (normals.permute(1, 2, 0) @ Tw2v[:3, :3]).permute(2, 0, 1)
+        median_depths = torch.nan_to_num(median_depths, 0, 0)
+        depths = torch.nan_to_num(depths, 0, 0)
+        surf_depth = depths * (1 - depth_ratio) + depth_ratio * median_depths
+        surf_normal = depth_to_normal(Tw2v, Tv2c, (W, H), surf_depth).permute(2, 0, 1)
+        surf_normal = surf_normal * opacities.detach()
     return {
         'images': images, 'normals': normals, 'opacity': opacities, 'distortion': distortion,
         'surf_depth': surf_depth, 'surf_normal': surf_normal, 'radii': radii, 'viewspace_points': means2D,
-        'visibility_filter': radii > 0, 'flows': flows,
+        'visibility_filter': visible, 'flows': flow[0] if flow else None,
     }
 
 

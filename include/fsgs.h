@@ -148,6 +148,16 @@ int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t*
                        uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges,
                        void* bins, size_t bins_bytes, void* stream);
 int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream);
+/* The two parts for the "fast" surfels (tiles that pass the corner test; keep_masks of the preprocess). Unlike
+ * fsgs_gs_2d_fast_prepare_fill no padding entries are written behind the kept instances. */
+int fsgs_gs_2d_fast_view_count(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
+                               const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters,
+                               int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges, void* bins,
+                               size_t bins_bytes, void* stream);
+int fsgs_gs_2d_fast_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                              const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R,
+                              int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
+                              size_t workspace_bytes, void* stream);
 
 /* ---- per-tile alpha blend ------------------------------------------------------------------------------------- */
 
@@ -227,6 +237,13 @@ int fsgs_gs_2d_fast_preprocess_forward(int P, int W, int H, int sh_degree, int n
     int means2D_preserve, float* means2D, float* colors, float* trans_mat, float* inverse_m, float* normal_opacity,
     float* depths, int32_t* radii, int32_t* tiles_touched, uint32_t* keep_masks, void* stream);
 
+/* The same with the record slots of fsgs_gs_2d_view_preprocess and the visibility. */
+int fsgs_gs_2d_fast_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
+    int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, void* stream);
+
 /* Binning half of gs_2d_fast_preprocess_forward -- gs_2d_fast_preprocess.cu:264-327 (duplicateWithKeys with the
  * per-tile corner test, x-major, unused slots padded with key = T << 32 / value = -1), :711-778 (sort on
  * 32 + msb(T + 1) bits, ranges). The prefix scan is fsgs_gs_prepare_scan. point_list[R] keeps the -1 padding entries
@@ -296,6 +313,16 @@ int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n, double f
     float* g_colors, float* g_means2D, float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R,
     const int64_t* point_offsets, const int32_t* radii, void* workspace, size_t workspace_bytes,
     const uint32_t* keep_masks, void* stream);
+
+/* The same (back-to-front form) with the record slots of fsgs_gs_2d_fast_view_preprocess. */
+int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
+    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
+    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
+    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
+    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const uint32_t* keep_masks, void* stream);
 
 /* The per-splat decomposition of gs_2d_fast_redner.cu:563-837 itself (fsgs_gs_2d_fast_render_backward with
  * per_splat_form = 1 returns the same derivative through the back-to-front kernel, which is faster here): a lane owns
@@ -571,7 +598,7 @@ int fsgs_gaussian_rasterize_bucket_backward(int P, int W, int H, int E, int B, c
  * (gs_2d_render.py:439-470: normalised cross product of the central differences of the back-projected surf_depth, zero
  * on the one-pixel border) times opacity; and, when composited is not NULL, composited[3,H,W] = images + (1 - opacity)
  * * background[3] (fast_2d_gs/network.py:725-726). Tw2v[4,4] must be affine (last row 0 0 0 1), Tv2c[4,4] is the
- * projection; both are read on the device. Every output element is written. */
+ * projection; both are read on the device. Every output element is written; `depths` is optional. */
 int fsgs_gs_2d_epilogue_forward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
     const float* extras, const float* opacity, const float* images, const float* background, float* normals,
     float* depths, float* surf_depth, float* surf_normal, float* composited, void* stream);
@@ -584,8 +611,9 @@ int fsgs_gs_2d_epilogue_backward(int W, int H, double depth_ratio, const float* 
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
     float* g_extras, float* g_opacity, void* stream);
-/* The same, with the gradient the opacity map has from elsewhere added into g_opacity (g_opacity_in[H,W], optional). */
-int fsgs_gs_2d_view_epilogue_backward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
+/* The same, with the gradient the opacity map has from elsewhere added into g_opacity (g_opacity_in[H,W], optional) and
+ * `channels` channels in g_extras (9, or 8 for the "fast" blend's maps; those from the seventh on are zero). */
+int fsgs_gs_2d_view_epilogue_backward(int W, int H, int channels, double depth_ratio, const float* Tw2v, const float* Tv2c,
     const float* extras, const float* opacity, const float* background, const float* g_normals, const float* g_depths,
     const float* g_surf_depth, const float* g_surf_normal, const float* g_distortion, const float* g_composited,
     const float* g_opacity_in, float* g_extras, float* g_opacity, void* stream);

@@ -104,3 +104,47 @@ def test_surfel_views_on_two_streams_and_threads(device):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize('P,W,H,mode', [(1, 16, 16, 'sh'), (257, 49, 31, 'split'), (256, 64, 48, 'colors'),
+                                        (300, 49, 31, 'partial'), (16_385, 161, 99, 'culling'), (20_000, 250, 130, 'flow')])
+def test_fast_surfel_view_equals_operators(P, W, H, mode, device):
+    """The fused tail's maps to the rounding of its 3x3 inverses; everything else bit for bit."""
+    from fast_sp_gs_amd.renderer import gs_2d_fast_render as m
+    from fast_sp_gs_amd.renderer.gs_2d_render import depth_to_normal
+    s, cam_h, g = _scene(P, W, H, P + 2)
+    cam = cam_h.to(device)
+    params = _leaves(device, s.means3D, s.scales, s.rotations, s.opacities)
+    rest, degree = None, 2 if mode == 'partial' else 3
+    if mode == 'split':
+        sh, rest = _leaves(device, s.shs[:, :1].contiguous(), s.shs[:, 1:].contiguous())
+    else:
+        sh, = _leaves(device, s.shs[:, 0].contiguous() if mode == 'colors' else s.shs)
+    culling = (torch.rand(P, generator=g) < 0.3).to(device) if mode == 'culling' else None
+    t2 = torch.randn(P, 3, 3, generator=g).to(device) if mode == 'flow' else None
+    out = m.GS_2D_fast_render(*params, (W, H), cam.Tw2v, cam.Tv2c, cam.Tv2s, campos=cam.campos, sh_degree=degree,
+                              colors=sh if mode == 'colors' else None, sh_features=None if mode == 'colors' else sh,
+                              sh_features_rest=rest, culling=culling, trans_mat_t2=t2)
+    m2 = torch.zeros(P, 2, device=device, requires_grad=True)
+    img, opac, extras, flow, n_contrib, radii = m._Fast_Render.apply(
+        *params, sh, rest, cam.Tw2v, cam.Tv2c, cam.Tv2s, cam.campos, (W, H), -1 if mode == 'colors' else degree, False, 0.2,
+        100.0, False, None, m2, t2, culling, None, None, None)
+    depth = torch.nan_to_num(extras[4:5], 0, 0)  # depth_ratio = 1
+    normals = (extras[1:4].permute(1, 2, 0) @ cam.Tw2v[:3, :3]).permute(2, 0, 1)
+    surf_normal = depth_to_normal(cam.Tw2v, cam.Tv2c, (W, H), depth).permute(2, 0, 1) * opac.detach()
+    same = lambda a, b: a.shape == b.shape and torch.equal(a, b)
+    assert same(out['images'], img) and same(out['opacity'], opac) and same(out['distortion'], extras[5:6])
+    assert same(out['radii'], radii) and same(out['visibility_filter'], radii > 0)
+    assert same(out['viewspace_points'], m2) and same(out['surf_depth'], depth)
+    assert torch.allclose(out['normals'], normals, atol=1e-6)
+    assert (out['surf_normal'] - surf_normal).norm() <= 2e-3 * surf_normal.norm() + 1e-6
+    assert (out['flows'] is None and flow is None) or same(out['flows'], flow)
+    up = [torch.randn(t.shape, generator=g).to(device) for t in (img, opac, extras[5:6], normals, depth)]
+    wanted = params + [sh] + ([rest] if rest is not None else [])
+    got = torch.autograd.grad([out[k] for k in ('images', 'opacity', 'distortion', 'normals', 'surf_depth')] +
+                              ([out['flows']] if flow is not None else []), wanted + [out['viewspace_points']],
+                              up + ([torch.ones_like(flow)] if flow is not None else []))
+    ref = torch.autograd.grad([img, opac, extras[5:6], normals, depth] + ([flow] if flow is not None else []), wanted + [m2],
+                              up + ([torch.ones_like(flow)] if flow is not None else []))
+    for a, b in zip(got, ref):
+        assert (a - b).norm() <= 1e-5 * b.norm() + 1e-7
