@@ -11,6 +11,8 @@
 // moved between HBM and LDS by the whole block on consecutive addresses as in the surfel preprocess. Every output row
 // is written (zeros for Gaussians that are not rendered), so callers allocate uninitialised memory.
 #include "common.hpp"
+#include "cull_bound.hpp"
+#include "instance_slots.hpp"
 #include "sh.hpp"
 #include "sh_stage.hpp"
 
@@ -256,8 +258,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
     const float* __restrict__ cov3D_precomp, const float* __restrict__ cov2D_precomp,
     int means2D_preserve, float2* __restrict__ means2D, float* __restrict__ depths, float* __restrict__ colors,
     int32_t* __restrict__ radii, int32_t* __restrict__ tiles_touched, float* __restrict__ cov3Ds,
-    float4* __restrict__ conic_opacity) {
+    float4* __restrict__ conic_opacity, uint32_t* __restrict__ keep_masks, ViewOutputs view) {
   constexpr bool kStage = kSh == 16;
+  __shared__ int s_wave_slots[4];
   __shared__ float s_Tw2v[16], s_Tv2c[16];
   __shared__ float s_rows[kStage ? kShStageRows * kShStageStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
@@ -303,6 +306,11 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
                          Tw2v, sc);
   } while (false);
 
+  if (view.counters) {  // how many instances the view has
+    int total;
+    (void) slots_in_block(ok ? sc.area : 0, s_wave_slots, total);
+    if (threadIdx.x == 0) atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+  }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
     if (kWave) {
@@ -334,9 +342,29 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   }
   depths[i]        = ok ? sc.depth : 0.0f;
   radii[i]         = ok ? f2i_sat(sc.radius) : 0;
-  tiles_touched[i] = ok ? sc.area : 0;
+  if (tiles_touched) tiles_touched[i] = ok ? sc.area : 0;
+  if (view.visible) view.visible[i] = ok && f2i_sat(sc.radius) > 0;
   if (ok || !means2D_preserve) means2D[i] = ok ? make_float2(sc.px, sc.py) : make_float2(0.0f, 0.0f);
-  conic_opacity[i] = ok ? make_float4(sc.conic[0], sc.conic[1], sc.conic[2], opacities[i]) : make_float4(0, 0, 0, 0);
+  const float opacity = opacities[i];
+  conic_opacity[i] = ok ? make_float4(sc.conic[0], sc.conic[1], sc.conic[2], opacity) : make_float4(0, 0, 0, 0);
+  if (keep_masks) {
+    // which tiles of the rectangle some pixel of which can blend the Gaussian (as conic_cull_mask_kernel finds it), here
+    // where centre and conic are in registers
+    uint32_t m = 0xffffffffu;
+    if (ok) {
+      const TileRect r = tile_rect(sc.px, sc.py, f2i_sat(sc.radius), gx, gy);
+      const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
+      if (w * h <= kCullMaskTiles) {
+        const CullBounds cb = conic_cull_bounds(sc.conic[0], sc.conic[1], sc.conic[2], opacity);
+        m = 0u;
+        int e = 0;
+        for (int y = 0; y < h; ++y)
+          for (int x = 0; x < w; ++x, ++e)
+            if (cull_keeps_tile(cb, sc.px, sc.py, r.x0 + x, r.y0 + y)) m |= 1u << e;
+      }
+    }
+    keep_masks[i] = m;
+  }
 }
 
 template <int kSh, bool kWave>
@@ -650,12 +678,13 @@ FSGS_API int fsgs_gs_compute_cov2D_backward(int N, const float* cov3D, const flo
   return check_launch("gs_compute_cov2D_backward");
 }
 
-FSGS_API int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
+namespace {
+int gs3d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
     const float* means3D, const float* scales, const float* rotations, const float* opacities, const float* shs,
     const float* sh_rest, const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy,
     const uint8_t* culling, const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve,
     float* means2D, float* depths, float* colors, int32_t* radii, int32_t* tiles_touched, float* cov3Ds,
-    float* conic_opacity, void* stream) {
+    float* conic_opacity, uint32_t* keep_masks, const ViewOutputs& view, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0 && tan_fovx > 0 && tan_fovy > 0, "gs_preprocess_forward: bad sizes");
   FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_preprocess_forward: sh_degree %d > %d not supported", sh_degree,
                kMaxShDegree);
@@ -664,7 +693,7 @@ FSGS_API int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int 
                  "gs_preprocess_forward: %d SH coefficients are too few for degree %d", n_sh, sh_degree);
   if (P == 0) return kOk;
   FSGS_REQUIRE(means3D && scales && rotations && opacities && shs && Tw2v && Tv2c && campos && means2D && depths &&
-                   radii && tiles_touched && (cov3Ds || cov3D_precomp) && conic_opacity && (colors || sh_degree < 0),
+                   radii && (tiles_touched || view.counters) && (cov3Ds || cov3D_precomp) && conic_opacity && (colors || sh_degree < 0),
                "gs_preprocess_forward: null pointer");
   const bool wave_rows = sh_degree == 3 && n_sh == 16 && !sh_rest && (uintptr_t) shs % 16 == 0;
   auto kernel = sh_degree > 3 ? gs3d_preprocess_forward_kernel<64, false>
@@ -674,8 +703,34 @@ FSGS_API int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int 
                      is_opengl, means3D, scales, (const float4*) rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
                      campos, (float) tan_fovx, (float) tan_fovy, culling, cov3D_precomp, cov2D_precomp, means2D_preserve,
                      (float2*) means2D, depths, colors, radii, tiles_touched, cov3D_precomp ? nullptr : cov3Ds,
-                     (float4*) conic_opacity);
+                     (float4*) conic_opacity, keep_masks, view);
   return check_launch("gs_preprocess_forward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
+    const float* means3D, const float* scales, const float* rotations, const float* opacities, const float* shs,
+    const float* sh_rest, const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy,
+    const uint8_t* culling, const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve,
+    float* means2D, float* depths, float* colors, int32_t* radii, int32_t* tiles_touched, float* cov3Ds,
+    float* conic_opacity, void* stream) {
+  return gs3d_preprocess_forward(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest,
+                                 Tw2v, Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp,
+                                 means2D_preserve, means2D, depths, colors, radii, tiles_touched, cov3Ds, conic_opacity,
+                                 nullptr, ViewOutputs{}, stream);
+}
+
+FSGS_API int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
+    const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
+    float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
+    uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_view_preprocess: slot_counters are required");
+  return gs3d_preprocess_forward(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest,
+                                 Tw2v, Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp,
+                                 means2D_preserve, means2D, depths, colors, radii, nullptr, cov3Ds, conic_opacity, keep_masks,
+                                 ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible}, stream);
 }
 
 FSGS_API int fsgs_gs_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,

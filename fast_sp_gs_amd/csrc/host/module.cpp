@@ -2,6 +2,7 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include "fast_surfel.hpp"
+#include "gaussian.hpp"
 #include "surfel.hpp"
 
 namespace py = pybind11;
@@ -42,9 +43,23 @@ py::tuple fast_surfel_render_py(const Tensor& points, const Tensor& scales, cons
   return py::make_tuple(r.maps, r.radii, r.visible);
 }
 
+py::tuple gaussian_render_py(const Tensor& points, const Tensor& scales, const Tensor& rotations, const Tensor& opacities,
+                             const Tensor& shs, const OptTensor& sh_rest, const OptTensor& cov3D, const OptTensor& cov2D,
+                             const Tensor& means2D, const OptTensor& extras, const Tensor& Tw2v, const Tensor& Tv2c,
+                             const Tensor& campos, const OptTensor& culling, const OptTensor& accum_max_count,
+                             const OptTensor& accum_weights_p, const OptTensor& accum_weights_count, double tan_x,
+                             double tan_y, int W, int H, int sh_degree, bool is_opengl, bool preserve, bool cull) {
+  const GaussianView v{points, scales, rotations, opacities, shs, sh_rest, cov3D, cov2D, means2D, extras, Tw2v, Tv2c, campos,
+                       culling, accum_max_count, accum_weights_p, accum_weights_count, tan_x, tan_y, W, H, sh_degree,
+                       is_opengl, preserve, cull};
+  const GaussianResult r = without_gil([&] { return gaussian_render(v); });
+  return py::make_tuple(r.maps, r.n_contrib, r.radii, r.visible, r.ranges, r.point_list);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
   m.def("surfel_render", &surfel_render_py);
   m.def("fast_surfel_render", &fast_surfel_render_py);
+  m.def("gaussian_render", &gaussian_render_py);
 }

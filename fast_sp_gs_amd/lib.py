@@ -128,3 +128,4 @@ def require_dtype(what: str, name: str, t: torch.Tensor, dtype) -> None:
 _host = _host_layer()
 surfel_render = _host.surfel_render
 fast_surfel_render = _host.fast_surfel_render
+gaussian_render = _host.gaussian_render

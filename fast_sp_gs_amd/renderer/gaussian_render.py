@@ -5,12 +5,14 @@ with covariances from scales + rotations or pre-computed (3D or 2D), gradients t
 position, and `_render_extra` / `render_extra` :925-962 for further feature tables of any width."""
 from __future__ import annotations
 
+import math
 from typing import NamedTuple, Optional, Tuple
 
 import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
+from fast_sp_gs_amd.lib import gaussian_render as native_render
 from fast_sp_gs_amd.renderer.gs_2d_render import GS_prepare
 
 _cull_masks = get_C_function('gs_cull_masks')
@@ -308,6 +310,42 @@ def RasterizeGaussians(means3D: Tensor, means2D: Optional[Tensor], colors: Tenso
                        tanFoV: Tensor, is_opengl: bool, culling: Optional[Tensor], accum_max_count: Optional[Tensor],
                        accum_weights_p: Optional[Tensor], accum_weights_count: Optional[Tensor], *other_extras: Tensor):
     """gaussian_render.py:226-274: preprocess -> binning -> blend."""
+    if means2D is None:
+        means2D = torch.zeros((means3D.shape[0], 2), dtype=torch.float32, device=means3D.device)
+    return _rasterize(means3D, means2D, True, colors, sh_rest, opacities, scales, rotations, cov3Ds_precomp,
+                      cov2Ds_precomp, extras, image_size, sh_degree, Tw2v, Tv2c, cam_pos, tanFoV, is_opengl, culling,
+                      accum_max_count, accum_weights_p, accum_weights_count, *other_extras)[:-1]
+
+
+def _rasterize(means3D, means2D, preserve, colors, sh_rest, opacities, scales, rotations, cov3D, cov2D, extras,
+               image_size, sh_degree, Tw2v, Tv2c, cam_pos, tanFoV, is_opengl, culling, accum_max_count, accum_weights_p,
+               accum_weights_count, *other_extras):
+    """`RasterizeGaussians` with the visibility in front of the result; `preserve` False: means2D holds nothing yet."""
+    W, H = int(image_size[0]), int(image_size[1])
+    tanFoV = tuple(tanFoV.detach().reshape(2).tolist()) if isinstance(tanFoV, Tensor) else tanFoV
+    if DETERMINISTIC_SUMS or (torch.is_grad_enabled() and (Tw2v.requires_grad or cam_pos.requires_grad)):
+        # fixed-order sums, or camera gradients: the view on the operators, one call each
+        if not preserve:
+            with torch.no_grad():
+                means2D.zero_()
+        return _rasterize_operators(means3D, means2D, colors, sh_rest, opacities, scales, rotations, cov3D, cov2D,
+                                    extras, (W, H), sh_degree, Tw2v, Tv2c, cam_pos, tanFoV, is_opengl, culling,
+                                    accum_max_count, accum_weights_p, accum_weights_count, *other_extras)
+    maps, n_contrib, radii, visible, tile_ranges, point_list = native_render(
+        means3D, scales, rotations, opacities, colors, sh_rest, cov3D, cov2D, means2D, extras, Tw2v, Tv2c, cam_pos,
+        culling, accum_max_count, accum_weights_p, accum_weights_count, float(tanFoV[0]), float(tanFoV[1]), W, H,
+        int(sh_degree), bool(is_opengl), preserve, bool(CULL_LISTS))
+    image, opacity, screen, conic_opacity, *out_extras = maps
+    buffer = RasterizeBuffer3D(W, H, len(opacities), point_list.shape[0], tile_ranges, point_list, n_contrib,
+                               conic_opacity, screen, opacity)
+    others = [_render_extra.apply(W, H, x, screen, conic_opacity, tile_ranges, point_list, n_contrib, opacity)
+              for x in other_extras]
+    return (image, opacity, out_extras[0] if out_extras else None, radii, buffer, *others, visible)
+
+
+def _rasterize_operators(means3D, means2D, colors, sh_rest, opacities, scales, rotations, cov3Ds_precomp, cov2Ds_precomp,
+                         extras, image_size, sh_degree, Tw2v, Tv2c, cam_pos, tanFoV, is_opengl, culling, accum_max_count,
+                         accum_weights_p, accum_weights_count, *other_extras):
     W, H = image_size
     means2D, depths, colors, radii, tiles_touched, conic_opacity = preprocess(
         means3D, scales, rotations, opacities, colors, sh_rest, Tw2v, Tv2c, cam_pos, tanFoV, W, H, sh_degree,
@@ -325,7 +363,7 @@ def RasterizeGaussians(means3D: Tensor, means2D: Optional[Tensor], colors: Tenso
                                conic_opacity, means2D, out_opacities)
     out_other_extras = [_render_extra.apply(W, H, extras_, means2D, conic_opacity, tile_ranges, point_list, n_contrib,
                                             out_opacities) for extras_ in other_extras]
-    return (out_pixels, out_opacities, out_extras, radii, buffer, *out_other_extras)
+    return (out_pixels, out_opacities, out_extras, radii, buffer, *out_other_extras, radii > 0)
 
 
 def render(Tw2v: Tensor, Tv2c: Tensor, size: Tuple[int, int], points: Tensor, opacity: Tensor, scales: Tensor = None,
@@ -335,13 +373,15 @@ def render(Tw2v: Tensor, Tv2c: Tensor, size: Tuple[int, int], points: Tensor, op
            accum_max_count: Tensor = None, accum_weights_p: Tensor = None, accum_weights_count: Tensor = None,
            **kwargs):
     """Same inputs, outputs and dict keys as the reference's `render` (gaussian_render.py:277-359)."""
-    means2D = torch.zeros_like(points[:, :2]).contiguous().requires_grad_()
+    # the preprocess kernel writes every row (zeros for Gaussians that are not rendered)
+    means2D = torch.empty((points.shape[0], 2), dtype=torch.float32, device=points.device, requires_grad=True)
     if campos is None:
         campos = Tw2v.inverse()[:3, 3].contiguous()
     if FoV is None:
         tanFoV = 0.5 * torch.as_tensor(size, device=Tw2v.device) / focals
     else:
-        tanFoV = torch.tan(torch.as_tensor(FoV) * 0.5)
+        tanFoV = (torch.tan(FoV * 0.5) if isinstance(FoV, Tensor) else
+                  [math.tan(0.5 * float(angle)) for angle in FoV])
     extras, extra_key = None, None
     for k, v in list(kwargs.items()):
         if isinstance(v, Tensor) and v.shape[-1] <= 4:
@@ -350,13 +390,13 @@ def render(Tw2v: Tensor, Tv2c: Tensor, size: Tuple[int, int], points: Tensor, op
             break
     c = lambda t: None if t is None else t.contiguous()
     others = {k: v for k, v in kwargs.items() if isinstance(v, Tensor)}
-    image, out_opacity, out_extra, radii, buffer, *out_others = RasterizeGaussians(
-        points.contiguous(), means2D, c(sh_features) if colors is None else colors.contiguous(), c(sh_features_rest),
+    image, out_opacity, out_extra, radii, buffer, *out_others, visible = _rasterize(
+        points.contiguous(), means2D, False, c(sh_features) if colors is None else colors.contiguous(), c(sh_features_rest),
         opacity.contiguous(), c(scales), c(rotations), c(cov3Ds), c(cov2Ds), c(extras), size,
         sh_degree if colors is None else -1, Tw2v.view(4, 4).contiguous(), Tv2c.view(4, 4).contiguous(),
-        campos.view(3).contiguous(), tanFoV.view(2), is_opengl, culling, accum_max_count, accum_weights_p,
+        campos.view(3).contiguous(), tanFoV, is_opengl, culling, accum_max_count, accum_weights_p,
         accum_weights_count, *others.values())
-    out = {'images': image, 'opacity': out_opacity, 'viewspace_points': means2D, 'visibility_filter': radii > 0,
+    out = {'images': image, 'opacity': out_opacity, 'viewspace_points': means2D, 'visibility_filter': visible,
            'radii': radii, 'buffer': buffer}
     out.update(zip(others.keys(), out_others))  # each [H,W,E], pixel-major as in the reference
     if extra_key is not None:

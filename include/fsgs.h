@@ -477,6 +477,15 @@ int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, int
     float* means2D, float* depths, float* colors, int32_t* radii, int32_t* tiles_touched, float* cov3Ds,
     float* conic_opacity, void* stream);
 
+/* The same for a whole view: counts the view's instances into slot_counters (as fsgs_gs_2d_view_preprocess) and leaves
+ * the visibility and the keep masks of fsgs_gs_cull_masks (both optional). */
+int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
+    const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
+    float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
+    uint32_t* keep_masks, void* stream);
+
 /* gs_preprocess_backward -- gaussian_preprocess.cu:567-636 (kernel :246-372, with gaussian_compute_cov2D.cu:64-186 and
  * gaussian_compute_cov3D.cu:76-118). grad_mean2D[P,2] is rewritten in place as (0.5 W g.x, +-0.5 H g.y) as in the
  * reference; grad_conic[P,4] carries dL/dconic and dL/dopacity. All gradient rows are assigned (zeros for Gaussians

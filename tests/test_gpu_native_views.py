@@ -148,3 +148,53 @@ def test_fast_surfel_view_equals_operators(P, W, H, mode, device):
                               up + ([torch.ones_like(flow)] if flow is not None else []))
     for a, b in zip(got, ref):
         assert (a - b).norm() <= 1e-5 * b.norm() + 1e-7
+
+
+@pytest.mark.parametrize('P,W,H,mode', [(1, 16, 16, 'sh'), (257, 49, 31, 'split'), (256, 64, 48, 'colors'),
+                                        (300, 49, 31, 'extras'), (16_385, 161, 99, 'culling'), (3_000, 120, 90, 'opengl'),
+                                        (3_000, 120, 90, 'later')])
+def test_gaussian_view_equals_operators(P, W, H, mode, device):
+    """Maps bit for bit; gradients to the order of the sums over a Gaussian's tiles. 'later': a further table blended with
+    the view's weights, whose gradient reaches the geometry through the buffer."""
+    import math
+
+    from fast_sp_gs_amd.renderer import gaussian_render as m
+    s, cam_h, g = _scene(P, W, H, P + 3)
+    cam = cam_h.to(device)
+    third = torch.exp(torch.randn(P, 1, generator=g) * 0.5 - 4.2)
+    params = _leaves(device, s.means3D, torch.cat([s.scales, third], dim=1), s.rotations, s.opacities)
+    rest = extras = table = None
+    if mode == 'split':
+        sh, rest = _leaves(device, s.shs[:, :1].contiguous(), s.shs[:, 1:].contiguous())
+    else:
+        sh, = _leaves(device, s.shs[:, 0].contiguous() if mode == 'colors' else s.shs)
+    if mode == 'extras':
+        extras, = _leaves(device, torch.randn(P, 3, generator=g))
+    if mode == 'later':
+        table, = _leaves(device, torch.randn(P, 6, generator=g))
+    culling = (torch.rand(P, generator=g) < 0.3).to(device) if mode == 'culling' else None
+    tan = (math.tan(math.radians(25.0)), math.tan(math.radians(25.0)) * H / W)
+    out = m.render(cam.Tw2v, cam.Tv2c, (W, H), params[0], params[3], params[1], params[2], campos=cam.campos,
+                   FoV=tuple(2 * math.atan(t) for t in tan), sh_degree=3, is_opengl=mode == 'opengl', culling=culling,
+                   colors=sh if mode == 'colors' else None, sh_features=None if mode == 'colors' else sh,
+                   sh_features_rest=rest, **({} if extras is None else {'feature': extras}))
+    m2 = torch.zeros(P, 2, device=device, requires_grad=True)
+    img, opac, maps, radii, buf, visible = m._rasterize_operators(
+        params[0], m2, sh, rest, params[3], params[1], params[2], None, None, extras, (W, H), -1 if mode == 'colors' else 3,
+        cam.Tw2v, cam.Tv2c, cam.campos, tan, mode == 'opengl', culling, None, None, None)
+    same = lambda a, b: a.shape == b.shape and torch.equal(a, b)
+    assert same(out['images'], img) and same(out['opacity'], opac) and same(out['radii'], radii)
+    assert same(out['visibility_filter'], visible) and same(out['viewspace_points'], m2)
+    assert same(out['buffer'].conic_opacity, buf.conic_opacity) and same(out['buffer'].n_contribed, buf.n_contribed)
+    got_maps, ref_maps = [out['images'], out['opacity']], [img, opac]
+    wanted = params + [sh] + [t for t in (rest, extras, table) if t is not None]
+    if extras is not None:
+        assert same(out['feature'], maps)
+        got_maps, ref_maps = got_maps + [out['feature']], ref_maps + [maps]
+    if table is not None:
+        got_maps, ref_maps = got_maps + [m.render_extra(out['buffer'], table)], ref_maps + [m.render_extra(buf, table)]
+    up = [torch.randn(t.shape, generator=g).to(device) for t in got_maps]
+    got = torch.autograd.grad(got_maps, wanted + [out['viewspace_points']], up)
+    ref = torch.autograd.grad(ref_maps, wanted + [m2], up)
+    for a, b in zip(got, ref):
+        assert (a - b).norm() <= 1e-4 * b.norm() + 1e-7
