@@ -1198,7 +1198,7 @@ def lbs_blend(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Tensor, sp_
     ws = _workspace(lib.fsgs_lbs_blend_workspace_bytes(M), points.device)
     with _timed('lbs_blend'):
         rc = lib.fsgs_lbs_blend(N, M, K, warp, weight, float(temperature), L.ptr(points), L.ptr(sp_points),
-                                L.ptr(sp_t), L.ptr(sp_rot), L.ptr(sp_r), L.ptr(sp_s), S, L.ptr(pair_in), L.ptr(index),
+                                L.ptr(sp_t), L.ptr(sp_rot), L.ptr(sp_r), L.ptr(sp_s), S, S, L.ptr(pair_in), L.ptr(index),
                                 L.ptr(sp_log_radius) if weight == 1 else None,
                                 L.ptr(sp_weight_logit) if weight == 1 else None, L.ptr(weights), L.ptr(d_xyz),
                                 L.ptr(d_rot), L.ptr(d_scale), L.ptr(ws), ws.numel(), L.current_stream())
@@ -1243,10 +1243,10 @@ def lbs_blend_backward(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Te
     with _timed('lbs_blend_backward'):
         rc = lib.fsgs_lbs_blend_backward(
             N, M, K, warp, weight, float(temperature), L.ptr(points), L.ptr(sp_points), L.ptr(sp_t), L.ptr(sp_rot),
-            L.ptr(sp_r), L.ptr(sp_s), S, L.ptr(pair_in), L.ptr(index), L.ptr(sp_log_radius) if weight == 1 else None,
+            L.ptr(sp_r), L.ptr(sp_s), S, S, L.ptr(pair_in), L.ptr(index), L.ptr(sp_log_radius) if weight == 1 else None,
             L.ptr(sp_weight_logit) if weight == 1 else None, L.ptr(grad_xyz), L.ptr(grad_rot), L.ptr(grad_scale),
             L.ptr(g_points), L.ptr(g_pair), L.ptr(g_sp_points), L.ptr(g_sp_t), L.ptr(g_sp_rot), L.ptr(g_sp_r),
-            L.ptr(g_sp_s), L.ptr(g_rad), L.ptr(g_wl), L.ptr(ws), ws.numel(), L.current_stream())
+            L.ptr(g_sp_s), S, L.ptr(g_rad), L.ptr(g_wl), L.ptr(ws), ws.numel(), L.current_stream())
     L.check(rc, what)
     return dict(g_points=g_points, g_pair=g_pair, g_sp_points=g_sp_points, g_sp_t=g_sp_t, g_sp_rot=g_sp_rot,
                 g_sp_r=g_sp_r, g_sp_s=g_sp_s, g_log_radius=g_rad, g_weight_logit=g_wl)
@@ -1346,7 +1346,8 @@ def mlp_forward(inputs: Tensor, packed: Tensor, bias: Tensor, n_layers: int, ski
                 save: bool = False):
     """Fused n_layers x (Linear(256)+ReLU) + heads forward on the matrix cores (bf16 in, fp32 accumulate);
     network.py:1757-1776. inputs[B,Din] fp32, bias[n_layers*256 + n_out] fp32 -> out[B,n_out] fp32; with `save` also
-    the [n_layers,B,256] bf16 (stored as int16) post-ReLU states that `mlp_backward` needs -> (out, saved)."""
+    the [n_layers,B,256] bf16 (stored as int16, batch innermost) post-ReLU states that `mlp_backward` needs -> (out,
+    saved)."""
     what = 'mlp_forward'
     _f32(what, inputs=inputs, bias=bias)
     L.require_cuda(what, packed=packed)
@@ -1355,14 +1356,23 @@ def mlp_forward(inputs: Tensor, packed: Tensor, bias: Tensor, n_layers: int, ski
         raise RuntimeError(f'{what}: bias must have {n_layers * 256 + n_out} elements')
     if packed.numel() != _lib().fsgs_mlp_packed_elems(Din, n_layers, skip):
         raise RuntimeError(f'{what}: packed weight buffer has the wrong size')
+    lib = _lib()
     out = torch.empty((B, n_out), dtype=torch.float32, device=inputs.device)
-    saved = torch.empty((n_layers, B, 256), dtype=torch.int16, device=inputs.device) if save else None
+    saved = saved_in = None
+    if save:
+        B_pad = _mlp_rows(B)
+        saved_in = torch.empty((Din, B_pad), dtype=torch.int16, device=inputs.device)
+        saved = torch.empty((n_layers, 256, B_pad), dtype=torch.int16, device=inputs.device)
     with _timed('mlp_forward'):
-        rc = _lib().fsgs_mlp_forward(B, Din, 256, n_layers, skip, n_out, L.ptr(inputs),
-                                     L.ptr(packed), L.ptr(bias),
-                                     L.ptr(out), L.ptr(saved), L.current_stream())
+        rc = lib.fsgs_mlp_forward(B, Din, 256, n_layers, skip, n_out, L.ptr(inputs), L.ptr(packed), L.ptr(bias),
+                                  L.ptr(out), L.ptr(saved_in), L.ptr(saved), L.current_stream())
     L.check(rc, what)
-    return (out, saved) if save else out
+    # the kernels keep the batch innermost; callers see [n_layers, B, 256]
+    return (out, saved[:, :, :B].transpose(1, 2)) if save else out
+
+
+def _mlp_rows(B: int) -> int:
+    return max(B + 31, 32) // 32 * 32
 
 
 def mlp_pack_transposed(weights: List[Tensor]) -> Tensor:
@@ -1387,7 +1397,9 @@ def mlp_backward(inputs: Tensor, packed_t: Tensor, head_weights: Tensor, saved: 
     forms the gradient of the network's input (dZ_0 W_0 + dZ_{skip+1} W_{skip+1}[:, :Din])."""
     what = 'mlp_backward'
     _f32(what, inputs=inputs, head_weights=head_weights, grad_out=grad_out)
-    L.require_cuda(what, packed_t=packed_t, saved=saved)
+    L.require_cuda(what, packed_t=packed_t)
+    if not saved.is_cuda:
+        raise RuntimeError(f'{what}: saved must be a CUDA tensor')
     B, Din = inputs.shape
     n_out = head_weights.shape[0]
     if tuple(saved.shape) != (n_layers, B, 256) or saved.dtype != torch.int16:
@@ -1396,18 +1408,24 @@ def mlp_backward(inputs: Tensor, packed_t: Tensor, head_weights: Tensor, saved: 
         raise RuntimeError(f'{what}: grad_out / head_weights shapes do not match')
     if packed_t.numel() < max(n_layers - 1, 1) * 65536:
         raise RuntimeError(f'{what}: packed_t is too small for {n_layers} layers')
+    B_pad = _mlp_rows(B)
+    if B and saved.stride() != (256 * B_pad, 1, B_pad):  # not as the forward left it
+        laid_out = saved.new_zeros((n_layers, 256, B_pad))
+        laid_out[:, :, :B] = saved.transpose(1, 2)
+        saved = laid_out
     n_w = 256 * Din + (n_layers - 1) * 65536 + 256 * Din + n_out * 256
     g = torch.empty((n_w + n_layers * 256 + n_out,), dtype=torch.float32, device=inputs.device)
     g_w, g_b = g[:n_w], g[n_w:]
     lib = _lib()
-    ws = _workspace(lib.fsgs_mlp_backward_workspace_bytes(B, n_layers), inputs.device)
+    ws = _workspace(lib.fsgs_mlp_backward_workspace_bytes(B, Din, n_layers), inputs.device)
     with _timed('mlp_backward'):
         rc = lib.fsgs_mlp_backward(B, Din, 256, n_layers, skip, n_out, L.ptr(inputs), L.ptr(packed_t),
                                    L.ptr(head_weights), L.ptr(saved), L.ptr(grad_out), L.ptr(g_w), L.ptr(g_b),
                                    L.ptr(ws), ws.numel(), L.current_stream())
     L.check(rc, what)
     if return_dz:
-        return g_w, g_b, ws[:n_layers * B * 256 * 2].view(torch.bfloat16).view(n_layers, B, 256)
+        dz = ws[:n_layers * B_pad * 256 * 2].view(torch.bfloat16).view(n_layers, 256, B_pad)
+        return g_w, g_b, dz[:, :, :B].transpose(1, 2)
     return g_w, g_b
 
 

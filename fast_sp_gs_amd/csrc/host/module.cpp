@@ -1,6 +1,7 @@
 // Python entry points of the native host layer (fast_sp_gs_amd._host).
 #include <torch/csrc/utils/pybind.h>
 
+#include "deform.hpp"
 #include "fast_surfel.hpp"
 #include "gaussian.hpp"
 #include "surfel.hpp"
@@ -56,10 +57,39 @@ py::tuple gaussian_render_py(const Tensor& points, const Tensor& scales, const T
   return py::make_tuple(r.maps, r.n_contrib, r.radii, r.visible, r.ranges, r.point_list);
 }
 
+py::object or_none(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
+
+py::tuple superpoint_warp_py(const Tensor& points, const Tensor& sp_points, const Tensor& sp_t, const Tensor& sp_r,
+                             const OptTensor& sp_s, const OptTensor& sp_rot, const OptTensor& sp_radius,
+                             const OptTensor& sp_weight, int scale_columns, int64_t K, double temperature, int warp_mode,
+                             int weight_mode) {
+  const SuperpointWarp w{points, sp_points, sp_t, sp_r, sp_s, sp_rot, sp_radius, sp_weight, scale_columns, K, temperature,
+                         warp_mode, weight_mode};
+  const variable_list r = without_gil([&] { return superpoint_warp(w); });
+  return py::make_tuple(r[0], r[1], or_none(r[2]), r[3], r[4]);
+}
+
+variable_list deform_mlp_py(const Tensor& x, const Tensor& t, const OptTensor& in, const Tensor& packed, const Tensor& bias,
+                            const OptTensor& packed_t, const OptTensor& heads_w, int degree_x, double scale_x, int degree_t,
+                            double scale_t, int n_layers, int skip, const std::vector<int>& head_rows,
+                            const std::vector<Tensor>& params) {
+  const DeformMlp m{x, t, in, packed, bias, packed_t, heads_w, degree_x, degree_t, n_layers, skip, scale_x, scale_t, head_rows};
+  return without_gil([&] { return deform_mlp(m, params); });
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
   m.def("surfel_render", &surfel_render_py);
   m.def("fast_surfel_render", &fast_surfel_render_py);
   m.def("gaussian_render", &gaussian_render_py);
+  m.def("superpoint_warp", &superpoint_warp_py);
+  m.def("deform_mlp", &deform_mlp_py);
+  const auto released = py::call_guard<py::gil_scoped_release>();
+  m.def("knn_points", &knn_points, released);
+  m.def("deform_apply", &deform_apply, released);
+  m.def("mlp_pack", &mlp_pack, released);
+  m.def("image_loss", &image_loss, released);
+  m.def("adam_masked", &adam_masked, released);
+  m.def("adam_dense", &adam_dense, released);
 }

@@ -50,7 +50,7 @@ struct LbsPoint {
   float w[kMaxK], X[kMaxK];
 };
 template <int kMaxK>
-__device__ __forceinline__ void lbs_point_backward(int n, int M, int K, int S, int warp_mode, int weight_mode,
+__device__ __forceinline__ void lbs_point_backward(int n, int M, int K, int S, int sp_s_ld, int warp_mode, int weight_mode,
     float inv_t, const float* __restrict__ points, const float* __restrict__ xf, const float* __restrict__ sp_r,
     const float* __restrict__ sp_s, const float* __restrict__ pair_in, const int64_t* __restrict__ index,
     const float* __restrict__ g_xyz, const float* __restrict__ g_rot, const float* __restrict__ g_scale,
@@ -89,7 +89,7 @@ __device__ __forceinline__ void lbs_point_backward(int n, int M, int K, int S, i
     for (int a = 0; a < 4; ++a) vk += P.gr[a] * sp_r[4 * j + a];
 #pragma unroll
     for (int a = 0; a < 4; ++a)
-      if (a < S) vk += P.gs[a] * sp_s[(size_t) S * j + a];
+      if (a < S) vk += P.gs[a] * sp_s[(size_t) sp_s_ld * j + a];
     v[k] = vk, P.w[k] = w;
     dot += w * vk;
   }
@@ -120,7 +120,7 @@ __device__ __forceinline__ void lbs_point_backward(int n, int M, int K, int S, i
 // kMode 0: atomics into a zeroed accumulator in global memory. 1: block-private table in LDS, stored as one partial.
 constexpr int kStageTable = 11264;  // table floats of the binned variant below (44 KB: 512 control points x 22 columns)
 template <int kMode>
-__global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(int N, int M, int K, int S,
+__global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(int N, int M, int K, int S, int sp_s_ld,
     int warp_mode, int weight_mode, float temperature, const float* __restrict__ points, const float* __restrict__ xf,
     const float* __restrict__ sp_r, const float* __restrict__ sp_s, const float* __restrict__ pair_in,
     const int64_t* __restrict__ index, const float* __restrict__ g_xyz, const float* __restrict__ g_rot,
@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(in
   const float inv_t = 1.0f / temperature;
   for (int n = blockIdx.x * kAccThreads + threadIdx.x; n < N; n += gridDim.x * kAccThreads) {
     LbsPoint<16> P;
-    lbs_point_backward<16>(n, M, K, S, warp_mode, weight_mode, inv_t, points, xf, sp_r, sp_s, pair_in, index, g_xyz,
+    lbs_point_backward<16>(n, M, K, S, sp_s_ld, warp_mode, weight_mode, inv_t, points, xf, sp_r, sp_s, pair_in, index, g_xyz,
                            g_rot, g_scale, g_points, g_pair, P);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(in
 // one lane over its control point's bin from the points' gradients parked in LDS. Partial tables go out as in mode 1.
 constexpr int kBinK = 4;
 constexpr int kBinFeat = 14;  // g[3] p[3] g_rot[4] g_scale[<= 4] per point
-__global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N, int M, int K, int S, int warp_mode,
+__global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N, int M, int K, int S, int sp_s_ld, int warp_mode,
     int weight_mode, float temperature, const float* __restrict__ points, const float* __restrict__ xf,
     const float* __restrict__ sp_r, const float* __restrict__ sp_s, const float* __restrict__ pair_in,
     const int64_t* __restrict__ index, const float* __restrict__ g_xyz, const float* __restrict__ g_rot,
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N,
     __syncthreads();
     LbsPoint<kBinK> P;
     if (live) {
-      lbs_point_backward<kBinK>(n, M, K, S, warp_mode, weight_mode, inv_t, points, xf, sp_r, sp_s, pair_in, index,
+      lbs_point_backward<kBinK>(n, M, K, S, sp_s_ld, warp_mode, weight_mode, inv_t, points, xf, sp_r, sp_s, pair_in, index,
                                 g_xyz, g_rot, g_scale, g_points, g_pair, P);
       float* ft = s_feat[tid];
 #pragma unroll
@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(512) partial_sum_kernel(int cells, int G, cons
   }
 }
 
-__global__ void __launch_bounds__(256) lbs_backward_finish_kernel(int M, int S, int warp_mode, int weight_mode,
+__global__ void __launch_bounds__(256) lbs_backward_finish_kernel(int M, int S, int g_sp_s_ld, int warp_mode, int weight_mode,
     const float* __restrict__ sp_points, const float* __restrict__ xf, const float* __restrict__ acc,
     float* __restrict__ g_sp_points, float* __restrict__ g_sp_t, float* __restrict__ g_sp_rot,
     float* __restrict__ g_sp_r, float* __restrict__ g_sp_s, float* __restrict__ g_log_radius,
@@ -369,7 +369,8 @@ __global__ void __launch_bounds__(256) lbs_backward_finish_kernel(int M, int S, 
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) g_sp_r[4 * j + k] = a[C.oR + k];
-  for (int k = 0; k < S; ++k) g_sp_s[(size_t) S * j + k] = a[C.oS + k];
+  if (S > 0)
+    for (int k = 0; k < g_sp_s_ld; ++k) g_sp_s[(size_t) g_sp_s_ld * j + k] = k < S ? a[C.oS + k] : 0.0f;
   if (weight_mode == 1) {
     // u = e * sig + 1e-7 with e = exp(-d2 * i2), i2 = 1 / (2 r^2), r = exp(rho): du/drho = e sig d2 2 i2, du/domega =
     // e sig (1 - sig)
@@ -409,11 +410,12 @@ FSGS_API size_t fsgs_lbs_blend_backward_workspace_bytes(int N, int M, int S) {
 
 FSGS_API int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
     const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
-    const float* sp_s, int S, const float* pair_in, const int64_t* index, const float* sp_log_radius,
+    const float* sp_s, int S, int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius,
     const float* sp_weight_logit, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_points,
-    float* g_pair, float* g_sp_points, float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s,
+    float* g_pair, float* g_sp_points, float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s, int g_sp_s_ld,
     float* g_log_radius, float* g_weight_logit, void* workspace, size_t workspace_bytes, void* stream) {
-  FSGS_REQUIRE(N >= 0 && M > 0 && K > 0 && K <= 16 && S >= 0 && S <= 4, "lbs_blend_backward: bad sizes (K <= 16, S <= 4)");
+  FSGS_REQUIRE(N >= 0 && M > 0 && K > 0 && K <= 16 && S >= 0 && S <= 4 && sp_s_ld >= S && g_sp_s_ld >= S,
+               "lbs_blend_backward: bad sizes (K <= 16, S <= 4)");
   FSGS_REQUIRE(warp_mode >= 0 && warp_mode <= 2 && weight_mode >= 0 && weight_mode <= 3,
                "lbs_blend_backward: unknown mode");
   FSGS_REQUIRE(sp_points && sp_t && sp_r && g_sp_t && g_sp_r && (S == 0 || (sp_s && g_scale && g_sp_s)) && workspace,
@@ -444,18 +446,18 @@ FSGS_API int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int wei
     if (plan.lds) {
       const bool binned = cells <= kStageTable && M <= kAccThreads && K <= kBinK;
       auto kernel = binned ? lbs_backward_binned_kernel : lbs_backward_accumulate_kernel<1>;
-      hipLaunchKernelGGL(kernel, dim3(plan.blocks), dim3(kAccThreads), 0, s, N, M, K, S, warp_mode, weight_mode,
-                         (float) temperature, points, xf, sp_r, sp_s, pair_in, index, g_xyz, g_rot, g_scale, g_points,
+      hipLaunchKernelGGL(kernel, dim3(plan.blocks), dim3(kAccThreads), 0, s, N, M, K, S, sp_s_ld, warp_mode,
+                         weight_mode, (float) temperature, points, xf, sp_r, sp_s, pair_in, index, g_xyz, g_rot, g_scale, g_points,
                          g_pair, partial);
       hipLaunchKernelGGL(partial_sum_kernel, dim3(div_up(cells, kWave)), dim3(512), 0, s, cells, plan.blocks, partial,
                          acc);
     } else {
       hipLaunchKernelGGL(lbs_backward_accumulate_kernel<0>, dim3(plan.blocks), dim3(kAccThreads), 0, s, N, M, K, S,
-                         warp_mode, weight_mode, (float) temperature, points, xf, sp_r, sp_s, pair_in, index, g_xyz,
+                         sp_s_ld, warp_mode, weight_mode, (float) temperature, points, xf, sp_r, sp_s, pair_in, index, g_xyz,
                          g_rot, g_scale, g_points, g_pair, acc);
     }
   }
-  hipLaunchKernelGGL(lbs_backward_finish_kernel, dim3(div_up(M, 256)), dim3(256), 0, s, M, S, warp_mode, weight_mode,
+  hipLaunchKernelGGL(lbs_backward_finish_kernel, dim3(div_up(M, 256)), dim3(256), 0, s, M, S, g_sp_s_ld, warp_mode, weight_mode,
                      sp_points, xf, acc, g_sp_points, g_sp_t, g_sp_rot, g_sp_r, g_sp_s, g_log_radius, g_weight_logit);
   return check_launch("lbs_blend_backward");
 }

@@ -10,17 +10,24 @@
 // Each of the 8 wavefronts computes a 32 x 32 slab of a layer's output with v_mfma_f32_32x32x16_bf16: A fragments
 // (activations) come from LDS as one 16-byte read per lane, B fragments (weights, packed in fragment order, see
 // frag_index) as one 16-byte global read per lane; both use the same (lane / 32, element) -> k mapping, so the product
-// is independent of how the hardware orders k inside a fragment.
+// is independent of how the hardware orders k inside a fragment. The input rows are either given or formed here from
+// positions and time (the frequency encoding), which spares three launches and a [B][84] tensor.
 //
-// Training: the forward optionally stores every layer's post-ReLU hidden state (bf16, [layer][B][256]). The backward
-// (the reference leaves it to torch autograd: one addmm-backward pair and a ReLU mask per layer, ~30 launches) is two
-// kernels:
+// Training: the forward optionally stores every layer's post-ReLU hidden state and the input rows, in bf16 and with the
+// batch innermost ([layer][256][B_pad], B_pad = B rounded up to 32): an accumulator's four consecutive registers are four
+// consecutive rows of one column, so that layout takes 8-byte stores, and it is what the weight gradients read. The
+// backward (the reference leaves it to torch autograd: one addmm-backward pair and a ReLU mask per layer, ~30 launches)
+// is two kernels:
 //   * a chain kernel with the forward's structure, one block per 32 rows: dZ_L-1 = (g_out . W_heads) masked by the saved
 //     state, then for each layer dH_l-1 = dZ_l . W_l[:, hidden part] on the matrix cores against a transposed bf16 copy
-//     of the weights, masked, kept in LDS for the next layer and written to HBM as dZ[l][B][256];
-//   * a weight-gradient kernel over all layers at once: every block owns a 32 x 128 tile of one layer's dW = dZ^T X,
-//     walks the batch in 32-row chunks transposed through LDS, and the first tile column of a layer also sums dZ over
-//     the batch for the bias gradient. No atomics: every output element has one writer.
+//     of the weights, masked, kept in LDS for the next layer and written to HBM as dZ[l][256][B_pad];
+//   * a weight-gradient kernel over all layers at once, dW = dZ^T X: with the batch innermost both operands' fragments are
+//     16-byte loads of consecutive memory. A block owns a 64 x 64 tile, its four wavefronts take a share of the batch each
+//     with every load of 128 rows in flight, and add their sums through LDS in wavefront order; the first tile column of a
+//     layer also sums dZ over the batch for the bias gradient. No atomics: every output element has one writer.
+// Both chains are bound by latency: 16 blocks at B = 512, nine dependent layers. At B = 512, 8 layers (us): forward 48,
+// chain 42, weight gradients 48 before the loads of a layer were ordered so that none waits for the next layer's
+// prefetched weights and the weight gradients' operands went through LDS transposed two bytes at a time.
 // Gradients with respect to the (frequency-encoded) input are not produced; the reference detaches it
 // (network.py:586).
 #include <algorithm>
@@ -97,31 +104,68 @@ __global__ void __launch_bounds__(256) pack_jobs_kernel(PackTable table) {
   ((uint16_t*) j.dst)[frag_index(j.dst_row0 + r, k, j.K_pad)] = f32_to_bf16(v);
 }
 
+__global__ void __launch_bounds__(256) fill_zero_kernel(size_t n, float* __restrict__ p) {
+  for (size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t) gridDim.x * blockDim.x) p[i] = 0.0f;
+}
+
 // D layout of the 32x32 accumulator: register r of lane l holds row 8 * (r / 4) + 4 * (l / 32) + (r % 4), column l % 32.
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
+__device__ __forceinline__ int div_up_dev(int a, int b) { return (a + b - 1) / b; }
+
+constexpr int kMaxHeads = 8;
+struct MlpHeads {  // the outputs' (or their gradients') columns: head h is [B][width[h]] and holds columns first[h] ..
+  float* at[kMaxHeads];
+  int first[kMaxHeads + 1];
+  int n;
+};
+__device__ __forceinline__ float* head_cell(const MlpHeads& h, int row, int col) {
+  int q = 0;
+#pragma unroll
+  for (int k = 1; k < kMaxHeads; ++k) q += (k < h.n && col >= h.first[k]) ? 1 : 0;
+  float* base = h.at[0];
+  int first = h.first[0], width = h.first[1];
+#pragma unroll
+  for (int k = 1; k < kMaxHeads; ++k)
+    if (q == k) base = h.at[k], first = h.first[k], width = h.first[k + 1] - h.first[k];
+  return base ? base + (size_t) row * width + (col - first) : nullptr;
+}
+
+// The frequency encoding of positions x[B,3] and one time t[1]: [x | sin 2^d s x, cos 2^d s x ...] then the same for t.
+struct FreqInput {
+  const float* x;
+  const float* t;
+  int degree_x, degree_t;
+  float scale_x, scale_t;
+};
+__device__ __forceinline__ float encoded(const FreqInput& f, int row, int k) {
+  const int wide = 3 * (1 + 2 * f.degree_x);
+  int q;
+  float v, scale;
+  if (k < wide) q = k / 3, v = f.x[3 * (size_t) row + (k - 3 * q)], scale = f.scale_x;
+  else q = k - wide, v = f.t[0], scale = f.scale_t;
+  if (q == 0) return v;
+  v = ldexpf(v * scale, (q - 1) >> 1);
+  return ((q - 1) & 1) ? cosf(v) : sinf(v);
+}
+
+__device__ __forceinline__ uint2 pack4(const uint16_t* h) {
+  return make_uint2((uint32_t) h[0] | ((uint32_t) h[1] << 16), (uint32_t) h[2] | ((uint32_t) h[3] << 16));
+}
+
+// `in` or `freq.x` gives the input rows. in_t / saved (kSave): see the file's head.
 template <bool kSave>
 __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int Din, int n_layers, int skip, int n_out,
-    const float* __restrict__ in, const uint16_t* __restrict__ packed, const float* __restrict__ bias,
-    float* __restrict__ out, uint16_t* __restrict__ saved) {
+    const float* __restrict__ in, FreqInput freq, const uint16_t* __restrict__ packed, const float* __restrict__ bias,
+    MlpHeads heads, uint16_t* __restrict__ in_t, uint16_t* __restrict__ saved) {
   __shared__ __attribute__((aligned(16))) uint16_t s_act[2][kMlpRows][kMlpStride];
   __shared__ __attribute__((aligned(16))) uint16_t s_in[kMlpRows][kMlpMaxIn + 8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * kMlpRows;
   const int Din_pad = (Din + 15) & ~15;
+  const size_t B_pad = (size_t) gridDim.x * kMlpRows;
+  const int arow = lane & 31, kofs = 8 * (lane >> 5), col = wave * 32 + (lane & 31);
 
-  // stage the (bf16) input rows, zero padded
-  for (int e = threadIdx.x; e < kMlpRows * Din_pad; e += kChainThreads) {
-    const int r = e / Din_pad, k = e - r * Din_pad;
-    const float v = (row0 + r < B && k < Din) ? in[(size_t) (row0 + r) * Din + k] : 0.0f;
-    const uint16_t h = f32_to_bf16(v);
-    s_in[r][k] = h;
-    s_act[0][r][k] = h;
-  }
-  __syncthreads();
-
-  int cur = 0;
-  int K = Din, K_pad = Din_pad;
   const uint16_t* W = packed;
   const float* bl   = bias;
   // Fragment u (k-step u, clamped to the layer's last step) of row tile `wave` of a layer whose weights start at Wl;
@@ -130,304 +174,330 @@ __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int D
     const int steps = K_pad_l >> 4;
     return *(const bf16x8*) (Wl + ((size_t) wave * steps + min(u, steps - 1)) * 512 + lane * 8);
   };
-  // The weights do not depend on the activations: the first sixteen fragments of the NEXT layer are requested at the
-  // start of each layer and arrive while this layer's products, epilogue and barrier run.
+  // The weights do not depend on the activations: the first sixteen fragments (and the bias) of the NEXT layer are
+  // requested at the start of each layer and arrive while this layer's products, epilogue and barrier run. Nothing else is
+  // loaded behind them: loads complete in order, and a wait for a later one would be a wait for all of these.
   bf16x8 ahead[16];
+  float bias_ahead = bl[col];
 #pragma unroll
-  for (int u = 0; u < 16; ++u) ahead[u] = fragment(W, K_pad, u);
+  for (int u = 0; u < 16; ++u) ahead[u] = fragment(W, Din_pad, u);
+
+  // stage the (bf16) input rows, zero padded
+  for (int e = threadIdx.x; e < kMlpRows * Din_pad; e += kChainThreads) {
+    const int r = e / Din_pad, k = e - r * Din_pad;
+    float v = 0.0f;
+    if (row0 + r < B && k < Din) v = in ? in[(size_t) (row0 + r) * Din + k] : encoded(freq, row0 + r, k);
+    const uint16_t h = f32_to_bf16(v);
+    s_in[r][k] = h;
+    s_act[0][r][k] = h;
+  }
+  __syncthreads();
+  if (kSave) {
+    for (int e = threadIdx.x; e < Din * (kMlpRows / 4); e += kChainThreads) {
+      const int k = e >> 3, r = (e & 7) * 4;
+      const uint16_t h[4] = {s_in[r][k], s_in[r + 1][k], s_in[r + 2][k], s_in[r + 3][k]};
+      *(uint2*) (in_t + (size_t) k * B_pad + row0 + r) = pack4(h);
+    }
+  }
+
+  int cur = 0, K_pad = Din_pad;
   for (int layer = 0; layer < n_layers; ++layer) {
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    const int arow = lane & 31, kofs = 8 * (lane >> 5);
-    const uint16_t* wrow = W + (size_t) wave * (K_pad >> 4) * 512 + lane * 8;
-    bf16x8 b[16];
+    bf16x8 b[16], tail[6];
+    const float bv = bias_ahead;
 #pragma unroll
     for (int u = 0; u < 16; ++u) b[u] = ahead[u];
+    const int steps = K_pad >> 4;
+    if (steps > 16) {  // the layer behind the re-concatenated input: up to six k-steps more
+#pragma unroll
+      for (int u = 0; u < 6; ++u) tail[u] = fragment(W, K_pad, 16 + u);
+    }
+    const int K_next = layer == skip ? Din + kMlpWidth : kMlpWidth, K_next_pad = (K_next + 15) & ~15;
+    const uint16_t* W_next = W + (size_t) kMlpWidth * K_pad;
     if (layer + 1 < n_layers) {
-      const int K_after = (((layer == skip) ? Din + kMlpWidth : kMlpWidth) + 15) & ~15;
+      bias_ahead = bl[kMlpWidth + col];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) ahead[u] = fragment(W + (size_t) kMlpWidth * K_pad, K_after, u);
+      for (int u = 0; u < 16; ++u) ahead[u] = fragment(W_next, K_next_pad, u);
     }
-    const int first = min(K_pad >> 4, 16);
+    const uint16_t* arow_at = &s_act[cur][arow][kofs];
+    if (steps >= 16) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if (u < first) {
-        const bf16x8 a = *(const bf16x8*) &s_act[cur][arow][16 * u + kofs];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[u], acc, 0, 0, 0);
+      for (int u = 0; u < 16; ++u)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 16 * u), b[u], acc, 0, 0, 0);
+      if (steps > 16) {
+#pragma unroll
+        for (int u = 0; u < 6; ++u)
+          if (16 + u < steps)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 256 + 16 * u), tail[u], acc, 0, 0, 0);
       }
-    int k0 = 16 * first;
-    for (; k0 + 64 <= K_pad; k0 += 64) {
-      bf16x8 b[4];
+    } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) b[u] = *(const bf16x8*) (wrow + (k0 + 16 * u) * 32);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const bf16x8 a = *(const bf16x8*) &s_act[cur][arow][k0 + 16 * u + kofs];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[u], acc, 0, 0, 0);
-      }
-    }
-    for (; k0 < K_pad; k0 += 16) {
-      const bf16x8 a = *(const bf16x8*) &s_act[cur][arow][k0 + kofs];
-      const bf16x8 b = *(const bf16x8*) (wrow + k0 * 32);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+      for (int u = 0; u < 6; ++u)
+        if (u < steps)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 16 * u), b[u], acc, 0, 0, 0);
     }
     // bias + ReLU -> bf16 into the other buffer; after the skip layer the input goes in front of the hidden state
     const int nxt = cur ^ 1;
     const int col_shift = (layer == skip) ? Din : 0;
-    {
-      const int col  = wave * 32 + (lane & 31);
-      const float bv = bl[col];
+    uint16_t h[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float v    = fmaxf(acc[r] + bv, 0.0f);
-        const uint16_t h = f32_to_bf16(v);
-        const int row    = acc_row(r, lane);
-        s_act[nxt][row][col_shift + col] = h;
-        if (kSave && row0 + row < B) saved[((size_t) layer * B + row0 + row) * kMlpWidth + col] = h;
-      }
+    for (int r = 0; r < 16; ++r) {
+      h[r] = f32_to_bf16(fmaxf(acc[r] + bv, 0.0f));
+      s_act[nxt][acc_row(r, lane)][col_shift + col] = h[r];
     }
-    int K_next = kMlpWidth;
+    if (kSave) {
+      uint16_t* dst = saved + ((size_t) layer * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) *(uint2*) (dst + 8 * g) = pack4(h + 4 * g);
+    }
     if (layer == skip) {
-      K_next = Din + kMlpWidth;
       for (int e = threadIdx.x; e < kMlpRows * Din; e += kChainThreads) {
         const int r = e / Din, k = e - r * Din;
         s_act[nxt][r][k] = s_in[r][k];
       }
-    }
-    const int K_next_pad = (K_next + 15) & ~15;
-    for (int e = threadIdx.x; e < kMlpRows * (K_next_pad - K_next); e += kChainThreads) {
-      const int r = e / (K_next_pad - K_next), k = e - r * (K_next_pad - K_next);
-      s_act[nxt][r][K_next + k] = 0;
+      for (int e = threadIdx.x; e < kMlpRows * 16; e += kChainThreads)
+        if (K_next + (e & 15) < K_next_pad) s_act[nxt][e >> 4][K_next + (e & 15)] = 0;
     }
     lds_barrier();
-    W += (size_t) kMlpWidth * K_pad;
+    W = W_next;
     bl += kMlpWidth;
-    K = K_next, K_pad = K_next_pad;
+    K_pad = K_next_pad;
     cur = nxt;
   }
-  (void) K;
 
   // heads: one padded 32-column tile, wavefront 0 only
   if (wave == 0) {
+    const int head_col = lane & 31;
+    const float bv = head_col < n_out ? bl[head_col] : 0.0f;
+    bf16x8 b[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) b[u] = *(const bf16x8*) (W + u * 512 + lane * 8);
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    const int arow = lane & 31, kofs = 8 * (lane >> 5);
-    const uint16_t* wrow = W + lane * 8;
-    for (int k0 = 0; k0 < K_pad; k0 += 16) {
-      const bf16x8 a = *(const bf16x8*) &s_act[cur][arow][k0 + kofs];
-      const bf16x8 b = *(const bf16x8*) (wrow + k0 * 32);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    const int col = lane & 31;
-    if (col < n_out) {
-      const float bv = bl[col];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) &s_act[cur][arow][kofs + 16 * u], b[u], acc, 0, 0, 0);
+    if (head_col < n_out) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = row0 + acc_row(r, lane);
-        if (row < B) out[(size_t) row * n_out + col] = acc[r] + bv;
+        if (row < B) *head_cell(heads, row, head_col) = acc[r] + bv;
       }
     }
   }
 }
 
-
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t) h << 16); }
 
-// dZ[l] for every layer, back to front. packed_t holds, for l = 1 .. n_layers-1, the hidden part of W_l transposed:
-// [256 inputs][256 outputs] bf16.
-__global__ void __launch_bounds__(kChainThreads) mlp_backward_chain_kernel(int B, int n_layers, int n_out,
-    const float* __restrict__ heads_w /*[n_out][256] fp32*/, const uint16_t* __restrict__ packed_t,
-    const uint16_t* __restrict__ saved, const float* __restrict__ g_out, uint16_t* __restrict__ dz) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_dz[kMlpRows][kMlpWidth + 8];
-  __shared__ float s_g[kMlpRows][32];
+// dZ[l] for every layer, back to front, and the outputs' gradient in the same form (g_t[32][B_pad]); in_t (optional): the
+// input rows too, for callers whose forward did not leave them. packed_t holds, for l = 1 .. n_layers-1, the hidden part
+// of W_l transposed: [256 inputs][256 outputs] bf16. Rows past the batch are zeros in every output.
+__global__ void __launch_bounds__(kChainThreads) mlp_backward_chain_kernel(int B, int Din, int n_layers, int n_out,
+    const float* __restrict__ in, const float* __restrict__ heads_w /*[n_out][256] fp32*/,
+    const uint16_t* __restrict__ packed_t, const uint16_t* __restrict__ saved, MlpHeads heads,
+    uint16_t* __restrict__ dz, uint16_t* __restrict__ g_t, uint16_t* __restrict__ in_t) {
+  __shared__ __attribute__((aligned(16))) uint16_t s_dz[2][kMlpRows][kMlpWidth + 8];
+  __shared__ float s_g[kMlpRows][33];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * kMlpRows;
-  {
-    // dZ of the last layer: (g_out . W_heads) where the stored state is non-zero. Lane t owns column t of all 32 rows.
-    for (int e = threadIdx.x; e < kMlpRows * 32; e += kChainThreads) {
-      const int r = e >> 5, k = e & 31;
-      s_g[r][k] = (row0 + r < B && k < n_out) ? g_out[(size_t) (row0 + r) * n_out + k] : 0.0f;
-    }
-    __syncthreads();
-    if (threadIdx.x < kMlpWidth) {
-    const int c = threadIdx.x;
-    const size_t top = (size_t) (n_layers - 1) * B;
-    uint16_t keep[kMlpRows];  // read at clamped rows, unconditionally, so the loads overlap the products below
-#pragma unroll
-    for (int r = 0; r < kMlpRows; ++r) keep[r] = saved[(top + min(row0 + r, B - 1)) * kMlpWidth + c];
-    float v[kMlpRows];
-#pragma unroll
-    for (int r = 0; r < kMlpRows; ++r) v[r] = 0.0f;
-    for (int k = 0; k < n_out; ++k) {
-      const float wv = heads_w[k * kMlpWidth + c];
-#pragma unroll
-      for (int r = 0; r < kMlpRows; ++r) v[r] += s_g[r][k] * wv;
-    }
-#pragma unroll
-    for (int r = 0; r < kMlpRows; ++r) {
-      const bool live  = row0 + r < B;
-      const uint16_t h = (live && keep[r] != 0) ? f32_to_bf16(v[r]) : (uint16_t) 0;
-      if (live) dz[(top + row0 + r) * kMlpWidth + c] = h;
-      s_dz[r][c] = h;
-    }
-    }
-  }
-  // all sixteen weight fragments of a wavefront's tile are requested together, one layer ahead (they do not depend on
-  // dZ), and the stored states that mask a layer's result are fetched while the matrix cores run
+  const size_t B_pad = (size_t) gridDim.x * kMlpRows;
+  const int arow = lane & 31, kofs = 8 * (lane >> 5), col = wave * 32 + (lane & 31);
   auto fragment = [&](int layer, int u) {
     return *(const bf16x8*) (packed_t + ((size_t) ((layer - 1) * 8 + wave) * (kMlpWidth / 16) + u) * 512 + lane * 8);
   };
+  // the stored states that mask a layer's result: four consecutive rows of the lane's column per load
+  auto mask_of = [&](int layer, uint2* keep) {
+    const uint16_t* src = saved + ((size_t) layer * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) keep[g] = *(const uint2*) (src + 8 * g);
+  };
+  // one layer ahead of their use, the masks in front of the weights (loads complete in order)
+  uint2 keep_ahead[4];
   bf16x8 ahead[16];
-  if (n_layers >= 2)
+  if (n_layers >= 2) {
+    mask_of(n_layers - 2, keep_ahead);
 #pragma unroll
     for (int u = 0; u < 16; ++u) ahead[u] = fragment(n_layers - 1, u);
+  }
+  for (int e = threadIdx.x; e < kMlpRows * 32; e += kChainThreads) {
+    const int r = e >> 5, k = e & 31;
+    const float* cell = (row0 + r < B && k < n_out) ? head_cell(heads, row0 + r, k) : nullptr;
+    s_g[r][k] = cell ? *cell : 0.0f;
+  }
+  if (in_t) {
+    for (int e = threadIdx.x; e < Din * kMlpRows; e += kChainThreads) {
+      const int r = e / Din, k = e - r * Din;
+      in_t[(size_t) k * B_pad + row0 + r] = row0 + r < B ? f32_to_bf16(in[(size_t) (row0 + r) * Din + k]) : (uint16_t) 0;
+    }
+  }
   __syncthreads();
+  for (int e = threadIdx.x; e < 32 * kMlpRows; e += kChainThreads)
+    g_t[(size_t) (e >> 5) * B_pad + row0 + (e & 31)] = f32_to_bf16(s_g[e & 31][e >> 5]);
+  {
+    // dZ of the last layer: (g_out . W_heads) where the stored state is non-zero. A lane owns 16 rows of one column.
+    const int c = threadIdx.x & 255, r0 = 16 * (threadIdx.x >> 8);
+    const size_t top = ((size_t) (n_layers - 1) * kMlpWidth + c) * B_pad + row0 + r0;
+    uint4 keep[2] = {*(const uint4*) (saved + top), *(const uint4*) (saved + top + 8)};
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = 0.0f;
+    for (int k = 0; k < n_out; ++k) {
+      const float wv = heads_w[k * kMlpWidth + c];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] += s_g[r0 + r][k] * wv;
+    }
+    const uint32_t words[8] = {keep[0].x, keep[0].y, keep[0].z, keep[0].w, keep[1].x, keep[1].y, keep[1].z, keep[1].w};
+    uint16_t h[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const bool on = ((words[r >> 1] >> (16 * (r & 1))) & 0xffffu) != 0u && row0 + r0 + r < B;
+      h[r] = on ? f32_to_bf16(v[r]) : (uint16_t) 0;
+      s_dz[0][r0 + r][c] = h[r];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *(uint2*) (dz + top + 4 * g) = pack4(h + 4 * g);
+  }
+  __syncthreads();
+  int cur = 0;
   for (int layer = n_layers - 1; layer >= 1; --layer) {
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    const int arow = lane & 31, kofs = 8 * (lane >> 5);
     bf16x8 b[16];
+    uint2 keep[4];
 #pragma unroll
     for (int u = 0; u < 16; ++u) b[u] = ahead[u];
-    if (layer >= 2)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) keep[g] = keep_ahead[g];
+    if (layer >= 2) {
+      mask_of(layer - 2, keep_ahead);
 #pragma unroll
       for (int u = 0; u < 16; ++u) ahead[u] = fragment(layer - 1, u);
-    const size_t base = (size_t) (layer - 1) * B;
-    uint16_t keep[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      // rows past the batch reuse the last row's mask: their results stay in LDS and are never stored
-      const int row = min(row0 + acc_row(r, lane), B - 1);
-      keep[r] = saved[(base + row) * kMlpWidth + wave * 32 + (lane & 31)];
     }
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const bf16x8 a = *(const bf16x8*) &s_dz[arow][16 * u + kofs];
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[u], acc, 0, 0, 0);
-    }
-    lds_barrier();  // every wavefront has read dZ[layer] before it is overwritten
-    {
-      const int col = wave * 32 + (lane & 31);
+    for (int u = 0; u < 16; ++u)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) &s_dz[cur][arow][16 * u + kofs], b[u], acc, 0, 0, 0);
+    uint16_t* dst = dz + ((size_t) (layer - 1) * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row    = acc_row(r, lane);
-        const uint16_t h = keep[r] != 0 ? f32_to_bf16(acc[r]) : (uint16_t) 0;
-        if (row0 + row < B) dz[(base + row0 + row) * kMlpWidth + col] = h;
-        s_dz[row][col] = h;
+    for (int g = 0; g < 4; ++g) {
+      uint16_t h[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t word = k < 2 ? keep[g].x : keep[g].y;
+        const bool on = ((word >> (16 * (k & 1))) & 0xffffu) != 0u;  // rows past the batch: dZ is zero since the last layer
+        h[k] = on ? f32_to_bf16(acc[4 * g + k]) : (uint16_t) 0;
+        s_dz[cur ^ 1][acc_row(4 * g + k, lane)][col] = h[k];
       }
+      *(uint2*) (dst + 8 * g) = pack4(h);
     }
     lds_barrier();
+    cur ^= 1;
   }
 }
 
-// dW_l = dZ_l^T X_l and db_l = column sums of dZ_l for l = 0 .. n_layers (l == n_layers: the heads, whose "dZ" is g_out).
-// X_0 = in, X_{skip+1} = [in | H_skip], X_l = H_{l-1} otherwise. g_w is the layers' [256][K_l] gradients back to back
-// followed by the heads' [n_out][256]; g_b has the layout of the forward's bias vector.
+// dW_l = dZ_l^T X_l and db_l = row sums of dZ_l for l = 0 .. n_layers (l == n_layers: the heads, whose dZ is g_t).
+// X_0 = in, X_{skip+1} = [in | H_skip], X_l = H_{l-1} otherwise, all with the batch innermost. g_w is the layers' [256][K_l]
+// gradients back to back followed by the heads' [n_out][256]; g_b has the layout of the forward's bias vector.
+constexpr int kWgTile = 64;
+constexpr int kWgSteps = 8;  // k-steps of 16 rows that a wavefront has in flight
 __global__ void __launch_bounds__(kMlpThreads) mlp_backward_weights_kernel(int B, int Din, int n_layers, int skip,
-    int n_out, const float* __restrict__ in, const uint16_t* __restrict__ saved, const uint16_t* __restrict__ dz,
-    const float* __restrict__ g_out, float* __restrict__ g_w, float* __restrict__ g_b) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_a[32][kMlpRows + 8];   // [output o][batch row]
-  __shared__ __attribute__((aligned(16))) uint16_t s_b[128][kMlpRows + 8];  // [input i][batch row]
-  // which (layer, output tile, input group) this block owns
+    int n_out, const uint16_t* __restrict__ in_t, const uint16_t* __restrict__ saved, const uint16_t* __restrict__ dz,
+    const uint16_t* __restrict__ g_t, float* __restrict__ g_w, float* __restrict__ g_b) {
+  __shared__ float s_sum[kWgTile][kWgTile + 1];
+  __shared__ float s_bias[kMlpThreads / kWave][kWgTile];
+  // which (layer, output tile, input tile) this block owns
   int layer = 0, K = Din, tile = blockIdx.x;
   size_t w_off = 0;
   for (;; ++layer) {
     const int rows = layer < n_layers ? kMlpWidth : n_out;
-    const int tiles = ((rows + 31) / 32) * ((K + 127) / 128);
+    const int tiles = div_up_dev(rows, kWgTile) * div_up_dev(K, kWgTile);
     if (tile < tiles || layer == n_layers) break;
     tile -= tiles;
     w_off += (size_t) rows * K;
     K = (layer == skip) ? Din + kMlpWidth : kMlpWidth;
   }
-  const int rows   = layer < n_layers ? kMlpWidth : n_out;
-  const int groups = (K + 127) / 128;
-  const int o0 = (tile / groups) * 32, i0 = (tile % groups) * 128;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // X_l's hidden part comes from this saved state, shifted by `shift` columns (the re-concatenated input)
-  const int shift = (layer == skip + 1) ? Din : 0;
-  const uint16_t* hidden = layer > 0 ? saved + (size_t) (layer - 1) * B * kMlpWidth : nullptr;
-  floatx16 acc;
+  const int rows = layer < n_layers ? kMlpWidth : n_out, across = div_up_dev(K, kWgTile);
+  const int o0 = (tile / across) * kWgTile, i0 = (tile % across) * kWgTile;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kofs = 8 * (lane >> 5);
+  const size_t B_pad = (size_t) ((B + kMlpRows - 1) / kMlpRows) * kMlpRows;
+  const int shift = layer == 0 ? Din : (layer == skip + 1 ? Din : 0);  // columns of X_l that are the input
+  const uint16_t *arow[2], *brow[2];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  float bias_sum = 0.0f;
-  for (int b0 = 0; b0 < B; b0 += kMlpRows) {
-    // Loads are unconditional on clamped addresses and out-of-range elements are zeroed afterwards. The empty asm after
-    // each group takes all of its values at once: without it the compiler sinks every load into a branch of its own
-    // with a full wait behind it; with it a chunk's 20 loads are in flight together.
-    uint16_t va[4], vb[16];
-    unsigned ra[4], rb[16];
-    float fb[16];
+  for (int t = 0; t < 2; ++t) {
+    const int o = min(o0 + 32 * t + (lane & 31), rows - 1), i = min(i0 + 32 * t + (lane & 31), K - 1);
+    arow[t] = (layer < n_layers ? dz + ((size_t) layer * kMlpWidth + o) * B_pad : g_t + (size_t) o * B_pad) + kofs;
+    brow[t] = (i < shift ? in_t + (size_t) i * B_pad
+                         : saved + ((size_t) (layer - 1) * kMlpWidth + (i - shift)) * B_pad) + kofs;
+  }
+  floatx16 acc[2][2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads, b = e >> 5, o = e & 31;
-      const int bc = min(b0 + b, B - 1), oc = min(o0 + o, rows - 1);
-      ra[q] = layer < n_layers ? dz[((size_t) layer * B + bc) * kMlpWidth + oc]
-                               : f32_to_bf16(g_out[(size_t) bc * n_out + oc]);
-    }
-    const bool from_in = layer == 0 || (shift > 0 && i0 < shift);
-    const bool from_hidden = layer > 0;
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads, b = e >> 7, gi = i0 + (e & 127);
-      const int bc = min(b0 + b, B - 1);
-      fb[q] = from_in ? in[(size_t) bc * Din + min(gi, Din - 1)] : 0.0f;
-      rb[q] = from_hidden ? hidden[(size_t) bc * kMlpWidth + min(max(gi - shift, 0), kMlpWidth - 1)] : 0u;
-    }
-    asm volatile("" : "+v"(ra[0]), "+v"(ra[1]), "+v"(ra[2]), "+v"(ra[3]));
-    asm volatile("" : "+v"(rb[0]), "+v"(rb[1]), "+v"(rb[2]), "+v"(rb[3]), "+v"(rb[4]), "+v"(rb[5]), "+v"(rb[6]),
-                      "+v"(rb[7]), "+v"(rb[8]), "+v"(rb[9]), "+v"(rb[10]), "+v"(rb[11]), "+v"(rb[12]), "+v"(rb[13]),
-                      "+v"(rb[14]), "+v"(rb[15]));
-    asm volatile("" : "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]), "+v"(fb[3]), "+v"(fb[4]), "+v"(fb[5]), "+v"(fb[6]),
-                      "+v"(fb[7]), "+v"(fb[8]), "+v"(fb[9]), "+v"(fb[10]), "+v"(fb[11]), "+v"(fb[12]), "+v"(fb[13]),
-                      "+v"(fb[14]), "+v"(fb[15]));
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads, b = e >> 5, o = e & 31;
-      va[q] = (b0 + b < B && o0 + o < rows) ? (uint16_t) ra[q] : (uint16_t) 0;
+      for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.0f;
+  float bias[2] = {0.0f, 0.0f};
+  const bool wants_bias = i0 == 0;
+  const int last = (int) B_pad - 16;
+  constexpr int kChunk = 16 * kWgSteps;
+  for (int b0 = wave * kChunk; b0 < (int) B_pad; b0 += (kMlpThreads / kWave) * kChunk) {
+    bf16x8 a[2][kWgSteps], b[2][kWgSteps];
+#pragma unroll
+    for (int u = 0; u < kWgSteps; ++u) {
+      const int at = min(b0 + 16 * u, last);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) a[t][u] = *(const bf16x8*) (arow[t] + at), b[t][u] = *(const bf16x8*) (brow[t] + at);
     }
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads, b = e >> 7, gi = i0 + (e & 127);
-      const uint16_t h = (layer == 0 || gi < shift) ? f32_to_bf16(fb[q]) : (uint16_t) rb[q];
-      vb[q] = (b0 + b < B && gi < K) ? h : (uint16_t) 0;
-    }
+    for (int u = 0; u < kWgSteps; ++u) {
+      if (b0 + 16 * u > last) break;  // uniform
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads;
-      s_a[e & 31][e >> 5] = va[q];
-    }
+      for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int e = threadIdx.x + q * kMlpThreads;
-      s_b[e & 127][e >> 7] = vb[q];
-    }
-    __syncthreads();
-    const int kofs = 8 * (lane >> 5);
+        for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][u], b[y][u], acc[x][y], 0, 0, 0);
+      if (wants_bias) {
 #pragma unroll
-    for (int k0 = 0; k0 < kMlpRows; k0 += 16) {
-      const bf16x8 a = *(const bf16x8*) &s_a[lane & 31][k0 + kofs];
-      const bf16x8 b = *(const bf16x8*) &s_b[wave * 32 + (lane & 31)][k0 + kofs];
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    if (i0 == 0 && threadIdx.x < 32) {
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int b = 0; b < kMlpRows; ++b) bias_sum += bf16_to_f32(s_a[threadIdx.x][b]);
+          for (int k = 0; k < 8; ++k) bias[t] += (float) a[t][u][k];
+      }
+    }
+  }
+  if (wants_bias) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      bias[t] += __shfl_xor(bias[t], 32, kWave);
+      if (lane < 32) s_bias[wave][32 * t + lane] = bias[t];
+    }
+  }
+  // the wavefronts' sums in wavefront order
+  for (int w = 0; w < kMlpThreads / kWave; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            float* cell = &s_sum[32 * x + acc_row(r, lane)][32 * y + (lane & 31)];
+            *cell = w == 0 ? acc[x][y][r] : *cell + acc[x][y][r];
+          }
     }
     __syncthreads();
   }
-  const int i = i0 + wave * 32 + (lane & 31);
-  if (i < K) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int o = o0 + acc_row(r, lane);
-      if (o < rows) g_w[w_off + (size_t) o * K + i] = acc[r];
-    }
+  for (int e = threadIdx.x; e < kWgTile * kWgTile; e += kMlpThreads) {
+    const int o = e >> 6, i = e & 63;
+    if (o0 + o < rows && i0 + i < K) g_w[w_off + (size_t) (o0 + o) * K + i0 + i] = s_sum[o][i];
   }
-  if (i0 == 0 && threadIdx.x < 32 && o0 + threadIdx.x < rows)
-    g_b[(size_t) layer * kMlpWidth + o0 + threadIdx.x] = bias_sum;
+  if (wants_bias && threadIdx.x < kWgTile && o0 + (int) threadIdx.x < rows) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kMlpThreads / kWave; ++w) v += s_bias[w][threadIdx.x];
+    g_b[(size_t) layer * kMlpWidth + o0 + threadIdx.x] = v;
+  }
 }
 
 }  // namespace
@@ -504,50 +574,101 @@ FSGS_API size_t fsgs_mlp_packed_elems(int Din, int n_layers, int skip) {
   return n;
 }
 
-FSGS_API int fsgs_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
-                              const uint16_t* packed, const float* bias, float* out, uint16_t* saved, void* stream) {
-  FSGS_REQUIRE(B >= 0 && in && packed && bias && out, "mlp_forward: bad arguments");
+namespace {
+size_t padded_rows(int B) { return (size_t) div_up(std::max(B, 1), kMlpRows) * kMlpRows; }
+
+bool make_heads(MlpHeads& h, int n_heads, const int* head_rows, float* const* at) {
+  if (n_heads < 1 || n_heads > kMaxHeads) return false;
+  h.n = n_heads, h.first[0] = 0;
+  for (int k = 0; k < n_heads; ++k) {
+    if (head_rows[k] < 1) return false;
+    h.at[k] = at[k], h.first[k + 1] = h.first[k] + head_rows[k];
+  }
+  return h.first[n_heads] <= 32;
+}
+}  // namespace
+
+FSGS_API size_t fsgs_mlp_saved_elems(int B, int n_layers) { return (size_t) n_layers * kMlpWidth * padded_rows(B); }
+FSGS_API size_t fsgs_mlp_saved_input_elems(int B, int Din) { return (size_t) Din * padded_rows(B); }
+
+FSGS_API int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
+    const float* in, const float* x, const float* t, int degree_x, double scale_x, int degree_t, double scale_t,
+    const uint16_t* packed, const float* bias, float* const* outs, uint16_t* saved_in, uint16_t* saved, void* stream) {
+  FSGS_REQUIRE(B >= 0 && (in || (x && t)) && packed && bias && head_rows && outs, "mlp_forward: bad arguments");
+  FSGS_REQUIRE(in || (degree_x >= 0 && degree_t >= 0 && Din == 3 * (1 + 2 * degree_x) + 1 + 2 * degree_t),
+               "mlp_forward: the encoding has another width than the network's input");
   FSGS_REQUIRE(width == kMlpWidth, "mlp_forward: width %d is not supported (only %d)", width, kMlpWidth);
   FSGS_REQUIRE(Din > 0 && ((Din + 15) & ~15) <= kMlpMaxIn, "mlp_forward: input width %d exceeds %d", Din, kMlpMaxIn);
-  FSGS_REQUIRE(n_layers >= 1 && skip < n_layers - 1 && n_out >= 1 && n_out <= 32,
-               "mlp_forward: bad layer structure (layers %d, skip %d, outputs %d)", n_layers, skip, n_out);
+  FSGS_REQUIRE((saved == nullptr) == (saved_in == nullptr), "mlp_forward: saved_in and saved go together");
+  MlpHeads heads{};
+  FSGS_REQUIRE(make_heads(heads, n_heads, head_rows, outs), "mlp_forward: bad heads (at most %d with 32 rows)", kMaxHeads);
+  for (int h = 0; h < n_heads; ++h) FSGS_REQUIRE(outs[h], "mlp_forward: null output");
+  const int n_out = heads.first[n_heads];
+  FSGS_REQUIRE(n_layers >= 1 && skip < n_layers - 1, "mlp_forward: bad layer structure (layers %d, skip %d, outputs %d)",
+               n_layers, skip, n_out);
   if (B == 0) return kOk;
+  const FreqInput freq{x, t, degree_x, degree_t, (float) scale_x, (float) scale_t};
   auto kernel = saved ? mlp_forward_kernel<true> : mlp_forward_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(B, kMlpRows)), dim3(kChainThreads), 0, (hipStream_t) stream, B, Din, n_layers,
-                     skip, n_out, in, packed, bias, out, saved);
+                     skip, n_out, in, freq, packed, bias, heads, saved_in, saved);
   return check_launch("mlp_forward");
 }
 
-FSGS_API size_t fsgs_mlp_backward_workspace_bytes(int B, int n_layers) {
-  if (B < 0 || n_layers < 1) return 0;
-  return align_up((size_t) n_layers * (B > 0 ? B : 1) * kMlpWidth * sizeof(uint16_t), 256);
+FSGS_API size_t fsgs_mlp_backward_workspace_bytes(int B, int Din, int n_layers) {
+  if (B < 0 || n_layers < 1 || Din < 1) return 0;
+  return align_up(((size_t) n_layers * kMlpWidth + 32 + Din) * padded_rows(B) * sizeof(uint16_t), 256);
+}
+
+FSGS_API int fsgs_deform_mlp_backward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
+    const float* in, const uint16_t* saved_in, const uint16_t* packed_t, const float* heads_w, const uint16_t* saved,
+    const float* const* g_outs, float* g_w, float* g_b, void* workspace, size_t workspace_bytes, void* stream) {
+  FSGS_REQUIRE(B >= 0 && (in || saved_in) && packed_t && heads_w && saved && head_rows && g_outs && g_w && g_b && workspace,
+               "mlp_backward: bad arguments");
+  FSGS_REQUIRE(width == kMlpWidth, "mlp_backward: width %d is not supported (only %d)", width, kMlpWidth);
+  FSGS_REQUIRE(Din > 0 && ((Din + 15) & ~15) <= kMlpMaxIn, "mlp_backward: input width %d exceeds %d", Din, kMlpMaxIn);
+  MlpHeads heads{};
+  FSGS_REQUIRE(make_heads(heads, n_heads, head_rows, (float* const*) g_outs), "mlp_backward: bad heads");
+  const int n_out = heads.first[n_heads];
+  FSGS_REQUIRE(n_layers >= 1 && n_layers <= 64 && skip < n_layers - 1,
+               "mlp_backward: bad layer structure (layers %d, skip %d, outputs %d)", n_layers, skip, n_out);
+  if (workspace_bytes < fsgs_mlp_backward_workspace_bytes(B, Din, n_layers))
+    return fail(kWorkspaceSmall, "mlp_backward: workspace %zu < %zu bytes", workspace_bytes,
+                fsgs_mlp_backward_workspace_bytes(B, Din, n_layers));
+  hipStream_t s = (hipStream_t) stream;
+  const size_t B_pad = padded_rows(B);
+  uint16_t* dz   = (uint16_t*) workspace;
+  uint16_t* g_t  = dz + (size_t) n_layers * kMlpWidth * B_pad;
+  uint16_t* in_t = saved_in ? nullptr : g_t + 32 * B_pad;
+  if (B == 0) {  // no rows: the gradients are zeros
+    const size_t n_w = (size_t) kMlpWidth * Din * (skip >= 0 ? 2 : 1) + (size_t) (n_layers - 1) * kMlpWidth * kMlpWidth +
+                       (size_t) n_out * kMlpWidth;
+    hipLaunchKernelGGL(fill_zero_kernel, dim3(256), dim3(256), 0, s, n_w, g_w);
+    hipLaunchKernelGGL(fill_zero_kernel, dim3(16), dim3(256), 0, s, (size_t) n_layers * kMlpWidth + n_out, g_b);
+    return check_launch("mlp_backward");
+  }
+  hipLaunchKernelGGL(mlp_backward_chain_kernel, dim3(div_up(B, kMlpRows)), dim3(kChainThreads), 0, s, B, Din, n_layers, n_out,
+                     in, heads_w, packed_t, saved, heads, dz, g_t, in_t);
+  int tiles = 0, K = Din;
+  for (int l = 0; l <= n_layers; ++l) {
+    tiles += div_up(l < n_layers ? kMlpWidth : n_out, kWgTile) * div_up(K, kWgTile);
+    K = (l == skip) ? Din + kMlpWidth : kMlpWidth;
+  }
+  hipLaunchKernelGGL(mlp_backward_weights_kernel, dim3(tiles), dim3(kMlpThreads), 0, s, B, Din, n_layers, skip, n_out,
+                     saved_in ? saved_in : in_t, saved, dz, g_t, g_w, g_b);
+  return check_launch("mlp_backward");
+}
+
+FSGS_API int fsgs_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
+                              const uint16_t* packed, const float* bias, float* out, uint16_t* saved_in, uint16_t* saved,
+                              void* stream) {
+  return fsgs_deform_mlp_forward(B, Din, width, n_layers, skip, 1, &n_out, in, nullptr, nullptr, 0, 1.0, 0, 1.0, packed, bias,
+                                 &out, saved_in, saved, stream);
 }
 
 FSGS_API int fsgs_mlp_backward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
     const uint16_t* packed_t, const float* heads_w, const uint16_t* saved, const float* g_out, float* g_w, float* g_b,
     void* workspace, size_t workspace_bytes, void* stream) {
-  FSGS_REQUIRE(B >= 0 && in && packed_t && heads_w && saved && g_out && g_w && g_b && workspace,
-               "mlp_backward: bad arguments");
-  FSGS_REQUIRE(width == kMlpWidth, "mlp_backward: width %d is not supported (only %d)", width, kMlpWidth);
-  FSGS_REQUIRE(Din > 0 && ((Din + 15) & ~15) <= kMlpMaxIn, "mlp_backward: input width %d exceeds %d", Din, kMlpMaxIn);
-  FSGS_REQUIRE(n_layers >= 1 && n_layers <= 64 && skip < n_layers - 1 && n_out >= 1 && n_out <= 32,
-               "mlp_backward: bad layer structure (layers %d, skip %d, outputs %d)", n_layers, skip, n_out);
-  if (workspace_bytes < fsgs_mlp_backward_workspace_bytes(B, n_layers))
-    return fail(kWorkspaceSmall, "mlp_backward: workspace %zu < %zu bytes", workspace_bytes,
-                fsgs_mlp_backward_workspace_bytes(B, n_layers));
-  hipStream_t s = (hipStream_t) stream;
-  uint16_t* dz  = (uint16_t*) workspace;
-  // with an empty batch the weight kernel's chunk loop does not run and it writes zeros
-  if (B > 0)
-    hipLaunchKernelGGL(mlp_backward_chain_kernel, dim3(div_up(B, kMlpRows)), dim3(kChainThreads), 0, s, B, n_layers,
-                       n_out, heads_w, packed_t, saved, g_out, dz);
-  int tiles = 0, K = Din;
-  for (int l = 0; l <= n_layers; ++l) {
-    const int rows = l < n_layers ? kMlpWidth : n_out;
-    tiles += ((rows + 31) / 32) * ((K + 127) / 128);
-    K = (l == skip) ? Din + kMlpWidth : kMlpWidth;
-  }
-  hipLaunchKernelGGL(mlp_backward_weights_kernel, dim3(tiles), dim3(kMlpThreads), 0, s, B, Din, n_layers, skip, n_out,
-                     in, saved, dz, g_out, g_w, g_b);
-  return check_launch("mlp_backward");
+  FSGS_REQUIRE(g_out, "mlp_backward: bad arguments");
+  return fsgs_deform_mlp_backward(B, Din, width, n_layers, skip, 1, &n_out, in, nullptr, packed_t, heads_w, saved, &g_out,
+                                  g_w, g_b, workspace, workspace_bytes, stream);
 }

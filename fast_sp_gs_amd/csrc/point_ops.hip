@@ -384,7 +384,7 @@ __global__ void __launch_bounds__(256) knn_topk_kernel(int N, int M, int D, int 
 
 // ---- LBS skinning (per-control-point table and weights: lbs.hpp) -----------------------------------------------------
 template <int kMaxK>
-__global__ void __launch_bounds__(256) lbs_blend_kernel(int N, int M, int K, int S, int warp_mode, int weight_mode,
+__global__ void __launch_bounds__(256) lbs_blend_kernel(int N, int M, int K, int S, int sp_s_ld, int warp_mode, int weight_mode,
     float temperature, const float* __restrict__ points, const float* __restrict__ xf, const float* __restrict__ sp_r,
     const float* __restrict__ sp_s, const float* __restrict__ pair_in, const int64_t* __restrict__ index,
     float* __restrict__ weights_out, float* __restrict__ d_xyz, float* __restrict__ d_rot,
@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(256) lbs_blend_kernel(int N, int M, int K, int
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a) ar[a] += w * sp_r[4 * j + a];
-    for (int a = 0; a < S; ++a) as[a] += w * sp_s[(size_t) S * j + a];
+    for (int a = 0; a < S; ++a) as[a] += w * sp_s[(size_t) sp_s_ld * j + a];
     if (weights_out) weights_out[(size_t) n * K + k] = w;
   }
 #pragma unroll
@@ -456,6 +456,48 @@ __global__ void __launch_bounds__(256) adam_masked_kernel(int64_t total, int64_t
     *(float4*) (v + e)     = *(float4*) vv;
   } else {
     param[e] = pp[0], m[e] = mm[0], v[e] = vv[0];
+  }
+}
+
+// torch.optim.Adam's update (no weight decay, no amsgrad) for up to kMaxDenseTensors tensors in one launch: the moments,
+// then param -= step_size * m / (sqrt(v) / root_c2 + eps) with step_size = lr / (1 - b1^t), root_c2 = sqrt(1 - b2^t) from
+// the host. The deformation network's 25 tensors hold 0.56M floats: 16 MB of traffic, 5 us; torch's fused form cuts them
+// into 26 chunks of 64K elements, one block each, and took 44.
+constexpr int kMaxDenseTensors = 32;
+struct DenseAdamTable {
+  float* param[kMaxDenseTensors];
+  const float* grad[kMaxDenseTensors];
+  float* m[kMaxDenseTensors];
+  float* v[kMaxDenseTensors];
+  int64_t count[kMaxDenseTensors];
+  float step_size[kMaxDenseTensors], inv_root_c2[kMaxDenseTensors];
+  unsigned first_block[kMaxDenseTensors + 1];
+  int n;
+};
+constexpr int kDensePerBlock = 1024;  // four elements a lane, 256 lanes apart
+__global__ void __launch_bounds__(256) adam_dense_multi_kernel(DenseAdamTable t, float b1, float b2, float c1,
+                                                               float c2, float eps) {
+  int q = 0;
+  while (q + 1 < t.n && blockIdx.x >= t.first_block[q + 1]) ++q;
+  const int64_t base = (int64_t) (blockIdx.x - t.first_block[q]) * kDensePerBlock + threadIdx.x, n = t.count[q];
+  float* __restrict__ param = t.param[q];
+  const float* __restrict__ grad = t.grad[q];
+  float* __restrict__ m = t.m[q];
+  float* __restrict__ v = t.v[q];
+  float g[4], mm[4], vv[4], pp[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t e = base + 256 * k;
+    const bool on = e < n;
+    g[k] = on ? grad[e] : 0.0f, mm[k] = on ? m[e] : 0.0f, vv[k] = on ? v[e] : 0.0f, pp[k] = on ? param[e] : 0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t e = base + 256 * k;
+    if (e >= n) continue;
+    const float m1 = b1 * mm[k] + c1 * g[k], v1 = b2 * vv[k] + c2 * g[k] * g[k];
+    param[e] = pp[k] - t.step_size[q] * m1 / (sqrtf(v1) * t.inv_root_c2[q] + eps);
+    m[e] = m1, v[e] = v1;
   }
 }
 
@@ -616,6 +658,33 @@ FSGS_API int fsgs_deform_apply_backward(int N, int S, int log_scales, const floa
   hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, (hipStream_t) stream, N, log_scales, scales, rot,
                      d_rot, g_out_scales, g_out_rot, g_scales, g_rot);
   return check_launch("deform_apply_backward");
+}
+
+FSGS_API int fsgs_adam_update_max_tensors(void) { return kMaxDenseTensors; }
+
+FSGS_API int fsgs_adam_update_multi(int n_tensors, const int64_t* count, const double* step_size, const double* root_c2,
+    double b1, double b2, double eps, float* const* param, const float* const* grad, float* const* m, float* const* v,
+    void* stream) {
+  FSGS_REQUIRE(n_tensors >= 0 && n_tensors <= kMaxDenseTensors, "adam_update: at most %d tensors", kMaxDenseTensors);
+  if (n_tensors == 0) return kOk;
+  FSGS_REQUIRE(count && step_size && root_c2 && param && grad && m && v, "adam_update: null pointer");
+  DenseAdamTable t{};
+  t.n = n_tensors;
+  unsigned blocks = 0;
+  for (int q = 0; q < n_tensors; ++q) {
+    FSGS_REQUIRE(count[q] >= 0 && (count[q] == 0 || (param[q] && grad[q] && m[q] && v[q])), "adam_update: bad tensor %d", q);
+    t.param[q] = param[q], t.grad[q] = grad[q], t.m[q] = m[q], t.v[q] = v[q], t.count[q] = count[q];
+    t.step_size[q] = (float) step_size[q], t.inv_root_c2[q] = (float) (1.0 / root_c2[q]);
+    t.first_block[q] = blocks;
+    const int64_t nb = div_up(count[q], (int64_t) kDensePerBlock);
+    FSGS_REQUIRE((int64_t) blocks + nb < (int64_t) 0x7fffffff, "adam_update: too many elements");
+    blocks += (unsigned) nb;
+  }
+  t.first_block[n_tensors] = blocks;
+  if (blocks == 0) return kOk;
+  hipLaunchKernelGGL(adam_dense_multi_kernel, dim3(blocks), dim3(256), 0, (hipStream_t) stream, t, (float) b1, (float) b2,
+                     (float) (1.0 - b1), (float) (1.0 - b2), (float) eps);
+  return check_launch("adam_update");
 }
 
 FSGS_API int fsgs_adam_masked_update_max_tensors(void) { return kMaxAdamTensors; }
@@ -851,10 +920,11 @@ FSGS_API size_t fsgs_lbs_blend_workspace_bytes(int M) { return align_up((size_t)
 
 FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
     const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
-    const float* sp_s, int S, const float* pair_in, const int64_t* index, const float* sp_log_radius,
+    const float* sp_s, int S, int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius,
     const float* sp_weight_logit, float* weights_out, float* d_xyz, float* d_rot, float* d_scale, void* workspace,
     size_t workspace_bytes, void* stream) {
-  FSGS_REQUIRE(N >= 0 && M > 0 && K > 0 && K <= 16 && S >= 0 && S <= 4, "lbs_blend: bad sizes (K <= 16, S <= 4)");
+  FSGS_REQUIRE(N >= 0 && M > 0 && K > 0 && K <= 16 && S >= 0 && S <= 4 && sp_s_ld >= S,
+               "lbs_blend: bad sizes (K <= 16, S <= 4)");
   FSGS_REQUIRE(warp_mode >= 0 && warp_mode <= 2 && weight_mode >= 0 && weight_mode <= 3, "lbs_blend: unknown mode");
   FSGS_REQUIRE(points && sp_points && sp_t && sp_r && pair_in && index && d_xyz && d_rot &&
                    (S == 0 || (sp_s && d_scale)) && workspace, "lbs_blend: null pointer");
@@ -871,7 +941,7 @@ FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode,
   hipLaunchKernelGGL(lbs_prepare_kernel, dim3(div_up(M, 256)), dim3(256), 0, s, M, warp_mode, sp_points, sp_t, sp_rot,
                      weight_mode == 1 ? sp_log_radius : nullptr, weight_mode == 1 ? sp_weight_logit : nullptr, xf);
   auto kernel = K <= 4 ? lbs_blend_kernel<4> : lbs_blend_kernel<16>;
-  hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, s, N, M, K, S, warp_mode, weight_mode,
+  hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, s, N, M, K, S, sp_s_ld, warp_mode, weight_mode,
                      (float) temperature, points, xf, sp_r, sp_s, pair_in, index, weights_out, d_xyz, d_rot, d_scale);
   return check_launch("lbs_blend");
 }

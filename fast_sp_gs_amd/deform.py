@@ -11,6 +11,7 @@ import torch
 from torch import Tensor, nn
 
 from fast_sp_gs_amd._C import get_C_function
+from fast_sp_gs_amd.lib import host
 from fast_sp_gs_amd.ops import FreqEncoder
 
 __all__ = ['DeformNetwork', 'superpoint_deform', 'deform_apply', 'calc_LBS_weight', 'warp', 'knn_points']
@@ -64,14 +65,9 @@ class DeformNetwork(nn.Module):
 
     def pack(self, transposed: bool = True):
         """Refresh the bf16 weight buffers, the bias vector and the stacked head rows from the parameters in one launch
-        (call after every optimiser step on these parameters). `transposed` also makes the copy the backward reads."""
-        heads = self._heads()
-        packed, packed_t, bias, heads_w = get_C_function('mlp_pack_all')(
-            [l.weight.detach() for l in self.linear], [l.bias.detach() for l in self.linear],
-            [h.weight.detach() for h in heads], [h.bias.detach() for h in heads], self.skip, transposed)
+        (call after every optimiser step on these parameters), the copy the backward reads among them."""
+        packed, self._packed_t, bias, self._heads_w = host.mlp_pack(self._mlp_parameters(), self.D, self.skip)
         self._packed = (packed, bias)
-        self._packed_t = packed_t
-        self._heads_w = heads_w
         return self._packed
 
     def encode(self, x: Tensor, t: Tensor) -> Tensor:
@@ -94,21 +90,27 @@ class DeformNetwork(nn.Module):
         (network.py:1776). With gradients enabled the weights are re-packed when they changed since the last call and
         the output carries a backward (see `_DeformMlp`); under `torch.no_grad()` the cached pack is used."""
         params = self._mlp_parameters()
-        x_enc = self.encode(x, t)
-        n_out = 14 if self.local_frame else 10
-        track = torch.is_grad_enabled() and (x_enc.requires_grad or any(p.requires_grad for p in params))
+        track = torch.is_grad_enabled() and any(p.requires_grad for p in params)
         versions = tuple(p._version for p in params)
-        if self._packed is None or (track and (getattr(self, '_packed_versions', None) != versions or
-                                               self._packed_t is None)):
-            self.pack(transposed=track)
+        if self._packed is None or (track and getattr(self, '_packed_versions', None) != versions):
+            self.pack()
             self._packed_versions = versions
         packed, bias = self._packed
-        if track:
-            out = _DeformMlp.apply(x_enc, packed, bias, self._packed_t, self._heads_w, self.D, self.skip, n_out,
-                                   *params)
-        else:
-            out = get_C_function('mlp_forward')(x_enc.detach(), packed, bias, self.D, self.skip, n_out)
-        return self._split(out)
+        # the kernel forms the encoding itself for plain positions and one time
+        x_enc = None
+        if self.is_blender or t.numel() != 1 or x.dtype != torch.float32 or t.dtype != torch.float32 or \
+                (torch.is_grad_enabled() and (x.requires_grad or t.requires_grad)):
+            x_enc = self.encode(x, t)
+            if torch.is_grad_enabled() and x_enc.requires_grad:  # a gradient to the input: the time network, or the caller
+                return self._split(_DeformMlp.apply(x_enc, packed, bias, self._packed_t, self._heads_w, self.D, self.skip,
+                                                    14 if self.local_frame else 10, *params))
+        pos, time = self.pos_enc_p, self.pos_enc_t
+        d_xyz, rotation, scaling, *local = host.deform_mlp(
+            x.contiguous(), t.contiguous(), x_enc, packed, bias, self._packed_t, self._heads_w, pos.degree, pos.scale,
+            time.degree, time.scale, self.D, self.skip, [h.out_features for h in self._heads()], params)
+        if self.max_d_scale > 0:
+            scaling = torch.tanh(scaling) * math.log(self.max_d_scale)
+        return d_xyz, rotation, scaling, (local[0] if local else None)
 
     def forward_fp32(self, x: Tensor, t: Tensor):
         """The same network in plain fp32 torch (what the reference computes); used to state the bf16 tolerance."""
@@ -161,21 +163,6 @@ class _DeformMlp(torch.autograd.Function):
         return (g_in,) + (None,) * 7 + tuple(g if n else None for g, n in zip(grads, need))
 
 
-class _KnnTopk(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, y, K):
-        d2, idx = get_C_function('knn_topk')(x, y, K)
-        ctx.save_for_backward(x, y, idx)
-        ctx.mark_non_differentiable(idx)
-        return d2, idx
-
-    @staticmethod
-    def backward(ctx, g_d2, _):
-        x, y, idx = ctx.saved_tensors
-        g_x, g_y = get_C_function('knn_topk_backward')(x, y, idx, g_d2.contiguous(), ctx.needs_input_grad[0])
-        return g_x, (g_y if ctx.needs_input_grad[1] else None), None
-
-
 class _LbsBlend(torch.autograd.Function):
     """lbs_blend / lbs_blend_backward as one differentiable operator. Optional tensors are passed as None."""
 
@@ -220,7 +207,7 @@ def knn_points(points: Tensor, sp_points: Tensor, K: int):
     """Squared distances (ascending) and indices of the K nearest rows of `sp_points` for every row of `points`: the
     reference's `pytorch3d.ops.knn_points(points[None], sp_points[None], K=K)` (network.py:504) without the batch
     dimension. Differentiable in both point sets through the distances."""
-    return _KnnTopk.apply(points.contiguous(), sp_points.contiguous(), K)
+    return host.knn_points(points, sp_points, K)
 
 
 def calc_LBS_weight(points: Tensor, sp_points: Tensor, feature: Tensor = None, sp_feature: Tensor = None, K: int = 3,
@@ -284,6 +271,21 @@ def warp(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Tensor, sp_s: Te
     return d_xyz, d_rot, d_scale
 
 
+_FUSED_WEIGHTS = {'dist': 0, 'kernel': 1, 'weighted_kernel': 1}
+_FUSED_WARPS = {'LBS': 1, 'LBS_c': 2}
+
+
+def _fused_deform(points, sp_points, sp_t, sp_r, sp_s, sp_rot, K, temperature, warp_method, LBS_method, sp_radius,
+                  sp_weight, scale_columns):
+    """K-NN, weights and warp as one call and one autograd node; the scales are the first `scale_columns` of sp_s."""
+    mode = _FUSED_WEIGHTS[LBS_method]
+    if mode == 1 and (sp_radius is None or (LBS_method == 'weighted_kernel' and sp_weight is None)):
+        raise RuntimeError('superpoint_deform: the kernel weights need sp_radius, weighted_kernel also sp_weight')
+    return host.superpoint_warp(points, sp_points, sp_t, sp_r, sp_s, sp_rot, sp_radius if mode == 1 else None,
+                                sp_weight if LBS_method == 'weighted_kernel' else None, scale_columns, K,
+                                float(temperature), 0 if sp_rot is None else _FUSED_WARPS[warp_method], mode)
+
+
 def superpoint_deform(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Tensor, sp_s: Tensor,
                       sp_rot: Tensor = None, K: int = 3, temperature: float = 1.0, warp_method: str = 'LBS',
                       LBS_method: str = 'dist', sp_radius: Tensor = None, sp_weight: Tensor = None,
@@ -297,12 +299,15 @@ def superpoint_deform(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Ten
     sp_radius, sp_weight and sp_W; the returned weights are detached. As in the reference the Gaussians' positions are
     detached (:577, :501)."""
     points = points.detach()
+    if LBS_method in _FUSED_WEIGHTS and warp_method in _FUSED_WARPS and (feature is None or sp_feature is None):
+        return _fused_deform(points, sp_points, sp_t, sp_r, sp_s, sp_rot, K, temperature, warp_method, LBS_method,
+                             sp_radius, sp_weight, 0 if sp_s is None else sp_s.shape[1])
     if feature is not None and sp_feature is not None:
         x = torch.cat([points, feature], dim=-1)
         y = torch.cat([sp_points.detach(), sp_feature], dim=-1)
     else:
         x, y = points, sp_points
-    d2, idx = _KnnTopk.apply(x.contiguous(), y.contiguous(), K)
+    d2, idx = host.knn_points(x, y, K)
     if LBS_method == 'W':
         pair_in, radius, weight = torch.gather(sp_W, dim=1, index=idx), None, None
     elif LBS_method in ('kernel', 'weighted_kernel'):
@@ -322,37 +327,9 @@ def superpoint_deform(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Ten
     return d_xyz, d_rot, d_scale, w, idx
 
 
-class _DeformApply(torch.autograd.Function):
-    """points + d_xyz, act(scales) + d_scale, normalize(rotations + d_rotation) (network.py:630, :643, :645) as one
-    kernel forward and one backward; sums hand their upstream gradient to both addends unchanged."""
-
-    @staticmethod
-    def forward(ctx, points, d_xyz, scales, d_scale, rotations, d_rotation, log_scales):
-        args = [t.contiguous() for t in (points, d_xyz, scales, d_scale, rotations, d_rotation)]
-        out = get_C_function('deform_apply_forward')(*args, log_scales)
-        ctx.save_for_backward(args[2], args[4], args[5])
-        ctx.log_scales = log_scales
-        return out
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, g_points, g_scales, g_rot):
-        scales, rotations, d_rotation = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        gs = g_r = None
-        if need[4] or need[5] or (ctx.log_scales and need[2]):
-            gs, g_r = get_C_function('deform_apply_backward')(
-                scales, rotations, d_rotation, g_scales.contiguous() if ctx.log_scales else None, g_rot.contiguous(),
-                ctx.log_scales)
-        if not ctx.log_scales:
-            gs = g_scales
-        pick = lambda g, k: g if need[k] else None
-        return pick(g_points, 0), pick(g_points, 1), pick(gs, 2), pick(g_scales, 3), pick(g_r, 4), pick(g_r, 5), None
-
-
 def deform_apply(points: Tensor, d_xyz: Tensor, scales: Tensor, d_scale: Tensor, rotations: Tensor, d_rotation: Tensor,
                  log_scales: bool = False):
     """The deformed parameters handed to the renderer (reference: fast_2d_gs/network.py:630, :643, :645 with
     apply_rotate == 'add'): (points + d_xyz, scales + d_scale, normalize(rotations + d_rotation)); with `log_scales`
     the scales are stored as logarithms and exp is applied first (gaussian_splatting.py:142)."""
-    return _DeformApply.apply(points, d_xyz, scales, d_scale, rotations, d_rotation, bool(log_scales))
+    return tuple(host.deform_apply(points, d_xyz, scales, d_scale, rotations, d_rotation, bool(log_scales)))

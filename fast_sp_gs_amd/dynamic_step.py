@@ -14,9 +14,9 @@ from typing import Optional
 import torch
 from torch import Tensor
 
-from fast_sp_gs_amd.deform import DeformNetwork, deform_apply, superpoint_deform
+from fast_sp_gs_amd.deform import _FUSED_WARPS, DeformNetwork, _fused_deform, deform_apply, superpoint_deform
 from fast_sp_gs_amd.renderer import GS_2D_render
-from fast_sp_gs_amd.sparse_gaussian_adam import SparseGaussianAdam
+from fast_sp_gs_amd.sparse_gaussian_adam import DenseAdam, SparseGaussianAdam
 from fast_sp_gs_amd.ssim import l1_dssim_loss
 
 __all__ = ['DynamicStep']
@@ -38,7 +38,7 @@ class DynamicStep:
         self.params = [getattr(scene, k).detach().clone().requires_grad_(True) for k in PARAM_NAMES]
         self.opt = SparseGaussianAdam([{'params': [p], 'name': k} for p, k in zip(self.params, PARAM_NAMES)], lr=lr,
                                       eps=1e-15)
-        self.net_opt = torch.optim.Adam(list(self.net.parameters()) + [self.ctrl], lr=net_lr, fused=True)
+        self.net_opt = DenseAdam(list(self.net.parameters()) + [self.ctrl], lr=net_lr)
         self.sh_degree = scene.sh_degree
         # the reference's training render passes `accum_max_count` on every step (network.py:706): per Gaussian, the
         # number of (pixel, blended entry) events at which it was the pixel's strongest contributor so far
@@ -48,9 +48,16 @@ class DynamicStep:
         """-> (loss, render outputs). Differentiable in the Gaussians' parameters, the control points and the network."""
         means3D, scales, rotations, opacities, shs = self.params
         c_xyz, c_rot, c_scale, c_local = self.net(self.ctrl.detach(), t)
-        d_xyz, d_rot, d_scale, _, _ = superpoint_deform(
-            means3D.detach(), self.ctrl, c_xyz, c_rot, c_scale[:, :scales.shape[1]], sp_rot=c_local, K=self.K,
-            temperature=self.temperature, warp_method=self.warp_method, LBS_method=self.LBS_method)
+        columns = scales.shape[1]
+        if self.LBS_method == 'dist' and self.warp_method in _FUSED_WARPS:
+            # the network's scaling head as it is: no slice, no slice's gradient
+            d_xyz, d_rot, d_scale, _, _ = _fused_deform(
+                means3D.detach(), self.ctrl, c_xyz, c_rot, c_scale, c_local, self.K, self.temperature, self.warp_method,
+                self.LBS_method, None, None, columns)
+        else:
+            d_xyz, d_rot, d_scale, _, _ = superpoint_deform(
+                means3D.detach(), self.ctrl, c_xyz, c_rot, c_scale[:, :columns], sp_rot=c_local, K=self.K,
+                temperature=self.temperature, warp_method=self.warp_method, LBS_method=self.LBS_method)
         xyz, sc, rot = deform_apply(means3D, d_xyz, scales, d_scale, rotations, d_rot)
         cam = self.cam
         out = GS_2D_render(xyz, sc, rot, opacities, (cam.W, cam.H), cam.Tw2v, cam.Tv2c, campos=cam.campos,
@@ -61,8 +68,12 @@ class DynamicStep:
     def step(self, t: Tensor):
         """One full iteration; returns (loss, visibility mask) as device tensors (nothing is copied to the host)."""
         loss, out = self.forward_loss(t)
-        loss.backward()
-        visible = out['radii'] > 0
+        leaves = self.params + list(self.net.parameters()) + [self.ctrl]
+        # straight from the graph to the optimisers: accumulation into .grad would copy what two leaves share
+        for p, g in zip(leaves, torch.autograd.grad(loss, leaves, allow_unused=True)):
+            if g is not None:
+                p.grad = g if p.grad is None else p.grad + g
+        visible = out['visibility_filter']
         self.opt.set_before_step(visible, self.params[0].shape[0])
         self.opt.step()
         self.opt.zero_grad(set_to_none=True)

@@ -125,7 +125,4 @@ def require_dtype(what: str, name: str, t: torch.Tensor, dtype) -> None:
         raise RuntimeError(f"{what}: {name} must have dtype {dtype}, got {t.dtype}")
 
 
-_host = _host_layer()
-surfel_render = _host.surfel_render
-fast_surfel_render = _host.fast_surfel_render
-gaussian_render = _host.gaussian_render
+host = _host_layer()

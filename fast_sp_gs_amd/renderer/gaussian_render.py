@@ -12,7 +12,7 @@ import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
-from fast_sp_gs_amd.lib import gaussian_render as native_render
+from fast_sp_gs_amd.lib import host
 from fast_sp_gs_amd.renderer.gs_2d_render import GS_prepare
 
 _cull_masks = get_C_function('gs_cull_masks')
@@ -331,7 +331,7 @@ def _rasterize(means3D, means2D, preserve, colors, sh_rest, opacities, scales, r
         return _rasterize_operators(means3D, means2D, colors, sh_rest, opacities, scales, rotations, cov3D, cov2D,
                                     extras, (W, H), sh_degree, Tw2v, Tv2c, cam_pos, tanFoV, is_opengl, culling,
                                     accum_max_count, accum_weights_p, accum_weights_count, *other_extras)
-    maps, n_contrib, radii, visible, tile_ranges, point_list = native_render(
+    maps, n_contrib, radii, visible, tile_ranges, point_list = host.gaussian_render(
         means3D, scales, rotations, opacities, colors, sh_rest, cov3D, cov2D, means2D, extras, Tw2v, Tv2c, cam_pos,
         culling, accum_max_count, accum_weights_p, accum_weights_count, float(tanFoV[0]), float(tanFoV[1]), W, H,
         int(sh_degree), bool(is_opengl), preserve, bool(CULL_LISTS))

@@ -9,7 +9,7 @@ import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
-from fast_sp_gs_amd.lib import fast_surfel_render
+from fast_sp_gs_amd.lib import host
 from .gs_2d_render import depth_to_normal
 
 __all__ = ['GS_2D_fast_render', 'GS_2D_fast_preprocess', 'GS_2D_fast_rasterize', 'GS_2D_fast_rasterize_v2',
@@ -260,7 +260,7 @@ def GS_2D_fast_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity
     # camera optimisation: the fused epilogue produces no camera gradients, take the reference's torch ops
     fused = not (Tw2v.requires_grad or Tv2c.requires_grad)
     depth_ratio = float(depth_ratio)
-    maps, radii, visible = fast_surfel_render(
+    maps, radii, visible = host.fast_surfel_render(
         points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest, means2D,
         Tw2v.contiguous(), Tv2c.contiguous(), Tv2s.contiguous(), campos.contiguous(), trans_mat_t2, culling,
         accum_max_count, accum_weights_p, accum_weights_count, W, H, int(sh_degree) if colors is None else -1,

@@ -11,7 +11,7 @@ import torch
 from torch import Tensor
 
 from fast_sp_gs_amd._C import get_C_function
-from fast_sp_gs_amd.lib import surfel_render
+from fast_sp_gs_amd.lib import host
 
 __all__ = ['GS_2D_render', 'RasterizeBuffer', 'GS_2D_topk_weights', 'GS_prepare', 'render_step']
 
@@ -149,7 +149,7 @@ def GS_2D_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity: Ten
     # camera optimisation: the fused epilogue produces no camera gradients, take the reference's torch ops
     fused = not (Tw2v.requires_grad or Tv2c.requires_grad)
     near, far, depth_ratio = float(near), float(far), float(depth_ratio)
-    maps, n_contrib, radii, visible, tile_range, point_list, normal_opacity, trans_mat = surfel_render(
+    maps, n_contrib, radii, visible, tile_range, point_list, normal_opacity, trans_mat = host.surfel_render(
         points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest, means2D,
         Tw2v.contiguous(), Tv2c.contiguous(), campos.contiguous(),
         background.detach().reshape(3).contiguous() if fused and background is not None else None, trans_mat_t2, culling,

@@ -5,14 +5,13 @@ import torch
 import torch.optim
 
 from fast_sp_gs_amd._C import get_C_function
+from fast_sp_gs_amd.lib import host
 
-__all__ = ['SparseGaussianAdam']
+__all__ = ['SparseGaussianAdam', 'DenseAdam']
 
 
 class SparseGaussianAdam(torch.optim.Adam):
     _update_C = staticmethod(get_C_function('AdamMasksedUpdated'))
-    _update_multi_C = staticmethod(get_C_function('AdamMasksedUpdatedMulti'))
-    _MAX = 12  # tensors per launch (fsgs_adam_masked_update_max_tensors)
 
     def __init__(self, params, lr, eps):
         super().__init__(params=params, lr=lr, eps=eps)
@@ -33,7 +32,7 @@ class SparseGaussianAdam(torch.optim.Adam):
     @torch.no_grad()
     def step(self):
         """One masked Adam update of every parameter group that has a gradient (sparse_gaussian_adam.py:20-45), the
-        groups' kernels folded into one launch per `_MAX` tensors; the arithmetic per element is the single-tensor
+        groups' kernels folded into one launch; the arithmetic per element is the single-tensor
         kernel's."""
         jobs = []  # (param, grad, first moment, second moment, effective rate, eps)
         corrections = {}  # step count -> the two bias corrections, shared by the groups that are at that count
@@ -56,9 +55,46 @@ class SparseGaussianAdam(torch.optim.Adam):
             root_c2, c1 = corrections[key]
             jobs.append((param, param.grad, state["exp_avg"], state["exp_avg_sq"],
                          float(np.float32(group["lr"]) * root_c2 / c1), group["eps"]))
-        for i in range(0, len(jobs), self._MAX):
-            p, g, m, v, rates, epss = map(list, zip(*jobs[i:i + self._MAX]))
-            self._update_multi_C(p, g, m, v, self.visibility, rates, 0.9, 0.999, epss, self.N)
+        if jobs:
+            p, g, m, v, rates, epss = map(list, zip(*jobs))
+            host.adam_masked(p, g, m, v, self.visibility, rates, 0.9, 0.999, epss, self.N)
 
     def set_before_step(self, visibility, N):
         self.visibility, self.N = visibility, N
+
+
+class DenseAdam(torch.optim.Adam):
+    """torch.optim.Adam with the plain update (no weight decay, amsgrad, maximize, capturable) of all of a group's float32
+    tensors in one launch; state keys as torch's, so checkpoints load either way. Any other setting takes torch's step. As
+    with torch's fused step the parameters' version counters stay: whoever keeps copies of them (`DeformNetwork.pack`)
+    refreshes those itself."""
+
+    @torch.no_grad()
+    def step(self, closure=None):
+        groups = self.param_groups
+        if closure is not None or any(g['weight_decay'] or g['amsgrad'] or g['maximize'] or g['capturable'] or g['fused'] or
+                                      g['differentiable'] or isinstance(g['lr'], torch.Tensor) for g in groups):
+            return super().step(closure)
+        if any(p.grad is not None and (p.grad.is_sparse or p.dtype != torch.float32 or not p.is_cuda or not p.is_contiguous())
+               for g in groups for p in g['params']):
+            return super().step()
+        for group in groups:
+            params = [p for p in group['params'] if p.grad is not None]
+            if not params:
+                continue
+            fresh = [p for p in params if not self.state[p]]
+            if fresh:
+                count = torch.zeros((), dtype=torch.float32)
+                for p in fresh:
+                    self.state[p].update(step=count, exp_avg=torch.zeros_like(p), exp_avg_sq=torch.zeros_like(p))
+            states = [self.state[p] for p in params]
+            counts = {id(s['step']): s['step'] for s in states}  # tensors first seen together share theirs
+            b1, b2 = group['betas']
+            factors = {}
+            for key, count in counts.items():
+                count += 1
+                t = count.item()
+                factors[key] = (group['lr'] / (1 - b1 ** t), (1 - b2 ** t) ** 0.5)
+            per = [factors[id(s['step'])] for s in states]
+            host.adam_dense(params, [p.grad for p in params], [s['exp_avg'] for s in states],
+                            [s['exp_avg_sq'] for s in states], [f[0] for f in per], [f[1] for f in per], b1, b2, group['eps'])

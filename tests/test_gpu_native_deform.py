@@ -1,0 +1,83 @@
+"""The deformation branch through the native host layer against the operators and torch: the network with its encoding
+formed in the kernel (rows around a block of 32, one head missing its gradient), the K-NN + warp node with a slice of a wider scaling head, the dense Adam."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('B', [1, 31, 32, 33, 300])
+@pytest.mark.parametrize('local_frame', [False, True])
+def test_network_equals_encoded_rows(B, local_frame, device):
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.deform import DeformNetwork, _DeformMlp
+    torch.manual_seed(B)
+    net = DeformNetwork(local_frame=local_frame).to(device)
+    g = torch.Generator().manual_seed(B)
+    x, t = (torch.rand(B, 3, generator=g) * 2 - 1).to(device), torch.rand(1, generator=g).to(device)
+    out = [o for o in net(x, t) if o is not None]
+    params = net._mlp_parameters()
+    rows = sum(h.out_features for h in net._heads())
+    ref = _DeformMlp.apply(net.encode(x, t), *net._packed, net._packed_t, net._heads_w, net.D, net.skip, rows, *params)
+    assert torch.equal(torch.cat(out, 1), ref)
+    with torch.no_grad():
+        assert all(torch.equal(a, b) for a, b in zip(net(x, t), out))
+    up = torch.randn(B, rows, generator=g).to(device)
+    up[:, 3:7] = 0  # the rotation head gets no gradient below
+    parts = [p for p in up.split([h.out_features for h in net._heads()], dim=1)]
+    keep = [k for k in range(len(out)) if k != 1]
+    got = torch.autograd.grad([out[k] for k in keep], params, [parts[k].contiguous() for k in keep], allow_unused=True)
+    want = torch.autograd.grad(ref, params, up)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    hidden = get_C_function('mlp_forward')(net.encode(x, t), *net._packed, net.D, net.skip, rows, True)[1]
+    assert hidden.shape == (net.D, B, 256) and bool((hidden.view(torch.bfloat16) >= 0).all())
+
+
+@pytest.mark.parametrize('N,M,K,warp,columns', [(1, 1, 1, 'LBS', 3), (1000, 40, 3, 'LBS', 2), (1025, 300, 4, 'LBS_c', 2),
+                                                (777, 65, 5, None, 1)])
+def test_warp_node_equals_operators(N, M, K, warp, columns, device):
+    from fast_sp_gs_amd.deform import _fused_deform, _LbsBlend, knn_points
+    g = torch.Generator().manual_seed(N)
+    mk = lambda *s: torch.randn(*s, generator=g).to(device).requires_grad_(True)
+    points, ctrl, sp_t, sp_r, sp_s = mk(N, 3).detach(), mk(M, 3), mk(M, 3), mk(M, 4), mk(M, 3)
+    sp_rot = mk(M, 4) if warp else None
+    out = _fused_deform(points, ctrl, sp_t, sp_r, sp_s, sp_rot, K, 0.5, warp or 'LBS', 'dist', None, None, columns)
+    d2, idx = knn_points(points, ctrl, K)
+    ref = _LbsBlend.apply(points, ctrl, sp_t, sp_r, sp_s[:, :columns], sp_rot, d2, idx, None, None, 0.5, warp, 'dist')
+    for a, b in zip(out[:4], ref):
+        assert torch.equal(a, b)
+    assert torch.equal(out[4], idx)
+    up = [torch.randn(o.shape, generator=g).to(device) for o in ref[:3]]
+    wanted = [ctrl, sp_t, sp_r, sp_s] + ([sp_rot] if warp else [])
+    for a, b in zip(torch.autograd.grad(out[:3], wanted, up), torch.autograd.grad(ref[:3], wanted, up)):
+        assert (a - b).norm() <= 1e-5 * b.norm() + 1e-7
+
+
+def test_dense_adam_follows_torch(device):
+    from fast_sp_gs_amd.deform import DeformNetwork
+    from fast_sp_gs_amd.sparse_gaussian_adam import DenseAdam
+    g = torch.Generator().manual_seed(3)
+    shapes = [(1,), (1023,), (1024,), (1025,), (256, 340)] * 7  # more tensors than one launch takes
+    values = [torch.randn(s, generator=g) for s in shapes]
+    mine, theirs = ([v.clone().to(device).requires_grad_(True) for v in values] for _ in range(2))
+    a, b = DenseAdam(mine, lr=1e-2), torch.optim.Adam(theirs, lr=1e-2)
+    for _ in range(3):
+        for p, q in zip(mine, theirs):
+            p.grad = torch.randn(p.shape, generator=g).to(device)
+            q.grad = p.grad.clone()
+        a.step(), b.step()
+    for p, q in zip(mine, theirs):
+        assert torch.allclose(p, q, rtol=0, atol=1e-6) and float(a.state[p]['step']) == 3
+        assert torch.allclose(a.state[p]['exp_avg_sq'], b.state[q]['exp_avg_sq'], rtol=1e-5, atol=1e-9)
+    b.load_state_dict(a.state_dict())
+    net = DeformNetwork().to(device)
+    opt = DenseAdam(net.parameters(), lr=1e-2)
+    x, t = torch.rand(64, 3, generator=g).to(device), torch.rand(1, generator=g).to(device)
+    first = net(x, t)[0]
+    first.sum().backward()
+    opt.step()
+    net.pack()
+    second = net(x, t)[0]
+    assert not torch.equal(first, second)  # the step's weights are in use
+    assert (second - net.forward_fp32(x, t)[0]).norm() <= 2e-2 * second.norm() + 1e-5
