@@ -5,11 +5,11 @@
 // linear maps of the last hidden state (gaussian_warp 3, gaussian_rotation 4, gaussian_scaling 3 stacked into one
 // [n_out, 256] matrix by the caller).
 //
-// One block owns 32 rows (control points) and keeps their activations in LDS for the whole network, so the only HBM/L2
+// One block owns 16 rows (control points) and keeps their activations in LDS for the whole network, so the only HBM/L2
 // traffic is the weights (about 1 MB in bf16, shared by all blocks through L2) and 40 bytes of output per row.
-// Each of the 8 wavefronts computes a 32 x 32 slab of a layer's output with v_mfma_f32_32x32x16_bf16: A fragments
+// Each of the 8 wavefronts computes a 16 x 32 slab of a layer's output with v_mfma_f32_16x16x32_bf16: A fragments
 // (activations) come from LDS as one 16-byte read per lane, B fragments (weights, packed in fragment order, see
-// frag_index) as one 16-byte global read per lane; both use the same (lane / 32, element) -> k mapping, so the product
+// frag_index) as one 16-byte global read per lane; both use the same (lane / 16, element) -> k mapping, so the product
 // is independent of how the hardware orders k inside a fragment. The input rows are either given or formed here from
 // positions and time (the frequency encoding), which spares three launches and a [B][84] tensor.
 //
@@ -25,9 +25,9 @@
 //     16-byte loads of consecutive memory. A block owns a 64 x 64 tile, its four wavefronts take a share of the batch each
 //     with every load of 128 rows in flight, and add their sums through LDS in wavefront order; the first tile column of a
 //     layer also sums dZ over the batch for the bias gradient. No atomics: every output element has one writer.
-// Both chains are bound by latency: 16 blocks at B = 512, nine dependent layers. At B = 512, 8 layers (us): forward 48,
-// chain 42, weight gradients 48 before the loads of a layer were ordered so that none waits for the next layer's
-// prefetched weights and the weight gradients' operands went through LDS transposed two bytes at a time.
+// The chains' time is nine dependent layers of one block, so what a layer costs a compute unit counts: LDS reads, matrix
+// products and the epilogue's conversions all halve with 16 rows in place of 32. At B = 512 and 8 layers: forward 39 -> 20
+// us, backward chain 41 -> 27, weight gradients (operands transposed through LDS two bytes at a time before) 48 -> 11.
 // Gradients with respect to the (frequency-encoded) input are not produced; the reference detaches it
 // (network.py:586).
 #include <algorithm>
@@ -39,15 +39,16 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMlpWidth   = 256;
-constexpr int kMlpRows    = 32;                       // rows per block
+constexpr int kMlpRows    = 16;                       // rows per block of the chains
+constexpr int kMlpRowPad  = 32;                       // the saved tensors' batch is padded to this
 constexpr int kMlpMaxIn   = 96;                       // padded input width limit
 constexpr int kMlpStride  = kMlpWidth + kMlpMaxIn + 8;  // LDS row stride in bf16 (+8 keeps 16-byte rows off one bank)
 constexpr int kMlpThreads = 256;
-// Forward and backward chain: eight wavefronts per block, one 32 x 32 output tile each. The batch is small (16 blocks at
-// B = 512) and the nine layers depend on each other, so a layer's time is the latency of its weight fragments: with one
-// tile per wavefront a whole layer's 16 fragments fit in registers and are requested together.
+// Forward and backward chain: eight wavefronts per block, 16 x 32 outputs each. With that little per wavefront a whole
+// layer's 16 fragments fit in registers and are requested together.
 constexpr int kChainThreads = 512;
 
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {  // round to nearest even
@@ -153,38 +154,77 @@ __device__ __forceinline__ uint2 pack4(const uint16_t* h) {
   return make_uint2((uint32_t) h[0] | ((uint32_t) h[1] << 16), (uint32_t) h[2] | ((uint32_t) h[3] << 16));
 }
 
+// Two values rounded to nearest even by the conversion instruction (the chains' epilogues are vector-bound: with the
+// rounding written out in integer arithmetic a layer's epilogue was 760 instructions, half of its time).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 h = {(__bf16) lo, (__bf16) hi};
+  return __builtin_bit_cast(uint32_t, h);
+}
+
+// A block streams all of the weights, 1.1 MB, through one compute unit, and how fast it can is a matter of latency: about
+// 35 GB/s when the lines come from beyond the L2 (30 us). With few row blocks most of the chip is idle, so some blocks more
+// fetch the weights into every L2 (blocks go round the 8 XCDs in turn), all of them together from the first layer on.
+constexpr int kFetchParts = 8;                // blocks per XCD that fetch
+constexpr int kFetchBlocks = 8 * kFetchParts;
+constexpr int kFetchBelow = 128;              // row blocks; with more of them the weights are in every L2 soon enough
+__device__ __forceinline__ void fetch_to_l2(const uint16_t* __restrict__ data, size_t elems, int part) {
+  const uint4* p = (const uint4*) data;
+  const size_t n = elems / 8;
+  for (size_t e = (size_t) part * kChainThreads + threadIdx.x; e < n; e += (size_t) kFetchParts * kChainThreads * 4) {
+    uint4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = p[min(e + (size_t) k * kFetchParts * kChainThreads, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) asm volatile("" ::"v"(v[k].x));
+  }
+}
+
+// B fragments of a wavefront's two 16-column tiles for k-step kk (32 values of k) of the matrix whose row tile (32 rows, one
+// per output) starts at `tile`: tile elements are laid out by frag_index, so a fragment is four runs of 256 bytes. A
+// matrix with an odd number of 16-column steps ends in half a step; its missing half re-reads the last one and meets zeros.
+__device__ __forceinline__ void load_fragments(const uint16_t* __restrict__ tile, int kk, int last_step, bf16x8 (&b)[2]) {
+  const int lane = threadIdx.x & 63, ks = min(2 * kk + (lane >> 5), last_step), half = (lane >> 4) & 1;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) b[t] = *(const bf16x8*) (tile + ks * 512 + (16 * t + (lane & 15) + 32 * half) * 8);
+}
+
+// D layout of the 16x16 accumulator: register r of lane l holds row 4 * (l / 16) + r, column l % 16.
 // `in` or `freq.x` gives the input rows. in_t / saved (kSave): see the file's head.
 template <bool kSave>
 __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int Din, int n_layers, int skip, int n_out,
     const float* __restrict__ in, FreqInput freq, const uint16_t* __restrict__ packed, const float* __restrict__ bias,
-    MlpHeads heads, uint16_t* __restrict__ in_t, uint16_t* __restrict__ saved) {
+    MlpHeads heads, uint16_t* __restrict__ in_t, uint16_t* __restrict__ saved, int row_blocks, size_t packed_elems) {
+  if ((int) blockIdx.x >= row_blocks) {
+    fetch_to_l2(packed, packed_elems, ((int) blockIdx.x - row_blocks) / 8);
+    return;
+  }
   __shared__ __attribute__((aligned(16))) uint16_t s_act[2][kMlpRows][kMlpStride];
   __shared__ __attribute__((aligned(16))) uint16_t s_in[kMlpRows][kMlpMaxIn + 8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * kMlpRows;
   const int Din_pad = (Din + 15) & ~15;
-  const size_t B_pad = (size_t) gridDim.x * kMlpRows;
-  const int arow = lane & 31, kofs = 8 * (lane >> 5), col = wave * 32 + (lane & 31);
+  const size_t B_pad = (size_t) row_blocks * kMlpRows;
+  const int arow = lane & 15, kofs = 8 * (lane >> 4), col = wave * 32 + (lane & 15);  // and column col + 16
 
   const uint16_t* W = packed;
   const float* bl   = bias;
-  // Fragment u (k-step u, clamped to the layer's last step) of row tile `wave` of a layer whose weights start at Wl;
-  // consecutive k-steps are 512 elements apart.
-  auto fragment = [&](const uint16_t* Wl, int K_pad_l, int u) {
-    const int steps = K_pad_l >> 4;
-    return *(const bf16x8*) (Wl + ((size_t) wave * steps + min(u, steps - 1)) * 512 + lane * 8);
-  };
-  // The weights do not depend on the activations: the first sixteen fragments (and the bias) of the NEXT layer are
+  auto tile_of = [&](const uint16_t* Wl, int K_pad_l) { return Wl + wave * (K_pad_l >> 4) * 512; };
+  // The weights do not depend on the activations: the first eight k-steps' fragments (and the bias) of the NEXT layer are
   // requested at the start of each layer and arrive while this layer's products, epilogue and barrier run. Nothing else is
   // loaded behind them: loads complete in order, and a wait for a later one would be a wait for all of these.
-  bf16x8 ahead[16];
-  float bias_ahead = bl[col];
+  // Two register sets take turns: handing one over to the next layer by copies would make the compiler wait for the
+  // prefetch where the copies are, in front of the products.
+  bf16x8 even[8][2], odd[8][2];
+  float bias_even[2] = {bl[col], bl[col + 16]}, bias_odd[2] = {0.0f, 0.0f};
 #pragma unroll
-  for (int u = 0; u < 16; ++u) ahead[u] = fragment(W, Din_pad, u);
+  for (int u = 0; u < 8; ++u)
+    if (32 * u < Din_pad) load_fragments(tile_of(W, Din_pad), u, (Din_pad >> 4) - 1, even[u]);
 
-  // stage the (bf16) input rows, zero padded
-  for (int e = threadIdx.x; e < kMlpRows * Din_pad; e += kChainThreads) {
-    const int r = e / Din_pad, k = e - r * Din_pad;
+  // stage the (bf16) input rows, zero padded to whole k-steps
+  constexpr int kInPad = kMlpMaxIn;
+  for (int e = threadIdx.x; e < kMlpRows * kInPad; e += kChainThreads) {
+    const int r = e / kInPad, k = e - r * kInPad;
     float v = 0.0f;
     if (row0 + r < B && k < Din) v = in ? in[(size_t) (row0 + r) * Din + k] : encoded(freq, row0 + r, k);
     const uint16_t h = f32_to_bf16(v);
@@ -194,97 +234,109 @@ __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int D
   __syncthreads();
   if (kSave) {
     for (int e = threadIdx.x; e < Din * (kMlpRows / 4); e += kChainThreads) {
-      const int k = e >> 3, r = (e & 7) * 4;
+      const int k = e >> 2, r = (e & 3) * 4;
       const uint16_t h[4] = {s_in[r][k], s_in[r + 1][k], s_in[r + 2][k], s_in[r + 3][k]};
       *(uint2*) (in_t + (size_t) k * B_pad + row0 + r) = pack4(h);
     }
   }
 
   int cur = 0, K_pad = Din_pad;
-  for (int layer = 0; layer < n_layers; ++layer) {
-    floatx16 acc;
+  auto run_layer = [&](int layer, const bf16x8 (&b)[8][2], const float (&bv)[2], bf16x8 (&ahead)[8][2], float (&bias_ahead)[2]) {
+    floatx4 acc[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    bf16x8 b[16], tail[6];
-    const float bv = bias_ahead;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 16; ++u) b[u] = ahead[u];
-    const int steps = K_pad >> 4;
-    if (steps > 16) {  // the layer behind the re-concatenated input: up to six k-steps more
+      for (int r = 0; r < 4; ++r) acc[t][r] = 0.0f;
+    bf16x8 tail[3][2];
+    const int last_step = (K_pad >> 4) - 1;
+    if (K_pad > kMlpWidth) {  // the layer behind the re-concatenated input: up to three k-steps more
 #pragma unroll
-      for (int u = 0; u < 6; ++u) tail[u] = fragment(W, K_pad, 16 + u);
+      for (int u = 0; u < 3; ++u) load_fragments(tile_of(W, K_pad), 8 + u, last_step, tail[u]);
     }
     const int K_next = layer == skip ? Din + kMlpWidth : kMlpWidth, K_next_pad = (K_next + 15) & ~15;
     const uint16_t* W_next = W + (size_t) kMlpWidth * K_pad;
     if (layer + 1 < n_layers) {
-      bias_ahead = bl[kMlpWidth + col];
+      bias_ahead[0] = bl[kMlpWidth + col], bias_ahead[1] = bl[kMlpWidth + col + 16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) ahead[u] = fragment(W_next, K_next_pad, u);
+      for (int u = 0; u < 8; ++u) load_fragments(tile_of(W_next, K_next_pad), u, 15, ahead[u]);
     }
     const uint16_t* arow_at = &s_act[cur][arow][kofs];
-    if (steps >= 16) {
+    auto product = [&](int kk, const bf16x8 (&w)[2]) {
+      const bf16x8 a = *(const bf16x8*) (arow_at + 32 * kk);
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 16 * u), b[u], acc, 0, 0, 0);
-      if (steps > 16) {
+      for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[t], acc[t], 0, 0, 0);
+    };
+    if (K_pad >= kMlpWidth) {
 #pragma unroll
-        for (int u = 0; u < 6; ++u)
-          if (16 + u < steps)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 256 + 16 * u), tail[u], acc, 0, 0, 0);
+      for (int u = 0; u < 8; ++u) product(u, b[u]);
+      if (K_pad > kMlpWidth) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+          if (kMlpWidth + 32 * u < K_pad) product(8 + u, tail[u]);
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < 6; ++u)
-        if (u < steps)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) (arow_at + 16 * u), b[u], acc, 0, 0, 0);
+      for (int u = 0; u < 3; ++u)
+        if (32 * u < K_pad) product(u, b[u]);
     }
     // bias + ReLU -> bf16 into the other buffer; after the skip layer the input goes in front of the hidden state
     const int nxt = cur ^ 1;
     const int col_shift = (layer == skip) ? Din : 0;
-    uint16_t h[16];
+    uint16_t* to = &s_act[nxt][4 * (lane >> 4)][col_shift + col];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      h[r] = f32_to_bf16(fmaxf(acc[r] + bv, 0.0f));
-      s_act[nxt][acc_row(r, lane)][col_shift + col] = h[r];
-    }
-    if (kSave) {
-      uint16_t* dst = saved + ((size_t) layer * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
+    for (int t = 0; t < 2; ++t) {
+      float v[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) *(uint2*) (dst + 8 * g) = pack4(h + 4 * g);
+      for (int k = 0; k < 4; ++k) v[k] = fmaxf(acc[t][k] + bv[t], 0.0f);
+      const uint2 h = make_uint2(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]));
+      uint16_t* row = to + 16 * t;
+      row[0] = (uint16_t) h.x, row[kMlpStride] = (uint16_t) (h.x >> 16);
+      row[2 * kMlpStride] = (uint16_t) h.y, row[3 * kMlpStride] = (uint16_t) (h.y >> 16);
+      if (kSave) *(uint2*) (saved + ((size_t) layer * kMlpWidth + col + 16 * t) * B_pad + row0 + 4 * (lane >> 4)) = h;
     }
     if (layer == skip) {
-      for (int e = threadIdx.x; e < kMlpRows * Din; e += kChainThreads) {
-        const int r = e / Din, k = e - r * Din;
-        s_act[nxt][r][k] = s_in[r][k];
+      for (int e = threadIdx.x; e < kMlpRows * kInPad; e += kChainThreads) {
+        const int r = e / kInPad, k = e - r * kInPad;
+        if (k < Din) s_act[nxt][r][k] = s_in[r][k];
+        else s_act[nxt][r][kMlpWidth + k] = 0;  // columns Din + 256 .. 256 + kInPad
       }
-      for (int e = threadIdx.x; e < kMlpRows * 16; e += kChainThreads)
-        if (K_next + (e & 15) < K_next_pad) s_act[nxt][e >> 4][K_next + (e & 15)] = 0;
     }
     lds_barrier();
     W = W_next;
     bl += kMlpWidth;
     K_pad = K_next_pad;
     cur = nxt;
+  };
+  for (int layer = 0; layer < n_layers; layer += 2) {
+    run_layer(layer, even, bias_even, odd, bias_odd);
+    if (layer + 1 < n_layers) run_layer(layer + 1, odd, bias_odd, even, bias_even);
   }
 
   // heads: one padded 32-column tile, wavefront 0 only
   if (wave == 0) {
-    const int head_col = lane & 31;
-    const float bv = head_col < n_out ? bl[head_col] : 0.0f;
-    bf16x8 b[16];
+    bf16x8 b[8][2];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) b[u] = *(const bf16x8*) (W + u * 512 + lane * 8);
-    floatx16 acc;
+    for (int u = 0; u < 8; ++u) load_fragments(W, u, 15, b[u]);
+    floatx4 acc[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) &s_act[cur][arow][kofs + 16 * u], b[u], acc, 0, 0, 0);
-    if (head_col < n_out) {
+      for (int r = 0; r < 4; ++r) acc[t][r] = 0.0f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = row0 + acc_row(r, lane);
-        if (row < B) *head_cell(heads, row, head_col) = acc[r] + bv;
+    for (int u = 0; u < 8; ++u) {
+      const bf16x8 a = *(const bf16x8*) &s_act[cur][arow][kofs + 32 * u];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[u][t], acc[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int head_col = 16 * t + (lane & 15);
+      if (head_col >= n_out) continue;
+      const float bv = bl[head_col];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = row0 + 4 * (lane >> 4) + r;
+        if (row < B) *head_cell(heads, row, head_col) = acc[t][r] + bv;
       }
     }
   }
@@ -298,30 +350,35 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_floa
 __global__ void __launch_bounds__(kChainThreads) mlp_backward_chain_kernel(int B, int Din, int n_layers, int n_out,
     const float* __restrict__ in, const float* __restrict__ heads_w /*[n_out][256] fp32*/,
     const uint16_t* __restrict__ packed_t, const uint16_t* __restrict__ saved, MlpHeads heads,
-    uint16_t* __restrict__ dz, uint16_t* __restrict__ g_t, uint16_t* __restrict__ in_t) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_dz[2][kMlpRows][kMlpWidth + 8];
+    uint16_t* __restrict__ dz, uint16_t* __restrict__ g_t, uint16_t* __restrict__ in_t, int row_blocks) {
+  if ((int) blockIdx.x >= row_blocks) {
+    // the last layer's weights are used first: whole layers from the back
+    for (int l = n_layers - 1; l >= 1; --l)
+      fetch_to_l2(packed_t + (size_t) (l - 1) * kMlpWidth * kMlpWidth, kMlpWidth * kMlpWidth, ((int) blockIdx.x - row_blocks) / 8);
+    return;
+  }
+  constexpr int kStride = kMlpWidth + 8;
+  __shared__ __attribute__((aligned(16))) uint16_t s_dz[2][kMlpRows][kStride];
   __shared__ float s_g[kMlpRows][33];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * kMlpRows;
-  const size_t B_pad = (size_t) gridDim.x * kMlpRows;
-  const int arow = lane & 31, kofs = 8 * (lane >> 5), col = wave * 32 + (lane & 31);
-  auto fragment = [&](int layer, int u) {
-    return *(const bf16x8*) (packed_t + ((size_t) ((layer - 1) * 8 + wave) * (kMlpWidth / 16) + u) * 512 + lane * 8);
-  };
-  // the stored states that mask a layer's result: four consecutive rows of the lane's column per load
-  auto mask_of = [&](int layer, uint2* keep) {
-    const uint16_t* src = saved + ((size_t) layer * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
+  const size_t B_pad = (size_t) row_blocks * kMlpRows;
+  const int arow = lane & 15, kofs = 8 * (lane >> 4), col = wave * 32 + (lane & 15);  // and column col + 16
+  auto fetch_weights = [&](int layer, bf16x8 (&b)[8][2]) {
+    const uint16_t* tile = packed_t + ((layer - 1) * 8 + wave) * (kMlpWidth / 16) * 512;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) keep[g] = *(const uint2*) (src + 8 * g);
+    for (int u = 0; u < 8; ++u) load_fragments(tile, u, 15, b[u]);
+  };
+  // the stored states that mask a layer's result: four consecutive rows of a column per load
+  auto fetch_mask = [&](int layer, uint2 (&keep)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      keep[t] = *(const uint2*) (saved + ((size_t) layer * kMlpWidth + col + 16 * t) * B_pad + row0 + 4 * (lane >> 4));
   };
   // one layer ahead of their use, the masks in front of the weights (loads complete in order)
-  uint2 keep_ahead[4];
-  bf16x8 ahead[16];
-  if (n_layers >= 2) {
-    mask_of(n_layers - 2, keep_ahead);
-#pragma unroll
-    for (int u = 0; u < 16; ++u) ahead[u] = fragment(n_layers - 1, u);
-  }
+  uint2 keep_even[2], keep_odd[2];
+  bf16x8 even[8][2], odd[8][2];
+  if (n_layers >= 2) fetch_mask(n_layers - 2, keep_even), fetch_weights(n_layers - 1, even);
   for (int e = threadIdx.x; e < kMlpRows * 32; e += kChainThreads) {
     const int r = e >> 5, k = e & 31;
     const float* cell = (row0 + r < B && k < n_out) ? head_cell(heads, row0 + r, k) : nullptr;
@@ -335,66 +392,64 @@ __global__ void __launch_bounds__(kChainThreads) mlp_backward_chain_kernel(int B
   }
   __syncthreads();
   for (int e = threadIdx.x; e < 32 * kMlpRows; e += kChainThreads)
-    g_t[(size_t) (e >> 5) * B_pad + row0 + (e & 31)] = f32_to_bf16(s_g[e & 31][e >> 5]);
+    g_t[(size_t) (e / kMlpRows) * B_pad + row0 + e % kMlpRows] = f32_to_bf16(s_g[e % kMlpRows][e / kMlpRows]);
   {
-    // dZ of the last layer: (g_out . W_heads) where the stored state is non-zero. A lane owns 16 rows of one column.
-    const int c = threadIdx.x & 255, r0 = 16 * (threadIdx.x >> 8);
+    // dZ of the last layer: (g_out . W_heads) where the stored state is non-zero. A lane owns 8 rows of one column.
+    const int c = threadIdx.x & 255, r0 = 8 * (threadIdx.x >> 8);
     const size_t top = ((size_t) (n_layers - 1) * kMlpWidth + c) * B_pad + row0 + r0;
-    uint4 keep[2] = {*(const uint4*) (saved + top), *(const uint4*) (saved + top + 8)};
-    float v[16];
+    const uint4 keep = *(const uint4*) (saved + top);
+    float v[8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = 0.0f;
+    for (int r = 0; r < 8; ++r) v[r] = 0.0f;
     for (int k = 0; k < n_out; ++k) {
       const float wv = heads_w[k * kMlpWidth + c];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) v[r] += s_g[r0 + r][k] * wv;
+      for (int r = 0; r < 8; ++r) v[r] += s_g[r0 + r][k] * wv;
     }
-    const uint32_t words[8] = {keep[0].x, keep[0].y, keep[0].z, keep[0].w, keep[1].x, keep[1].y, keep[1].z, keep[1].w};
-    uint16_t h[16];
+    const uint32_t words[4] = {keep.x, keep.y, keep.z, keep.w};
+    uint32_t h[4];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const bool on = ((words[r >> 1] >> (16 * (r & 1))) & 0xffffu) != 0u && row0 + r0 + r < B;
-      h[r] = on ? f32_to_bf16(v[r]) : (uint16_t) 0;
-      s_dz[0][r0 + r][c] = h[r];
+    for (int q = 0; q < 4; ++q) {
+      const bool lo = (words[q] & 0xffffu) != 0u && row0 + r0 + 2 * q < B, hi = (words[q] >> 16) != 0u && row0 + r0 + 2 * q + 1 < B;
+      h[q] = bf16_pair(lo ? v[2 * q] : 0.0f, hi ? v[2 * q + 1] : 0.0f);
+      s_dz[0][r0 + 2 * q][c] = (uint16_t) h[q], s_dz[0][r0 + 2 * q + 1][c] = (uint16_t) (h[q] >> 16);
     }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) *(uint2*) (dz + top + 4 * g) = pack4(h + 4 * g);
+    *(uint4*) (dz + top) = make_uint4(h[0], h[1], h[2], h[3]);
   }
   __syncthreads();
   int cur = 0;
-  for (int layer = n_layers - 1; layer >= 1; --layer) {
-    floatx16 acc;
+  auto run_layer = [&](int layer, const bf16x8 (&b)[8][2], const uint2 (&keep)[2], bf16x8 (&ahead)[8][2], uint2 (&keep_ahead)[2]) {
+    floatx4 acc[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    bf16x8 b[16];
-    uint2 keep[4];
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 16; ++u) b[u] = ahead[u];
+      for (int r = 0; r < 4; ++r) acc[t][r] = 0.0f;
+    if (layer >= 2) fetch_mask(layer - 2, keep_ahead), fetch_weights(layer - 1, ahead);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) keep[g] = keep_ahead[g];
-    if (layer >= 2) {
-      mask_of(layer - 2, keep_ahead);
+    for (int u = 0; u < 8; ++u) {
+      const bf16x8 a = *(const bf16x8*) &s_dz[cur][arow][32 * u + kofs];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) ahead[u] = fragment(layer - 1, u);
+      for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[u][t], acc[t], 0, 0, 0);
     }
+    uint16_t* to = &s_dz[cur ^ 1][4 * (lane >> 4)][col];
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*) &s_dz[cur][arow][16 * u + kofs], b[u], acc, 0, 0, 0);
-    uint16_t* dst = dz + ((size_t) (layer - 1) * kMlpWidth + col) * B_pad + row0 + 4 * (lane >> 5);
+    for (int t = 0; t < 2; ++t) {
+      float v[4];  // rows past the batch: dZ is zero since the last layer
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      uint16_t h[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t word = k < 2 ? keep[g].x : keep[g].y;
-        const bool on = ((word >> (16 * (k & 1))) & 0xffffu) != 0u;  // rows past the batch: dZ is zero since the last layer
-        h[k] = on ? f32_to_bf16(acc[4 * g + k]) : (uint16_t) 0;
-        s_dz[cur ^ 1][acc_row(4 * g + k, lane)][col] = h[k];
-      }
-      *(uint2*) (dst + 8 * g) = pack4(h);
+      for (int k = 0; k < 4; ++k)
+        v[k] = (((k < 2 ? keep[t].x : keep[t].y) >> (16 * (k & 1))) & 0xffffu) != 0u ? acc[t][k] : 0.0f;
+      const uint2 h = make_uint2(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]));
+      uint16_t* row = to + 16 * t;
+      row[0] = (uint16_t) h.x, row[kStride] = (uint16_t) (h.x >> 16);
+      row[2 * kStride] = (uint16_t) h.y, row[3 * kStride] = (uint16_t) (h.y >> 16);
+      *(uint2*) (dz + ((size_t) (layer - 1) * kMlpWidth + col + 16 * t) * B_pad + row0 + 4 * (lane >> 4)) = h;
     }
     lds_barrier();
     cur ^= 1;
+  };
+  for (int layer = n_layers - 1; layer >= 1; layer -= 2) {
+    run_layer(layer, even, keep_even, odd, keep_odd);
+    if (layer >= 2) run_layer(layer - 1, odd, keep_odd, even, keep_even);
   }
 }
 
@@ -422,7 +477,7 @@ __global__ void __launch_bounds__(kMlpThreads) mlp_backward_weights_kernel(int B
   const int rows = layer < n_layers ? kMlpWidth : n_out, across = div_up_dev(K, kWgTile);
   const int o0 = (tile / across) * kWgTile, i0 = (tile % across) * kWgTile;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kofs = 8 * (lane >> 5);
-  const size_t B_pad = (size_t) ((B + kMlpRows - 1) / kMlpRows) * kMlpRows;
+  const size_t B_pad = (size_t) ((B + kMlpRowPad - 1) / kMlpRowPad) * kMlpRowPad;
   const int shift = layer == 0 ? Din : (layer == skip + 1 ? Din : 0);  // columns of X_l that are the input
   const uint16_t *arow[2], *brow[2];
 #pragma unroll
@@ -575,7 +630,7 @@ FSGS_API size_t fsgs_mlp_packed_elems(int Din, int n_layers, int skip) {
 }
 
 namespace {
-size_t padded_rows(int B) { return (size_t) div_up(std::max(B, 1), kMlpRows) * kMlpRows; }
+size_t padded_rows(int B) { return (size_t) div_up(std::max(B, 1), kMlpRowPad) * kMlpRowPad; }
 
 bool make_heads(MlpHeads& h, int n_heads, const int* head_rows, float* const* at) {
   if (n_heads < 1 || n_heads > kMaxHeads) return false;
@@ -609,8 +664,10 @@ FSGS_API int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, in
   if (B == 0) return kOk;
   const FreqInput freq{x, t, degree_x, degree_t, (float) scale_x, (float) scale_t};
   auto kernel = saved ? mlp_forward_kernel<true> : mlp_forward_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(div_up(B, kMlpRows)), dim3(kChainThreads), 0, (hipStream_t) stream, B, Din, n_layers,
-                     skip, n_out, in, freq, packed, bias, heads, saved_in, saved);
+  const int row_blocks = (int) (padded_rows(B) / kMlpRows);
+  hipLaunchKernelGGL(kernel, dim3(row_blocks + (row_blocks < kFetchBelow ? kFetchBlocks : 0)), dim3(kChainThreads), 0,
+                     (hipStream_t) stream, B, Din, n_layers, skip, n_out, in, freq, packed, bias, heads, saved_in, saved,
+                     row_blocks, fsgs_mlp_packed_elems(Din, n_layers, skip));
   return check_launch("mlp_forward");
 }
 
@@ -646,8 +703,10 @@ FSGS_API int fsgs_deform_mlp_backward(int B, int Din, int width, int n_layers, i
     hipLaunchKernelGGL(fill_zero_kernel, dim3(16), dim3(256), 0, s, (size_t) n_layers * kMlpWidth + n_out, g_b);
     return check_launch("mlp_backward");
   }
-  hipLaunchKernelGGL(mlp_backward_chain_kernel, dim3(div_up(B, kMlpRows)), dim3(kChainThreads), 0, s, B, Din, n_layers, n_out,
-                     in, heads_w, packed_t, saved, heads, dz, g_t, in_t);
+  const int row_blocks = (int) (padded_rows(B) / kMlpRows);
+  hipLaunchKernelGGL(mlp_backward_chain_kernel, dim3(row_blocks + (row_blocks < kFetchBelow ? kFetchBlocks : 0)),
+                     dim3(kChainThreads), 0, s, B, Din, n_layers, n_out, in, heads_w, packed_t, saved, heads, dz, g_t, in_t,
+                     row_blocks);
   int tiles = 0, K = Din;
   for (int l = 0; l <= n_layers; ++l) {
     tiles += div_up(l < n_layers ? kMlpWidth : n_out, kWgTile) * div_up(K, kWgTile);
