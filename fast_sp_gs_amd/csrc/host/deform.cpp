@@ -55,7 +55,7 @@ struct Nearest : public torch::autograd::Function<Nearest> {
   }
 };
 
-variable_list warp_forward(const SuperpointWarp& w, Tensor& d2) {
+variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   const char* what = "lbs_blend";
   Tensor index;
   nearest(w.points, w.sp_points, w.K, d2, index);
@@ -76,11 +76,11 @@ variable_list warp_forward(const SuperpointWarp& w, Tensor& d2) {
   Tensor d_xyz = empty({N, 3}, w.points), d_rot = empty({N, 4}, w.points), d_scale, weights = empty({N, K}, w.points);
   if (S) d_scale = empty({N, S}, w.points);
   const size_t bytes = fsgs_lbs_blend_workspace_bytes((int) M);
-  const Tensor ws = byte_buffer(bytes, w.points);
+  table = byte_buffer(bytes, w.points);
   check(fsgs_lbs_blend((int) N, (int) M, (int) K, w.warp_mode, w.weight_mode, w.temperature, f32(w.points), f32(w.sp_points),
                        f32(w.sp_t), f32(opt(w.sp_rot)), f32(w.sp_r), f32(opt(w.sp_s)), S, ld, f32(d2), i64(index),
                        f32(opt(w.sp_radius)), f32(opt(w.sp_weight)), f32(weights), f32(d_xyz), f32(d_rot), f32(d_scale),
-                       ws.data_ptr(), bytes, stream_of(w.points)),
+                       table.data_ptr(), bytes, stream_of(w.points)),
         what);
   variable_list out = {d_xyz, d_rot, weights, index};
   if (S) out.push_back(d_scale);
@@ -99,10 +99,10 @@ struct Warp : public torch::autograd::Function<Warp> {
                                const OptTensor& sp_weight, const SuperpointWarp* warp) {
     (void) sp_points, (void) sp_t, (void) sp_r, (void) sp_s, (void) sp_rot, (void) sp_radius, (void) sp_weight;
     const SuperpointWarp& w = *warp;
-    Tensor d2;
-    variable_list out = warp_forward(w, d2);
+    Tensor d2, table;
+    variable_list out = warp_forward(w, d2, table);
     ctx->save_for_backward({w.points, w.sp_points, w.sp_t, w.sp_r, opt(w.sp_s), opt(w.sp_rot), opt(w.sp_radius),
-                            opt(w.sp_weight), d2, out[3]});
+                            opt(w.sp_weight), d2, out[3], table});
     auto m = c10::make_intrusive<WarpModes>();
     m->warp_mode = w.warp_mode, m->weight_mode = w.weight_mode, m->temperature = w.temperature, m->S = w.scale_columns;
     ctx->saved_data["modes"] = c10::IValue::make_capsule(m);
@@ -113,7 +113,7 @@ struct Warp : public torch::autograd::Function<Warp> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto t = ctx->get_saved_variables();
     const Tensor &points = t[0], &sp_points = t[1], &sp_t = t[2], &sp_r = t[3], &sp_s = t[4], &sp_rot = t[5],
-                 &radius = t[6], &weight = t[7], &d2 = t[8], &index = t[9];
+                 &radius = t[6], &weight = t[7], &d2 = t[8], &index = t[9], &table = t[10];
     const auto capsule = ctx->saved_data["modes"].toCapsule();
     const WarpModes& m = *static_cast<const WarpModes*>(capsule.get());
     at::AutoDispatchBelowADInplaceOrView no_graph;
@@ -123,7 +123,7 @@ struct Warp : public torch::autograd::Function<Warp> {
       return x.defined() ? contiguous(x) : at::zeros({N, columns}, points.options());
     };
     const Tensor g_xyz = given(g[0], 3), g_rot = given(g[1], 4), g_scale = S ? given(g[4], S) : Tensor();
-    Tensor g_pair = empty({N, K}, points), g_c = empty({M, 3}, points), g_t = empty({M, 3}, points), g_r = empty({M, 4}, points);
+    Tensor g_c = empty({M, 3}, points), g_t = empty({M, 3}, points), g_r = empty({M, 4}, points);
     Tensor g_sp_rot, g_s, g_radius, g_weight;
     if (m.warp_mode) g_sp_rot = empty({M, 4}, points);
     if (S) g_s = empty({M, sp_s.size(1)}, points);
@@ -131,6 +131,17 @@ struct Warp : public torch::autograd::Function<Warp> {
     const size_t bytes = fsgs_lbs_blend_backward_workspace_bytes((int) N, (int) M, S);
     const Tensor ws = byte_buffer(bytes, points);
     const int ld = S ? (M > 1 ? (int) sp_s.stride(0) : (int) sp_s.size(1)) : 0;
+    auto pick = [&](size_t k, const Tensor& x) { return ctx->needs_input_grad(k) ? x : Tensor(); };
+    if (fsgs_superpoint_backward_is_fused((int) M, (int) K, m.warp_mode, m.weight_mode, S)) {
+      check(fsgs_superpoint_backward((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
+                                     f32(sp_points), f32(sp_t), f32(sp_rot), f32(sp_r), f32(sp_s), S, ld, f32(d2), i64(index),
+                                     f32(radius), f32(weight), table.data_ptr(), f32(g_xyz), f32(g_rot), f32(g_scale), f32(g_c),
+                                     f32(g_t), f32(g_sp_rot), f32(g_r), f32(g_s), S ? (int) sp_s.size(1) : 0, f32(g_radius),
+                                     f32(g_weight), ws.data_ptr(), bytes, stream_of(points)),
+            "superpoint_backward");
+      return {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()};
+    }
+    const Tensor g_pair = empty({N, K}, points);
     check(fsgs_lbs_blend_backward((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
                                   f32(sp_points), f32(sp_t), f32(sp_rot), f32(sp_r), f32(sp_s), S, ld, f32(d2), i64(index),
                                   f32(radius), f32(weight), f32(g_xyz), f32(g_rot), f32(g_scale), nullptr, f32(g_pair),
@@ -142,7 +153,6 @@ struct Warp : public torch::autograd::Function<Warp> {
       nearest_backward(points, sp_points, index, g_pair, false, none, g_y);
       g_c = m.warp_mode == 2 ? g_c.add_(g_y) : g_y;  // the pivot's gradient exists in that mode only
     }
-    auto pick = [&](size_t k, const Tensor& x) { return ctx->needs_input_grad(k) ? x : Tensor(); };
     return {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()};
   }
 };
@@ -343,9 +353,9 @@ variable_list superpoint_warp(const SuperpointWarp& given) {
   const bool train = at::GradMode::is_enabled() &&
                      (w.sp_points.requires_grad() || w.sp_t.requires_grad() || w.sp_r.requires_grad() || wants(w.sp_s) ||
                       wants(w.sp_rot) || wants(w.sp_radius) || wants(w.sp_weight));
-  Tensor d2;
+  Tensor d2, table;
   const variable_list r = train ? Warp::apply(w.sp_points, w.sp_t, w.sp_r, w.sp_s, w.sp_rot, w.sp_radius, w.sp_weight, &w)
-                                : warp_forward(w, d2);
+                                : warp_forward(w, d2, table);
   return {r[0], r[1], r.size() > 4 ? r[4] : Tensor(), r[2], r[3]};
 }
 

@@ -384,45 +384,53 @@ __global__ void __launch_bounds__(256) knn_topk_kernel(int N, int M, int D, int 
 
 // ---- LBS skinning (per-control-point table and weights: lbs.hpp) -----------------------------------------------------
 template <int kMaxK>
-__global__ void __launch_bounds__(256) lbs_blend_kernel(int N, int M, int K, int S, int sp_s_ld, int warp_mode, int weight_mode,
-    float temperature, const float* __restrict__ points, const float* __restrict__ xf, const float* __restrict__ sp_r,
-    const float* __restrict__ sp_s, const float* __restrict__ pair_in, const int64_t* __restrict__ index,
+__global__ void __launch_bounds__(256) lbs_blend_kernel(int N, int M, int K, int S, int warp_mode, int weight_mode,
+    float temperature, const float* __restrict__ points, const float* __restrict__ xf, const float* __restrict__ pair_in, const int64_t* __restrict__ index,
     float* __restrict__ weights_out, float* __restrict__ d_xyz, float* __restrict__ d_rot,
     float* __restrict__ d_scale) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= N) return;
-  const int64_t* id = index + (size_t) n * K;
-  float u[kMaxK], inv_den;
-  lbs_weights<kMaxK>(weight_mode, K, M, 1.0f / temperature, pair_in + (size_t) n * K, id, xf, u, inv_den);
+  const LbsPairs<kMaxK> pair(K, M, pair_in + (size_t) n * K, index + (size_t) n * K);
   const float p[3] = {points[3 * (size_t) n], points[3 * (size_t) n + 1], points[3 * (size_t) n + 2]};
+  float u[kMaxK], inv_den;
+  lbs_weights<kMaxK>(weight_mode, 1.0f / temperature, pair, xf, u, inv_den);
   float acc[3] = {0, 0, 0}, ar[4] = {0, 0, 0, 0}, as[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int k = 0; k < kMaxK; ++k) {
-    if (k >= K) break;
-    const int64_t j = id[k];
-    if (j < 0 || j >= M) {
-      if (weights_out) weights_out[(size_t) n * K + k] = 0.0f;
-      continue;
+  for (int k0 = 0; k0 < kMaxK; k0 += 4) {  // four neighbours' rows in flight
+    if (k0 >= K) break;
+    float4 row[4][5];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int c = 0; c < 5; ++c) row[q][c] = ((const float4*) (xf + (size_t) kXf * max(pair.j[k0 + q], 0)))[c];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = k0 + q;
+      if (k >= K) break;
+      const bool on = pair.j[k] >= 0;
+      const float w = on ? u[k] * inv_den : 0.0f;
+      if (on) {
+        const LbsTransform X(row[q]);
+        if (warp_mode != 0) {
+#pragma unroll
+          for (int a = 0; a < 3; ++a) acc[a] += w * (X.R(a * 3) * p[0] + X.R(a * 3 + 1) * p[1] + X.R(a * 3 + 2) * p[2] + X.t(a));
+        } else {
+#pragma unroll
+          for (int a = 0; a < 3; ++a) acc[a] += w * X.t(a);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) ar[a] += w * X.rot(a), as[a] += w * X.scale(a);
+      }
+      if (weights_out) weights_out[(size_t) n * K + k] = w;
     }
-    const float w  = u[k] * inv_den;
-    const float* X = xf + (size_t) kXf * j;
-    if (warp_mode != 0) {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) acc[a] += w * (X[a * 3] * p[0] + X[a * 3 + 1] * p[1] + X[a * 3 + 2] * p[2] + X[9 + a]);
-    } else {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) acc[a] += w * X[9 + a];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) ar[a] += w * sp_r[4 * j + a];
-    for (int a = 0; a < S; ++a) as[a] += w * sp_s[(size_t) sp_s_ld * j + a];
-    if (weights_out) weights_out[(size_t) n * K + k] = w;
   }
 #pragma unroll
   for (int a = 0; a < 3; ++a) d_xyz[3 * (size_t) n + a] = warp_mode != 0 ? acc[a] - p[a] : acc[a];
 #pragma unroll
   for (int a = 0; a < 4; ++a) d_rot[4 * (size_t) n + a] = ar[a];
-  for (int a = 0; a < S; ++a) d_scale[(size_t) S * n + a] = as[a];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+    if (a < S) d_scale[(size_t) S * n + a] = as[a];
 }
 
 // ---- masked Adam ------------------------------------------------------------------------------------------------------------
@@ -939,10 +947,10 @@ FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode,
   hipStream_t s = (hipStream_t) stream;
   float* xf     = (float*) workspace;
   hipLaunchKernelGGL(lbs_prepare_kernel, dim3(div_up(M, 256)), dim3(256), 0, s, M, warp_mode, sp_points, sp_t, sp_rot,
-                     weight_mode == 1 ? sp_log_radius : nullptr, weight_mode == 1 ? sp_weight_logit : nullptr, xf);
+                     sp_r, sp_s, S, sp_s_ld, weight_mode == 1 ? sp_log_radius : nullptr, weight_mode == 1 ? sp_weight_logit : nullptr, xf);
   auto kernel = K <= 4 ? lbs_blend_kernel<4> : lbs_blend_kernel<16>;
-  hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, s, N, M, K, S, sp_s_ld, warp_mode, weight_mode,
-                     (float) temperature, points, xf, sp_r, sp_s, pair_in, index, weights_out, d_xyz, d_rot, d_scale);
+  hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, s, N, M, K, S, warp_mode, weight_mode,
+                     (float) temperature, points, xf, pair_in, index, weights_out, d_xyz, d_rot, d_scale);
   return check_launch("lbs_blend");
 }
 

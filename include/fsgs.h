@@ -453,6 +453,18 @@ int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int weight_mode,
     float* g_pair, float* g_sp_points, float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s, int g_sp_s_ld,
     float* g_log_radius, float* g_weight_logit, void* workspace, size_t workspace_bytes, void* stream);
 
+/* fsgs_lbs_blend_backward and fsgs_knn_topk_backward of the control points in one: g_sp_points is the whole gradient of
+ * sp_points, through the weights' distances and (warp mode 2) the pivots; weight modes 0 and 1, whose pair input is the
+ * squared distance. blend_workspace: what fsgs_lbs_blend left in its workspace; workspace as for fsgs_lbs_blend_backward.
+ * For the sizes for which _is_fused returns 1 (M <= 1024, K <= 4, M * (columns + 3) <= 11264); others take the two calls. */
+int fsgs_superpoint_backward_is_fused(int M, int K, int warp_mode, int weight_mode, int S);
+int fsgs_superpoint_backward(int N, int M, int K, int warp_mode, int weight_mode, double temperature, const float* points,
+    const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r, const float* sp_s, int S, int sp_s_ld,
+    const float* dist2, const int64_t* index, const float* sp_log_radius, const float* sp_weight_logit,
+    const void* blend_workspace, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_sp_points,
+    float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s, int g_sp_s_ld, float* g_log_radius, float* g_weight_logit,
+    void* workspace, size_t workspace_bytes, void* stream);
+
 /* Backward of fsgs_knn_topk's squared distances (what autograd through pytorch3d.ops.knn_points gives at
  * fast_2d_gs/network.py:504): g_x[N,D] (optional) = sum_k 2 g_dist2[n,k] (x_n - y_index), g_y[M,D] = minus the same
  * summed over the queries that selected the row. Slots with index -1 are skipped. Both outputs fully written. */
