@@ -134,7 +134,10 @@ static_assert(kCoopThreshold == kCullMaskTiles, "a lane's serial walk covers exa
 // Empty tiles get (0, 0) as the reference's zero-initialised ranges have. Tile grids above kMaxLdsTiles tiles (no room
 // for one LDS counter per tile) count and scatter with 64-bit global atomics on ranges[t].y instead (tile_emit_kernel).
 
-constexpr int kMaxLdsTiles = 16384;  // one counter per tile in LDS
+// One counter per tile in LDS: 64 KB, two blocks on a compute unit, for grids up to kNarrowTiles; all of a compute unit's
+// 160 KB for those up to kMaxLdsTiles (a 4K picture has 32 400 tiles). With device-scope atomics in their place a 4K view of
+// 400k surfels spent 292 us counting and 482 us scattering, against 33 and 157 (and 34 against 7 in the scan by one block).
+constexpr int kNarrowTiles = 16384, kMaxLdsTiles = 40960;
 
 // Which tiles of a surfel's rectangle are visited: all of them (the reference's lists), those that pass the fast path's
 // corner test (CornerTest, from the surfel's adjugate and opacity), or those whose bit is set in the surfel's keep mask
@@ -279,8 +282,10 @@ __global__ void __launch_bounds__(256) cull_mask_kernel(int P, int gx, int gy, c
 
 // Layout of the `bins` buffer of the bucket binning: the queue length of the long segments in front of the B x T matrix
 // of per-(walk block, tile) instance counts.
-constexpr size_t kBinsHeader = 256;
 constexpr int kPrefixTiles = 64, kPrefixWaves = 16, kPrefixChunk = 32;  // walk blocks <= kPrefixWaves * kPrefixChunk
+constexpr size_t kBinsSums = 256;  // behind the queue length: the instances of every 64 tiles
+constexpr size_t kBinsHeader = 4096;
+static_assert(kBinsSums + (kMaxLdsTiles / kPrefixTiles) * sizeof(uint32_t) <= kBinsHeader, "the sums fit the header");
 struct BinsLayout {
   int blocks;      // walk blocks B (0: the tile grid is too large for LDS counters, the global-atomic path is used)
   int per_block;   // surfels per walk block
@@ -289,9 +294,10 @@ struct BinsLayout {
 inline BinsLayout bins_layout(int P, int T) {
   BinsLayout l{0, 0, kBinsHeader};
   if (T > kMaxLdsTiles || P <= 0) return l;
-  // one 1024-lane block per 1024 surfels while that keeps every block resident at once (two fit on a compute unit),
-  // beyond that the blocks grow
-  l.per_block = 1024 * std::max(1, div_up(P, 1024 * kPrefixWaves * kPrefixChunk));
+  // one 1024-lane block per 1024 surfels while that keeps every block resident at once (two fit on a compute unit, one
+  // with a large grid's counters), beyond that the blocks grow
+  const int most = T > kNarrowTiles ? kPrefixWaves * kPrefixChunk / 2 : kPrefixWaves * kPrefixChunk;
+  l.per_block = 1024 * std::max(1, div_up(P, 1024 * most));
   l.blocks    = div_up(P, l.per_block);
   l.bytes     = kBinsHeader + align_up((size_t) l.blocks * T * sizeof(uint32_t), 256);
   return l;
@@ -301,11 +307,11 @@ inline BinsLayout bins_layout(int P, int T) {
 // stores (zeros included, so the matrix needs no clearing). No global atomics: device-scope atomics on one address are
 // served one after the other at fabric latency, and with surfels in no spatial order every block touches nearly
 // every tile.
-template <int kMode>
+template <int kMode, int kTiles>
 __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, int gx, int gy,
     const float2* __restrict__ means2D, const int32_t* __restrict__ radii, WalkInputs in,
     uint32_t* __restrict__ hist, SlotPublish publish) {
-  __shared__ unsigned s_count[kMaxLdsTiles];
+  __shared__ unsigned s_count[kTiles];
   // first of all, so that the instance count reaches the host while the rest of the counting is still running
   if (publish.counters && blockIdx.x == 0 && threadIdx.x < kWave) publish_slot_regions(publish);
   const int T = gx * gy;
@@ -325,22 +331,28 @@ __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, i
 }
 
 // Step 2: per tile, the exclusive prefix of its column over the walk blocks (in place) and the column total, which goes
-// to ranges[t].y for tile_scan_kernel. 64 tiles per block, lane = tile, the 16 wavefronts share the walk blocks in
+// to ranges[t].y for tile_scan_kernel, and the sum over the block's tiles to sums[blockIdx.x]. 64 tiles per block, lane = tile, the 16 wavefronts share the walk blocks in
 // contiguous chunks so that a wavefront's loads are all in flight at once.
 __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kernel(int T, int B,
-    uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges) {
+    uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges, uint32_t* __restrict__ sums) {
   __shared__ uint32_t s_sum[kPrefixWaves][kPrefixTiles];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = blockIdx.x * kPrefixTiles + lane;
   const int chunk = (B + kPrefixWaves - 1) / kPrefixWaves, b0 = wave * chunk;
   // a wavefront's whole chunk of the column is loaded before anything is written back (B <= 512: at most 32 values per
-  // lane), so the loads are in flight together; a load placed behind a store to the same array would wait for it
+  // lane), eight loads in flight at least: at clamped addresses, for a load under a condition is waited for on the spot
   uint32_t c[kPrefixChunk], sum = 0;
 #pragma unroll
-  for (int i = 0; i < kPrefixChunk; ++i) {
-    const int b = b0 + i;
-    c[i] = (t < T && i < chunk && b < B) ? hist[(size_t) b * T + t] : 0u;
-    sum += c[i];
+  for (int i0 = 0; i0 < kPrefixChunk; i0 += 8) {
+    if (i0 < chunk) {  // uniform
+#pragma unroll
+      for (int i = i0; i < i0 + 8; ++i) c[i] = hist[(size_t) min(b0 + i, B - 1) * T + min(t, T - 1)];
+    }
+#pragma unroll
+    for (int i = i0; i < i0 + 8; ++i) {
+      c[i] = t < T && i < chunk && b0 + i < B ? c[i] : 0u;
+      sum += c[i];
+    }
   }
   s_sum[wave][lane] = sum;
   __syncthreads();
@@ -360,16 +372,22 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
     }
     if (wave == 0) ranges[2 * (size_t) t + 1] = total;
   }
+  if (wave == 0) {
+    uint32_t all = t < T ? total : 0u;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) all += __shfl_xor(all, d, kWave);
+    if (lane == 0) sums[blockIdx.x] = all;
+  }
 }
 
 // Step 3: the walk of step 1 again; a block's cursor of a tile starts at the tile's start plus the instances of the
 // blocks in front of it, so the placement needs no global atomics either.
-template <int kMode>
+template <int kMode, int kTiles>
 __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block, int gx, int gy, int64_t R,
     const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
     WalkInputs in, const uint32_t* __restrict__ hist, const unsigned long long* __restrict__ ranges,
     uint64_t* __restrict__ entries, int* __restrict__ order_table) {
-  __shared__ unsigned s_cursor[kMaxLdsTiles];
+  __shared__ unsigned s_cursor[kTiles];
   // One block more than the walk needs, when the frame's blockIdx -> tile schedule is still to be built: the ranges are
   // final, nothing in this kernel reads the table, and the per-tile sorts and the blend kernels that follow do.
   if (order_table && blockIdx.x == gridDim.x - 1) {
@@ -392,14 +410,28 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
   }
 }
 
-// One block: exclusive scan of the per-tile counts, 4 tiles per lane and step.
+// Exclusive scan of the per-tile counts, 4 tiles per lane and step.
+// With `sums` (the instances of every 64 tiles) block b scans the tiles from 4096 b on and adds what lies in front of them
+// itself; without, one block walks all tiles.
 // ends = false: ranges[t] = (start, start), for a scatter that advances ranges[t].y; ends = true: (start, end).
 __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long long* __restrict__ ranges,
-                                                         int* __restrict__ large_count, bool ends) {
+                                                         const uint32_t* __restrict__ sums, int* __restrict__ large_count,
+                                                         bool ends) {
   __shared__ unsigned long long s_wave[16];
   const int lane = __lane_id(), wave = threadIdx.x / kWave;
   unsigned long long carry = 0;
-  for (int start = 0; start < T; start += 4096) {
+  const int first = sums ? blockIdx.x * 4096 : 0, last = sums ? min(T, first + 4096) : T;
+  if (first > 0) {
+    unsigned long long before = 0;
+    for (int b = threadIdx.x; b < first / kPrefixTiles; b += blockDim.x) before += sums[b];
+    const unsigned long long inc = wave_inclusive_scan(before);
+    if (lane == kWave - 1) s_wave[wave] = inc;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) carry += s_wave[w];
+    __syncthreads();
+  }
+  for (int start = first; start < last; start += 4096) {
     const int t0 = start + threadIdx.x * 4;
     unsigned long long c[4], sum = 0;
 #pragma unroll
@@ -423,7 +455,7 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
     }
     carry += total;
   }
-  if (threadIdx.x == 0) large_count[0] = 0, large_count[1] = (int) carry;  // queue length | instances in all tiles
+  if (threadIdx.x == 0 && last == T) large_count[0] = 0, large_count[1] = (int) carry;  // queue length | instances in all tiles
 }
 
 // Where element i of a segment sits in LDS. With kPad one slot in five stays empty: the rounds of the sorting network
@@ -865,13 +897,13 @@ size_t fast_bucket_bins_bytes(int P, int W, int H) {
 }
 
 namespace {
-#define FSGS_BY_WALK_MODE(IN, CALL)                                     \
+#define FSGS_BY_WALK_MODE(IN, ...)                                     \
   do {                                                                  \
     switch ((IN).mode()) {                                              \
-      case kWalkAll: { constexpr int kMode = kWalkAll; CALL; break; }   \
-      case kWalkCorner: { constexpr int kMode = kWalkCorner; CALL; break; } \
-      case kWalkMask: { constexpr int kMode = kWalkMask; CALL; break; } \
-      case kWalkCornerMask: { constexpr int kMode = kWalkCornerMask; CALL; break; } \
+      case kWalkAll: { constexpr int kMode = kWalkAll; __VA_ARGS__; break; }   \
+      case kWalkCorner: { constexpr int kMode = kWalkCorner; __VA_ARGS__; break; } \
+      case kWalkMask: { constexpr int kMode = kWalkMask; __VA_ARGS__; break; } \
+      case kWalkCornerMask: { constexpr int kMode = kWalkCornerMask; __VA_ARGS__; break; } \
     }                                                                   \
   } while (0)
 
@@ -886,11 +918,15 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
   const BinsLayout bl = bins_layout(P, T);
   if (bl.blocks > 0) {
     uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
-    FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_hist_kernel<kMode>), dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block,
-                                             gx, gy, (const float2*) means2D, radii, in, hist, publish));
+    uint32_t* sums = (uint32_t*) ((char*) bins + kBinsSums);
+    FSGS_BY_WALK_MODE(in, {
+      auto kernel = T > kNarrowTiles ? tile_hist_kernel<kMode, kMaxLdsTiles> : tile_hist_kernel<kMode, kNarrowTiles>;
+      hipLaunchKernelGGL(kernel, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy, (const float2*) means2D, radii, in,
+                         hist, publish);
+    });
     hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
-                       bl.blocks, hist, rng);
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, true);
+                       bl.blocks, hist, rng, sums);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
     // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
     // sorts) is built from them by an extra block of the scatter, in the second part.
   } else {
@@ -901,7 +937,7 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
       FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, false>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx,
                                                gy, (int64_t) 0, (const float2*) means2D, (const float*) nullptr, radii, in,
                                                rng, (uint64_t*) nullptr));
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, header, false);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, (const uint32_t*) nullptr, header, false);
   }
   return check_launch("gs_prepare_count");
 }
@@ -925,9 +961,12 @@ int fill_sort(int P, int W, int H, const float* means2D, const float* depths, co
   if (bl.blocks > 0) {
     int* build = nullptr;
     (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
-    FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_scatter_kernel<kMode>), dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), 0, s,
-                                             P, bl.per_block, gx, gy, R, (const float2*) means2D, depths, radii, in,
-                                             (const uint32_t*) ((const char*) bins + kBinsHeader), rng, entries, build));
+    FSGS_BY_WALK_MODE(in, {
+      auto kernel = T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles> : tile_scatter_kernel<kMode, kNarrowTiles>;
+      hipLaunchKernelGGL(kernel, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), 0, s, P, bl.per_block, gx, gy, R,
+                         (const float2*) means2D, depths, radii, in, (const uint32_t*) ((const char*) bins + kBinsHeader), rng,
+                         entries, build);
+    });
   } else {
     FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, true>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy,
                                              R, (const float2*) means2D, depths, radii, in, rng, entries));
