@@ -97,10 +97,10 @@ __device__ __forceinline__ void fast_transmat_backward(float sx, float sy, const
   gq[3] = 2 * (x * (dR[7] - dR[5]) + y * (dR[2] - dR[6]) + z * (dR[3] - dR[1]));
 }
 
-// kWave: complete degree-3 rows in one 16-byte aligned [P,16,3] tensor, moved by each wavefront on its own (sh_stage.hpp).
+// kRow: floats of a row that each wavefront moves on its own (sh_stage.hpp), 45 with the first coefficient apart; 0: none
 constexpr int kCoopThreshold = 32;  // rectangles with more tiles are walked (and corner-tested) by a whole wavefront
 
-template <int kSh, bool kWave>
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ opacities, const float* __restrict__ shs,
@@ -110,7 +110,9 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     float* __restrict__ inverse_m, float4* __restrict__ normal_opacity, float* __restrict__ depths,
     int32_t* __restrict__ radii, int32_t* __restrict__ tiles_touched, uint32_t* __restrict__ keep_masks,
     ViewOutputs view) {
-  __shared__ float s_rows[kWave ? kShStageRows * kShStageStride : 1];
+  constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
+  constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
+  __shared__ __align__(16) float s_rows[kWave ? kShStageRows * kStride : 1];
   const int i0     = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i0 < P;
   __shared__ int s_wave_slots[4];
@@ -130,15 +132,17 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
   for (int k = 0; k < 9; ++k) M[k] = 0.0f;
   const float p[3] = {means3D[3 * (size_t) i], means3D[3 * (size_t) i + 1], means3D[3 * (size_t) i + 2]};
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kShStageStride : 0];
-  ShWaveRows sh_regs;
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
+  float dc[3] = {0, 0, 0};
   if (kWave) {
     // the two cheapest rejections decide which rows are fetched; the fetch is then in flight during the geometry
     bool maybe = valid && !(culling && culling[i]);
     maybe = maybe && !((Tw2v[8] * p[0] + Tw2v[9] * p[1] + Tw2v[10] * p[2] + Tw2v[11]) <= 0.2f);
     wanted = __ballot(maybe);
-    if (wanted) wave_fetch_sh_rows(sh_regs, wanted, wave_base, (const float4*) shs);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   }
   do {
     if (!valid || (culling && culling[i])) break;
@@ -177,7 +181,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     if (threadIdx.x == 0) block_slot = atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
   }
   if (kWave) {
-    if (wanted) wave_rows_to_lds(sh_regs, s_wave_rows);
+    if (wanted) sh_regs.to_lds(s_wave_rows, wave_base, P);
     wave_lds_sync();
   }
   if (ok && sh_degree >= 0) {
@@ -185,9 +189,10 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     view_dir(p, campos, x, y, z);
     sh_eval(sh_degree, x, y, z, Y);
     const int n = sh_count(sh_degree);
-    const float* c0 = kWave ? &s_rows[threadIdx.x * kShStageStride] : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
-    float r = c0[0] * Y[0], g = c0[1] * Y[0], b = c0[2] * Y[0];
-    const float* cr = kWave ? c0 : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
+    const float* row = &s_rows[kWave ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
+    const float* c0 = kWave ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
+    float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
+    const float* cr = kWave ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
     for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
     rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
   }
@@ -327,7 +332,7 @@ __global__ void __launch_bounds__(256) fast_duplicate_keys_kernel(int P, int gx,
   }
 }
 
-template <int kSh, bool kWave>
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -337,13 +342,15 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     const float* __restrict__ grad_colors, const float4* __restrict__ grad_normal_opacity,
     float* __restrict__ g_means3D, float2* __restrict__ g_scales, float4* __restrict__ g_rot,
     float* __restrict__ g_opac, float* __restrict__ g_shs, float* __restrict__ g_sh_rest) {
-  __shared__ float s_rows[kWave ? kShStageRows * kShStageStride : 1];
+  constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
+  constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
+  __shared__ __align__(16) float s_rows[kWave ? kShStageRows * kStride : 1];
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
   const bool vis   = valid && radii[i] > 0;
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kShStageStride : 0];
-  float* my_row       = &s_rows[kWave ? threadIdx.x * kShStageStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  float* my_row       = &s_rows[kWave ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
   // Rows of surfels that were not rendered get explicit zeros, so the outputs need no initialisation (the reference
   // leaves them to the caller's zero fill; a caller that zero-fills gets the same result).
   auto zero_geometry = [&]() {
@@ -356,24 +363,22 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     const unsigned long long wanted = __ballot(vis);
     if (wanted == 0ull) {  // nothing of this wavefront was rendered: its gradient rows are zeros
       if (wave_base < P) {
-#pragma unroll
-        for (int k = 0; k < kShWavePieces; ++k) {
-          int r, c4;
-          wave_piece(k, r, c4);
-          if (wave_base + r < P)
-            ((float4*) g_shs)[(size_t) (wave_base + r) * kShWavePieces + c4] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
+        ShWaveRows<kWave ? kRow : 48>::zeros_to_global(wave_base, P, kSplit ? g_sh_rest : g_shs);
+        if (kSplit && valid && g_shs)
+          g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       }
       if (valid) zero_geometry();
       return;
     }
-    ShWaveRows sh_regs;
-    wave_fetch_sh_rows(sh_regs, wanted, wave_base, (const float4*) shs);
-    wave_rows_to_lds(sh_regs, s_wave_rows);
+    ShWaveRows<kWave ? kRow : 48> sh_regs;
+    sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    sh_regs.to_lds(s_wave_rows, wave_base, P);
     wave_lds_sync();
     if (!vis) {
 #pragma unroll
-      for (int c = 0; c < kShStageFloats; ++c) my_row[c] = 0.0f;
+      for (int c = kSplit ? 3 : 0; c < kShStageFloats; ++c) my_row[c] = 0.0f;
+      if (kSplit && valid && g_shs)
+        g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       if (valid) zero_geometry();
     }
   } else if (!vis) {
@@ -444,7 +449,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     // with kWave the coefficients are read from the lane's staged row and the gradient row is written over them
     const float* c0 = kWave ? my_row : shs + (size_t) i * m1 * 3;
     const float* cr = kWave ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-    float* o0  = kWave ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
+    float* o0  = kWave && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
     float* orr = kWave ? my_row
                        : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
     if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
@@ -474,7 +479,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
   }
   if (kWave) {
     wave_lds_sync();
-    wave_rows_to_global(s_wave_rows, wave_base, P, (float4*) g_shs);
+    ShWaveRows<kWave ? kRow : 48>::to_global(s_wave_rows, wave_base, P, kSplit ? g_sh_rest : g_shs);
   }
 }
 
@@ -540,10 +545,11 @@ int fast_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const 
                    (colors || sh_degree < 0),
                "gs_2d_fast_preprocess_forward: null pointer");
   if (P == 0) return kOk;
-  const bool wave_rows = sh_degree == 3 && n_sh == 16 && !sh_rest && (uintptr_t) shs % 16 == 0;
-  auto kernel = sh_degree > 3 ? fast_preprocess_forward_kernel<64, false>
-                              : (wave_rows ? fast_preprocess_forward_kernel<16, true>
-                                           : fast_preprocess_forward_kernel<16, false>);
+  const int rows = wave_row_floats(sh_degree, n_sh, shs, sh_rest);
+  auto kernel = sh_degree > 3 ? fast_preprocess_forward_kernel<64, 0>
+                : rows == 48  ? fast_preprocess_forward_kernel<16, 48>
+                : rows == 45  ? fast_preprocess_forward_kernel<16, 45>
+                              : fast_preprocess_forward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh,
                      means3D, (const float2*) scales, (const float4*) rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
                      campos, trans_precomp, culling, means2D_preserve, (float2*) means2D, colors, trans_mat, inverse_m,
@@ -639,11 +645,12 @@ FSGS_API int fsgs_gs_2d_fast_preprocess_backward(int P, int W, int H, int sh_deg
   if (sh_degree >= 0)
     FSGS_REQUIRE(shs && colors && grad_colors, "gs_2d_fast_preprocess_backward: SH path needs shs, colors, grad_colors");
   if (P == 0) return kOk;
-  const bool wave_rows = sh_degree == 3 && n_sh == 16 && !sh_rest && g_shs && (uintptr_t) shs % 16 == 0 &&
-                         (uintptr_t) g_shs % 16 == 0;
-  auto kernel = sh_degree > 3 ? fast_preprocess_backward_kernel<64, false>
-                              : (wave_rows ? fast_preprocess_backward_kernel<16, true>
-                                           : fast_preprocess_backward_kernel<16, false>);
+  float* g_rows  = sh_rest ? g_sh_rest : g_shs;
+  const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
+  auto kernel = sh_degree > 3 ? fast_preprocess_backward_kernel<64, 0>
+                : rows == 48  ? fast_preprocess_backward_kernel<16, 48>
+                : rows == 45  ? fast_preprocess_backward_kernel<16, 45>
+                              : fast_preprocess_backward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh,
                      means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v, Tv2s, campos,
                      trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_inv_m, grad_colors,

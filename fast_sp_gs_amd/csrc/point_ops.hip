@@ -25,23 +25,27 @@ namespace fsgs {
 namespace {
 
 // ---- SH -> RGB ----------------------------------------------------------------------------------------------------
-// kRows: all 16 coefficients of a point sit in one 16-byte-aligned 192-byte row (F == 16, degree 3). A lane that walks its
-// own row touches one 128-byte line per load instruction (920 GB/s measured at 1M points); each wavefront therefore moves
-// its 64 rows as twelve 16-byte pieces per lane, 1 KB of consecutive addresses per instruction, through its own slice of
-// LDS, and every lane then reads its row there (the scheme of the preprocess kernels, sh_stage.hpp).
-template <int kSh, bool kRows>
+// kRow: a point has exactly the coefficients of its degree, in rows of kRow floats (12, 27, 48) behind a 16-byte boundary.
+// A lane that walks its own row touches one 128-byte line per load instruction (920 GB/s measured at 1M points); each
+// wavefront therefore moves its 64 rows as 16-byte pieces, 1 KB of consecutive addresses per instruction, through its own
+// slice of LDS, and every lane then reads its row there (the scheme of the preprocess kernels, sh_stage.hpp). 0: other rows.
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) sh_to_rgb_forward_kernel(int P, int F, int degree, int clamp,
     const float* __restrict__ pos, const float* __restrict__ campos, const float* __restrict__ sh,
     float* __restrict__ rgb) {
-  __shared__ float s_rows[kRows ? 4 * kWave * kShStageStride : 1];
+  constexpr bool kRows  = kRow != 0;
+  using Rows            = ShWaveRows<kRows ? kRow : 48>;
+  constexpr int kStride = Rows::kStride;
+  __shared__ __align__(16) float s_rows[kRows ? 4 * kWave * kStride : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kShStageStride : 0);
+  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kStride : 0);
   if (kRows) {
     const unsigned long long live = __ballot(i < P);
     if (live != 0ull) {
-      ShWaveRows regs;
-      wave_fetch_sh_rows(regs, live, (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63)), (const float4*) sh);
-      wave_rows_to_lds(regs, my_rows);
+      const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
+      Rows regs;
+      regs.fetch(live, wave_base, P, sh);
+      regs.to_lds(my_rows, wave_base, P);
       wave_lds_sync();
     }
   }
@@ -54,7 +58,7 @@ __global__ void __launch_bounds__(256) sh_to_rgb_forward_kernel(int P, int F, in
   float Y[kSh];
   sh_eval(degree, x, y, z, Y);
   const int n    = sh_count(degree);
-  const float* c = kRows ? my_rows + (threadIdx.x & 63) * kShStageStride : sh + (size_t) i * F * 3;
+  const float* c = kRows ? my_rows + (threadIdx.x & 63) * kStride : sh + (size_t) i * F * 3;
   float r = c[0] * Y[0], g = c[1] * Y[0], b = c[2] * Y[0];
   for (int l = 1; l < n; ++l) r += c[3 * l] * Y[l], g += c[3 * l + 1] * Y[l], b += c[3 * l + 2] * Y[l];
   r += 0.5f, g += 0.5f, b += 0.5f;
@@ -68,22 +72,25 @@ __device__ __forceinline__ float wave_sum_xor(float v) {
   return v;
 }
 
-template <int kSh, bool kRows>
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, int degree, int clamp,
     const float* __restrict__ pos, const float* __restrict__ campos, const float* __restrict__ sh,
     const float* __restrict__ rgb, const float* __restrict__ grad_rgb, float* __restrict__ grad_dir,
     float* __restrict__ grad_campos, float* __restrict__ grad_sh) {
   __shared__ float s_cam[4][3];
-  __shared__ float s_rows[kRows ? 4 * kWave * kShStageStride : 1];
+  constexpr bool kRows  = kRow != 0;
+  using Rows            = ShWaveRows<kRows ? kRow : 48>;
+  constexpr int kStride = Rows::kStride;
+  __shared__ __align__(16) float s_rows[kRows ? 4 * kWave * kStride : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
-  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kShStageStride : 0);
+  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kStride : 0);
   if (kRows) {  // coefficient rows in through LDS; the gradient rows leave the same way (a lane overwrites its own row)
     const unsigned long long live = __ballot(i < P);
     if (live != 0ull) {
-      ShWaveRows regs;
-      wave_fetch_sh_rows(regs, live, wave_base, (const float4*) sh);
-      wave_rows_to_lds(regs, my_rows);
+      Rows regs;
+      regs.fetch(live, wave_base, P, sh);
+      regs.to_lds(my_rows, wave_base, P);
       wave_lds_sync();
     }
   }
@@ -101,7 +108,7 @@ __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, i
     float Y[kSh], tl[kSh];
     sh_eval(degree, x, y, z, Y);
     const int n    = sh_count(degree);
-    float* row     = my_rows + (threadIdx.x & 63) * kShStageStride;
+    float* row     = my_rows + (threadIdx.x & 63) * kStride;
     const float* c = kRows ? row : sh + (size_t) i * F * 3;
     float* o       = kRows ? (grad_sh ? row : nullptr) : (grad_sh ? grad_sh + (size_t) i * F * 3 : nullptr);
     tl[0] = 0.0f;
@@ -122,7 +129,7 @@ __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, i
   }
   if (kRows && grad_sh) {
     wave_lds_sync();
-    wave_rows_to_global(my_rows, wave_base, P, (float4*) grad_sh);
+    Rows::to_global(my_rows, wave_base, P, grad_sh);
   }
   if (grad_campos) {  // block reduction, then 3 atomics per block (spherical_harmonics.cu:56-65)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -145,13 +152,30 @@ template <typename T> struct Arith { using type = T; };
 template <> struct Arith<_Float16> { using type = float; };
 
 // ---- bare SH encoder ------------------------------------------------------------------------------------------------
-template <int kSh, typename T>
+// kRow: rows of 9 or 16 floats behind a 16-byte boundary go through LDS, so that a store (load) instruction covers 1 KB of
+// consecutive addresses; a lane that walks its own 64-byte row touches a line of its own with each. 1M directions, degree
+// 3: forward 24 -> 13 us, backward 30 -> 21 us. Rows of 4 floats are one 16-byte access per lane anyway. 0: other rows.
+template <int kSh, typename T, int kRow>
 __global__ void __launch_bounds__(256) sh_encode_forward_kernel(int B, int D, int C, const T* __restrict__ in,
                                                                 T* __restrict__ out) {
   using A = typename Arith<T>::type;
+  using Rows = ShWaveRows<kRow ? kRow : 16>;
+  __shared__ __align__(16) float s_rows[kRow ? 4 * kWave * Rows::kStride : 1];
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+  if (!kRow && b >= B) return;
   A Y[kSh];
+  if constexpr (kRow != 0) {
+    const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
+    float* my_rows      = s_rows + (threadIdx.x >> 6) * kWave * Rows::kStride;
+    if (b < B) {
+      sh_eval(C, in[(size_t) b * D], in[(size_t) b * D + 1], in[(size_t) b * D + 2], Y);
+#pragma unroll
+      for (int l = 0; l < kRow; ++l) my_rows[(threadIdx.x & 63) * Rows::kStride + l] = Y[l];
+    }
+    wave_lds_sync();
+    Rows::to_global(my_rows, wave_base, B, out);
+    return;
+  }
   if constexpr (std::is_same<T, _Float16>::value && kSh == 16)
     sh_eval_half(C, (A) in[(size_t) b * D], (A) in[(size_t) b * D + 1], (A) in[(size_t) b * D + 2], Y);
   else
@@ -167,17 +191,32 @@ __global__ void __launch_bounds__(256) sh_encode_forward_kernel(int B, int D, in
   for (int l = 0; l < n; ++l) o[l] = (T) Y[l];
 }
 
-template <int kSh, typename T>
+template <int kSh, typename T, int kRow>
 __global__ void __launch_bounds__(256) sh_encode_backward_kernel(int B, int D, int C, const T* __restrict__ grad,
     const T* __restrict__ in, T* __restrict__ grad_in) {
   using A = typename Arith<T>::type;
+  using Rows = ShWaveRows<kRow ? kRow : 16>;
+  __shared__ __align__(16) float s_rows[kRow ? 4 * kWave * Rows::kStride : 1];
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
   const int n = sh_count(C);
   A t[kSh];
   const T* g = grad + (size_t) b * n;
   bool loaded = false;
-  if constexpr (std::is_same<T, float>::value) {
+  if constexpr (kRow != 0) {
+    const unsigned long long live = __ballot(b < B);
+    if (live == 0ull) return;
+    const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
+    float* my_rows      = s_rows + (threadIdx.x >> 6) * kWave * Rows::kStride;
+    Rows regs;
+    regs.fetch(live, wave_base, B, grad);
+    regs.to_lds(my_rows, wave_base, B);
+    wave_lds_sync();
+#pragma unroll
+    for (int l = 0; l < kRow; ++l) t[l] = my_rows[(threadIdx.x & 63) * Rows::kStride + l];
+    loaded = true;
+  }
+  if (b >= B) return;
+  if constexpr (std::is_same<T, float>::value && kRow == 0) {
     if ((n & 3) == 0) {
       for (int l = 0; l < n; l += 4) {
         const float4 v = *(const float4*) (g + l);
@@ -731,9 +770,12 @@ FSGS_API int fsgs_sh_to_rgb_forward(int P, int F, int degree, int clamp, const f
   FSGS_REQUIRE(0 <= degree && degree <= kMaxShDegree && (degree + 1) * (degree + 1) <= F,
                "SH_to_RGB_forward: degree %d unsupported or > features %d", degree, F);
   if (P == 0) return kOk;
-  const bool rows = degree == 3 && F == 16 && ((uintptr_t) sh & 15) == 0;
-  auto kernel = degree > 3 ? sh_to_rgb_forward_kernel<64, false>
-                           : (rows ? sh_to_rgb_forward_kernel<16, true> : sh_to_rgb_forward_kernel<16, false>);
+  const int rows = F == (degree + 1) * (degree + 1) && ((uintptr_t) sh & 15) == 0 ? degree : 0;
+  auto kernel = degree > 3  ? sh_to_rgb_forward_kernel<64, 0>
+                : rows == 3 ? sh_to_rgb_forward_kernel<16, 48>
+                : rows == 2 ? sh_to_rgb_forward_kernel<16, 27>
+                : rows == 1 ? sh_to_rgb_forward_kernel<16, 12>
+                            : sh_to_rgb_forward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, F, degree,
                      clamp, pos, campos, sh, rgb);
   return check_launch("SH_to_RGB_forward");
@@ -747,9 +789,12 @@ FSGS_API int fsgs_sh_to_rgb_backward(int P, int F, int degree, int clamp, const 
                "SH_to_RGB_backward: degree %d unsupported or > features %d", degree, F);
   FSGS_REQUIRE(!grad_campos || campos, "SH_to_RGB_backward: grad_campos without campos");
   if (P == 0) return kOk;
-  const bool rows = degree == 3 && F == 16 && (((uintptr_t) sh | (uintptr_t) grad_sh) & 15) == 0;
-  auto kernel = degree > 3 ? sh_to_rgb_backward_kernel<64, false>
-                           : (rows ? sh_to_rgb_backward_kernel<16, true> : sh_to_rgb_backward_kernel<16, false>);
+  const int rows = F == (degree + 1) * (degree + 1) && (((uintptr_t) sh | (uintptr_t) grad_sh) & 15) == 0 ? degree : 0;
+  auto kernel = degree > 3  ? sh_to_rgb_backward_kernel<64, 0>
+                : rows == 3 ? sh_to_rgb_backward_kernel<16, 48>
+                : rows == 2 ? sh_to_rgb_backward_kernel<16, 27>
+                : rows == 1 ? sh_to_rgb_backward_kernel<16, 12>
+                            : sh_to_rgb_backward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, F, degree,
                      clamp, pos, campos, sh, rgb, grad_rgb, grad_dir, grad_campos, grad_sh);
   return check_launch("SH_to_RGB_backward");
@@ -759,13 +804,21 @@ FSGS_API int fsgs_sh_to_rgb_backward(int P, int F, int degree, int clamp, const 
 namespace {
 template <typename T>
 int sh_encode_forward_t(int B, int D, int C, const void* in, void* out, hipStream_t s) {
-  auto kernel = C > 3 ? sh_encode_forward_kernel<64, T> : sh_encode_forward_kernel<16, T>;
+  auto kernel = C > 3 ? sh_encode_forward_kernel<64, T, 0> : sh_encode_forward_kernel<16, T, 0>;
+  if constexpr (std::is_same<T, float>::value) {
+    if (((uintptr_t) out & 15) == 0 && (C == 2 || C == 3))
+      kernel = C == 3 ? sh_encode_forward_kernel<16, float, 16> : sh_encode_forward_kernel<16, float, 9>;
+  }
   hipLaunchKernelGGL(kernel, dim3(div_up(B, 256)), dim3(256), 0, s, B, D, C, (const T*) in, (T*) out);
   return check_launch("sh_encode_forward");
 }
 template <typename T>
 int sh_encode_backward_t(int B, int D, int C, const void* grad, const void* in, void* grad_in, hipStream_t s) {
-  auto kernel = C > 3 ? sh_encode_backward_kernel<64, T> : sh_encode_backward_kernel<16, T>;
+  auto kernel = C > 3 ? sh_encode_backward_kernel<64, T, 0> : sh_encode_backward_kernel<16, T, 0>;
+  if constexpr (std::is_same<T, float>::value) {
+    if (((uintptr_t) grad & 15) == 0 && (C == 2 || C == 3))
+      kernel = C == 3 ? sh_encode_backward_kernel<16, float, 16> : sh_encode_backward_kernel<16, float, 9>;
+  }
   hipLaunchKernelGGL(kernel, dim3(div_up(B, 256)), dim3(256), 0, s, B, D, C, (const T*) grad, (const T*) in,
                      (T*) grad_in);
   return check_launch("sh_encode_backward");

@@ -82,8 +82,8 @@ __device__ __forceinline__ void transmat(int W, int H, const float* p, float sx,
   nrm[2] = Tw2v[8] * t0 + Tw2v[9] * t1 + Tw2v[10] * t2;
 }
 
-// kWave: complete degree-3 rows in one 16-byte aligned [P,16,3] tensor, moved by each wavefront on its own.
-template <int kSh, bool kWave>
+// kRow: floats of a row that each wavefront moves on its own (sh_stage.hpp), 45 with the first coefficient apart; 0: none
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ opacities, const float* __restrict__ shs,
@@ -93,9 +93,11 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     float4* __restrict__ normal_opacity, float* __restrict__ depths, int32_t* __restrict__ radii,
     int32_t* __restrict__ tiles_touched, float4* __restrict__ records, uint32_t* __restrict__ keep_masks,
     ViewOutputs view) {
+  constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
+  constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;  // degree <= 3: SH rows travel through LDS, read from HBM line by line
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ float s_rows[kStage ? kShStageRows * kShStageStride : 1];
+  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   __shared__ int s_wave_slots[4];
   __shared__ int s_block_slot;
@@ -112,15 +114,17 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   float p[3] = {0, 0, 0};
   if (valid) p[0] = means3D[3 * (size_t) i], p[1] = means3D[3 * (size_t) i + 1], p[2] = means3D[3 * (size_t) i + 2];
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kShStageStride : 0];
-  ShWaveRows sh_regs;
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
+  float dc[3] = {0, 0, 0};
   if (kWave) {
     // the two cheapest rejections decide which rows are fetched; the fetch is then in flight during the geometry
     bool maybe = valid && !(culling && culling[i]);
     maybe = maybe && !((s_Tw2v[8] * p[0] + s_Tw2v[9] * p[1] + s_Tw2v[10] * p[2] + s_Tw2v[11]) <= 0.2f);
     wanted = __ballot(maybe);
-    if (wanted) wave_fetch_sh_rows(sh_regs, wanted, wave_base, (const float4*) shs);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   }
   do {
     if (!valid || (culling && culling[i])) break;
@@ -164,7 +168,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
     if (kWave) {
-      if (wanted) wave_rows_to_lds(sh_regs, s_wave_rows);
+      if (wanted) sh_regs.to_lds(s_wave_rows, wave_base, P);
       wave_lds_sync();
     } else if (kStage) {
       s_flag[threadIdx.x] = ok;
@@ -176,9 +180,10 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       float x, y, z, Y[kSh];
       view_dir(p, campos, x, y, z);
       sh_eval(sh_degree, x, y, z, Y);
-      const float* c0 = kStage ? &s_rows[threadIdx.x * kShStageStride] : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
-      const float* cr = kStage ? c0 : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float r = c0[0] * Y[0], g = c0[1] * Y[0], b = c0[2] * Y[0];
+      const float* row = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
+      const float* c0 = kStage ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
+      const float* cr = kStage ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
+      float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
       for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
       rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
     }
@@ -280,7 +285,7 @@ __device__ __forceinline__ void transmat_backward(int W, int H, float sx, float 
   gq[3] = 2 * (x * (dR[9] - dR[6]) + y * (dR[2] - dR[8]) + z * (dR[4] - dR[1]));
 }
 
-template <int kSh, bool kWave>
+template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -290,9 +295,11 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     const float4* __restrict__ grad_normal_opacity, float* __restrict__ g_means3D, float2* __restrict__ g_scales,
     float4* __restrict__ g_rot, float* __restrict__ g_opac, float* __restrict__ g_shs,
     float* __restrict__ g_sh_rest) {
+  constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
+  constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ float s_rows[kStage ? kShStageRows * kShStageStride : 1];
+  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
@@ -300,20 +307,16 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   const bool vis   = valid && radii[i] > 0;
   const int n      = sh_degree >= 0 ? sh_count(sh_degree) : 0;
   const int m1     = sh_rest ? 1 : n_sh;
-  float* my_row    = &s_rows[kStage ? threadIdx.x * kShStageStride : 0];
+  float* my_row    = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kShStageStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   const unsigned long long wanted = kWave ? __ballot(vis) : 0ull;
   if (kWave) {
     if (wanted == 0ull) {  // nothing of this wavefront was rendered: its gradient rows are zeros
       if (wave_base < P) {
-#pragma unroll
-        for (int k = 0; k < kShWavePieces; ++k) {
-          int r, c4;
-          wave_piece(k, r, c4);
-          if (wave_base + r < P)
-            ((float4*) g_shs)[(size_t) (wave_base + r) * kShWavePieces + c4] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
+        ShWaveRows<kWave ? kRow : 48>::zeros_to_global(wave_base, P, kSplit ? g_sh_rest : g_shs);
+        if (kSplit && valid && g_shs)
+          g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       }
       if (valid) {
         g_opac[i] = 0.0f;
@@ -323,9 +326,9 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       }
       return;
     }
-    ShWaveRows sh_regs;
-    wave_fetch_sh_rows(sh_regs, wanted, wave_base, (const float4*) shs);
-    wave_rows_to_lds(sh_regs, s_wave_rows);
+    ShWaveRows<kWave ? kRow : 48> sh_regs;
+    sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    sh_regs.to_lds(s_wave_rows, wave_base, P);
     wave_lds_sync();
   } else if (kStage && sh_degree >= 0) {
     s_flag[threadIdx.x] = vis;
@@ -375,7 +378,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       // was computed from (a lane only ever touches its own row)
       const float* c0 = kStage ? my_row : shs + (size_t) i * m1 * 3;
       const float* cr = kStage ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float* o0  = kStage ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
+      float* o0  = kStage && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
       float* orr = kStage ? my_row
                           : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
       if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
@@ -410,7 +413,9 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     g_rot[i]    = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (sh_degree >= 0) {
       if (kStage) {
-        for (int c = 0; c < n * 3; ++c) my_row[c] = 0.0f;
+        for (int c = kSplit ? 3 : 0; c < n * 3; ++c) my_row[c] = 0.0f;
+        if (kSplit && g_shs)
+          g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       } else {
         if (g_shs)
           for (int c = 0; c < m1 * 3; ++c) g_shs[(size_t) i * m1 * 3 + c] = 0.0f;
@@ -421,7 +426,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   }
   if (kWave) {
     wave_lds_sync();
-    wave_rows_to_global(s_wave_rows, wave_base, P, (float4*) g_shs);
+    ShWaveRows<kWave ? kRow : 48>::to_global(s_wave_rows, wave_base, P, kSplit ? g_sh_rest : g_shs);
   } else if (kStage && sh_degree >= 0 && (g_shs || g_sh_rest)) {
     __syncthreads();
     unstage_sh_grads(s_rows, blockIdx.x * blockDim.x, P, n, n_sh, sh_rest != nullptr, g_shs, g_sh_rest);
@@ -489,9 +494,11 @@ int preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float
                    (colors || sh_degree < 0),
                "gs_2d_preprocess_forward: null pointer");
   if (P == 0) return kOk;
-  const bool wave_rows = sh_degree == 3 && n_sh == 16 && !sh_rest && (uintptr_t) shs % 16 == 0;
-  auto kernel = sh_degree > 3 ? preprocess_forward_kernel<64, false>
-                              : (wave_rows ? preprocess_forward_kernel<16, true> : preprocess_forward_kernel<16, false>);
+  const int rows = wave_row_floats(sh_degree, n_sh, shs, sh_rest);
+  auto kernel = sh_degree > 3 ? preprocess_forward_kernel<64, 0>
+                : rows == 48  ? preprocess_forward_kernel<16, 48>
+                : rows == 45  ? preprocess_forward_kernel<16, 45>
+                              : preprocess_forward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, opacities, shs,
                      sh_rest, Tw2v, Tv2c, campos, trans_precomp, culling, means2D_preserve, (float2*) means2D, colors,
                      trans_mat, (float4*) normal_opacity, depths, radii, tiles_touched, (float4*) records, keep_masks, view);
@@ -535,10 +542,12 @@ FSGS_API int fsgs_gs_2d_preprocess_backward(int P, int W, int H, int sh_degree, 
   if (sh_degree >= 0)
     FSGS_REQUIRE(shs && colors && grad_colors, "gs_2d_preprocess_backward: SH path needs shs, colors and grad_colors");
   if (P == 0) return kOk;
-  const bool wave_rows = sh_degree == 3 && n_sh == 16 && !sh_rest && g_shs && (uintptr_t) shs % 16 == 0 &&
-                         (uintptr_t) g_shs % 16 == 0;
-  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, false>
-                              : (wave_rows ? preprocess_backward_kernel<16, true> : preprocess_backward_kernel<16, false>);
+  float* g_rows  = sh_rest ? g_sh_rest : g_shs;
+  const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
+  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, 0>
+                : rows == 48  ? preprocess_backward_kernel<16, 48>
+                : rows == 45  ? preprocess_backward_kernel<16, 45>
+                              : preprocess_backward_kernel<16, 0>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v,
                      Tv2c, campos, trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_colors,
                      (const float4*) grad_normal_opacity, g_means3D, (float2*) g_scales, (float4*) g_rot, g_opac,

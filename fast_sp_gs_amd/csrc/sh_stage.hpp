@@ -77,47 +77,96 @@ __device__ __forceinline__ void unstage_sh_grads(const float* __restrict__ s_row
   }
 }
 
-// ---- wavefront-private variant for complete degree-3 rows -----------------------------------------------------------
-// With all 16 coefficients in one [P,16,3] tensor a row is twelve 16-byte pieces. A wavefront then moves its own 64 rows
-// by itself: piece e = k * 64 + lane (k < 12) of the wavefront's 768 pieces belongs to row e / 12, so every load or store
-// instruction covers 1 KB of consecutive addresses, the loads can be issued before the data is needed (they are held in
-// registers while the lane does its geometry) and no block-wide barrier is involved.
-constexpr int kShWavePieces = 12;
+// ---- wavefront-private variant for complete rows ---------------------------------------------------------------------
+// A [P, kFloats / 3, 3] tensor of complete rows (all coefficients of the active degree and no others) that starts on a
+// 16-byte boundary: the 64 rows of a wavefront are 16 * kFloats consecutive 16-byte pieces, whatever the length of a row.
+// A wavefront moves them by itself: every load or store instruction covers 1 KB of consecutive addresses, the loads can be
+// issued before the data is needed (they are held in registers while the lane does its geometry) and no block-wide barrier
+// is involved. Rows of 48 floats are all coefficients of degree 3 in one tensor, of 45 the fifteen above the first where a
+// model keeps that one apart, of 27 and 12 degrees 2 and 1. Forward preprocess with 45 floats, 400k surfels (the rows are
+// 72 MB of its 150): 127 us through stage_sh_rows (4-byte loads behind a block barrier), 64 us this way.
+// In LDS a row has an odd stride, so lanes that read their own rows hit different banks: rows of odd length lie as they
+// do in memory (a piece is one 16-byte LDS write), rows of even length get one float more.
+using ShPiece = float __attribute__((ext_vector_type(4)));
 
+template <int kFloats>
 struct ShWaveRows {
-  float4 v[kShWavePieces];
+  static_assert(kFloats % 2 == 1 || kFloats % 4 == 0, "a piece lies in one row or rows are stored without a gap");
+  static constexpr int kStride = kFloats | 1;
+  static constexpr int kPieces = 16 * kFloats;          // of 64 rows
+  static constexpr int kVecs   = (kPieces + 63) / 64;   // of a lane
+  ShPiece v[kVecs];
+  float tail;
+
+  // floats and complete pieces of the wavefront's existing rows
+  static __device__ __forceinline__ int floats(int wave_base, int P) { return max(min(64, P - wave_base), 0) * kFloats; }
+
+  // `flags` has bit r set for the rows that are needed (all of them existing rows); a piece of other rows re-reads the
+  // first needed row's instead of branching. flags must not be 0.
+  __device__ __forceinline__ void fetch(unsigned long long flags, int wave_base, int P, const float* __restrict__ src) {
+    const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
+    const int first  = (__builtin_ctzll(flags) * kFloats) >> 2;
+    const float* row = src + (size_t) wave_base * kFloats;
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const int e = k * 64 + lane;
+      const int r0 = (4 * e) / kFloats, r1 = (4 * e + 3) / kFloats;
+      const bool on = e < whole && (((flags >> (r0 & 63)) | (flags >> (r1 & 63))) & 1ull);
+      v[k] = ((const ShPiece*) row)[on ? e : first];
+    }
+    if (kFloats % 4 != 0) {  // up to three floats behind the last piece of the last wavefront
+      tail = 0.0f;
+      if (lane < (all & 3)) tail = row[4 * whole + lane];
+    }
+  }
+
+  __device__ __forceinline__ void to_lds(float* __restrict__ s_wave_rows, int wave_base, int P) const {
+    const int lane = (int) __lane_id();
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const int e = k * 64 + lane;
+      if (kFloats % 2 == 1) {
+        if (e < kPieces) *(ShPiece*) (s_wave_rows + 4 * e) = v[k];
+      } else {
+        const int r = (4 * e) / kFloats;
+        float* d = s_wave_rows + r * kStride + (4 * e - r * kFloats);
+        d[0] = v[k].x, d[1] = v[k].y, d[2] = v[k].z, d[3] = v[k].w;
+      }
+    }
+    if (kFloats % 4 != 0) {
+      const int all = floats(wave_base, P);
+      if (lane < (all & 3)) s_wave_rows[(all & ~3) + lane] = tail;
+    }
+  }
+
+  // Writes the wavefront's staged rows (every existing row) to dst.
+  static __device__ __forceinline__ void to_global(const float* __restrict__ s_wave_rows, int wave_base, int P,
+                                                   float* __restrict__ dst) {
+    const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
+    float* row = dst + (size_t) wave_base * kFloats;
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const int e = k * 64 + lane;
+      if (kFloats % 2 == 1) {
+        if (e < whole) ((ShPiece*) row)[e] = *(const ShPiece*) (s_wave_rows + 4 * e);
+      } else if (e < whole) {
+        const int r = (4 * e) / kFloats;
+        const float* s = s_wave_rows + r * kStride + (4 * e - r * kFloats);
+        ((float4*) row)[e] = make_float4(s[0], s[1], s[2], s[3]);
+      }
+    }
+    if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = s_wave_rows[4 * whole + lane];
+  }
+
+  static __device__ __forceinline__ void zeros_to_global(int wave_base, int P, float* __restrict__ dst) {
+    const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
+    float* row = dst + (size_t) wave_base * kFloats;
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k)
+      if (k * 64 + lane < whole) ((float4*) row)[k * 64 + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = 0.0f;
+  }
 };
-
-__device__ __forceinline__ void wave_piece(int k, int& r, int& c4) {
-  const int e = k * 64 + (int) __lane_id();
-  r  = (e * 5462) >> 16;  // e / 12 for 0 <= e < 768
-  c4 = e - r * 12;
-}
-
-// `flags` has bit r set for the rows that are needed (all of them existing rows); the others re-read the first needed
-// row's line instead of branching. flags must not be 0.
-__device__ __forceinline__ void wave_fetch_sh_rows(ShWaveRows& regs, unsigned long long flags, int wave_base,
-                                                   const float4* __restrict__ shs4) {
-  const int first = __builtin_ctzll(flags);
-#pragma unroll
-  for (int k = 0; k < kShWavePieces; ++k) {
-    int r, c4;
-    wave_piece(k, r, c4);
-    const bool on   = (flags >> r) & 1ull;
-    const size_t at = (size_t) (wave_base + (on ? r : first)) * kShWavePieces + (on ? c4 : 0);
-    regs.v[k]       = shs4[at];
-  }
-}
-
-__device__ __forceinline__ void wave_rows_to_lds(const ShWaveRows& regs, float* __restrict__ s_wave_rows) {
-#pragma unroll
-  for (int k = 0; k < kShWavePieces; ++k) {
-    int r, c4;
-    wave_piece(k, r, c4);
-    float* d = s_wave_rows + r * kShStageStride + 4 * c4;
-    d[0] = regs.v[k].x, d[1] = regs.v[k].y, d[2] = regs.v[k].z, d[3] = regs.v[k].w;
-  }
-}
 
 // Orders a wavefront's LDS writes before its later LDS reads of other lanes' data (no instruction is generated: a
 // wavefront's LDS operations complete in order; this only stops the compiler from moving them across).
@@ -127,18 +176,13 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Writes the wavefront's 64 staged rows (every existing row) to g4[P,12].
-__device__ __forceinline__ void wave_rows_to_global(const float* __restrict__ s_wave_rows, int wave_base, int P,
-                                                    float4* __restrict__ g4) {
-#pragma unroll
-  for (int k = 0; k < kShWavePieces; ++k) {
-    int r, c4;
-    wave_piece(k, r, c4);
-    if (wave_base + r < P) {
-      const float* s = s_wave_rows + r * kShStageStride + 4 * c4;
-      g4[(size_t) (wave_base + r) * kShWavePieces + c4] = make_float4(s[0], s[1], s[2], s[3]);
-    }
-  }
+// Which rows of a preprocess kernel move this way: 48 (one tensor), 45 (the first coefficient apart) or 0 (every other
+// degree, number of coefficients or alignment: stage_sh_rows, or the lane's own walk). The gradients' tensors, where there
+// are any, have to be aligned like the coefficients'.
+inline int wave_row_floats(int sh_degree, int n_sh, const float* shs, const float* sh_rest, const float* g_rows = nullptr) {
+  if (sh_degree != 3 || n_sh != (sh_rest ? 15 : 16)) return 0;
+  if ((((uintptr_t) (sh_rest ? sh_rest : shs) | (uintptr_t) g_rows) & 15) != 0) return 0;
+  return sh_rest ? 45 : 48;
 }
 
 }  // namespace fsgs

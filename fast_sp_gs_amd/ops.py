@@ -28,7 +28,8 @@ def _sh_launch(fwd, needs, dirs, degree):
 
 def _sh_grads(bwd, needs, keep, degree, g_basis):
     dirs, = keep
-    g_dirs = torch.zeros_like(dirs)  # the operator writes the first three columns only
+    # the operator writes the first three columns
+    g_dirs = torch.empty_like(dirs) if dirs.shape[1] == 3 else torch.zeros_like(dirs)
     bwd(g_basis, dirs, dirs.shape[0], dirs.shape[1], degree, g_dirs)
     return g_dirs, None
 
@@ -51,8 +52,11 @@ def _rgb_launch(fwd, needs, sh, dirs, campos, degree, clamp):
 def _rgb_grads(bwd, needs, keep, remember, g_rgb):
     sh, dirs, campos, rgb = keep
     degree, clamp = remember
-    want = lambda i, like: torch.zeros_like(like) if like is not None and needs[i] else None
-    g_sh, g_dirs, g_campos = want(0, sh), want(1, dirs), want(2, campos)
+    want = lambda i, like, make: make(like) if like is not None and needs[i] else None
+    # the operator writes whole rows of the directions and the coefficients of its degree, and adds to the camera centre's
+    whole = sh.shape[-2] == (degree + 1) ** 2
+    g_sh = want(0, sh, torch.empty_like if whole else torch.zeros_like)
+    g_dirs, g_campos = want(1, dirs, torch.empty_like), want(2, campos, torch.zeros_like)
     bwd(degree, clamp, dirs, campos, sh, rgb, g_rgb, g_dirs, g_campos, g_sh)
     return g_sh, g_dirs, g_campos, None, None
 
