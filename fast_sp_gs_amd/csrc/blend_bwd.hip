@@ -628,7 +628,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_render_backward: bad sizes");
   if (P == 0) return kOk;
   FSGS_REQUIRE(means2D && normal_opacity && colors && trans_mat && out_opacity && dL_dpix && dL_dopacity && ranges &&
-                   n_contrib && g_colors && g_means2D && g_trans && g_normal_opacity,
+                   n_contrib && (source.region || (g_colors && g_means2D && g_trans && g_normal_opacity)),
                "GS_2D_render_backward: null pointer");
   const bool aux  = out_extras && dL_dextras;
   const bool flow = dL_dflow != nullptr;
@@ -660,13 +660,14 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
     if (aux && flow) FSGS_LAUNCH_BWD(true, true, true);
     else if (aux) FSGS_LAUNCH_BWD(true, false, true);
     else FSGS_LAUNCH_BWD(false, false, true);
-    const int waves = div_up(P, 7);  // kPerWave surfels per wavefront
+    const dim3 sums(div_up((int64_t) div_up(P, 7) * 64, 256));  // kPerWave surfels per wavefront
+    if (source.region) return check_launch("GS_2D_render_backward");  // summed by the preprocess backward
     if (keep_masks && culling_enabled())
-      hipLaunchKernelGGL(slot_reduce_culled_kernel, dim3(div_up((int64_t) waves * 64, 256)), dim3(256), 0, s, P,
-                         source, keep_masks, slot_grads, g_colors, g_means2D, g_trans, g_normal_opacity);
+      hipLaunchKernelGGL(slot_reduce_culled_kernel, sums, dim3(256), 0, s, P, source, keep_masks, slot_grads, g_colors,
+                         g_means2D, g_trans, g_normal_opacity);
     else
-      hipLaunchKernelGGL(slot_reduce_kernel, dim3(div_up((int64_t) waves * 64, 256)), dim3(256), 0, s, P, source,
-                         slot_grads, g_colors, g_means2D, g_trans, g_normal_opacity);
+      hipLaunchKernelGGL(slot_reduce_kernel, sums, dim3(256), 0, s, P, source, slot_grads, g_colors, g_means2D, g_trans,
+                         g_normal_opacity);
   } else {
     if (aux && flow) FSGS_LAUNCH_BWD(true, true, false);
     else if (aux) FSGS_LAUNCH_BWD(true, false, false);
@@ -705,20 +706,20 @@ FSGS_API int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_
                          workspace_bytes, records, keep_masks, stream);
 }
 
-// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp).
+// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp): the records stay in the
+// workspace, the preprocess backward sums them.
 FSGS_API int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
     const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
     const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
-    const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
-    float* g_normal_opacity, int64_t R, const int32_t* slot_offsets, const int32_t* slot_regions,
-    const int32_t* tiles_touched, const int32_t* radii, void* workspace, size_t workspace_bytes, const float* records,
-    const uint32_t* keep_masks, void* stream) {
+    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const float* records, void* stream) {
   FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && records),
                "gs_2d_view_backward: record slots and packed records are required");
   return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
-                         g_colors, g_means2D, g_trans, g_normal_opacity, R,
+                         nullptr, nullptr, nullptr, nullptr, R,
                          SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
-                         workspace_bytes, records, keep_masks, stream);
+                         workspace_bytes, records, nullptr, stream);
 }

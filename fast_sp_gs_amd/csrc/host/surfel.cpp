@@ -225,8 +225,6 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
     if (want_rest) g_rest = at::empty_like(sh_rest);
     if (P > 0) {
       Slab scratch;
-      const size_t g_no = scratch.reserve((size_t) P * 16), g_trans = scratch.reserve((size_t) P * 36),
-                   g_colors = scratch.reserve((size_t) P * 12);
       const size_t ws_bytes = fsgs_gs_2d_render_backward_workspace_bytes(s.R);
       const size_t ws = scratch.reserve(ws_bytes);
       scratch.allocate(points);
@@ -237,19 +235,17 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
                                      f32(trans_mat), f32(t2), f32(opacity), aux ? f32(extras) : nullptr,
                                      g_flow.defined() ? f32(flow) : nullptr, f32(g_image), f32(g_opacity),
                                      f32(g_extras), f32(g_flow), i64(ranges), i32(point_list), i32(n_contrib),
-                                     scratch.at<float>(g_colors), f32(g_means2D), scratch.at<float>(g_trans),
-                                     scratch.at<float>(g_no), s.R, (const int32_t*) keep(s.offsets),
-                                     (const int32_t*) keep(s.regions), (const int32_t*) keep(s.tiles), i32(radii),
-                                     scratch.at<void>(ws), ws_bytes, (const float*) keep(s.records),
-                                     holder->cull ? (const uint32_t*) keep(s.masks) : nullptr, stream),
+                                     s.R, (const int32_t*) keep(s.offsets), (const int32_t*) keep(s.regions),
+                                     (const int32_t*) keep(s.tiles), i32(radii), scratch.at<void>(ws), ws_bytes,
+                                     (const float*) keep(s.records), stream),
             "GS_2D_render_backward");
-      check(fsgs_gs_2d_preprocess_backward((int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations),
-                                           f32(shs), has_rest && sh_rest.numel() > 0 ? f32(sh_rest) : nullptr, f32(Tw2v),
-                                           f32(Tv2c), f32(campos), f32(trans_mat), i32(radii), colors, f32(g_means2D),
-                                           scratch.at<float>(g_trans), scratch.at<float>(g_colors),
-                                           scratch.at<float>(g_no), f32(g_points), f32(g_scales), f32(g_rot),
-                                           f32(g_opac), s.sh_degree >= 0 ? f32(g_sh) : nullptr,
-                                           has_rest && sh_rest.numel() > 0 ? f32(g_rest) : nullptr, stream),
+      check(fsgs_gs_2d_view_preprocess_backward(
+                (int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations), f32(shs),
+                has_rest && sh_rest.numel() > 0 ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2c), f32(campos),
+                f32(trans_mat), i32(radii), colors, (const int32_t*) keep(s.offsets), (const int32_t*) keep(s.regions),
+                (const int32_t*) keep(s.tiles), holder->cull ? (const uint32_t*) keep(s.masks) : nullptr,
+                scratch.at<const float>(ws), f32(g_means2D), f32(g_points), f32(g_scales), f32(g_rot), f32(g_opac),
+                s.sh_degree >= 0 ? f32(g_sh) : nullptr, has_rest && sh_rest.numel() > 0 ? f32(g_rest) : nullptr, stream),
             "gs_2d_preprocess_backward");
     }
     return {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_means2D, Tensor(), Tensor()};

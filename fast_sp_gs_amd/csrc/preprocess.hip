@@ -13,6 +13,7 @@
 #include "surfel_geom.hpp"
 
 namespace fsgs {
+bool culling_enabled();  // host-side switch (api.hip)
 namespace {
 
 #pragma clang fp contract(off)
@@ -285,7 +286,82 @@ __device__ __forceinline__ void transmat_backward(int W, int H, float sx, float 
   gq[3] = 2 * (x * (dR[9] - dR[6]) + y * (dR[2] - dR[8]) + z * (dR[4] - dR[1]));
 }
 
-template <int kSh, int kRow>
+// The records of a view: per-instance gradients in the order of the surfels (instance_slots.hpp), and which were written.
+struct ViewRecords {
+  SlotSource slots;
+  const uint32_t* masks = nullptr;   // keep masks of culled lists, nullptr: every position was written
+  const float* records = nullptr;    // [R][kGradFloats]
+};
+constexpr int kGradFloats = 18;  // 0-2 colours | 3-11 transform | 12-14 normal | 15 opacity | 16-17 centre
+constexpr int kSumStride  = 19;
+
+// Sums of the records of the wavefront's 64 surfels, in position order, to s_sums[64][kSumStride] (rows of surfels that
+// were not rendered stay as they are). Nine lanes of a surfel read a record's 72 bytes; rendered surfels are taken seven at
+// a time and three such groups together, four kept positions of each surfel in flight, so the wavefront pays a handful of
+// trips to memory for all of its surfels. `vis`: this lane's surfel was rendered.
+// `first`, `count` and `mask` are its span and keep mask (any values where it was not).
+__device__ __forceinline__ void wave_record_sums(const ViewRecords& in, int first, int count, uint32_t mask, bool vis,
+                                                 float* __restrict__ s_sums) {
+  static_assert(kCullMaskTiles == 32, "a mask word holds a small rectangle's positions");
+  constexpr int kLanes = kGradFloats / 2, kPerPass = 7, kGroups = 3, kDepth = 4;
+  const int lane = (int) __lane_id(), sub = lane / kLanes, k = lane - sub * kLanes;
+  const unsigned long long live_mask = __ballot(vis);
+  const int live = __popcll(live_mask);
+  // lane r of the first `live` lanes learns which lane holds the r-th rendered surfel
+  const int before = __popcll(live_mask & ((1ull << lane) - 1ull));
+  const int holder = __builtin_amdgcn_ds_permute((vis ? before : live + lane - before) * 4, lane);
+  for (int r0 = 0; r0 < live; r0 += kGroups * kPerPass) {
+    const float2* src[kGroups];
+    int who[kGroups], cnt[kGroups], most = 0;
+    uint32_t keep[kGroups];
+    float2 acc[kGroups];
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+      const int r   = r0 + q * kPerPass + sub;
+      const bool on = sub < kPerPass && r < live;
+      who[q] = __shfl(holder, on ? r : 0, 64);
+      const int e = __shfl(first, who[q], 64), c = __shfl(count, who[q], 64);
+      keep[q] = __shfl(mask, who[q], 64);
+      cnt[q]  = on ? c : 0;
+      who[q]  = on ? who[q] : -1;
+      src[q]  = (const float2*) in.records + (size_t) e * kLanes + k;
+      acc[q]  = make_float2(0.0f, 0.0f);
+      most    = max(most, cnt[q]);
+    }
+    for (int base = 0; __ballot(base < most) != 0ull; base += 32) {
+      uint32_t bits[kGroups];
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q) {
+        const int left = cnt[q] - base;
+        bits[q] = left <= 0 ? 0u : left >= 32 ? 0xffffffffu : (1u << left) - 1u;
+        if (cnt[q] <= kCullMaskTiles) bits[q] &= keep[q];
+      }
+      while (__ballot((bits[0] | bits[1] | bits[2]) != 0u) != 0ull) {
+        float2 v[kGroups][kDepth];
+#pragma unroll
+        for (int q = 0; q < kGroups; ++q)
+#pragma unroll
+          for (int j = 0; j < kDepth; ++j) {
+            v[q][j] = make_float2(0.0f, 0.0f);
+            if (bits[q]) v[q][j] = src[q][(size_t) (base + __builtin_ctz(bits[q])) * kLanes];
+            bits[q] &= bits[q] - 1u;
+          }
+#pragma unroll
+        for (int q = 0; q < kGroups; ++q)
+#pragma unroll
+          for (int j = 0; j < kDepth; ++j) acc[q].x += v[q][j].x, acc[q].y += v[q][j].y;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q)
+      if (who[q] >= 0) s_sums[who[q] * kSumStride + 2 * k] = acc[q].x, s_sums[who[q] * kSumStride + 2 * k + 1] = acc[q].y;
+  }
+}
+
+// kRecords: the upstream gradients are the sums of the view's records, taken here: summed by a kernel of its own they went
+// through memory once more (72 bytes per surfel out and in), and that kernel waited for three dependent loads per seven
+// surfels and wavefront. 3M surfels 1352x1014: sum 244 + preprocess 325 us -> 376 us; 300k 800x800: 34 + 36 -> 65 us.
+template <int kSh, int kRow, bool kRecords>
 __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -294,16 +370,24 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     float2* __restrict__ grad_mean2D, const float* __restrict__ grad_trans, const float* __restrict__ grad_colors,
     const float4* __restrict__ grad_normal_opacity, float* __restrict__ g_means3D, float2* __restrict__ g_scales,
     float4* __restrict__ g_rot, float* __restrict__ g_opac, float* __restrict__ g_shs,
-    float* __restrict__ g_sh_rest) {
+    float* __restrict__ g_sh_rest, ViewRecords view) {
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
+  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : kRecords ? kShStageRows * kSumStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
+  int first = 0, count = 0;
+  uint32_t mask = 0xffffffffu;
+  if (kRecords && valid) {  // beside the radius, not behind it
+    int64_t e0;
+    slot_span(view.slots, i, e0, count);
+    first = (int) e0;  // the number of instances is below 2^31
+    if (view.masks) mask = view.masks[i];
+  }
   const bool vis   = valid && radii[i] > 0;
   const int n      = sh_degree >= 0 ? sh_count(sh_degree) : 0;
   const int m1     = sh_rest ? 1 : n_sh;
@@ -311,6 +395,37 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   const unsigned long long wanted = kWave ? __ballot(vis) : 0ull;
+  ShWaveRows<kWave ? kRow : 48> sh_regs;
+  float up[kRecords ? kGradFloats : 1];
+  if (kWave && wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
+  // what the geometry reads of the surfel
+  float M[9], p[3] = {0, 0, 0}, col[3] = {0, 0, 0};
+  float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float2 s = make_float2(0.0f, 0.0f);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) M[k] = 0.0f;
+  if (vis) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) M[k] = trans_mat[9 * (size_t) i + k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[k] = means3D[3 * (size_t) i + k];
+    q = rotations[i], s = scales[i];
+    if (sh_degree >= 0)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) col[k] = colors[3 * (size_t) i + k];
+  }
+  if (kRecords) {  // the rows of coefficients and the above are on their way meanwhile
+    float* s_sums = &s_rows[(threadIdx.x & ~63) * (kStage ? kStride : kSumStride)];
+    wave_record_sums(view, first, count, mask, vis, s_sums);
+    wave_lds_sync();
+    if (vis) {
+#pragma unroll
+      for (int c = 0; c < kGradFloats; ++c) up[kRecords ? c : 0] = s_sums[(threadIdx.x & 63) * kSumStride + c];
+    } else if (valid) {
+      grad_mean2D[i] = make_float2(0.0f, 0.0f);
+    }
+    wave_lds_sync();
+  }
   if (kWave) {
     if (wanted == 0ull) {  // nothing of this wavefront was rendered: its gradient rows are zeros
       if (wave_base < P) {
@@ -326,8 +441,6 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       }
       return;
     }
-    ShWaveRows<kWave ? kRow : 48> sh_regs;
-    sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs);
     sh_regs.to_lds(s_wave_rows, wave_base, P);
     wave_lds_sync();
   } else if (kStage && sh_degree >= 0) {
@@ -342,17 +455,16 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
 #pragma unroll
     for (int k = 0; k < 16; ++k) Tw2v[k] = s_Tw2v[k], Tw2c[k] = s_Tw2c[k];
 
-    const float4 gno = grad_normal_opacity[i];
+    constexpr int kUp = kRecords ? 1 : 0;  // indexes of `up` where it is there
+    const float4 gno = kRecords ? make_float4(up[12 * kUp], up[13 * kUp], up[14 * kUp], up[15 * kUp]) : grad_normal_opacity[i];
     g_opac[i]        = gno.w;
-    float gM[9], M[9], gM_in2, gM_in5;
+    float gM[9], gM_in2, gM_in5;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) gM[k] = grad_trans[9 * (size_t) i + k], M[k] = trans_mat[9 * (size_t) i + k];
+    for (int k = 0; k < 9; ++k) gM[k] = kRecords ? up[(3 + k) * kUp] : grad_trans[9 * (size_t) i + k];
     gM_in2 = gM[2], gM_in5 = gM[5];
-    const float2 g2 = grad_mean2D[i];
+    const float2 g2 = kRecords ? make_float2(up[16 * kUp], up[17 * kUp]) : grad_mean2D[i];
     bound_backward(M, g2.x, g2.y, gM);
 
-    const float4 q   = rotations[i];
-    const float p[3] = {means3D[3 * (size_t) i], means3D[3 * (size_t) i + 1], means3D[3 * (size_t) i + 2]};
     const float t0 = 2 * (q.y * q.w + q.x * q.z), t1 = 2 * (q.y * q.z - q.x * q.w),
                 t2 = 1 - 2 * (q.x * q.x + q.y * q.y);
     const float nrm[3] = {Tw2v[0] * t0 + Tw2v[1] * t1 + Tw2v[2] * t2, Tw2v[4] * t0 + Tw2v[5] * t1 + Tw2v[6] * t2,
@@ -363,7 +475,6 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     const float cosv = -(pv[0] * nrm[0] + pv[1] * nrm[1] + pv[2] * nrm[2]);
     const float mult = cosv > 0 ? 1.0f : -1.0f;
     const float gN[3] = {mult * gno.x, mult * gno.y, mult * gno.z};
-    const float2 s = scales[i];
     float gp[3], gs[2], gq[4];
     transmat_backward(W, H, s.x, s.y, q, Tw2c, Tw2v, gM, gN, gp, gs, gq);
 
@@ -373,7 +484,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       sh_eval(sh_degree, x, y, z, Y);
       float g[3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) g[c] = grad_colors[3 * (size_t) i + c] * (float) (colors[3 * (size_t) i + c] > 0);
+      for (int c = 0; c < 3; ++c) g[c] = (kRecords ? up[c * kUp] : grad_colors[3 * (size_t) i + c]) * (float) (col[c] > 0);
       // coefficient rows are read from LDS when staged, and each gradient row is written over the coefficients it
       // was computed from (a lane only ever touches its own row)
       const float* c0 = kStage ? my_row : shs + (size_t) i * m1 * 3;
@@ -528,31 +639,62 @@ FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int 
                             ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
 }
 
+namespace {
+template <bool kRecords>
+int preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
+    const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v, const float* Tv2c,
+    const float* campos, const float* trans_mat, const int32_t* radii, const float* colors, float* grad_mean2D,
+    const float* grad_trans, const float* grad_colors, const float* grad_normal_opacity, float* g_means3D,
+    float* g_scales, float* g_rot, float* g_opac, float* g_shs, float* g_sh_rest, const ViewRecords& view, void* stream) {
+  FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_preprocess_backward: bad sizes");
+  FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_2d_preprocess_backward: sh_degree %d > %d not supported", sh_degree,
+               kMaxShDegree);
+  FSGS_REQUIRE(means3D && scales && rotations && Tw2v && Tv2c && campos && trans_mat && radii && grad_mean2D &&
+                   (kRecords || (grad_trans && grad_normal_opacity)) && g_means3D && g_scales && g_rot && g_opac,
+               "gs_2d_preprocess_backward: null pointer");
+  if (sh_degree >= 0)
+    FSGS_REQUIRE(shs && colors && (kRecords || grad_colors),
+                 "gs_2d_preprocess_backward: SH path needs shs, colors and grad_colors");
+  if (P == 0) return kOk;
+  float* g_rows  = sh_rest ? g_sh_rest : g_shs;
+  const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
+  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, 0, kRecords>
+                : rows == 48  ? preprocess_backward_kernel<16, 48, kRecords>
+                : rows == 45  ? preprocess_backward_kernel<16, 45, kRecords>
+                              : preprocess_backward_kernel<16, 0, kRecords>;
+  hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v,
+                     Tv2c, campos, trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_colors,
+                     (const float4*) grad_normal_opacity, g_means3D, (float2*) g_scales, (float4*) g_rot, g_opac,
+                     g_shs, g_sh_rest, view);
+  return check_launch("gs_2d_preprocess_backward");
+}
+}  // namespace
+
 FSGS_API int fsgs_gs_2d_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
     float* grad_mean2D, const float* grad_trans, const float* grad_colors, const float* grad_normal_opacity,
     float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs, float* g_sh_rest, void* stream) {
-  FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_preprocess_backward: bad sizes");
-  FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_2d_preprocess_backward: sh_degree %d > %d not supported", sh_degree,
-               kMaxShDegree);
-  FSGS_REQUIRE(means3D && scales && rotations && Tw2v && Tv2c && campos && trans_mat && radii && grad_mean2D &&
-                   grad_trans && grad_normal_opacity && g_means3D && g_scales && g_rot && g_opac,
-               "gs_2d_preprocess_backward: null pointer");
-  if (sh_degree >= 0)
-    FSGS_REQUIRE(shs && colors && grad_colors, "gs_2d_preprocess_backward: SH path needs shs, colors and grad_colors");
-  if (P == 0) return kOk;
-  float* g_rows  = sh_rest ? g_sh_rest : g_shs;
-  const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
-  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, 0>
-                : rows == 48  ? preprocess_backward_kernel<16, 48>
-                : rows == 45  ? preprocess_backward_kernel<16, 45>
-                              : preprocess_backward_kernel<16, 0>;
-  hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v,
-                     Tv2c, campos, trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_colors,
-                     (const float4*) grad_normal_opacity, g_means3D, (float2*) g_scales, (float4*) g_rot, g_opac,
-                     g_shs, g_sh_rest);
-  return check_launch("gs_2d_preprocess_backward");
+  return preprocess_backward<false>(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c, campos,
+                                    trans_mat, radii, colors, grad_mean2D, grad_trans, grad_colors, grad_normal_opacity,
+                                    g_means3D, g_scales, g_rot, g_opac, g_shs, g_sh_rest, ViewRecords{}, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
+    const float* slot_grads, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
+    float* g_sh_rest, void* stream) {
+  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && slot_grads),
+               "gs_2d_view_preprocess_backward: record slots and records are required");
+  ViewRecords view;
+  view.slots   = SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched};
+  view.masks   = culling_enabled() ? keep_masks : nullptr;
+  view.records = slot_grads;
+  return preprocess_backward<true>(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c, campos,
+                                   trans_mat, radii, colors, g_means2D, nullptr, nullptr, nullptr, g_means3D, g_scales,
+                                   g_rot, g_opac, g_shs, g_sh_rest, view, stream);
 }
 
 FSGS_API int fsgs_gs_2d_compute_transmat_forward(int P, int W, int H, const float* means3D, const float* scales,

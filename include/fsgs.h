@@ -211,15 +211,23 @@ int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_n, double
     float* g_normal_opacity, int64_t R, const int64_t* point_offsets, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const float* records, const uint32_t* keep_masks, void* stream);
 
-/* The same with the record slots of fsgs_gs_2d_view_preprocess; keep_masks nullptr for full lists. */
+/* The same with the record slots of fsgs_gs_2d_view_preprocess: leaves an 18-float record per instance at the start of the
+ * workspace (0-2 colours | 3-11 transform | 12-14 normal | 15 opacity | 16-17 centre) and sums nothing. */
 int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
     const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
     const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
-    const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
-    float* g_normal_opacity, int64_t R, const int32_t* slot_offsets, const int32_t* slot_regions,
-    const int32_t* tiles_touched, const int32_t* radii, void* workspace, size_t workspace_bytes, const float* records,
-    const uint32_t* keep_masks, void* stream);
+    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const float* records, void* stream);
+/* fsgs_gs_2d_preprocess_backward whose upstream gradients are the sums of those records (keep_masks nullptr for full lists);
+ * g_means2D[P,2] receives the densification proxy, zeros for surfels that were not rendered. */
+int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
+    const float* slot_grads, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot, float* g_opac,
+    float* g_shs, float* g_sh_rest, void* stream);
 
 /* ---- "fast" surfel path: transform through camera intrinsics Tv2s[3,3], adjugate-based intersection, fused
  * corner-test binning. Optical flow (trans_mat_t2) is carried by the two blend entry points below. ---- */
