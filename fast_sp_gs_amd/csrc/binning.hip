@@ -619,6 +619,51 @@ constexpr int kSmallSegment = 2048;   // entries sorted by a 256-lane block in 2
                                       // (512 lanes per block instead of 256: 27.5 against 29.6 us)
 constexpr int kLargeSegment = 16384;  // entries sorted by a 1024-lane block in 128 KB of LDS
 
+// Sorts n <= 256 entries held in LDS, ~0 behind them, by a 256-lane block: a lane keeps one entry in registers and learns
+// where it belongs. First its rank among the 64 of its wavefront's chunk, by counting (LDS broadcasts, no dependent step);
+// then runs of 64 and 128 are merged two by two, an entry's place being its place in its own run plus the number of smaller
+// entries in the other one, a binary search of log2 + 1 dependent reads. Such a segment is bound by its chain of LDS reads
+// and barriers: at most 15 reads and 4 barriers behind the chunks, where the network takes 20 rounds of read, exchange and
+// write by the one wavefront in four that has work there. Entries differ (their low halves are surfel numbers, one of each
+// in a tile). Kernel, lists of about 100 entries: 10k surfels 256x256 7.7 -> 5.3 us, 25k Gaussians 639x361 7.8 -> 5.2, fast
+// path 150k 1001x667 11.4 -> 8.5. Not for longer segments: with two to eight entries per lane the 64-bit comparisons of the
+// counting outweigh the chain (300k 800x800, lists of about 600: 24 us by the network, 32 this way).
+constexpr int kMergeSegment = 256;
+
+__device__ __forceinline__ void merge_sort_lds(uint64_t* e, int n) {
+  const int p = threadIdx.x, chunk = p & ~(kWave - 1);
+  const bool on = p < n;
+  const uint64_t key = e[p];
+  int at = p;
+  if (chunk < n) {  // the whole wavefront
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < kWave; j += 2) {
+      const ulonglong2 two = *(const ulonglong2*) (e + chunk + j);
+      rank += two.x < key, rank += two.y < key;
+    }
+    at = chunk + rank;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // a chunk is read and written by one wavefront
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (on) e[at] = key;
+  __syncthreads();
+  for (int run = kWave; run < n; run <<= 1) {
+    const int other = (at & ~(run - 1)) ^ run;
+    int below = 0;
+    for (int step = run; step > 0; step >>= 1) {
+      const int t      = below + step;
+      const bool there = on && t <= run && other + t <= n;
+      if (e[there ? other + t - 1 : 0] < key && there) below = t;
+    }
+    __syncthreads();
+    at = (at & ~(2 * run - 1)) + (at & (run - 1)) + below;
+    if (on) e[at] = key;
+    __syncthreads();
+  }
+}
+
 // One block per tile: segments up to kSmallSegment entries are sorted in LDS, longer ones are queued for
 // tile_sort_large_kernel; empty tiles get the (0, 0) range the reference's zero-initialised output has.
 // `order` (optional): the blend kernels' blockIdx -> tile table, longest lists first, so that the long segments start
@@ -627,7 +672,7 @@ __global__ void __launch_bounds__(256) tile_sort_small_kernel(int64_t* __restric
     const uint64_t* __restrict__ entries, int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out,
     int* __restrict__ large_count, int* __restrict__ large_list, const int* __restrict__ order, int n_tiles,
     int64_t R, const int* __restrict__ kept, uint64_t pad_key) {
-  __shared__ uint64_t s_e[kSmallSegment + kSmallSegment / 4];
+  __shared__ __align__(16) uint64_t s_e[kSmallSegment + kSmallSegment / 4];
   // Blocks past the tile grid (the fast path launches some): that path reserves one list position per tile of a
   // surfel's rectangle, and the positions behind the instances that passed the corner test hold the reference's padding
   // entries (key = T << 32, value = -1), which its sort leaves at the tail of the list. Written here, beside the sorts,
@@ -652,6 +697,13 @@ __global__ void __launch_bounds__(256) tile_sort_small_kernel(int64_t* __restric
     return;
   }
   const int n = (int) len;
+  if (n <= kMergeSegment) {
+    s_e[threadIdx.x] = (int) threadIdx.x < n ? entries[start + threadIdx.x] : ~0ull;
+    __syncthreads();
+    merge_sort_lds(s_e, n);
+    tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
+    return;
+  }
   const int m = padded_length(n);
   for (int k = threadIdx.x; k < m; k += 256) s_e[lds_slot<true>(k)] = k < n ? entries[start + k] : ~0ull;
   __syncthreads();

@@ -1,0 +1,27 @@
+"""Sorting of a tile's list at the lengths where the number of runs, of entries per lane or the kernel changes, bit for bit
+against the oracle: one tile, every surfel in it, depths with many values in common (the surfel's number then decides)."""
+import numpy as np
+import pytest
+import torch
+
+from util import npy
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('n', [1, 2, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 449, 511, 512, 513, 1000, 1024, 1025,
+                               1536, 1601, 2047, 2048, 2049])
+@pytest.mark.parametrize('depths', ['equal', 'few', 'rising', 'falling', 'random'])
+def test_list_of_one_tile(n, depths, device, oracle_mod):
+    from fast_sp_gs_amd._C import get_C_function
+    print(f'[tile sort] n={n} {depths}', flush=True)
+    g = torch.Generator().manual_seed(n)
+    dep = {'equal': torch.ones(n), 'few': torch.randint(1, 4, (n,), generator=g).float(), 'rising': torch.arange(1.0, n + 1),
+           'falling': torch.arange(float(n), 0.0, -1.0), 'random': torch.rand(n, generator=g) + 0.5}[depths]
+    m2 = torch.full((n, 2), 8.0)
+    radii, touched = torch.full((n,), 3, dtype=torch.int32), torch.ones(n, dtype=torch.int32)
+    ranges, pl, keys = get_C_function('GS_prepare')(16, 16, m2.to(device), dep.to(device), radii.to(device),
+                                                    touched.to(device), False, return_keys=True)[:3]
+    want_ranges, want_pl, want_keys = oracle_mod.prepare(16, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
+    assert want_pl.size == n
+    assert np.array_equal(npy(ranges), want_ranges) and np.array_equal(npy(pl), want_pl) and np.array_equal(npy(keys), want_keys)
