@@ -1,4 +1,5 @@
-"""Binning bit for bit against the oracle around the tile counts at which the counters change places (16 384 tiles: half of a
+"""Binning bit for bit against the oracle around the sizes at which one block does the prefixes and the scan (1024 tiles, 65 536
+surfels), around the tile counts at which the counters change places (16 384 tiles: half of a
 compute unit's LDS; 40 960: all of it; beyond: global memory) and around one turn of the scan's 4096 tiles per block."""
 import numpy as np
 import pytest
@@ -9,8 +10,9 @@ from util import npy
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize('gx,gy,P', [(64, 64, 3000), (17, 241, 2000), (128, 128, 5000), (5, 3277, 3000), (256, 160, 4000),
-                                     (17, 2410, 3000), (240, 135, 70_000)])
+@pytest.mark.parametrize('gx,gy,P', [(2, 2, 500), (4, 256, 2000), (41, 25, 1025), (32, 32, 65_536),
+                                     (32, 32, 65_537), (33, 31, 8193), (64, 64, 3000), (17, 241, 2000), (128, 128, 5000), (5, 3277, 300), (256, 160, 4000),
+                                     (17, 2410, 300), (240, 135, 70_000)])
 def test_lists_on_wide_grids(gx, gy, P, device, oracle_mod):
     from fast_sp_gs_amd import scenes
     from fast_sp_gs_amd._C import get_C_function
