@@ -353,6 +353,43 @@ struct G3Scatter {
   }
 };
 
+// Nine per-lane values summed over the 64 lanes: lane l of 0..8 returns the total of v[l]. The first eight go through three
+// steps of the transposed butterfly and meet their row's other half in one addition, the ninth is summed along its row and
+// takes the other half's place: 27 instructions in front of the exchange between rows, 45 for a butterfly of sixteen.
+__device__ __forceinline__ float wave_sum9_transposed(const float (&v)[9]) {
+#pragma clang fp contract(off)
+  const int lane = __lane_id();
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+  float w[4], x[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = v[2 * i + 1] + dpp_shift_zero<0x111, 0xf, 0xf>(v[2 * i + 1]);  // row_shr:1, kept by odd lanes
+    const float b = v[2 * i] + dpp_shift_zero<0x101, 0xf, 0xf>(v[2 * i]);          // row_shl:1, kept by even lanes
+    w[i] = b0 ? a : b;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = w[2 * i + 1] + dpp_shift_zero<0x112, 0xf, 0xf>(w[2 * i + 1]);
+    const float b = w[2 * i] + dpp_shift_zero<0x102, 0xf, 0xf>(w[2 * i]);
+    x[i] = b1 ? a : b;
+  }
+  const float a = x[1] + dpp_shift_zero<0x114, 0xf, 0xf>(x[1]);
+  const float b = x[0] + dpp_shift_zero<0x104, 0xf, 0xf>(x[0]);
+  float y = b2 ? a : b;
+  y += dpp_shift_zero<0x128, 0xf, 0xf>(y);  // row_ror:8
+  float z = v[8];
+  z += dpp_shift_zero<0x128, 0xf, 0xf>(z);
+  z += dpp_shift_zero<0x124, 0xf, 0xf>(z);
+  z += dpp_shift_zero<0x122, 0xf, 0xf>(z);
+  z += dpp_shift_zero<0x121, 0xf, 0xf>(z);
+  return cross_row_sum(b3 ? z : y);
+}
+
+// The walk is bound by the vector instructions of a (wavefront, entry) pair: without extra channels nine sums cross the lanes,
+// not sixteen, and the factor -opacity, the same for every pixel, is applied to the sums. The flush was bound by its atomics:
+// one lane per Gaussian and one instruction per component made every lane of it a memory request of its own, from one
+// wavefront while three waited. Sixteen lanes per Gaussian, a component each, are three requests (a line per gradient
+// tensor) and keep all wavefronts busy. 300k Gaussians 800x800: 226 -> 182 us.
 // kSlots: the per-Gaussian sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
 template <int E, bool kSlots>
 __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
@@ -364,9 +401,13 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     float* __restrict__ g_extras, const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii,
     float* __restrict__ slot_records) {
   constexpr int kB = 64;
+  // components that cross the lanes: 0-2 colour | 3-6 extras | 7-8 mean2D | 9-11 conic | 12 opacity, without extras close up
+  constexpr bool kNine = E == 0;
+  constexpr int kGeom = kNine ? 3 : 7, kSums = kNine ? 9 : 16, kRow = kNine ? 9 : 17;
   __shared__ G3Hot s_hot[kB];
   __shared__ float s_feat[kB][3 + kMaxExtra + 1];
-  __shared__ float s_part[4][kB][17];  // each wavefront's sums per staged Gaussian: plain stores, added in wavefront order
+  __shared__ float s_part[4][kB][kRow];  // each wavefront's sums per staged Gaussian: plain stores, added in wavefront order
+  __shared__ float2 s_tag[2][kB];  // number | opacity of the staged Gaussians: the flush reads them while the next are staged
   __shared__ int s_max_contrib;
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int tile = scheduled_tile(flags, tile_order), tile_x = tile % gx, tile_y = tile / gx;
@@ -385,7 +426,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) wave_max = max(wave_max, __shfl_xor(wave_max, d, kWave));
   if (lane == 0) atomicMax(&s_max_contrib, wave_max);
-  for (int e = threadIdx.x; e < 4 * kB * 17; e += kBlendThreads) (&s_part[0][0][0])[e] = 0.0f;
+  for (int e = threadIdx.x; e < 4 * kB * kRow; e += kBlendThreads) (&s_part[0][0][0])[e] = 0.0f;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));
   const int rounds = (n_todo + kB - 1) / kB;
@@ -427,6 +468,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     if ((int) threadIdx.x < n_here) {
       next.hot.mask = conic_quadrant_mask(next.hot, tile_x * kTile, tile_y * kTile, flags);
       s_hot[threadIdx.x] = next.hot;
+      if (!kSlots) s_tag[b & 1][threadIdx.x] = make_float2(__int_as_float(next.hot.id), next.hot.opacity);
 #pragma unroll
       for (int k = 0; k < 3 + E; ++k) s_feat[threadIdx.x][k] = next.feat[k];
       if (kSlots) {
@@ -452,68 +494,77 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
       // Under `hit`: the pixel's back-to-front state and two factors (zero in a lane that does not blend the entry). The
       // components are their products with quantities that are finite in every lane, formed by all lanes alike, so none
       // needs a zero of its own.
-      float g[16];
+      float g[kSums];
       const G3Hot& hot = s_hot[j];
-      float dch = 0.0f, dL_dalpha = 0.0f;
+      float dch = 0.0f, GdA = 0.0f;
       if (hit) {
         T   = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
         dch = h.alpha * T;
+        float dL_dalpha = 0.0f;
 #pragma unroll
         for (int k = 0; k < 3 + E; ++k) {
           const float v = s_feat[j][k];
           dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
           accum[k] += v * dch;
         }
-        dL_dalpha = (dL_dalpha - T_final * dL_dT) * __builtin_amdgcn_rcpf(1.0f - h.alpha);
+        GdA = (dL_dalpha - T_final * dL_dT) * __builtin_amdgcn_rcpf(1.0f - h.alpha) * h.G;
+      }
+      if (!kNine) {
+#pragma unroll
+        for (int c = 0; c < kSums; ++c) g[c] = 0.0f;
       }
 #pragma unroll
-      for (int c = 0; c < 16; ++c) g[c] = 0.0f;
-#pragma unroll
-      for (int k = 0; k < 3 + E; ++k) g[k < 3 ? k : 3 + (k - 3)] = dch * g_out[k];
-      // G = exp(power) overflows in a lane whose conic gives a large positive power; such a lane never blends
-      const float G     = hit ? h.G : 0.0f;
-      const float dL_dG = -hot.opacity * G * dL_dalpha;
-      g[7]  = dL_dG * (hot.a * h.dx + hot.b * h.dy);
-      g[8]  = dL_dG * (hot.c * h.dy + hot.b * h.dx);
-      g[9]  = 0.5f * h.dx * h.dx * dL_dG;
-      g[10] = h.dx * h.dy * dL_dG;
-      g[11] = 0.5f * h.dy * h.dy * dL_dG;
-      g[12] = G * dL_dalpha;
-      const float tot = wave_sum16_transposed(g);
-      if (lane < 16) s_part[wave][j][lane] = tot;  // a wavefront meets an entry once per batch
+      for (int k = 0; k < 3 + E; ++k) g[k] = dch * g_out[k];
+      // the geometry's part without the factor -opacity
+      g[kGeom]     = GdA * (hot.a * h.dx + hot.b * h.dy);
+      g[kGeom + 1] = GdA * (hot.c * h.dy + hot.b * h.dx);
+      g[kGeom + 2] = h.dx * h.dx * GdA;
+      g[kGeom + 3] = h.dx * h.dy * GdA;
+      g[kGeom + 4] = h.dy * h.dy * GdA;
+      g[kGeom + 5] = GdA;
+      float tot;
+      if constexpr (kNine) tot = wave_sum9_transposed(g);
+      else tot = wave_sum16_transposed(g);
+      if (lane < kSums) s_part[wave][j][lane] = tot;  // a wavefront meets an entry once per batch
     }
     __syncthreads();
-    if ((int) threadIdx.x < n_here) {
-      float a[16];
+    if (kSlots && (int) threadIdx.x < n_here) {
+      float sums[kSums], a[16];
 #pragma unroll
-      for (int c = 0; c < 16; ++c) {
+      for (int c = 0; c < kSums; ++c) {
         float sum = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) sum += s_part[w][threadIdx.x][c], s_part[w][threadIdx.x][c] = 0.0f;
-        a[c] = sum;
+        sums[c] = sum;
       }
-      if (kSlots) {
-        float4* dst = (float4*) (slot_records + slot * kG3Slots);
+      const float no = -s_hot[threadIdx.x].opacity;
 #pragma unroll
-        for (int c = 0; c < kG3Slots / 4; ++c) dst[c] = make_float4(a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]);
-      } else {
-        const int id = s_hot[threadIdx.x].id;
+      for (int c = 0; c < 16; ++c) a[c] = c < 3 + E ? sums[c < kGeom ? c : 0] : 0.0f;
+      a[7] = no * sums[kGeom], a[8] = no * sums[kGeom + 1];
+      a[9] = 0.5f * no * sums[kGeom + 2], a[10] = no * sums[kGeom + 3], a[11] = 0.5f * no * sums[kGeom + 4];
+      a[12] = sums[kGeom + 5];
+      float4* dst = (float4*) (slot_records + slot * kG3Slots);
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-          if (a[c] != 0.0f) atomicAdd(&g_colors[3 * (size_t) id + c], a[c]);
+      for (int c = 0; c < kG3Slots / 4; ++c) dst[c] = make_float4(a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]);
+    }
+    if (!kSlots) {
+      const int c = (int) threadIdx.x & 15, g = c - kGeom;  // component, and its number among the geometry's six
+      if (c < 3 + E || (g >= 0 && g < 6)) {
+        float* const out = c < 3 ? g_colors + c : c < 3 + E ? g_extras + (c - 3) : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
+        const size_t row = c < 3 ? 3 : c < 3 + E ? E : g < 2 ? 2 : 4;
+        for (int e = (int) threadIdx.x >> 4; e < n_here; e += kBlendThreads / 16) {
+          float sum = 0.0f;
 #pragma unroll
-        for (int c = 0; c < E; ++c)
-          if (a[3 + c] != 0.0f) atomicAdd(&g_extras[(size_t) E * id + c], a[3 + c]);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          if (a[7 + c] != 0.0f) atomicAdd(&g_means2D[2 * (size_t) id + c], a[7 + c]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (a[9 + c] != 0.0f) atomicAdd(&g_conic_opacity[4 * (size_t) id + c], a[9 + c]);
+          for (int w = 0; w < 4; ++w) sum += s_part[w][e][c], s_part[w][e][c] = 0.0f;
+          const float2 tag = s_tag[b & 1][e];
+          if (g >= 0 && g < 5) sum *= -tag.y;
+          if (g == 2 || g == 4) sum *= 0.5f;
+          if (sum != 0.0f) atomicAdd(out + row * (size_t) __float_as_int(tag.x), sum);
+        }
       }
     }
-    // a lane only touches its own rows of s_part and its staged entry between this flush and the barrier that follows
-    // the next batch's LDS store
+    // between this flush and the barrier that follows the next batch's LDS store, wavefronts touch s_part (the flush) and
+    // the other copy of s_tag; with kSlots a lane touches its own rows of s_part and its own staged entry
   }
 }
 
