@@ -389,7 +389,8 @@ __device__ __forceinline__ float wave_sum9_transposed(const float (&v)[9]) {
 // not sixteen, and the factor -opacity, the same for every pixel, is applied to the sums. The flush was bound by its atomics:
 // one lane per Gaussian and one instruction per component made every lane of it a memory request of its own, from one
 // wavefront while three waited. Sixteen lanes per Gaussian, a component each, are three requests (a line per gradient
-// tensor) and keep all wavefronts busy. 300k Gaussians 800x800: 226 -> 182 us.
+// tensor) and keep all wavefronts busy. 300k Gaussians 800x800: 226 -> 182 us, 178 with
+// the next entry requested ahead.
 // kSlots: the per-Gaussian sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
 template <int E, bool kSlots>
 __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
@@ -483,19 +484,24 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
 
     unsigned long long todo = __ballot(lane < n_here && ((s_hot[lane].mask >> wave) & 1u) &&
                                        (n_todo - 1 - (b * kB + lane)) < wave_max);
-    while (todo) {
-      const int j = __builtin_ctzll(todo);
-      todo &= todo - 1;
+    // The next entry's record and channels are requested before the current entry is evaluated, into alternating registers: a
+    // wavefront walks its list alone, and an exposed LDS round trip per entry sits on the tile's critical path.
+    struct Staged {
+      G3Hot hot;
+      float feat[3 + E];
+    };
+    auto entry = [&](const Staged& at, int j) {
+      const G3Hot& hot        = at.hot;
+      const float* const feat = at.feat;
       const int pos = n_todo - 1 - (b * kB + j);  // 0-based position in the tile's list
       G3Hit h;
       unsigned long long pass;
-      const bool hit = conic_alpha_flat(s_hot[j], pxf, pyf, h, &pass) && (pos < last_contrib);
-      if ((pass & wave_ballot(pos < last_contrib)) == 0ull) continue;
+      const bool hit = conic_alpha_flat(hot, pxf, pyf, h, &pass) && (pos < last_contrib);
+      if ((pass & wave_ballot(pos < last_contrib)) == 0ull) return;
       // Under `hit`: the pixel's back-to-front state and two factors (zero in a lane that does not blend the entry). The
       // components are their products with quantities that are finite in every lane, formed by all lanes alike, so none
       // needs a zero of its own.
       float g[kSums];
-      const G3Hot& hot = s_hot[j];
       float dch = 0.0f, GdA = 0.0f;
       if (hit) {
         T   = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
@@ -503,7 +509,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
         float dL_dalpha = 0.0f;
 #pragma unroll
         for (int k = 0; k < 3 + E; ++k) {
-          const float v = s_feat[j][k];
+          const float v = feat[k];
           dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
           accum[k] += v * dch;
         }
@@ -526,6 +532,37 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
       if constexpr (kNine) tot = wave_sum9_transposed(g);
       else tot = wave_sum16_transposed(g);
       if (lane < kSums) s_part[wave][j][lane] = tot;  // a wavefront meets an entry once per batch
+    };
+    auto pop = [&]() {
+      const int j = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      return j;
+    };
+    auto peek = [&]() {
+      const int j = todo ? (int) __builtin_ctzll(todo) : 0;
+      Staged at;
+      at.hot = s_hot[j];
+#pragma unroll
+      for (int k = 0; k < 3 + E; ++k) at.feat[k] = s_feat[j][k];
+      return at;
+    };
+    if (todo != 0ull) {
+      Staged one = peek(), two;
+      while (todo) {
+        {
+          const int j = pop();
+          two         = peek();
+          __builtin_amdgcn_sched_barrier(0);
+          entry(one, j);
+        }
+        if (todo == 0ull) break;
+        {
+          const int j = pop();
+          one         = peek();
+          __builtin_amdgcn_sched_barrier(0);
+          entry(two, j);
+        }
+      }
     }
     __syncthreads();
     if (kSlots && (int) threadIdx.x < n_here) {
