@@ -167,9 +167,14 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
     const Tensor g_image = given(g[0], {3, H, W}), g_opacity = given(g[1], {H, W});
     const Tensor g_maps = s.E ? given(g[4], {s.E, H, W}) : Tensor();
 
-    auto like_if = [&](size_t input, const Tensor& x) {
-      return x.defined() && ctx->needs_input_grad(input) ? at::empty_like(x) : Tensor();
-    };
+    // the context numbers the node's edges, and an optional input that was left out has none
+    size_t edge = 0;
+    auto wanted = [&](const Tensor& x) { return x.defined() && ctx->needs_input_grad(edge++); };
+    wanted(points);
+    const bool want_scales = wanted(scales), want_rot = wanted(rotations);
+    wanted(opacities);
+    const bool want_sh = wanted(shs), want_rest = wanted(sh_rest), want_cov3D = wanted(cov3D), want_cov2D = wanted(cov2D);
+    auto like_if = [](bool want, const Tensor& x) { return want ? at::empty_like(x) : Tensor(); };
     // the blend adds its sums to these: screen positions 2 | conic and opacity 4 | colours 3 | extras E
     const Tensor sums = at::zeros({P * (9 + s.E)}, points.options());
     Tensor g_means2D = sums.narrow(0, 0, 2 * P).view({P, 2}), g_conic = sums.narrow(0, 2 * P, 4 * P).view({P, 4}),
@@ -179,10 +184,10 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
     Tensor g_points = at::empty_like(points), g_opac = at::empty_like(opacities), g_scales, g_rot, g_cov3D, g_cov2D, g_sh,
            g_rest;
     // which covariance was given decides where its gradient goes
-    if (cov2D.defined()) g_cov2D = like_if(7, cov2D);
-    else if (cov3D.defined()) g_cov3D = like_if(6, cov3D);
-    else g_scales = like_if(1, scales), g_rot = like_if(2, rotations);
-    if (sh) g_sh = like_if(4, shs), g_rest = like_if(5, sh_rest);
+    if (cov2D.defined()) g_cov2D = like_if(want_cov2D, cov2D);
+    else if (cov3D.defined()) g_cov3D = like_if(want_cov3D, cov3D);
+    else g_scales = like_if(want_scales, scales), g_rot = like_if(want_rot, rotations);
+    if (sh) g_sh = like_if(want_sh, shs), g_rest = like_if(want_rest, sh_rest);
     if (P > 0) {
       const float* colors = sh ? keep(s.colors) : f32(shs);
       const int M = rest_used ? (int) sh_rest.size(1) : shs.dim() == 3 ? (int) shs.size(1) : 0;
@@ -203,7 +208,7 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
                                         nullptr, stream),
             "gs_preprocess_backward");
     }
-    if (!sh && ctx->needs_input_grad(4)) g_sh = g_colors;  // pre-computed colours: the blend's sums are their gradient
+    if (!sh && want_sh) g_sh = g_colors;  // pre-computed colours: the blend's sums are their gradient
     return {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_cov3D, g_cov2D, g_means2D, g_extras, Tensor(), Tensor()};
   }
 };

@@ -198,3 +198,43 @@ def test_gaussian_view_equals_operators(P, W, H, mode, device):
     ref = torch.autograd.grad(ref_maps, wanted + [m2], up)
     for a, b in zip(got, ref):
         assert (a - b).norm() <= 1e-4 * b.norm() + 1e-7
+
+
+@pytest.mark.parametrize('split', [False, True])
+@pytest.mark.parametrize('table', [False, True])
+@pytest.mark.parametrize('given', ['cov3D', 'cov2D'])
+def test_gaussian_view_with_given_covariance(given, split, table, device):
+    """Pre-computed covariances with and without the optional inputs in front of and behind them, through `.backward()` and
+    as the only gradient asked for, with the caller's screen positions and without."""
+    import math
+
+    from fast_sp_gs_amd.renderer import gaussian_render as m
+    P, W, H = 300, 49, 31
+    s, cam_h, g = _scene(P, W, H, 7)
+    cam = cam_h.to(device)
+    third = torch.exp(torch.randn(P, 1, generator=g) * 0.5 - 4.2)
+    means, scales, rot, opac = _leaves(device, s.means3D, torch.cat([s.scales, third], dim=1), s.rotations, s.opacities)
+    tan = (math.tan(math.radians(25.0)), math.tan(math.radians(25.0)) * H / W)
+    cov = m.compute_cov3D(scales, rot).detach()
+    if given == 'cov2D':
+        cov = m.compute_cov2D(means, cov, cam.Tw2v, W / (2 * tan[0]), H / (2 * tan[1]), *tan).detach()
+    cov.requires_grad_(True)
+    sh, rest = (_leaves(device, s.shs[:, :1].contiguous(), s.shs[:, 1:].contiguous()) if split else
+                (*_leaves(device, s.shs), None))
+    extras = _leaves(device, torch.randn(P, 3, generator=g))[0] if table else None
+    args = (sh, rest, opac, scales, rot, *((cov, None) if given == 'cov3D' else (None, cov)), extras, (W, H), 3, cam.Tw2v,
+            cam.Tv2c, cam.campos, tan, False, None, None, None, None)
+    up = [torch.randn(n, H, W, generator=g).to(device) for n in (3, 1, 3)]
+    loss = lambda o: (o[0] * up[0]).sum() + (o[1] * up[1]).sum() + ((o[2] * up[2]).sum() if table else 0)
+    screen = lambda: torch.zeros(P, 2, device=device, requires_grad=True)
+    wanted = [cov, means, opac, sh] + ([rest] if split else []) + ([extras] if table else [])
+    want = torch.autograd.grad(loss(m._rasterize_operators(means, screen(), *args)), wanted)
+    for m2 in (screen(), None):
+        value = loss(m.RasterizeGaussians(means, m2, *args))
+        alone, = torch.autograd.grad(value, [cov], retain_graph=True)
+        value.backward()
+        for t, w in zip([alone] + [t.grad for t in wanted], [want[0], *want]):
+            assert t is not None and (t - w).norm() <= 1e-4 * w.norm() + 1e-7
+        assert scales.grad is None and rot.grad is None
+        for t in wanted:
+            t.grad = None
