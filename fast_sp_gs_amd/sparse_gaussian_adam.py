@@ -69,6 +69,14 @@ class DenseAdam(torch.optim.Adam):
     with torch's fused step the parameters' version counters stay: whoever keeps copies of them (`DeformNetwork.pack`)
     refreshes those itself."""
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        # one step count per parameter, also where the loaded state shares tensors (between parameters, or with the optimiser
+        # it was taken from): torch's step advances each parameter's in place
+        for entry in self.state.values():
+            if isinstance(entry.get('step'), torch.Tensor):
+                entry['step'] = entry['step'].clone()
+
     @torch.no_grad()
     def step(self, closure=None):
         groups = self.param_groups
@@ -82,19 +90,19 @@ class DenseAdam(torch.optim.Adam):
             params = [p for p in group['params'] if p.grad is not None]
             if not params:
                 continue
-            fresh = [p for p in params if not self.state[p]]
-            if fresh:
-                count = torch.zeros((), dtype=torch.float32)
-                for p in fresh:
-                    self.state[p].update(step=count, exp_avg=torch.zeros_like(p), exp_avg_sq=torch.zeros_like(p))
+            for p in params:
+                if not self.state[p]:
+                    self.state[p].update(step=torch.zeros((), dtype=torch.float32), exp_avg=torch.zeros_like(p),
+                                         exp_avg_sq=torch.zeros_like(p))
             states = [self.state[p] for p in params]
-            counts = {id(s['step']): s['step'] for s in states}  # tensors first seen together share theirs
             b1, b2 = group['betas']
-            factors = {}
-            for key, count in counts.items():
-                count += 1
-                t = count.item()
-                factors[key] = (group['lr'] / (1 - b1 ** t), (1 - b2 ** t) ** 0.5)
-            per = [factors[id(s['step'])] for s in states]
+            torch._foreach_add_([s['step'] for s in states], 1)
+            factors = {}  # step count -> the rate and the root of the bias corrections
+            per = []
+            for s in states:
+                t = s['step'].item()
+                if t not in factors:
+                    factors[t] = (group['lr'] / (1 - b1 ** t), (1 - b2 ** t) ** 0.5)
+                per.append(factors[t])
             host.adam_dense(params, [p.grad for p in params], [s['exp_avg'] for s in states],
                             [s['exp_avg_sq'] for s in states], [f[0] for f in per], [f[1] for f in per], b1, b2, group['eps'])

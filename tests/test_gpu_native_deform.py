@@ -81,3 +81,38 @@ def test_dense_adam_follows_torch(device):
     second = net(x, t)[0]
     assert not torch.equal(first, second)  # the step's weights are in use
     assert (second - net.forward_fp32(x, t)[0]).norm() <= 2e-2 * second.norm() + 1e-5
+
+
+@pytest.mark.parametrize('change', ['torch', 'dense', 'weight_decay'])
+def test_dense_adam_state_goes_on_in_torch(change, device):
+    """Three plain steps, then two more: in torch's Adam or a new DenseAdam with the saved state, or in the same optimiser
+    with a setting that takes torch's step. Step counts and parameters as torch's throughout."""
+    import io
+
+    from fast_sp_gs_amd.sparse_gaussian_adam import DenseAdam
+    g = torch.Generator().manual_seed(4)
+    values = [torch.randn(n, generator=g) for n in (1, 3, 64, 1025)]
+    mine, theirs = ([v.clone().to(device).requires_grad_(True) for v in values] for _ in range(2))
+    a, b = DenseAdam(mine, lr=1e-2), torch.optim.Adam(theirs, lr=1e-2)
+
+    def step(first, second):
+        for p, q in zip(mine, theirs):
+            p.grad = torch.randn(p.shape, generator=g).to(device)
+            q.grad = p.grad.clone()
+        first.step(), second.step()
+
+    for _ in range(3):
+        step(a, b)
+    if change == 'weight_decay':
+        for opt in (a, b):
+            opt.param_groups[0]['weight_decay'] = 1e-2
+    else:
+        file = io.BytesIO()
+        torch.save(a.state_dict(), file)
+        file.seek(0)
+        a = (torch.optim.Adam if change == 'torch' else DenseAdam)(mine, lr=1e-2)
+        a.load_state_dict(torch.load(file, weights_only=True))
+    for _ in range(2):
+        step(a, b)
+    for p, q in zip(mine, theirs):
+        assert float(a.state[p]['step']) == 5 and torch.allclose(p, q, rtol=0, atol=1e-6)

@@ -392,3 +392,19 @@ def test_freq_encoder_double_tensor_goes_through_single_precision(oracle_mod):
     assert np.abs(out - np.concatenate(parts, -1)).max() < 1.5e-7
     assert np.array_equal(out[:, :D], x)  # the pass-through columns keep the double values
     assert np.abs(out - exact).max() > 4e-6
+
+
+def test_dense_adam_counts_every_parameter_by_itself():
+    """A loaded state whose step counts are one tensor, and the optimiser it came from, both go on counting by ones."""
+    from fast_sp_gs_amd.sparse_gaussian_adam import DenseAdam
+    params = [torch.ones(3, requires_grad=True) for _ in range(4)]
+    for p in params:
+        p.grad = torch.ones(3)
+    a, b = DenseAdam(params, lr=1e-2), DenseAdam(params, lr=1e-2)
+    a.step()
+    state, count = a.state_dict(), torch.ones(())
+    for entry in state['state'].values():
+        entry['step'] = count
+    b.load_state_dict(state)
+    b.step()
+    assert [float(b.state[p]['step']) for p in params] == [2.0] * 4 and float(count) == 1.0
