@@ -51,7 +51,7 @@ struct Nearest : public torch::autograd::Function<Nearest> {
     at::AutoDispatchBelowADInplaceOrView no_graph;
     Tensor g_x, g_y;
     nearest_backward(t[0], t[1], t[2], contiguous(g[0]), ctx->needs_input_grad(0), g_x, g_y);
-    return {g_x, ctx->needs_input_grad(1) ? g_y : Tensor(), Tensor()};
+    return first_order_only(g, {t[0], t[1]}, {g_x, ctx->needs_input_grad(1) ? g_y : Tensor(), Tensor()});
   }
 };
 
@@ -119,6 +119,7 @@ struct Warp : public torch::autograd::Function<Warp> {
     at::AutoDispatchBelowADInplaceOrView no_graph;
     const int64_t N = points.size(0), M = sp_points.size(0), K = index.size(1);
     const int S = sp_s.defined() ? m.S : 0;
+    const variable_list inputs = {sp_points, sp_t, sp_r, sp_s, sp_rot, radius, weight};
     auto given = [&](const Tensor& x, int64_t columns) {
       return x.defined() ? contiguous(x) : at::zeros({N, columns}, points.options());
     };
@@ -139,7 +140,7 @@ struct Warp : public torch::autograd::Function<Warp> {
                                      f32(g_t), f32(g_sp_rot), f32(g_r), f32(g_s), S ? (int) sp_s.size(1) : 0, f32(g_radius),
                                      f32(g_weight), ws.data_ptr(), bytes, stream_of(points)),
             "superpoint_backward");
-      return {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()};
+      return first_order_only(g, inputs, {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()});
     }
     const Tensor g_pair = empty({N, K}, points);
     check(fsgs_lbs_blend_backward((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
@@ -153,7 +154,7 @@ struct Warp : public torch::autograd::Function<Warp> {
       nearest_backward(points, sp_points, index, g_pair, false, none, g_y);
       g_c = m.warp_mode == 2 ? g_c.add_(g_y) : g_y;  // the pivot's gradient exists in that mode only
     }
-    return {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()};
+    return first_order_only(g, inputs, {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()});
   }
 };
 
@@ -188,6 +189,7 @@ struct Apply : public torch::autograd::Function<Apply> {
     const auto t = ctx->get_saved_variables();
     const bool log_scales = ctx->saved_data["log"].toBool();
     at::AutoDispatchBelowADInplaceOrView no_graph;
+    const variable_list upstream = g;
     for (auto& x : g) x = contiguous(x);
     Tensor g_s = g[1], g_r;  // the sums hand their upstream gradient to both addends
     const bool rot = g[2].defined(), logs = log_scales && g[1].defined();
@@ -203,7 +205,8 @@ struct Apply : public torch::autograd::Function<Apply> {
       if (!rot) g_r = Tensor();
     }
     auto pick = [&](size_t k, const Tensor& x) { return ctx->needs_input_grad(k) ? x : Tensor(); };
-    return {pick(0, g[0]), pick(1, g[0]), pick(2, g_s), pick(3, g[1]), pick(4, g_r), pick(5, g_r), Tensor()};
+    return first_order_only(upstream, {t[0], t[1], t[2]}, {pick(0, g[0]), pick(1, g[0]), pick(2, g_s), pick(3, g[1]), pick(4, g_r),
+                                                           pick(5, g_r), Tensor()});
   }
 };
 
@@ -261,6 +264,7 @@ struct Mlp : public torch::autograd::Function<Mlp> {
     const auto capsule = ctx->saved_data["shape"].toCapsule();
     const MlpShape& s = *static_cast<const MlpShape*>(capsule.get());
     at::AutoDispatchBelowADInplaceOrView no_graph;
+    const variable_list upstream = g;
     const int64_t B = s.B, Din = s.Din, L = s.n_layers;
     int64_t n_out = 0;
     std::vector<const float*> up;
@@ -286,7 +290,7 @@ struct Mlp : public torch::autograd::Function<Mlp> {
     for (size_t k = 0; k < grads.size(); ++k)
       if (!ctx->needs_input_grad(k)) grads[k] = Tensor();
     grads.push_back(Tensor());
-    return grads;
+    return first_order_only(upstream, {}, std::move(grads));
   }
 };
 
@@ -327,7 +331,7 @@ struct Loss : public torch::autograd::Function<Loss> {
                                    ctx->saved_data["lambda"].toDouble(), f32(img), f32(target), f32(up), d, d + n, d + 2 * n,
                                    f32(grad), stream_of(img)),
           "image_loss_backward");
-    return {grad, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return first_order_only(g, {img}, {grad, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()});
   }
 };
 

@@ -178,6 +178,7 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
     const int W = s.W, H = s.H;
     const int64_t P = points.size(0);
     void* stream = stream_of(points);
+    const variable_list upstream = g;
     for (auto& x : g) x = contiguous(x);
 
     Tensor g_image = g[0], g_opacity = g[1], g_extras, g_flow;
@@ -234,7 +235,8 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
                                                 stream),
             "gs_2d_fast_preprocess_backward");
     }
-    return {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_means2D, Tensor(), Tensor()};
+    return first_order_only(upstream, {points, scales, rotations, opacities, shs, sh_rest, means2D},
+                            {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_means2D, Tensor(), Tensor()});
   }
 };
 

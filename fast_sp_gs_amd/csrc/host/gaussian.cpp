@@ -162,6 +162,7 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
     const int W = s.W, H = s.H;
     const int64_t P = points.size(0);
     void* stream = stream_of(points);
+    const variable_list upstream = g;
     for (auto& x : g) x = contiguous(x);
     auto given = [&](const Tensor& x, at::IntArrayRef shape) { return x.defined() ? x : at::zeros(shape, points.options()); };
     const Tensor g_image = given(g[0], {3, H, W}), g_opacity = given(g[1], {H, W});
@@ -209,7 +210,9 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
             "gs_preprocess_backward");
     }
     if (!sh && want_sh) g_sh = g_colors;  // pre-computed colours: the blend's sums are their gradient
-    return {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_cov3D, g_cov2D, g_means2D, g_extras, Tensor(), Tensor()};
+    return first_order_only(upstream, {points, scales, rotations, opacities, shs, sh_rest, cov3D, cov2D, means2D, extras},
+                            {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_cov3D, g_cov2D, g_means2D, g_extras, Tensor(),
+                             Tensor()});
   }
 };
 

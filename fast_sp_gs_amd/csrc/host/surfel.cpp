@@ -190,6 +190,7 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
     const int W = s.W, H = s.H;
     const int64_t P = points.size(0);
     void* stream = stream_of(points);
+    const variable_list upstream = g;
     for (auto& x : g) x = contiguous(x);
 
     Tensor g_image = g[0], g_opacity = g[1], g_extras, g_flow;
@@ -248,7 +249,8 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
                 s.sh_degree >= 0 ? f32(g_sh) : nullptr, has_rest && sh_rest.numel() > 0 ? f32(g_rest) : nullptr, stream),
             "gs_2d_preprocess_backward");
     }
-    return {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_means2D, Tensor(), Tensor()};
+    return first_order_only(upstream, {points, scales, rotations, opacities, shs, sh_rest, means2D},
+                            {g_points, g_scales, g_rot, g_opac, g_sh, g_rest, g_means2D, Tensor(), Tensor()});
   }
 };
 

@@ -1,5 +1,7 @@
 #include "torch_util.hpp"
 
+#include <torch/csrc/autograd/functions/basic_ops.h>
+
 #include <map>
 
 namespace fsgs_host {
@@ -69,6 +71,21 @@ void require_accumulators(const char* what, const OptTensor& max_count, const Op
   one("accum_max_count", max_count, at::kInt);
   one("accum_weights_count", weights_count, at::kInt);
   one("accum_weights_p", weights_p, at::kFloat);
+}
+
+variable_list first_order_only(const variable_list& upstream, const variable_list& inputs, variable_list grads) {
+  bool recorded = false;
+  if (at::GradMode::is_enabled())
+    for (const Tensor& g : upstream) recorded = recorded || (g.defined() && g.requires_grad());
+  if (!recorded) return grads;
+  variable_list from = upstream;
+  from.insert(from.end(), inputs.begin(), inputs.end());
+  const auto refuse = std::make_shared<torch::autograd::Error>(
+      "trying to differentiate twice a function whose backward is differentiable once only",
+      torch::autograd::collect_next_edges(from));
+  for (Tensor& g : grads)
+    if (g.defined()) torch::autograd::create_gradient_edge(g = g.detach(), refuse);
+  return grads;
 }
 
 int64_t* pinned_count() {

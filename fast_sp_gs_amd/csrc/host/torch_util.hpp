@@ -63,6 +63,11 @@ inline Tensor empty(at::IntArrayRef shape, const Tensor& like, at::ScalarType ty
 }
 inline Tensor contiguous(const Tensor& t) { return t.defined() ? t.contiguous() : t; }
 
+// A node's gradients come from kernels, outside the graph. Where the backward itself is recorded (create_graph=True) they
+// get a node that raises when it is differentiated, reached from what they depend on (the upstream gradients and the saved
+// inputs); without it they would pass for constants.
+variable_list first_order_only(const variable_list& upstream, const variable_list& inputs, variable_list grads);
+
 inline void* stream_of(const Tensor& t) { return (void*) c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // One uninitialised allocation handed out in 256-byte aligned pieces: a view's scratch, or what only its backward reads.

@@ -1,0 +1,83 @@
+"""The native host layer's autograd nodes where autograd does more than one backward: a recorded backward."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+P, W, H, M = 300, 49, 31, 40
+NODES = ['surfel', 'fast_surfel', 'gaussian', 'deform_apply', 'knn', 'warp', 'network', 'loss']
+
+
+def _scene(device):
+    from fast_sp_gs_amd import scenes
+    g = torch.Generator().manual_seed(7)
+    s = scenes._surfels(g, P, 'cube', -4.2, 0.7, 0.0, 1.5).to(device)
+    return s, scenes.pinhole(W, H, 50.0, torch.tensor([0.3, 0.2, 4.0])).to(device), g
+
+
+def _surfel(points, scene, cam, **kw):
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    return GS_2D_render(points, scene.scales, scene.rotations, scene.opacities, (W, H), cam.Tw2v, cam.Tv2c, campos=cam.campos,
+                        sh_degree=3, sh_features=scene.shs, **kw)
+
+
+def _fast_surfel(points, scene, cam):
+    from fast_sp_gs_amd.renderer.gs_2d_fast_render import GS_2D_fast_render
+    return GS_2D_fast_render(points, scene.scales, scene.rotations, scene.opacities, (W, H), cam.Tw2v, cam.Tv2c, cam.Tv2s,
+                             campos=cam.campos, sh_degree=3, sh_features=scene.shs)
+
+
+def _gaussian(points, scene, cam):
+    from fast_sp_gs_amd.renderer.gaussian_render import render
+    tan = math.tan(math.radians(25.0))
+    scales = torch.cat([scene.scales, scene.scales[:, :1]], dim=1)
+    return render(cam.Tw2v, cam.Tv2c, (W, H), points, scene.opacities, scales, scene.rotations, campos=cam.campos,
+                  FoV=(2 * math.atan(tan), 2 * math.atan(tan * H / W)), sh_degree=3, sh_features=scene.shs)
+
+
+def _node(which, device):
+    """(function of one tensor through the node, a value for it)"""
+    from fast_sp_gs_amd.deform import DeformNetwork, deform_apply, knn_points, superpoint_deform
+    from fast_sp_gs_amd.ssim import l1_dssim_loss
+    scene, cam, g = _scene(device)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(device)
+    if which in ('surfel', 'fast_surfel', 'gaussian'):
+        view = {'surfel': _surfel, 'fast_surfel': _fast_surfel, 'gaussian': _gaussian}[which]
+        return lambda x: view(x, scene, cam)['images'], scene.means3D
+    if which == 'deform_apply':
+        rest = [r(P, 3), r(P, 2), r(P, 2), r(P, 4)]
+        return lambda x: deform_apply(r0, *rest, x)[2], (r0 := r(P, 3), r(P, 4))[1]
+    controls = r(M, 3)
+    if which == 'knn':
+        return lambda x: knn_points(x, controls, 3)[0], r(P, 3)
+    if which == 'warp':
+        points, rest = r(P, 3), (r(M, 4), r(M, 2), r(M, 4))
+        return lambda x: superpoint_deform(points, controls, x, *rest)[0], r(M, 3)
+    if which == 'network':
+        net, t = DeformNetwork().to(device), torch.rand(1, generator=g).to(device)
+
+        def run(x):
+            bias = net.gaussian_warp.bias
+            net.gaussian_warp._parameters['bias'] = x
+            try:
+                return net(controls, t)[0]
+            finally:
+                net.gaussian_warp._parameters['bias'] = bias
+        return run, r(3)
+    target = torch.rand(3, H, W, generator=g).to(device)
+    return lambda x: l1_dssim_loss(x, target), torch.rand(3, H, W, generator=g).to(device)
+
+
+@pytest.mark.parametrize('which', NODES)
+def test_recorded_backward(which, device):
+    """Under create_graph=True the first derivative is the plain one, and a second one raises instead of being zero."""
+    f, x = _node(which, device)
+    x = x.clone().requires_grad_(True)
+    plain, = torch.autograd.grad((f(x) ** 2).sum(), [x])
+    recorded, = torch.autograd.grad((f(x) ** 2).sum(), [x], create_graph=True)
+    # device atomics add a point's tiles in another order
+    assert (recorded - plain).norm() <= 1e-4 * plain.norm() and recorded.requires_grad
+    with pytest.raises(RuntimeError, match='differentiate twice'):
+        torch.autograd.grad((recorded ** 2).sum(), [x])
