@@ -12,6 +12,7 @@ bool wants(const OptTensor& t) { return has(t) && t->requires_grad(); }
 
 void nearest(const Tensor& x, const Tensor& y, int64_t K, Tensor& d2, Tensor& index) {
   const char* what = "knn_topk";
+  refuse_duals("knn_points", x, y);
   require(what, "x", x, at::kFloat), require(what, "y", y, at::kFloat);
   if (x.dim() != 2 || y.dim() != 2 || x.size(1) != y.size(1)) fail("knn_topk: feature dimensions differ");
   const int64_t N = x.size(0), M = y.size(0), D = x.size(1);
@@ -57,6 +58,7 @@ struct Nearest : public torch::autograd::Function<Nearest> {
 
 variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   const char* what = "lbs_blend";
+  refuse_duals("superpoint_deform", w.sp_t, w.sp_r, w.sp_s, w.sp_rot, w.sp_radius, w.sp_weight);
   Tensor index;
   nearest(w.points, w.sp_points, w.K, d2, index);
   require(what, "sp_t", w.sp_t, at::kFloat), require(what, "sp_r", w.sp_r, at::kFloat);
@@ -161,6 +163,7 @@ struct Warp : public torch::autograd::Function<Warp> {
 variable_list apply_forward(const Tensor& points, const Tensor& d_xyz, const Tensor& scales, const Tensor& d_scale,
                             const Tensor& rotations, const Tensor& d_rotation, bool log_scales) {
   const char* what = "deform_apply_forward";
+  refuse_duals("deform_apply", points, d_xyz, scales, d_scale, rotations, d_rotation);
   require(what, "points", points, at::kFloat), require(what, "d_xyz", d_xyz, at::kFloat);
   require(what, "scales", scales, at::kFloat), require(what, "d_scale", d_scale, at::kFloat);
   require(what, "rotations", rotations, at::kFloat), require(what, "d_rotation", d_rotation, at::kFloat);
@@ -374,6 +377,8 @@ variable_list deform_apply(const Tensor& points, const Tensor& d_xyz, const Tens
 }
 
 variable_list deform_mlp(const DeformMlp& m, const std::vector<Tensor>& params) {
+  refuse_duals("DeformNetwork", m.x, m.t, m.in);
+  for (const Tensor& p : params) refuse_duals("DeformNetwork", p);
   bool train = false;
   for (const Tensor& p : params) train = train || p.requires_grad();
   if (train && at::GradMode::is_enabled()) return Mlp::apply(at::TensorList(params), &m);
@@ -411,6 +416,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> mlp_pack(const std::vector<Tensor>& p
 }
 
 std::tuple<Tensor, Tensor> image_loss(const Tensor& img, const Tensor& target, double C1, double C2, double lambda_dssim) {
+  refuse_duals("image_loss", img, target);
   if (at::GradMode::is_enabled() && target.requires_grad()) fail("image_loss: differentiable in its first image only");
   const bool train = at::GradMode::is_enabled() && img.requires_grad();
   const variable_list out = Loss::apply(img.contiguous(), target.contiguous(), C1, C2, lambda_dssim, train);

@@ -26,6 +26,8 @@ struct Buffers {
 
 Buffers forward_view(const FastSurfelView& v, bool train) {
   const char* what = "gs_2d_fast_preprocess_forward";
+  refuse_duals("GS_2D_fast_render", v.points, v.scales, v.rotations, v.opacities, v.shs, v.sh_rest, v.means2D, v.Tw2v, v.Tv2c,
+               v.Tv2s, v.campos, v.trans_mat_t2, v.accum_weights_p);
   require(what, "means3D", v.points, at::kFloat), require(what, "scales", v.scales, at::kFloat);
   require(what, "rotations", v.rotations, at::kFloat), require(what, "opacities", v.opacities, at::kFloat);
   require(what, "shs", v.shs, at::kFloat), require(what, "Tw2v", v.Tw2v, at::kFloat);

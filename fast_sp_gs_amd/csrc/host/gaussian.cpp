@@ -22,6 +22,8 @@ struct Buffers {
 
 Buffers forward_view(const GaussianView& v, bool train) {
   const char* what = "gs_preprocess_forward";
+  refuse_duals("RasterizeGaussians", v.points, v.scales, v.rotations, v.opacities, v.shs, v.sh_rest, v.cov3D, v.cov2D, v.means2D,
+               v.extras, v.Tw2v, v.Tv2c, v.campos, v.accum_weights_p);
   require(what, "means3D", v.points, at::kFloat), require(what, "scales", v.scales, at::kFloat);
   require(what, "rotations", v.rotations, at::kFloat), require(what, "opacities", v.opacities, at::kFloat);
   require(what, "shs", v.shs, at::kFloat), require(what, "Tw2v", v.Tw2v, at::kFloat);

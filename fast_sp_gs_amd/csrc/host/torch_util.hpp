@@ -43,6 +43,14 @@ void require_shape(const char* what, const char* name, const Tensor& t, at::IntA
 inline bool has(const OptTensor& t) { return t.has_value() && t->defined(); }
 inline Tensor opt(const OptTensor& t) { return has(t) ? *t : Tensor(); }
 
+// Forward-mode derivatives are not implemented; a dual tensor would lose its tangent on the way through a kernel.
+inline bool is_dual(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
+inline bool is_dual(const OptTensor& t) { return has(t) && is_dual(*t); }
+template <typename... T>
+void refuse_duals(const char* what, const T&... t) {
+  if ((is_dual(t) || ...)) fail(std::string(what) + ": forward-mode differentiation is not implemented");
+}
+
 // Stored SH coefficients per point beside the split-off first one: checks [P,M,3] (or [P,1,3] + [P,M,3], or colours [P,3]
 // for degree < 0) and returns M.
 int sh_coefficients(const char* what, const Tensor& shs, const OptTensor& sh_rest, int sh_degree, int64_t P);

@@ -152,7 +152,7 @@ def GS_2D_render(points: Tensor, scales: Tensor, rotations: Tensor, opacity: Ten
     maps, n_contrib, radii, visible, tile_range, point_list, normal_opacity, trans_mat = host.surfel_render(
         points, scales, rotations, opacity, sh_features if colors is None else colors, sh_features_rest, means2D,
         Tw2v.contiguous(), Tv2c.contiguous(), campos.contiguous(),
-        background.detach().reshape(3).contiguous() if fused and background is not None else None, trans_mat_t2, culling,
+        background.reshape(3).contiguous() if fused and background is not None else None, trans_mat_t2, culling,
         accum_max_count, accum_weights_p, accum_weights_count, W, H, int(sh_degree) if colors is None else -1, near, far,
         depth_ratio, fused, bool(CULL_LISTS))
     buffer = RasterizeBuffer(W, H, points.shape[0], point_list.shape[0], near, far, tile_range, point_list, n_contrib,

@@ -1,4 +1,5 @@
-"""The native host layer's autograd nodes where autograd does more than one backward: a recorded backward."""
+"""The native host layer's autograd nodes beyond one backward: recorded backwards, forward mode."""
+import dataclasses
 import math
 
 import pytest
@@ -81,3 +82,28 @@ def test_recorded_backward(which, device):
     assert (recorded - plain).norm() <= 1e-4 * plain.norm() and recorded.requires_grad
     with pytest.raises(RuntimeError, match='differentiate twice'):
         torch.autograd.grad((recorded ** 2).sum(), [x])
+
+
+@pytest.mark.parametrize('grad', [False, True])
+@pytest.mark.parametrize('which', NODES + ['camera', 'background', 'positions', 'target'])
+def test_forward_mode_is_refused(which, grad, device):
+    """A dual tensor raises whether or not gradients are recorded, as an input of the node and as one beside it."""
+    from fast_sp_gs_amd.deform import DeformNetwork
+    from fast_sp_gs_amd.ssim import l1_dssim_loss
+    scene, cam, g = _scene(device)
+    if which == 'camera':
+        f, x = lambda x: _surfel(scene.means3D, scene, dataclasses.replace(cam, Tw2v=x)), cam.Tw2v
+    elif which == 'background':
+        f, x = lambda x: _surfel(scene.means3D, scene, cam, background=x), torch.ones(3, device=device)
+    elif which == 'positions':
+        net = DeformNetwork().to(device)
+        f, x = lambda x: net(x, torch.full((1,), 0.3, device=device)), torch.randn(M, 3, generator=g).to(device)
+    elif which == 'target':
+        image = torch.rand(3, H, W, generator=g).to(device)
+        f, x = lambda x: l1_dssim_loss(image, x), torch.rand(3, H, W, generator=g).to(device)
+    else:
+        f, x = _node(which, device)
+    with torch.set_grad_enabled(grad), torch.autograd.forward_ad.dual_level():
+        x = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(RuntimeError, match='forward-mode'):
+            f(x)
