@@ -40,19 +40,17 @@ void require_shape(const char* what, const char* name, const Tensor& t, at::IntA
 
 int sh_coefficients(const char* what, const Tensor& shs, const OptTensor& sh_rest, int sh_degree, int64_t P) {
   const int64_t need = (int64_t) (1 + sh_degree) * (1 + sh_degree);
-  if (has(sh_rest) && sh_rest->numel() > 0) {
-    require(what, "sh_rest", *sh_rest, at::kFloat);
-    const auto s = sh_rest->sizes();
-    if (!(s.size() == 3 && s[0] == P && s[1] >= need - 1 && s[2] == 3)) fail("Error shape for sh features");
-    return (int) s[1];
+  const bool rest = has(sh_rest) && sh_rest->numel() > 0;
+  const Tensor& table = rest ? *sh_rest : shs;
+  if (rest) require(what, "sh_rest", table, at::kFloat);
+  if (rest || sh_degree >= 0) {
+    const auto s = table.sizes();
+    if (!(s.size() == 3 && s[0] == P && s[1] >= need - (rest ? 1 : 0) && s[2] == 3)) fail("Error shape for sh features");
   }
-  if (sh_degree < 0) {
-    require_shape(what, "shs", shs, {P, 3});
-    return 0;
-  }
-  const auto s = shs.sizes();
-  if (!(s.size() == 3 && s[0] == P && s[1] >= need && s[2] == 3)) fail("Error shape for sh features");
-  return (int) s[1];
+  // what is read of shs itself: the colours, the first coefficients beside sh_rest, or the table above
+  if (sh_degree < 0) require_shape(what, "shs", shs, {P, 3});
+  else if (rest && shs.numel() < 3 * P) fail("Error shape for sh features");
+  return table.dim() == 3 ? (int) table.size(1) : 0;
 }
 
 void require_point_mask(const char* what, const OptTensor& culling, int64_t P) {

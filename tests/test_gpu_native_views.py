@@ -238,3 +238,34 @@ def test_gaussian_view_with_given_covariance(given, split, table, device):
         assert scales.grad is None and rot.grad is None
         for t in wanted:
             t.grad = None
+
+
+@pytest.mark.parametrize('split', [False, True])
+@pytest.mark.parametrize('view', ['surfel', 'fast_surfel', 'gaussian'])
+def test_colours_of_a_wrong_shape_are_refused(view, split, device):
+    """On the host, before anything is launched: pre-computed colours beside a table of further coefficients or not, and
+    fewer first coefficients than points beside such a table."""
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    from fast_sp_gs_amd.renderer.gaussian_render import render
+    from fast_sp_gs_amd.renderer.gs_2d_fast_render import GS_2D_fast_render
+    P, W, H = 300, 49, 31
+    s, cam_h, _ = _scene(P, W, H, 7)
+    s, cam = s.to(device), cam_h.to(device)
+    rest = s.shs[:, 1:].contiguous() if split else None
+
+    def picture(**kw):
+        kw.update(campos=cam.campos, sh_degree=3, sh_features_rest=rest)
+        if view == 'gaussian':
+            scales = torch.cat([s.scales, s.scales[:, :1]], dim=1)
+            return render(cam.Tw2v, cam.Tv2c, (W, H), s.means3D, s.opacities, scales, s.rotations, FoV=(0.8, 0.6), **kw)
+        args = (s.means3D, s.scales, s.rotations, s.opacities, (W, H), cam.Tw2v, cam.Tv2c)
+        return GS_2D_render(*args, **kw) if view == 'surfel' else GS_2D_fast_render(*args, cam.Tv2s, **kw)
+
+    for shape in ((P - 1, 3), (P + 1, 3), (P, 4), (P, 1, 3), (3 * P,)):
+        with pytest.raises(RuntimeError, match='shs must have shape'):
+            picture(colors=torch.zeros(shape, device=device))
+    if split:
+        with pytest.raises(RuntimeError, match='Error shape for sh features'):
+            picture(sh_features=s.shs[1:, :1].contiguous())
+        assert torch.isfinite(picture(sh_features=s.shs[:, :1].contiguous())['images']).all()
+    assert torch.isfinite(picture(colors=torch.zeros(P, 3, device=device))['images']).all()
