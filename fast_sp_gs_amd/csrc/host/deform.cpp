@@ -3,6 +3,8 @@
 // iteration spent 1.2 ms of host time on a dozen autograd nodes and the two optimisers, more than the GPU needs for it.
 #include "deform.hpp"
 
+#include <climits>
+
 namespace fsgs_host {
 namespace {
 
@@ -56,6 +58,12 @@ struct Nearest : public torch::autograd::Function<Nearest> {
   }
 };
 
+// The kernels take a table [M,C] whose rows are whole and lie one behind the other, with a stride between them.
+int row_stride(const Tensor& t) { return (int) (t.size(0) > 1 ? t.stride(0) : t.size(1)); }
+bool rows_of_floats(const Tensor& t) {
+  return (t.size(1) <= 1 || t.stride(1) == 1) && (t.size(0) <= 1 || (t.stride(0) >= t.size(1) && t.stride(0) <= INT_MAX));
+}
+
 variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   const char* what = "lbs_blend";
   refuse_duals("superpoint_deform", w.sp_t, w.sp_r, w.sp_s, w.sp_rot, w.sp_radius, w.sp_weight);
@@ -70,10 +78,10 @@ variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   int S = 0, ld = 0;
   if (has(w.sp_s)) {
     const Tensor& s = *w.sp_s;
-    if (!s.is_cuda() || s.scalar_type() != at::kFloat || s.dim() != 2 || s.size(0) != M || s.stride(1) != 1 ||
+    if (!s.is_cuda() || s.scalar_type() != at::kFloat || s.dim() != 2 || s.size(0) != M || !rows_of_floats(s) ||
         s.size(1) < w.scale_columns)
       fail("lbs_blend: sp_s must be a float32 CUDA tensor [M,S]");
-    S = w.scale_columns, ld = M > 1 ? (int) s.stride(0) : (int) s.size(1);
+    S = w.scale_columns, ld = row_stride(s);
   }
   Tensor d_xyz = empty({N, 3}, w.points), d_rot = empty({N, 4}, w.points), d_scale, weights = empty({N, K}, w.points);
   if (S) d_scale = empty({N, S}, w.points);
@@ -133,7 +141,7 @@ struct Warp : public torch::autograd::Function<Warp> {
     if (m.weight_mode == 1) g_radius = at::empty_like(radius), g_weight = weight.defined() ? at::empty_like(weight) : Tensor();
     const size_t bytes = fsgs_lbs_blend_backward_workspace_bytes((int) N, (int) M, S);
     const Tensor ws = byte_buffer(bytes, points);
-    const int ld = S ? (M > 1 ? (int) sp_s.stride(0) : (int) sp_s.size(1)) : 0;
+    const int ld = S ? row_stride(sp_s) : 0;
     auto pick = [&](size_t k, const Tensor& x) { return ctx->needs_input_grad(k) ? x : Tensor(); };
     if (fsgs_superpoint_backward_is_fused((int) M, (int) K, m.warp_mode, m.weight_mode, S)) {
       check(fsgs_superpoint_backward((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
@@ -356,7 +364,7 @@ variable_list superpoint_warp(const SuperpointWarp& given) {
   w.sp_t = w.sp_t.contiguous(), w.sp_r = w.sp_r.contiguous();
   auto whole = [](OptTensor& t) { if (has(t)) t = t->contiguous(); };
   whole(w.sp_rot), whole(w.sp_radius), whole(w.sp_weight);
-  if (has(w.sp_s) && w.sp_s->dim() == 2 && w.sp_s->stride(1) != 1) w.sp_s = w.sp_s->contiguous();
+  if (has(w.sp_s) && w.sp_s->dim() == 2 && !rows_of_floats(*w.sp_s)) w.sp_s = w.sp_s->contiguous();
   const bool train = at::GradMode::is_enabled() &&
                      (w.sp_points.requires_grad() || w.sp_t.requires_grad() || w.sp_r.requires_grad() || wants(w.sp_s) ||
                       wants(w.sp_rot) || wants(w.sp_radius) || wants(w.sp_weight));

@@ -116,3 +116,23 @@ def test_dense_adam_state_goes_on_in_torch(change, device):
         step(a, b)
     for p, q in zip(mine, theirs):
         assert float(a.state[p]['step']) == 5 and torch.allclose(p, q, rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize('M', [1, 40])
+@pytest.mark.parametrize('layout', ['broadcast', 'transposed', 'column', 'one_column', 'overlapping', 'slice'])
+def test_scale_table_of_any_layout(layout, M, device):
+    from fast_sp_gs_amd.deform import superpoint_deform
+    g = torch.Generator().manual_seed(M)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(device)
+    points, controls, sp_t, sp_r, up = r(100, 3), r(M, 3), r(M, 3), r(M, 4), r(100, 2)
+    base, view = {'broadcast': (r(1, 2), lambda t: t.expand(M, 2)), 'transposed': (r(2, M), lambda t: t.t()),
+                  'column': (r(3, M), lambda t: t.t()[:, :1]), 'one_column': (r(M, 3), lambda t: t[:, 1:2]),
+                  'overlapping': (r(M + 1), lambda t: t.as_strided((M, 2), (1, 1))),
+                  'slice': (r(M, 5), lambda t: t[:, 2:4])}[layout]
+    results = []
+    for table in (view, lambda t: view(t).clone(memory_format=torch.contiguous_format)):
+        leaf = base.clone().requires_grad_(True)
+        out = superpoint_deform(points, controls, sp_t, sp_r, table(leaf), K=min(3, M))[2]
+        results.append((out, *torch.autograd.grad((out * up[:, :out.shape[1]]).sum(), [leaf])))
+    assert torch.equal(results[0][0], results[1][0])
+    assert torch.allclose(results[0][1], results[1][1], rtol=1e-6, atol=1e-6)
