@@ -125,7 +125,7 @@ variable_list outputs_of(const GaussianView& v, const Buffers& b) {
   Tensor screen;
   {
     at::AutoDispatchBelowADInplaceOrView plain;  // shares the leaf's storage, no view in the graph's sense
-    screen = at::alias(v.means2D);
+    screen = sharing_edits(v.means2D, at::alias(v.means2D));
   }
   variable_list out = {b.image, b.opacity, screen, b.conic_opacity};
   if (b.extras.defined()) out.push_back(b.extras);

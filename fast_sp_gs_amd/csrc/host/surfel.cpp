@@ -147,7 +147,7 @@ variable_list outputs_of(const Buffers& b) {
   Tensor distortion;
   {
     at::AutoDispatchBelowADInplaceOrView plain;  // shares extras' storage, no view in the graph's sense
-    distortion = b.extras.narrow(0, 5, 1);
+    distortion = sharing_edits(b.extras, b.extras.narrow(0, 5, 1));
   }
   out = {b.composited.defined() ? b.composited : b.image, b.opacity, b.normals, b.depths, b.surf_depth, b.surf_normal,
          distortion};

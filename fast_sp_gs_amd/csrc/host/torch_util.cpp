@@ -71,6 +71,12 @@ void require_accumulators(const char* what, const OptTensor& max_count, const Op
   one("accum_weights_p", weights_p, at::kFloat);
 }
 
+Tensor sharing_edits(const Tensor& whole, Tensor part) {
+  namespace impl = torch::autograd::impl;
+  impl::set_version_counter(part, impl::version_counter(whole));
+  return part;
+}
+
 variable_list first_order_only(const variable_list& upstream, const variable_list& inputs, variable_list grads) {
   bool recorded = false;
   if (at::GradMode::is_enabled())

@@ -71,6 +71,10 @@ inline Tensor empty(at::IntArrayRef shape, const Tensor& like, at::ScalarType ty
 }
 inline Tensor contiguous(const Tensor& t) { return t.defined() ? t.contiguous() : t; }
 
+// `part`, a tensor over some of `whole`'s storage made outside the graph, as an output of its own that counts edits with
+// `whole`: the backward reads that storage, and an in-place edit of either has to be noticed there.
+Tensor sharing_edits(const Tensor& whole, Tensor part);
+
 // A node's gradients come from kernels, outside the graph. Where the backward itself is recorded (create_graph=True) they
 // get a node that raises when it is differentiated, reached from what they depend on (the upstream gradients and the saved
 // inputs); without it they would pass for constants.

@@ -14,7 +14,7 @@ NODES = ['surfel', 'fast_surfel', 'gaussian', 'deform_apply', 'knn', 'warp', 'ne
 def _scene(device):
     from fast_sp_gs_amd import scenes
     g = torch.Generator().manual_seed(7)
-    s = scenes._surfels(g, P, 'cube', -4.2, 0.7, 0.0, 1.5).to(device)
+    s = scenes._surfels(g, P, 'cube', -2.5, 0.7, 0.0, 1.5).to(device)
     return s, scenes.pinhole(W, H, 50.0, torch.tensor([0.3, 0.2, 4.0])).to(device), g
 
 
@@ -79,7 +79,7 @@ def test_recorded_backward(which, device):
     plain, = torch.autograd.grad((f(x) ** 2).sum(), [x])
     recorded, = torch.autograd.grad((f(x) ** 2).sum(), [x], create_graph=True)
     # device atomics add a point's tiles in another order
-    assert (recorded - plain).norm() <= 1e-4 * plain.norm() and recorded.requires_grad
+    assert plain.norm() > 0 and (recorded - plain).norm() <= 1e-4 * plain.norm() and recorded.requires_grad
     with pytest.raises(RuntimeError, match='differentiate twice'):
         torch.autograd.grad((recorded ** 2).sum(), [x])
 
@@ -107,3 +107,26 @@ def test_forward_mode_is_refused(which, grad, device):
         x = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
         with pytest.raises(RuntimeError, match='forward-mode'):
             f(x)
+
+
+@pytest.mark.parametrize('which,name', [('surfel', 'distortion'), ('fast_surfel', 'distortion'), ('gaussian', 'means2D'),
+                                        ('surfel', 'opacity'), ('gaussian', 'conic_opacity')])
+def test_edited_output_is_noticed(which, name, device):
+    """Outputs that share their storage with what the backward reads: an edit in place raises there; without one the
+    gradients are there, under inference mode the picture is."""
+    scene, cam, _ = _scene(device)
+    view = {'surfel': _surfel, 'fast_surfel': _fast_surfel, 'gaussian': _gaussian}[which]
+    points = scene.means3D.clone().requires_grad_(True)
+    for edited in (False, True):
+        out = view(points, scene, cam)
+        shared = out[name] if name in out else getattr(out['buffer'], name)
+        if edited:
+            with torch.no_grad():
+                shared.add_(0.5)
+            with pytest.raises(RuntimeError, match='inplace operation'):
+                out['images'].sum().backward()
+        else:
+            out['images'].sum().backward()
+            assert points.grad.abs().sum() > 0
+    with torch.inference_mode():
+        assert torch.equal(view(scene.means3D, scene, cam)['images'], view(points, scene, cam)['images'])
