@@ -68,11 +68,7 @@ class DynamicStep:
     def step(self, t: Tensor):
         """One full iteration; returns (loss, visibility mask) as device tensors (nothing is copied to the host)."""
         loss, out = self.forward_loss(t)
-        leaves = self.params + list(self.net.parameters()) + [self.ctrl]
-        # straight from the graph to the optimisers: accumulation into .grad would copy what two leaves share
-        for p, g in zip(leaves, torch.autograd.grad(loss, leaves, allow_unused=True)):
-            if g is not None:
-                p.grad = g if p.grad is None else p.grad + g
+        loss.backward()
         visible = out['visibility_filter']
         self.opt.set_before_step(visible, self.params[0].shape[0])
         self.opt.step()

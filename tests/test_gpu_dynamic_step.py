@@ -152,3 +152,18 @@ def test_autograd_edges_against_torch_formulation(warp_method, LBS_method, devic
     # the leaves that reach the loss through the renderer alone
     for name in ('opacities', 'shs'):
         assert got_by_name[name] is not None and float(got_by_name[name].abs().max()) > 0
+
+
+def test_step_runs_hooks_and_reaches_other_leaves(device):
+    """What hangs on a leaf's gradient accumulation (a gradient all-reduce) runs once per leaf and step, and a leaf that
+    belongs to neither optimiser (the time) receives its gradient."""
+    state, _ = _state(device, 2000, 48, 64, 5)
+    leaves = state.params + list(state.net.parameters()) + [state.ctrl]
+    seen = []
+    for k, p in enumerate(leaves):
+        p.register_post_accumulate_grad_hook(lambda p, k=k: seen.append((k, p.grad is not None)))
+    t = torch.full((1,), 0.3, device=device, requires_grad=True)
+    state.step(t)
+    assert sorted(seen) == [(k, True) for k in range(len(leaves))]
+    assert t.grad is not None and float(t.grad.abs()) > 0
+    assert all(p.grad is None for p in leaves)
