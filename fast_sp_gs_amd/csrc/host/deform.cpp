@@ -4,6 +4,7 @@
 #include "deform.hpp"
 
 #include <climits>
+#include <cmath>
 
 namespace fsgs_host {
 namespace {
@@ -480,13 +481,20 @@ void adam_masked(const std::vector<Tensor>& params, const std::vector<Tensor>& g
 }
 
 void adam_dense(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
-                const std::vector<Tensor>& v, const std::vector<double>& step_size, const std::vector<double>& root_c2,
-                double b1, double b2, double eps) {
+                const std::vector<Tensor>& v, const std::vector<Tensor>& steps, double lr, double b1, double b2, double eps) {
   const AdamPointers t("adam_update", params, grads, m, v);
   const size_t n = params.size(), most = (size_t) fsgs_adam_update_max_tensors();
-  if (step_size.size() != n || root_c2.size() != n) fail("adam_update: a step size and a bias correction per parameter tensor");
+  if (steps.size() != n) fail("adam_update: a step count per parameter tensor");
   std::vector<int64_t> count;
-  for (const Tensor& p : params) count.push_back(p.numel());
+  std::vector<double> step_size, root_c2;
+  for (size_t k = 0; k < n; ++k) {
+    const Tensor& step = steps[k];
+    if (step.numel() != 1) fail("adam_update: a step count is one number");
+    const bool plain = step.is_cpu() && step.scalar_type() == at::kFloat;  // as torch keeps it
+    const double taken = plain ? (double) (*step.data_ptr<float>() += 1.0f) : step.add_(1).item<double>();
+    count.push_back(params[k].numel());
+    step_size.push_back(lr / (1 - std::pow(b1, taken))), root_c2.push_back(std::sqrt(1 - std::pow(b2, taken)));
+  }
   for (size_t k = 0; k < n; k += most)
     check(fsgs_adam_update_multi((int) std::min(most, n - k), count.data() + k, step_size.data() + k, root_c2.data() + k, b1, b2,
                                  eps, t.p.data() + k, t.g.data() + k, t.m.data() + k, t.v.data() + k, stream_of(params[0])),

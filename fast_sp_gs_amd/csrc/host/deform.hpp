@@ -40,8 +40,8 @@ std::tuple<Tensor, Tensor> image_loss(const Tensor& img, const Tensor& target, d
 void adam_masked(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
                  const std::vector<Tensor>& v, const Tensor& mask, const std::vector<double>& lr, double b1, double b2,
                  const std::vector<double>& eps, int64_t N);
+// torch.optim.Adam's plain step; `steps` (one count per parameter) are advanced by it
 void adam_dense(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
-                const std::vector<Tensor>& v, const std::vector<double>& step_size, const std::vector<double>& root_c2,
-                double b1, double b2, double eps);
+                const std::vector<Tensor>& v, const std::vector<Tensor>& steps, double lr, double b1, double b2, double eps);
 
 }  // namespace fsgs_host
