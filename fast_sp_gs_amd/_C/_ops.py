@@ -1198,7 +1198,7 @@ def lbs_blend(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Tensor, sp_
     ws = _workspace(lib.fsgs_lbs_blend_workspace_bytes(M), points.device)
     with _timed('lbs_blend'):
         rc = lib.fsgs_lbs_blend(N, M, K, warp, weight, float(temperature), L.ptr(points), L.ptr(sp_points),
-                                L.ptr(sp_t), L.ptr(sp_rot), L.ptr(sp_r), L.ptr(sp_s), S, S, L.ptr(pair_in), L.ptr(index),
+                                L.ptr(sp_t), L.ptr(sp_rot), L.ptr(sp_r), L.ptr(sp_s), S, L.ptr(pair_in), L.ptr(index),
                                 L.ptr(sp_log_radius) if weight == 1 else None,
                                 L.ptr(sp_weight_logit) if weight == 1 else None, L.ptr(weights), L.ptr(d_xyz),
                                 L.ptr(d_rot), L.ptr(d_scale), L.ptr(ws), ws.numel(), L.current_stream())
@@ -1243,10 +1243,10 @@ def lbs_blend_backward(points: Tensor, sp_points: Tensor, sp_t: Tensor, sp_r: Te
     with _timed('lbs_blend_backward'):
         rc = lib.fsgs_lbs_blend_backward(
             N, M, K, warp, weight, float(temperature), L.ptr(points), L.ptr(sp_points), L.ptr(sp_t), L.ptr(sp_rot),
-            L.ptr(sp_r), L.ptr(sp_s), S, S, L.ptr(pair_in), L.ptr(index), L.ptr(sp_log_radius) if weight == 1 else None,
+            L.ptr(sp_r), L.ptr(sp_s), S, L.ptr(pair_in), L.ptr(index), L.ptr(sp_log_radius) if weight == 1 else None,
             L.ptr(sp_weight_logit) if weight == 1 else None, L.ptr(grad_xyz), L.ptr(grad_rot), L.ptr(grad_scale),
             L.ptr(g_points), L.ptr(g_pair), L.ptr(g_sp_points), L.ptr(g_sp_t), L.ptr(g_sp_rot), L.ptr(g_sp_r),
-            L.ptr(g_sp_s), S, L.ptr(g_rad), L.ptr(g_wl), L.ptr(ws), ws.numel(), L.current_stream())
+            L.ptr(g_sp_s), L.ptr(g_rad), L.ptr(g_wl), L.ptr(ws), ws.numel(), L.current_stream())
     L.check(rc, what)
     return dict(g_points=g_points, g_pair=g_pair, g_sp_points=g_sp_points, g_sp_t=g_sp_t, g_sp_rot=g_sp_rot,
                 g_sp_r=g_sp_r, g_sp_s=g_sp_s, g_log_radius=g_rad, g_weight_logit=g_wl)
@@ -1363,9 +1363,11 @@ def mlp_forward(inputs: Tensor, packed: Tensor, bias: Tensor, n_layers: int, ski
         B_pad = _mlp_rows(B)
         saved_in = torch.empty((Din, B_pad), dtype=torch.int16, device=inputs.device)
         saved = torch.empty((n_layers, 256, B_pad), dtype=torch.int16, device=inputs.device)
+    heads, outs = (ctypes.c_int * 1)(n_out), (ctypes.c_void_p * 1)(out.data_ptr())  # all rows as one head
     with _timed('mlp_forward'):
-        rc = lib.fsgs_mlp_forward(B, Din, 256, n_layers, skip, n_out, L.ptr(inputs), L.ptr(packed), L.ptr(bias),
-                                  L.ptr(out), L.ptr(saved_in), L.ptr(saved), L.current_stream())
+        rc = lib.fsgs_deform_mlp_forward(B, Din, 256, n_layers, skip, 1, ctypes.addressof(heads), L.ptr(inputs), None, None,
+                                         0, 1.0, 0, 1.0, L.ptr(packed), L.ptr(bias), ctypes.addressof(outs),
+                                         L.ptr(saved_in), L.ptr(saved), L.current_stream())
     L.check(rc, what)
     # the kernels keep the batch innermost; callers see [n_layers, B, 256]
     return (out, saved[:, :, :B].transpose(1, 2)) if save else out
@@ -1417,11 +1419,12 @@ def mlp_backward(inputs: Tensor, packed_t: Tensor, head_weights: Tensor, saved: 
     g = torch.empty((n_w + n_layers * 256 + n_out,), dtype=torch.float32, device=inputs.device)
     g_w, g_b = g[:n_w], g[n_w:]
     lib = _lib()
-    ws = _workspace(lib.fsgs_mlp_backward_workspace_bytes(B, Din, n_layers), inputs.device)
+    ws = _workspace(lib.fsgs_deform_mlp_backward_workspace_bytes(B, Din, n_layers), inputs.device)
+    heads, ups = (ctypes.c_int * 1)(n_out), (ctypes.c_void_p * 1)(grad_out.data_ptr())
     with _timed('mlp_backward'):
-        rc = lib.fsgs_mlp_backward(B, Din, 256, n_layers, skip, n_out, L.ptr(inputs), L.ptr(packed_t),
-                                   L.ptr(head_weights), L.ptr(saved), L.ptr(grad_out), L.ptr(g_w), L.ptr(g_b),
-                                   L.ptr(ws), ws.numel(), L.current_stream())
+        rc = lib.fsgs_deform_mlp_backward(B, Din, 256, n_layers, skip, 1, ctypes.addressof(heads), L.ptr(inputs), None,
+                                          L.ptr(packed_t), L.ptr(head_weights), L.ptr(saved), ctypes.addressof(ups),
+                                          L.ptr(g_w), L.ptr(g_b), L.ptr(ws), ws.numel(), L.current_stream())
     L.check(rc, what)
     if return_dz:
         dz = ws[:n_layers * B_pad * 256 * 2].view(torch.bfloat16).view(n_layers, 256, B_pad)

@@ -88,7 +88,7 @@ variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   if (S) d_scale = empty({N, S}, w.points);
   const size_t bytes = fsgs_lbs_blend_workspace_bytes((int) M);
   table = byte_buffer(bytes, w.points);
-  check(fsgs_lbs_blend((int) N, (int) M, (int) K, w.warp_mode, w.weight_mode, w.temperature, f32(w.points), f32(w.sp_points),
+  check(fsgs_lbs_blend_strided((int) N, (int) M, (int) K, w.warp_mode, w.weight_mode, w.temperature, f32(w.points), f32(w.sp_points),
                        f32(w.sp_t), f32(opt(w.sp_rot)), f32(w.sp_r), f32(opt(w.sp_s)), S, ld, f32(d2), i64(index),
                        f32(opt(w.sp_radius)), f32(opt(w.sp_weight)), f32(weights), f32(d_xyz), f32(d_rot), f32(d_scale),
                        table.data_ptr(), bytes, stream_of(w.points)),
@@ -154,7 +154,7 @@ struct Warp : public torch::autograd::Function<Warp> {
       return first_order_only(g, inputs, {pick(0, g_c), g_t, g_r, g_s, g_sp_rot, g_radius, g_weight, Tensor()});
     }
     const Tensor g_pair = empty({N, K}, points);
-    check(fsgs_lbs_blend_backward((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
+    check(fsgs_lbs_blend_backward_strided((int) N, (int) M, (int) K, m.warp_mode, m.weight_mode, m.temperature, f32(points),
                                   f32(sp_points), f32(sp_t), f32(sp_rot), f32(sp_r), f32(sp_s), S, ld, f32(d2), i64(index),
                                   f32(radius), f32(weight), f32(g_xyz), f32(g_rot), f32(g_scale), nullptr, f32(g_pair),
                                   f32(g_c), f32(g_t), f32(g_sp_rot), f32(g_r), f32(g_s), S ? (int) sp_s.size(1) : 0,
@@ -283,7 +283,7 @@ struct Mlp : public torch::autograd::Function<Mlp> {
     for (size_t h = 0; h < s.head_rows.size(); ++h) n_out += s.head_rows[h], g[h] = contiguous(g[h]), up.push_back(f32(g[h]));
     const int64_t n_w = 256 * Din + (L - 1) * 65536 + 256 * Din + n_out * 256;
     const Tensor flat = empty({n_w + L * 256 + n_out}, t[3]);
-    const size_t bytes = fsgs_mlp_backward_workspace_bytes((int) B, (int) Din, (int) L);
+    const size_t bytes = fsgs_deform_mlp_backward_workspace_bytes((int) B, (int) Din, (int) L);
     const Tensor ws = byte_buffer(bytes, t[3]);
     check(fsgs_deform_mlp_backward((int) B, (int) Din, 256, (int) L, s.skip, (int) s.head_rows.size(), s.head_rows.data(),
                                    nullptr, data<uint16_t>(t[0]), data<uint16_t>(t[2]), f32(t[3]), data<uint16_t>(t[1]),

@@ -526,7 +526,7 @@ int lbs_backward(int N, int M, int K, int warp_mode, int weight_mode, double tem
 }
 }  // namespace
 
-FSGS_API int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
+FSGS_API int fsgs_lbs_blend_backward_strided(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
     const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
     const float* sp_s, int S, int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius,
     const float* sp_weight_logit, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_points,
@@ -536,6 +536,18 @@ FSGS_API int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int wei
                       pair_in, index, sp_log_radius, sp_weight_logit, g_xyz, g_rot, g_scale, g_points, g_pair, g_sp_points,
                       g_sp_t, g_sp_rot, g_sp_r, g_sp_s, g_sp_s_ld, g_log_radius, g_weight_logit, nullptr, false, workspace,
                       workspace_bytes, stream);
+}
+
+FSGS_API int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
+    const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
+    const float* sp_s, int S, const float* pair_in, const int64_t* index, const float* sp_log_radius,
+    const float* sp_weight_logit, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_points,
+    float* g_pair, float* g_sp_points, float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s,
+    float* g_log_radius, float* g_weight_logit, void* workspace, size_t workspace_bytes, void* stream) {
+  return fsgs_lbs_blend_backward_strided(N, M, K, warp_mode, weight_mode, temperature, points, sp_points, sp_t, sp_rot, sp_r,
+                                         sp_s, S, S, pair_in, index, sp_log_radius, sp_weight_logit, g_xyz, g_rot, g_scale,
+                                         g_points, g_pair, g_sp_points, g_sp_t, g_sp_rot, g_sp_r, g_sp_s, S, g_log_radius,
+                                         g_weight_logit, workspace, workspace_bytes, stream);
 }
 
 FSGS_API int fsgs_superpoint_backward_is_fused(int M, int K, int warp_mode, int weight_mode, int S) {

@@ -190,8 +190,11 @@ __device__ __forceinline__ void load_fragments(const uint16_t* __restrict__ tile
 }
 
 // D layout of the 16x16 accumulator: register r of lane l holds row 4 * (l / 16) + r, column l % 16.
-// `in` or `freq.x` gives the input rows. in_t / saved (kSave): see the file's head.
-template <bool kSave>
+// What the forward stores of the hidden states: nothing; them and the input rows batch innermost (see the file's head); or
+// the states alone as rows, [layer][B][256], the form that fsgs_mlp_forward's callers keep.
+enum class Keep { kNothing, kBatchInnermost, kRows };
+// `in` or `freq.x` gives the input rows; in_t goes with kBatchInnermost.
+template <Keep kKeep>
 __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int Din, int n_layers, int skip, int n_out,
     const float* __restrict__ in, FreqInput freq, const uint16_t* __restrict__ packed, const float* __restrict__ bias,
     MlpHeads heads, uint16_t* __restrict__ in_t, uint16_t* __restrict__ saved, int row_blocks, size_t packed_elems) {
@@ -232,7 +235,7 @@ __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int D
     s_act[0][r][k] = h;
   }
   __syncthreads();
-  if (kSave) {
+  if (kKeep == Keep::kBatchInnermost) {
     for (int e = threadIdx.x; e < Din * (kMlpRows / 4); e += kChainThreads) {
       const int k = e >> 2, r = (e & 3) * 4;
       const uint16_t h[4] = {s_in[r][k], s_in[r + 1][k], s_in[r + 2][k], s_in[r + 3][k]};
@@ -292,7 +295,16 @@ __global__ void __launch_bounds__(kChainThreads) mlp_forward_kernel(int B, int D
       uint16_t* row = to + 16 * t;
       row[0] = (uint16_t) h.x, row[kMlpStride] = (uint16_t) (h.x >> 16);
       row[2 * kMlpStride] = (uint16_t) h.y, row[3 * kMlpStride] = (uint16_t) (h.y >> 16);
-      if (kSave) *(uint2*) (saved + ((size_t) layer * kMlpWidth + col + 16 * t) * B_pad + row0 + 4 * (lane >> 4)) = h;
+      if (kKeep == Keep::kBatchInnermost)
+        *(uint2*) (saved + ((size_t) layer * kMlpWidth + col + 16 * t) * B_pad + row0 + 4 * (lane >> 4)) = h;
+      if (kKeep == Keep::kRows) {
+        const uint16_t state[4] = {(uint16_t) h.x, (uint16_t) (h.x >> 16), (uint16_t) h.y, (uint16_t) (h.y >> 16)};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int r = row0 + 4 * (lane >> 4) + k;
+          if (r < B) saved[((size_t) layer * B + r) * kMlpWidth + col + 16 * t] = state[k];
+        }
+      }
     }
     if (layer == skip) {
       for (int e = threadIdx.x; e < kMlpRows * kInPad; e += kChainThreads) {
@@ -555,6 +567,25 @@ __global__ void __launch_bounds__(kMlpThreads) mlp_backward_weights_kernel(int B
   }
 }
 
+// Hidden states or their gradients between the callers' rows [layer][B][256] and the kernels' [layer][256][B_pad] (zeros
+// past the batch), 32 x 32 through LDS: grid (B_pad / 32, 8, layers).
+template <bool kToRows>
+__global__ void __launch_bounds__(256) mlp_transpose_kernel(int B, int B_pad, const uint16_t* __restrict__ from,
+                                                            uint16_t* __restrict__ to) {
+  __shared__ uint16_t s_tile[32][33];
+  const int x = threadIdx.x & 31, r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
+  const size_t rows = (size_t) blockIdx.z * B, columns = (size_t) blockIdx.z * kMlpWidth;
+  for (int y = threadIdx.x >> 5; y < 32; y += 8) {
+    if (kToRows) s_tile[y][x] = from[(columns + c0 + y) * B_pad + r0 + x];
+    else s_tile[y][x] = r0 + y < B ? from[(rows + r0 + y) * kMlpWidth + c0 + x] : (uint16_t) 0;
+  }
+  __syncthreads();
+  for (int y = threadIdx.x >> 5; y < 32; y += 8) {
+    if (!kToRows) to[(columns + c0 + y) * B_pad + r0 + x] = s_tile[x][y];
+    else if (r0 + y < B) to[(rows + r0 + y) * kMlpWidth + c0 + x] = s_tile[x][y];
+  }
+}
+
 }  // namespace
 }  // namespace fsgs
 
@@ -646,15 +677,15 @@ bool make_heads(MlpHeads& h, int n_heads, const int* head_rows, float* const* at
 FSGS_API size_t fsgs_mlp_saved_elems(int B, int n_layers) { return (size_t) n_layers * kMlpWidth * padded_rows(B); }
 FSGS_API size_t fsgs_mlp_saved_input_elems(int B, int Din) { return (size_t) Din * padded_rows(B); }
 
-FSGS_API int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
-    const float* in, const float* x, const float* t, int degree_x, double scale_x, int degree_t, double scale_t,
-    const uint16_t* packed, const float* bias, float* const* outs, uint16_t* saved_in, uint16_t* saved, void* stream) {
-  FSGS_REQUIRE(B >= 0 && (in || (x && t)) && packed && bias && head_rows && outs, "mlp_forward: bad arguments");
-  FSGS_REQUIRE(in || (degree_x >= 0 && degree_t >= 0 && Din == 3 * (1 + 2 * degree_x) + 1 + 2 * degree_t),
+namespace {
+int launch_forward(Keep keep, int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
+    const float* in, const FreqInput& freq, const uint16_t* packed, const float* bias, float* const* outs, uint16_t* saved_in,
+    uint16_t* saved, void* stream) {
+  FSGS_REQUIRE(B >= 0 && (in || (freq.x && freq.t)) && packed && bias && head_rows && outs, "mlp_forward: bad arguments");
+  FSGS_REQUIRE(in || (freq.degree_x >= 0 && freq.degree_t >= 0 && Din == 3 * (1 + 2 * freq.degree_x) + 1 + 2 * freq.degree_t),
                "mlp_forward: the encoding has another width than the network's input");
   FSGS_REQUIRE(width == kMlpWidth, "mlp_forward: width %d is not supported (only %d)", width, kMlpWidth);
   FSGS_REQUIRE(Din > 0 && ((Din + 15) & ~15) <= kMlpMaxIn, "mlp_forward: input width %d exceeds %d", Din, kMlpMaxIn);
-  FSGS_REQUIRE((saved == nullptr) == (saved_in == nullptr), "mlp_forward: saved_in and saved go together");
   MlpHeads heads{};
   FSGS_REQUIRE(make_heads(heads, n_heads, head_rows, outs), "mlp_forward: bad heads (at most %d with 32 rows)", kMaxHeads);
   for (int h = 0; h < n_heads; ++h) FSGS_REQUIRE(outs[h], "mlp_forward: null output");
@@ -662,16 +693,27 @@ FSGS_API int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, in
   FSGS_REQUIRE(n_layers >= 1 && skip < n_layers - 1, "mlp_forward: bad layer structure (layers %d, skip %d, outputs %d)",
                n_layers, skip, n_out);
   if (B == 0) return kOk;
-  const FreqInput freq{x, t, degree_x, degree_t, (float) scale_x, (float) scale_t};
-  auto kernel = saved ? mlp_forward_kernel<true> : mlp_forward_kernel<false>;
+  auto kernel = keep == Keep::kNothing ? mlp_forward_kernel<Keep::kNothing>
+                : keep == Keep::kRows  ? mlp_forward_kernel<Keep::kRows>
+                                       : mlp_forward_kernel<Keep::kBatchInnermost>;
   const int row_blocks = (int) (padded_rows(B) / kMlpRows);
   hipLaunchKernelGGL(kernel, dim3(row_blocks + (row_blocks < kFetchBelow ? kFetchBlocks : 0)), dim3(kChainThreads), 0,
                      (hipStream_t) stream, B, Din, n_layers, skip, n_out, in, freq, packed, bias, heads, saved_in, saved,
                      row_blocks, fsgs_mlp_packed_elems(Din, n_layers, skip));
   return check_launch("mlp_forward");
 }
+}  // namespace
 
-FSGS_API size_t fsgs_mlp_backward_workspace_bytes(int B, int Din, int n_layers) {
+FSGS_API int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
+    const float* in, const float* x, const float* t, int degree_x, double scale_x, int degree_t, double scale_t,
+    const uint16_t* packed, const float* bias, float* const* outs, uint16_t* saved_in, uint16_t* saved, void* stream) {
+  FSGS_REQUIRE((saved == nullptr) == (saved_in == nullptr), "mlp_forward: saved_in and saved go together");
+  return launch_forward(saved ? Keep::kBatchInnermost : Keep::kNothing, B, Din, width, n_layers, skip, n_heads, head_rows, in,
+                        FreqInput{x, t, degree_x, degree_t, (float) scale_x, (float) scale_t}, packed, bias, outs, saved_in,
+                        saved, stream);
+}
+
+FSGS_API size_t fsgs_deform_mlp_backward_workspace_bytes(int B, int Din, int n_layers) {
   if (B < 0 || n_layers < 1 || Din < 1) return 0;
   return align_up(((size_t) n_layers * kMlpWidth + 32 + Din) * padded_rows(B) * sizeof(uint16_t), 256);
 }
@@ -688,9 +730,9 @@ FSGS_API int fsgs_deform_mlp_backward(int B, int Din, int width, int n_layers, i
   const int n_out = heads.first[n_heads];
   FSGS_REQUIRE(n_layers >= 1 && n_layers <= 64 && skip < n_layers - 1,
                "mlp_backward: bad layer structure (layers %d, skip %d, outputs %d)", n_layers, skip, n_out);
-  if (workspace_bytes < fsgs_mlp_backward_workspace_bytes(B, Din, n_layers))
+  if (workspace_bytes < fsgs_deform_mlp_backward_workspace_bytes(B, Din, n_layers))
     return fail(kWorkspaceSmall, "mlp_backward: workspace %zu < %zu bytes", workspace_bytes,
-                fsgs_mlp_backward_workspace_bytes(B, Din, n_layers));
+                fsgs_deform_mlp_backward_workspace_bytes(B, Din, n_layers));
   hipStream_t s = (hipStream_t) stream;
   const size_t B_pad = padded_rows(B);
   uint16_t* dz   = (uint16_t*) workspace;
@@ -717,17 +759,46 @@ FSGS_API int fsgs_deform_mlp_backward(int B, int Din, int width, int n_layers, i
   return check_launch("mlp_backward");
 }
 
+// The entry points whose callers keep the states as rows. The backward lays them out for the kernels and its result dZ back.
 FSGS_API int fsgs_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
-                              const uint16_t* packed, const float* bias, float* out, uint16_t* saved_in, uint16_t* saved,
-                              void* stream) {
-  return fsgs_deform_mlp_forward(B, Din, width, n_layers, skip, 1, &n_out, in, nullptr, nullptr, 0, 1.0, 0, 1.0, packed, bias,
-                                 &out, saved_in, saved, stream);
+                              const uint16_t* packed, const float* bias, float* out, uint16_t* saved, void* stream) {
+  FSGS_REQUIRE(in && out, "mlp_forward: bad arguments");
+  return launch_forward(saved ? Keep::kRows : Keep::kNothing, B, Din, width, n_layers, skip, 1, &n_out, in, FreqInput{}, packed,
+                        bias, &out, nullptr, saved, stream);
+}
+
+namespace {
+struct RowsWorkspace {  // dZ as rows | the states batch innermost | the kernels' own, dZ batch innermost in front
+  size_t states, own, bytes;
+  RowsWorkspace(int B, int n_layers) {
+    states = align_up((size_t) n_layers * std::max(B, 1) * kMlpWidth * sizeof(uint16_t), 256);
+    own    = states + align_up(fsgs_mlp_saved_elems(B, n_layers) * sizeof(uint16_t), 256);
+    bytes  = own + fsgs_deform_mlp_backward_workspace_bytes(B, kMlpMaxIn, n_layers);
+  }
+};
+}  // namespace
+
+FSGS_API size_t fsgs_mlp_backward_workspace_bytes(int B, int n_layers) {
+  return B < 0 || n_layers < 1 ? 0 : RowsWorkspace(B, n_layers).bytes;
 }
 
 FSGS_API int fsgs_mlp_backward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
     const uint16_t* packed_t, const float* heads_w, const uint16_t* saved, const float* g_out, float* g_w, float* g_b,
     void* workspace, size_t workspace_bytes, void* stream) {
-  FSGS_REQUIRE(g_out, "mlp_backward: bad arguments");
-  return fsgs_deform_mlp_backward(B, Din, width, n_layers, skip, 1, &n_out, in, nullptr, packed_t, heads_w, saved, &g_out,
-                                  g_w, g_b, workspace, workspace_bytes, stream);
+  FSGS_REQUIRE(B >= 0 && in && saved && g_out && workspace, "mlp_backward: bad arguments");
+  FSGS_REQUIRE(n_layers >= 1 && n_layers <= 64, "mlp_backward: bad layer structure (%d layers)", n_layers);
+  const RowsWorkspace at(B, n_layers);
+  if (workspace_bytes < at.bytes) return fail(kWorkspaceSmall, "mlp_backward: workspace %zu < %zu bytes", workspace_bytes, at.bytes);
+  uint16_t* rows   = (uint16_t*) workspace;
+  uint16_t* states = (uint16_t*) ((char*) workspace + at.states);
+  uint16_t* own    = (uint16_t*) ((char*) workspace + at.own);
+  const int B_pad = (int) padded_rows(B);
+  const dim3 grid(B_pad / 32, kMlpWidth / 32, n_layers);
+  if (B > 0)
+    hipLaunchKernelGGL(mlp_transpose_kernel<false>, grid, dim3(256), 0, (hipStream_t) stream, B, B_pad, saved, states);
+  const int rc = fsgs_deform_mlp_backward(B, Din, width, n_layers, skip, 1, &n_out, in, nullptr, packed_t, heads_w, states,
+                                          &g_out, g_w, g_b, own, at.bytes - at.own, stream);
+  if (rc != kOk || B == 0) return rc;
+  hipLaunchKernelGGL(mlp_transpose_kernel<true>, grid, dim3(256), 0, (hipStream_t) stream, B, B_pad, own, rows);
+  return check_launch("mlp_backward");
 }

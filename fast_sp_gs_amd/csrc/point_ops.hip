@@ -979,7 +979,7 @@ FSGS_API int fsgs_knn_topk(int N, int M, int D, int K, const float* x, const flo
 
 FSGS_API size_t fsgs_lbs_blend_workspace_bytes(int M) { return align_up((size_t) (M > 0 ? M : 1) * kXf * 4, 256); }
 
-FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
+FSGS_API int fsgs_lbs_blend_strided(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
     const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
     const float* sp_s, int S, int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius,
     const float* sp_weight_logit, float* weights_out, float* d_xyz, float* d_rot, float* d_scale, void* workspace,
@@ -1005,6 +1005,16 @@ FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode,
   hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, s, N, M, K, S, warp_mode, weight_mode,
                      (float) temperature, points, xf, pair_in, index, weights_out, d_xyz, d_rot, d_scale);
   return check_launch("lbs_blend");
+}
+
+FSGS_API int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
+    const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
+    const float* sp_s, int S, const float* pair_in, const int64_t* index, const float* sp_log_radius,
+    const float* sp_weight_logit, float* weights_out, float* d_xyz, float* d_rot, float* d_scale, void* workspace,
+    size_t workspace_bytes, void* stream) {
+  return fsgs_lbs_blend_strided(N, M, K, warp_mode, weight_mode, temperature, points, sp_points, sp_t, sp_rot, sp_r, sp_s, S, S,
+                                pair_in, index, sp_log_radius, sp_weight_logit, weights_out, d_xyz, d_rot, d_scale, workspace,
+                                workspace_bytes, stream);
 }
 
 FSGS_API int fsgs_adam_masked_update(int64_t N, int64_t M, const uint8_t* mask, double lr, double b1, double b2,

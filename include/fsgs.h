@@ -435,9 +435,15 @@ int fsgs_knn_topk_ws(int N, int M, int D, int K, const float* x, const float* y,
  *   1  'LBS' with sp_rot[M,4] (:545-556): q_j = normalize(sp_rot_j + (0,0,0,1)), d_xyz = sum_k w_k (R(q_j) p + sp_t_j) - p;
  *   2  'LBS_c': as 1 with sp_t_j replaced by sp_t_j + c_j - R(q_j) c_j, c = sp_points (:548-549).
  * Always: d_rot[N,4] = sum_k w_k sp_r[j_k] (apply_rotate 'add', :565-566), d_scale[N,S] = sum_k w_k sp_s[j_k] (S <= 4; S = 0
- * and NULL pointers when the net predicts no scale residual; the rows of sp_s are sp_s_ld floats apart). weights_out[N,K] is optional. K <= 16. */
+ * and NULL pointers when the net predicts no scale residual). weights_out[N,K] is optional. K <= 16.
+ * _strided: the rows of sp_s are sp_s_ld >= S floats apart, so that S columns of a wider table are taken as they are. */
 size_t fsgs_lbs_blend_workspace_bytes(int M);
 int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode, double temperature, const float* points,
+    const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r, const float* sp_s, int S,
+    const float* pair_in, const int64_t* index, const float* sp_log_radius, const float* sp_weight_logit,
+    float* weights_out, float* d_xyz, float* d_rot, float* d_scale, void* workspace, size_t workspace_bytes,
+    void* stream);
+int fsgs_lbs_blend_strided(int N, int M, int K, int warp_mode, int weight_mode, double temperature, const float* points,
     const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r, const float* sp_s, int S,
     int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius, const float* sp_weight_logit,
     float* weights_out, float* d_xyz, float* d_rot, float* d_scale, void* workspace, size_t workspace_bytes,
@@ -449,12 +455,19 @@ int fsgs_lbs_blend(int N, int M, int K, int warp_mode, int weight_mode, double t
  * gradient of pair_in: of the squared distances in weight modes 0 and 1, of the logits in mode 2, of the weights in
  * mode 3), g_sp_points[M,3] (optional; the pivot term of warp mode 2, zeros otherwise -- the dependence of the distances
  * on sp_points goes through g_pair and fsgs_knn_topk_backward), g_sp_t[M,3], g_sp_rot[M,4] (warp modes 1, 2), g_sp_r[M,4],
- * g_sp_s[M,g_sp_s_ld] (zeros behind the first S columns), and in weight mode 1 g_log_radius[M] and (optional, with sp_weight_logit) g_weight_logit[M].
+ * g_sp_s[M,S], and in weight mode 1 g_log_radius[M] and (optional, with sp_weight_logit) g_weight_logit[M].
+ * _strided: sp_s as in fsgs_lbs_blend_strided, g_sp_s[M,g_sp_s_ld] with zeros behind the first S columns.
  * Per-control-point sums are taken without float atomics, in a fixed order, when M <= 1024, K <= 4 and M * columns <=
  * 11264 (columns = 7 + S, + 9 with a rotation, + 2 in weight mode 1); larger cases use LDS float atomics inside a block
  * (up to 36864 table cells) or device-scope float atomics, whose last bits can differ between runs. */
 size_t fsgs_lbs_blend_backward_workspace_bytes(int N, int M, int S);
 int fsgs_lbs_blend_backward(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
+    const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
+    const float* sp_s, int S, const float* pair_in, const int64_t* index, const float* sp_log_radius,
+    const float* sp_weight_logit, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_points,
+    float* g_pair, float* g_sp_points, float* g_sp_t, float* g_sp_rot, float* g_sp_r, float* g_sp_s,
+    float* g_log_radius, float* g_weight_logit, void* workspace, size_t workspace_bytes, void* stream);
+int fsgs_lbs_blend_backward_strided(int N, int M, int K, int warp_mode, int weight_mode, double temperature,
     const float* points, const float* sp_points, const float* sp_t, const float* sp_rot, const float* sp_r,
     const float* sp_s, int S, int sp_s_ld, const float* pair_in, const int64_t* index, const float* sp_log_radius,
     const float* sp_weight_logit, const float* g_xyz, const float* g_rot, const float* g_scale, float* g_points,
@@ -703,12 +716,14 @@ int fsgs_image_loss_forward_static(int B, int CH, int H, int W, double C1, doubl
  * and 16), in the order the matrix cores read it: 32-row x 16-column tiles, tile (r / 32, k / 16) at
  * ((r / 32) * (K_pad / 16) + k / 16) * 512 elements, element (r, k) inside it at (r % 32 + 32 * ((k % 16) / 8)) * 8 +
  * k % 8.
- * bias[n_layers*256 + n_out] fp32. out[B,n_out] fp32. saved_in and saved: both NULL, or [Din][B_pad] and
- * [n_layers][256][B_pad] bf16 (B_pad = B rounded up to 32; fsgs_mlp_saved_input_elems, fsgs_mlp_saved_elems) that receive
- * the input rows and every layer's post-ReLU hidden state, batch innermost, for the backward.
+ * bias[n_layers*256 + n_out] fp32. out[B,n_out] fp32. saved: NULL, or [n_layers][B][256] bf16 that receives every
+ * layer's post-ReLU hidden state for fsgs_mlp_backward.
  * fsgs_deform_mlp_forward writes the outputs as n_heads separate [B][head_rows[h]] tensors (at most 8) and forms the input
  * itself when `in` is NULL: the frequency encodings (input included) of the positions x[B,3] and of one time t[1], as
- * fsgs_freq_encode_forward has them, side by side. head_rows and outs are host arrays. */
+ * fsgs_freq_encode_forward has them, side by side. head_rows and outs are host arrays. Its saved_in and saved are both NULL
+ * or, as the kernels read them, [Din][B_pad] and [n_layers][256][B_pad] bf16 (B_pad = B rounded up to 32;
+ * fsgs_mlp_saved_input_elems, fsgs_mlp_saved_elems) with the input rows and the hidden states, batch innermost, for
+ * fsgs_deform_mlp_backward. */
 int fsgs_pack_bf16(int rows, int K, int rows_pad, int K_pad, const float* src, uint16_t* dst, void* stream);
 size_t fsgs_mlp_packed_elems(int Din, int n_layers, int skip);
 /* Every buffer fsgs_mlp_forward / fsgs_mlp_backward read, refreshed from the fp32 torch.nn.Linear parameters in one
@@ -721,8 +736,7 @@ int fsgs_mlp_pack_all(int Din, int n_layers, int skip, const float* const* weigh
     int n_heads, const float* const* head_weights, const float* const* head_biases, const int* head_rows,
     uint16_t* packed, uint16_t* packed_t, float* bias_out, float* heads_w_out, void* stream);
 int fsgs_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
-                     const uint16_t* packed, const float* bias, float* out, uint16_t* saved_in, uint16_t* saved,
-                     void* stream);
+                     const uint16_t* packed, const float* bias, float* out, uint16_t* saved, void* stream);
 size_t fsgs_mlp_saved_elems(int B, int n_layers);
 size_t fsgs_mlp_saved_input_elems(int B, int Din);
 int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
@@ -730,21 +744,23 @@ int fsgs_deform_mlp_forward(int B, int Din, int width, int n_layers, int skip, i
     const uint16_t* packed, const float* bias, float* const* outs, uint16_t* saved_in, uint16_t* saved, void* stream);
 
 /* Backward of fsgs_mlp_forward with respect to the weights and biases (torch autograd in the reference:
- * fast_2d_gs/network.py:1757-1776 is plain nn.Linear / relu). `saved` is the post-ReLU state the forward wrote; packed_t
- * holds, for layers 1 .. n_layers-1, the last 256 input columns of the weight transposed to [256 in][256 out] bf16
- * (fsgs_pack_bf16 of the transposed slice); heads_w[n_out][256] and g_out[B][n_out] are fp32. Outputs, fully written: g_w =
- * the layers' [256][K_l] gradients back to back (unpadded, K_0 = Din, K_{skip+1} = Din + 256, else 256) followed by the
- * heads' [n_out][256]; g_b[n_layers*256 + n_out].
+ * fast_2d_gs/network.py:1757-1776 is plain nn.Linear / relu). `saved` is the [n_layers][B][256] bf16 post-ReLU state the
+ * forward wrote when given a non-NULL `saved`; packed_t holds, for layers 1 .. n_layers-1, the last 256 input columns
+ * of the weight transposed to [256 in][256 out] bf16 (fsgs_pack_bf16 of the transposed slice); heads_w[n_out][256] and
+ * g_out[B][n_out] are fp32. Outputs, fully written: g_w = the layers' [256][K_l] gradients back to back (unpadded,
+ * K_0 = Din, K_{skip+1} = Din + 256, else 256) followed by the heads' [n_out][256]; g_b[n_layers*256 + n_out].
  * Operands are bf16, accumulation fp32. No gradient is produced for `in` directly; the workspace carries what a caller
- * needs to form it: after the call it starts with dZ[n_layers][256][B_pad] in bf16, the gradient of every layer's
- * pre-activation (masked by the stored state's zeros), so that
- * dL/d in = dZ[0]^T W_0 + dZ[skip+1]^T W_{skip+1}[:, :Din]. The rest of the workspace is scratch.
- * fsgs_deform_mlp_backward takes the outputs' gradients head by head (a NULL one is zero) and the forward's saved_in in
- * place of `in` (one of the two). */
-size_t fsgs_mlp_backward_workspace_bytes(int B, int Din, int n_layers);
+ * needs to form it: after the call its first n_layers * B * 256 * 2 bytes hold dZ[n_layers][B][256] in bf16, the
+ * gradient of every layer's pre-activation (masked by the stored state's zeros), so that
+ * dL/d in = dZ[0] W_0 + dZ[skip+1] W_{skip+1}[:, :Din]. The rest of the workspace is scratch.
+ * fsgs_deform_mlp_backward takes the outputs' gradients head by head (a NULL one is zero), the states as
+ * fsgs_deform_mlp_forward left them and its saved_in in place of `in` (one of the two); its workspace starts with
+ * dZ[n_layers][256][B_pad]. */
+size_t fsgs_mlp_backward_workspace_bytes(int B, int n_layers);
 int fsgs_mlp_backward(int B, int Din, int width, int n_layers, int skip, int n_out, const float* in,
     const uint16_t* packed_t, const float* heads_w, const uint16_t* saved, const float* g_out, float* g_w, float* g_b,
     void* workspace, size_t workspace_bytes, void* stream);
+size_t fsgs_deform_mlp_backward_workspace_bytes(int B, int Din, int n_layers);
 int fsgs_deform_mlp_backward(int B, int Din, int width, int n_layers, int skip, int n_heads, const int* head_rows,
     const float* in, const uint16_t* saved_in, const uint16_t* packed_t, const float* heads_w, const uint16_t* saved,
     const float* const* g_outs, float* g_w, float* g_b, void* workspace, size_t workspace_bytes, void* stream);

@@ -99,6 +99,14 @@ def test_c_abi_rejects_bad_sizes_without_touching_the_gpu():
     assert L.fsgs_gs_prepare_scan(0, None, None, None, 0, ctypes.addressof(R), None) == 0 and R.value == 0
 
 
+def test_entry_points_keep_their_parameters():
+    """Programs built against an earlier header call these by name; wider forms have names of their own."""
+    from fast_sp_gs_amd import lib
+    for name, parameters in {'fsgs_lbs_blend': 24, 'fsgs_lbs_blend_backward': 32, 'fsgs_mlp_forward': 12,
+                             'fsgs_mlp_backward': 16, 'fsgs_mlp_backward_workspace_bytes': 2}.items():
+        assert len(lib.prototypes()[name][1]) == parameters, name
+
+
 def test_renderer_wrapper_is_importable_and_binds_by_name():
     from fast_sp_gs_amd.renderer import gs_2d_render as m
     from fast_sp_gs_amd._C import get_C_function

@@ -136,3 +136,35 @@ def test_scale_table_of_any_layout(layout, M, device):
         results.append((out, *torch.autograd.grad((out * up[:, :out.shape[1]]).sum(), [leaf])))
     assert torch.equal(results[0][0], results[1][0])
     assert torch.allclose(results[0][1], results[1][1], rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize('B', [1, 31, 32, 33, 300])
+def test_network_entry_points_with_states_as_rows(B, device):
+    """fsgs_mlp_forward / _backward, whose callers keep [layer][B][256] states and read dZ in that form, against the
+    operators, which keep the batch innermost: the same numbers."""
+    from fast_sp_gs_amd import lib as L
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.deform import DeformNetwork
+    torch.manual_seed(B)
+    net, lib = DeformNetwork().to(device), L.load()
+    net.pack()
+    x = net.encode(torch.rand(B, 3, device=device) * 2 - 1, torch.rand(1, device=device)).detach()
+    rows, Din = 10, x.shape[1]
+    want, states = get_C_function('mlp_forward')(x, *net._packed, net.D, net.skip, rows, True)
+    up = torch.randn(B, rows, device=device)
+    w_want, b_want, dz_want = get_C_function('mlp_backward')(x, net._packed_t, net._heads_w, states, up, net.D, net.skip, True)
+    out = torch.full((B, rows), float('nan'), device=device)
+    saved = torch.zeros(net.D, B, 256, dtype=torch.int16, device=device)
+    stream = L.current_stream()
+    rc = lib.fsgs_mlp_forward(B, Din, 256, net.D, net.skip, rows, L.ptr(x), *map(L.ptr, net._packed), L.ptr(out), L.ptr(saved),
+                              stream)
+    L.check(rc, 'fsgs_mlp_forward')
+    assert torch.equal(out, want) and torch.equal(saved, states)
+    g_w, g_b = (torch.full_like(t, float('nan')) for t in (w_want, b_want))
+    ws = torch.empty(lib.fsgs_mlp_backward_workspace_bytes(B, net.D), dtype=torch.uint8, device=device)
+    args = (B, Din, 256, net.D, net.skip, rows, L.ptr(x), L.ptr(net._packed_t), L.ptr(net._heads_w), L.ptr(saved), L.ptr(up),
+            L.ptr(g_w), L.ptr(g_b), L.ptr(ws))
+    L.check(lib.fsgs_mlp_backward(*args, ws.numel(), stream), 'fsgs_mlp_backward')
+    dz = ws[:net.D * B * 512].view(torch.bfloat16).view(net.D, B, 256)
+    assert torch.equal(g_w, w_want) and torch.equal(g_b, b_want) and torch.equal(dz, dz_want)
+    assert lib.fsgs_mlp_backward(*args, ws.numel() - 1, stream) != 0
