@@ -74,8 +74,13 @@ variable_list warp_forward(const SuperpointWarp& w, Tensor& d2, Tensor& table) {
   const int64_t N = w.points.size(0), M = w.sp_points.size(0), K = w.K;
   require_shape(what, "sp_t", w.sp_t, {M, 3}), require_shape(what, "sp_r", w.sp_r, {M, 4});
   if (has(w.sp_rot)) require(what, "sp_rot", *w.sp_rot, at::kFloat), require_shape(what, "sp_rot", *w.sp_rot, {M, 4});
-  if (has(w.sp_radius)) require(what, "sp_log_radius", *w.sp_radius, at::kFloat);
-  if (has(w.sp_weight)) require(what, "sp_weight_logit", *w.sp_weight, at::kFloat);
+  if (w.points.size(1) < 3) fail("lbs_blend: positions [N,3] and [M,3] are expected");
+  auto per_control = [&](const char* name, const OptTensor& t) {
+    if (!has(t)) return;
+    require(what, name, *t, at::kFloat);
+    if (t->numel() < M) fail(std::string(what) + ": " + name + " must hold a value per control point");
+  };
+  per_control("sp_log_radius", w.sp_radius), per_control("sp_weight_logit", w.sp_weight);
   int S = 0, ld = 0;
   if (has(w.sp_s)) {
     const Tensor& s = *w.sp_s;

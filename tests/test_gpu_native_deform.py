@@ -168,3 +168,19 @@ def test_network_entry_points_with_states_as_rows(B, device):
     dz = ws[:net.D * B * 512].view(torch.bfloat16).view(net.D, B, 256)
     assert torch.equal(g_w, w_want) and torch.equal(g_b, b_want) and torch.equal(dz, dz_want)
     assert lib.fsgs_mlp_backward(*args, ws.numel() - 1, stream) != 0
+
+
+def test_short_control_tables_are_refused(device):
+    """On the host: fewer radii or weights than control points, positions with fewer than three coordinates."""
+    from fast_sp_gs_amd.deform import superpoint_deform
+    g = torch.Generator().manual_seed(5)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(device)
+    M, points, moves = 40, r(100, 3), (r(40, 3), r(40, 4), r(40, 2))
+    kernel = lambda radius, weight: superpoint_deform(points, r(M, 3), *moves, LBS_method='weighted_kernel', sp_radius=radius,
+                                                      sp_weight=weight)[0]
+    assert torch.isfinite(kernel(r(M), r(M, 1))).all()
+    for radius, weight in ((r(M - 1), r(M)), (r(M), r(M - 1))):
+        with pytest.raises(RuntimeError, match='a value per control point'):
+            kernel(radius, weight)
+    with pytest.raises(RuntimeError, match='positions'):
+        superpoint_deform(points[:, :2], r(M, 2), *moves)
