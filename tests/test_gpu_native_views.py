@@ -269,3 +269,87 @@ def test_colours_of_a_wrong_shape_are_refused(view, split, device):
             picture(sh_features=s.shs[1:, :1].contiguous())
         assert torch.isfinite(picture(sh_features=s.shs[:, :1].contiguous())['images']).all()
     assert torch.isfinite(picture(colors=torch.zeros(P, 3, device=device))['images']).all()
+
+
+def _tail_in_double(Tw2v, Tv2c, size, extras, opacity, depth_ratio):
+    """normals, depths, surf_depth, surf_normal of the blend's maps in 64 bits, and per pixel how far single precision
+    throws the pseudo normal: the points p carry about eight roundings each, the unit normal of the differences a and b
+    turns by their error times (|a| + |b|) / |a x b|."""
+    Tw2v, Tv2c, (W, H) = Tw2v.double(), Tv2c.double(), size
+    pixels = torch.tensor([[W / 2, 0, 0, W / 2], [0, H / 2, 0, H / 2], [0, 0, 0, 1]], dtype=torch.float64, device=Tw2v.device)
+    y, x = torch.meshgrid(torch.arange(H, device=Tw2v.device), torch.arange(W, device=Tw2v.device), indexing='ij')
+    at = torch.stack([x, y, torch.ones_like(x)], dim=-1).double()
+    rays = at @ ((pixels @ Tv2c)[:, :3].inverse().T @ Tw2v[:3, :3].inverse().T)
+    normals = (extras[1:4].permute(1, 2, 0) @ Tw2v[:3, :3]).permute(2, 0, 1)
+    depths, median = torch.nan_to_num(extras[0:1], 0, 0), torch.nan_to_num(extras[4:5], 0, 0)
+    surf_depth = depths * (1 - depth_ratio) + depth_ratio * median
+    p = surf_depth.reshape(H, W, 1) * rays + Tw2v.inverse()[:3, 3]
+    a, b = p[2:, 1:-1] - p[:-2, 1:-1], p[1:-1, 2:] - p[1:-1, :-2]
+    c = torch.cross(a, b, dim=-1)
+    surf_normal = torch.nn.functional.pad(torch.nn.functional.normalize(c, dim=-1).permute(2, 0, 1), (1, 1, 1, 1))
+    far = p.norm(dim=-1)
+    far = torch.stack([far[2:, 1:-1], far[:-2, 1:-1], far[1:-1, 2:], far[1:-1, :-2]]).amax(0)
+    turn = 8 * 2.0 ** -24 * far * (a.norm(dim=-1) + b.norm(dim=-1)) / c.norm(dim=-1)
+    turn = torch.nn.functional.pad(torch.nan_to_num(turn.detach(), nan=1.0, posinf=1.0), (1, 1, 1, 1), value=0.0)
+    return normals, median, surf_depth, surf_normal * opacity, turn
+
+
+@pytest.mark.parametrize('P,W,H,mode', [(1, 16, 16, 'sh'), (257, 49, 31, 'split'), (256, 64, 48, 'colors'),
+                                        (300, 49, 31, 'partial'), (3_000, 161, 99, 'culling'), (4_000, 120, 90, 'ratio')])
+@pytest.mark.parametrize('view', ['surfel', 'fast_surfel'])
+def test_surfel_tails_against_double(view, P, W, H, mode, device):
+    """Surfels of several pixels, so that the small pictures are covered too. Every map of the fused tail and the gradients
+    of all of them together, surf_normal among them, against the tail in 64 bits around the operators."""
+    from fast_sp_gs_amd.renderer import gs_2d_fast_render, gs_2d_render
+    s, cam_h, g = _scene(P, W, H, P + 4, scale=-2.0 if P < 1000 else -3.0)
+    cam = cam_h.to(device)
+    params = _leaves(device, s.means3D, s.scales, s.rotations, s.opacities)
+    rest, degree, ratio = None, 2 if mode == 'partial' else 3, 0.25 if mode == 'ratio' else 1.0
+    if mode == 'split':
+        sh, rest = _leaves(device, s.shs[:, :1].contiguous(), s.shs[:, 1:].contiguous())
+    else:
+        sh, = _leaves(device, s.shs[:, 0].contiguous() if mode == 'colors' else s.shs)
+    culling = (torch.rand(P, generator=g) < 0.3).to(device) if mode == 'culling' else None
+    kw = dict(campos=cam.campos, sh_degree=degree, colors=sh if mode == 'colors' else None,
+              sh_features=None if mode == 'colors' else sh, sh_features_rest=rest, culling=culling, depth_ratio=ratio)
+    m2, size, cams = torch.zeros(P, 2, device=device, requires_grad=True), (W, H), (cam.Tw2v, cam.Tv2c)
+    drawn = (cam.campos, size, -1 if mode == 'colors' else degree, False, 0.2, 100.0, False, None, m2, None, culling, None, None,
+             None)
+    background = None
+    if view == 'surfel':
+        background = torch.rand(3, generator=g).to(device)
+        out = gs_2d_render.GS_2D_render(*params, size, *cams, background=background, **kw)
+        img, opac, extras, *_ = gs_2d_render._GS_2D_Render.apply(*params, sh, rest, *cams, *drawn)
+    else:
+        out = gs_2d_fast_render.GS_2D_fast_render(*params, size, *cams, cam.Tv2s, **kw)
+        img, opac, extras, *_ = gs_2d_fast_render._Fast_Render.apply(*params, sh, rest, *cams, cam.Tv2s, *drawn)
+    assert mode == 'sh' or float((opac > 0.1).float().mean()) > 0.2
+
+    maps64 = extras.detach().double().requires_grad_(True)
+    normals, median, surf_depth, surf_normal, turn = _tail_in_double(*cams, size, maps64, opac.detach().double(), ratio)
+    for name, want in (('normals', normals), ('depths', median), ('surf_depth', surf_depth)):
+        assert name not in out or torch.allclose(out[name].double(), want, rtol=1e-6, atol=1e-6), name
+    steady = turn < 1e-4
+    assert mode == 'sh' or float((steady & (opac > 0.1)).float().mean()) > 0.1
+    off = (out['surf_normal'].detach().double() - surf_normal.detach()).norm(dim=0)
+    assert bool((off <= turn + 1e-6)[steady].all())
+
+    names = [k for k in ('images', 'opacity', 'normals', 'depths', 'surf_depth', 'surf_normal', 'distortion') if k in out]
+    up = {k: torch.randn(out[k].shape, generator=g).to(device) for k in names}
+    up['surf_normal'] = up['surf_normal'] * steady
+    wanted = params + [sh] + ([rest] if rest is not None else [])
+    keep = [k for k in names if k not in ('images', 'opacity')]
+    of64 = {'normals': normals, 'depths': median, 'surf_depth': surf_depth, 'surf_normal': surf_normal,
+            'distortion': maps64[5:6]}
+    for some in (keep, ['surf_normal']):
+        got = torch.autograd.grad([out[k] for k in ['images', 'opacity'] + some], wanted + [out['viewspace_points']],
+                                  [up[k] for k in ['images', 'opacity'] + some], retain_graph=True, allow_unused=True)
+        g_maps, = torch.autograd.grad([of64[k] for k in some], [maps64], [up[k].double() for k in some], retain_graph=True)
+        g_opac = up['opacity'] if background is None else up['opacity'] - (background[:, None, None] * up['images']).sum(0)
+        ref = torch.autograd.grad([img, opac, extras], wanted + [m2], [up['images'], g_opac.reshape(opac.shape), g_maps.float()],
+                                  retain_graph=True, allow_unused=True)
+        for k, (a, b) in enumerate(zip(got, ref)):
+            assert (a is None) == (b is None)
+            if a is not None:
+                # a pixel's part is off by its turn, once for the direction and twice for the two differences' lengths
+                assert (a - b).norm() <= 3e-4 * b.norm() + 1e-7
