@@ -15,9 +15,9 @@
 //      whose cell has more than 128 candidates, or that lie outside the grid are taken by the whole wavefront one at a
 //      time (64 control points per step), or all together by the search over all control points when they are many.
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.30 ms this way (lists
-// 0.048, queries 0.248; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by the address path
-// of the vector memory (busy 0.7 of the time: every lane reads its own list lines), vector issue is 0.6.
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.29 ms a call this way
+// (traced: lists 0.044, queries 0.272; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
+// the address path of the vector memory (TA busy 0.82 of the time: every lane reads its own list lines); vector issue 0.70.
 // 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
 
@@ -28,7 +28,7 @@ namespace {
 
 constexpr int kListCap   = 128;   // candidates per cell: seven position bits
 constexpr int kCoarse    = 8;     // coarse cells per axis
-constexpr int kMaxPoints = 2560;  // control points a block keeps in LDS, 16 bytes each (55 KB in the list kernel)
+constexpr int kMaxPoints = 2560;  // control points a block keeps in LDS, 16 bytes each (41 of the list kernel's 72 KB at G = 32, of its 51 KB at G = 16)
 constexpr int kMaxK      = 8;
 constexpr int kOctantCap = 1024;  // candidates of an octant of a coarse cell
 constexpr int kAhead = 4;
@@ -44,7 +44,9 @@ enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 // Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
 // alone) and N * M / 4e12 s when they fill the chip; a wavefront per query 0.8 (M = 512) to 2.0 ns (M = 2048) a query;
 // building the lists 10 us (G = 16, 512 control points) to 48 us (G = 32, 2048). With G = 16 the lists of more than 640
-// control points outgrow their 128 entries; below that the finer grid pays from a million queries on.
+// control points outgrow their 128 entries; below that the finer grid pays from a million queries on. Behind the limits
+// the walk over all pairs takes over at its own price: 3M queries, K = 4: 232 us for 2560 control points, 1597 for 2561; 2048
+// control points, K = 8: 313 us, K = 9: 5908. 200 000 queries, K = 4: 90 and 204 us.
 Scheme knn_scheme(int N, int M, int D, int K) {
   if (D != 3 || K > kMaxK || M > kMaxPoints || M < 96) return kAllPairs;
   if (N <= kFewQueries) return kAlone;

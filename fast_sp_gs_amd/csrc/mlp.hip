@@ -18,7 +18,7 @@
 // consecutive rows of one column, so that layout takes 8-byte stores, and it is what the weight gradients read. The
 // backward (the reference leaves it to torch autograd: one addmm-backward pair and a ReLU mask per layer, ~30 launches)
 // is two kernels:
-//   * a chain kernel with the forward's structure, one block per 32 rows: dZ_L-1 = (g_out . W_heads) masked by the saved
+//   * a chain kernel with the forward's structure, one block per 16 rows: dZ_L-1 = (g_out . W_heads) masked by the saved
 //     state, then for each layer dH_l-1 = dZ_l . W_l[:, hidden part] on the matrix cores against a transposed bf16 copy
 //     of the weights, masked, kept in LDS for the next layer and written to HBM as dZ[l][256][B_pad];
 //   * a weight-gradient kernel over all layers at once, dW = dZ^T X: with the batch innermost both operands' fragments are
