@@ -6,6 +6,10 @@ Gaussians, Adam on the network and the control points.
 
 `DynamicStep` owns the state (parameters, the two optimisers); `forward_loss` is the differentiable part alone so that
 tests can compare its gradients with other formulations.
+
+The network runs on the bf16 copies of its weights that it made when it was first called, since the network's optimiser
+leaves the parameters' version counters alone, as torch's fused Adam does: a training loop calls `step.net.pack()` after
+each step to have the stepped weights in use.
 """
 from __future__ import annotations
 
