@@ -8,6 +8,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
 
 #include <mutex>
 #include <stdexcept>
@@ -43,12 +44,14 @@ void require_shape(const char* what, const char* name, const Tensor& t, at::IntA
 inline bool has(const OptTensor& t) { return t.has_value() && t->defined(); }
 inline Tensor opt(const OptTensor& t) { return has(t) ? *t : Tensor(); }
 
-// Forward-mode derivatives are not implemented; a dual tensor would lose its tangent on the way through a kernel.
+// Forward-mode derivatives are not implemented; a dual tensor would lose its tangent on the way through a kernel. There
+// are dual tensors only while a dual level (torch has one, 0) is open.
 inline bool is_dual(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 inline bool is_dual(const OptTensor& t) { return has(t) && is_dual(*t); }
 template <typename... T>
 void refuse_duals(const char* what, const T&... t) {
-  if ((is_dual(t) || ...)) fail(std::string(what) + ": forward-mode differentiation is not implemented");
+  if (torch::autograd::ForwardADLevel::try_get_by_idx(0) && (is_dual(t) || ...))
+    fail(std::string(what) + ": forward-mode differentiation is not implemented");
 }
 
 // Stored SH coefficients per point beside the split-off first one: checks [P,M,3] (or [P,1,3] + [P,M,3], or colours [P,3]
