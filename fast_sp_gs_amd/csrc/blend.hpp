@@ -421,6 +421,17 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v) {
   return v;
 }
 
+// Sum over each aligned group of 8 or 16 lanes; the total is valid in the group's last lane only.
+template <int kLanes>
+__device__ __forceinline__ float block_sum_to_last(float v) {
+#pragma clang fp contract(off)
+  v += dpp_shift_zero<0x111, 0xf, 0xf>(v);
+  v += dpp_shift_zero<0x112, 0xf, 0xf>(v);
+  v += dpp_shift_zero<0x114, 0xf, 0xf>(v);
+  if (kLanes == 16) v += dpp_shift_zero<0x118, 0xf, 0xf>(v);
+  return v;
+}
+
 // ---- per-surfel side sums of the forward blends ---------------------------------------------------------------------
 // accum_weights_p / accum_weights_count: a wavefront blends one list entry at a time, so the up to 64 per-pixel adds of
 // an entry go to one address. They are summed in the wavefront first (one DPP reduction, one population count) and lane 63

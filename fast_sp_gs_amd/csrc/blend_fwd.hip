@@ -8,25 +8,30 @@
 // or per pixel first and issues few atomics (see ArgmaxRun and the weight staging below) instead of up to three per
 // pair.
 //
-// Layout: one 256-lane block per 16x16 tile; wavefront w owns an 8x8 pixel quadrant. Surfels of the tile's sorted
-// range are gathered 128 at a time (one per lane of the first two wavefronts, colours included so the blend never goes back to HBM) into LDS as
-// 48-byte "hot" + 32-byte "cold" records; the next batch's gather is issued before the current batch is blended so its
-// HBM latency overlaps the arithmetic. All lanes of a wavefront read the same LDS record (broadcast, conflict free).
-#include "blend.hpp"
+// Layout: one 256-lane block per 16x16 tile; wavefront w owns an 8x8 pixel quadrant, eight lanes at a time a 2x4 block of
+// it with a work list of its own (block_lists.hpp). Surfels of the tile's sorted range are gathered 192 at a time (one per
+// lane of the first three wavefronts, colours included so the blend never goes back to HBM) into LDS as 80-byte records; the
+// next batch's gather is issued before the current batch is blended so its HBM latency overlaps the arithmetic.
+// Bound by vector issue (60 instructions a step, three of them transcendental). 300k surfels 800x800: 147 us with one list
+// per quadrant, 107 with lists per 4x4 block, 94 per 2x4 block; 3M 1352x1014: 506, 333, 282; 400k 3840x2160: 930, 845, 849;
+// 10k 256x256: 28, 19, 18. Batches of 64 / 128 / 192 surfels (a list's length varies less over a long batch), 2x4: 113 / 97 /
+// 94 us at 300k, 346 / 297 / 282 at 3M.
+#include "block_lists.hpp"
 
 namespace fsgs {
 namespace {
 
 #ifndef FSGS_FWD_BATCH
-#define FSGS_FWD_BATCH 128
+#define FSGS_FWD_BATCH 192
 #endif
+#ifndef FSGS_FWD_LANES
+#define FSGS_FWD_LANES 8
+#endif
+constexpr int kFwdLanes = FSGS_FWD_LANES;  // lanes (pixels) that share a work list
 constexpr int kFwdBatch = FSGS_FWD_BATCH;  // surfels staged per round (<= block size)
 
 // kAccum: 0 = no side outputs, 1 = accum_max_count only (what the reference's training loop passes on every step),
 // 2 = accum_weights_p and / or accum_weights_count as well.
-constexpr int kAccSlots  = 16;  // entries whose per-pixel weights a wavefront stages before it sums them
-constexpr int kAccStride = 68;  // floats per staged entry: 64 lanes + 4, so that the 16 readers of a row hit 16 x 4 banks
-
 template <bool kAux, bool kFlow, int kAccum>
 __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
@@ -36,21 +41,20 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
     float* __restrict__ out_color, float* __restrict__ out_opacity, float* __restrict__ out_extras,
     float2* __restrict__ out_flow, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
     int32_t* __restrict__ accum_weights_count) {
-  __shared__ SplatHot s_hot[kFwdBatch];
-  __shared__ SplatCold s_cold[kFwdBatch];
+  using Shape = BlockShape<kFwdLanes>;
+  __shared__ Splat s_splat[kFwdBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kFwdBatch * 9 : 1];
-  __shared__ unsigned char s_mask[kFwdBatch];  // which 8x8 quadrants of the tile each staged surfel can reach
-  // accum_weights_*: every lane of a wavefront blends the same entry, so an entry's per-pixel weights all go to one
-  // address. Each wavefront parks them in its own LDS rows (one plain store per entry), and after kAccSlots entries sums
-  // all rows at once -- lane l adds 16 lanes' worth of entry l & 15, two row / half swaps finish the sum -- and lanes
-  // 0..15 issue one atomic per entry and output.
-  __shared__ __attribute__((aligned(16))) float s_accw[kAccum == 2 ? 4 * kAccSlots * kAccStride : 4];
-  __shared__ int s_accid[kAccum == 2 ? 4 * kAccSlots : 1], s_accn[kAccum == 2 ? 4 * kAccSlots : 1];
+  __shared__ unsigned s_mask[kFwdBatch];  // which blocks of the tile each staged surfel can reach
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[Shape::kPerTile * kFwdBatch + 16];
+  // accum_weights_*: the weights of the tile's pixels per staged surfel, summed over a row in registers, over the tile's
+  // rows here; one global atomic per staged surfel and output
+  __shared__ float s_accw[kAccum == 2 ? kFwdBatch : 1];
+  __shared__ int s_accn[kAccum == 2 ? kFwdBatch : 1];
 
   const int gx = (W + kTile - 1) / kTile;
   const int tile = scheduled_tile(ordered, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW   = (size_t) H * W;
   const size_t pix  = (size_t) W * py + px;
@@ -61,32 +65,26 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
   const int n_todo = (int) (r1 - r0);
   const int rounds = (n_todo + kFwdBatch - 1) / kFwdBatch;
 
-  // A pixel stops blending once its transmittance would fall below 1e-4. The state is a float, not a bool: the test
-  // is then one comparison whose lane mask feeds the branches directly (a bool carried round the loop lives in a
-  // register as 0 / 1 and is turned into a mask again at every use).
-  float live = inside ? 1.0f : -1.0f;
-  // the same for the wavefront, as a lane mask in scalar registers: "is anybody still blending" costs no vector work
+  // The pixels still blending (their transmittance has not fallen below 1e-4), as a lane mask in scalar registers: neither
+  // keeping it nor asking "is anybody left" costs vector work.
   unsigned long long live_lanes = wave_ballot(inside);
   const float far_scale = far_n / (far_n - near_n), far_near = far_scale * near_n;
   float T = 1.0f, C0 = 0, C1 = 0, C2 = 0;
   float N0 = 0, N1 = 0, N2 = 0, D = 0, M1 = 0, M2 = 0, dist = 0, median = 0, wsum = 0, f0 = 0, f1 = 0;
   int last = 0, median_c = -1;
   ArgmaxRun argmax;
-  int acc_slot = 0;  // staged entries of this wavefront (wave-uniform)
+  // this thread's staged surfel: its sums of the batch before go out, its places are cleared for the next
   auto flush_weights = [&]() {
-    if (acc_slot == 0) return;
-    const float4* src = (const float4*) &s_accw[(wave * kAccSlots + (lane & 15)) * kAccStride + (lane >> 4) * 16];
-    const float4 a = src[0], b = src[1], c = src[2], d = src[3];
-    float t = (((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w))) +
-              (((c.x + c.y) + (c.z + c.w)) + ((d.x + d.y) + (d.z + d.w)));
-    t = cross_row_sum(t);
-    if (lane < acc_slot) {
-      const int id = s_accid[wave * kAccSlots + lane];
-      if (accum_weights_p) atomicAdd(&accum_weights_p[id], t);
-      if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[wave * kAccSlots + lane]);
-    }
-    acc_slot = 0;
+    const int t = (int) threadIdx.x;
+    if (t >= kFwdBatch || s_accn[t] == 0) return;
+    const int id = s_splat[t].cold.id;
+    if (accum_weights_p) atomicAdd(&accum_weights_p[id], s_accw[t]);
+    if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[t]);
+    s_accw[t] = 0.0f, s_accn[t] = 0;
   };
+  if (threadIdx.x == 0) s_splat[kFwdBatch] = Splat{};  // all zero: p_z == 0 everywhere
+  if (threadIdx.x < 4) ((unsigned*) &s_list[Shape::kPerTile * kFwdBatch])[threadIdx.x] = 0u;
+  if (kAccum == 2 && threadIdx.x < kFwdBatch) s_accw[threadIdx.x] = 0.0f, s_accn[threadIdx.x] = 0;
 
   Splat next;
   float next_t2[9];
@@ -99,15 +97,19 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
 
   for (int b = 0; b < rounds; ++b) {
     // everyone has finished reading the previous batch; leave as soon as no pixel of the tile is still blending
-    if (__syncthreads_count(live < 0.0f) == kBlendThreads) break;
+    if (__syncthreads_and(live_lanes == 0ull)) break;
     const int n_here = min(kFwdBatch, n_todo - b * kFwdBatch);
-    if ((int) threadIdx.x < n_here) {
-      s_hot[threadIdx.x]  = next.hot;
-      s_cold[threadIdx.x] = next.cold;
-      s_mask[threadIdx.x] = (unsigned char) quadrant_mask(next.hot, tile_x * kTile, tile_y * kTile, ordered);
-      if (kFlow)
+    if (kAccum == 2) flush_weights();
+    if ((int) threadIdx.x < kFwdBatch) {
+      unsigned mask = 0u;
+      if ((int) threadIdx.x < n_here) {
+        s_splat[threadIdx.x] = next;
+        mask = surfel_blocks<kFwdLanes>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
+        if (kFlow)
 #pragma unroll
-        for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+      }
+      s_mask[threadIdx.x] = mask;
     }
     __syncthreads();
     const int nxt = (b + 1) * kFwdBatch + threadIdx.x;
@@ -118,38 +120,31 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
         for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
     }
 
-    // Each wavefront walks only the surfels that can reach its quadrant: the ballot of the mask bit over 64 staged
-    // surfels is the (depth-ordered) work list, consumed bit by bit with scalar instructions.
-    for (int c = 0; c < kFwdBatch / kWave; ++c) {
-      const int jj = c * kWave + lane;
-      unsigned long long todo = __ballot(jj < n_here && ((s_mask[jj] >> wave) & 1u));
-      if (todo == 0ull) continue;
-      // One list entry: `hot` was requested an entry earlier. A wavefront walks its list alone, so everything that
-      // waits -- the LDS round trip for a surfel's record, chains of nested divergent branches -- is paid once per
-      // entry on the tile's critical path (the launch lasts as long as its longest tile). Hence: the NEXT entry's record
-      // is requested before the current one is evaluated, into alternating registers; the intersection runs without
-      // early exits and yields one predicate; the blend is one divergent region.
-      auto blend_entry = [&](const SplatHot& hot, const SplatCold& cold, int j) {
-#pragma clang fp contract(off)  // two copies of this body exist (alternating registers): both must round alike
+    // One list entry per block of the wavefront. The intersection runs without early exits and yields one predicate; the
+    // blend is one divergent region.
+    unsigned char* const lists = &s_list[Shape::kPerWave * wave * kFwdBatch];
+    const int steps = build_block_lists<kFwdLanes, kFwdBatch>(lists, s_mask, wave, live_lanes);
+    auto blend_entry = [&](const SplatHot& hot, int j) {
+#pragma clang fp contract(off)  // several copies of this body exist (alternating registers): they must round alike
+        const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+        __builtin_amdgcn_sched_barrier(0);
         Hit h;
         unsigned long long pass;
-        const bool hit = intersect_flat(hot, pxf, pyf, near_n, h, &pass) && live > 0.0f;
+        intersect_flat(hot, pxf, pyf, near_n, h, &pass);
         pass &= live_lanes;
         if (pass == 0ull) return;
         const float test_T = T * (1.0f - h.alpha);
-        const bool sat     = hit && test_T < 0.0001f;
-        live               = sat ? -1.0f : live;
-        live_lanes &= ~(pass & wave_ballot(test_T < 0.0001f));
+        const unsigned long long sat = pass & wave_ballot(test_T < 0.0001f);
+        live_lanes &= ~sat;
+        const unsigned long long blends = pass & ~sat;
+        const bool blend = __builtin_amdgcn_inverse_ballot_w64(blends);
         const float w      = h.alpha * T;
         if (kAccum == 2) {
-          const unsigned long long who = wave_ballot(hit && !sat);
-          if (who != 0ull) {
-            s_accw[(wave * kAccSlots + acc_slot) * kAccStride + lane] = hit && !sat ? w : 0.0f;
-            if (lane == 0) s_accid[wave * kAccSlots + acc_slot] = cold.id, s_accn[wave * kAccSlots + acc_slot] = (int) __popcll(who);
-            if (++acc_slot == kAccSlots) flush_weights();
-          }
+          const int n = (int) __popcll(blends >> (lane & -kFwdLanes) & ((1ull << kFwdLanes) - 1ull));
+          const float sum = block_sum_to_last<kFwdLanes>(blend ? w : 0.0f);
+          if ((lane & (kFwdLanes - 1)) == kFwdLanes - 1 && n > 0) atomicAdd(&s_accw[j], sum), atomicAdd(&s_accn[j], n);
         }
-        if (hit && !sat) {
+        if (blend) {
           const int contributor = b * kFwdBatch + j + 1;
           if (kAux) {
             const float A  = 1.0f - T;
@@ -178,36 +173,15 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
           last = contributor;
         }
       };
-      auto pop = [&]() {
-        const int j = c * kWave + __builtin_ctzll(todo);
-        todo &= todo - 1;
-        return j;
-      };
-      auto peek = [&]() { return c * kWave + (todo ? __builtin_ctzll(todo) : 0); };
-      SplatHot hot_a = s_hot[peek()], hot_b;
-      while (todo) {
-        if (live_lanes == 0ull) break;  // every pixel of this quadrant is saturated
-        {
-          const int j = pop();
-          hot_b       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];  // read only if a pixel blends the surfel, but then without waiting
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_a, cold, j);
-        }
-        if (todo == 0ull || live_lanes == 0ull) break;
-        {
-          const int j = pop();
-          hot_a       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_b, cold, j);
-        }
-      }
-    }
+    walk_block_list(lists + lane / kFwdLanes * kFwdBatch, steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
+                    [&]() { return live_lanes != 0ull; });
   }
 
   if (kAccum != 0) argmax_run_flush(argmax, accum_max_count);
-  if (kAccum == 2) flush_weights();
+  if (kAccum == 2) {
+    __syncthreads();
+    flush_weights();
+  }
   if (inside) {
     out_opacity[pix]      = 1.0f - T;
     n_contrib[pix]        = last;

@@ -1,0 +1,193 @@
+// Work lists per small block of pixels: the bound that fills them and the lists themselves, shared by the blend kernels.
+//
+// The blend kernels are bound by the vector instructions of a (wavefront, entry) pass. A wavefront owns an 8x8 quadrant of a
+// tile; with one list for all of it, an entry that reaches any of its pixels costs a pass of 64 lanes, of which 0.15 (3M
+// small surfels, 1352x1014), 0.20 (300k, 800x800) or 0.50 (400k, 3840x2160) have something to blend. Here every group of
+// 16 (or 8) lanes owns a block of 4x4 (2x4) pixels and walks a list of its own, the staged entries that can reach the block,
+// in list order: all groups run one instruction stream on different entries. A pass then lasts as long as the longest of the
+// wavefront's lists, per staged batch; together with the tighter bound below, passes fall to 0.52, 0.60 and 0.72 (4x4) or
+// 0.43, 0.52 and 0.70 (2x4) of what they were. Blocks of 2x2 would bring 0.36, 0.46 and 0.67, against twice as many lists to
+// build and records to fetch as 2x4.
+#pragma once
+#include "blend.hpp"
+
+namespace fsgs {
+
+// Lanes of a block: 16 (4x4 pixels) or 8 (2 wide, 4 tall). Bit q * kPerWave + g of a block mask: block g of quadrant q.
+template <int kLanes>
+struct BlockShape {
+  static_assert(kLanes == 16 || kLanes == 8);
+  static constexpr int kWide = kLanes / 4, kColumns = kTile / kWide, kPerWave = kWave / kLanes, kPerTile = 4 * kPerWave;
+  // pixel of this lane: its wavefront's quadrant, its block (kPerWave / 2 beside each other, two rows of them), row-major inside
+  static __device__ __forceinline__ void lane_pixel(int tile_x, int tile_y, int& px, int& py) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / kLanes, in = lane % kLanes;
+    px = tile_x * kTile + (wave & 1) * 8 + g % (kPerWave / 2) * kWide + in % kWide;
+    py = tile_y * kTile + (wave >> 1) * 8 + g / (kPerWave / 2) * 4 + in / kWide;
+  }
+};
+
+// Where an entry can reach alpha >= 1/255, relative to a centre (ox, oy): the ellipse around (cx, cy) with half extents
+// (ex, ey) along the axes whose boundary at height y is cx + slope (y - cy) -+ wide sqrt(1 - (y - cy)^2 / ey^2), and the
+// disc of radius disc around the centre (0: none).
+struct Footprint {
+  float ox, oy;
+  float cx, cy, ex, ey;
+  float slope, wide, inv_hy, top;  // top: height (relative to cy) of the ellipse's rightmost point; its leftmost is at -top
+  float disc;
+  int state;  // 0: reaches no pixel; 1: no finite bound, every block is kept; 2: test
+};
+
+// hx, hy, hxy: the ellipse { d : d^T [[hx, hxy], [hxy, hy]]^-1 d <= 1 }. One so thin that hxy^2 is within rounding of
+// hx hy (a surfel seen edge-on, its intersections no more accurate than that) is replaced by its bounding box.
+__device__ __forceinline__ void footprint_ellipse(Footprint& f, float hx, float hy, float hxy) {
+#pragma clang fp contract(off)
+  hx = fmaxf(hx, 1e-4f), hy = fmaxf(hy, 1e-4f);
+  f.ex = __builtin_amdgcn_sqrtf(hx), f.ey = __builtin_amdgcn_sqrtf(hy);
+  f.inv_hy = __builtin_amdgcn_rcpf(hy);
+  f.slope  = hxy * f.inv_hy;
+  const float wide2 = hx - hxy * f.slope;
+  f.wide = __builtin_amdgcn_sqrtf(fmaxf(wide2, 0.0f));
+  f.top  = hxy * __builtin_amdgcn_rcpf(f.ex);
+  if (!(wide2 > 1e-5f * hx)) f.slope = 0.0f, f.wide = f.ex, f.inv_hy = 0.0f;
+}
+
+// The blocks of the tile whose pixel centres' hull meets the footprint. Per row of blocks (a slab of heights) the
+// ellipse's extent along x is exact: its right (left) boundary is highest at `top` (-top), or at the slab's nearer edge.
+// Against rounding the footprint is grown by 1/8 pixel and 0.5 % of its extent, as the other bounds are.
+template <int kLanes>
+__device__ __forceinline__ unsigned footprint_blocks(const Footprint& f, int tile_px, int tile_py) {
+#pragma clang fp contract(off)
+  using Shape = BlockShape<kLanes>;
+  constexpr unsigned kAll = (unsigned) ((1ull << Shape::kPerTile) - 1ull);
+  constexpr float kWidth = (float) Shape::kWide, kCols = (float) Shape::kColumns;
+  if (f.state != 2) return f.state == 1 ? kAll : 0u;
+  const float padx = kCullPad + 0.01f * f.ex, pady = kCullPad + 0.01f * f.ey, r2 = f.disc * f.disc;
+  const float qx = (float) tile_px - f.ox, qy = (float) tile_py - f.oy;  // first pixel of the tile
+  unsigned m = 0u;
+#pragma unroll
+  for (int by = 0; by < 4; ++by) {
+    const float y0 = qy + (float) (4 * by), y1 = y0 + 3.0f;
+    const float lo = y0 - f.cy - pady, hi = y1 - f.cy + pady;
+    const float yr = __builtin_amdgcn_fmed3f(f.top, lo, hi), yl = __builtin_amdgcn_fmed3f(-f.top, lo, hi);
+    const float sr = __builtin_amdgcn_sqrtf(fmaxf(1.0f - yr * yr * f.inv_hy, 0.0f));
+    const float sl = __builtin_amdgcn_sqrtf(fmaxf(1.0f - yl * yl * f.inv_hy, 0.0f));
+    float right = f.cx + (f.slope * yr + f.wide * sr) + padx, left = f.cx + (f.slope * yl - f.wide * sl) - padx;
+    const bool in_ellipse = lo <= f.ey && hi >= -f.ey;
+    right = in_ellipse ? right : -1e30f, left = in_ellipse ? left : 1e30f;
+    const float yd = __builtin_amdgcn_fmed3f(0.0f, y0 - kCullPad, y1 + kCullPad), t = r2 - yd * yd;
+    const float half = __builtin_amdgcn_sqrtf(fmaxf(t, 0.0f)) + kCullPad;
+    right = fmaxf(right, t >= 0.0f ? half : -1e30f), left = fminf(left, t >= 0.0f ? -half : 1e30f);
+    // columns [first, last) whose pixels meet [left, right]
+    const int last  = (int) __builtin_amdgcn_fmed3f(floorf((right - qx) / kWidth) + 1.0f, 0.0f, kCols);
+    const int first = (int) __builtin_amdgcn_fmed3f(ceilf((left - qx - (kWidth - 1.0f)) / kWidth), 0.0f, kCols);
+    const unsigned cols = ((1u << last) - 1u) & (0xffu << first);
+    constexpr int kHalf = Shape::kColumns / 2;  // a quadrant's columns, and its two rows of blocks
+    const int shift = (by >> 1) * 2 * Shape::kPerWave + (by & 1) * kHalf;
+    m |= (cols & ((1u << kHalf) - 1u)) << shift | (cols >> kHalf) << (shift + Shape::kPerWave);
+  }
+  return m;
+}
+
+// A surfel: the perspective image of its tangent plane's ellipse u^2 + v^2 <= tau and the low-pass disc (cull_bounds
+// explains both). `m`: its ray-splat matrix, (ox, oy): its projected centre.
+__device__ __forceinline__ Footprint surfel_footprint(const float* m, float ox, float oy, float opacity) {
+#pragma clang fp contract(off)
+  Footprint f;
+  f.ox = ox, f.oy = oy, f.state = 0;
+  const float oa = 255.0f * opacity;
+  if (!(oa >= 1.0f)) return f;
+  f.state = 1;
+  const float tau = 2.0f * __logf(oa) * 1.0001f + 1e-3f;
+  f.disc = __builtin_amdgcn_sqrtf(0.5f * tau);
+  const float u0 = m[0] - ox * m[6], u1 = m[1] - ox * m[7], u2 = m[2] - ox * m[8];
+  const float v0 = m[3] - oy * m[6], v1 = m[4] - oy * m[7], v2 = m[5] - oy * m[8];
+  const float d  = tau * (m[6] * m[6] + m[7] * m[7]) - m[8] * m[8];
+  if (!((m[8] > 0.0f) && (d < -1e-6f * m[8] * m[8]))) return f;  // reaches the camera plane
+  const float inv = __builtin_amdgcn_rcpf(d), f0 = tau * inv, f2 = -inv;
+  f.cx = f0 * (u0 * m[6] + u1 * m[7]) + f2 * (u2 * m[8]);
+  f.cy = f0 * (v0 * m[6] + v1 * m[7]) + f2 * (v2 * m[8]);
+  const float hx  = f.cx * f.cx - (f0 * (u0 * u0 + u1 * u1) + f2 * (u2 * u2));
+  const float hy  = f.cy * f.cy - (f0 * (v0 * v0 + v1 * v1) + f2 * (v2 * v2));
+  const float hxy = f.cx * f.cy - (f0 * (u0 * v0 + u1 * v1) + f2 * (u2 * v2));
+  if (!(hx < 1e30f) || !(hy < 1e30f) || !(fabsf(hxy) < 1e30f) || !(fabsf(f.cx) < 1e15f) || !(fabsf(f.cy) < 1e15f)) return f;
+  f.state = 2;
+  footprint_ellipse(f, hx, hy, hxy);
+  return f;
+}
+
+template <int kLanes>
+__device__ __forceinline__ unsigned surfel_blocks(const SplatHot& h, int tile_px, int tile_py, int flags) {
+  if (flags & kFlagNoCull) return (unsigned) ((1ull << BlockShape<kLanes>::kPerTile) - 1ull);
+  return footprint_blocks<kLanes>(surfel_footprint(h.m, h.cx, h.cy, h.opacity), tile_px, tile_py);
+}
+
+// Fills the lists of one wavefront from the masks of the batch's staged entries (zero past the last one): list g at
+// lists + g * kEntries, a byte per entry, padded with `kEntries` -- the number of a record that no pixel blends -- to its
+// full length. Blocks without a lane in `lanes` get an empty list. Returns the longest list's length. The LDS serves a
+// wavefront's accesses in order, so no barrier is needed before the lists are read.
+template <int kLanes, int kEntries>
+__device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lists, const unsigned* masks, int wave,
+                                                 unsigned long long lanes) {
+  static_assert(kEntries % kWave == 0 && kEntries < 256, "entry numbers and the padding are bytes");
+  constexpr int kPerWave = BlockShape<kLanes>::kPerWave;
+  const int lane = __lane_id();
+  constexpr unsigned kFill = 0x01010101u * (unsigned) kEntries;
+  uint2* fill = (uint2*) lists;
+#pragma unroll
+  for (int e = 0; e < kPerWave * kEntries / 8; e += kWave) fill[e + lane] = make_uint2(kFill, kFill);
+  unsigned m[kEntries / kWave];
+#pragma unroll
+  for (int c = 0; c < kEntries / kWave; ++c) m[c] = masks[c * kWave + lane] >> (kPerWave * wave);
+  int longest = 0;
+#pragma unroll
+  for (int g = 0; g < kPerWave; ++g) {
+    if ((lanes >> (g * kLanes) & ((1ull << kLanes) - 1ull)) == 0ull) continue;
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kEntries / kWave; ++c) {
+      const bool on = (m[c] & (1u << g)) != 0u;
+      const unsigned long long who = wave_ballot(on);
+      const int at = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned) who, n));
+      if (on) lists[g * kEntries + at] = (unsigned char) (c * kWave + lane);
+      n += (int) __popcll(who);
+    }
+    longest = max(longest, n);
+  }
+  return longest;
+}
+
+// Walks the lists of a wavefront: `load(j)` requests the record of entry j, `work(record, j)` evaluates it and `more()`
+// says whether any lane still blends. A wavefront walks alone, so what it would wait for sits on the tile's critical path: the
+// record of the next entry is requested before the present one is evaluated, into alternating registers, and the entry
+// numbers four at a time one step of four ahead. (Reads up to four bytes past the list: numbers of another list, or the
+// padding behind the last one; they are loaded but never evaluated.)
+template <typename Load, typename Work, typename More>
+__device__ __forceinline__ void walk_block_list(const unsigned char* __restrict__ list, int steps, Load load, Work work,
+                                                More more) {
+  if (steps == 0) return;
+  const unsigned* four = (const unsigned*) list;
+  unsigned now = four[0];
+  auto rec_a = load((int) (now & 255u));
+  for (int i = 0;; i += 4) {
+    const unsigned next = four[(i >> 2) + 1];
+    {
+      auto rec_b = load((int) (now >> 8 & 255u));
+      work(rec_a, (int) (now & 255u));
+      if (i + 1 >= steps || !more()) return;
+      rec_a = load((int) (now >> 16 & 255u));
+      work(rec_b, (int) (now >> 8 & 255u));
+      if (i + 2 >= steps || !more()) return;
+    }
+    {
+      auto rec_b = load((int) (now >> 24));
+      work(rec_a, (int) (now >> 16 & 255u));
+      if (i + 3 >= steps || !more()) return;
+      rec_a = load((int) (next & 255u));
+      work(rec_b, (int) (now >> 24));
+      if (i + 4 >= steps || !more()) return;
+    }
+    now = next;
+  }
+}
+
+}  // namespace fsgs
