@@ -488,39 +488,50 @@ __device__ __forceinline__ float cross_row_sum(float z) {
 #endif
 }
 
-// Sums 16 per-lane values over the 64 lanes at once ("transposed" butterfly): each step halves the number of live
-// registers while doubling the lanes a partial covers, so 16 wave-wide sums cost 15 merge steps (2 DPP adds + 1 select
-// each) plus two cross-row exchanges, instead of 16 x 6 dependent DPP adds. On return every lane holds the wave total of
-// v[lane & 15].
-// On return lane l of every 16-lane row holds that ROW's total of v[l & 15].
+// Sums 16 per-lane values over each 16-lane row at once ("transposed" butterfly): every step halves the number of live
+// registers while doubling the lanes a partial covers, 15 merges in all. On return lane l of every row holds that row's
+// total of v[l & 15]. A merge of a and b leaves a's sum over the lane and its partner in one half of the lanes, b's in the
+// other. Where the halves are whole banks of four lanes (partners 8 and 4 apart) the second addition writes its own banks
+// only, two instructions a merge; where they are not, both sums are formed and one is selected, three. (Selecting in all
+// four steps: 45 instructions; this: 33.) The masked additions are inline assembly, for the compiler knows no masked
+// result; the s_nop keep the two wait states between a register's write and its use by a DPP instruction, which the
+// compiler does not count across inline assembly.
 __device__ __forceinline__ float row_sum16_transposed(const float (&v)[16]) {
   // no contraction: an input that is a product would otherwise be formed twice, as a multiply for the shifted operand
   // and again inside a fused multiply-add for the lane's own, in place of one multiply and one DPP add
 #pragma clang fp contract(off)
   const int lane = __lane_id();
-  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+  const bool b0 = lane & 1, b1 = lane & 2;
   float w[8], x[4], y[2];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float a = v[2 * i + 1] + dpp_shift_zero<0x111, 0xf, 0xf>(v[2 * i + 1]);  // row_shr:1, kept by odd lanes
-    const float b = v[2 * i] + dpp_shift_zero<0x101, 0xf, 0xf>(v[2 * i]);          // row_shl:1, kept by even lanes
-    w[i] = b0 ? a : b;
-  }
+  for (int i = 0; i < 8; ++i) w[i] = v[i] + dpp_shift_zero<0x128, 0xf, 0xf>(v[i]);  // row_ror:8
+#define FSGS_MASKED_ADD(D, S, HOW) "v_add_f32_dpp " D ", " S ", " S " " HOW "\n\t"
+#define FSGS_ROR8 "row_ror:8 row_mask:0xf bank_mask:0xc"
+#define FSGS_SHR4 "row_shr:4 row_mask:0xf bank_mask:0xa"
+  asm volatile("s_nop 1\n\t" FSGS_MASKED_ADD("%0", "%8", FSGS_ROR8) FSGS_MASKED_ADD("%1", "%9", FSGS_ROR8)
+               FSGS_MASKED_ADD("%2", "%10", FSGS_ROR8) FSGS_MASKED_ADD("%3", "%11", FSGS_ROR8)
+               FSGS_MASKED_ADD("%4", "%12", FSGS_ROR8) FSGS_MASKED_ADD("%5", "%13", FSGS_ROR8)
+               FSGS_MASKED_ADD("%6", "%14", FSGS_ROR8) FSGS_MASKED_ADD("%7", "%15", FSGS_ROR8) "s_nop 1"
+               : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7])
+               : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = w[2 * i + 1] + dpp_shift_zero<0x112, 0xf, 0xf>(w[2 * i + 1]);  // row_shr:2
-    const float b = w[2 * i] + dpp_shift_zero<0x102, 0xf, 0xf>(w[2 * i]);          // row_shl:2
-    x[i] = b1 ? a : b;
-  }
+  for (int i = 0; i < 4; ++i) x[i] = w[i] + dpp_shift_zero<0x104, 0xf, 0xf>(w[i]);  // row_shl:4
+  asm volatile("s_nop 1\n\t" FSGS_MASKED_ADD("%0", "%4", FSGS_SHR4) FSGS_MASKED_ADD("%1", "%5", FSGS_SHR4)
+               FSGS_MASKED_ADD("%2", "%6", FSGS_SHR4) FSGS_MASKED_ADD("%3", "%7", FSGS_SHR4) "s_nop 1"
+               : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+               : "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]));
+#undef FSGS_MASKED_ADD
+#undef FSGS_ROR8
+#undef FSGS_SHR4
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const float a = x[2 * i + 1] + dpp_shift_zero<0x114, 0xf, 0xf>(x[2 * i + 1]);  // row_shr:4
-    const float b = x[2 * i] + dpp_shift_zero<0x104, 0xf, 0xf>(x[2 * i]);          // row_shl:4
-    y[i] = b2 ? a : b;
+    const float a = x[i + 2] + dpp_shift_zero<0x112, 0xf, 0xf>(x[i + 2]);  // row_shr:2, kept by lanes with bit 1
+    const float b = x[i] + dpp_shift_zero<0x102, 0xf, 0xf>(x[i]);          // row_shl:2
+    y[i] = b1 ? a : b;
   }
-  const float a = y[1] + dpp_shift_zero<0x118, 0xf, 0xf>(y[1]);  // row_shr:8
-  const float b = y[0] + dpp_shift_zero<0x108, 0xf, 0xf>(y[0]);  // row_shl:8
-  return b3 ? a : b;
+  const float a = y[1] + dpp_shift_zero<0x111, 0xf, 0xf>(y[1]);  // row_shr:1
+  const float b = y[0] + dpp_shift_zero<0x101, 0xf, 0xf>(y[0]);  // row_shl:1
+  return b0 ? a : b;
 }
 __device__ __forceinline__ float wave_sum16_transposed(const float (&v)[16]) {
   return cross_row_sum(row_sum16_transposed(v));

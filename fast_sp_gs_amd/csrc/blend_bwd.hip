@@ -5,26 +5,18 @@
 // tile's list backwards, gradient channels consumed are image, opacity, aux 0-5 (depth, normal, median depth,
 // distortion) and optional flow; the 0.99 alpha clamp is not masked in the gradient, as in the reference.
 //
-// Where the reference issues 18-21 global float atomics per (pixel, surfel) pair, this kernel splits the work of a pair
-// into the part that depends on the order of the pixel's list and the part that does not:
-//   1. order-bound, one wavefront per 8x8 pixel quadrant, one list entry per pass: the ray-splat intersection and the
-//      pixel's back-to-front recurrences. A pixel that blends the entry leaves three numbers (blend weight,
-//      G * dL/dalpha, dL/ddepth) and its (pixel, entry) pair in the wavefront's queue in LDS. Few lanes of a pass blend
-//      (a quarter on the benchmark scene), so this part is kept as short as the recurrences allow.
-//   2. order-free, all 64 lanes busy: the wavefront takes 64 queued pairs at a time -- an entry's pairs padded to a
-//      16-lane row -- recomputes the two planes through the pixel from the staged record, forms the 16 + 2 gradient
-//      components and sums them over each row with DPP row shifts (no LDS traffic); each row adds its 16 totals to the
-//      entry's row of the wavefront's accumulator in LDS.
-//   3. per staged batch the four wavefronts' accumulators are added in wavefront order and every staged (surfel, tile)
-//      instance writes one record at its position in surfel order; slot_reduce_kernel sums a surfel's records in a
-//      fixed order. (Without scan offsets: one global atomic per surfel, component and tile, as the reference's sums.)
-// Surfels behind the deepest contributor of the whole tile are never gathered. The optical-flow instantiation keeps
-// parts 1 and 2 in one pass per entry (its extra per-pair terms would double the queue record).
+// Where the reference issues 18-21 global float atomics per (pixel, surfel) pair, a 16-lane row of a wavefront owns a 4x4
+// block of pixels, walks its own list of the staged surfels that reach it (block_lists.hpp) and sums an entry's components
+// over its pixels with DPP row shifts; per staged batch the sums of a tile's 16 rows are added in row order, and every staged
+// (surfel, tile) instance writes one record at its position in surfel order; slot_reduce_kernel or the preprocess backward
+// sums a surfel's records in a fixed order. (Without scan offsets: one global atomic per surfel, component and tile.)
+// Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
+// the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
+// 1170 -> 950, 10k 256x256 58 -> 40.
 #include <algorithm>
 
-#include "blend.hpp"
+#include "block_lists.hpp"
 #include "instance_slots.hpp"
-#include "pair_queue.hpp"
 
 namespace fsgs {
 namespace {
@@ -33,19 +25,9 @@ namespace {
 // The first 16 go through one transposed row reduction; the means2D pair is only non-zero for pixels where the
 // screen-space low-pass filter wins (rho2d < rho3d) and is reduced separately when any lane took that branch.
 constexpr int kGradSlots = 18;
-#ifndef FSGS_BWD_BATCH
-#define FSGS_BWD_BATCH 64
-#endif
 #ifndef FSGS_BWD_WAVES
 #define FSGS_BWD_WAVES 4
 #endif
-constexpr int kBwdBatch = FSGS_BWD_BATCH;  // surfels staged per round
-static_assert(kBwdBatch == kWave, "one wavefront stages a batch, another flushes it, and a queued pair names its entry in 6 bits");
-// the two-pass form (queue of blended pairs per wavefront, pair_queue.hpp) can be switched off at build time
-#ifndef FSGS_BWD_QUEUE
-#define FSGS_BWD_QUEUE 1
-#endif
-constexpr bool kBwdQueue = FSGS_BWD_QUEUE != 0;
 
 template <bool kAux, bool kFlow, bool kSlots>
 __global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(FSGS_BWD_WAVES, FSGS_BWD_WAVES)))
@@ -59,30 +41,26 @@ blend_backward_kernel(
     float* __restrict__ g_normal_opacity, float* __restrict__ g_colors, float* __restrict__ g_trans,
     SlotSource slots, const int32_t* __restrict__ radii, float* __restrict__ slot_grads,
     const float4* __restrict__ records) {
-  constexpr bool kQueue = kBwdQueue && !kFlow;
   // First record slot of a surfel; `stored` is what its packed record says (-1: packed before the offsets were known).
   auto first_slot = [&](int id, int64_t stored) -> int64_t {
     if (slots.region) return (stored >= 0 ? stored : (int64_t) slots.offset[id]) + slots.region[slot_region(id)];
     return stored >= 0 ? stored : (id == 0 ? 0 : slots.scan[id - 1]);
   };
-  __shared__ SplatHot s_hot[kBwdBatch];
-  __shared__ SplatCold s_cold[kBwdBatch];
-  // Each wavefront's sums over its 64 pixels, one row per staged surfel; the flush adds the four rows in wavefront
-  // order, so a tile's sums do not depend on timing. +1: the odd stride keeps the flush free of bank conflicts.
-  __shared__ float s_part[4][kBwdBatch][kGradSlots + 1];
-  // Where a staged (surfel, tile) instance's sums go: its position in surfel order (kSlots) or the surfel's id. Two
-  // copies by batch parity: wavefront 1 stages batch b + 1 while wavefront 0 still flushes batch b.
-  __shared__ int s_slot[2][kBwdBatch];
-  __shared__ float s_t2[kFlow ? kBwdBatch * 9 : 1];
+  using Shape = BlockShape<16>;
+  __shared__ Splat s_splat[kRowBatch + 1];  // the last one is what padding names: no pixel blends it
+  __shared__ float s_t2[kFlow ? kRowBatch * 9 : 1];
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kRowSteps + 16];
+  __shared__ float s_sum[16][kRowSteps][kGradSlots];
+  // What the flush of a batch reads is kept twice, by batch parity: the next batch is staged while others still flush.
+  __shared__ unsigned s_mask[2][kRowMasks];  // which 4x4 blocks of the tile each staged surfel can reach
+  __shared__ uint4 s_rank[2][kRowBatch];     // at which step each of the 16 rows meets it
+  __shared__ int s_slot[2][kRowBatch];       // where its sums go: its position in surfel order (kSlots) or the surfel's id
   __shared__ int s_max_contrib;
-  __shared__ unsigned char s_mask[kBwdBatch];  // which 8x8 quadrants of the tile each staged surfel can reach
-  // queued pairs
-  __shared__ float4 s_queue[kQueue ? 4 : 1][kQueue ? kQueueItems : 1];
 
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int tile = scheduled_tile(ordered, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW   = (size_t) H * W;
   const size_t pix  = (size_t) W * py + px;
@@ -96,14 +74,17 @@ blend_backward_kernel(
   // deepest list position any pixel of the tile blended: nothing behind it needs to be gathered
   if (threadIdx.x == 0) s_max_contrib = 0;
   __syncthreads();
-  int wave_max_contrib = last_contrib;  // deepest position blended by this wavefront's quadrant
+  int row_max = last_contrib;  // deepest position blended in this lane's 4x4 block
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) wave_max_contrib = max(wave_max_contrib, __shfl_xor(wave_max_contrib, d, kWave));
-  if (lane == 0) atomicMax(&s_max_contrib, wave_max_contrib);
-  for (int e = threadIdx.x; e < 4 * kBwdBatch * (kGradSlots + 1); e += kBlendThreads) (&s_part[0][0][0])[e] = 0.0f;
+  for (int d = 8; d >= 1; d >>= 1) row_max = max(row_max, __shfl_xor(row_max, d, kWave));
+  int row_last[4];  // the same of the wavefront's four blocks
+#pragma unroll
+  for (int r = 0; r < 4; ++r) row_last[r] = __builtin_amdgcn_readlane(row_max, 16 * r);
+  if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
+  if (threadIdx.x == 0) s_splat[kRowBatch] = Splat{};  // all zero: p_z == 0 everywhere
+  if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kRowSteps])[threadIdx.x] = 0u;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));  // positions [0, n_todo) of the tile's list, walked from n_todo-1 down to 0
-  const int rounds = (n_todo + kBwdBatch - 1) / kBwdBatch;
   // No zero fill of the records: the instances behind the tile's deepest contributor are never staged, their records
   // are cleared here; every staged instance writes its record at the flush, zeros included
   if (kSlots) {
@@ -164,21 +145,17 @@ blend_backward_kernel(
   float acc_lin = 0;
   float last_alpha = 0, acc_w = 0;
   float acc_f0 = 0, acc_f1 = 0, last_f0 = 0, last_f1 = 0;
-  PairQueue q;                                 // the wavefront's queue of blended pairs
-  const int row_shift = (lane >> 4) * 8;       // this lane's byte of the four rows of a pass
-  const float qx0 = (float) (tile_x * kTile + (wave & 1) * 8), qy0 = (float) (tile_y * kTile + (wave >> 1) * 8);
 
   Splat next;
   float next_t2[9];
   int next_radius = 0;
   int64_t next_off = 0;
-  // Gathering and staging are wavefront 1's job, the flush of a finished batch wavefront 0's: both sit between the same
-  // two barriers, where the other wavefronts wait, and so run side by side instead of one after the other.
-  const int st = (int) threadIdx.x - kWave;  // staging slot of this lane (wavefront 1: 0 .. 63)
-  if (st >= 0 && st < min(n_todo, kBwdBatch)) {
+  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  auto gather = [&](int done) {
+    const int e = (int) threadIdx.x;
+    if (e >= min(kRowBatch, n_todo - done)) return;
     SplatExtra ex;
-    next = gather_splat(point_list[r0 + (n_todo - 1 - st)], means2D, colors, normal_opacity, trans_mat,
-                        records, &ex);
+    next = gather_splat(point_list[r0 + (n_todo - 1 - done - e)], means2D, colors, normal_opacity, trans_mat, records, &ex);
     if (kFlow)
 #pragma unroll
       for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
@@ -188,52 +165,48 @@ blend_backward_kernel(
       next_radius = records && ex.radius >= 0 ? ex.radius : radii[next.cold.id];
       next_off    = first_slot(next.cold.id, records ? ex.offset : -1);
     }
-  }
+  };
+  gather(0);
 
-  for (int b = 0; b < rounds; ++b) {
-    const int n_here = min(kBwdBatch, n_todo - b * kBwdBatch);
-    if (st >= 0 && st < n_here) {
-      s_hot[st]  = next.hot;
-      s_cold[st] = next.cold;
-      s_mask[st] = (unsigned char) quadrant_mask(next.hot, tile_x * kTile, tile_y * kTile, ordered);
-      if (kFlow)
+  for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    const int n_staged = min(kRowBatch, n_todo - done);
+    if ((int) threadIdx.x < kRowMasks) {
+      const int e = (int) threadIdx.x;
+      unsigned mask = 0u;
+      if (e < n_staged) {
+        s_splat[e] = next;
+        mask = surfel_blocks<16>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
+        if (kFlow)
 #pragma unroll
-        for (int k = 0; k < 9; ++k) s_t2[st * 9 + k] = next_t2[k];
-      if (kSlots) {
-        // position of this instance in the surfel-ordered key list: the binning emits a surfel's tiles row-major
-        // over its rectangle, starting at the surfel's prefix-scan offset (gaussian_prepare.cu:47-83)
-        const TileRect r = tile_rect(next.hot.cx, next.hot.cy, next_radius, gx, gy);
-        s_slot[b & 1][st] = (int) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
-      } else {
-        s_slot[b & 1][st] = next.cold.id;
+          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
+        if (kSlots) {
+          // position of this instance in the surfel-ordered key list: the binning emits a surfel's tiles row-major
+          // over its rectangle, starting at the surfel's prefix-scan offset (gaussian_prepare.cu:47-83)
+          const TileRect r = tile_rect(next.hot.cx, next.hot.cy, next_radius, gx, gy);
+          s_slot[parity][e] = (int) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
+        } else {
+          s_slot[parity][e] = next.cold.id;
+        }
+        s_rank[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
       }
+      s_mask[parity][e] = mask;
     }
     __syncthreads();
-    const int nxt = (b + 1) * kBwdBatch + st;
-    if (st >= 0 && st < kBwdBatch && nxt < n_todo) {
-      SplatExtra ex;
-      next = gather_splat(point_list[r0 + (n_todo - 1 - nxt)], means2D, colors, normal_opacity, trans_mat, records,
-                          &ex);
-      if (kFlow)
-#pragma unroll
-        for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
-      if (kSlots) {
-        next_radius = records && ex.radius >= 0 ? ex.radius : radii[next.cold.id];
-        next_off    = first_slot(next.cold.id, records ? ex.offset : -1);
-      }
-    }
-
-    // Work list of this wavefront for the staged surfels: those that can reach its quadrant and are not behind its
-    // deepest contributor; consumed bit by bit with scalar instructions.
-    unsigned long long todo = __ballot(lane < n_here && ((s_mask[lane] >> wave) & 1u) &&
-                                       (n_todo - 1 - (b * kBwdBatch + lane)) < wave_max_contrib);
+    const unsigned masks[2] = {s_mask[parity][lane], s_mask[parity][kWave + lane]};
+    const int n_here = row_batch(masks, n_staged);
+    gather(done + n_here);
+    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+    const int behind = n_todo - done;
+    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+    const int steps = build_row_lists(&s_list[4 * kRowSteps * wave], (unsigned char*) s_rank[parity], masks, wave, first, n_here);
+    const int my_first = behind - last_contrib, my_median = behind - median_contrib;
     // ---- order-bound part of one (pixel, entry) pair: advances the pixel's back-to-front state -------------------------
     // All channels that enter the image linearly (colour, depth, opacity, normal) share one recurrence: with
     // c = <upstream gradient, channel values of this surfel>, the reference's per-channel accumulators
     // acc_x = last_alpha * last_x + (1 - last_alpha) * acc_x contract to a single scalar, updated at the end of the
     // pair that supplies alpha and x. Leaves the blend weight w, dL/dalpha and dL/ddepth of the pair; call under `hit`
     // only.
-    auto advance_pixel = [&](const SplatCold& cold, int pos, const Hit& h, float& w, float& dL_dalpha, float& dL_dz) {
+    auto advance_pixel = [&](const SplatCold& cold, int j, const Hit& h, float& w, float& dL_dalpha, float& dL_dz) {
       const float keep = 1.0f - h.alpha;
       T = T * __builtin_amdgcn_rcpf(keep);
       w = h.alpha * T;
@@ -250,7 +223,7 @@ blend_backward_kernel(
         c_lin = fmaf(cold.nx, dLn0, fmaf(cold.ny, dLn1, fmaf(cold.nz, dLn2, c_lin)));
         // dL/ddepth: through the distortion's normalised depth, the depth map, and the median depth
         const float per_w = fmaf(fmaf(m_d, reg_2A, -reg_2D), dmd_dd, dL_ddepth);
-        dL_dz = fmaf(w, per_w, pos == median_contrib - 1 ? dL_dmedian : 0.0f);
+        dL_dz = fmaf(w, per_w, j == my_median ? dL_dmedian : 0.0f);
       } else {
         c_lin = 0.0f;
       }
@@ -259,127 +232,16 @@ blend_backward_kernel(
       dL_dalpha = c_lin - acc_lin;
       acc_lin   = fmaf(keep, acc_lin, h.alpha * c_lin);
     };
-    if (kQueue) {
-      // ---- order-free part: 64 queued pairs at a time, four 16-lane rows, every row one entry ---------------------------
-      // A lane rebuilds the two planes through its pair's pixel from the staged record and forms the 16 + 2 components
-      // as products of the three queued numbers with quantities that are finite in every lane (padding items carry
-      // zeros and no flags, and the reciprocal of p_z is only taken under the pair's flags), so no component needs a
-      // zero of its own; the projected-centre case is the intersection case with a zero in place of 1 / p_z.
-      auto drain = [&](int n_valid) {
-        // the entries of the four rows come from the wavefront's scalar bookkeeping, so the queued item, the staged
-        // record and the accumulator row are requested together (one LDS round trip instead of three in a chain)
-        const unsigned jrows = queue_front_rows(q);  // byte r = entry of row r
-        const int j = (int) ((jrows >> row_shift) & 63u);
-        const float4 it = s_queue[wave][q.head + lane];
-        const SplatHot hot = s_hot[j];
-        float* const acc = &s_part[wave][j][lane & 15];
-        const float before = *acc;
-        const int bits = __float_as_int(it.w);
-        const int qp = bits & 63;
-        const bool blends = (bits & kItemHit) != 0, by_ray = (bits & kItemRay) != 0;
-        // the upstream gradients of the pair's pixel sit in the registers of the lane that owns it (lane qp of this
-        // wavefront): fetched with lane permutes, no LDS copy of them is kept
-        auto from_owner = [&](float v) {
-          return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(qp << 2, __builtin_bit_cast(int, v)));
-        };
-        const float up_x = from_owner(dLp0), up_y = from_owner(dLp1), up_z = from_owner(dLp2);
-        const float fx = qx0 + (float) (qp & 7), fy = qy0 + (float) (qp >> 3);
-        const float w = it.x, GdA = it.y, dL_dz = it.z;
-        const float kx = fx * hot.m[6] - hot.m[0], ky = fx * hot.m[7] - hot.m[1], kz = fx * hot.m[8] - hot.m[2];
-        const float lx = fy * hot.m[6] - hot.m[3], ly = fy * hot.m[7] - hot.m[4], lz = fy * hot.m[8] - hot.m[5];
-        const float p_x = ky * lz - kz * ly, p_y = kz * lx - kx * lz, p_z = kx * ly - ky * lx;
-        const float rz_s = blends ? __builtin_amdgcn_rcpf(p_z) : 0.0f;  // s is used by both cases of a blending pair
-        const float rz_p = by_ray ? rz_s : 0.0f;                         // d/dp only by the intersection case
-        const float sx = p_x * rz_s, sy = p_y * rz_s;
-        const float oG = hot.opacity * GdA;
-        float dsx = -(oG * sx), dsy = -(oG * sy);
-        if (kAux) dsx += dL_dz * hot.m[6], dsy += dL_dz * hot.m[7];
-        const float s_ds = dsx * sx + dsy * sy;
-        // d/dp of the homogeneous intersection point p = k x l, negated (the components below are minus the plane
-        // gradients): p_xy = s p_z, so dp_xy = ds / p_z and dp_z = -<ds, s> / p_z
-        const float npx = -(dsx * rz_p), npy = -(dsy * rz_p), npz = s_ds * rz_p;
-        float g[16];
-        g[0] = w * up_x, g[1] = w * up_y, g[2] = w * up_z;
-        g[3] = ly * npz - lz * npy, g[4] = lz * npx - lx * npz, g[5] = lx * npy - ly * npx;
-        g[6] = npy * kz - npz * ky, g[7] = npz * kx - npx * kz, g[8] = npx * ky - npy * kx;
-        g[9]  = dL_dz * sx - (fx * g[3] + fy * g[6]);
-        g[10] = dL_dz * sy - (fx * g[4] + fy * g[7]);
-        g[11] = dL_dz - (fx * g[5] + fy * g[8]);
-        if (kAux) {
-          g[12] = w * from_owner(dLn0), g[13] = w * from_owner(dLn1), g[14] = w * from_owner(dLn2);
-        } else {
-          g[12] = g[13] = g[14] = 0.0f;
-        }
-        g[15] = GdA;
-        // lane (row, c) holds the row's total of component c
-        queue_accumulate(acc, before, row_sum16_transposed(g), jrows, n_valid, true);
-        const bool filtered = blends && !by_ray;
-        if (wave_ballot(filtered) != 0ull) {  // some pair met its surfel by the projected centre
-          const float to_centre = filtered ? -2.0f * oG : 0.0f;
-          float cx = to_centre * (hot.cx - fx), cy = to_centre * (hot.cy - fy);  // totals of a row end up in its lane 15
-          cx += dpp_shift_zero<0x111, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x111, 0xf, 0xf>(cy);
-          cx += dpp_shift_zero<0x112, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x112, 0xf, 0xf>(cy);
-          cx += dpp_shift_zero<0x114, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x114, 0xf, 0xf>(cy);
-          cx += dpp_shift_zero<0x118, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x118, 0xf, 0xf>(cy);
-          if ((lane >> 4) < ((n_valid + 15) >> 4) && (lane & 15) == 15)
-            atomicAdd(&s_part[wave][j][16], cx), atomicAdd(&s_part[wave][j][17], cy);
-        }
-        queue_pop(q, n_valid);
-      };
-      // ---- order-bound part of one entry, and the append of its blending pixels to the queue -----------------------------
-      auto queue_entry = [&](const SplatHot& hot, const SplatCold& cold, int j) {
-        const int pos = n_todo - 1 - (b * kBwdBatch + j);  // 0-based position in the tile's list
-        Hit h;
-        unsigned long long pass;
-        const bool hit = intersect_flat(hot, pxf, pyf, near_n, h, &pass) && (pos < last_contrib);
-        pass &= wave_ballot(pos < last_contrib);
-        if (pass == 0ull) return;  // wave-uniform: nobody in this quadrant blends the surfel
-        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f;
-        if (hit) {
-          advance_pixel(cold, pos, h, w, dL_dalpha, dL_dz);
-          dL_dalpha *= T * h.G;  // only G * dL/dalpha is ever used
-        }
-        const int flags = h.rho3d <= h.rho2d ? (kItemHit | kItemRay) : kItemHit;
-        if (queue_append(s_queue[wave], q, j, hit, pass, w, dL_dalpha, dL_dz, flags)) drain(kWave);
-      };
-      if (todo != 0ull) {
-        auto pop = [&]() {
-          const int j = __builtin_ctzll(todo);
-          todo &= todo - 1;
-          return j;
-        };
-        auto peek = [&]() { return todo ? (int) __builtin_ctzll(todo) : 0; };
-        SplatHot hot_a = s_hot[peek()], hot_b;
-        while (todo) {
-          {
-            const int j = pop();
-            hot_b       = s_hot[peek()];
-            const SplatCold cold = s_cold[j];
-            __builtin_amdgcn_sched_barrier(0);
-            queue_entry(hot_a, cold, j);
-          }
-          if (todo == 0ull) break;
-          {
-            const int j = pop();
-            hot_a       = s_hot[peek()];
-            const SplatCold cold = s_cold[j];
-            __builtin_amdgcn_sched_barrier(0);
-            queue_entry(hot_b, cold, j);
-          }
-        }
-        if (q.count > 0) drain(q.count);  // the staged records are replaced after the next barrier
-      }
-    } else {
-     // Gradient terms of one (pixel, entry) pair, formed in the pass that advances the pixel. The part under `hit` leaves
+     // Gradient terms of one (pixel, entry) pair. The part under `hit` leaves
      // a few factors (zero for a lane whose pixel does not blend the entry); the 16 + 2 per-surfel components are
      // products of those factors with quantities that are finite in every lane, formed by all lanes alike, so no
      // component needs a zero of its own and the two ways a surfel is met (ray-splat intersection / projected centre)
      // share one instruction stream.
-     auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, int pos, const Hit& h, bool hit,
-                               float (&g)[16], float& g2x, float& g2y, unsigned long long& ray_lanes) {
+     auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, const Hit& h, bool hit,
+                               float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
        if (hit) {
-         advance_pixel(cold, pos, h, w, dL_dalpha, dL_dz);
+         advance_pixel(cold, j, h, w, dL_dalpha, dL_dz);
          if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
          if (kFlow) {
            const float* Q = &s_t2[j * 9];
@@ -411,7 +273,7 @@ blend_backward_kernel(
        }
        const bool by_ray   = h.rho3d <= h.rho2d;
        const bool filtered = hit && !by_ray;
-       ray_lanes           = wave_ballot(by_ray);  // taken where the comparison is made: its own lane mask, no instruction
+       filtered_lanes      = ~wave_ballot(by_ray);  // taken where the comparison is made: its own lane mask, no instruction
        // d/dp of the homogeneous intersection point p = k x l, negated (the components below are minus the plane
        // gradients): p_xy = s p_z, so dp_xy = ds / p_z and dp_z = -<ds, s> / p_z
        const float rz  = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
@@ -430,97 +292,76 @@ blend_backward_kernel(
        const float to_centre = filtered ? hot.opacity * dL_dalpha * (-2.0f * h.G) : 0.0f;
        g2x = to_centre * h.dx, g2y = to_centre * h.dy;
      };
-     auto backward_entry = [&](const SplatHot& hot, const SplatCold& cold, int j) {
-      const int pos = n_todo - 1 - (b * kBwdBatch + j);  // 0-based position in the tile's list
+     float* const sums = &s_sum[4 * wave + (lane >> 4)][0][lane & 15];         // component lane & 15 of step 0
+     float* const centre = &s_sum[4 * wave + (lane >> 4)][0][16 + (lane >> 3 & 1)];  // lanes 0 and 8 of a row: means2D
+     auto backward_entry = [&](const SplatHot& hot, int j, int i) {
+      const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+      __builtin_amdgcn_sched_barrier(0);
       Hit h;
-      unsigned long long pass;
-      const bool hit = intersect_flat(hot, pxf, pyf, near_n, h, &pass) && (pos < last_contrib);
-      pass &= wave_ballot(pos < last_contrib);
-      if (pass == 0ull) return;  // wave-uniform: nobody in this quadrant blends the surfel
-
-      float g[16], g2x, g2y;
-      unsigned long long ray_lanes;
-      pair_gradients(hot, cold, j, pos, h, hit, g, g2x, g2y, ray_lanes);
-      const float tot = wave_sum16_transposed(g);
-      if (lane < 16) s_part[wave][j][lane] = tot;  // a wavefront meets an entry once per batch: a plain store
-      if ((pass & ~ray_lanes) != 0ull) {  // some lane met the surfel by its projected centre
-        const float sx = wave_sum_to_lane63(g2x), sy = wave_sum_to_lane63(g2y);
-        if (lane == 63) s_part[wave][j][16] = sx, s_part[wave][j][17] = sy;
+      unsigned long long pass, filtered = 0ull;
+      intersect_flat(hot, pxf, pyf, near_n, h, &pass);
+      pass &= wave_ballot(j >= my_first);
+      float tot = 0.0f, mid = 0.0f;
+      if (pass != 0ull) {
+        float g[16], g2x, g2y;
+        pair_gradients(hot, cold, j, h, __builtin_amdgcn_inverse_ballot_w64(pass), g, g2x, g2y, filtered);
+        tot = row_sum16_transposed(g);
+        if ((pass & filtered) != 0ull) {  // some lane met the surfel by its projected centre
+          g2x += dpp_shift_zero<0x128, 0xf, 0xf>(g2x), g2y += dpp_shift_zero<0x128, 0xf, 0xf>(g2y);  // row_ror:8
+          mid = (lane & 8) ? g2y : g2x;
+          mid += dpp_shift_zero<0x104, 0xf, 0xf>(mid);  // row_shl:4, 2, 1: totals in lanes 0 and 8
+          mid += dpp_shift_zero<0x102, 0xf, 0xf>(mid);
+          mid += dpp_shift_zero<0x101, 0xf, 0xf>(mid);
+        }
       }
+      sums[i * kGradSlots] = tot;  // zeros, too, have their place
+      if ((lane & 7) == 0) centre[i * kGradSlots] = mid;
      };
-     // The record of the next entry is requested before the current one is evaluated (alternating registers): a
-     // wavefront walks its list alone, so an exposed LDS round trip per entry sits on the tile's critical path.
-     if (todo != 0ull) {
-      auto pop = [&]() {
-        const int j = __builtin_ctzll(todo);
-        todo &= todo - 1;
-        return j;
-      };
-      auto peek = [&]() { return todo ? (int) __builtin_ctzll(todo) : 0; };
-      SplatHot hot_a = s_hot[peek()], hot_b;
-      while (todo) {
-        {
-          const int j = pop();
-          hot_b       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];
-          __builtin_amdgcn_sched_barrier(0);
-          backward_entry(hot_a, cold, j);
-        }
-        if (todo == 0ull) break;
-        {
-          const int j = pop();
-          hot_a       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];
-          __builtin_amdgcn_sched_barrier(0);
-          backward_entry(hot_b, cold, j);
-        }
-      }
-     }
-    }
+     walk_block_list(&s_list[(4 * wave + (lane >> 4)) * kRowSteps], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
+                     [] { return true; });
     __syncthreads();
-    // flush the batch (wavefront 0: lane = staged surfel), adding the four wavefronts' rows in wavefront order
-    if ((int) threadIdx.x < n_here) {
-      float a[kGradSlots];
+    // Flush the batch: four lanes per entry, each a quarter of its float2 pairs, add the sums of the rows that hold it, in
+    // row order.
+    for (int e = (int) threadIdx.x >> 2; e < n_here; e += kBlendThreads / 4) {
+      const int q = (int) threadIdx.x & 3;
+      float2 a[3] = {make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f)};
+      const unsigned char* rank = (const unsigned char*) &s_rank[parity][e];
+      for (unsigned rows = s_mask[parity][e]; rows != 0u; rows &= rows - 1u) {
+        const int r = __ffs((int) rows) - 1, at = rank[r];
+        if (at == kNotInRow) continue;
+        const float2* src = (const float2*) &s_sum[r][at][0];
 #pragma unroll
-      for (int c = 0; c < kGradSlots; ++c) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) sum += s_part[w][threadIdx.x][c], s_part[w][threadIdx.x][c] = 0.0f;
-        a[c] = sum;
+        for (int k = 0; k < 3; ++k)
+          if (k < 2 || q == 0) a[k].x += src[4 * k + q].x, a[k].y += src[4 * k + q].y;
       }
       if (kSlots) {
         // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order; the per-surfel
-        // sums are taken afterwards by slot_reduce_kernel. Every staged instance writes its record, zeros included (the
-        // instances that are never staged were cleared at the start), so nobody has to clear the buffer beforehand. A
-        // streaming zero fill of all records in front of this kernel took 13 us; the extra stores here move about as
-        // many bytes (partial lines are written back more than once) but ride on memory pipes this kernel leaves
-        // idle: operator 0.442 -> 0.434 ms. (Also measured, and slower than the fill: a "written" byte per instance
-        // with the sum skipping unwritten records, 0.505 ms against 0.488 ms for the operator.)
-        {
-          float2* dst = (float2*) (slot_grads + (size_t) s_slot[b & 1][threadIdx.x] * kGradSlots);
+        // sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that are never
+        // staged were cleared at the start), so nobody has to clear the buffer beforehand.
+        float2* dst = (float2*) (slot_grads + (size_t) s_slot[parity][e] * kGradSlots);
 #pragma unroll
-          for (int c = 0; c < kGradSlots / 2; ++c) dst[c] = make_float2(a[2 * c], a[2 * c + 1]);
-        }
+        for (int k = 0; k < 3; ++k)
+          if (k < 2 || q == 0) dst[4 * k + q] = a[k];
       } else {
         // one global atomic per surfel and component for this tile
-        const int id = s_slot[b & 1][threadIdx.x];
+        const int id = s_slot[parity][e];
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-          if (a[c] != 0.0f) atomicAdd(&g_colors[3 * (size_t) id + c], a[c]);
+        for (int k = 0; k < 3; ++k)
 #pragma unroll
-        for (int c = 0; c < 9; ++c)
-          if (a[3 + c] != 0.0f) atomicAdd(&g_trans[9 * (size_t) id + c], a[3 + c]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (a[12 + c] != 0.0f) atomicAdd(&g_normal_opacity[4 * (size_t) id + c], a[12 + c]);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          if (a[16 + c] != 0.0f) atomicAdd(&g_means2D[2 * (size_t) id + c], a[16 + c]);
+          for (int c2 = 0; c2 < 2; ++c2) {
+            const int c = 2 * (4 * k + q) + c2;
+            const float v = c2 ? a[k].y : a[k].x;
+            if (c >= kGradSlots || v == 0.0f) continue;
+            if (c < 3) atomicAdd(&g_colors[3 * (size_t) id + c], v);
+            else if (c < 12) atomicAdd(&g_trans[9 * (size_t) id + (c - 3)], v);
+            else if (c < 16) atomicAdd(&g_normal_opacity[4 * (size_t) id + (c - 12)], v);
+            else atomicAdd(&g_means2D[2 * (size_t) id + (c - 16)], v);
+          }
       }
     }
-    // No barrier needed here: between this flush and the barrier that follows the next batch's LDS store, wavefront 0
-    // touches its lanes' rows of s_part and this batch's copy of s_slot, wavefront 1 the staging arrays and the other
-    // copy of s_slot.
+    done += n_here;
+    // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
+    // records, which nobody reads before, and the other copy of what the flush reads.
   }
 }
 

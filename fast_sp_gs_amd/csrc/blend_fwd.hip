@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
     // blend is one divergent region.
     unsigned char* const lists = &s_list[Shape::kPerWave * wave * kFwdBatch];
     const int steps = build_block_lists<kFwdLanes, kFwdBatch>(lists, s_mask, wave, live_lanes);
-    auto blend_entry = [&](const SplatHot& hot, int j) {
+    auto blend_entry = [&](const SplatHot& hot, int j, int) {
 #pragma clang fp contract(off)  // several copies of this body exist (alternating registers): they must round alike
         const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
         __builtin_amdgcn_sched_barrier(0);
