@@ -12,7 +12,8 @@
 // sums a surfel's records in a fixed order. (Without scan offsets: one global atomic per surfel, component and tile.)
 // Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
 // the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
-// 1170 -> 950, 10k 256x256 58 -> 40.
+// 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260
+// instructions less per staged wavefront, for 7 us more in the forward) 245, 805 and 36.
 #include <algorithm>
 
 #include "block_lists.hpp"
@@ -40,7 +41,7 @@ blend_backward_kernel(
     const float* __restrict__ dL_dopacity, const float2* __restrict__ dL_dflow, float* __restrict__ g_means2D,
     float* __restrict__ g_normal_opacity, float* __restrict__ g_colors, float* __restrict__ g_trans,
     SlotSource slots, const int32_t* __restrict__ radii, float* __restrict__ slot_grads,
-    const float4* __restrict__ records) {
+    const float4* __restrict__ records, const uint32_t* __restrict__ hit_blocks) {
   // First record slot of a surfel; `stored` is what its packed record says (-1: packed before the offsets were known).
   auto first_slot = [&](int id, int64_t stored) -> int64_t {
     if (slots.region) return (stored >= 0 ? stored : (int64_t) slots.offset[id]) + slots.region[slot_region(id)];
@@ -149,12 +150,14 @@ blend_backward_kernel(
   Splat next;
   float next_t2[9];
   int next_radius = 0;
+  unsigned next_hits = 0u;
   int64_t next_off = 0;
   // entry e of the batch that starts behind `done` entries, counted from the back of the list
   auto gather = [&](int done) {
     const int e = (int) threadIdx.x;
     if (e >= min(kRowBatch, n_todo - done)) return;
     SplatExtra ex;
+    if (hit_blocks) next_hits = hit_blocks[r0 + (n_todo - 1 - done - e)];
     next = gather_splat(point_list[r0 + (n_todo - 1 - done - e)], means2D, colors, normal_opacity, trans_mat, records, &ex);
     if (kFlow)
 #pragma unroll
@@ -175,7 +178,7 @@ blend_backward_kernel(
       unsigned mask = 0u;
       if (e < n_staged) {
         s_splat[e] = next;
-        mask = surfel_blocks<16>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
+        mask = hit_blocks ? pair_blocks(next_hits) : surfel_blocks<16>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
         if (kFlow)
 #pragma unroll
           for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
@@ -320,43 +323,39 @@ blend_backward_kernel(
      walk_block_list(&s_list[(4 * wave + (lane >> 4)) * kRowSteps], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
                      [] { return true; });
     __syncthreads();
-    // Flush the batch: four lanes per entry, each a quarter of its float2 pairs, add the sums of the rows that hold it, in
-    // row order.
-    for (int e = (int) threadIdx.x >> 2; e < n_here; e += kBlendThreads / 4) {
-      const int q = (int) threadIdx.x & 3;
-      float2 a[3] = {make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f)};
+    // Flush the batch: two lanes per entry, nine components each, add the sums of the rows that hold it, in row order.
+    for (int e = (int) threadIdx.x >> 1; e < n_here; e += kBlendThreads / 2) {
+      constexpr int kHalf = kGradSlots / 2;
+      const int h = (int) threadIdx.x & 1;
+      float a[kHalf];
+#pragma unroll
+      for (int k = 0; k < kHalf; ++k) a[k] = 0.0f;
       const unsigned char* rank = (const unsigned char*) &s_rank[parity][e];
       for (unsigned rows = s_mask[parity][e]; rows != 0u; rows &= rows - 1u) {
         const int r = __ffs((int) rows) - 1, at = rank[r];
         if (at == kNotInRow) continue;
-        const float2* src = (const float2*) &s_sum[r][at][0];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (k < 2 || q == 0) a[k].x += src[4 * k + q].x, a[k].y += src[4 * k + q].y;
+        for (int k = 0; k < kHalf; ++k) a[k] += s_sum[r][at][h * kHalf + k];
       }
       if (kSlots) {
         // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order; the per-surfel
         // sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that are never
         // staged were cleared at the start), so nobody has to clear the buffer beforehand.
-        float2* dst = (float2*) (slot_grads + (size_t) s_slot[parity][e] * kGradSlots);
+        float* dst = slot_grads + (size_t) s_slot[parity][e] * kGradSlots + h * kHalf;
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (k < 2 || q == 0) dst[4 * k + q] = a[k];
+        for (int k = 0; k < kHalf; ++k) dst[k] = a[k];
       } else {
         // one global atomic per surfel and component for this tile
         const int id = s_slot[parity][e];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2) {
-            const int c = 2 * (4 * k + q) + c2;
-            const float v = c2 ? a[k].y : a[k].x;
-            if (c >= kGradSlots || v == 0.0f) continue;
-            if (c < 3) atomicAdd(&g_colors[3 * (size_t) id + c], v);
-            else if (c < 12) atomicAdd(&g_trans[9 * (size_t) id + (c - 3)], v);
-            else if (c < 16) atomicAdd(&g_normal_opacity[4 * (size_t) id + (c - 12)], v);
-            else atomicAdd(&g_means2D[2 * (size_t) id + (c - 16)], v);
-          }
+        for (int k = 0; k < kHalf; ++k) {
+          const int c = h * kHalf + k;
+          if (a[k] == 0.0f) continue;
+          if (c < 3) atomicAdd(&g_colors[3 * (size_t) id + c], a[k]);
+          else if (c < 12) atomicAdd(&g_trans[9 * (size_t) id + (c - 3)], a[k]);
+          else if (c < 16) atomicAdd(&g_normal_opacity[4 * (size_t) id + (c - 12)], a[k]);
+          else atomicAdd(&g_means2D[2 * (size_t) id + (c - 16)], a[k]);
+        }
       }
     }
     done += n_here;
@@ -465,7 +464,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
     const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
     const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D, float* g_trans,
     float* g_normal_opacity, int64_t R, const SlotSource& source, const int32_t* radii, void* workspace,
-    size_t workspace_bytes, const float* records, const uint32_t* keep_masks, void* stream) {
+    size_t workspace_bytes, const float* records, const uint32_t* keep_masks, const uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_render_backward: bad sizes");
   if (P == 0) return kOk;
   FSGS_REQUIRE(means2D && normal_opacity && colors && trans_mat && out_opacity && dL_dpix && dL_dopacity && ranges &&
@@ -496,7 +495,7 @@ int render_backward(int P, int W, int H, double near_n, double far_n, const floa
                      (const float4*) normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity, out_extras,       \
                      (const float2*) out_flow, dL_dpix, dL_dextras, dL_dopacity, (const float2*) dL_dflow,           \
                      g_means2D, g_normal_opacity, g_colors, g_trans, source, radii, slot_grads,               \
-                     (const float4*) records)
+                     (const float4*) records, hit_blocks)
   if (slots) {
     if (aux && flow) FSGS_LAUNCH_BWD(true, true, true);
     else if (aux) FSGS_LAUNCH_BWD(true, false, true);
@@ -529,7 +528,7 @@ FSGS_API int fsgs_gs_2d_render_backward(int P, int W, int H, double near_n, doub
   return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
                          g_colors, g_means2D, g_trans, g_normal_opacity, R, SlotSource{point_offsets}, radii, workspace,
-                         workspace_bytes, records, nullptr, stream);
+                         workspace_bytes, records, nullptr, nullptr, stream);
 }
 
 FSGS_API int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_n, double far_n, const float* means2D,
@@ -544,7 +543,7 @@ FSGS_API int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_
   return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
                          g_colors, g_means2D, g_trans, g_normal_opacity, R, SlotSource{point_offsets}, radii, workspace,
-                         workspace_bytes, records, keep_masks, stream);
+                         workspace_bytes, records, keep_masks, nullptr, stream);
 }
 
 // The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp): the records stay in the
@@ -562,5 +561,22 @@ FSGS_API int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double
                          out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
                          nullptr, nullptr, nullptr, nullptr, R,
                          SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
-                         workspace_bytes, records, nullptr, stream);
+                         workspace_bytes, records, nullptr, nullptr, stream);
+}
+
+// The same over the blocks that blended an entry, as the forward noted them (nullptr: bounded here).
+FSGS_API int fsgs_gs_2d_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
+    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
+    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
+    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const float* records, const uint32_t* hit_blocks, void* stream) {
+  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && records),
+               "gs_2d_view_backward: record slots and packed records are required");
+  return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
+                         out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
+                         nullptr, nullptr, nullptr, nullptr, R,
+                         SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
+                         workspace_bytes, records, nullptr, hit_blocks, stream);
 }

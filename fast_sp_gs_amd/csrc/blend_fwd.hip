@@ -32,15 +32,17 @@ constexpr int kFwdBatch = FSGS_FWD_BATCH;  // surfels staged per round (<= block
 
 // kAccum: 0 = no side outputs, 1 = accum_max_count only (what the reference's training loop passes on every step),
 // 2 = accum_weights_p and / or accum_weights_count as well.
-template <bool kAux, bool kFlow, int kAccum>
-__global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
+// kHits: notes which blocks blended an entry (hit_blocks), for the backward.
+template <bool kAux, bool kFlow, int kAccum, bool kHits>
+__global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(!kFlow && kAccum < 2 ? 5 : 1)))
+blend_forward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
     const float2* __restrict__ means2D, const float* __restrict__ colors, const float* __restrict__ trans_mat,
     const float4* __restrict__ normal_opacity, const float4* __restrict__ records,
     const float* __restrict__ trans_mat_t2, int32_t* __restrict__ n_contrib,
     float* __restrict__ out_color, float* __restrict__ out_opacity, float* __restrict__ out_extras,
     float2* __restrict__ out_flow, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
-    int32_t* __restrict__ accum_weights_count) {
+    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks) {
   using Shape = BlockShape<kFwdLanes>;
   __shared__ Splat s_splat[kFwdBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kFwdBatch * 9 : 1];
@@ -50,6 +52,7 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
   // rows here; one global atomic per staged surfel and output
   __shared__ float s_accw[kAccum == 2 ? kFwdBatch : 1];
   __shared__ int s_accn[kAccum == 2 ? kFwdBatch : 1];
+  __shared__ uint4 s_hit[kHits ? kFwdBatch : 1][2];  // which blocks blended each staged surfel, a byte per block (hit_bits)
 
   const int gx = (W + kTile - 1) / kTile;
   const int tile = scheduled_tile(ordered, tile_order), tile_x = tile % gx, tile_y = tile / gx;
@@ -82,6 +85,15 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
     if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[t]);
     s_accw[t] = 0.0f, s_accn[t] = 0;
   };
+  // the same for the blocks that blended it; `b` is the batch
+  auto flush_hits = [&](int b) {
+    const int t = (int) threadIdx.x;
+    if (t >= kFwdBatch) return;
+    if (b * kFwdBatch + t < n_todo) hit_blocks[r0 + b * kFwdBatch + t] = hit_bits(s_hit[t][0], s_hit[t][1]);
+    s_hit[t][0] = s_hit[t][1] = make_uint4(0u, 0u, 0u, 0u);
+  };
+  if (kHits && threadIdx.x < kFwdBatch) s_hit[threadIdx.x][0] = s_hit[threadIdx.x][1] = make_uint4(0u, 0u, 0u, 0u);
+  unsigned char* const my_hit = (unsigned char*) &s_hit[0][0] + ((Shape::kPerWave * wave + lane / kFwdLanes) ^ 3);
   if (threadIdx.x == 0) s_splat[kFwdBatch] = Splat{};  // all zero: p_z == 0 everywhere
   if (threadIdx.x < 4) ((unsigned*) &s_list[Shape::kPerTile * kFwdBatch])[threadIdx.x] = 0u;
   if (kAccum == 2 && threadIdx.x < kFwdBatch) s_accw[threadIdx.x] = 0.0f, s_accn[threadIdx.x] = 0;
@@ -95,11 +107,13 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
       for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
   }
 
-  for (int b = 0; b < rounds; ++b) {
+  int b = 0;
+  for (; b < rounds; ++b) {
     // everyone has finished reading the previous batch; leave as soon as no pixel of the tile is still blending
     if (__syncthreads_and(live_lanes == 0ull)) break;
     const int n_here = min(kFwdBatch, n_todo - b * kFwdBatch);
     if (kAccum == 2) flush_weights();
+    if (kHits && b > 0) flush_hits(b - 1);
     if ((int) threadIdx.x < kFwdBatch) {
       unsigned mask = 0u;
       if ((int) threadIdx.x < n_here) {
@@ -145,6 +159,7 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
           if ((lane & (kFwdLanes - 1)) == kFwdLanes - 1 && n > 0) atomicAdd(&s_accw[j], sum), atomicAdd(&s_accn[j], n);
         }
         if (blend) {
+          if (kHits) my_hit[j * 32] = 1;
           const int contributor = b * kFwdBatch + j + 1;
           if (kAux) {
             const float A  = 1.0f - T;
@@ -178,10 +193,9 @@ __global__ void __launch_bounds__(kBlendThreads) blend_forward_kernel(
   }
 
   if (kAccum != 0) argmax_run_flush(argmax, accum_max_count);
-  if (kAccum == 2) {
-    __syncthreads();
-    flush_weights();
-  }
+  if (kAccum == 2 || kHits) __syncthreads();
+  if (kAccum == 2) flush_weights();
+  if (kHits && b > 0) flush_hits(b - 1);  // entries behind it are behind every pixel's last one
   if (inside) {
     out_opacity[pix]      = 1.0f - T;
     n_contrib[pix]        = last;
@@ -243,11 +257,13 @@ FSGS_API int fsgs_gs_2d_pack_records(int P, const float* means2D, const float* c
   return check_launch("gs_2d_pack_records");
 }
 
-FSGS_API int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
+namespace {
+// hit_blocks[R], if given: per list entry the 2x4 blocks of its tile with a pixel that blended it
+int render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
     const float* means2D, const float* colors, const float* normal_opacity, const float* trans_mat,
     const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
     float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
-    float* out_flow, int32_t* n_contrib, const float* records, void* stream) {
+    float* out_flow, int32_t* n_contrib, const float* records, uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_render_forward: bad sizes");
   FSGS_REQUIRE(ranges && out_color && out_opacity && n_contrib, "GS_2D_render_forward: null pointer");
   FSGS_REQUIRE(P == 0 || records || (means2D && colors && normal_opacity && trans_mat),
@@ -263,20 +279,46 @@ FSGS_API int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, doubl
   hipStream_t s = (hipStream_t) stream;
   const int* tile_order = nullptr;
   const int ordered = launch_tile_order(gx, gy, ranges, s, &tile_order);
-#define FSGS_LAUNCH_FWD(AUX, FLOW, ACC)                                                                              \
-  hipLaunchKernelGGL((blend_forward_kernel<AUX, FLOW, ACC>), grid, block, 0, s, ordered, tile_order, W, H, (float) near_n, (float) far_n, \
-                     ranges, point_list, (const float2*) means2D, colors, trans_mat, (const float4*) normal_opacity, \
-                     (const float4*) records, trans_mat_t2, n_contrib, out_color, out_opacity, out_extras, (float2*) out_flow,                \
-                     accum_max_count, accum_weights_p, accum_weights_count)
-  if (!aux) FSGS_LAUNCH_FWD(false, false, 0);
-  else if (flow && accum == 2) FSGS_LAUNCH_FWD(true, true, 2);
-  else if (flow && accum == 1) FSGS_LAUNCH_FWD(true, true, 1);
-  else if (flow) FSGS_LAUNCH_FWD(true, true, 0);
-  else if (accum == 2) FSGS_LAUNCH_FWD(true, false, 2);
-  else if (accum == 1) FSGS_LAUNCH_FWD(true, false, 1);
-  else FSGS_LAUNCH_FWD(true, false, 0);
+#define FSGS_LAUNCH_FWD(AUX, FLOW, ACC, HITS)                                                                        \
+  hipLaunchKernelGGL((blend_forward_kernel<AUX, FLOW, ACC, HITS>), grid, block, 0, s, ordered, tile_order, W, H, (float) near_n, \
+                     (float) far_n, ranges, point_list, (const float2*) means2D, colors, trans_mat,                  \
+                     (const float4*) normal_opacity, (const float4*) records, trans_mat_t2, n_contrib, out_color, out_opacity, \
+                     out_extras, (float2*) out_flow, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks)
+#define FSGS_LAUNCH_FWD_HITS(FLOW, ACC)              \
+  if (hit_blocks) FSGS_LAUNCH_FWD(true, FLOW, ACC, true); \
+  else FSGS_LAUNCH_FWD(true, FLOW, ACC, false)
+  if (!aux) FSGS_LAUNCH_FWD(false, false, 0, false);
+  else if (flow && accum == 2) { FSGS_LAUNCH_FWD_HITS(true, 2); }
+  else if (flow && accum == 1) { FSGS_LAUNCH_FWD_HITS(true, 1); }
+  else if (flow) { FSGS_LAUNCH_FWD_HITS(true, 0); }
+  else if (accum == 2) { FSGS_LAUNCH_FWD_HITS(false, 2); }
+  else if (accum == 1) { FSGS_LAUNCH_FWD_HITS(false, 1); }
+  else { FSGS_LAUNCH_FWD_HITS(false, 0); }
+#undef FSGS_LAUNCH_FWD_HITS
 #undef FSGS_LAUNCH_FWD
   return check_launch("GS_2D_render_forward");
+}
+
+}  // namespace
+
+FSGS_API int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
+    const float* means2D, const float* colors, const float* normal_opacity, const float* trans_mat,
+    const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
+    float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
+    float* out_flow, int32_t* n_contrib, const float* records, void* stream) {
+  return render_forward(P, W, H, near_n, far_n, only_image, means2D, colors, normal_opacity, trans_mat, point_list, ranges,
+                        trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count, out_color, out_opacity, out_extras,
+                        out_flow, n_contrib, records, nullptr, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* colors, const float* normal_opacity, const float* trans_mat, const int32_t* point_list,
+    const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count, float* accum_weights_p,
+    int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras, float* out_flow,
+    int32_t* n_contrib, const float* records, uint32_t* hit_blocks, void* stream) {
+  return render_forward(P, W, H, near_n, far_n, 0, means2D, colors, normal_opacity, trans_mat, point_list, ranges, trans_mat_t2,
+                        accum_max_count, accum_weights_p, accum_weights_count, out_color, out_opacity, out_extras, out_flow,
+                        n_contrib, records, hit_blocks, stream);
 }
 
 FSGS_API int fsgs_debug_tile_order(int gx, int gy, const int64_t* ranges, int32_t* table, void* stream) {

@@ -190,6 +190,27 @@ __device__ __forceinline__ void walk_block_list(const unsigned char* __restrict_
   }
 }
 
+// ---- which blocks blended an entry ---------------------------------------------------------------------------------------
+// A forward kernel (2x4 blocks) can note, per staged entry, the blocks with a pixel that blended it, a byte per block; the
+// backward then walks exactly these instead of bounding every footprint again. Block b's byte is b ^ 3: the product below
+// gathers the low bits of four bytes, the last byte's first.
+__device__ __forceinline__ unsigned hit_bits(const uint4& lo, const uint4& hi) {
+  const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  unsigned m = 0u;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) m |= (w[k] * 0x08040201u >> 24) << (4 * k);
+  return m;
+}
+
+// Mask of the 4x4 blocks that hold a set 2x4 block: pairs of neighbouring bits joined, every second bit kept.
+__device__ __forceinline__ unsigned pair_blocks(unsigned m) {
+  m = (m | m >> 1) & 0x55555555u;
+  m = (m | m >> 1) & 0x33333333u;
+  m = (m | m >> 2) & 0x0f0f0f0fu;
+  m = (m | m >> 4) & 0x00ff00ffu;
+  return (m | m >> 8) & 0xffffu;
+}
+
 // ---- lists of the backward kernels: per 4x4 block, with a place for each entry's sums -------------------------------
 // A row of 16 lanes sums an entry's gradient components over its 16 pixels with DPP shifts and stores the totals at the
 // step's place, [row of the tile][step]: an entry's sums from different rows never meet, so nothing is read back, added or

@@ -17,6 +17,7 @@ struct Buffers {
   Tensor trans_mat, normal_opacity, radii, visible, ranges, point_list, n_contrib;
   Tensor image, opacity, extras, flow;                       // what the blend writes
   Tensor normals, depths, surf_depth, surf_normal, composited;  // what the epilogue writes
+  Tensor hit_blocks;                                          // per list entry, for the backward
   Slab keep;                                                  // what only the backward reads
   Saved saved;
 };
@@ -118,11 +119,12 @@ Buffers forward_view(const SurfelView& v, bool train) {
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
   }
-  check(fsgs_gs_2d_render_forward((int) P, W, H, v.near_n, v.far_n, 0, f32(v.means2D), colors, f32(b.normal_opacity),
+  if (train) b.hit_blocks = empty({s.R}, like, at::kInt);
+  check(fsgs_gs_2d_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, f32(b.normal_opacity),
                                   f32(b.trans_mat), i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
                                   i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
                                   i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
-                                  f32(b.flow), i32(b.n_contrib), records, stream),
+                                  f32(b.flow), i32(b.n_contrib), records, (uint32_t*) i32(b.hit_blocks), stream),
         blend);
   if (v.epilogue) {
     b.normals = empty({3, H, W}, like), b.depths = empty({1, H, W}, like), b.surf_depth = empty({1, H, W}, like);
@@ -166,7 +168,8 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
     const Buffers& b = *out;
     ctx->save_for_backward({v.points, v.scales, v.rotations, v.opacities, v.shs, opt(v.sh_rest), v.means2D, v.Tw2v,
                             v.Tv2c, v.campos, opt(v.background), opt(v.trans_mat_t2), b.trans_mat, b.normal_opacity,
-                            b.radii, b.ranges, b.point_list, b.n_contrib, b.opacity, b.extras, b.flow, b.keep.memory()});
+                            b.radii, b.ranges, b.point_list, b.n_contrib, b.opacity, b.extras, b.flow, b.keep.memory(),
+                            b.hit_blocks});
     ctx->saved_data["view"] = c10::IValue::make_capsule(c10::make_intrusive<SavedHolder>(b.saved, v.cull));
     ctx->set_materialize_grads(false);
     return outputs_of(b);
@@ -234,13 +237,13 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
       const bool aux = g_extras.defined();
       const float* colors = s.sh_degree < 0 ? f32(shs) : (const float*) keep(s.colors);
       const int M = has_rest && sh_rest.numel() > 0 ? (int) sh_rest.size(1) : shs.dim() == 3 ? (int) shs.size(1) : 0;
-      check(fsgs_gs_2d_view_backward((int) P, W, H, s.near_n, s.far_n, f32(means2D), f32(normal_opacity), colors,
+      check(fsgs_gs_2d_view_backward_hits((int) P, W, H, s.near_n, s.far_n, f32(means2D), f32(normal_opacity), colors,
                                      f32(trans_mat), f32(t2), f32(opacity), aux ? f32(extras) : nullptr,
                                      g_flow.defined() ? f32(flow) : nullptr, f32(g_image), f32(g_opacity),
                                      f32(g_extras), f32(g_flow), i64(ranges), i32(point_list), i32(n_contrib),
                                      s.R, (const int32_t*) keep(s.offsets), (const int32_t*) keep(s.regions),
                                      (const int32_t*) keep(s.tiles), i32(radii), scratch.at<void>(ws), ws_bytes,
-                                     (const float*) keep(s.records), stream),
+                                     (const float*) keep(s.records), (const uint32_t*) i32(t[22]), stream),
             "GS_2D_render_backward");
       check(fsgs_gs_2d_view_preprocess_backward(
                 (int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations), f32(shs),

@@ -182,6 +182,15 @@ int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, double far_n, 
     float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
     float* out_flow, int32_t* n_contrib, const float* records, void* stream);
 
+/* The same with all maps, for a view that will be back-propagated: hit_blocks[R] (nullptr: not wanted) receives, per list
+ * entry, a bit for every block of 2x4 pixels of its tile with a pixel that blended it; entries behind the last one that any
+ * pixel of the tile blended keep what the buffer held. */
+int fsgs_gs_2d_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D, const float* colors,
+    const float* normal_opacity, const float* trans_mat, const int32_t* point_list, const int64_t* ranges,
+    const float* trans_mat_t2, int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count,
+    float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib, const float* records,
+    uint32_t* hit_blocks, void* stream);
+
 /* GS_2D_render_backward -- gs_2d_redner.cu:631-717 (kernel :238-539). Two ways of summing a surfel's gradient over the
  * tiles it touches:
  *  - point_offsets == NULL: device-scope float atomics, as the reference does; g_colors[P,3] g_means2D[P,2]
@@ -220,6 +229,14 @@ int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, c
     const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
     const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const float* records, void* stream);
+/* The same with the hit_blocks that fsgs_gs_2d_view_forward left for these lists (nullptr: footprints are bounded again). */
+int fsgs_gs_2d_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
+    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
+    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
+    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const float* records, const uint32_t* hit_blocks, void* stream);
 /* fsgs_gs_2d_preprocess_backward whose upstream gradients are the sums of those records (keep_masks nullptr for full lists);
  * g_means2D[P,2] receives the densification proxy, zeros for surfels that were not rendered. */
 int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,

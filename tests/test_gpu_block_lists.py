@@ -58,3 +58,37 @@ def test_surfel_blend(shape, P, device):
     for k in a:
         if k.startswith('g_') and a[k] is not None:  # sums of at most 1e4 terms: 1e-5 of the largest is 100 roundings
             assert (a[k] - b[k]).abs().max() <= 1e-5 * b[k].abs().max(), k
+
+
+def _params(scene, axes=2):
+    scales = scene.scales if axes == 2 else torch.cat([scene.scales, scene.scales.mean(1, keepdim=True)], 1)
+    return {k: v.clone().requires_grad_(True) for k, v in
+            dict(points=scene.means3D, scales=scales, rotations=scene.rotations, opacity=scene.opacities,
+                 sh_features=scene.shs).items()}
+
+
+def _gradients(params, maps, seed=5):
+    g = torch.Generator().manual_seed(seed)
+    up = [torch.randn(m.shape, generator=g).to(m.device) for m in maps]
+    return torch.autograd.grad(maps, list(params.values()), up, allow_unused=True)
+
+
+@pytest.mark.parametrize("P", [1, 95, 96, 97, 700])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_surfel_view(shape, P, device):
+    """The view's backward walks the blocks that the forward noted as blended instead of bounding footprints."""
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    scene, cam = _scene(shape, P, device)
+
+    def run():
+        params = _params(scene)
+        out = GS_2D_render(size=(cam.W, cam.H), Tw2v=cam.Tw2v, Tv2c=cam.Tv2c, campos=cam.campos, near=cam.near, far=cam.far,
+                           sh_degree=3, background=torch.ones(3, device=device), **params)
+        maps = [out[k] for k in ('images', 'normals', 'surf_depth', 'distortion')]
+        return maps, _gradients(params, maps)
+
+    (maps, grads), (maps_all, grads_all) = _both(run)
+    for a, b in zip(maps, maps_all):
+        assert torch.equal(a, b)
+    for a, b in zip(grads, grads_all):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
