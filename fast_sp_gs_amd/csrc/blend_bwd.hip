@@ -13,7 +13,9 @@
 // Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
 // the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
 // 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260
-// instructions less per staged wavefront, for 7 us more in the forward) 245, 805 and 36.
+// instructions less per staged wavefront, for 7 us more in the forward) 245, 805 and 36; with batches of up to 128 entries
+// whose rows share out one pool of places, instead of 96 with 24 places a row, and a flush that waits for no entry's rows one by
+// one, 230, 782 and 37. One tile of 1800 entries alone, which the launch cannot be shorter than: 179 -> 127.
 #include <algorithm>
 
 #include "block_lists.hpp"
@@ -50,12 +52,12 @@ blend_backward_kernel(
   using Shape = BlockShape<16>;
   __shared__ Splat s_splat[kRowBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kRowBatch * 9 : 1];
-  __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kRowSteps + 16];
-  __shared__ float s_sum[16][kRowSteps][kGradSlots];
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kRowBatch + 16];
+  __shared__ float s_sum[kRowPlaces + 1][kGradSlots];
   // What the flush of a batch reads is kept twice, by batch parity: the next batch is staged while others still flush.
-  __shared__ unsigned s_mask[2][kRowMasks];  // which 4x4 blocks of the tile each staged surfel can reach
-  __shared__ uint4 s_rank[2][kRowBatch];     // at which step each of the 16 rows meets it
-  __shared__ int s_slot[2][kRowBatch];       // where its sums go: its position in surfel order (kSlots) or the surfel's id
+  __shared__ uint4 s_place[2][kRowBatch];  // where each of the 16 rows stores its sums of each staged surfel
+  __shared__ int s_slot[2][kRowBatch];     // where they go from there: its position in surfel order (kSlots) or the surfel's id
+  __shared__ unsigned s_mask[kRowBatch];   // which 4x4 blocks of the tile it can reach
   __shared__ int s_max_contrib;
 
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
@@ -83,7 +85,8 @@ blend_backward_kernel(
   for (int r = 0; r < 4; ++r) row_last[r] = __builtin_amdgcn_readlane(row_max, 16 * r);
   if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
   if (threadIdx.x == 0) s_splat[kRowBatch] = Splat{};  // all zero: p_z == 0 everywhere
-  if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kRowSteps])[threadIdx.x] = 0u;
+  if (threadIdx.x < kGradSlots) s_sum[kNoPlace][threadIdx.x] = 0.0f;
+  if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kRowBatch])[threadIdx.x] = 0u;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));  // positions [0, n_todo) of the tile's list, walked from n_todo-1 down to 0
   // No zero fill of the records: the instances behind the tile's deepest contributor are never staged, their records
@@ -173,12 +176,12 @@ blend_backward_kernel(
 
   for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
     const int n_staged = min(kRowBatch, n_todo - done);
-    if ((int) threadIdx.x < kRowMasks) {
+    if ((int) threadIdx.x < kRowBatch) {
       const int e = (int) threadIdx.x;
       unsigned mask = 0u;
       if (e < n_staged) {
         s_splat[e] = next;
-        mask = hit_blocks ? pair_blocks(next_hits) : surfel_blocks<16>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
+        mask = hit_blocks ? pair_blocks(next_hits) : surfel_blocks<16>(next.hot, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
         if (kFlow)
 #pragma unroll
           for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
@@ -190,18 +193,20 @@ blend_backward_kernel(
         } else {
           s_slot[parity][e] = next.cold.id;
         }
-        s_rank[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        s_place[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
       }
-      s_mask[parity][e] = mask;
+      s_mask[e] = mask;
     }
     __syncthreads();
-    const unsigned masks[2] = {s_mask[parity][lane], s_mask[parity][kWave + lane]};
-    const int n_here = row_batch(masks, n_staged);
+    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    int start, before[4];
+    const int n_here = row_batch(masks, n_staged, wave, start);
     gather(done + n_here);
     // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
     const int behind = n_todo - done;
     const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
-    const int steps = build_row_lists(&s_list[4 * kRowSteps * wave], (unsigned char*) s_rank[parity], masks, wave, first, n_here);
+    const int steps = build_row_lists(&s_list[4 * kRowBatch * wave], (unsigned char*) s_place[parity], masks, wave, first, start,
+                                      before, n_here);
     const int my_first = behind - last_contrib, my_median = behind - median_contrib;
     // ---- order-bound part of one (pixel, entry) pair: advances the pixel's back-to-front state -------------------------
     // All channels that enter the image linearly (colour, depth, opacity, normal) share one recurrence: with
@@ -295,8 +300,9 @@ blend_backward_kernel(
        const float to_centre = filtered ? hot.opacity * dL_dalpha * (-2.0f * h.G) : 0.0f;
        g2x = to_centre * h.dx, g2y = to_centre * h.dy;
      };
-     float* const sums = &s_sum[4 * wave + (lane >> 4)][0][lane & 15];         // component lane & 15 of step 0
-     float* const centre = &s_sum[4 * wave + (lane >> 4)][0][16 + (lane >> 3 & 1)];  // lanes 0 and 8 of a row: means2D
+     const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+     float* const sums   = &s_sum[place][lane & 15];               // component lane & 15 of the row's first place
+     float* const centre = &s_sum[place][16 + (lane >> 3 & 1)];  // the row's lanes 0 and 8: means2D
      auto backward_entry = [&](const SplatHot& hot, int j, int i) {
       const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
       __builtin_amdgcn_sched_barrier(0);
@@ -317,45 +323,40 @@ blend_backward_kernel(
           mid += dpp_shift_zero<0x101, 0xf, 0xf>(mid);
         }
       }
-      sums[i * kGradSlots] = tot;  // zeros, too, have their place
-      if ((lane & 7) == 0) centre[i * kGradSlots] = mid;
+      if (j != kRowBatch) {  // not a padding step; zeros, too, have their place
+        sums[i * kGradSlots] = tot;
+        if ((lane & 7) == 0) centre[i * kGradSlots] = mid;
+      }
      };
-     walk_block_list(&s_list[(4 * wave + (lane >> 4)) * kRowSteps], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
+     walk_block_list(&s_list[(4 * wave + row) * kRowBatch], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
                      [] { return true; });
     __syncthreads();
-    // Flush the batch: two lanes per entry, nine components each, add the sums of the rows that hold it, in row order.
-    for (int e = (int) threadIdx.x >> 1; e < n_here; e += kBlendThreads / 2) {
-      constexpr int kHalf = kGradSlots / 2;
-      const int h = (int) threadIdx.x & 1;
-      float a[kHalf];
-#pragma unroll
-      for (int k = 0; k < kHalf; ++k) a[k] = 0.0f;
-      const unsigned char* rank = (const unsigned char*) &s_rank[parity][e];
-      for (unsigned rows = s_mask[parity][e]; rows != 0u; rows &= rows - 1u) {
-        const int r = __ffs((int) rows) - 1, at = rank[r];
-        if (at == kNotInRow) continue;
-#pragma unroll
-        for (int k = 0; k < kHalf; ++k) a[k] += s_sum[r][at][h * kHalf + k];
-      }
-      if (kSlots) {
-        // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order; the per-surfel
-        // sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that are never
-        // staged were cleared at the start), so nobody has to clear the buffer beforehand.
+    // Flush the batch: add the sums of the rows that hold an entry, in row order.
+    if (kSlots) {
+      // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order, nine components per lane; the
+      // per-surfel sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that
+      // are never staged were cleared at the start), so nobody has to clear the buffer beforehand.
+      static_assert(kBlendThreads == 2 * kRowBatch);
+      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
+        constexpr int kHalf = kGradSlots / 2;
+        const int h = (int) threadIdx.x & 1;
+        float a[kHalf];
+        sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], h * kHalf, a);
         float* dst = slot_grads + (size_t) s_slot[parity][e] * kGradSlots + h * kHalf;
 #pragma unroll
         for (int k = 0; k < kHalf; ++k) dst[k] = a[k];
-      } else {
-        // one global atomic per surfel and component for this tile
-        const int id = s_slot[parity][e];
-#pragma unroll
-        for (int k = 0; k < kHalf; ++k) {
-          const int c = h * kHalf + k;
-          if (a[k] == 0.0f) continue;
-          if (c < 3) atomicAdd(&g_colors[3 * (size_t) id + c], a[k]);
-          else if (c < 12) atomicAdd(&g_trans[9 * (size_t) id + (c - 3)], a[k]);
-          else if (c < 16) atomicAdd(&g_normal_opacity[4 * (size_t) id + (c - 12)], a[k]);
-          else atomicAdd(&g_means2D[2 * (size_t) id + (c - 16)], a[k]);
-        }
+      }
+    } else {
+      // one global atomic per surfel and component for this tile, a lane per component: a surfel's are a few requests
+      for (int t = (int) threadIdx.x; t < n_here * kGradSlots; t += kBlendThreads) {
+        const int e = t / kGradSlots, c = t - e * kGradSlots, id = s_slot[parity][e];
+        float a[1];
+        sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
+        float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
+                           : c < 12 ? g_trans + 9 * (size_t) id + (c - 3)
+                           : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
+                                    : g_means2D + 2 * (size_t) id + (c - 16);
+        if (a[0] != 0.0f) atomicAdd(out, a[0]);
       }
     }
     done += n_here;

@@ -85,11 +85,12 @@ blend_forward_kernel(
     if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[t]);
     s_accw[t] = 0.0f, s_accn[t] = 0;
   };
+  uint32_t* const tile_hits = hit_blocks + (kHits ? r0 : 0);
   // the same for the blocks that blended it; `b` is the batch
   auto flush_hits = [&](int b) {
     const int t = (int) threadIdx.x;
     if (t >= kFwdBatch) return;
-    if (b * kFwdBatch + t < n_todo) hit_blocks[r0 + b * kFwdBatch + t] = hit_bits(s_hit[t][0], s_hit[t][1]);
+    if (b * kFwdBatch + t < n_todo) tile_hits[keep_local(b * kFwdBatch + t)] = hit_bits(s_hit[t][0], s_hit[t][1]);
     s_hit[t][0] = s_hit[t][1] = make_uint4(0u, 0u, 0u, 0u);
   };
   if (kHits && threadIdx.x < kFwdBatch) s_hit[threadIdx.x][0] = s_hit[threadIdx.x][1] = make_uint4(0u, 0u, 0u, 0u);
@@ -118,7 +119,7 @@ blend_forward_kernel(
       unsigned mask = 0u;
       if ((int) threadIdx.x < n_here) {
         s_splat[threadIdx.x] = next;
-        mask = surfel_blocks<kFwdLanes>(next.hot, tile_x * kTile, tile_y * kTile, ordered);
+        mask = surfel_blocks<kFwdLanes>(next.hot, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
         if (kFlow)
 #pragma unroll
           for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
@@ -137,7 +138,10 @@ blend_forward_kernel(
     // One list entry per block of the wavefront. The intersection runs without early exits and yields one predicate; the
     // blend is one divergent region.
     unsigned char* const lists = &s_list[Shape::kPerWave * wave * kFwdBatch];
-    const int steps = build_block_lists<kFwdLanes, kFwdBatch>(lists, s_mask, wave, live_lanes);
+    unsigned masks[kFwdBatch / kWave];
+#pragma unroll
+    for (int c = 0; c < kFwdBatch / kWave; ++c) masks[c] = s_mask[c * kWave + lane];
+    const int steps = build_block_lists<kFwdLanes, kFwdBatch>(lists, masks, wave, live_lanes);
     auto blend_entry = [&](const SplatHot& hot, int j, int) {
 #pragma clang fp contract(off)  // several copies of this body exist (alternating registers): they must round alike
         const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting

@@ -54,14 +54,14 @@ __device__ __forceinline__ void footprint_ellipse(Footprint& f, float hx, float 
 // The blocks of the tile whose pixel centres' hull meets the footprint. Per row of blocks (a slab of heights) the
 // ellipse's extent along x is exact: its right (left) boundary is highest at `top` (-top), or at the slab's nearer edge.
 // Against rounding the footprint is grown by 1/8 pixel and 0.5 % of its extent, as the other bounds are.
-template <int kLanes>
+template <int kLanes, bool kDisc>
 __device__ __forceinline__ unsigned footprint_blocks(const Footprint& f, int tile_px, int tile_py) {
 #pragma clang fp contract(off)
   using Shape = BlockShape<kLanes>;
   constexpr unsigned kAll = (unsigned) ((1ull << Shape::kPerTile) - 1ull);
   constexpr float kWidth = (float) Shape::kWide, kCols = (float) Shape::kColumns;
   if (f.state != 2) return f.state == 1 ? kAll : 0u;
-  const float padx = kCullPad + 0.01f * f.ex, pady = kCullPad + 0.01f * f.ey, r2 = f.disc * f.disc;
+  const float padx = kCullPad + 0.01f * f.ex, pady = kCullPad + 0.01f * f.ey, r2 = kDisc ? f.disc * f.disc : 0.0f;
   const float qx = (float) tile_px - f.ox, qy = (float) tile_py - f.oy;  // first pixel of the tile
   unsigned m = 0u;
 #pragma unroll
@@ -74,9 +74,11 @@ __device__ __forceinline__ unsigned footprint_blocks(const Footprint& f, int til
     float right = f.cx + (f.slope * yr + f.wide * sr) + padx, left = f.cx + (f.slope * yl - f.wide * sl) - padx;
     const bool in_ellipse = lo <= f.ey && hi >= -f.ey;
     right = in_ellipse ? right : -1e30f, left = in_ellipse ? left : 1e30f;
-    const float yd = __builtin_amdgcn_fmed3f(0.0f, y0 - kCullPad, y1 + kCullPad), t = r2 - yd * yd;
-    const float half = __builtin_amdgcn_sqrtf(fmaxf(t, 0.0f)) + kCullPad;
-    right = fmaxf(right, t >= 0.0f ? half : -1e30f), left = fminf(left, t >= 0.0f ? -half : 1e30f);
+    if (kDisc) {
+      const float yd = __builtin_amdgcn_fmed3f(0.0f, y0 - kCullPad, y1 + kCullPad), t = r2 - yd * yd;
+      const float half = __builtin_amdgcn_sqrtf(fmaxf(t, 0.0f)) + kCullPad;
+      right = fmaxf(right, t >= 0.0f ? half : -1e30f), left = fminf(left, t >= 0.0f ? -half : 1e30f);
+    }
     // columns [first, last) whose pixels meet [left, right]
     const int last  = (int) __builtin_amdgcn_fmed3f(floorf((right - qx) / kWidth) + 1.0f, 0.0f, kCols);
     const int first = (int) __builtin_amdgcn_fmed3f(ceilf((left - qx - (kWidth - 1.0f)) / kWidth), 0.0f, kCols);
@@ -118,15 +120,41 @@ __device__ __forceinline__ Footprint surfel_footprint(const float* m, float ox, 
 template <int kLanes>
 __device__ __forceinline__ unsigned surfel_blocks(const SplatHot& h, int tile_px, int tile_py, int flags) {
   if (flags & kFlagNoCull) return (unsigned) ((1ull << BlockShape<kLanes>::kPerTile) - 1ull);
-  return footprint_blocks<kLanes>(surfel_footprint(h.m, h.cx, h.cy, h.opacity), tile_px, tile_py);
+  return footprint_blocks<kLanes, true>(surfel_footprint(h.m, h.cx, h.cy, h.opacity), tile_px, tile_py);
 }
 
-// Fills the lists of one wavefront from the masks of the batch's staged entries (zero past the last one): list g at
+// A 3D Gaussian's conic Q = [[a, b], [b, c]] around (x, y): the ellipse d^T Q d <= 2 ln(255 o). One that is not positive definite
+// has no finite bound.
+__device__ __forceinline__ Footprint conic_footprint(float x, float y, float a, float b, float c, float opacity) {
+#pragma clang fp contract(off)
+  Footprint f;
+  f.ox = x, f.oy = y, f.cx = f.cy = f.disc = 0.0f, f.state = 0;
+  const float oa = 255.0f * opacity;
+  if (!(oa >= 1.0f)) return f;
+  f.state = 1;
+  const float det = a * c - b * b;
+  if (!(det > 0.0f) || !(a > 0.0f)) return f;
+  const float s = 2.0f * (__logf(oa) * 1.0001f + 1e-3f) * __builtin_amdgcn_rcpf(det);
+  if (!(s * a < 1e30f) || !(s * c < 1e30f) || !(fabsf(x) < 1e15f) || !(fabsf(y) < 1e15f)) return f;
+  f.state = 2;
+  footprint_ellipse(f, s * c, s * a, -(s * b));
+  return f;
+}
+
+template <int kLanes>
+__device__ __forceinline__ unsigned conic_blocks(float x, float y, float a, float b, float c, float opacity, int tile_px,
+                                                 int tile_py, int flags) {
+  if (flags & kFlagNoCull) return (unsigned) ((1ull << BlockShape<kLanes>::kPerTile) - 1ull);
+  return footprint_blocks<kLanes, false>(conic_footprint(x, y, a, b, c, opacity), tile_px, tile_py);
+}
+
+// Fills the lists of one wavefront from the masks of the batch's staged entries (lane l holds those of entries
+// l, 64 + l, ...; zero past the last one): list g at
 // lists + g * kEntries, a byte per entry, padded with `kEntries` -- the number of a record that no pixel blends -- to its
 // full length. Blocks without a lane in `lanes` get an empty list. Returns the longest list's length. The LDS serves a
 // wavefront's accesses in order, so no barrier is needed before the lists are read.
 template <int kLanes, int kEntries>
-__device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lists, const unsigned* masks, int wave,
+__device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lists, const unsigned (&masks)[kEntries / kWave], int wave,
                                                  unsigned long long lanes) {
   static_assert(kEntries % kWave == 0 && kEntries < 256, "entry numbers and the padding are bytes");
   constexpr int kPerWave = BlockShape<kLanes>::kPerWave;
@@ -137,7 +165,7 @@ __device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lis
   for (int e = 0; e < kPerWave * kEntries / 8; e += kWave) fill[e + lane] = make_uint2(kFill, kFill);
   unsigned m[kEntries / kWave];
 #pragma unroll
-  for (int c = 0; c < kEntries / kWave; ++c) m[c] = masks[c * kWave + lane] >> (kPerWave * wave);
+  for (int c = 0; c < kEntries / kWave; ++c) m[c] = masks[c] >> (kPerWave * wave);
   int longest = 0;
 #pragma unroll
   for (int g = 0; g < kPerWave; ++g) {
@@ -213,50 +241,79 @@ __device__ __forceinline__ unsigned pair_blocks(unsigned m) {
 
 // ---- lists of the backward kernels: per 4x4 block, with a place for each entry's sums -------------------------------
 // A row of 16 lanes sums an entry's gradient components over its 16 pixels with DPP shifts and stores the totals at the
-// step's place, [row of the tile][step]: an entry's sums from different rows never meet, so nothing is read back, added or
-// ordered while the lists are walked. The flush of the batch adds an entry's up to 16 places in row order. A row has
-// kRowSteps places, which bounds its list: a batch is cut to a half or a quarter of the staged entries when some block is
-// reached by more, and a quarter always fits.
-// 24 places: four blocks of 40.7 KB of LDS per compute unit. 16 (batches of 64) and 32 (three blocks per unit) measure 324 and
-// 413 us on 300k surfels 800x800 against 289.
-constexpr int kRowSteps = 24, kRowBatch = 4 * kRowSteps;
-constexpr int kRowMasks = 128;             // staged masks, padded to whole wavefronts with zeros
-constexpr unsigned char kNotInRow = 0xff;  // rank of an entry that a row's list does not hold
+// step's place: an entry's sums from different rows never meet, so nothing is read back, added or ordered while the lists
+// are walked. The flush of the batch adds an entry's up to 16 places in row order. The rows share out a pool of places by
+// the lengths of their lists; a batch is as many of the staged entries as the pool holds (a long batch evens out the lists'
+// lengths and pays the waits between batches less often).
+constexpr int kRowBatch  = 128;  // entries staged at most: a byte names one, two wavefronts stage them
+constexpr int kRowPlaces = 255;  // a byte names a place; one more, kNoPlace, holds zeros
+constexpr int kNoPlace   = kRowPlaces;
 
-// How many of the `n` staged entries make up the batch. Every wavefront comes to the same answer.
-__device__ __forceinline__ int row_batch(const unsigned (&m)[2], int n) {
-  int most_all = 0, most_half = 0;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const unsigned long long lo = wave_ballot((m[0] & (1u << r)) != 0u), hi = wave_ballot((m[1] & (1u << r)) != 0u);
-    most_all  = max(most_all, (int) (__popcll(lo) + __popcll(hi)));
-    most_half = max(most_half, (int) __popcll(lo & ((1ull << (kRowBatch / 2)) - 1ull)));
-  }
-  return min(n, most_all <= kRowSteps ? kRowBatch : most_half <= kRowSteps ? kRowBatch / 2 : kRowBatch / 4);
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int scan_step(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, true);
+}
+__device__ __forceinline__ int wave_scan(int v) {  // inclusive prefix sums over the lanes
+  v = scan_step<0x111, 0xf>(v), v = scan_step<0x112, 0xf>(v), v = scan_step<0x114, 0xf>(v), v = scan_step<0x118, 0xf>(v);
+  return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
 }
 
-// As build_block_lists, for the four rows of a wavefront: entries [first[r], n) of row r. ranks[e * 16 + row]: the step at
-// which the row meets entry e (kNotInRow was stored there before).
-__device__ __forceinline__ int build_row_lists(unsigned char* __restrict__ lists, unsigned char* __restrict__ ranks,
-                                               const unsigned (&m)[2], int wave, const int (&first)[4], int n) {
+// How many of the staged entries make up the batch (m[c]: masks of entries 64 c + lane, zero past the last of `n`), and
+// `start`, the first place of this wavefront's rows. Every wavefront comes to the same batch.
+__device__ __forceinline__ int row_batch(const unsigned (&m)[2], int n, int wave, int& start) {
+  const unsigned lower = (1u << (4 * wave)) - 1u;  // rows of the wavefronts before this one: counted in the high half
+  const int lo = wave_scan(__popc(m[0]) + (__popc(m[0] & lower) << 16));
+  const int hi = wave_scan(__popc(m[1]) + (__popc(m[1] & lower) << 16)) + __builtin_amdgcn_readlane(lo, 63);
+  const int fits = (int) (__popcll(wave_ballot((lo & 0xffff) <= kRowPlaces)) + __popcll(wave_ballot((hi & 0xffff) <= kRowPlaces)));
+  n = min(n, fits);  // an entry takes 16 places at most, so there is always a batch
+  start = (n > kWave ? __builtin_amdgcn_readlane(hi, n - 1 - kWave) : __builtin_amdgcn_readlane(lo, n - 1)) >> 16;
+  return n;
+}
+
+// As build_block_lists, for the four rows of a wavefront: entries [first[r], n) of row r; the rows' places follow each
+// other from `start` on, before[r] becomes row r's first. places[e * 16 + row]: where the row will store its sums of entry e
+// (kNoPlace was stored there before).
+__device__ __forceinline__ int build_row_lists(unsigned char* __restrict__ lists, unsigned char* __restrict__ places,
+                                               const unsigned (&masks)[2], int wave, const int (&first)[4], int start,
+                                               int (&before)[4], int n) {
   const int lane = __lane_id();
-  if (lane < kRowSteps) ((unsigned*) lists)[lane] = 0x01010101u * (unsigned) kRowBatch;
+  constexpr unsigned kFill = 0x01010101u * (unsigned) kRowBatch;
+  ((uint2*) lists)[lane] = make_uint2(kFill, kFill);
+  const unsigned m[2] = {masks[0] >> (4 * wave), masks[1] >> (4 * wave)};
   int longest = 0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     int count = 0;
+    before[r] = start;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int e = c * kWave + lane;
-      const bool on = (m[c] >> (4 * wave) & (1u << r)) != 0u && e >= first[r] && e < n;
+      const bool on = (m[c] & (1u << r)) != 0u && e >= first[r] && e < n;
       const unsigned long long who = wave_ballot(on);
       const int at = (int) __builtin_amdgcn_mbcnt_hi((unsigned) (who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned) who, count));
-      if (on) lists[r * kRowSteps + at] = (unsigned char) e, ranks[e * 16 + 4 * wave + r] = (unsigned char) at;
+      if (on) lists[r * kRowBatch + at] = (unsigned char) e, places[e * 16 + 4 * wave + r] = (unsigned char) (start + at);
       count += (int) __popcll(who);
     }
+    start += count;
     longest = max(longest, count);
   }
   return longest;
+}
+
+// One entry's sums over the rows that hold it, in row order: kCount components from `first` on of the places named by the 16
+// bytes of `places`. All places are read (rows that do not hold the entry name the zeros), four at a time.
+template <int kStride, int kCount>
+__device__ __forceinline__ void sum_places(const float* __restrict__ sums, const uint4& places, int first, float (&a)[kCount]) {
+  const unsigned w[4] = {places.x, places.y, places.z, places.w};
+#pragma unroll
+  for (int c = 0; c < kCount; ++c) a[c] = 0.0f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const float* src = sums + (w[r >> 2] >> (8 * (r & 3)) & 255u) * kStride + first;
+#pragma unroll
+    for (int c = 0; c < kCount; ++c) a[c] += src[c];
+    if ((r & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four places in flight: what the registers hold
+  }
 }
 
 }  // namespace fsgs

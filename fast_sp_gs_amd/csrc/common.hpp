@@ -57,6 +57,13 @@ __device__ __forceinline__ void lds_barrier() {
 // the compiler materialise the predicate in a register and compare it again.
 __device__ __forceinline__ unsigned long long wave_ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 
+// Makes a value opaque at this point of a loop, so that what is computed from it is not hoisted out: a long inner loop
+// beside it keeps the registers that the hoisted values would hold.
+__device__ __forceinline__ int keep_local(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // float -> int with saturation and NaN -> 0 (what v_cvt_i32_f32 does; spelled out so the result does not depend on
