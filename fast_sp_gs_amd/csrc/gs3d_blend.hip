@@ -8,20 +8,19 @@
 // each tile's list back to front, rebuilding T by division, with the reference's accumulators
 // (sum of c * alpha * T behind the current Gaussian) and without masking the 0.99 clamp.
 //
-// Same skeleton as the surfel blend: one block = one 16x16 tile = 4 wavefronts x 8x8 quadrant, a batch of Gaussians
-// staged in LDS with the next batch's gather in flight, a conservative per-quadrant footprint test (bounding box of the
-// alpha >= 1/255 ellipse) whose ballot is the wavefront's work list, longest lists scheduled first. Where the
-// reference issues 9 + E global float atomics per (pixel, Gaussian) pair, the backward sums the 9 + E gradient
-// components over the 64 pixels of a wavefront with one transposed DPP butterfly, stores each wavefront's partial in
-// its own LDS row (LDS float atomics cost about three cycles per lane here), adds the four rows in wavefront order and
-// flushes one global atomic per Gaussian, component and tile.
-#include "blend.hpp"
+// Same skeleton as the surfel blend: one block = one 16x16 tile = 4 wavefronts, a batch of Gaussians staged in LDS with the
+// next batch's gather in flight, a work list per small block of pixels from an exact bound of the alpha >= 1/255 ellipse
+// (block_lists.hpp), longest lists scheduled first. Where the reference issues 9 + E global float atomics per (pixel,
+// Gaussian) pair, the backward sums the 9 + E gradient components over a 4x4 block with DPP row shifts, adds the tile's rows
+// in row order and flushes one global atomic per Gaussian, component and tile. (The top-k, per-Gaussian and wide-feature kernels
+// below keep one list per 8x8 quadrant.)
+#include "block_lists.hpp"
 #include "ordered_sums.hpp"
 
 namespace fsgs {
 namespace {
 
-constexpr int kG3Batch = 128;   // Gaussians staged per round
+constexpr int kG3Batch = 128;   // Gaussians staged per round of the top-k and wide-feature kernels
 constexpr int kMaxExtra = 4;    // the reference dispatches E = 0..4 (gaussian_render.cu:455-481)
 
 struct __attribute__((aligned(16))) G3Hot {
@@ -36,6 +35,28 @@ struct G3Entry {
   G3Hot hot;
   float feat[3 + kMaxExtra];
 };
+
+// A Gaussian staged for the blend: 48 bytes with at most two extra channels, 64 with more.
+template <int E>
+struct __attribute__((aligned(16))) G3Splat {
+  float x, y, a, b, c, opacity;
+  float feat[3 + E];
+  int id;
+};
+
+template <int E>
+__device__ __forceinline__ G3Splat<E> gather_splat3(int id, const float2* __restrict__ means2D,
+    const float4* __restrict__ conic_opacity, const float* __restrict__ colors, const float* __restrict__ extras) {
+  G3Splat<E> g;
+  const float2 m = means2D[id];
+  const float4 co = conic_opacity[id];
+  g.x = m.x, g.y = m.y, g.a = co.x, g.b = co.y, g.c = co.z, g.opacity = co.w, g.id = id;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) g.feat[k] = colors[3 * (size_t) id + k];
+#pragma unroll
+  for (int k = 0; k < E; ++k) g.feat[3 + k] = extras[(size_t) E * id + k];
+  return g;
+}
 
 template <int E>
 __device__ __forceinline__ G3Entry gather_gaussian(int id, const float2* __restrict__ means2D,
@@ -83,7 +104,8 @@ struct G3Hit {
 // exit, and every fused multiply-add is written out with contraction off: a kernel that inlines this twice gets the
 // same rounding from both copies.
 // `lanes`, if given: mask of the lanes that pass, from the two comparisons' own lane masks (scalar registers).
-__device__ __forceinline__ bool conic_alpha_flat(const G3Hot& h, float pxf, float pyf, G3Hit& o,
+template <typename Gaussian>
+__device__ __forceinline__ bool conic_alpha_flat(const Gaussian& h, float pxf, float pyf, G3Hit& o,
                                                  unsigned long long* lanes = nullptr) {
 #pragma clang fp contract(off)
   o.dx = h.x - pxf, o.dy = h.y - pyf;
@@ -98,7 +120,10 @@ __device__ __forceinline__ bool conic_alpha_flat(const G3Hot& h, float pxf, floa
 // kSnap (gaussian_render.cu:51-63, :100-106, :168-172): the state of every pixel still blending before each 32nd list
 // entry -- sampled_T[B,256], sampled_ar[B,3+E,256] by row-major position inside the tile -- plus bucket_to_tile[B] and
 // the tile's deepest contributor max_contrib[T], which the per-Gaussian backward of the reference consumes.
-template <int E, bool kAccum, bool kSnap>
+// Bound by vector issue (35 instructions a step without extra channels). 300k Gaussians 800x800: 96 -> 59 us with lists per
+// 2x4 block instead of 8x8 quadrant; 25k 639x361: 28 -> 18.
+// kHits: notes which blocks blended an entry (hit_blocks), for the backward.
+template <int E, bool kAccum, bool kSnap, bool kHits>
 __global__ void __launch_bounds__(kBlendThreads) gs3d_forward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
     const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list, const float2* __restrict__ means2D,
     const float4* __restrict__ conic_opacity, const float* __restrict__ colors, const float* __restrict__ extras,
@@ -106,21 +131,28 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_forward_kernel(int flags, 
     int32_t* __restrict__ n_contrib, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
     int32_t* __restrict__ accum_weights_count, const int64_t* __restrict__ bucket_offset,
     int32_t* __restrict__ max_contrib, int32_t* __restrict__ bucket_to_tile, float* __restrict__ sampled_T,
-    float* __restrict__ sampled_ar) {
-  __shared__ G3Hot s_hot[kG3Batch];
-  __shared__ float s_feat[kG3Batch][3 + kMaxExtra + 1];  // odd stride
+    float* __restrict__ sampled_ar, uint32_t* __restrict__ hit_blocks) {
+  // With snapshots the lists end at the buckets of 32 entries, two of which are staged at a time.
+  constexpr int kLanes = 8, kB = kSnap ? 64 : 192;
+  using Shape = BlockShape<kLanes>;
+  __shared__ G3Splat<E> s_splat[kB + 1];  // the last one is what padding names: no pixel blends it
+  __shared__ unsigned s_mask[kB];         // which blocks of the tile each staged Gaussian can reach
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[Shape::kPerTile * kB + 16];
+  __shared__ float s_accw[kAccum ? kB : 1];  // accum_weights_*: sums over the tile per staged Gaussian
+  __shared__ int s_accn[kAccum ? kB : 1];
+  __shared__ uint4 s_hit[kHits ? kB : 1][2];  // which blocks blended each staged Gaussian, a byte per block (hit_bits)
   __shared__ int s_max_contrib;
   const int gx = (W + kTile - 1) / kTile;
   const int tile = scheduled_tile(flags, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW = (size_t) H * W, pix = (size_t) W * py + px;
   const float pxf = (float) px, pyf = (float) py;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t r0 = ranges[2 * (size_t) tile], r1 = ranges[2 * (size_t) tile + 1];
   const int n_todo = (int) (r1 - r0);
-  const int rounds = (n_todo + kG3Batch - 1) / kG3Batch;
+  const int rounds = (n_todo + kB - 1) / kB;
   const int rank = (py - tile_y * kTile) * kTile + (px - tile_x * kTile);  // row-major position inside the tile
   int64_t bucket0 = 0;
   if (kSnap) {
@@ -130,9 +162,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_forward_kernel(int flags, 
     if (threadIdx.x == 0) s_max_contrib = 0;
   }
 
-  // blending state of the pixel (float: its test is one comparison) and of the wavefront (a lane mask in scalar
-  // registers: "is anybody still blending" costs no vector instruction)
-  float live = inside ? 1.0f : -1.0f;
+  // the pixels still blending, as a lane mask in scalar registers
   unsigned long long live_lanes = wave_ballot(inside);
   float T = 1.0f, C[3 + (E > 0 ? E : 1)];
 #pragma unroll
@@ -141,98 +171,104 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_forward_kernel(int flags, 
   float wmax = 0.0f;
   bool flag = false;
 
-  G3Entry next;
-  if ((int) threadIdx.x < min(n_todo, kG3Batch))
-    next = gather_gaussian<E>(point_list[r0 + threadIdx.x], means2D, conic_opacity, colors, extras);
-  for (int b = 0; b < rounds; ++b) {
-    if (__syncthreads_count(live < 0.0f) == kBlendThreads) break;
-    const int n_here = min(kG3Batch, n_todo - b * kG3Batch);
-    if ((int) threadIdx.x < n_here) {
-      next.hot.mask = conic_quadrant_mask(next.hot, tile_x * kTile, tile_y * kTile, flags);
-      s_hot[threadIdx.x] = next.hot;
-#pragma unroll
-      for (int k = 0; k < 3 + E; ++k) s_feat[threadIdx.x][k] = next.feat[k];
+  const bool weights = kAccum && (accum_weights_p || accum_weights_count);
+  // this thread's staged Gaussian: its sums of the batch before go out, its places are cleared for the next
+  auto flush = [&](int b) {
+    const int t = (int) threadIdx.x;
+    if (t >= kB) return;
+    if (weights && s_accn[t] != 0) {
+      const int id = s_splat[t].id;
+      if (accum_weights_p) atomicAdd(&accum_weights_p[id], s_accw[t]);
+      if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[t]);
+      s_accw[t] = 0.0f, s_accn[t] = 0;
+    }
+    if (kHits) {
+      if (b * kB + t < n_todo) hit_blocks[r0 + b * kB + t] = hit_bits(s_hit[t][0], s_hit[t][1]);
+      s_hit[t][0] = s_hit[t][1] = make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  if (threadIdx.x == 0) s_splat[kB] = G3Splat<E>{};  // all zero: alpha is 0
+  if (threadIdx.x < 4) ((unsigned*) &s_list[Shape::kPerTile * kB])[threadIdx.x] = 0u;
+  if (kAccum && threadIdx.x < kB) s_accw[threadIdx.x] = 0.0f, s_accn[threadIdx.x] = 0;
+  if (kHits && threadIdx.x < kB) s_hit[threadIdx.x][0] = s_hit[threadIdx.x][1] = make_uint4(0u, 0u, 0u, 0u);
+  unsigned char* const my_hit = (unsigned char*) &s_hit[0][0] + ((Shape::kPerWave * wave + lane / kLanes) ^ 3);
+  unsigned char* const lists  = &s_list[Shape::kPerWave * wave * kB];
+
+  G3Splat<E> next;
+  if ((int) threadIdx.x < min(n_todo, kB))
+    next = gather_splat3<E>(point_list[r0 + threadIdx.x], means2D, conic_opacity, colors, extras);
+  int b = 0;
+  for (; b < rounds; ++b) {
+    if (__syncthreads_and(live_lanes == 0ull)) break;
+    const int n_here = min(kB, n_todo - b * kB);
+    if ((kAccum || kHits) && b > 0) flush(b - 1);
+    if ((int) threadIdx.x < kB) {
+      unsigned mask = 0u;
+      if ((int) threadIdx.x < n_here) {
+        mask = conic_blocks<kLanes>(next.x, next.y, next.a, next.b, next.c, next.opacity, tile_x * kTile, tile_y * kTile, flags);
+        s_splat[threadIdx.x] = next;
+      }
+      s_mask[threadIdx.x] = mask;
     }
     __syncthreads();
-    const int nxt = (b + 1) * kG3Batch + (int) threadIdx.x;
-    if ((int) threadIdx.x < kG3Batch && nxt < n_todo)
-      next = gather_gaussian<E>(point_list[r0 + nxt], means2D, conic_opacity, colors, extras);
-    for (int c = 0; c < kG3Batch / kWave; ++c) {
-      const int jj = c * kWave + lane;
-      unsigned long long todo = __ballot(jj < n_here && ((s_hot[jj < kG3Batch ? jj : 0].mask >> wave) & 1u));
-      if (!kSnap && todo == 0ull) continue;  // with snapshots the state is stored even where nothing blends
-      // One list entry. A wavefront walks its list alone and the launch lasts as long as its longest tile, so the next
-      // entry's record is requested before the current one is evaluated (alternating registers) and the blend is one
-      // divergent region behind one predicate.
-      auto blend_entry = [&](const G3Hot& hot, int j) {
-#pragma clang fp contract(off)  // two copies of this body exist: both must round alike
-        G3Hit h;
-        unsigned long long pass;
-        const bool hit = conic_alpha_flat(hot, pxf, pyf, h, &pass) && live > 0.0f;
-        pass &= live_lanes;
-        if (pass == 0ull) return;
-        const float test_T = T * (1.0f - h.alpha);
-        const bool sat     = hit && test_T < 0.0001f;
-        live               = sat ? -1.0f : live;
-        live_lanes &= ~(pass & wave_ballot(test_T < 0.0001f));
-        const float w      = h.alpha * T;
-        if (kAccum && (accum_weights_p || accum_weights_count))
-          wave_accumulate_weights(hit && !sat, w, hot.id, accum_weights_p, accum_weights_count);
-        if (hit && !sat) {
-#pragma unroll
-          for (int k = 0; k < 3 + E; ++k) C[k] = fmaf(s_feat[j][k], w, C[k]);
-          if (kAccum) {
-            if (wmax < w) wmax = w, wmax_id = hot.id, flag = true;
-          }
-          T    = test_T;
-          last = b * kG3Batch + j + 1;
-        }
-      };
-      if (kSnap) {
-        // the chunk of 64 staged entries holds two buckets of 32: the state is stored in front of each
-        for (int half = 0; half < 2; ++half) {
-          const int base = c * kWave + half * 32;
-          if (base >= n_here) break;
-          if (live > 0.0f) {
-            const size_t bk = (size_t) (bucket0 + (b * kG3Batch + base) / 32);
-            sampled_T[bk * 256 + rank] = T;
-#pragma unroll
-            for (int k = 0; k < 3 + E; ++k) sampled_ar[(bk * (3 + E) + k) * 256 + rank] = C[k];
-          }
-          unsigned long long part = todo & (half ? 0xffffffff00000000ull : 0x00000000ffffffffull);
-          while (part) {
-            if (live_lanes == 0ull) break;
-            const int j = c * kWave + __builtin_ctzll(part);
-            part &= part - 1;
-            blend_entry(s_hot[j], j);
-          }
-        }
-        continue;
+    const int nxt = (b + 1) * kB + (int) threadIdx.x;
+    if ((int) threadIdx.x < kB && nxt < n_todo)
+      next = gather_splat3<E>(point_list[r0 + nxt], means2D, conic_opacity, colors, extras);
+    auto blend_entry = [&](const G3Splat<E>& splat, int j, int) {
+#pragma clang fp contract(off)  // several copies of this body exist: they must round alike
+      G3Hit h;
+      unsigned long long pass;
+      conic_alpha_flat(splat, pxf, pyf, h, &pass);
+      pass &= live_lanes;
+      if (pass == 0ull) return;
+      const float test_T = T * (1.0f - h.alpha);
+      const unsigned long long sat = pass & wave_ballot(test_T < 0.0001f);
+      live_lanes &= ~sat;
+      const unsigned long long blends = pass & ~sat;
+      const bool blend = __builtin_amdgcn_inverse_ballot_w64(blends);
+      const float w    = h.alpha * T;
+      if (weights) {
+        const int n = (int) __popcll(blends >> (lane & -kLanes) & ((1ull << kLanes) - 1ull));
+        const float sum = block_sum_to_last<kLanes>(blend ? w : 0.0f);
+        if ((lane & (kLanes - 1)) == kLanes - 1 && n > 0) atomicAdd(&s_accw[j], sum), atomicAdd(&s_accn[j], n);
       }
-      auto pop = [&]() {
-        const int j = c * kWave + __builtin_ctzll(todo);
-        todo &= todo - 1;
-        return j;
-      };
-      auto peek = [&]() { return c * kWave + (todo ? __builtin_ctzll(todo) : 0); };
-      G3Hot hot_a = s_hot[peek()], hot_b;
-      while (todo) {
-        if (live_lanes == 0ull) break;
-        {
-          const int j = pop();
-          hot_b       = s_hot[peek()];
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_a, j);
+      if (blend) {
+        if (kHits) my_hit[j * 32] = 1;
+#pragma unroll
+        for (int k = 0; k < 3 + E; ++k) C[k] = fmaf(splat.feat[k], w, C[k]);
+        if (kAccum) {
+          if (wmax < w) wmax = w, wmax_id = splat.id, flag = true;
         }
-        if (todo == 0ull || live_lanes == 0ull) break;
-        {
-          const int j = pop();
-          hot_a       = s_hot[peek()];
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_b, j);
-        }
+        T    = test_T;
+        last = b * kB + j + 1;
       }
+    };
+    unsigned masks[kB / kWave];
+    auto walk = [&]() {
+      const int steps = build_block_lists<kLanes, kB>(lists, masks, wave, live_lanes);
+      walk_block_list(lists + lane / kLanes * kB, steps, [&](int j) { return s_splat[j]; }, blend_entry,
+                      [&]() { return live_lanes != 0ull; });
+    };
+    if (kSnap) {
+      for (int half = 0; half < 2 && half * 32 < n_here; ++half) {
+        if (__builtin_amdgcn_inverse_ballot_w64(live_lanes)) {
+          const size_t bk = (size_t) (bucket0 + (b * kB + half * 32) / 32);
+          sampled_T[bk * 256 + rank] = T;
+#pragma unroll
+          for (int k = 0; k < 3 + E; ++k) sampled_ar[(bk * (3 + E) + k) * 256 + rank] = C[k];
+        }
+        masks[0] = lane >> 5 == half ? s_mask[lane] : 0u;
+        walk();
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < kB / kWave; ++c) masks[c] = s_mask[c * kWave + lane];
+      walk();
     }
+  }
+  if (kAccum || kHits) {
+    __syncthreads();
+    if (b > 0) flush(b - 1);  // entries behind it are behind every pixel's last one
   }
   if (kAccum && flag && accum_max_count) atomicAdd(&accum_max_count[wmax_id], 1);
   if (inside) {
@@ -353,44 +389,45 @@ struct G3Scatter {
   }
 };
 
-// Nine per-lane values summed over the 64 lanes: lane l of 0..8 returns the total of v[l]. The first eight go through three
-// steps of the transposed butterfly and meet their row's other half in one addition, the ninth is summed along its row and
-// takes the other half's place: 27 instructions in front of the exchange between rows, 45 for a butterfly of sixteen.
-__device__ __forceinline__ float wave_sum9_transposed(const float (&v)[9]) {
+// Nine per-lane values summed over each 16-lane row, as row_sum16_transposed does: an even lane l returns the row's total of
+// v[(l >> 3) * 4 + (l >> 2 & 1) * 2 + (l >> 1 & 1)], an odd one that of v[8]. 21 instructions.
+__device__ __forceinline__ float row_sum9_transposed(const float (&v)[9]) {
 #pragma clang fp contract(off)
   const int lane = __lane_id();
-  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
-  float w[4], x[2];
+  float w[5], x[3];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = v[2 * i + 1] + dpp_shift_zero<0x111, 0xf, 0xf>(v[2 * i + 1]);  // row_shr:1, kept by odd lanes
-    const float b = v[2 * i] + dpp_shift_zero<0x101, 0xf, 0xf>(v[2 * i]);          // row_shl:1, kept by even lanes
-    w[i] = b0 ? a : b;
-  }
+  for (int i = 0; i < 4; ++i) w[i] = v[i] + dpp_shift_zero<0x128, 0xf, 0xf>(v[i]);  // row_ror:8
+  w[4] = v[8] + dpp_shift_zero<0x128, 0xf, 0xf>(v[8]);
+  asm volatile("s_nop 1\n\t"
+               "v_add_f32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "v_add_f32_dpp %1, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "v_add_f32_dpp %2, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "v_add_f32_dpp %3, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "s_nop 1"
+               : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3])
+               : "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float a = w[2 * i + 1] + dpp_shift_zero<0x112, 0xf, 0xf>(w[2 * i + 1]);
-    const float b = w[2 * i] + dpp_shift_zero<0x102, 0xf, 0xf>(w[2 * i]);
-    x[i] = b1 ? a : b;
-  }
-  const float a = x[1] + dpp_shift_zero<0x114, 0xf, 0xf>(x[1]);
-  const float b = x[0] + dpp_shift_zero<0x104, 0xf, 0xf>(x[0]);
-  float y = b2 ? a : b;
-  y += dpp_shift_zero<0x128, 0xf, 0xf>(y);  // row_ror:8
-  float z = v[8];
-  z += dpp_shift_zero<0x128, 0xf, 0xf>(z);
-  z += dpp_shift_zero<0x124, 0xf, 0xf>(z);
-  z += dpp_shift_zero<0x122, 0xf, 0xf>(z);
-  z += dpp_shift_zero<0x121, 0xf, 0xf>(z);
-  return cross_row_sum(b3 ? z : y);
+  for (int i = 0; i < 2; ++i) x[i] = w[i] + dpp_shift_zero<0x104, 0xf, 0xf>(w[i]);  // row_shl:4
+  x[2] = w[4] + dpp_shift_zero<0x124, 0xf, 0xf>(w[4]);                               // row_ror:4, of halves that are alike
+  asm volatile("s_nop 1\n\t"
+               "v_add_f32_dpp %0, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+               "v_add_f32_dpp %1, %3, %3 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+               "s_nop 1"
+               : "+v"(x[0]), "+v"(x[1])
+               : "v"(w[2]), "v"(w[3]));
+  const float a = x[1] + dpp_shift_zero<0x112, 0xf, 0xf>(x[1]);  // row_shr:2, kept by lanes with bit 1
+  const float b = x[0] + dpp_shift_zero<0x102, 0xf, 0xf>(x[0]);  // row_shl:2
+  const float y = (lane & 2) ? a : b;
+  const float z = x[2] + dpp_shift_zero<0x122, 0xf, 0xf>(x[2]);  // row_ror:2, of quarters that are alike
+  const float c = z + dpp_shift_zero<0x111, 0xf, 0xf>(z);        // row_shr:1, kept by odd lanes
+  const float d = y + dpp_shift_zero<0x101, 0xf, 0xf>(y);        // row_shl:1
+  return (lane & 1) ? c : d;
 }
 
-// The walk is bound by the vector instructions of a (wavefront, entry) pair: without extra channels nine sums cross the lanes,
-// not sixteen, and the factor -opacity, the same for every pixel, is applied to the sums. The flush was bound by its atomics:
-// one lane per Gaussian and one instruction per component made every lane of it a memory request of its own, from one
-// wavefront while three waited. Sixteen lanes per Gaussian, a component each, are three requests (a line per gradient
-// tensor) and keep all wavefronts busy. 300k Gaussians 800x800: 226 -> 182 us, 178 with
-// the next entry requested ahead.
+// Bound by vector issue. Without extra channels nine sums cross the lanes, not sixteen, and the factor -opacity, the same for
+// every pixel, is applied to the sums; the flush takes sixteen lanes per Gaussian, a component each, whose atomics are three
+// requests (a line per gradient tensor). 300k Gaussians 800x800: 177 -> 140 us with a row of lanes per 4x4 block instead of
+// a wavefront per 8x8 quadrant, over the blocks that the forward noted.
 // kSlots: the per-Gaussian sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
 template <int E, bool kSlots>
 __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
@@ -400,20 +437,25 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     const float* __restrict__ dL_dout_extras, const float* __restrict__ dL_dout_opacity,
     float* __restrict__ g_means2D, float* __restrict__ g_conic_opacity, float* __restrict__ g_colors,
     float* __restrict__ g_extras, const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii,
-    float* __restrict__ slot_records) {
-  constexpr int kB = 64;
+    float* __restrict__ slot_records, const uint32_t* __restrict__ hit_blocks) {
+  constexpr int kB = kRowBatch;
+  using Shape = BlockShape<16>;
   // components that cross the lanes: 0-2 colour | 3-6 extras | 7-8 mean2D | 9-11 conic | 12 opacity, without extras close up
   constexpr bool kNine = E == 0;
-  constexpr int kGeom = kNine ? 3 : 7, kSums = kNine ? 9 : 16, kRow = kNine ? 9 : 17;
-  __shared__ G3Hot s_hot[kB];
-  __shared__ float s_feat[kB][3 + kMaxExtra + 1];
-  __shared__ float s_part[4][kB][kRow];  // each wavefront's sums per staged Gaussian: plain stores, added in wavefront order
-  __shared__ float2 s_tag[2][kB];  // number | opacity of the staged Gaussians: the flush reads them while the next are staged
+  constexpr int kGeom = kNine ? 3 : 7, kSums = kNine ? 9 : 16;
+  __shared__ G3Splat<E> s_splat[kB + 1];  // the last one is what padding names: no pixel blends it
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kB + 16];
+  __shared__ float s_sum[kRowPlaces + 1][kSums];
+  __shared__ float s_total[kB][kSums + (kNine ? 0 : 1)];  // over the tile, written and read by the same wavefront
+  // What the flush of a batch reads is kept twice, by batch parity: the next batch is staged while others still flush.
+  __shared__ uint4 s_place[2][kB];  // where each of the 16 rows stores its sums of each staged Gaussian
+  __shared__ float2 s_tag[2][kB];   // its number and opacity
+  __shared__ unsigned s_mask[kB];   // which 4x4 blocks of the tile it can reach
   __shared__ int s_max_contrib;
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int tile = scheduled_tile(flags, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW = (size_t) H * W, pix = (size_t) W * py + px;
   const float pxf = (float) px, pyf = (float) py;
@@ -423,14 +465,18 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
 
   if (threadIdx.x == 0) s_max_contrib = 0;
   __syncthreads();
-  int wave_max = last_contrib;
+  int row_max = last_contrib;  // deepest position blended in this lane's 4x4 block
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) wave_max = max(wave_max, __shfl_xor(wave_max, d, kWave));
-  if (lane == 0) atomicMax(&s_max_contrib, wave_max);
-  for (int e = threadIdx.x; e < 4 * kB * kRow; e += kBlendThreads) (&s_part[0][0][0])[e] = 0.0f;
+  for (int d = 8; d >= 1; d >>= 1) row_max = max(row_max, __shfl_xor(row_max, d, kWave));
+  int row_last[4];  // the same of the wavefront's four blocks
+#pragma unroll
+  for (int r = 0; r < 4; ++r) row_last[r] = __builtin_amdgcn_readlane(row_max, 16 * r);
+  if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
+  if (threadIdx.x == 0) s_splat[kB] = G3Splat<E>{};  // all zero: alpha is 0
+  if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kB])[threadIdx.x] = 0u;
+  if (threadIdx.x < kSums) s_sum[kNoPlace][threadIdx.x] = 0.0f;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));
-  const int rounds = (n_todo + kB - 1) / kB;
   // No zero fill of the record buffer: every staged instance writes its record at the flush, zeros included, and the
   // instances behind the tile's deepest contributor, which are never staged, are cleared here.
   if (kSlots) {
@@ -455,49 +501,66 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     g_out[k] = !inside ? 0.0f : (k < 3 ? dL_dpix[k * HW + pix] : dL_dout_extras[(k - 3) * HW + pix]);
   }
 
-  G3Entry next;
+  G3Splat<E> next;
+  unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
   size_t slot = 0;  // record position of the entry this lane staged (the same lane flushes it)
-  auto gather = [&](int at) {
-    next = gather_gaussian<E>(point_list[r0 + at], means2D, conic_opacity, colors, extras);
-    if (kSlots) next_radius = radii[next.hot.id], next_off = next.hot.id == 0 ? 0 : point_offsets[next.hot.id - 1];
+  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  auto gather = [&](int done) {
+    const int e = (int) threadIdx.x;
+    if (e >= min(kB, n_todo - done)) return;
+    const int64_t at = r0 + (n_todo - 1 - done - e);
+    if (hit_blocks) next_hits = hit_blocks[at];
+    next = gather_splat3<E>(point_list[at], means2D, conic_opacity, colors, extras);
+    if (kSlots) next_radius = radii[next.id], next_off = next.id == 0 ? 0 : point_offsets[next.id - 1];
   };
-  if ((int) threadIdx.x < min(n_todo, kB)) gather(n_todo - 1 - (int) threadIdx.x);
-  for (int b = 0; b < rounds; ++b) {
-    const int n_here = min(kB, n_todo - b * kB);
-    if ((int) threadIdx.x < n_here) {
-      next.hot.mask = conic_quadrant_mask(next.hot, tile_x * kTile, tile_y * kTile, flags);
-      s_hot[threadIdx.x] = next.hot;
-      if (!kSlots) s_tag[b & 1][threadIdx.x] = make_float2(__int_as_float(next.hot.id), next.hot.opacity);
-#pragma unroll
-      for (int k = 0; k < 3 + E; ++k) s_feat[threadIdx.x][k] = next.feat[k];
-      if (kSlots) {
-        // the binning emits a Gaussian's tiles row-major over its rectangle, from its prefix-scan offset on
-        const TileRect r = tile_rect(next.hot.x, next.hot.y, next_radius, gx, gy);
-        slot = (size_t) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
+  gather(0);
+  for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    const int n_staged = min(kB, n_todo - done);
+    if ((int) threadIdx.x < kB) {
+      const int e = (int) threadIdx.x;
+      unsigned mask = 0u;
+      if (e < n_staged) {
+        mask = hit_blocks ? pair_blocks(next_hits)
+                          : conic_blocks<16>(next.x, next.y, next.a, next.b, next.c, next.opacity, tile_x * kTile,
+                                             tile_y * kTile, flags);
+        s_splat[e]       = next;
+        s_tag[parity][e] = make_float2(__int_as_float(next.id), next.opacity);
+        s_place[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        if (kSlots) {
+          // the binning emits a Gaussian's tiles row-major over its rectangle, from its prefix-scan offset on
+          const TileRect r = tile_rect(next.x, next.y, next_radius, gx, gy);
+          slot = (size_t) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
+        }
       }
+      s_mask[e] = mask;
     }
     __syncthreads();
-    const int nxt = (b + 1) * kB + (int) threadIdx.x;
-    if ((int) threadIdx.x < kB && nxt < n_todo) gather(n_todo - 1 - nxt);
-
-    unsigned long long todo = __ballot(lane < n_here && ((s_hot[lane].mask >> wave) & 1u) &&
-                                       (n_todo - 1 - (b * kB + lane)) < wave_max);
-    // The next entry's record and channels are requested before the current entry is evaluated, into alternating registers: a
-    // wavefront walks its list alone, and an exposed LDS round trip per entry sits on the tile's critical path.
-    struct Staged {
-      G3Hot hot;
-      float feat[3 + E];
-    };
-    auto entry = [&](const Staged& at, int j) {
-      const G3Hot& hot        = at.hot;
-      const float* const feat = at.feat;
-      const int pos = n_todo - 1 - (b * kB + j);  // 0-based position in the tile's list
+    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    int start, before[4];
+    const int n_here = row_batch(masks, n_staged, wave, start);
+    gather(done + n_here);
+    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+    const int behind = n_todo - done;
+    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+    const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
+                                      n_here);
+    const int my_first = behind - last_contrib;
+    // component that this lane stores, and its place of step 0
+    const int my_part = !kNine ? lane & 15 : (lane & 1) ? 8 : (lane >> 3 & 1) * 4 + (lane >> 2 & 1) * 2 + (lane >> 1 & 1);
+    const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+    float* const sums = &s_sum[place][my_part];
+    auto entry = [&](const G3Splat<E>& splat, int j, int i) {
       G3Hit h;
       unsigned long long pass;
-      const bool hit = conic_alpha_flat(hot, pxf, pyf, h, &pass) && (pos < last_contrib);
-      if ((pass & wave_ballot(pos < last_contrib)) == 0ull) return;
+      conic_alpha_flat(splat, pxf, pyf, h, &pass);
+      pass &= wave_ballot(j >= my_first);
+      if (pass == 0ull) {
+        if (j != kB) sums[i * kSums] = 0.0f;  // not a padding step; zeros, too, have their place
+        return;
+      }
+      const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
       // Under `hit`: the pixel's back-to-front state and two factors (zero in a lane that does not blend the entry). The
       // components are their products with quantities that are finite in every lane, formed by all lanes alike, so none
       // needs a zero of its own.
@@ -509,7 +572,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
         float dL_dalpha = 0.0f;
 #pragma unroll
         for (int k = 0; k < 3 + E; ++k) {
-          const float v = feat[k];
+          const float v = splat.feat[k];
           dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
           accum[k] += v * dch;
         }
@@ -522,59 +585,36 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
 #pragma unroll
       for (int k = 0; k < 3 + E; ++k) g[k] = dch * g_out[k];
       // the geometry's part without the factor -opacity
-      g[kGeom]     = GdA * (hot.a * h.dx + hot.b * h.dy);
-      g[kGeom + 1] = GdA * (hot.c * h.dy + hot.b * h.dx);
+      g[kGeom]     = GdA * (splat.a * h.dx + splat.b * h.dy);
+      g[kGeom + 1] = GdA * (splat.c * h.dy + splat.b * h.dx);
       g[kGeom + 2] = h.dx * h.dx * GdA;
       g[kGeom + 3] = h.dx * h.dy * GdA;
       g[kGeom + 4] = h.dy * h.dy * GdA;
       g[kGeom + 5] = GdA;
       float tot;
-      if constexpr (kNine) tot = wave_sum9_transposed(g);
-      else tot = wave_sum16_transposed(g);
-      if (lane < kSums) s_part[wave][j][lane] = tot;  // a wavefront meets an entry once per batch
+      if constexpr (kNine) tot = row_sum9_transposed(g);
+      else tot = row_sum16_transposed(g);
+      if (j != kB) sums[i * kSums] = tot;
     };
-    auto pop = [&]() {
-      const int j = __builtin_ctzll(todo);
-      todo &= todo - 1;
-      return j;
-    };
-    auto peek = [&]() {
-      const int j = todo ? (int) __builtin_ctzll(todo) : 0;
-      Staged at;
-      at.hot = s_hot[j];
-#pragma unroll
-      for (int k = 0; k < 3 + E; ++k) at.feat[k] = s_feat[j][k];
-      return at;
-    };
-    if (todo != 0ull) {
-      Staged one = peek(), two;
-      while (todo) {
-        {
-          const int j = pop();
-          two         = peek();
-          __builtin_amdgcn_sched_barrier(0);
-          entry(one, j);
-        }
-        if (todo == 0ull) break;
-        {
-          const int j = pop();
-          one         = peek();
-          __builtin_amdgcn_sched_barrier(0);
-          entry(two, j);
-        }
-      }
-    }
+    walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j]; }, entry,
+                    [] { return true; });
     __syncthreads();
+    // Two lanes per entry add its rows; a wavefront keeps the totals of its 32 entries for itself.
+    static_assert(kBlendThreads == 2 * kB);
+    if (const int e = (int) threadIdx.x >> 1; e < n_here) {
+      constexpr int kHalf = (kSums + 1) / 2;
+      const int h = (int) threadIdx.x & 1;
+      float a[kHalf];
+      sum_places<kSums>(&s_sum[0][0], s_place[parity][e], h * (kSums / 2), a);
+#pragma unroll
+      for (int c = 0; c < kHalf; ++c) s_total[e][h * (kSums / 2) + c] = a[c];
+    }
+    if (kSlots) __syncthreads();
     if (kSlots && (int) threadIdx.x < n_here) {
       float sums[kSums], a[16];
 #pragma unroll
-      for (int c = 0; c < kSums; ++c) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) sum += s_part[w][threadIdx.x][c], s_part[w][threadIdx.x][c] = 0.0f;
-        sums[c] = sum;
-      }
-      const float no = -s_hot[threadIdx.x].opacity;
+      for (int c = 0; c < kSums; ++c) sums[c] = s_total[threadIdx.x][c];
+      const float no = -s_tag[parity][threadIdx.x].y;
 #pragma unroll
       for (int c = 0; c < 16; ++c) a[c] = c < 3 + E ? sums[c < kGeom ? c : 0] : 0.0f;
       a[7] = no * sums[kGeom], a[8] = no * sums[kGeom + 1];
@@ -589,19 +629,20 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
       if (c < 3 + E || (g >= 0 && g < 6)) {
         float* const out = c < 3 ? g_colors + c : c < 3 + E ? g_extras + (c - 3) : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
         const size_t row = c < 3 ? 3 : c < 3 + E ? E : g < 2 ? 2 : 4;
-        for (int e = (int) threadIdx.x >> 4; e < n_here; e += kBlendThreads / 16) {
-          float sum = 0.0f;
-#pragma unroll
-          for (int w = 0; w < 4; ++w) sum += s_part[w][e][c], s_part[w][e][c] = 0.0f;
-          const float2 tag = s_tag[b & 1][e];
+        for (int k = 0; k < kB / 16; ++k) {
+          const int e = wave * (kB / 4) + 4 * k + (lane >> 4);
+          if (e >= n_here) break;
+          float sum = s_total[e][c];
+          const float2 tag = s_tag[parity][e];
           if (g >= 0 && g < 5) sum *= -tag.y;
           if (g == 2 || g == 4) sum *= 0.5f;
           if (sum != 0.0f) atomicAdd(out + row * (size_t) __float_as_int(tag.x), sum);
         }
       }
     }
-    // between this flush and the barrier that follows the next batch's LDS store, wavefronts touch s_part (the flush) and
-    // the other copy of s_tag; with kSlots a lane touches its own rows of s_part and its own staged entry
+    done += n_here;
+    // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
+    // Gaussians, which nobody reads before, and the other copy of what the flush reads.
   }
 }
 
@@ -997,11 +1038,13 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_extra_backward_kernel(int 
 
 using namespace fsgs;
 
-FSGS_API int fsgs_gaussian_rasterize_forward(int P, int W, int H, int E, const float* means2D,
+namespace {
+// hit_blocks[R], if given (without snapshots): per list entry the 2x4 blocks of its tile with a pixel that blended it
+int rasterize_forward(int P, int W, int H, int E, const float* means2D,
     const float* conic_opacity, const float* colors, const float* extras, const int32_t* point_list,
     const int64_t* ranges, int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count,
     const int64_t* bucket_offset, float* out_color, float* out_opacity, float* out_extras, int32_t* n_contrib,
-    int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_ar, void* stream) {
+    int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_ar, uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gaussian_rasterize_forward: bad sizes");
   const bool snap = bucket_offset != nullptr;
   FSGS_REQUIRE(!snap || (max_contrib && bucket_to_tile && sampled_T && sampled_ar),
@@ -1016,17 +1059,19 @@ FSGS_API int fsgs_gaussian_rasterize_forward(int P, int W, int H, int E, const f
   const int flags = launch_tile_order(gx, gy, ranges, s, &tile_order);
   const dim3 grid(gx * gy), block(kBlendThreads);
   const bool accum = accum_max_count || accum_weights_p || accum_weights_count;
-#define FSGS_G3_FWD(EE, ACC, SNAP)                                                                                  \
-  hipLaunchKernelGGL((gs3d_forward_kernel<EE, ACC, SNAP>), grid, block, 0, s, flags, tile_order, W, H, ranges,      \
+#define FSGS_G3_FWD(EE, ACC, SNAP, HITS)                                                                            \
+  hipLaunchKernelGGL((gs3d_forward_kernel<EE, ACC, SNAP, HITS>), grid, block, 0, s, flags, tile_order, W, H, ranges,      \
                      point_list, (const float2*) means2D, (const float4*) conic_opacity, colors, extras, out_color, \
                      out_opacity, out_extras, n_contrib, accum_max_count, accum_weights_p, accum_weights_count,     \
-                     bucket_offset, max_contrib, bucket_to_tile, sampled_T, sampled_ar)
+                     bucket_offset, max_contrib, bucket_to_tile, sampled_T, sampled_ar, hit_blocks)
 #define FSGS_G3_FWD_E(EE)                                     \
   do {                                                        \
-    if (accum && snap) FSGS_G3_FWD(EE, true, true);           \
-    else if (accum) FSGS_G3_FWD(EE, true, false);             \
-    else if (snap) FSGS_G3_FWD(EE, false, true);              \
-    else FSGS_G3_FWD(EE, false, false);                       \
+    if (accum && snap) FSGS_G3_FWD(EE, true, true, false);    \
+    else if (snap) FSGS_G3_FWD(EE, false, true, false);       \
+    else if (accum && hit_blocks) FSGS_G3_FWD(EE, true, false, true); \
+    else if (accum) FSGS_G3_FWD(EE, true, false, false);      \
+    else if (hit_blocks) FSGS_G3_FWD(EE, false, false, true); \
+    else FSGS_G3_FWD(EE, false, false, false);                \
   } while (0)
   switch (E) {
     case 0: FSGS_G3_FWD_E(0); break;
@@ -1038,6 +1083,26 @@ FSGS_API int fsgs_gaussian_rasterize_forward(int P, int W, int H, int E, const f
 #undef FSGS_G3_FWD_E
 #undef FSGS_G3_FWD
   return check_launch("gaussian_rasterize_forward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gaussian_rasterize_forward(int P, int W, int H, int E, const float* means2D,
+    const float* conic_opacity, const float* colors, const float* extras, const int32_t* point_list,
+    const int64_t* ranges, int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count,
+    const int64_t* bucket_offset, float* out_color, float* out_opacity, float* out_extras, int32_t* n_contrib,
+    int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_ar, void* stream) {
+  return rasterize_forward(P, W, H, E, means2D, conic_opacity, colors, extras, point_list, ranges, accum_max_count,
+                           accum_weights_p, accum_weights_count, bucket_offset, out_color, out_opacity, out_extras, n_contrib,
+                           max_contrib, bucket_to_tile, sampled_T, sampled_ar, nullptr, stream);
+}
+
+FSGS_API int fsgs_gaussian_view_forward(int P, int W, int H, int E, const float* means2D, const float* conic_opacity,
+    const float* colors, const float* extras, const int32_t* point_list, const int64_t* ranges, int32_t* accum_max_count,
+    float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
+    int32_t* n_contrib, uint32_t* hit_blocks, void* stream) {
+  return rasterize_forward(P, W, H, E, means2D, conic_opacity, colors, extras, point_list, ranges, accum_max_count,
+                           accum_weights_p, accum_weights_count, nullptr, out_color, out_opacity, out_extras, n_contrib,
+                           nullptr, nullptr, nullptr, nullptr, hit_blocks, stream);
 }
 
 FSGS_API size_t fsgs_gaussian_rasterize_backward_workspace_bytes(int64_t R) {
@@ -1077,12 +1142,13 @@ FSGS_API int fsgs_gaussian_rasterize_clear_culled(int P, int64_t R, const int64_
   return check_launch("gaussian_rasterize_clear_culled");
 }
 
-FSGS_API int fsgs_gaussian_rasterize_backward(int P, int W, int H, int E, const float* means2D,
+namespace {
+int rasterize_backward(int P, int W, int H, int E, const float* means2D,
     const float* conic_opacity, const float* colors, const float* extras, const float* out_opacity,
     const int32_t* n_contrib, const float* dL_dpix, const float* dL_dout_extras, const float* dL_dout_opacity,
     const int32_t* point_list, const int64_t* ranges, float* g_means2D, float* g_conic_opacity, float* g_colors,
     float* g_extras, int64_t R, const int64_t* point_offsets, const int32_t* radii, void* workspace,
-    size_t workspace_bytes, void* stream) {
+    size_t workspace_bytes, const uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gaussian_rasterize_backward: bad sizes");
   FSGS_REQUIRE(E >= 0 && E <= kMaxExtra, "gaussian_rasterize_backward: only 0..%d extra channels are supported", kMaxExtra);
   if (P == 0) return kOk;
@@ -1109,7 +1175,7 @@ FSGS_API int fsgs_gaussian_rasterize_backward(int P, int W, int H, int E, const 
   hipLaunchKernelGGL((gs3d_backward_kernel<EE, SL>), grid, block, 0, s, flags, tile_order, W, H, ranges, point_list, \
                      (const float2*) means2D, (const float4*) conic_opacity, colors, extras, out_opacity, n_contrib, \
                      dL_dpix, dL_dout_extras, dL_dout_opacity, g_means2D, g_conic_opacity, g_colors, g_extras,      \
-                     point_offsets, radii, ws.records)
+                     point_offsets, radii, ws.records, hit_blocks)
 #define FSGS_G3_BWD_E(EE)                                                                                           \
   do {                                                                                                              \
     if (slots) {                                                                                                    \
@@ -1129,6 +1195,28 @@ FSGS_API int fsgs_gaussian_rasterize_backward(int P, int W, int H, int E, const 
 #undef FSGS_G3_BWD_E
 #undef FSGS_G3_BWD
   return check_launch("gaussian_rasterize_backward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gaussian_rasterize_backward(int P, int W, int H, int E, const float* means2D,
+    const float* conic_opacity, const float* colors, const float* extras, const float* out_opacity,
+    const int32_t* n_contrib, const float* dL_dpix, const float* dL_dout_extras, const float* dL_dout_opacity,
+    const int32_t* point_list, const int64_t* ranges, float* g_means2D, float* g_conic_opacity, float* g_colors,
+    float* g_extras, int64_t R, const int64_t* point_offsets, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, void* stream) {
+  return rasterize_backward(P, W, H, E, means2D, conic_opacity, colors, extras, out_opacity, n_contrib, dL_dpix, dL_dout_extras,
+                            dL_dout_opacity, point_list, ranges, g_means2D, g_conic_opacity, g_colors, g_extras, R,
+                            point_offsets, radii, workspace, workspace_bytes, nullptr, stream);
+}
+
+// Sums by atomics, over the blocks that blended an entry, as the forward noted them (nullptr: bounded here).
+FSGS_API int fsgs_gaussian_view_backward(int P, int W, int H, int E, const float* means2D, const float* conic_opacity,
+    const float* colors, const float* extras, const float* out_opacity, const int32_t* n_contrib, const float* dL_dpix,
+    const float* dL_dout_extras, const float* dL_dout_opacity, const int32_t* point_list, const int64_t* ranges,
+    float* g_means2D, float* g_conic_opacity, float* g_colors, float* g_extras, const uint32_t* hit_blocks, void* stream) {
+  return rasterize_backward(P, W, H, E, means2D, conic_opacity, colors, extras, out_opacity, n_contrib, dL_dpix, dL_dout_extras,
+                            dL_dout_opacity, point_list, ranges, g_means2D, g_conic_opacity, g_colors, g_extras, 0, nullptr,
+                            nullptr, nullptr, 0, hit_blocks, stream);
 }
 
 // The reference's second backward walks 32-entry buckets from the forward's snapshots, one warp per bucket

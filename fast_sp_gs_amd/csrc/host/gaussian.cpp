@@ -16,6 +16,7 @@ struct Saved : torch::CustomClassHolder {  // what the backward reads besides te
 struct Buffers {
   Tensor radii, visible, ranges, point_list, n_contrib, conic_opacity;
   Tensor image, opacity, extras;
+  Tensor hit_blocks;  // per list entry, for the backward
   Slab keep;
   c10::intrusive_ptr<Saved> saved;
 };
@@ -111,12 +112,12 @@ Buffers forward_view(const GaussianView& v, bool train) {
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
   }
-  check(fsgs_gaussian_rasterize_forward((int) P, W, H, E, f32(v.means2D), f32(b.conic_opacity), colors,
-                                        E ? f32(*v.extras) : nullptr, i32(b.point_list), i64(b.ranges),
-                                        i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
-                                        i32(opt(v.accum_weights_count)), nullptr, f32(b.image), f32(b.opacity),
-                                        E ? f32(b.extras) : nullptr, i32(b.n_contrib), nullptr, nullptr, nullptr, nullptr,
-                                        stream),
+  if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);
+  check(fsgs_gaussian_view_forward((int) P, W, H, E, f32(v.means2D), f32(b.conic_opacity), colors,
+                                   E ? f32(*v.extras) : nullptr, i32(b.point_list), i64(b.ranges),
+                                   i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
+                                   i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity),
+                                   E ? f32(b.extras) : nullptr, i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), stream),
         blend);
   return b;
 }
@@ -145,7 +146,7 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
     const Buffers& b = *out;
     ctx->save_for_backward({v.points, v.scales, v.rotations, v.opacities, v.shs, opt(v.sh_rest), opt(v.cov3D), opt(v.cov2D),
                             v.means2D, opt(v.extras), v.Tw2v, v.Tv2c, v.campos, b.radii, b.ranges, b.point_list,
-                            b.n_contrib, b.conic_opacity, b.opacity, b.keep.memory()});
+                            b.n_contrib, b.conic_opacity, b.opacity, b.keep.memory(), b.hit_blocks});
     ctx->saved_data["view"] = c10::IValue::make_capsule(b.saved);
     ctx->set_materialize_grads(false);
     return outputs_of(v, b);
@@ -194,11 +195,11 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
     if (P > 0) {
       const float* colors = sh ? keep(s.colors) : f32(shs);
       const int M = rest_used ? (int) sh_rest.size(1) : shs.dim() == 3 ? (int) shs.size(1) : 0;
-      check(fsgs_gaussian_rasterize_backward((int) P, W, H, s.E, f32(means2D), f32(conic_opacity), colors,
+      check(fsgs_gaussian_view_backward((int) P, W, H, s.E, f32(means2D), f32(conic_opacity), colors,
                                              s.E ? f32(extras) : nullptr, f32(opacity), i32(n_contrib), f32(g_image),
                                              f32(g_maps), f32(g_opacity), i32(point_list), i64(ranges), f32(g_means2D),
-                                             f32(g_conic), f32(g_colors), s.E ? f32(g_extras) : nullptr, 0, nullptr, nullptr,
-                                             nullptr, 0, stream),
+                                             f32(g_conic), f32(g_colors), s.E ? f32(g_extras) : nullptr,
+                                             (const uint32_t*) i32(t[20]), stream),
             "gaussian_rasterize_backward");
       if (g[2].defined()) g_means2D.add_(g[2]);
       if (g[3].defined()) g_conic.add_(g[3]);

@@ -600,6 +600,12 @@ int fsgs_gaussian_rasterize_forward(int P, int W, int H, int E, const float* mea
     int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count, const int64_t* bucket_offset,
     float* out_color, float* out_opacity, float* out_extras, int32_t* n_contrib, int32_t* max_contrib,
     int32_t* bucket_to_tile, float* sampled_T, float* sampled_ar, void* stream);
+/* The same without snapshots, for a view that will be back-propagated: hit_blocks[R] (nullptr: not wanted) as
+ * fsgs_gs_2d_view_forward leaves it. */
+int fsgs_gaussian_view_forward(int P, int W, int H, int E, const float* means2D, const float* conic_opacity,
+    const float* colors, const float* extras, const int32_t* point_list, const int64_t* ranges, int32_t* accum_max_count,
+    float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
+    int32_t* n_contrib, uint32_t* hit_blocks, void* stream);
 
 /* gaussian_rasterize_backward -- gaussian_render.cu:486-536 (kernel :296-444). g_means2D[P,2], g_conic_opacity[P,4],
  * g_colors[P,3], g_extras[P,E]. With point_offsets == NULL the per-Gaussian sums are accumulated with device-scope
@@ -620,6 +626,12 @@ int fsgs_gaussian_rasterize_backward(int P, int W, int H, int E, const float* me
     const float* dL_dpix, const float* dL_dout_extras, const float* dL_dout_opacity, const int32_t* point_list,
     const int64_t* ranges, float* g_means2D, float* g_conic_opacity, float* g_colors, float* g_extras, int64_t R,
     const int64_t* point_offsets, const int32_t* radii, void* workspace, size_t workspace_bytes, void* stream);
+/* Its sums by atomics (zero-filled outputs), with the hit_blocks that fsgs_gaussian_view_forward left for these lists (nullptr:
+ * footprints are bounded again). */
+int fsgs_gaussian_view_backward(int P, int W, int H, int E, const float* means2D, const float* conic_opacity,
+    const float* colors, const float* extras, const float* out_opacity, const int32_t* n_contrib, const float* dL_dpix,
+    const float* dL_dout_extras, const float* dL_dout_opacity, const int32_t* point_list, const int64_t* ranges,
+    float* g_means2D, float* g_conic_opacity, float* g_colors, float* g_extras, const uint32_t* hit_blocks, void* stream);
 
 /* gaussian_rasterize_fast_backward -- gaussian_render.cu:760-812 (kernel :540-694): the reference's per-Gaussian
  * backward over the forward's bucket snapshots. It is the same derivative as gaussian_rasterize_backward and runs

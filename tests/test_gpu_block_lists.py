@@ -92,3 +92,23 @@ def test_surfel_view(shape, P, device):
         assert torch.equal(a, b)
     for a, b in zip(grads, grads_all):
         assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("P", [1, 127, 128, 129, 191, 192, 193, 900])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_gaussian_view(shape, P, device):
+    from fast_sp_gs_amd.renderer.gaussian_render import render
+    scene, cam = _scene(shape, P, device)
+    fov = (math.radians(40.0), 2 * math.atan(math.tan(math.radians(20.0)) * cam.H / cam.W))
+
+    def run():
+        params = _params(scene, axes=3)
+        out = render(cam.Tw2v, cam.Tv2c, (cam.W, cam.H), campos=cam.campos, FoV=fov, sh_degree=3, **params)
+        maps = [out['images'], out['opacity']]
+        return maps, _gradients(params, maps)
+
+    (maps, grads), (maps_all, grads_all) = _both(run)
+    for a, b in zip(maps, maps_all):
+        assert torch.equal(a, b)
+    for a, b in zip(grads, grads_all):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
