@@ -28,6 +28,7 @@ namespace {
 // The first 16 go through one transposed row reduction; the means2D pair is only non-zero for pixels where the
 // screen-space low-pass filter wins (rho2d < rho3d) and is reduced separately when any lane took that branch.
 constexpr int kGradSlots = 18;
+constexpr int kRowPlaces = 255;  // of a batch: with 36.5 KB of LDS four blocks share a compute unit
 #ifndef FSGS_BWD_WAVES
 #define FSGS_BWD_WAVES 4
 #endif
@@ -85,7 +86,7 @@ blend_backward_kernel(
   for (int r = 0; r < 4; ++r) row_last[r] = __builtin_amdgcn_readlane(row_max, 16 * r);
   if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
   if (threadIdx.x == 0) s_splat[kRowBatch] = Splat{};  // all zero: p_z == 0 everywhere
-  if (threadIdx.x < kGradSlots) s_sum[kNoPlace][threadIdx.x] = 0.0f;
+  if (threadIdx.x < kGradSlots) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
   if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kRowBatch])[threadIdx.x] = 0u;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));  // positions [0, n_todo) of the tile's list, walked from n_todo-1 down to 0
@@ -193,14 +194,14 @@ blend_backward_kernel(
         } else {
           s_slot[parity][e] = next.cold.id;
         }
-        s_place[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        s_place[parity][e] = no_places(kRowPlaces);
       }
       s_mask[e] = mask;
     }
     __syncthreads();
     const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
     int start, before[4];
-    const int n_here = row_batch(masks, n_staged, wave, start);
+    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
     gather(done + n_here);
     // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
     const int behind = n_todo - done;
@@ -247,7 +248,7 @@ blend_backward_kernel(
      // share one instruction stream.
      auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, const Hit& h, bool hit,
                                float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
-       float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
+       float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
        if (hit) {
          advance_pixel(cold, j, h, w, dL_dalpha, dL_dz);
          if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
@@ -268,12 +269,11 @@ blend_backward_kernel(
            acc_w = last_alpha + (1.0f - last_alpha) * acc_w;
            dL_dalpha += (1.0f - acc_w) * dL_dsum_w;
          }
-         dL_dalpha *= T;
+         GdA = dL_dalpha * T * h.G;
          last_alpha = h.alpha;
          // the Gaussian's own part of d/ds: only the intersection case uses it (times 1 / p_z below)
-         const float dL_dG = hot.opacity * dL_dalpha;
-         dsx += dL_dG * -h.G * h.sx;
-         dsy += dL_dG * -h.G * h.sy;
+         oG = hot.opacity * GdA;
+         dsx -= oG * h.sx, dsy -= oG * h.sy;
          // s is not finite in a lane whose plane pair degenerates (p_z == 0), and such a lane never blends: every use
          // of s sits on this side
          s_ds = dsx * h.sx + dsy * h.sy;
@@ -296,8 +296,8 @@ blend_backward_kernel(
        g[11] = dL_dz - (pxf * nkz + pyf * nlz);
        if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
        else      g[12] = g[13] = g[14] = 0.0f;
-       g[15] = h.G * dL_dalpha;
-       const float to_centre = filtered ? hot.opacity * dL_dalpha * (-2.0f * h.G) : 0.0f;
+       g[15] = GdA;
+       const float to_centre = filtered ? -2.0f * oG : 0.0f;
        g2x = to_centre * h.dx, g2y = to_centre * h.dy;
      };
      const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];

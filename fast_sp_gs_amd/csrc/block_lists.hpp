@@ -245,9 +245,8 @@ __device__ __forceinline__ unsigned pair_blocks(unsigned m) {
 // are walked. The flush of the batch adds an entry's up to 16 places in row order. The rows share out a pool of places by
 // the lengths of their lists; a batch is as many of the staged entries as the pool holds (a long batch evens out the lists'
 // lengths and pays the waits between batches less often).
-constexpr int kRowBatch  = 128;  // entries staged at most: a byte names one, two wavefronts stage them
-constexpr int kRowPlaces = 255;  // a byte names a place; one more, kNoPlace, holds zeros
-constexpr int kNoPlace   = kRowPlaces;
+constexpr int kRowBatch = 128;  // entries staged at most: a byte names one, two wavefronts stage them
+// A byte names one of a pool's kPlaces <= 255 places, too; one more behind them, number kPlaces, holds zeros.
 
 template <int kCtrl, int kRows>
 __device__ __forceinline__ int scan_step(int v) {
@@ -258,13 +257,20 @@ __device__ __forceinline__ int wave_scan(int v) {  // inclusive prefix sums over
   return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
 }
 
+__device__ __forceinline__ uint4 no_places(int zeros) {
+  const unsigned w = 0x01010101u * (unsigned) zeros;
+  return make_uint4(w, w, w, w);
+}
+
 // How many of the staged entries make up the batch (m[c]: masks of entries 64 c + lane, zero past the last of `n`), and
 // `start`, the first place of this wavefront's rows. Every wavefront comes to the same batch.
+template <int kPlaces>
 __device__ __forceinline__ int row_batch(const unsigned (&m)[2], int n, int wave, int& start) {
+  static_assert(kPlaces >= 16 && kPlaces <= 255);
   const unsigned lower = (1u << (4 * wave)) - 1u;  // rows of the wavefronts before this one: counted in the high half
   const int lo = wave_scan(__popc(m[0]) + (__popc(m[0] & lower) << 16));
   const int hi = wave_scan(__popc(m[1]) + (__popc(m[1] & lower) << 16)) + __builtin_amdgcn_readlane(lo, 63);
-  const int fits = (int) (__popcll(wave_ballot((lo & 0xffff) <= kRowPlaces)) + __popcll(wave_ballot((hi & 0xffff) <= kRowPlaces)));
+  const int fits = (int) (__popcll(wave_ballot((lo & 0xffff) <= kPlaces)) + __popcll(wave_ballot((hi & 0xffff) <= kPlaces)));
   n = min(n, fits);  // an entry takes 16 places at most, so there is always a batch
   start = (n > kWave ? __builtin_amdgcn_readlane(hi, n - 1 - kWave) : __builtin_amdgcn_readlane(lo, n - 1)) >> 16;
   return n;
@@ -272,7 +278,7 @@ __device__ __forceinline__ int row_batch(const unsigned (&m)[2], int n, int wave
 
 // As build_block_lists, for the four rows of a wavefront: entries [first[r], n) of row r; the rows' places follow each
 // other from `start` on, before[r] becomes row r's first. places[e * 16 + row]: where the row will store its sums of entry e
-// (kNoPlace was stored there before).
+// (the place of zeros was named there before).
 __device__ __forceinline__ int build_row_lists(unsigned char* __restrict__ lists, unsigned char* __restrict__ places,
                                                const unsigned (&masks)[2], int wave, const int (&first)[4], int start,
                                                int (&before)[4], int n) {

@@ -14,15 +14,12 @@
 // (:366, :704), and the per-splat form subtracts the DIVIDED final flow from its partial sums (:706), which amounts to
 // an opacity-map gradient lowered by (final flow . dL/dflow) -- reproduced here in that algebraic form.
 //
-// Layout as in the standard blend: one 256-lane block per tile, wavefront w owns an 8x8 quadrant, surfels staged in
-// LDS (64-byte hot record with the adjugate, 32-byte cold record), per-quadrant work lists from a conservative bound;
-// the backward queues its blended (pixel, entry) pairs and forms their gradient components 64 pairs at a time
-// (pair_queue.hpp).
+// Layout as in the standard blend: one 256-lane block per tile, surfels staged in LDS as 96-byte records with the adjugate, a
+// work list per 2x4 (forward) or 4x4 (backward) block of pixels (block_lists.hpp).
 #include "binning.hpp"
-#include "blend.hpp"
+#include "block_lists.hpp"
 #include "instance_slots.hpp"
 #include "ordered_sums.hpp"
-#include "pair_queue.hpp"
 
 namespace fsgs {
 namespace {
@@ -33,10 +30,12 @@ struct __attribute__((aligned(16))) FastHot {
   float cx, cy, opacity, pad;
 };
 
-struct FastSplat {
+struct FastRecord {
   FastHot hot;
   SplatCold cold;
-  float m[6];  // first two rows of the transform, only used for the quadrant bound while staging
+};
+struct FastSplat : FastRecord {
+  float m[6];  // first two rows of the transform, only used for the footprint's bound while staging
 };
 
 __device__ __forceinline__ FastSplat gather_fast(int id, const float2* __restrict__ means2D,
@@ -61,13 +60,14 @@ __device__ __forceinline__ FastSplat gather_fast(int id, const float2* __restric
   return s;
 }
 
-__device__ __forceinline__ unsigned fast_quadrant_mask(const FastSplat& s, int tile_px, int tile_py, int flags) {
+template <int kLanes>
+__device__ __forceinline__ unsigned fast_blocks(const FastSplat& s, int tile_px, int tile_py, int flags) {
   SplatHot h;
 #pragma unroll
   for (int k = 0; k < 6; ++k) h.m[k] = s.m[k];
   h.m[6] = s.hot.tw0, h.m[7] = s.hot.tw1, h.m[8] = s.hot.tw2;
   h.cx = s.hot.cx, h.cy = s.hot.cy, h.opacity = s.hot.opacity;
-  return quadrant_mask(h, tile_px, tile_py, flags);
+  return surfel_blocks<kLanes>(h, tile_px, tile_py, flags);
 }
 
 struct FastHit {
@@ -104,35 +104,36 @@ __device__ __forceinline__ bool fast_intersect_flat(const FastHot& h, float pxf,
   return c0 & c1 & c3;
 }
 
-// Sums 8 per-lane values over each 16-lane row at once: three merge steps inside aligned groups of 8 lanes, one rotate
-// by 8 inside the row. On return lane l of every row holds that row's total of v[l & 7].
-__device__ __forceinline__ float row_sum8_transposed(const float (&v)[8]) {
+// Five per-lane values summed over each 16-lane row, as row_sum16_transposed does: a lane with bit 1 returns the row's total of
+// v[4], another that of v[(l >> 2 & 1) * 2 + (l >> 3)]. 12 instructions.
+__device__ __forceinline__ float row_sum5_transposed(const float (&v)[5]) {
 #pragma clang fp contract(off)  // an input that is a product must not be formed a second time inside a fused add
   const int lane = __lane_id();
-  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
-  float w[4], x[2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = v[2 * i + 1] + dpp_shift_zero<0x111, 0xf, 0xf>(v[2 * i + 1]);  // row_shr:1
-    const float b = v[2 * i] + dpp_shift_zero<0x101, 0xf, 0xf>(v[2 * i]);          // row_shl:1
-    w[i] = b0 ? a : b;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float a = w[2 * i + 1] + dpp_shift_zero<0x112, 0xf, 0xf>(w[2 * i + 1]);  // row_shr:2
-    const float b = w[2 * i] + dpp_shift_zero<0x102, 0xf, 0xf>(w[2 * i]);          // row_shl:2
-    x[i] = b1 ? a : b;
-  }
-  const float a = x[1] + dpp_shift_zero<0x114, 0xf, 0xf>(x[1]);  // row_shr:4
-  const float b = x[0] + dpp_shift_zero<0x104, 0xf, 0xf>(x[0]);  // row_shl:4
-  float z = b2 ? a : b;
-  z += dpp_shift_zero<0x128, 0xf, 0xf>(z);  // row_ror:8
-  return z;
+  float w0 = v[0] + dpp_shift_zero<0x128, 0xf, 0xf>(v[0]), w1 = v[2] + dpp_shift_zero<0x128, 0xf, 0xf>(v[2]);  // row_ror:8
+  float w2 = v[4] + dpp_shift_zero<0x128, 0xf, 0xf>(v[4]);
+  asm volatile("s_nop 1\n\t"
+               "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "v_add_f32_dpp %1, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+               "s_nop 1"
+               : "+v"(w0), "+v"(w1)
+               : "v"(v[1]), "v"(v[3]));
+  float x = w0 + dpp_shift_zero<0x104, 0xf, 0xf>(w0);              // row_shl:4
+  const float y = w2 + dpp_shift_zero<0x124, 0xf, 0xf>(w2);        // row_ror:4, of halves that are alike
+  asm volatile("s_nop 1\n\t"
+               "v_add_f32_dpp %0, %1, %1 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+               "s_nop 1"
+               : "+v"(x)
+               : "v"(w1));
+  const float a = y + dpp_shift_zero<0x112, 0xf, 0xf>(y);  // row_shr:2, kept by lanes with bit 1
+  const float b = x + dpp_shift_zero<0x102, 0xf, 0xf>(x);  // row_shl:2
+  const float z = (lane & 2) ? a : b;
+  return z + dpp_shift_zero<0xb1, 0xf, 0xf>(z);  // quad_perm [1,0,3,2]
 }
-// The same over the 64 lanes: every lane holds the wave total of v[lane & 7].
-__device__ __forceinline__ float wave_sum8_transposed(const float (&v)[8]) { return cross_row_sum(row_sum8_transposed(v)); }
 
-template <bool kAux, bool kSnap, bool kAccum, bool kFlow>
+// Bound by vector issue. 150k surfels 1001x667: 62 -> 57 us with lists per 2x4 block instead of 8x8 quadrant,
+// noting the blocks (batches of 192 surfels instead of 128: 58; held to five wavefronts per SIMD, which spills: 62).
+// kHits: notes which blocks blended an entry (hit_blocks), for the backward.
+template <bool kAux, bool kSnap, bool kAccum, bool kFlow, bool kHits>
 __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
     const float2* __restrict__ means2D, const float* __restrict__ colors, const float* __restrict__ trans_mat,
@@ -142,18 +143,24 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
     float2* __restrict__ out_flow, int32_t* __restrict__ max_contrib,
     int32_t* __restrict__ bucket_to_tile, float* __restrict__ sampled_T, float* __restrict__ sampled_acc,
     float* __restrict__ sampled_aux, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
-    int32_t* __restrict__ accum_weights_count) {
-  __shared__ FastHot s_hot[kBatch];
-  __shared__ SplatCold s_cold[kBatch];
-  __shared__ float s_t2[kFlow ? kBatch * 9 : 1];  // second-time-step transforms of the staged surfels
-  __shared__ unsigned char s_mask[kBatch];
+    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks) {
+  // With snapshots the lists end at the buckets of 32 entries, two of which are staged at a time.
+  constexpr int kLanes = 8, kB = kSnap ? 64 : 128;
+  using Shape = BlockShape<kLanes>;
+  __shared__ FastRecord s_splat[kB + 1];      // the last one is what padding names: no pixel blends it
+  __shared__ float s_t2[kFlow ? kB * 9 : 1];  // second-time-step transforms of the staged surfels
+  __shared__ unsigned s_mask[kB];             // which blocks of the tile each staged surfel can reach
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[Shape::kPerTile * kB + 16];
+  __shared__ float s_accw[kAccum ? kB : 1];  // accum_weights_*: sums over the tile per staged surfel
+  __shared__ int s_accn[kAccum ? kB : 1];
+  __shared__ uint4 s_hit[kHits ? kB : 1][2];  // which blocks blended each staged surfel, a byte per block (hit_bits)
   __shared__ int s_max_contrib;
   constexpr int kNum = kFlow ? 10 : 8;  // channels of a snapshot
 
   const int gx = (W + kTile - 1) / kTile;
   const int tile = scheduled_tile(ordered, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW   = (size_t) H * W;
   const size_t pix  = (size_t) W * py + px;
@@ -163,7 +170,7 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
 
   const int64_t r0 = ranges[2 * (size_t) tile], r1 = ranges[2 * (size_t) tile + 1];
   const int n_todo = (int) (r1 - r0);
-  const int rounds = (n_todo + kBatch - 1) / kBatch;
+  const int rounds = (n_todo + kB - 1) / kB;
 
   int64_t bucket0 = 0;
   if (kSnap) {
@@ -173,9 +180,7 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
     if (threadIdx.x == 0) s_max_contrib = 0;
   }
 
-  // blending state of the pixel (float: its test is one comparison) and of the wavefront (a lane mask in scalar
-  // registers: "is anybody still blending" costs no vector instruction)
-  float live = inside ? 1.0f : -1.0f;
+  // the pixels still blending, as a lane mask in scalar registers
   unsigned long long live_lanes = wave_ballot(inside);
   const float far_scale = far_n / (far_n - near_n);
   float T = 1.0f, C0 = 0, C1 = 0, C2 = 0;
@@ -183,143 +188,155 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
   int last = 0, median_c = -1;
   ArgmaxRun argmax;
 
+  const bool weights = kAccum && (accum_weights_p || accum_weights_count);
+  uint32_t* const tile_hits = hit_blocks + (kHits ? r0 : 0);
+  // this thread's staged surfel: its sums of the batch before go out, its places are cleared for the next
+  auto flush = [&](int b) {
+    const int t = (int) threadIdx.x;
+    if (t >= kB) return;
+    if (weights && s_accn[t] != 0) {
+      const int id = s_splat[t].cold.id;
+      if (accum_weights_p) atomicAdd(&accum_weights_p[id], s_accw[t]);
+      if (accum_weights_count) atomicAdd(&accum_weights_count[id], s_accn[t]);
+      s_accw[t] = 0.0f, s_accn[t] = 0;
+    }
+    if (kHits) {
+      if (b * kB + t < n_todo) tile_hits[keep_local(b * kB + t)] = hit_bits(s_hit[t][0], s_hit[t][1]);
+      s_hit[t][0] = s_hit[t][1] = make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  if (threadIdx.x == 0) s_splat[kB] = FastRecord{};  // all zero: p_z == 0 everywhere
+  if (threadIdx.x < 4) ((unsigned*) &s_list[Shape::kPerTile * kB])[threadIdx.x] = 0u;
+  if (kAccum && threadIdx.x < kB) s_accw[threadIdx.x] = 0.0f, s_accn[threadIdx.x] = 0;
+  if (kHits && threadIdx.x < kB) s_hit[threadIdx.x][0] = s_hit[threadIdx.x][1] = make_uint4(0u, 0u, 0u, 0u);
+  unsigned char* const my_hit = (unsigned char*) &s_hit[0][0] + ((Shape::kPerWave * wave + lane / kLanes) ^ 3);
+  unsigned char* const lists  = &s_list[Shape::kPerWave * wave * kB];
+
   FastSplat next;
   float next_t2[9];
-  if ((int) threadIdx.x < n_todo) {
-    const int id = point_list[r0 + threadIdx.x];
+  auto gather = [&](int at) {
+    if ((int) threadIdx.x >= kB || at >= n_todo) return;
+    const int id = point_list[r0 + at];
     next = gather_fast(id, means2D, colors, normal_opacity, trans_mat, inverse_m);
     if (kFlow) {
 #pragma unroll
       for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) id + k];
     }
-  }
+  };
+  gather((int) threadIdx.x);
 
-  for (int b = 0; b < rounds; ++b) {
-    if (__syncthreads_count(live < 0.0f) == kBlendThreads) break;
-    const int n_here = min(kBatch, n_todo - b * kBatch);
-    if ((int) threadIdx.x < n_here) {
-      s_hot[threadIdx.x]  = next.hot;
-      s_cold[threadIdx.x] = next.cold;
-      s_mask[threadIdx.x] = (unsigned char) fast_quadrant_mask(next, tile_x * kTile, tile_y * kTile, ordered);
-      if (kFlow) {
+  int b = 0;
+  for (; b < rounds; ++b) {
+    if (__syncthreads_and(live_lanes == 0ull)) break;
+    const int n_here = min(kB, n_todo - b * kB);
+    if ((kAccum || kHits) && b > 0) flush(b - 1);
+    if ((int) threadIdx.x < kB) {
+      unsigned mask = 0u;
+      if ((int) threadIdx.x < n_here) {
+        s_splat[threadIdx.x] = next;
+        mask = fast_blocks<kLanes>(next, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
+        if (kFlow) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+        }
       }
+      s_mask[threadIdx.x] = mask;
     }
     __syncthreads();
-    const int nxt = (b + 1) * kBatch + (int) threadIdx.x;
-    if (nxt < n_todo) {
-      const int id = point_list[r0 + nxt];
-      next = gather_fast(id, means2D, colors, normal_opacity, trans_mat, inverse_m);
-      if (kFlow) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) id + k];
-      }
-    }
+    gather((b + 1) * kB + (int) threadIdx.x);
 
-    for (int c = 0; c < kBatch / kWave; ++c) {
-      const int jj = c * kWave + lane;
-      const unsigned long long todo_all = __ballot(jj < n_here && ((s_mask[jj] >> wave) & 1u));
-      for (int half = 0; half < (kSnap ? 2 : 1); ++half) {
-        unsigned long long todo = todo_all;
-        if (kSnap) {
-          const int base = c * kWave + half * 32;
-          if (base >= n_here) break;
-          if (live > 0.0f) {
-            // state before list entry b * 256 + base, which starts a bucket of 32 (gs_2d_fast_redner.cu:126-147)
-            const size_t bk = (size_t) (bucket0 + (b * kBatch + base) / 32);
-            sampled_T[bk * 256 + rank]             = T;
-            sampled_acc[(bk * 3 + 0) * 256 + rank] = C0;
-            sampled_acc[(bk * 3 + 1) * 256 + rank] = C1;
-            sampled_acc[(bk * 3 + 2) * 256 + rank] = C2;
-            if (kAux) {
-              sampled_aux[(bk * kNum + 0) * 256 + rank] = D;
-              sampled_aux[(bk * kNum + 1) * 256 + rank] = N0;
-              sampled_aux[(bk * kNum + 2) * 256 + rank] = N1;
-              sampled_aux[(bk * kNum + 3) * 256 + rank] = N2;
-              sampled_aux[(bk * kNum + 5) * 256 + rank] = dist;
-              sampled_aux[(bk * kNum + 6) * 256 + rank] = M1;
-              sampled_aux[(bk * kNum + 7) * 256 + rank] = M2;
-              if (kFlow) {
-                sampled_aux[(bk * kNum + 8) * 256 + rank] = f0;
-                sampled_aux[(bk * kNum + 9) * 256 + rank] = f1;
-              }
-            }
-          }
-          todo &= half ? 0xffffffff00000000ull : 0x00000000ffffffffull;
-        }
-        // one entry of the wavefront's work list; its records were requested from LDS while the entry before it ran
-        auto blend_entry = [&](const FastHot& hot, const SplatCold& cold, int j) {
-#pragma clang fp contract(off)  // two copies of this body exist (alternating registers): both must round alike
-          FastHit h;
-          unsigned long long pass;
-          const bool hit = fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass) && live > 0.0f;
-          pass &= live_lanes;
-          if (pass == 0ull) return;
-          const float test_T = T * (1.0f - h.alpha);
-          const bool sat     = hit && test_T < 0.0001f;
-          live               = sat ? -1.0f : live;
-          live_lanes &= ~(pass & wave_ballot(test_T < 0.0001f));
-          const float w         = h.alpha * T;
-          if (kAccum && (accum_weights_p || accum_weights_count))
-            wave_accumulate_weights(hit && !sat, w, cold.id, accum_weights_p, accum_weights_count);
-          if (!hit || sat) return;
-          const int contributor = b * kBatch + j + 1;
-          if (kAux) {
-            const float A = 1.0f - T;
-            const float m = far_scale * (1.0f - near_n * __builtin_amdgcn_rcpf(h.depth));
-            const float mm = m * m;
-            dist = fmaf(fmaf(mm, A, fmaf(-2.0f * m, M1, M2)), w, dist);
-            D    = fmaf(h.depth, w, D);
-            M1   = fmaf(m, w, M1);
-            M2   = fmaf(mm, w, M2);
-            if (T > 0.5f) median = h.depth, median_c = contributor;
-            N0 = fmaf(cold.nx, w, N0), N1 = fmaf(cold.ny, w, N1), N2 = fmaf(cold.nz, w, N2);
-            if (kAccum) argmax_run_step(argmax, w, cold.id, accum_max_count);
-            if (kFlow) {
-              const float* Q = &s_t2[j * 9];
-              const float u2 = fmaf(Q[0], h.sx, fmaf(Q[1], h.sy, Q[2]));
-              const float v2 = fmaf(Q[3], h.sx, fmaf(Q[4], h.sy, Q[5]));
-              float w2       = fmaf(Q[6], h.sx, fmaf(Q[7], h.sy, Q[8]));
-              w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-              f0 = fmaf(u2 / w2 - pxf, w, f0);
-              f1 = fmaf(v2 / w2 - pyf, w, f1);
-            }
-          }
-          C0 = fmaf(cold.r, w, C0), C1 = fmaf(cold.g, w, C1), C2 = fmaf(cold.b, w, C2);
-          T    = test_T;
-          last = contributor;
-        };
-        if (todo == 0ull) continue;
-        auto pop = [&]() {
-          const int j = c * kWave + __builtin_ctzll(todo);
-          todo &= todo - 1;
-          return j;
-        };
-        auto peek = [&]() { return c * kWave + (todo ? __builtin_ctzll(todo) : 0); };
-        FastHot hot_a = s_hot[peek()], hot_b;
-        while (todo) {
-          if (live_lanes == 0ull) break;  // every pixel of this quadrant is saturated
-          {
-            const int j = pop();
-            hot_b       = s_hot[peek()];
-            const SplatCold cold = s_cold[j];  // used only if a pixel blends the surfel, but then without waiting
-            __builtin_amdgcn_sched_barrier(0);
-            blend_entry(hot_a, cold, j);
-          }
-          if (todo == 0ull || live_lanes == 0ull) break;
-          {
-            const int j = pop();
-            hot_a       = s_hot[peek()];
-            const SplatCold cold = s_cold[j];
-            __builtin_amdgcn_sched_barrier(0);
-            blend_entry(hot_b, cold, j);
-          }
-        }
+    auto blend_entry = [&](const FastHot& hot, int j, int) {
+#pragma clang fp contract(off)  // several copies of this body exist (alternating registers): they must round alike
+      const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+      __builtin_amdgcn_sched_barrier(0);
+      FastHit h;
+      unsigned long long pass;
+      fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass);
+      pass &= live_lanes;
+      if (pass == 0ull) return;
+      const float test_T = T * (1.0f - h.alpha);
+      const unsigned long long sat = pass & wave_ballot(test_T < 0.0001f);
+      live_lanes &= ~sat;
+      const unsigned long long blends = pass & ~sat;
+      const bool blend = __builtin_amdgcn_inverse_ballot_w64(blends);
+      const float w    = h.alpha * T;
+      if (weights) {
+        const int n = (int) __popcll(blends >> (lane & -kLanes) & ((1ull << kLanes) - 1ull));
+        const float sum = block_sum_to_last<kLanes>(blend ? w : 0.0f);
+        if ((lane & (kLanes - 1)) == kLanes - 1 && n > 0) atomicAdd(&s_accw[j], sum), atomicAdd(&s_accn[j], n);
       }
+      if (blend) {
+        if (kHits) my_hit[j * 32] = 1;
+        const int contributor = b * kB + j + 1;
+        if (kAux) {
+          const float A = 1.0f - T;
+          const float m = far_scale * (1.0f - near_n * __builtin_amdgcn_rcpf(h.depth));
+          const float mm = m * m;
+          dist = fmaf(fmaf(mm, A, fmaf(-2.0f * m, M1, M2)), w, dist);
+          D    = fmaf(h.depth, w, D);
+          M1   = fmaf(m, w, M1);
+          M2   = fmaf(mm, w, M2);
+          if (T > 0.5f) median = h.depth, median_c = contributor;
+          N0 = fmaf(cold.nx, w, N0), N1 = fmaf(cold.ny, w, N1), N2 = fmaf(cold.nz, w, N2);
+          if (kAccum) argmax_run_step(argmax, w, cold.id, accum_max_count);
+          if (kFlow) {
+            const float* Q = &s_t2[j * 9];
+            const float u2 = fmaf(Q[0], h.sx, fmaf(Q[1], h.sy, Q[2]));
+            const float v2 = fmaf(Q[3], h.sx, fmaf(Q[4], h.sy, Q[5]));
+            float w2       = fmaf(Q[6], h.sx, fmaf(Q[7], h.sy, Q[8]));
+            w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
+            f0 = fmaf(u2 / w2 - pxf, w, f0);
+            f1 = fmaf(v2 / w2 - pyf, w, f1);
+          }
+        }
+        C0 = fmaf(cold.r, w, C0), C1 = fmaf(cold.g, w, C1), C2 = fmaf(cold.b, w, C2);
+        T    = test_T;
+        last = contributor;
+      }
+    };
+    unsigned masks[kB / kWave];
+    auto walk = [&]() {
+      const int steps = build_block_lists<kLanes, kB>(lists, masks, wave, live_lanes);
+      walk_block_list(lists + lane / kLanes * kB, steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
+                      [&]() { return live_lanes != 0ull; });
+    };
+    if (kSnap) {
+      for (int half = 0; half < 2 && half * 32 < n_here; ++half) {
+        if (__builtin_amdgcn_inverse_ballot_w64(live_lanes)) {
+          // state before a list entry that starts a bucket of 32 (gs_2d_fast_redner.cu:126-147)
+          const size_t bk = (size_t) (bucket0 + (b * kB + half * 32) / 32);
+          sampled_T[bk * 256 + rank]             = T;
+          sampled_acc[(bk * 3 + 0) * 256 + rank] = C0;
+          sampled_acc[(bk * 3 + 1) * 256 + rank] = C1;
+          sampled_acc[(bk * 3 + 2) * 256 + rank] = C2;
+          if (kAux) {
+            sampled_aux[(bk * kNum + 0) * 256 + rank] = D;
+            sampled_aux[(bk * kNum + 1) * 256 + rank] = N0;
+            sampled_aux[(bk * kNum + 2) * 256 + rank] = N1;
+            sampled_aux[(bk * kNum + 3) * 256 + rank] = N2;
+            sampled_aux[(bk * kNum + 5) * 256 + rank] = dist;
+            sampled_aux[(bk * kNum + 6) * 256 + rank] = M1;
+            sampled_aux[(bk * kNum + 7) * 256 + rank] = M2;
+            if (kFlow) {
+              sampled_aux[(bk * kNum + 8) * 256 + rank] = f0;
+              sampled_aux[(bk * kNum + 9) * 256 + rank] = f1;
+            }
+          }
+        }
+        masks[0] = lane >> 5 == half ? s_mask[lane] : 0u;
+        walk();
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < kB / kWave; ++c) masks[c] = s_mask[c * kWave + lane];
+      walk();
     }
   }
 
+  if (kAccum || kHits) {
+    __syncthreads();
+    if (b > 0) flush(b - 1);  // entries behind it are behind every pixel's last one
+  }
   if (kAccum) argmax_run_flush(argmax, accum_max_count);
   if (inside) {
     out_opacity[pix]        = 1.0f - T;
@@ -441,11 +458,11 @@ __global__ void __launch_bounds__(256) fast_slot_sum_kernel(int P, int gx, int g
   out(i, 2 * k + 1, acc.y);
 }
 
+// Bound by vector issue and, like every launch here, by its longest tile; four blocks per compute unit. 150k surfels 1001x667:
+// 165 -> 132 us with a row of lanes per 4x4 block, over the blocks that the forward noted, instead of a wavefront per 8x8 quadrant
+// that queued its blended pairs.
 // kSlots: the per-surfel sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
 template <bool kAux, bool kPerSplat, bool kFlow, bool kSlots>
-// Four blocks per compute unit where the per-surfel sums go through records (the flush of the other form keeps more
-// values live and would spill in the loop over the entries): the launch lasts little longer than the block with the
-// longest list, and the more wavefronts share a SIMD with that block's, the sooner the other blocks are out of the way.
 __global__ void __launch_bounds__(kBlendThreads)
     __attribute__((amdgpu_waves_per_eu(kSlots && !kFlow ? 4 : 1, kSlots && !kFlow ? 4 : 8))) fast_blend_backward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
@@ -457,33 +474,28 @@ __global__ void __launch_bounds__(kBlendThreads)
     const float2* __restrict__ dL_dflow,
     float* __restrict__ g_means2D, float* __restrict__ g_normal_opacity, float* __restrict__ g_colors,
     float* __restrict__ g_trans, float* __restrict__ g_inv, const SlotSource slots,
-    const int32_t* __restrict__ radii, float* __restrict__ slot_records) {
-  constexpr int kB = 64;  // surfels staged per round
-  static_assert(kB == kWave, "one ballot covers a round, and a queued pair names its entry in a byte");
-  // Two passes (pair_queue.hpp): the order-bound recurrence queues the blending pairs, the components are formed and
-  // summed 64 pairs at a time. Not with a second set of transforms, whose per-pair terms would double the item.
-  constexpr bool kQueue = !kFlow;
-  __shared__ float4 s_queue[kQueue ? 4 : 1][kQueue ? kQueueItems : 1];
-  __shared__ FastHot s_hot[kB];
-  __shared__ SplatCold s_cold[kB];
+    const int32_t* __restrict__ radii, float* __restrict__ slot_records, const uint32_t* __restrict__ hit_blocks) {
+  constexpr int kB = kRowBatch, kRowPlaces = 224;  // 40 KB of LDS with records' stride
+  using Shape = BlockShape<16>;
+  __shared__ FastRecord s_splat[kB + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kB * 9 : 1];
-  // each wavefront's sums per staged surfel, written once per entry with a plain store and added in wavefront order at
-  // the flush (LDS float atomics cost about three cycles per lane)
-  __shared__ float s_part[4][kB][kFastGradSlots];
+  __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kB + 16];
+  __shared__ float s_sum[kRowPlaces + 1][kFastGradSlots];
+  // What the flush of a batch reads is kept twice, by batch parity: the next batch is staged while others still flush.
+  __shared__ uint4 s_place[2][kB];  // where each of the 16 rows stores its sums of each staged surfel
+  __shared__ int s_slot[2][kB];     // where they go from there: the instance's record (kSlots) or the surfel's number
+  __shared__ unsigned s_mask[kB];   // which 4x4 blocks of the tile it can reach
   __shared__ int s_max_contrib;
-  __shared__ unsigned char s_mask[kB];
 
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int tile = scheduled_tile(ordered, tile_order), tile_x = tile % gx, tile_y = tile / gx;
   int px, py;
-  lane_pixel(tile_x, tile_y, px, py);
+  Shape::lane_pixel(tile_x, tile_y, px, py);
   const bool inside = px < W && py < H;
   const size_t HW   = (size_t) H * W;
   const size_t pix  = (size_t) W * py + px;
   const float pxf = (float) px, pyf = (float) py;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const float qx0 = pxf - (float) (lane & 7), qy0 = pyf - (float) (lane >> 3);  // first pixel of the wavefront's quadrant
-  PairQueue q;
 
   const int64_t r0 = ranges[2 * (size_t) tile], r1 = ranges[2 * (size_t) tile + 1];
   const int last_contrib   = inside ? n_contrib[pix] : 0;
@@ -491,14 +503,18 @@ __global__ void __launch_bounds__(kBlendThreads)
 
   if (threadIdx.x == 0) s_max_contrib = 0;
   __syncthreads();
-  int wave_max_contrib = last_contrib;
+  int row_max = last_contrib;  // deepest position blended in this lane's 4x4 block
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) wave_max_contrib = max(wave_max_contrib, __shfl_xor(wave_max_contrib, d, kWave));
-  if (lane == 0) atomicMax(&s_max_contrib, wave_max_contrib);
-  for (int e = threadIdx.x; e < 4 * kB * kFastGradSlots; e += kBlendThreads) (&s_part[0][0][0])[e] = 0.0f;
+  for (int d = 8; d >= 1; d >>= 1) row_max = max(row_max, __shfl_xor(row_max, d, kWave));
+  int row_last[4];  // the same of the wavefront's four blocks
+#pragma unroll
+  for (int r = 0; r < 4; ++r) row_last[r] = __builtin_amdgcn_readlane(row_max, 16 * r);
+  if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
+  if (threadIdx.x == 0) s_splat[kB] = FastRecord{};  // all zero: p_z == 0 everywhere
+  if (threadIdx.x < kFastGradSlots) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
+  if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kB])[threadIdx.x] = 0u;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));
-  const int rounds = (n_todo + kB - 1) / kB;
   // No zero fill of the record buffer: every staged instance writes its record at the flush, zeros included, and the
   // instances behind the tile's deepest contributor, which are never staged, are cleared here.
   if (kSlots) {
@@ -555,11 +571,16 @@ __global__ void __launch_bounds__(kBlendThreads)
 
   FastSplat next;
   float next_t2[9];
+  unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
-  size_t slot = 0;  // record position of the entry this lane staged (the same lane flushes it)
-  auto gather = [&](int at) {
-    const int id = point_list[r0 + at];
+  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  auto gather = [&](int done) {
+    const int e = (int) threadIdx.x;
+    if (e >= min(kB, n_todo - done)) return;
+    const int64_t at = r0 + (n_todo - 1 - done - e);
+    if (hit_blocks) next_hits = hit_blocks[at];
+    const int id = point_list[at];
     next = gather_fast(id, means2D, colors, normal_opacity, trans_mat, inverse_m);
     if (kFlow) {
 #pragma unroll
@@ -567,34 +588,50 @@ __global__ void __launch_bounds__(kBlendThreads)
     }
     if (kSlots) next_radius = radii[id], next_off = slot_first(slots, id);
   };
-  if ((int) threadIdx.x < min(n_todo, kB)) gather(n_todo - 1 - (int) threadIdx.x);
+  gather(0);
 
-  for (int b = 0; b < rounds; ++b) {
-    const int n_here = min(kB, n_todo - b * kB);
-    if ((int) threadIdx.x < n_here) {
-      s_hot[threadIdx.x]  = next.hot;
-      s_cold[threadIdx.x] = next.cold;
-      s_mask[threadIdx.x] = (unsigned char) fast_quadrant_mask(next, tile_x * kTile, tile_y * kTile, ordered);
-      if (kFlow) {
+  for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    const int n_staged = min(kB, n_todo - done);
+    if ((int) threadIdx.x < kB) {
+      const int e = (int) threadIdx.x;
+      unsigned mask = 0u;
+      if (e < n_staged) {
+        s_splat[e] = next;
+        mask = hit_blocks ? pair_blocks(next_hits)
+                          : fast_blocks<16>(next, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
+        if (kFlow) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
+        }
+        if (kSlots) {
+          // The fused binning reserves one key position per tile of the surfel's rectangle, from its prefix-scan offset
+          // on (the tiles that pass its corner test are packed to the front of that span, the rest is padding). Any
+          // position of the span that no other tile of the surfel uses will do for the record: x-major over the rectangle.
+          const TileRect r = tile_rect(next.hot.cx, next.hot.cy, next_radius, gx, gy);
+          s_slot[parity][e] = (int) (next_off + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) + (tile_y - r.y0));
+        } else {
+          s_slot[parity][e] = next.cold.id;
+        }
+        s_place[parity][e] = no_places(kRowPlaces);
       }
-      if (kSlots) {
-        // The fused binning reserves one key position per tile of the surfel's rectangle, from its prefix-scan offset
-        // on (the tiles that pass its corner test are packed to the front of that span, the rest is padding). Any
-        // position of the span that no other tile of the surfel uses will do for the record: x-major over the rectangle.
-        const TileRect r = tile_rect(next.hot.cx, next.hot.cy, next_radius, gx, gy);
-        slot = (size_t) (next_off + (int64_t) (tile_x - r.x0) * (r.y1 - r.y0) + (tile_y - r.y0));
-      }
+      s_mask[e] = mask;
     }
     __syncthreads();
-    const int nxt = (b + 1) * kB + (int) threadIdx.x;
-    if ((int) threadIdx.x < kB && nxt < n_todo) gather(n_todo - 1 - nxt);
+    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    int start, before[4];
+    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
+    gather(done + n_here);
+    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+    const int behind = n_todo - done;
+    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+    const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
+                                      n_here);
+    const int my_first = behind - last_contrib, my_median = behind - median_contrib;
 
     // The part of a pair that is bound to the list's order: advances the pixel's back-to-front state and leaves the
     // pair's weight, dL/dalpha (times the transmittance in front of the pair), dL/d(depth along the ray) and, with a
     // second set of transforms, dL/d(intersection) through it. Only entered by lanes whose pixel blends the entry.
-    auto advance_pixel = [&](const SplatCold& cold, int j, int pos, const FastHit& h, float& w, float& dL_dalpha,
+    auto advance_pixel = [&](const SplatCold& cold, int j, const FastHit& h, float& w, float& dL_dalpha,
                              float& dL_dz, float& fsx, float& fsy) {
       T = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
       w = h.alpha * T;
@@ -605,7 +642,7 @@ __global__ void __launch_bounds__(kBlendThreads)
         const float rd     = __builtin_amdgcn_rcpf(h.depth);
         const float m_d    = far_scale - far_near * rd;
         const float dmd_dd = far_near * rd * rd;
-        if (pos == median_contrib - 1) dL_dz += dL_dmedian;
+        if (j == my_median) dL_dz += dL_dmedian;
         if (!kPerSplat) {
           // dL/dweight of the distortion enters dL/dalpha as a linear channel does (its value minus what the pairs
           // behind it accumulated, with the same weights): it rides on the shared recurrence
@@ -637,107 +674,39 @@ __global__ void __launch_bounds__(kBlendThreads)
       dL_dalpha *= T;
     };
 
-    // ---- order-free part: 64 queued pairs at a time, four 16-lane rows, every row one entry ---------------------------
-    // A lane rebuilds the intersection through its pair's pixel from the staged adjugate and forms the 16 + 5 components
-    // as products of the three queued numbers with quantities that are finite in every lane (padding items carry zeros
-    // and no flags, and the reciprocal of p_z is only taken under the pair's flags).
-    auto drain = [&](int n_valid) {
-      const unsigned jrows = queue_front_rows(q);
-      const int j = (int) ((jrows >> ((lane >> 4) * 8)) & 255u);
-      const float4 it = s_queue[wave][q.head + lane];
-      const FastHot hot = s_hot[j];
-      float* const acc  = &s_part[wave][j][lane & 15];
-      const bool second = (lane & 15) < 5;  // lanes 0-4 of a row add the five other components
-      float* const acc2 = &s_part[wave][j][16 + (second ? (lane & 15) : 0)];
-      const float before = *acc;
-      const float before2 = (kAux && second) ? *acc2 : 0.0f;
-      const int bits = __float_as_int(it.w);
-      const int qp = bits & 63;
-      const bool blends = (bits & kItemHit) != 0, by_ray = (bits & kItemRay) != 0;
-      // the upstream gradients of the pair's pixel sit in the registers of the lane that owns it
-      auto from_owner = [&](float v) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(qp << 2, __builtin_bit_cast(int, v)));
-      };
-      const float up_x = from_owner(dLp0), up_y = from_owner(dLp1), up_z = from_owner(dLp2);
-      const float fx = qx0 + (float) (qp & 7), fy = qy0 + (float) (qp >> 3);
-      const float w = it.x, GdA = it.y, dL_dz = it.z;
-      // the same fused forms as the per-pixel test: for a surfel seen edge-on p_z is a small difference of large terms
-      const float p0 = fmaf(hot.a[0], fx, fmaf(hot.a[1], fy, hot.a[2]));
-      const float p1 = fmaf(hot.a[3], fx, fmaf(hot.a[4], fy, hot.a[5]));
-      const float pz = fmaf(hot.a[6], fx, fmaf(hot.a[7], fy, hot.a[8]));
-      const float rz_s = blends ? __builtin_amdgcn_rcpf(pz) : 0.0f;  // s is used by both cases of a blending pair
-      const float rz_p = by_ray ? rz_s : 0.0f;                        // d/dp only by the intersection case
-      const float sx = p0 * rz_s, sy = p1 * rz_s;
-      const float oG = hot.opacity * GdA;
-      float dsx = -(oG * sx), dsy = -(oG * sy);
-      if (kAux) dsx += dL_dz * hot.tw0, dsy += dL_dz * hot.tw1;
-      const float s_ds = dsx * sx + dsy * sy;
-      const float da = dsx * rz_p, db = dsy * rz_p, dc = -(s_ds * rz_p);
-      float g[16];
-      g[0] = w * up_x, g[1] = w * up_y, g[2] = w * up_z;
-      g[3] = da * fx, g[4] = da * fy, g[5] = da;
-      g[6] = db * fx, g[7] = db * fy, g[8] = db;
-      g[9] = dc * fx, g[10] = dc * fy, g[11] = dc;
-      if (kAux) {
-        g[12] = w * from_owner(dLn0), g[13] = w * from_owner(dLn1), g[14] = w * from_owner(dLn2);
-      } else {
-        g[12] = g[13] = g[14] = 0.0f;
-      }
-      g[15] = GdA;
-      queue_accumulate(acc, before, row_sum16_transposed(g), jrows, n_valid, true);
-      const bool filtered = blends && !by_ray;
-      const float to_centre = filtered ? -2.0f * oG : 0.0f;
-      if (kAux) {
-        float g8[8];
-        g8[0] = dL_dz * sx, g8[1] = dL_dz * sy, g8[2] = dL_dz;
-        g8[3] = to_centre * (hot.cx - fx), g8[4] = to_centre * (hot.cy - fy);
-        g8[5] = g8[6] = g8[7] = 0.0f;
-        queue_accumulate(acc2, before2, row_sum8_transposed(g8), jrows, n_valid, second);
-      } else if (wave_ballot(filtered) != 0ull) {  // some pair met its surfel by the projected centre
-        float cx = to_centre * (hot.cx - fx), cy = to_centre * (hot.cy - fy);  // totals of a row end up in its lane 15
-        cx += dpp_shift_zero<0x111, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x111, 0xf, 0xf>(cy);
-        cx += dpp_shift_zero<0x112, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x112, 0xf, 0xf>(cy);
-        cx += dpp_shift_zero<0x114, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x114, 0xf, 0xf>(cy);
-        cx += dpp_shift_zero<0x118, 0xf, 0xf>(cx), cy += dpp_shift_zero<0x118, 0xf, 0xf>(cy);
-        if ((lane >> 4) < ((n_valid + 15) >> 4) && (lane & 15) == 15)
-          atomicAdd(&s_part[wave][j][19], cx), atomicAdd(&s_part[wave][j][20], cy);
-      }
-      queue_pop(q, n_valid);
-    };
-
-    // one entry of the wavefront's work list; its records were requested from LDS while the entry before it ran
-    auto blend_entry = [&](const FastHot& hot, const SplatCold& cold, int j) {
-        const int pos = n_todo - 1 - (b * kB + j);
+    const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+    float* const sums  = &s_sum[place][lane & 15];  // component lane & 15 of the row's first place
+    float* const sums2 = &s_sum[place][16 + ((lane & 2) ? 4 : (lane >> 2 & 1) * 2 + (lane >> 3 & 1))];
+    auto blend_entry = [&](const FastHot& hot, int j, int i) {
+        const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+        __builtin_amdgcn_sched_barrier(0);
         FastHit h;
         unsigned long long pass;
-        const bool hit = fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass) && (pos < last_contrib);
-        pass &= wave_ballot(pos < last_contrib);
-        if (pass == 0ull) return;
-        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, fsx = 0.0f, fsy = 0.0f;
-        if (kQueue) {
-          if (hit) {
-            advance_pixel(cold, j, pos, h, w, dL_dalpha, dL_dz, fsx, fsy);
-            dL_dalpha *= h.G;  // only G * dL/dalpha is ever used
+        fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass);
+        pass &= wave_ballot(j >= my_first);
+        if (pass == 0ull) {
+          if (j != kB) {  // not a padding step; zeros, too, have their place
+            sums[i * kFastGradSlots] = 0.0f;
+            if ((lane & 1) == 0) sums2[i * kFastGradSlots] = 0.0f;
           }
-          const int flags = h.rho3d <= h.rho2d ? (kItemHit | kItemRay) : kItemHit;
-          if (queue_append(s_queue[wave], q, j, hit, pass, w, dL_dalpha, dL_dz, flags)) drain(kWave);
           return;
         }
-
-        // One pass per entry (second set of transforms: its per-pair terms would double the queue's item). The part
-        // under `hit` leaves a few factors (zero in a lane whose pixel does not blend the entry); the components are
+        const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
+        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, fsx = 0.0f, fsy = 0.0f;
+        // The part under `hit` leaves a few factors (zero in a lane whose pixel does not blend the entry); the components are
         // products of those factors with quantities that are finite in every lane, formed by all lanes alike: no
         // component needs a zero of its own, and the projected-centre case is the intersection case with a zero in
         // place of 1 / p_z.
-        float g[16], g8[8];
-        float dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
+        float g[16], g5[5];
+        float GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
         if (hit) {
-          advance_pixel(cold, j, pos, h, w, dL_dalpha, dL_dz, fsx, fsy);
+          advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, fsx, fsy);
           // d/ds of the intersection case (times 1 / p_z below); s is not finite in a lane whose p_z is 0, and such a
           // lane never blends: every use of s sits on this side
-          const float dL_dG = hot.opacity * dL_dalpha;
-          dsx  = fsx + dL_dG * -h.G * h.sx + dL_dz * hot.tw0;
-          dsy  = fsy + dL_dG * -h.G * h.sy + dL_dz * hot.tw1;
+          GdA  = dL_dalpha * h.G;
+          oG   = hot.opacity * GdA;
+          dsx  = fsx - oG * h.sx, dsy = fsy - oG * h.sy;
+          if (kAux) dsx += dL_dz * hot.tw0, dsy += dL_dz * hot.tw1;
           s_ds = dsx * h.sx + dsy * h.sy;
           z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
         }
@@ -751,87 +720,50 @@ __global__ void __launch_bounds__(kBlendThreads)
         g[9] = dc * pxf, g[10] = dc * pyf, g[11] = dc;
         if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
         else      g[12] = g[13] = g[14] = 0.0f;
-        g[15] = h.G * dL_dalpha;
-        const float to_centre = filtered ? hot.opacity * dL_dalpha * (-2.0f * h.G) : 0.0f;
-        g8[0] = z_sx, g8[1] = z_sy, g8[2] = dL_dz;
-        g8[3] = to_centre * h.dx, g8[4] = to_centre * h.dy;
-        g8[5] = g8[6] = g8[7] = 0.0f;
-        const float tot = wave_sum16_transposed(g);
-        if (lane < 16) s_part[wave][j][lane] = tot;
-        if (kAux) {
-          const float tot8 = wave_sum8_transposed(g8);
-          if (lane < 5) s_part[wave][j][16 + lane] = tot8;
-        } else if (wave_ballot(filtered) != 0ull) {
-          const float sx = wave_sum_to_lane63(g8[3]), sy = wave_sum_to_lane63(g8[4]);
-          if (lane == 63) s_part[wave][j][19] = sx, s_part[wave][j][20] = sy;
+        g[15] = GdA;
+        const float to_centre = filtered ? -2.0f * oG : 0.0f;
+        g5[0] = z_sx, g5[1] = z_sy, g5[2] = dL_dz;
+        g5[3] = to_centre * h.dx, g5[4] = to_centre * h.dy;
+        const float tot = row_sum16_transposed(g), tot5 = row_sum5_transposed(g5);
+        if (j != kB) {
+          sums[i * kFastGradSlots] = tot;
+          if ((lane & 1) == 0) sums2[i * kFastGradSlots] = tot5;
         }
     };
-    unsigned long long todo = __ballot(lane < n_here && ((s_mask[lane] >> wave) & 1u) &&
-                                       (n_todo - 1 - (b * kB + lane)) < wave_max_contrib);
-    if (todo != 0ull) {
-      auto pop = [&]() {
-        const int j = __builtin_ctzll(todo);
-        todo &= todo - 1;
-        return j;
-      };
-      auto peek = [&]() { return todo ? (int) __builtin_ctzll(todo) : 0; };
-      FastHot hot_a = s_hot[peek()], hot_b;
-      while (todo) {
-        {
-          const int j = pop();
-          hot_b       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_a, cold, j);
-        }
-        if (todo == 0ull) break;
-        {
-          const int j = pop();
-          hot_a       = s_hot[peek()];
-          const SplatCold cold = s_cold[j];
-          __builtin_amdgcn_sched_barrier(0);
-          blend_entry(hot_b, cold, j);
-        }
-      }
-      if (kQueue && q.count > 0) drain(q.count);  // the staged records are replaced after the next barrier
-    }
+    walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
+                    [] { return true; });
     __syncthreads();
-    if ((int) threadIdx.x < n_here) {
-      const int id = s_cold[threadIdx.x].id;
-      float a[kFastGradSlots];
+    // Flush the batch: add the sums of the rows that hold an entry, in row order.
+    if (kSlots) {
+      // two lanes per entry, eleven of the record's floats each (component 10 is summed by both)
+      static_assert(kBlendThreads == 2 * kB && kFastGradSlots == 21 && kFastRecordSlots == 22);
+      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
+        const int h = (int) threadIdx.x & 1;
+        float a[11];
+        sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], 10 * h, a);
+        float* dst = slot_records + (size_t) s_slot[parity][e] * kFastRecordSlots + 11 * h;
 #pragma unroll
-      for (int c = 0; c < kFastGradSlots; ++c) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) sum += s_part[w][threadIdx.x][c], s_part[w][threadIdx.x][c] = 0.0f;
-        a[c] = sum;
+        for (int c = 0; c < 11; ++c) dst[c] = h == 0 ? a[c] : c < 10 ? a[c < 10 ? c + 1 : 0] : 0.0f;
       }
-      if (kSlots) {
-        float2* dst = (float2*) (slot_records + slot * kFastRecordSlots);
-#pragma unroll
-        for (int c = 0; c < kFastRecordSlots / 2; ++c)
-          dst[c] = make_float2(a[2 * c], 2 * c + 1 < kFastGradSlots ? a[2 * c + 1] : 0.0f);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-          if (a[c] != 0.0f) atomicAdd(&g_colors[3 * (size_t) id + c], a[c]);
-#pragma unroll
-        for (int c = 0; c < 9; ++c)
-          if (a[3 + c] != 0.0f) atomicAdd(&g_inv[9 * (size_t) id + c], a[3 + c]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (a[12 + c] != 0.0f) atomicAdd(&g_normal_opacity[4 * (size_t) id + c], a[12 + c]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-          if (a[16 + c] != 0.0f) atomicAdd(&g_trans[9 * (size_t) id + 6 + c], a[16 + c]);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          if (a[19 + c] != 0.0f) atomicAdd(&g_means2D[2 * (size_t) id + c], a[19 + c]);
+    } else {
+      // one global atomic per surfel and component for this tile, a lane per component
+      for (int t = (int) threadIdx.x; t < n_here * kFastGradSlots; t += kBlendThreads) {
+        const int e = t / kFastGradSlots, c = t - e * kFastGradSlots, id = s_slot[parity][e];
+        float a[1];
+        sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
+        float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
+                           : c < 12 ? g_inv + 9 * (size_t) id + (c - 3)
+                           : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
+                           : c < 19 ? g_trans + 9 * (size_t) id + 6 + (c - 16)
+                                    : g_means2D + 2 * (size_t) id + (c - 19);
+        if (a[0] != 0.0f) atomicAdd(out, a[0]);
       }
     }
+    done += n_here;
+    // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
+    // records, which nobody reads before, and the other copy of what the flush reads.
   }
 }
-
 
 // The reference's second backward (gs_2d_fast_redner.cu:563-837), the per-splat decomposition itself: a lane owns ONE
 // list entry of a tile and keeps that surfel's 21 gradient sums in registers, the tile's pixels pass through the lanes
@@ -1023,13 +955,15 @@ void launch_fast_slot_sum(int P, int gx, int gy, const SlotSource& slots, const 
 
 using namespace fsgs;
 
-FSGS_API int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
+namespace {
+// hit_blocks[R], if given (without snapshots): per list entry the 2x4 blocks of its tile with a pixel that blended it
+int fast_render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
     const float* means2D, const float* colors, const float* normal_opacity, const float* trans_mat,
     const float* inverse_m, const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2,
     int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count, const int64_t* bucket_offset,
     float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib,
     int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_acc, float* sampled_aux,
-    void* stream) {
+    uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_fast_render_forward: bad sizes");
   FSGS_REQUIRE(ranges && out_color && out_opacity && n_contrib, "GS_2D_fast_render_forward: null pointer");
   FSGS_REQUIRE(P == 0 || (means2D && colors && normal_opacity && trans_mat && inverse_m),
@@ -1047,22 +981,49 @@ FSGS_API int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, 
   hipStream_t s = (hipStream_t) stream;
   const int* tile_order = nullptr;
   const int ordered = launch_tile_order(gx, gy, ranges, s, &tile_order);
-#define FSGS_LAUNCH_FWD(AUX, SNAP, ACC, FLOW)                                                                        \
-  hipLaunchKernelGGL((fast_blend_forward_kernel<AUX, SNAP, ACC, FLOW>), grid, block, 0, s, ordered, tile_order, W, H,            \
+#define FSGS_LAUNCH_FWD(AUX, SNAP, ACC, FLOW, HITS)                                                                  \
+  hipLaunchKernelGGL((fast_blend_forward_kernel<AUX, SNAP, ACC, FLOW, HITS>), grid, block, 0, s, ordered, tile_order, W, H,      \
                      (float) near_n, (float) far_n, ranges, point_list, (const float2*) means2D, colors, trans_mat,  \
                      inverse_m, (const float4*) normal_opacity, trans_mat_t2, bucket_offset, n_contrib, out_color,   \
                      out_opacity, out_extras, (float2*) out_flow, max_contrib, bucket_to_tile, sampled_T,            \
-                     sampled_acc, sampled_aux, accum_max_count, accum_weights_p, accum_weights_count)
-#define FSGS_LAUNCH_FWD_F(AUX, SNAP, ACC) \
-  do { if (flow) FSGS_LAUNCH_FWD(AUX, SNAP, ACC, true); else FSGS_LAUNCH_FWD(AUX, SNAP, ACC, false); } while (0)
-  if (!aux) FSGS_LAUNCH_FWD(false, false, false, false);
-  else if (snap && accum) FSGS_LAUNCH_FWD_F(true, true, true);
-  else if (snap) FSGS_LAUNCH_FWD_F(true, true, false);
-  else if (accum) FSGS_LAUNCH_FWD_F(true, false, true);
-  else FSGS_LAUNCH_FWD_F(true, false, false);
+                     sampled_acc, sampled_aux, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks)
+#define FSGS_LAUNCH_FWD_F(AUX, SNAP, ACC, HITS) \
+  do { if (flow) FSGS_LAUNCH_FWD(AUX, SNAP, ACC, true, HITS); else FSGS_LAUNCH_FWD(AUX, SNAP, ACC, false, HITS); } while (0)
+  if (!aux) FSGS_LAUNCH_FWD(false, false, false, false, false);
+  else if (snap && accum) FSGS_LAUNCH_FWD_F(true, true, true, false);
+  else if (snap) FSGS_LAUNCH_FWD_F(true, true, false, false);
+  else if (accum && hit_blocks) FSGS_LAUNCH_FWD_F(true, false, true, true);
+  else if (accum) FSGS_LAUNCH_FWD_F(true, false, true, false);
+  else if (hit_blocks) FSGS_LAUNCH_FWD_F(true, false, false, true);
+  else FSGS_LAUNCH_FWD_F(true, false, false, false);
 #undef FSGS_LAUNCH_FWD_F
 #undef FSGS_LAUNCH_FWD
   return check_launch("GS_2D_fast_render_forward");
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, double far_n, int only_image,
+    const float* means2D, const float* colors, const float* normal_opacity, const float* trans_mat,
+    const float* inverse_m, const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2,
+    int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count, const int64_t* bucket_offset,
+    float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib,
+    int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_acc, float* sampled_aux,
+    void* stream) {
+  return fast_render_forward(P, W, H, near_n, far_n, only_image, means2D, colors, normal_opacity, trans_mat, inverse_m,
+                             point_list, ranges, trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count,
+                             bucket_offset, out_color, out_opacity, out_extras, out_flow, n_contrib, max_contrib,
+                             bucket_to_tile, sampled_T, sampled_acc, sampled_aux, nullptr, stream);
+}
+
+FSGS_API int fsgs_gs_2d_fast_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* colors, const float* normal_opacity, const float* trans_mat, const float* inverse_m,
+    const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
+    float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
+    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, void* stream) {
+  return fast_render_forward(P, W, H, near_n, far_n, 0, means2D, colors, normal_opacity, trans_mat, inverse_m, point_list,
+                             ranges, trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count, nullptr, out_color,
+                             out_opacity, out_extras, out_flow, n_contrib, nullptr, nullptr, nullptr, nullptr, nullptr,
+                             hit_blocks, stream);
 }
 
 FSGS_API size_t fsgs_gs_2d_fast_render_backward_workspace_bytes(int64_t R) {
@@ -1077,7 +1038,7 @@ int fast_render_backward(int P, int W, int H, double near_n, double far_n, int p
     const float* dL_dflow, const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib,
     float* g_colors, float* g_means2D, float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R,
     const SlotSource& source, const int32_t* radii, void* workspace, size_t workspace_bytes,
-    const uint32_t* keep_masks, void* stream) {
+    const uint32_t* keep_masks, const uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_fast_render_backward: bad sizes");
   if (P == 0) return kOk;
   FSGS_REQUIRE(means2D && normal_opacity && colors && trans_mat && inverse_m && out_opacity && dL_dpix && dL_dopacity &&
@@ -1109,7 +1070,7 @@ int fast_render_backward(int P, int W, int H, double near_n, double far_n, int p
                      (const float4*) normal_opacity, colors, trans_mat, inverse_m, trans_mat_t2, out_opacity,        \
                      out_extras, (const float2*) out_flow, dL_dpix, dL_dextras, dL_dopacity,                         \
                      (const float2*) dL_dflow, g_means2D, g_normal_opacity, g_colors, g_trans, g_inv, source,        \
-                     radii, ws.records)
+                     radii, ws.records, hit_blocks)
 #define FSGS_LAUNCH_BWD(AUX, SPLAT, FLOW) \
   do { if (slots) FSGS_LAUNCH_BWD_S(AUX, SPLAT, FLOW, true); else FSGS_LAUNCH_BWD_S(AUX, SPLAT, FLOW, false); } while (0)
   if (aux && per_splat_form && flow) FSGS_LAUNCH_BWD(true, true, true);
@@ -1138,7 +1099,7 @@ FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n,
   return fast_render_backward(P, W, H, near_n, far_n, per_splat_form, means2D, normal_opacity, colors, trans_mat, inverse_m,
                               trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
                               ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
-                              SlotSource{point_offsets}, radii, workspace, workspace_bytes, keep_masks, stream);
+                              SlotSource{point_offsets}, radii, workspace, workspace_bytes, keep_masks, nullptr, stream);
 }
 
 // The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp).
@@ -1156,7 +1117,25 @@ FSGS_API int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, d
                               trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
                               ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
                               SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
-                              workspace_bytes, keep_masks, stream);
+                              workspace_bytes, keep_masks, nullptr, stream);
+}
+
+// The same over the blocks that blended an entry, as the forward noted them (nullptr: bounded here).
+FSGS_API int fsgs_gs_2d_fast_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
+    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
+    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
+    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
+    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const uint32_t* keep_masks, const uint32_t* hit_blocks, void* stream) {
+  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched),
+               "gs_2d_fast_view_backward: record slots are required");
+  return fast_render_backward(P, W, H, near_n, far_n, 0, means2D, normal_opacity, colors, trans_mat, inverse_m,
+                              trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
+                              ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
+                              SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
+                              workspace_bytes, keep_masks, hit_blocks, stream);
 }
 
 // The per-splat decomposition itself (fast_bucket_backward_kernel), for callers that want the reference's second

@@ -438,7 +438,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     float* __restrict__ g_means2D, float* __restrict__ g_conic_opacity, float* __restrict__ g_colors,
     float* __restrict__ g_extras, const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii,
     float* __restrict__ slot_records, const uint32_t* __restrict__ hit_blocks) {
-  constexpr int kB = kRowBatch;
+  constexpr int kB = kRowBatch, kRowPlaces = 255;
   using Shape = BlockShape<16>;
   // components that cross the lanes: 0-2 colour | 3-6 extras | 7-8 mean2D | 9-11 conic | 12 opacity, without extras close up
   constexpr bool kNine = E == 0;
@@ -474,7 +474,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
   if (lane == 0) atomicMax(&s_max_contrib, max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3])));
   if (threadIdx.x == 0) s_splat[kB] = G3Splat<E>{};  // all zero: alpha is 0
   if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kB])[threadIdx.x] = 0u;
-  if (threadIdx.x < kSums) s_sum[kNoPlace][threadIdx.x] = 0.0f;
+  if (threadIdx.x < kSums) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
   __syncthreads();
   const int n_todo = min(s_max_contrib, (int) (r1 - r0));
   // No zero fill of the record buffer: every staged instance writes its record at the flush, zeros included, and the
@@ -527,7 +527,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
                                              tile_y * kTile, flags);
         s_splat[e]       = next;
         s_tag[parity][e] = make_float2(__int_as_float(next.id), next.opacity);
-        s_place[parity][e] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        s_place[parity][e] = no_places(kRowPlaces);
         if (kSlots) {
           // the binning emits a Gaussian's tiles row-major over its rectangle, from its prefix-scan offset on
           const TileRect r = tile_rect(next.x, next.y, next_radius, gx, gy);
@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     __syncthreads();
     const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
     int start, before[4];
-    const int n_here = row_batch(masks, n_staged, wave, start);
+    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
     gather(done + n_here);
     // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
     const int behind = n_todo - done;

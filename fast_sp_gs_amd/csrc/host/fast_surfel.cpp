@@ -20,6 +20,7 @@ struct Buffers {
   Tensor radii, visible, ranges, point_list, n_contrib;
   Tensor image, opacity, extras, flow;        // what the blend writes
   Tensor normals, surf_depth, surf_normal;    // what the epilogue writes
+  Tensor hit_blocks;                          // per list entry, for the backward
   Slab keep;                                  // per-surfel intermediates, read again by the backward
   c10::intrusive_ptr<Saved> saved;
 };
@@ -116,12 +117,12 @@ Buffers forward_view(const FastSurfelView& v, bool train) {
     b.point_list = empty({0}, like, at::kInt);
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream), what);
   }
-  check(fsgs_gs_2d_fast_render_forward((int) P, W, H, v.near_n, v.far_n, 0, f32(v.means2D), colors, normal_opacity, trans_mat,
-                                       inverse_m, i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
-                                       i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
-                                       i32(opt(v.accum_weights_count)), nullptr, f32(b.image), f32(b.opacity),
-                                       f32(b.extras), f32(b.flow), i32(b.n_contrib), nullptr, nullptr, nullptr, nullptr,
-                                       nullptr, stream),
+  if (train) b.hit_blocks = empty({s.R}, like, at::kInt);
+  check(fsgs_gs_2d_fast_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, normal_opacity, trans_mat,
+                                     inverse_m, i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
+                                     i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
+                                     i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
+                                     f32(b.flow), i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), stream),
         blend);
   if (v.epilogue) {
     b.normals = empty({3, H, W}, like), b.surf_depth = empty({1, H, W}, like), b.surf_normal = empty({3, H, W}, like);
@@ -161,7 +162,7 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
     const Buffers& b = *out;
     ctx->save_for_backward({v.points, v.scales, v.rotations, v.opacities, v.shs, opt(v.sh_rest), v.means2D, v.Tw2v, v.Tv2c,
                             v.Tv2s, v.campos, opt(v.trans_mat_t2), b.radii, b.ranges, b.point_list, b.n_contrib,
-                            b.opacity, b.extras, b.flow, b.keep.memory()});
+                            b.opacity, b.extras, b.flow, b.keep.memory(), b.hit_blocks});
     ctx->saved_data["view"] = c10::IValue::make_capsule(b.saved);
     ctx->set_materialize_grads(false);
     return outputs_of(b);
@@ -218,7 +219,7 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
       float* g_colors = sh || !want_sh ? scratch.at<float>(g_col) : f32(g_sh);
       const float* colors = sh ? keep(s.colors) : f32(shs);
       const int M = rest_used ? (int) sh_rest.size(1) : shs.dim() == 3 ? (int) shs.size(1) : 0;
-      check(fsgs_gs_2d_fast_view_backward((int) P, W, H, s.near_n, s.far_n, f32(means2D), keep(s.normal_opacity), colors,
+      check(fsgs_gs_2d_fast_view_backward_hits((int) P, W, H, s.near_n, s.far_n, f32(means2D), keep(s.normal_opacity), colors,
                                           keep(s.trans_mat), keep(s.inverse_m), f32(t2), f32(opacity),
                                           aux ? f32(extras) : nullptr, g_flow.defined() ? f32(flow) : nullptr, f32(g_image),
                                           f32(g_opacity), f32(g_extras), f32(g_flow), i64(ranges), i32(point_list),
@@ -226,7 +227,7 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
                                           scratch.at<float>(g_inv), scratch.at<float>(g_no), s.R,
                                           (const int32_t*) keep(s.offsets), (const int32_t*) keep(s.regions),
                                           (const int32_t*) keep(s.tiles), i32(radii), scratch.at<void>(ws), ws_bytes,
-                                          (const uint32_t*) keep(s.masks), stream),
+                                          (const uint32_t*) keep(s.masks), (const uint32_t*) i32(t[20]), stream),
             "GS_2D_fast_render_backward");
       check(fsgs_gs_2d_fast_preprocess_backward((int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations),
                                                 f32(shs), rest_used ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2s),

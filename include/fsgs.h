@@ -315,6 +315,13 @@ int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, double fa
     float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib,
     int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_acc, float* sampled_aux,
     void* stream);
+/* The same with all maps and without snapshots, for a view that will be back-propagated: hit_blocks[R] (nullptr: not wanted) as
+ * fsgs_gs_2d_view_forward leaves it. */
+int fsgs_gs_2d_fast_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* colors, const float* normal_opacity, const float* trans_mat, const float* inverse_m,
+    const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
+    float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
+    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, void* stream);
 
 /* GS_2D_fast_render_backward -- gs_2d_fast_redner.cu:955-1074. per_splat_form = 0: kernel :273-561 (image, opacity,
  * aux 0-5); per_splat_form = 1: the channel set of kernel :563-837 (image, opacity, aux 0-4 and 6-7, no distortion).
@@ -348,6 +355,15 @@ int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far
     float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
     const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const uint32_t* keep_masks, void* stream);
+/* The same with the hit_blocks that fsgs_gs_2d_fast_view_forward left for these lists (nullptr: footprints are bounded again). */
+int fsgs_gs_2d_fast_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
+    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
+    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
+    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
+    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const uint32_t* keep_masks, const uint32_t* hit_blocks, void* stream);
 
 /* The per-splat decomposition of gs_2d_fast_redner.cu:563-837 itself (fsgs_gs_2d_fast_render_backward with
  * per_splat_form = 1 returns the same derivative through the back-to-front kernel, which is faster here): a lane owns

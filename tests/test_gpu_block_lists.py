@@ -112,3 +112,23 @@ def test_gaussian_view(shape, P, device):
         assert torch.equal(a, b)
     for a, b in zip(grads, grads_all):
         assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("P", [1, 127, 128, 129, 191, 192, 193, 900])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_fast_surfel_view(shape, P, device):
+    from fast_sp_gs_amd.renderer.gs_2d_fast_render import GS_2D_fast_render
+    scene, cam = _scene(shape, P, device)
+
+    def run():
+        params = _params(scene)
+        out = GS_2D_fast_render(size=(cam.W, cam.H), Tw2v=cam.Tw2v, Tv2c=cam.Tv2c, Tv2s=cam.Tv2s, campos=cam.campos,
+                                near=cam.near, far=cam.far, sh_degree=3, **params)
+        maps = [out[k] for k in ('images', 'normals', 'surf_depth', 'distortion')]
+        return maps, _gradients(params, maps)
+
+    (maps, grads), (maps_all, grads_all) = _both(run)
+    for a, b in zip(maps, maps_all):
+        assert torch.equal(a, b)
+    for a, b in zip(grads, grads_all):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
