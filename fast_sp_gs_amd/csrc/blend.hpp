@@ -11,7 +11,6 @@ constexpr int kFlagOrdered = 1, kFlagNoCull = 2;
 bool culling_enabled();  // host-side switch, on by default
 
 constexpr int kBlendThreads = 256;  // one 16x16 tile per block = 4 wavefronts, each owning an 8x8 pixel quadrant
-constexpr int kBatch        = 256;  // surfels staged in LDS per round
 
 // Hot part of a staged surfel (what every pixel needs to decide whether the surfel touches it), 48 bytes.
 struct __attribute__((aligned(16))) SplatHot {
@@ -78,15 +77,6 @@ __device__ __forceinline__ void lane_pixel(int tile_x, int tile_y, int& px, int&
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   px = tile_x * kTile + (wave & 1) * 8 + (lane & 7);
   py = tile_y * kTile + (wave >> 1) * 8 + (lane >> 3);
-}
-
-// The same quadrant with every 16-lane DPP row on a 4x4 pixel block: row r = lane >> 4 is block (r & 1, r >> 1) of the
-// quadrant, lane & 15 runs row-major inside the block.
-__device__ __forceinline__ void lane_pixel_blocks(int tile_x, int tile_y, int& px, int& py) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = lane >> 4, in = lane & 15;
-  px = tile_x * kTile + (wave & 1) * 8 + (row & 1) * 4 + (in & 3);
-  py = tile_y * kTile + (wave >> 1) * 8 + (row >> 1) * 4 + (in >> 2);
 }
 
 struct Hit {
@@ -369,7 +359,7 @@ __global__ void __launch_bounds__(1024) tile_order_kernel(int gx, int gy, const 
 }
 
 // Launch flags of the blend kernels: bit 0 = the tile table was built for this launch (T small enough; otherwise blocks
-// map to tiles directly), bit 1 = per-quadrant culling switched off (verification aid, see fsgs_debug_set_culling).
+// map to tiles directly), bit 1 = culling switched off (verification aid, see fsgs_debug_set_culling).
 inline int launch_tile_order(int gx, int gy, const int64_t* ranges, hipStream_t s, const int** table) {
   int flags = culling_enabled() ? 0 : kFlagNoCull;
   *table    = nullptr;
@@ -409,22 +399,10 @@ __device__ __forceinline__ float dpp_shift_zero(float v) {
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, kRowMask, kBankMask, true));
 }
 
-// Sum over the 64 lanes; the total is valid in lane 63 only.
-__device__ __forceinline__ float wave_sum_to_lane63(float v) {
-#pragma clang fp contract(off)  // as in row_sum16_transposed: an input product must not be formed a second time
-  v += dpp_shift_zero<0x111, 0xf, 0xf>(v);  // row_shr:1
-  v += dpp_shift_zero<0x112, 0xf, 0xf>(v);  // row_shr:2
-  v += dpp_shift_zero<0x114, 0xf, 0xf>(v);  // row_shr:4
-  v += dpp_shift_zero<0x118, 0xf, 0xf>(v);  // row_shr:8  -> lane 15 of every row holds the row total
-  v += dpp_shift_zero<0x142, 0xa, 0xf>(v);  // row_bcast:15 into rows 1 and 3
-  v += dpp_shift_zero<0x143, 0xc, 0xf>(v);  // row_bcast:31 into rows 2 and 3 -> lane 63 holds the wave total
-  return v;
-}
-
 // Sum over each aligned group of 8 or 16 lanes; the total is valid in the group's last lane only.
 template <int kLanes>
 __device__ __forceinline__ float block_sum_to_last(float v) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(off)  // as in row_sum16_transposed: an input product must not be formed a second time
   v += dpp_shift_zero<0x111, 0xf, 0xf>(v);
   v += dpp_shift_zero<0x112, 0xf, 0xf>(v);
   v += dpp_shift_zero<0x114, 0xf, 0xf>(v);
@@ -433,20 +411,6 @@ __device__ __forceinline__ float block_sum_to_last(float v) {
 }
 
 // ---- per-surfel side sums of the forward blends ---------------------------------------------------------------------
-// accum_weights_p / accum_weights_count: a wavefront blends one list entry at a time, so the up to 64 per-pixel adds of
-// an entry go to one address. They are summed in the wavefront first (one DPP reduction, one population count) and lane 63
-// issues one atomic per output. Must be reached by all 64 lanes; `id` and the two pointers are wave-uniform.
-__device__ __forceinline__ void wave_accumulate_weights(bool blended, float w, int id, float* __restrict__ weights_p,
-                                                        int32_t* __restrict__ weights_count) {
-  const unsigned long long who = __ballot(blended);
-  if (who == 0ull) return;
-  const float total = wave_sum_to_lane63(blended ? w : 0.0f);
-  if ((threadIdx.x & 63) == 63) {
-    if (weights_p) atomicAdd(&weights_p[id], total);
-    if (weights_count) atomicAdd(&weights_count[id], (int) __popcll(who));
-  }
-}
-
 // accum_max_count in the surfel paths: the reference adds 1 to the count of the pixel's current arg-max surfel at EVERY
 // blended entry from the first one on (its flag is never reset). A pixel's arg-max changes a few times at most, so the
 // adds are kept as a run length and issued when the arg-max moves and once after the last entry: the same integer

@@ -12,8 +12,9 @@ constexpr float kCullPad = FSGS_CULL_PAD;  // pixels added around the footprint 
 
 // A pixel can only blend a surfel where alpha = min(0.99, o exp(-rho / 2)) >= 1/255, i.e. inside the perspective image of
 // the ellipse u^2 + v^2 <= tau = 2 ln(255 o) of the surfel's tangent plane, or inside the screen-space disc of the
-// low-pass filter. The blend kernels test the padded bounding box of that region and its extents along the two
-// diagonals against each 8x8 quadrant of a tile (quadrant_mask in blend.hpp); a (surfel, tile) instance that fails the
+// low-pass filter. The top-k blend tests the padded bounding box of that region and its extents along the two
+// diagonals against each 8x8 quadrant of a tile (quadrant_mask in blend.hpp; the blends proper bound the same region row
+// by row, block_lists.hpp); a (surfel, tile) instance that fails the
 // same test against the whole tile contributes to no pixel of it, so a binning that leaves it out of the tile's list
 // changes no image and no gradient (the lists get shorter, and the positions n_contrib counts in change with them).
 // The per-surfel part of the bound is formed once per surfel, the per-tile part is eight comparisons; it is evaluated

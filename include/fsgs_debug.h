@@ -15,7 +15,7 @@ extern "C" {
  * the achievable-bandwidth yardstick and counter calibration. */
 int fsgs_copy_probe(const void* src, void* dst, size_t nbytes, void* stream);
 
-/* The blend kernels skip, per 8x8 pixel quadrant, surfels whose alpha >= 1/255 footprint cannot reach it. enabled = 0
+/* The blend kernels skip, per pixel block (2x4 to 8x8), surfels whose alpha >= 1/255 footprint cannot reach it. enabled = 0
  * turns that skip off process-wide (every staged surfel is then evaluated at every pixel, as the reference does), so
  * tests can show that results do not depend on it. Default: on. Process-global: not for use next to concurrent renders. */
 int fsgs_debug_set_culling(int enabled);
