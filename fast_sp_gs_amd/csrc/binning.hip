@@ -130,7 +130,8 @@ static_assert(kCoopThreshold == kCullMaskTiles, "a lane's serial walk covers exa
 //   3. the same walk again scatters (depth bits << 32 | surfel) into the tile's segment; a block's cursor of a tile
 //      starts at the tile's start plus its column prefix, so neither step 1 nor step 3 issues a global atomic,
 //   4. one block per tile sorts its segment (unique 64-bit keys, so the arbitrary order inside a block's run does not
-//      matter): bitonic network in LDS for segments up to 16384 entries, in global memory beyond that.
+//      matter): by buckets of the depth bits in LDS for segments up to 2048 entries, by a bitonic network in LDS up to 16384
+//      entries and for depths that the buckets cannot part, in global memory beyond that.
 // Empty tiles get (0, 0) as the reference's zero-initialised ranges have. Tile grids above kMaxLdsTiles tiles (no room
 // for one LDS counter per tile) count and scatter with 64-bit global atomics on ranges[t].y instead (tile_emit_kernel).
 
@@ -677,7 +678,7 @@ constexpr int kLargeSegment = 16384;  // entries sorted by a 1024-lane block in 
 // entries in the other one, a binary search of log2 + 1 dependent reads. Such a segment is bound by its chain of LDS reads
 // and barriers: at most 15 reads and 4 barriers behind the chunks, where the network takes 20 rounds of read, exchange and
 // write by the one wavefront in four that has work there. Entries differ (their low halves are surfel numbers, one of each
-// in a tile). Kernel, lists of about 100 entries: 10k surfels 256x256 7.7 -> 5.3 us, 25k Gaussians 639x361 7.8 -> 5.2, fast
+// in a tile). Takes the segments that the buckets leave. Kernel, lists of about 100 entries: 10k surfels 256x256 7.7 -> 5.3 us, 25k Gaussians 639x361 7.8 -> 5.2, fast
 // path 150k 1001x667 11.4 -> 8.5. Not for longer segments: with two to eight entries per lane the 64-bit comparisons of the
 // counting outweigh the chain (300k 800x800, lists of about 600: 24 us by the network, 32 this way).
 constexpr int kMergeSegment = 256;
@@ -716,11 +717,146 @@ __device__ __forceinline__ void merge_sort_lds(uint64_t* e, int n) {
   }
 }
 
-// One block per tile: segments up to kSmallSegment entries are sorted in LDS, longer ones are queued for
+// ---- a tile's segment by buckets --------------------------------------------------------------------------------------
+constexpr int kSortBuckets = kSmallSegment / 2;  // their counters fill the LDS that the network's empty slots take
+constexpr int kBucketLimit = 32;                 // entries of one bucket that are put in order by counting
+
+// Exclusive prefix over the counters of a 256-lane block, in place, and the largest one: a lane owns kOwn neighbouring words of
+// kHalves counters (32 or 16 bits). s_wave: two words a wavefront. Two barriers; one more before the counters are read.
+template <int kOwn, int kHalves>
+__device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned* s_wave) {
+  constexpr unsigned kMask = kHalves == 2 ? 0xffffu : ~0u;
+  const int wave = threadIdx.x >> 6;
+  unsigned own[kOwn], sum = 0, most = 0;
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) {
+    const unsigned v = own[c] = s_count[kOwn * threadIdx.x + c];
+    sum += v & kMask, most = max(most, v & kMask);
+    if (kHalves == 2) sum += v >> 16, most = max(most, v >> 16);
+  }
+  const unsigned inc = (unsigned) wave_scan((int) sum);
+  most = wave_max_to_last(most);
+  if ((threadIdx.x & 63) == 63) s_wave[2 * wave] = inc, s_wave[2 * wave + 1] = most;
+  __syncthreads();
+  unsigned at = inc - sum;
+  most = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) at += s_wave[2 * w];
+    most = max(most, s_wave[2 * w + 1]);
+  }
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) {
+    const unsigned low = own[c] & kMask;
+    s_count[kOwn * threadIdx.x + c] = kHalves == 2 ? at | (at + low) << 16 : at;
+    at += kHalves == 2 ? low + (own[c] >> 16) : low;
+  }
+  __syncthreads();
+  return most;
+}
+
+// Sorts the n <= 256 * kPer entries at `entries` by a 256-lane block and writes list and keys. Bound by its chain of about ten
+// LDS round trips and five barriers, whatever n is, where the network takes 33 rounds and 7 barriers for 2048 entries: against
+// the network (merging up to 256 entries), 400k surfels 3840x2160 153 -> 41 us, 3M 1352x1014 62 -> 18, 300k 800x800 24 -> 7.6,
+// 300k Gaussians 29 -> 7.9, 150k 1001x667 9.2 -> 4.6, 10k 256x256 5.1 -> 3.7. With depths in two thin shells, which take the
+// second cut, 1100 entries a tile in 2500 tiles: 140 -> 94..124 us for the whole binning, 200 entries a tile: alike.
+// The buckets cut the span of the
+// segment's depth bits into equal parts, so they are in order among themselves; an entry's place is its bucket's start plus the
+// number of smaller entries in the bucket (all 64 bits compared), a few when the depths spread. When some bucket holds more
+// than kBucketLimit entries (surfaces at a few depths, a far outlier), every bucket is cut once more into as many parts as it
+// has entries. False, with nothing written and the keys in `key`, when that leaves too many together as well (equal depths):
+// the comparing sorts take such a segment.
+template <int kPer>
+__device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, const uint64_t* __restrict__ entries,
+                                            uint64_t (&key)[kPer], uint64_t* s_e, int32_t* __restrict__ point_list,
+                                            int64_t* __restrict__ keys_out) {
+  constexpr int kBuckets = kPer == 1 ? kSortBuckets / 2 : kSortBuckets, kOwn = kBuckets / 256;
+  unsigned* s_count = (unsigned*) (s_e + kSmallSegment);
+  unsigned* s_wave  = (unsigned*) s_e;  // before the entries come
+  const int wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) key[q] = entries[start + min((int) threadIdx.x + 256 * q, n - 1)];
+  unsigned lo = ~0u, hi = 0u;
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) s_count[kOwn * threadIdx.x + c] = 0u;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) lo = min(lo, (unsigned) (key[q] >> 32)), hi = max(hi, (unsigned) (key[q] >> 32));
+  lo = wave_max_to_last(~lo), hi = wave_max_to_last(hi);
+  if ((threadIdx.x & 63) == 63) s_wave[2 * wave] = lo, s_wave[2 * wave + 1] = hi;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) lo = w ? max(lo, s_wave[2 * w]) : s_wave[0], hi = w ? max(hi, s_wave[2 * w + 1]) : s_wave[1];
+  lo = ~lo;
+  const float scale = (float) kBuckets * __builtin_amdgcn_rcpf((float) (hi - lo) + 1.0f);
+  auto place  = [&](uint64_t k) { return (float) ((unsigned) (k >> 32) - lo) * scale; };  // monotone, like its integer part
+  auto bucket = [&](uint64_t k) { return min((int) place(k), kBuckets - 1); };
+  auto emit   = [&](uint64_t e, int first, int end) {
+    int to = first;
+    for (int i = first; i < end; ++i) to += s_e[i] < e;
+    point_list[start + to] = (int32_t) (uint32_t) e;
+    if (keys_out) keys_out[start + to] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
+  };
+  unsigned rank[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + 256 * q < n) rank[q] = atomicAdd(&s_count[bucket(key[q])], 1u);
+  __syncthreads();
+  if (prefix_counters<kOwn, 1>(s_count, s_wave) <= (unsigned) kBucketLimit) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      if ((int) threadIdx.x + 256 * q < n) s_e[s_count[bucket(key[q])] + rank[q]] = key[q];
+    __syncthreads();
+    // in bucket order now: a wavefront's lanes look through the same few buckets and write next to each other
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int p = threadIdx.x + 256 * q;
+      if (p < n) {
+        const uint64_t e = s_e[p];
+        const int b = bucket(e);
+        emit(e, s_count[b], b + 1 < kBuckets ? (int) s_count[b + 1] : n);
+      }
+    }
+    return true;
+  }
+  // part `fine` of n, 16-bit counters in the same words
+  constexpr int kOwnFine = kPer == 1 ? 1 : kPer / 2;
+  uint16_t* s_fine = (uint16_t*) s_count;
+  int fine[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int b = bucket(key[q]), first = s_count[b], held = (b + 1 < kBuckets ? (int) s_count[b + 1] : n) - first;
+    fine[q] = first + min((int) ((place(key[q]) - (float) b) * (float) held), max(held - 1, 0));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < kOwnFine; ++c) s_count[kOwnFine * threadIdx.x + c] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + 256 * q < n) {
+      const int shift = 16 * (fine[q] & 1);
+      rank[q] = (atomicAdd(&s_count[fine[q] >> 1], 1u << shift) >> shift) & 0xffffu;
+    }
+  __syncthreads();
+  if (prefix_counters<kOwnFine, 2>(s_count, s_wave) > (unsigned) kBucketLimit) return false;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + 256 * q < n) s_e[s_fine[fine[q]] + rank[q]] = key[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + 256 * q < n) emit(key[q], s_fine[fine[q]], fine[q] + 1 < n ? (int) s_fine[fine[q] + 1] : n);
+  return true;
+}
+
+// One block per tile: segments up to kSmallSegment entries are sorted in LDS by as many entries per lane as they need (the
+// first loads of all are in flight together), longer ones are queued for
 // tile_sort_large_kernel; empty tiles get the (0, 0) range the reference's zero-initialised output has.
+// Eight wavefronts per SIMD, as many as the LDS leaves room for: 49 -> 41 us at 400k surfels 3840x2160; what spills for it is
+// the second cut of segments above 1024 entries.
 // `order` (optional): the blend kernels' blockIdx -> tile table, longest lists first, so that the long segments start
 // sorting at once instead of wherever the image puts them in tile order (the launch ends with its slowest block).
-__global__ void __launch_bounds__(256) tile_sort_small_kernel(int64_t* __restrict__ ranges,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) tile_sort_small_kernel(int64_t* __restrict__ ranges,
     const uint64_t* __restrict__ entries, int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out,
     int* __restrict__ large_count, int* __restrict__ large_list, const int* __restrict__ order, int n_tiles,
     int64_t R, const int* __restrict__ kept, uint64_t pad_key) {
@@ -749,18 +885,31 @@ __global__ void __launch_bounds__(256) tile_sort_small_kernel(int64_t* __restric
     return;
   }
   const int n = (int) len;
-  if (n <= kMergeSegment) {
-    s_e[threadIdx.x] = (int) threadIdx.x < n ? entries[start + threadIdx.x] : ~0ull;
-    __syncthreads();
-    merge_sort_lds(s_e, n);
-    tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
-    return;
-  }
-  const int m = padded_length(n);
-  for (int k = threadIdx.x; k < m; k += 256) s_e[lds_slot<true>(k)] = k < n ? entries[start + k] : ~0ull;
-  __syncthreads();
-  bitonic_sort_lds<true>(s_e, m, 256);
-  tile_sort_output<true>(tile, start, n, s_e, point_list, keys_out);
+  auto sort = [&](auto per) {  // entries per lane
+    constexpr int kPer = decltype(per)::value;
+    uint64_t key[kPer];
+    if (bucket_sort(tile, start, n, entries, key, s_e, point_list, keys_out)) return;
+    if constexpr (kPer == 1) {
+      s_e[threadIdx.x] = (int) threadIdx.x < n ? key[0] : ~0ull;
+      __syncthreads();
+      merge_sort_lds(s_e, n);
+      tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
+    } else {
+      const int m = padded_length(n);
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int k = threadIdx.x + 256 * q;
+        if (k < m) s_e[lds_slot<true>(k)] = k < n ? key[q] : ~0ull;
+      }
+      __syncthreads();
+      bitonic_sort_lds<true>(s_e, m, 256);
+      tile_sort_output<true>(tile, start, n, s_e, point_list, keys_out);
+    }
+  };
+  if (n <= kMergeSegment) sort(std::integral_constant<int, 1>());
+  else if (n <= 512) sort(std::integral_constant<int, 2>());
+  else if (n <= 1024) sort(std::integral_constant<int, 4>());
+  else sort(std::integral_constant<int, 8>());
 }
 
 // A few blocks walk the queue of long segments: up to kLargeSegment entries in LDS, beyond that the same network on the

@@ -399,6 +399,25 @@ __device__ __forceinline__ float dpp_shift_zero(float v) {
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, kRowMask, kBankMask, true));
 }
 
+// Inclusive prefix sums over the 64 lanes.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int scan_step(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, true);
+}
+__device__ __forceinline__ int wave_scan(int v) {
+  v = scan_step<0x111, 0xf>(v), v = scan_step<0x112, 0xf>(v), v = scan_step<0x114, 0xf>(v), v = scan_step<0x118, 0xf>(v);
+  return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
+}
+
+// Largest of the 64 lanes' values; valid in lane 63 only.
+__device__ __forceinline__ unsigned wave_max_to_last(unsigned v) {
+  auto step = [&](unsigned o) { v = max(v, o); };
+  step(__builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false)), step(__builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false)), step(__builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false)), step(__builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+
 // Sum over each aligned group of 8 or 16 lanes; the total is valid in the group's last lane only.
 template <int kLanes>
 __device__ __forceinline__ float block_sum_to_last(float v) {

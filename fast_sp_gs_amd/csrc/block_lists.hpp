@@ -248,15 +248,6 @@ __device__ __forceinline__ unsigned pair_blocks(unsigned m) {
 constexpr int kRowBatch = 128;  // entries staged at most: a byte names one, two wavefronts stage them
 // A byte names one of a pool's kPlaces <= 255 places, too; one more behind them, number kPlaces, holds zeros.
 
-template <int kCtrl, int kRows>
-__device__ __forceinline__ int scan_step(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, true);
-}
-__device__ __forceinline__ int wave_scan(int v) {  // inclusive prefix sums over the lanes
-  v = scan_step<0x111, 0xf>(v), v = scan_step<0x112, 0xf>(v), v = scan_step<0x114, 0xf>(v), v = scan_step<0x118, 0xf>(v);
-  return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
-}
-
 __device__ __forceinline__ uint4 no_places(int zeros) {
   const unsigned w = 0x01010101u * (unsigned) zeros;
   return make_uint4(w, w, w, w);

@@ -25,3 +25,24 @@ def test_list_of_one_tile(n, depths, device, oracle_mod):
     want_ranges, want_pl, want_keys = oracle_mod.prepare(16, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
     assert want_pl.size == n
     assert np.array_equal(npy(ranges), want_ranges) and np.array_equal(npy(pl), want_pl) and np.array_equal(npy(keys), want_keys)
+
+
+@pytest.mark.parametrize('n', [1, 2, 65, 255, 256, 257, 512, 513, 1024, 1025, 1999, 2048])
+@pytest.mark.parametrize('depths', ['shells', 'outlier', 'signs', 'ties'])
+def test_list_of_one_tile_by_buckets(n, depths, device, oracle_mod):
+    """Depths that fill few buckets (two thin shells, one far value) or span all bit patterns, and buckets with ties."""
+    from fast_sp_gs_amd._C import get_C_function
+    print(f'[tile sort] n={n} {depths}', flush=True)
+    g = torch.Generator().manual_seed(n)
+    r = torch.rand(n, generator=g)
+    far = r + 1.0
+    far[n // 2] = 3e38
+    dep = {'shells': torch.randint(1, 3, (n,), generator=g).float() + 1e-3 * r, 'outlier': far,
+           'signs': torch.randn(n, generator=g) * 10.0 ** torch.randint(-30, 30, (n,), generator=g),
+           'ties': (r * n / 4).floor() + 1.0}[depths].float()
+    m2 = torch.full((n, 2), 8.0)
+    radii, touched = torch.full((n,), 3, dtype=torch.int32), torch.ones(n, dtype=torch.int32)
+    ranges, pl, keys = get_C_function('GS_prepare')(16, 16, m2.to(device), dep.to(device), radii.to(device),
+                                                    touched.to(device), False, return_keys=True)[:3]
+    want_ranges, want_pl, want_keys = oracle_mod.prepare(16, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
+    assert np.array_equal(npy(ranges), want_ranges) and np.array_equal(npy(pl), want_pl) and np.array_equal(npy(keys), want_keys)
