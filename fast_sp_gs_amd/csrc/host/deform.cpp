@@ -208,22 +208,28 @@ struct Apply : public torch::autograd::Function<Apply> {
     at::AutoDispatchBelowADInplaceOrView no_graph;
     const variable_list upstream = g;
     for (auto& x : g) x = contiguous(x);
-    Tensor g_s = g[1], g_r;  // the sums hand their upstream gradient to both addends
+    const Tensor &scales = t[0], &rotations = t[1];
     const bool rot = g[2].defined(), logs = log_scales && g[1].defined();
-    if (rot || logs) {
-      const Tensor &scales = t[0], &rotations = t[1];
-      g_r = at::empty_like(rotations);
-      const Tensor up = rot ? g[2] : at::zeros_like(rotations);
-      if (logs) g_s = at::empty_like(scales);
-      check(fsgs_deform_apply_backward((int) scales.size(0), (int) scales.size(1), logs, f32(scales), f32(rotations), f32(t[2]),
-                                       logs ? f32(g[1]) : nullptr, f32(up), logs ? f32(g_s) : nullptr, f32(g_r),
-                                       stream_of(scales)),
+    auto both = [&](size_t k) { return ctx->needs_input_grad(k) && ctx->needs_input_grad(k + 1); };
+    // the sums hand their upstream gradient to both addends: a tensor each, or a leaf's accumulation copies it once more
+    Tensor g_p = g[0], g_s = g[1], g_r, g_dr;
+    if (g[0].defined() && both(0)) g_p = at::empty_like(g[0]);
+    if (logs || (g[1].defined() && both(2))) g_s = at::empty_like(scales);
+    if (rot || logs) g_r = at::empty_like(rotations);
+    g_dr = rot && both(4) ? at::empty_like(rotations) : g_r;
+    const bool copy_p = g[0].defined() && both(0), copy_s = !logs && g[1].defined() && both(2), copy_r = rot && both(4);
+    if (rot || logs || copy_p || copy_s) {
+      const Tensor up = rot || !logs ? g[2] : at::zeros_like(rotations);
+      check(fsgs_deform_apply_backward_copies((int) scales.size(0), (int) scales.size(1), logs, f32(scales), f32(rotations),
+                                              f32(t[2]), f32(g[0]), f32(g[1]), f32(up), logs ? f32(g_s) : nullptr, f32(g_r),
+                                              copy_p ? f32(g_p) : nullptr, copy_s ? f32(g_s) : nullptr,
+                                              copy_r ? f32(g_dr) : nullptr, stream_of(scales)),
             "deform_apply_backward");
-      if (!rot) g_r = Tensor();
     }
+    if (!rot) g_r = g_dr = Tensor();
     auto pick = [&](size_t k, const Tensor& x) { return ctx->needs_input_grad(k) ? x : Tensor(); };
-    return first_order_only(upstream, {t[0], t[1], t[2]}, {pick(0, g[0]), pick(1, g[0]), pick(2, g_s), pick(3, g[1]), pick(4, g_r),
-                                                           pick(5, g_r), Tensor()});
+    return first_order_only(upstream, {t[0], t[1], t[2]}, {pick(0, g_p), pick(1, g[0]), pick(2, g_s), pick(3, g[1]), pick(4, g_r),
+                                                           pick(5, g_dr), Tensor()});
   }
 };
 

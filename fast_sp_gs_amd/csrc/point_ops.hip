@@ -573,17 +573,36 @@ __global__ void __launch_bounds__(256) deform_apply_forward_kernel(int N, int lo
   ((float4*) out_rot)[i] = make_float4(x * inv, y * inv, z * inv, w * inv);
 }
 
-// Gradients that are not the upstream gradient itself: through the normalisation to rotations / d_rotation (the same
-// tensor for both) and, for logarithmic scales, g * exp(scale). points, d_xyz and d_scale receive their output's
-// gradient unchanged, so nothing is computed for them.
+// Gradients that are not the upstream gradient itself: through the normalisation to rotations / d_rotation (the same for
+// both) and, for logarithmic scales, g * exp(scale). points, d_xyz and d_scale receive their output's gradient unchanged.
+// Where both addends of a sum want a gradient, `copy` takes a second one (points' from g_out_points, scales' from
+// g_out_scales, d_rot's): one tensor handed to both would be copied by a launch of its own when a leaf accumulates it. 200k
+// points: 5.4 us and three copies of 5 us -> 6.8 us.
+struct ApplyCopies {
+  const float* g_out_points;  // with points
+  float *points, *scales, *rot;
+};
 template <int S>
 __global__ void __launch_bounds__(256) deform_apply_backward_kernel(int N, int log_scales,
     const float* __restrict__ scales, const float* __restrict__ rot, const float* __restrict__ d_rot,
     const float* __restrict__ g_out_scales, const float* __restrict__ g_out_rot, float* __restrict__ g_scales,
-    float* __restrict__ g_rot) {
+    float* __restrict__ g_rot, ApplyCopies copy) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
+  // element for element, a block's 256 points in rows of 256 lanes
+  if (copy.points)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int64_t e = (int64_t) blockIdx.x * (3 * 256) + c * 256 + threadIdx.x;
+      if (e < 3 * (int64_t) N) copy.points[e] = copy.g_out_points[e];
+    }
+  if (copy.scales)
+#pragma unroll
+    for (int c = 0; c < S; ++c) {
+      const int64_t e = (int64_t) blockIdx.x * (S * 256) + c * 256 + threadIdx.x;
+      if (e < S * (int64_t) N) copy.scales[e] = g_out_scales[e];
+    }
+  if (i >= N || !g_rot) return;
   if (log_scales)
 #pragma unroll
     for (int c = 0; c < S; ++c)
@@ -601,6 +620,7 @@ __global__ void __launch_bounds__(256) deform_apply_backward_kernel(int N, int l
     o = make_float4(g.x * 1e12f, g.y * 1e12f, g.z * 1e12f, g.w * 1e12f);
   }
   ((float4*) g_rot)[i] = o;
+  if (copy.rot) ((float4*) copy.rot)[i] = o;
 }
 
 // The same update for every parameter tensor of a point set in one launch: the reference steps its parameter groups one
@@ -703,7 +723,23 @@ FSGS_API int fsgs_deform_apply_backward(int N, int S, int log_scales, const floa
                "deform_apply_backward: rotations must be 16-byte aligned");
   auto kernel = S == 2 ? deform_apply_backward_kernel<2> : deform_apply_backward_kernel<3>;
   hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, (hipStream_t) stream, N, log_scales, scales, rot,
-                     d_rot, g_out_scales, g_out_rot, g_scales, g_rot);
+                     d_rot, g_out_scales, g_out_rot, g_scales, g_rot, ApplyCopies{});
+  return check_launch("deform_apply_backward");
+}
+
+FSGS_API int fsgs_deform_apply_backward_copies(int N, int S, int log_scales, const float* scales, const float* rot,
+    const float* d_rot, const float* g_out_points, const float* g_out_scales, const float* g_out_rot, float* g_scales,
+    float* g_rot, float* copy_points, float* copy_scales, float* copy_rot, void* stream) {
+  FSGS_REQUIRE(N >= 0 && (S == 2 || S == 3), "deform_apply_backward: N >= 0 and 2 or 3 scales per point");
+  if (N == 0) return kOk;
+  FSGS_REQUIRE((!g_rot || (rot && d_rot && g_out_rot && (!log_scales || (scales && g_out_scales && g_scales)))) &&
+               (!copy_points || g_out_points) && (!copy_scales || g_out_scales) && (!copy_rot || g_rot),
+               "deform_apply_backward: null pointer");
+  FSGS_REQUIRE((((uintptr_t) rot | (uintptr_t) d_rot | (uintptr_t) g_out_rot | (uintptr_t) g_rot | (uintptr_t) copy_rot) & 15) == 0,
+               "deform_apply_backward: rotations must be 16-byte aligned");
+  auto kernel = S == 2 ? deform_apply_backward_kernel<2> : deform_apply_backward_kernel<3>;
+  hipLaunchKernelGGL(kernel, dim3(div_up(N, 256)), dim3(256), 0, (hipStream_t) stream, N, log_scales, scales, rot,
+                     d_rot, g_out_scales, g_out_rot, g_scales, g_rot, ApplyCopies{g_out_points, copy_points, copy_scales, copy_rot});
   return check_launch("deform_apply_backward");
 }
 

@@ -867,6 +867,11 @@ int fsgs_deform_apply_forward(int N, int S, int log_scales, const float* points,
     float* out_scales, float* out_rot, void* stream);
 int fsgs_deform_apply_backward(int N, int S, int log_scales, const float* scales, const float* rot, const float* d_rot,
     const float* g_out_scales, const float* g_out_rot, float* g_scales, float* g_rot, void* stream);
+/* The same, with second tensors for the addends of a sum that both want a gradient (each optional): copy_points[N,3] =
+ * g_out_points, copy_scales[N,S] = g_out_scales, copy_rot[N,4] = g_rot. g_rot == NULL: only copies are made. */
+int fsgs_deform_apply_backward_copies(int N, int S, int log_scales, const float* scales, const float* rot, const float* d_rot,
+    const float* g_out_points, const float* g_out_scales, const float* g_out_rot, float* g_scales, float* g_rot,
+    float* copy_points, float* copy_scales, float* copy_rot, void* stream);
 
 /* AdamMasksedUpdated -- fast_2d_gs/_C/src/other/adam_masked_update.cu:30-35 (kernel :9-28). Rows of the [N,M]
  * tensors whose mask byte is 0 are left untouched; eps is added to sqrt(v); lr carries the bias correction. */

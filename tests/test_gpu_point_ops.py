@@ -748,6 +748,37 @@ def test_deform_apply_matches_the_torch_operators(S, log_scales, device):
     assert torch.equal(c[5].grad, a[5].grad) and torch.equal(c[1].grad, a[1].grad)
 
 
+@pytest.mark.parametrize("N", [1, 255, 256, 257, 1025])
+@pytest.mark.parametrize("used", [(0,), (1,), (2,), (0, 1), (1, 2), (0, 1, 2)])
+@pytest.mark.parametrize("S,log_scales", [(2, False), (3, False), (2, True)])
+def test_deform_apply_gradients_of_both_addends(N, used, S, log_scales, device):
+    """Each addend gets a tensor of its own, whichever outputs are used: equal to the upstream gradient bit for bit, or to the
+    other addend's, and to the torch operators' gradients as in the test above."""
+    from fast_sp_gs_amd.deform import deform_apply
+    g = torch.Generator().manual_seed(N)
+    mk = lambda *s_: torch.randn(*s_, generator=g).to(device)
+    a = [t.requires_grad_(True) for t in (mk(N, 3), mk(N, 3), mk(N, S), mk(N, S), mk(N, 4), mk(N, 4))]
+    b = [t.detach().clone().requires_grad_(True) for t in a]
+    out = deform_apply(*a, log_scales=log_scales)
+    ref = (b[0] + b[1], (torch.exp(b[2]) if log_scales else b[2]) + b[3], torch.nn.functional.normalize(b[4] + b[5], dim=-1))
+    go = [mk(*o.shape) for o in out]
+    got = torch.autograd.grad([out[k] for k in used], a, [go[k] for k in used], allow_unused=True)
+    want = torch.autograd.grad([ref[k] for k in used], b, [go[k] for k in used], allow_unused=True)
+    for k in range(3):
+        x, y = got[2 * k], got[2 * k + 1]
+        assert (x is None) == (y is None) == (k not in used)
+        if k not in used:
+            continue
+        assert x.data_ptr() != y.data_ptr()
+        if k == 0:
+            assert torch.equal(x, go[0]) and torch.equal(y, go[0])
+        elif k == 1:
+            assert torch.equal(y, go[1]) and (log_scales or torch.equal(x, go[1]))
+        else:
+            assert torch.equal(x, y)
+        assert rel_err(npy(x), npy(want[2 * k])) < 1e-5 and rel_err(npy(y), npy(want[2 * k + 1])) < 1e-5
+
+
 def test_full_size_properties(device):
     """Full benchmark-size runs checked through size-independent properties (no oracle at this size)."""
     from fast_sp_gs_amd import scenes
