@@ -491,6 +491,37 @@ void adam_masked(const std::vector<Tensor>& params, const std::vector<Tensor>& g
           what);
 }
 
+namespace {
+// Advances a step count as torch keeps it (a float32 word on the host), or however a loaded state holds it.
+double advanced(const char* what, const Tensor& step) {
+  if (step.numel() != 1) fail(std::string(what) + ": a step count is one number");
+  const bool plain = step.is_cpu() && step.scalar_type() == at::kFloat;
+  return plain ? (double) (*step.data_ptr<float>() += 1.0f) : step.add_(1).item<double>();
+}
+}  // namespace
+
+void adam_masked_step(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
+                      const std::vector<Tensor>& v, const std::vector<Tensor>& steps, const Tensor& mask,
+                      const std::vector<double>& lr, double b1, double b2, const std::vector<double>& eps, int64_t N) {
+  const char* what = "AdamMasksedUpdatedMulti";
+  const size_t n = params.size();
+  if (steps.size() != n || lr.size() != n) fail("AdamMasksedUpdatedMulti: a step count and a rate per parameter tensor");
+  std::vector<double> rate;
+  double at_count = -1.0;  // count of the corrections at hand: the tensors of a step share it
+  float root_c2 = 0.0f, c1 = 0.0f;
+  for (size_t k = 0; k < n; ++k) {
+    const double taken = advanced(what, steps[k]);
+    if (taken != at_count) {
+      root_c2  = (float) at::pow(at::rsub(at::pow(b2, steps[k]), 1), 0.5).item<double>();
+      c1       = (float) at::rsub(at::pow(b1, steps[k]), 1).item<double>();
+      at_count = taken;
+    }
+    const float scaled = (float) lr[k] * root_c2;
+    rate.push_back((double) (scaled / c1));
+  }
+  adam_masked(params, grads, m, v, mask, rate, b1, b2, eps, N);
+}
+
 void adam_dense(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
                 const std::vector<Tensor>& v, const std::vector<Tensor>& steps, double lr, double b1, double b2, double eps) {
   const AdamPointers t("adam_update", params, grads, m, v);
@@ -499,10 +530,7 @@ void adam_dense(const std::vector<Tensor>& params, const std::vector<Tensor>& gr
   std::vector<int64_t> count;
   std::vector<double> step_size, root_c2;
   for (size_t k = 0; k < n; ++k) {
-    const Tensor& step = steps[k];
-    if (step.numel() != 1) fail("adam_update: a step count is one number");
-    const bool plain = step.is_cpu() && step.scalar_type() == at::kFloat;  // as torch keeps it
-    const double taken = plain ? (double) (*step.data_ptr<float>() += 1.0f) : step.add_(1).item<double>();
+    const double taken = advanced("adam_update", steps[k]);
     count.push_back(params[k].numel());
     step_size.push_back(lr / (1 - std::pow(b1, taken))), root_c2.push_back(std::sqrt(1 - std::pow(b2, taken)));
   }

@@ -41,6 +41,11 @@ void adam_masked(const std::vector<Tensor>& params, const std::vector<Tensor>& g
                  const std::vector<Tensor>& v, const Tensor& mask, const std::vector<double>& lr, double b1, double b2,
                  const std::vector<double>& eps, int64_t N);
 // torch.optim.Adam's plain step; `steps` (one count per parameter) are advanced by it
+// The same with step counts, which the call advances: the rates are lr * sqrt(1 - b2^t) / (1 - b1^t) on float32 tensors, as the
+// reference forms them (sparse_gaussian_adam.py:42-46): the powers are torch's, every operation rounds to float32.
+void adam_masked_step(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
+                      const std::vector<Tensor>& v, const std::vector<Tensor>& steps, const Tensor& mask,
+                      const std::vector<double>& lr, double b1, double b2, const std::vector<double>& eps, int64_t N);
 void adam_dense(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& m,
                 const std::vector<Tensor>& v, const std::vector<Tensor>& steps, double lr, double b1, double b2, double eps);
 

@@ -76,7 +76,10 @@ class DynamicStep:
         visible = out['visibility_filter']
         self.opt.set_before_step(visible, self.params[0].shape[0])
         self.opt.step()
-        self.opt.zero_grad(set_to_none=True)
         self.net_opt.step()
-        self.net_opt.zero_grad(set_to_none=True)
+        # what the optimisers' zero_grad does, without its hooks and per-device lists
+        for opt in (self.opt, self.net_opt):
+            for group in opt.param_groups:
+                for p in group['params']:
+                    p.grad = None
         return loss.detach(), visible
