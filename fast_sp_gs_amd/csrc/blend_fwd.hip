@@ -17,6 +17,7 @@
 // 10k 256x256: 28, 19, 18. Batches of 64 / 128 / 192 surfels (a list's length varies less over a long batch), 2x4: 113 / 97 /
 // 94 us at 300k, 346 / 297 / 282 at 3M.
 #include "block_lists.hpp"
+#include "view_maps.hpp"
 
 namespace fsgs {
 namespace {
@@ -42,7 +43,7 @@ blend_forward_kernel(
     const float* __restrict__ trans_mat_t2, int32_t* __restrict__ n_contrib,
     float* __restrict__ out_color, float* __restrict__ out_opacity, float* __restrict__ out_extras,
     float2* __restrict__ out_flow, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
-    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks) {
+    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks, ViewMaps maps) {
   using Shape = BlockShape<kFwdLanes>;
   __shared__ Splat s_splat[kFwdBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kFwdBatch * 9 : 1];
@@ -201,22 +202,26 @@ blend_forward_kernel(
   if (kAccum == 2) flush_weights();
   if (kHits && b > 0) flush_hits(b - 1);  // entries behind it are behind every pixel's last one
   if (inside) {
-    out_opacity[pix]      = 1.0f - T;
+    const float opacity   = 1.0f - T;
+    out_opacity[pix]      = opacity;
     n_contrib[pix]        = last;
     n_contrib[pix + HW]   = kAux ? median_c : 0;
-    out_color[pix]        = C0;
-    out_color[pix + HW]   = C1;
-    out_color[pix + 2 * HW] = C2;
+    out_color[pix]        = kAux ? maps.colour(0, C0, opacity) : C0;
+    out_color[pix + HW]   = kAux ? maps.colour(1, C1, opacity) : C1;
+    out_color[pix + 2 * HW] = kAux ? maps.colour(2, C2, opacity) : C2;
     if (kAux) {
-      out_extras[pix + 0 * HW] = D;
-      out_extras[pix + 1 * HW] = N0;
-      out_extras[pix + 2 * HW] = N1;
-      out_extras[pix + 3 * HW] = N2;
-      out_extras[pix + 4 * HW] = median;
-      out_extras[pix + 5 * HW] = dist;
-      out_extras[pix + 6 * HW] = M1;
-      out_extras[pix + 7 * HW] = M2;
-      out_extras[pix + 8 * HW] = wsum;
+      if (maps.normals) maps.write(HW, pix, N0, N1, N2, D, median, dist);
+      if (out_extras) {
+        out_extras[pix + 0 * HW] = D;
+        out_extras[pix + 1 * HW] = N0;
+        out_extras[pix + 2 * HW] = N1;
+        out_extras[pix + 3 * HW] = N2;
+        out_extras[pix + 4 * HW] = median;
+        out_extras[pix + 5 * HW] = dist;
+        out_extras[pix + 6 * HW] = M1;
+        out_extras[pix + 7 * HW] = M2;
+        out_extras[pix + 8 * HW] = wsum;
+      }
       if (kFlow) {
         const float ws = wsum == 0.0f ? 1e-7f : wsum;
         out_flow[pix]  = make_float2(f0 / ws, f1 / ws);
@@ -267,13 +272,15 @@ int render_forward(int P, int W, int H, double near_n, double far_n, int only_im
     const float* means2D, const float* colors, const float* normal_opacity, const float* trans_mat,
     const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
     float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
-    float* out_flow, int32_t* n_contrib, const float* records, uint32_t* hit_blocks, void* stream) {
+    float* out_flow, int32_t* n_contrib, const float* records, uint32_t* hit_blocks, const ViewMaps& maps, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_render_forward: bad sizes");
   FSGS_REQUIRE(ranges && out_color && out_opacity && n_contrib, "GS_2D_render_forward: null pointer");
   FSGS_REQUIRE(P == 0 || records || (means2D && colors && normal_opacity && trans_mat),
                "GS_2D_render_forward: null surfel tensor");
   FSGS_REQUIRE(((uintptr_t) records & 15) == 0, "GS_2D_render_forward: records must be 16-byte aligned");
-  FSGS_REQUIRE(only_image || out_extras, "GS_2D_render_forward: out_extras is required unless only_image");
+  FSGS_REQUIRE(only_image || out_extras || (maps.normals && maps.distortion),
+               "GS_2D_render_forward: out_extras is required unless only_image");
+  FSGS_REQUIRE(!maps.normals || (maps.Tw2v && maps.surf_depth), "GS_2D_render_forward: null map");
   const bool aux   = !only_image;
   const bool flow  = aux && trans_mat_t2 != nullptr;
   const int accum = !aux ? 0 : (accum_weights_p || accum_weights_count) ? 2 : accum_max_count ? 1 : 0;
@@ -287,7 +294,7 @@ int render_forward(int P, int W, int H, double near_n, double far_n, int only_im
   hipLaunchKernelGGL((blend_forward_kernel<AUX, FLOW, ACC, HITS>), grid, block, 0, s, ordered, tile_order, W, H, (float) near_n, \
                      (float) far_n, ranges, point_list, (const float2*) means2D, colors, trans_mat,                  \
                      (const float4*) normal_opacity, (const float4*) records, trans_mat_t2, n_contrib, out_color, out_opacity, \
-                     out_extras, (float2*) out_flow, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks)
+                     out_extras, (float2*) out_flow, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks, maps)
 #define FSGS_LAUNCH_FWD_HITS(FLOW, ACC)              \
   if (hit_blocks) FSGS_LAUNCH_FWD(true, FLOW, ACC, true); \
   else FSGS_LAUNCH_FWD(true, FLOW, ACC, false)
@@ -312,17 +319,19 @@ FSGS_API int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, doubl
     float* out_flow, int32_t* n_contrib, const float* records, void* stream) {
   return render_forward(P, W, H, near_n, far_n, only_image, means2D, colors, normal_opacity, trans_mat, point_list, ranges,
                         trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count, out_color, out_opacity, out_extras,
-                        out_flow, n_contrib, records, nullptr, stream);
+                        out_flow, n_contrib, records, nullptr, ViewMaps{}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* colors, const float* normal_opacity, const float* trans_mat, const int32_t* point_list,
     const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count, float* accum_weights_p,
     int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras, float* out_flow,
-    int32_t* n_contrib, const float* records, uint32_t* hit_blocks, void* stream) {
+    int32_t* n_contrib, const float* records, uint32_t* hit_blocks, double depth_ratio, const float* Tw2v,
+    const float* background, float* normals, float* depths, float* surf_depth, float* distortion, void* stream) {
   return render_forward(P, W, H, near_n, far_n, 0, means2D, colors, normal_opacity, trans_mat, point_list, ranges, trans_mat_t2,
                         accum_max_count, accum_weights_p, accum_weights_count, out_color, out_opacity, out_extras, out_flow,
-                        n_contrib, records, hit_blocks, stream);
+                        n_contrib, records, hit_blocks,
+                        ViewMaps{Tw2v, background, normals, depths, surf_depth, distortion, (float) depth_ratio}, stream);
 }
 
 FSGS_API int fsgs_debug_tile_order(int gx, int gy, const int64_t* ranges, int32_t* table, void* stream) {

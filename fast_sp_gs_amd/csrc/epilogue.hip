@@ -4,12 +4,12 @@
 // two depth maps, surf_depth mix, pseudo surface normal from the depth map, times the detached opacity), its helpers
 // depths_to_points / depth_to_normal (:439-470) and the background composite of fast_2d_gs/network.py:725-726. In the
 // reference these are ~25 elementwise / matmul / inverse launches over HW per view and as many again in autograd; here
-// one kernel each way. The 3x3 pixel -> world ray matrix (inverse intrinsics, then the camera-to-world rotation) and
+// one kernel each way, or for a whole view the pseudo normal alone behind a blend that wrote the rest (view_maps.hpp). The 3x3 pixel -> world ray matrix (inverse intrinsics, then the camera-to-world rotation) and
 // the camera centre are derived from Tw2v / Tv2c by the first lane of every block.
 //
 // intrins = ((c2w^T (Tv2c Tw2v)^T) ndc2pix^T)[:3,:3]^T of the reference equals (ndc2pix Tv2c)[:3,:3] because
 // c2w = Tw2v^-1; it is formed in that closed form.
-#include "common.hpp"
+#include "view_maps.hpp"
 
 namespace fsgs {
 namespace {
@@ -52,11 +52,6 @@ __device__ inline void pixel_rays(int W, int H, const float* __restrict__ Tw2v, 
     for (int b = 0; b < 3; ++b) out.m[a * 3 + b] = Ri[a * 3] * Ki[b] + Ri[a * 3 + 1] * Ki[3 + b] + Ri[a * 3 + 2] * Ki[6 + b];
 }
 
-// torch.nan_to_num(x, 0, 0): NaN and +inf become 0, -inf the lowest finite float.
-__device__ __forceinline__ float nan0(float v) {
-  if (v != v || v == __builtin_inff()) return 0.0f;
-  return v == -__builtin_inff() ? -3.4028234663852886e38f : v;
-}
 __device__ __forceinline__ bool finite_f(float v) { return v == v && fabsf(v) != __builtin_inff(); }
 
 struct Vec3 {
@@ -73,7 +68,7 @@ struct DepthMaps {
   int W;
   __device__ __forceinline__ float surf(int x, int y) const {
     const size_t p = (size_t) y * W + x;
-    return nan0(depth[p]) * (1.0f - ratio) + ratio * nan0(median[p]);
+    return mixed_depth(depth[p], median[p], ratio);
   }
 };
 
@@ -104,10 +99,9 @@ __global__ void __launch_bounds__(256) epilogue_forward_kernel(int W, int H, flo
   if (x >= W || y >= H) return;
   const size_t HW = (size_t) H * W, p = (size_t) y * W + x;
   const DepthMaps maps = {extras, extras + 4 * HW, ratio, W};
-  // normals to world space: row vector times Tw2v[:3,:3]
   const float n0 = extras[HW + p], n1 = extras[2 * HW + p], n2 = extras[3 * HW + p];
 #pragma unroll
-  for (int j = 0; j < 3; ++j) normals[j * HW + p] = n0 * Tw2v[j] + n1 * Tw2v[4 + j] + n2 * Tw2v[8 + j];
+  for (int j = 0; j < 3; ++j) normals[j * HW + p] = world_normal(Tw2v, j, n0, n1, n2);
   if (depths) depths[p] = nan0(maps.median[p]);
   surf_depth[p] = maps.surf(x, y);
   Vec3 n = {0.0f, 0.0f, 0.0f};
@@ -122,7 +116,51 @@ __global__ void __launch_bounds__(256) epilogue_forward_kernel(int W, int H, flo
   if (composited) {
     const float t = 1.0f - opacity[p];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) composited[c * HW + p] = images[c * HW + p] + t * background[c];
+    for (int c = 0; c < 3; ++c) composited[c * HW + p] = fmaf(t, background[c], images[c * HW + p]);
+  }
+}
+
+// The pseudo normal alone, for a view whose blend wrote the other maps (view_maps.hpp): 1 channel and its neighbours in, 3 out.
+// Bound by memory; the rays are formed by every lane for itself, four rows of pixels share them and the column's points.
+// 3840x2160: 167 us as the whole epilogue (9 channels in, 11 out) -> 37 (4.5 TB/s) and 22 more in the blend, which leaves out 8 of
+// its 9 extra channels when no backward will read them; 1352x1014 with a backward 30 -> 10 (blend +3), 800x800 11.4 -> 5.7 (+1.4).
+constexpr int kNormalRows = 4;
+__global__ void __launch_bounds__(256) surf_normal_kernel(int W, int H, const float* __restrict__ Tw2v,
+    const float* __restrict__ Tv2c, const float* __restrict__ surf_depth, const float* __restrict__ opacity,
+    float* __restrict__ surf_normal) {
+  PixelRays r;
+  pixel_rays(W, H, Tw2v, Tv2c, r);
+  const int x = blockIdx.x * 64 + threadIdx.x, y0 = (blockIdx.y * 4 + threadIdx.y) * kNormalRows;
+  if (x >= W || y0 >= H) return;
+  const size_t HW = (size_t) H * W;
+  auto depth = [&](int px, int py) { return surf_depth[(size_t) min(max(py, 0), H - 1) * W + min(max(px, 0), W - 1)]; };
+  float column[kNormalRows + 2], left[kNormalRows], right[kNormalRows], o[kNormalRows];
+#pragma unroll
+  for (int k = 0; k < kNormalRows + 2; ++k) column[k] = depth(x, y0 + k - 1);
+#pragma unroll
+  for (int k = 0; k < kNormalRows; ++k) {
+    left[k] = depth(x - 1, y0 + k), right[k] = depth(x + 1, y0 + k);
+    o[k]    = opacity[(size_t) min(y0 + k, H - 1) * W + x];
+  }
+  auto point = [&](int px, int py, float s) -> Vec3 {
+    const float fx = (float) px, fy = (float) py;
+    return {s * (r.m[0] * fx + r.m[1] * fy + r.m[2]) + r.o[0], s * (r.m[3] * fx + r.m[4] * fy + r.m[5]) + r.o[1],
+            s * (r.m[6] * fx + r.m[7] * fy + r.m[8]) + r.o[2]};
+  };
+#pragma unroll
+  for (int k = 0; k < kNormalRows; ++k) {
+    const int y = y0 + k;
+    if (y >= H) return;
+    Vec3 n = {0.0f, 0.0f, 0.0f};
+    if (x >= 1 && y >= 1 && x <= W - 2 && y <= H - 2) {
+      const Vec3 up = point(x, y - 1, column[k]), dn = point(x, y + 1, column[k + 2]);
+      const Vec3 lf = point(x - 1, y, left[k]), rt = point(x + 1, y, right[k]);
+      const Vec3 c    = cross3({dn.x - up.x, dn.y - up.y, dn.z - up.z}, {rt.x - lf.x, rt.y - lf.y, rt.z - lf.z});
+      const float inv = o[k] / fmaxf(sqrtf(c.x * c.x + c.y * c.y + c.z * c.z), 1e-12f);
+      n = {c.x * inv, c.y * inv, c.z * inv};
+    }
+    const size_t p = (size_t) y * W + x;
+    surf_normal[p] = n.x, surf_normal[HW + p] = n.y, surf_normal[2 * HW + p] = n.z;
   }
 }
 
@@ -216,6 +254,14 @@ __global__ void __launch_bounds__(256) epilogue_backward_kernel(int W, int H, in
 }  // namespace fsgs
 
 using namespace fsgs;
+
+FSGS_API int fsgs_gs_2d_view_surf_normal(int W, int H, const float* Tw2v, const float* Tv2c, const float* surf_depth,
+    const float* opacity, float* surf_normal, void* stream) {
+  FSGS_REQUIRE(W > 0 && H > 0 && Tw2v && Tv2c && surf_depth && opacity && surf_normal, "gs_2d_view_surf_normal: bad arguments");
+  hipLaunchKernelGGL(surf_normal_kernel, dim3(div_up(W, 64), div_up(H, 4 * kNormalRows)), dim3(64, 4), 0, (hipStream_t) stream, W,
+                     H, Tw2v, Tv2c, surf_depth, opacity, surf_normal);
+  return check_launch("gs_2d_view_surf_normal");
+}
 
 FSGS_API int fsgs_gs_2d_epilogue_forward(int W, int H, double depth_ratio, const float* Tw2v, const float* Tv2c,
     const float* extras, const float* opacity, const float* images, const float* background, float* normals,

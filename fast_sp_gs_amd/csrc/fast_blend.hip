@@ -20,6 +20,7 @@
 #include "block_lists.hpp"
 #include "instance_slots.hpp"
 #include "ordered_sums.hpp"
+#include "view_maps.hpp"
 
 namespace fsgs {
 namespace {
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
     float2* __restrict__ out_flow, int32_t* __restrict__ max_contrib,
     int32_t* __restrict__ bucket_to_tile, float* __restrict__ sampled_T, float* __restrict__ sampled_acc,
     float* __restrict__ sampled_aux, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
-    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks) {
+    int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks, ViewMaps maps) {
   // With snapshots the lists end at the buckets of 32 entries, two of which are staged at a time.
   constexpr int kLanes = 8, kB = kSnap ? 64 : 128;
   using Shape = BlockShape<kLanes>;
@@ -346,14 +347,17 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
     out_color[pix + HW]     = C1;
     out_color[pix + 2 * HW] = C2;
     if (kAux) {
-      out_extras[pix + 0 * HW] = D;
-      out_extras[pix + 1 * HW] = N0;
-      out_extras[pix + 2 * HW] = N1;
-      out_extras[pix + 3 * HW] = N2;
-      out_extras[pix + 4 * HW] = median;
-      out_extras[pix + 5 * HW] = dist;
-      out_extras[pix + 6 * HW] = M1;
-      out_extras[pix + 7 * HW] = M2;
+      if (!kSnap && maps.normals) maps.write(HW, pix, N0, N1, N2, D, median, dist);
+      if (kSnap || out_extras) {
+        out_extras[pix + 0 * HW] = D;
+        out_extras[pix + 1 * HW] = N0;
+        out_extras[pix + 2 * HW] = N1;
+        out_extras[pix + 3 * HW] = N2;
+        out_extras[pix + 4 * HW] = median;
+        out_extras[pix + 5 * HW] = dist;
+        out_extras[pix + 6 * HW] = M1;
+        out_extras[pix + 7 * HW] = M2;
+      }
       if (kFlow) {
         const float A = 1.0f - T;
         out_flow[pix] = A > 0.0f ? make_float2(f0 / A, f1 / A) : make_float2(0.0f, 0.0f);
@@ -963,12 +967,14 @@ int fast_render_forward(int P, int W, int H, double near_n, double far_n, int on
     int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count, const int64_t* bucket_offset,
     float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib,
     int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_acc, float* sampled_aux,
-    uint32_t* hit_blocks, void* stream) {
+    uint32_t* hit_blocks, const ViewMaps& maps, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_fast_render_forward: bad sizes");
   FSGS_REQUIRE(ranges && out_color && out_opacity && n_contrib, "GS_2D_fast_render_forward: null pointer");
   FSGS_REQUIRE(P == 0 || (means2D && colors && normal_opacity && trans_mat && inverse_m),
                "GS_2D_fast_render_forward: null surfel tensor");
-  FSGS_REQUIRE(only_image || out_extras, "GS_2D_fast_render_forward: out_extras is required unless only_image");
+  FSGS_REQUIRE(only_image || out_extras || (maps.normals && maps.distortion),
+               "GS_2D_fast_render_forward: out_extras is required unless only_image");
+  FSGS_REQUIRE(!maps.normals || (maps.Tw2v && maps.surf_depth), "GS_2D_fast_render_forward: null map");
   const bool aux   = !only_image;
   const bool snap  = aux && bucket_offset != nullptr;
   const bool accum = aux && (accum_max_count || accum_weights_p || accum_weights_count);
@@ -986,7 +992,7 @@ int fast_render_forward(int P, int W, int H, double near_n, double far_n, int on
                      (float) near_n, (float) far_n, ranges, point_list, (const float2*) means2D, colors, trans_mat,  \
                      inverse_m, (const float4*) normal_opacity, trans_mat_t2, bucket_offset, n_contrib, out_color,   \
                      out_opacity, out_extras, (float2*) out_flow, max_contrib, bucket_to_tile, sampled_T,            \
-                     sampled_acc, sampled_aux, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks)
+                     sampled_acc, sampled_aux, accum_max_count, accum_weights_p, accum_weights_count, hit_blocks, maps)
 #define FSGS_LAUNCH_FWD_F(AUX, SNAP, ACC, HITS) \
   do { if (flow) FSGS_LAUNCH_FWD(AUX, SNAP, ACC, true, HITS); else FSGS_LAUNCH_FWD(AUX, SNAP, ACC, false, HITS); } while (0)
   if (!aux) FSGS_LAUNCH_FWD(false, false, false, false, false);
@@ -1012,18 +1018,20 @@ FSGS_API int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, 
   return fast_render_forward(P, W, H, near_n, far_n, only_image, means2D, colors, normal_opacity, trans_mat, inverse_m,
                              point_list, ranges, trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count,
                              bucket_offset, out_color, out_opacity, out_extras, out_flow, n_contrib, max_contrib,
-                             bucket_to_tile, sampled_T, sampled_acc, sampled_aux, nullptr, stream);
+                             bucket_to_tile, sampled_T, sampled_acc, sampled_aux, nullptr, ViewMaps{}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_fast_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* colors, const float* normal_opacity, const float* trans_mat, const float* inverse_m,
     const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
     float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
-    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, void* stream) {
+    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, double depth_ratio, const float* Tw2v, float* normals,
+    float* surf_depth, float* distortion, void* stream) {
   return fast_render_forward(P, W, H, near_n, far_n, 0, means2D, colors, normal_opacity, trans_mat, inverse_m, point_list,
                              ranges, trans_mat_t2, accum_max_count, accum_weights_p, accum_weights_count, nullptr, out_color,
                              out_opacity, out_extras, out_flow, n_contrib, nullptr, nullptr, nullptr, nullptr, nullptr,
-                             hit_blocks, stream);
+                             hit_blocks,
+                             ViewMaps{Tw2v, nullptr, normals, nullptr, surf_depth, distortion, (float) depth_ratio}, stream);
 }
 
 FSGS_API size_t fsgs_gs_2d_fast_render_backward_workspace_bytes(int64_t R) {

@@ -19,7 +19,8 @@ struct Saved : torch::CustomClassHolder {  // what the backward reads besides te
 struct Buffers {
   Tensor radii, visible, ranges, point_list, n_contrib;
   Tensor image, opacity, extras, flow;        // what the blend writes
-  Tensor normals, surf_depth, surf_normal;    // what the epilogue writes
+  Tensor normals, surf_depth, surf_normal;    // the epilogue's maps
+  Tensor distortion;                          // instead of the extras, when nothing is kept for a backward
   Tensor hit_blocks;                          // per list entry, for the backward
   Slab keep;                                  // per-surfel intermediates, read again by the backward
   c10::intrusive_ptr<Saved> saved;
@@ -81,7 +82,9 @@ Buffers forward_view(const FastSurfelView& v, bool train) {
         *normal_opacity = b.keep.at<float>(s.normal_opacity);
   uint32_t* masks = b.keep.at<uint32_t>(s.masks);
   auto blend_maps = [&] {
-    b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.extras = empty({8, H, W}, like);
+    b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like);
+    if (train || !v.epilogue) b.extras = empty({8, H, W}, like);
+    else b.distortion = empty({1, H, W}, like);
     b.n_contrib = empty({2, H, W}, like, at::kInt);
     if (flow) b.flow = empty({H, W, 2}, like);
   };
@@ -118,19 +121,20 @@ Buffers forward_view(const FastSurfelView& v, bool train) {
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream), what);
   }
   if (train) b.hit_blocks = empty({s.R}, like, at::kInt);
+  // the blend writes the maps that need no neighbour, and the extra channels only where a backward will read them
+  if (v.epilogue)
+    b.normals = empty({3, H, W}, like), b.surf_depth = empty({1, H, W}, like), b.surf_normal = empty({3, H, W}, like);
   check(fsgs_gs_2d_fast_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, normal_opacity, trans_mat,
                                      inverse_m, i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
                                      i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
                                      i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
-                                     f32(b.flow), i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), stream),
+                                     f32(b.flow), i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), v.depth_ratio,
+                                     f32(v.Tw2v), f32(b.normals), f32(b.surf_depth), f32(b.distortion), stream),
         blend);
-  if (v.epilogue) {
-    b.normals = empty({3, H, W}, like), b.surf_depth = empty({1, H, W}, like), b.surf_normal = empty({3, H, W}, like);
-    check(fsgs_gs_2d_epilogue_forward(W, H, v.depth_ratio, f32(v.Tw2v), f32(v.Tv2c), f32(b.extras), f32(b.opacity), nullptr,
-                                      nullptr, f32(b.normals), nullptr, f32(b.surf_depth), f32(b.surf_normal), nullptr,
+  if (v.epilogue)
+    check(fsgs_gs_2d_view_surf_normal(W, H, f32(v.Tw2v), f32(v.Tv2c), f32(b.surf_depth), f32(b.opacity), f32(b.surf_normal),
                                       stream),
           "gs_2d_epilogue_forward");
-  }
   return b;
 }
 
@@ -140,8 +144,8 @@ variable_list outputs_of(const Buffers& b) {
   if (!b.saved->epilogue) {
     out = {b.image, b.opacity, b.extras};
   } else {
-    Tensor distortion;
-    {
+    Tensor distortion = b.distortion;
+    if (b.extras.defined()) {
       at::AutoDispatchBelowADInplaceOrView plain;  // shares extras' storage, no view in the graph's sense
       distortion = sharing_edits(b.extras, b.extras.narrow(0, 5, 1));
     }

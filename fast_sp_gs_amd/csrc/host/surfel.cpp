@@ -16,7 +16,8 @@ struct Saved {  // what the backward reads besides tensors
 struct Buffers {
   Tensor trans_mat, normal_opacity, radii, visible, ranges, point_list, n_contrib;
   Tensor image, opacity, extras, flow;                       // what the blend writes
-  Tensor normals, depths, surf_depth, surf_normal, composited;  // what the epilogue writes
+  Tensor normals, depths, surf_depth, surf_normal;  // the epilogue's maps; the image is composited then, given a background
+  Tensor distortion;                                          // instead of the extras, when nothing is kept for a backward
   Tensor hit_blocks;                                          // per list entry, for the backward
   Slab keep;                                                  // what only the backward reads
   Saved saved;
@@ -77,6 +78,12 @@ Buffers forward_view(const SurfelView& v, bool train) {
   const float* colors = v.sh_degree < 0 ? f32(v.shs) : b.keep.at<float>(s.colors);
   uint32_t* masks = v.cull ? b.keep.at<uint32_t>(s.masks) : nullptr;
   float* records  = b.keep.at<float>(s.records);
+  auto blend_maps = [&] {
+    b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.n_contrib = empty({2, H, W}, like, at::kInt);
+    if (train || !v.epilogue) b.extras = empty({9, H, W}, like);
+    else b.distortion = empty({1, H, W}, like);
+    if (flow) b.flow = empty({H, W, 2}, like);
+  };
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
@@ -95,10 +102,7 @@ Buffers forward_view(const SurfelView& v, bool train) {
                              scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
     counters.give_back();
-    // what does not depend on the count is allocated while the device gets there
-    b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.extras = empty({9, H, W}, like);
-    b.n_contrib = empty({2, H, W}, like, at::kInt);
-    if (flow) b.flow = empty({H, W, 2}, like);
+    blend_maps();  // what does not depend on the count is allocated while the device gets there
     check(fsgs_gs_view_wait(count, stream), "GS_prepare");
     s.R = *count;
     b.point_list = empty({s.R}, like, at::kInt);
@@ -112,29 +116,30 @@ Buffers forward_view(const SurfelView& v, bool train) {
                                                fill.data_ptr(), fill_bytes, stream),
           "GS_prepare");
   } else {
-    b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.extras = empty({9, H, W}, like);
-    b.n_contrib = empty({2, H, W}, like, at::kInt);
-    if (flow) b.flow = empty({H, W, 2}, like);
+    blend_maps();
     b.point_list = empty({0}, like, at::kInt);
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
   }
   if (train) b.hit_blocks = empty({s.R}, like, at::kInt);
+  // the blend writes the maps that need no neighbour, and the extra channels only where a backward will read them
+  if (v.epilogue) {
+    b.normals = empty({3, H, W}, like), b.depths = empty({1, H, W}, like), b.surf_depth = empty({1, H, W}, like);
+    b.surf_normal = empty({3, H, W}, like);
+  }
+  const bool composite = v.epilogue && has(v.background);
   check(fsgs_gs_2d_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, f32(b.normal_opacity),
                                   f32(b.trans_mat), i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
                                   i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
                                   i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
-                                  f32(b.flow), i32(b.n_contrib), records, (uint32_t*) i32(b.hit_blocks), stream),
+                                  f32(b.flow), i32(b.n_contrib), records, (uint32_t*) i32(b.hit_blocks), v.depth_ratio,
+                                  f32(v.Tw2v), composite ? f32(*v.background) : nullptr, f32(b.normals), f32(b.depths),
+                                  f32(b.surf_depth), f32(b.distortion), stream),
         blend);
-  if (v.epilogue) {
-    b.normals = empty({3, H, W}, like), b.depths = empty({1, H, W}, like), b.surf_depth = empty({1, H, W}, like);
-    b.surf_normal = empty({3, H, W}, like);
-    if (has(v.background)) b.composited = empty({3, H, W}, like);
-    check(fsgs_gs_2d_epilogue_forward(W, H, v.depth_ratio, f32(v.Tw2v), f32(v.Tv2c), f32(b.extras), f32(b.opacity),
-                                      f32(b.image), f32(opt(v.background)), f32(b.normals), f32(b.depths),
-                                      f32(b.surf_depth), f32(b.surf_normal), f32(b.composited), stream),
+  if (v.epilogue)
+    check(fsgs_gs_2d_view_surf_normal(W, H, f32(v.Tw2v), f32(v.Tv2c), f32(b.surf_depth), f32(b.opacity), f32(b.surf_normal),
+                                      stream),
           "gs_2d_epilogue_forward");
-  }
   return b;
 }
 
@@ -146,12 +151,12 @@ variable_list outputs_of(const Buffers& b) {
     if (b.flow.defined()) out.push_back(b.flow);
     return out;
   }
-  Tensor distortion;
-  {
+  Tensor distortion = b.distortion;
+  if (b.extras.defined()) {
     at::AutoDispatchBelowADInplaceOrView plain;  // shares extras' storage, no view in the graph's sense
     distortion = sharing_edits(b.extras, b.extras.narrow(0, 5, 1));
   }
-  out = {b.composited.defined() ? b.composited : b.image, b.opacity, b.normals, b.depths, b.surf_depth, b.surf_normal,
+  out = {b.image, b.opacity, b.normals, b.depths, b.surf_depth, b.surf_normal,
          distortion};
   if (b.flow.defined()) out.push_back(b.flow);
   return out;

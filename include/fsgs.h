@@ -184,12 +184,19 @@ int fsgs_gs_2d_render_forward(int P, int W, int H, double near_n, double far_n, 
 
 /* The same with all maps, for a view that will be back-propagated: hit_blocks[R] (nullptr: not wanted) receives, per list
  * entry, a bit for every block of 2x4 pixels of its tile with a pixel that blended it; entries behind the last one that any
- * pixel of the tile blended keep what the buffer held. */
+ * pixel of the tile blended keep what the buffer held. With normals[3,H,W] (nullptr: raw maps only) the maps of
+ * fsgs_gs_2d_epilogue_forward that need no neighbour are written as well: normals, depths[H,W] (optional), surf_depth[H,W], and
+ * with background[3] out_color is the composited picture. out_extras may then be nullptr, distortion[H,W] receives its channel 5
+ * (optional beside it). */
 int fsgs_gs_2d_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D, const float* colors,
     const float* normal_opacity, const float* trans_mat, const int32_t* point_list, const int64_t* ranges,
     const float* trans_mat_t2, int32_t* accum_max_count, float* accum_weights_p, int32_t* accum_weights_count,
     float* out_color, float* out_opacity, float* out_extras, float* out_flow, int32_t* n_contrib, const float* records,
-    uint32_t* hit_blocks, void* stream);
+    uint32_t* hit_blocks, double depth_ratio, const float* Tw2v, const float* background, float* normals, float* depths,
+    float* surf_depth, float* distortion, void* stream);
+/* surf_normal[3,H,W] of such a view: the part of fsgs_gs_2d_epilogue_forward that needs a pixel's neighbours. */
+int fsgs_gs_2d_view_surf_normal(int W, int H, const float* Tw2v, const float* Tv2c, const float* surf_depth,
+    const float* opacity, float* surf_normal, void* stream);
 
 /* GS_2D_render_backward -- gs_2d_redner.cu:631-717 (kernel :238-539). Two ways of summing a surfel's gradient over the
  * tiles it touches:
@@ -316,12 +323,13 @@ int fsgs_gs_2d_fast_render_forward(int P, int W, int H, double near_n, double fa
     int32_t* max_contrib, int32_t* bucket_to_tile, float* sampled_T, float* sampled_acc, float* sampled_aux,
     void* stream);
 /* The same with all maps and without snapshots, for a view that will be back-propagated: hit_blocks[R] (nullptr: not wanted) as
- * fsgs_gs_2d_view_forward leaves it. */
+ * fsgs_gs_2d_view_forward leaves it, and normals, surf_depth and distortion as there. */
 int fsgs_gs_2d_fast_view_forward(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* colors, const float* normal_opacity, const float* trans_mat, const float* inverse_m,
     const int32_t* point_list, const int64_t* ranges, const float* trans_mat_t2, int32_t* accum_max_count,
     float* accum_weights_p, int32_t* accum_weights_count, float* out_color, float* out_opacity, float* out_extras,
-    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, void* stream);
+    float* out_flow, int32_t* n_contrib, uint32_t* hit_blocks, double depth_ratio, const float* Tw2v, float* normals,
+    float* surf_depth, float* distortion, void* stream);
 
 /* GS_2D_fast_render_backward -- gs_2d_fast_redner.cu:955-1074. per_splat_form = 0: kernel :273-561 (image, opacity,
  * aux 0-5); per_splat_form = 1: the channel set of kernel :563-837 (image, opacity, aux 0-4 and 6-7, no distortion).
