@@ -266,17 +266,28 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   __shared__ float s_Tw2v[16], s_Tv2c[16];
   __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
-  if (threadIdx.x < 16) s_Tw2v[threadIdx.x] = Tw2v_g[threadIdx.x], s_Tv2c[threadIdx.x] = Tv2c_g[threadIdx.x];
-  __syncthreads();
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
+  // the Gaussian's own values are on their way while the block waits for the camera
+  float p[3] = {0, 0, 0}, own_scale[3] = {0, 0, 0}, opacity = 0.0f;
+  float4 own_rot = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (valid) {
+    p[0] = means3D[3 * (size_t) i], p[1] = means3D[3 * (size_t) i + 1], p[2] = means3D[3 * (size_t) i + 2];
+    if (!cov2D_precomp && !cov3D_precomp) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) own_scale[k] = scales[3 * (size_t) i + k];
+      own_rot = rotations[i];
+    }
+    opacity = opacities[i];
+  }
+  if (threadIdx.x < 16) s_Tw2v[threadIdx.x] = Tw2v_g[threadIdx.x], s_Tv2c[threadIdx.x] = Tv2c_g[threadIdx.x];
+  __syncthreads();
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const float fx = 0.5f * (float) W / tanx, fy = 0.5f * (float) H / tany;
 
   bool ok = false;
-  float p[3] = {0, 0, 0}, c3[6] = {0, 0, 0, 0, 0, 0}, rgb[3] = {0, 0, 0};
+  float c3[6] = {0, 0, 0, 0, 0, 0}, rgb[3] = {0, 0, 0};
   Screen sc = {};
-  if (valid) p[0] = means3D[3 * (size_t) i], p[1] = means3D[3 * (size_t) i + 1], p[2] = means3D[3 * (size_t) i + 2];
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
@@ -295,19 +306,14 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
     Projected pr;
     project(p, Tw2v, Tv2c, pr);
     if (is_opengl ? (pr.proj[2] < -1.0f || pr.proj[2] > 1.0f) : pr.pv[2] <= 0.2f) break;
-    float cov2[3] = {0, 0, 0};
-    if (cov2D_precomp) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) cov2[k] = cov2D_precomp[3 * (size_t) i + k];
-    } else if (cov3D_precomp) {
+    if (cov3D_precomp && !cov2D_precomp) {
 #pragma unroll
       for (int k = 0; k < 6; ++k) c3[k] = cov3D_precomp[6 * (size_t) i + k];
-    } else {
-      const float s[3] = {scales[3 * (size_t) i], scales[3 * (size_t) i + 1], scales[3 * (size_t) i + 2]};
-      cov3d_forward(s, rotations[i], c3);  // kept even when a later test rejects the Gaussian, as in the reference
+    } else if (!cov2D_precomp) {
+      cov3d_forward(own_scale, own_rot, c3);  // kept even when a later test rejects the Gaussian, as in the reference
     }
-    ok = screen_geometry(W, H, gx, gy, is_opengl != 0, p, pr, c3, cov2D_precomp ? cov2 : nullptr, fx, fy, tanx, tany,
-                         Tw2v, sc);
+    ok = screen_geometry(W, H, gx, gy, is_opengl != 0, p, pr, c3,
+                         cov2D_precomp ? cov2D_precomp + 3 * (size_t) i : nullptr, fx, fy, tanx, tany, Tw2v, sc);
   } while (false);
 
   if (view.counters) {  // how many instances the view has
@@ -338,11 +344,26 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
       rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
     }
   }
+  // cov3Ds is absent with a pre-computed 3D covariance: the caller hands that tensor on as the operator's output
+  // rows of 24 and 12 bytes leave through LDS (wave_rows_out); with the early requests above 300k Gaussians 32 -> 30 us
+  const bool rows = kWave && (((uintptr_t) cov3Ds | (uintptr_t) colors) & 15) == 0;
+  if (rows) {
+    const int lane = threadIdx.x & 63;
+    float *s_cov = s_wave_rows, *s_rgb = s_cov + 384;
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s_cov[6 * lane + k] = c3[k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s_rgb[3 * lane + k] = rgb[k];
+    wave_lds_sync();
+    if (cov3Ds) wave_rows_out<6>(s_cov, wave_base, P, cov3Ds);
+    wave_rows_out<3>(s_rgb, wave_base, P, colors);
+  }
   if (!valid) return;
-  if (cov3Ds)  // absent with a pre-computed 3D covariance: the caller hands that tensor on as the operator's output
+  if (!rows && cov3Ds)
 #pragma unroll
     for (int k = 0; k < 6; ++k) cov3Ds[6 * (size_t) i + k] = c3[k];
-  if (sh_degree >= 0) {
+  if (!rows && sh_degree >= 0) {
     colors[3 * (size_t) i] = rgb[0], colors[3 * (size_t) i + 1] = rgb[1], colors[3 * (size_t) i + 2] = rgb[2];
   }
   depths[i]        = ok ? sc.depth : 0.0f;
@@ -350,7 +371,6 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   if (tiles_touched) tiles_touched[i] = ok ? sc.area : 0;
   if (view.visible) view.visible[i] = ok && f2i_sat(sc.radius) > 0;
   if (ok || !means2D_preserve) means2D[i] = ok ? make_float2(sc.px, sc.py) : make_float2(0.0f, 0.0f);
-  const float opacity = opacities[i];
   conic_opacity[i] = ok ? make_float4(sc.conic[0], sc.conic[1], sc.conic[2], opacity) : make_float4(0, 0, 0, 0);
   if (keep_masks) {
     // which tiles of the rectangle some pixel of which can blend the Gaussian (as conic_cull_mask_kernel finds it), here

@@ -102,9 +102,18 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   __shared__ unsigned char s_flag[kShStageRows];
   __shared__ int s_wave_slots[4];
   __shared__ int s_block_slot;
-  load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
+  // the surfel's own values are on their way while the block waits for the camera
+  float p[3] = {0, 0, 0}, opac = 0.0f;
+  float2 own_scale = make_float2(0.0f, 0.0f);
+  float4 own_rot = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (valid) {
+    p[0] = means3D[3 * (size_t) i], p[1] = means3D[3 * (size_t) i + 1], p[2] = means3D[3 * (size_t) i + 2];
+    if (trans_precomp == nullptr) own_scale = scales[i], own_rot = rotations[i];
+    opac = opacities[i];
+  }
+  load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
 
   bool ok = false;
@@ -112,8 +121,6 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   int area = 0;
 #pragma unroll
   for (int k = 0; k < 9; ++k) M[k] = 0.0f;
-  float p[3] = {0, 0, 0};
-  if (valid) p[0] = means3D[3 * (size_t) i], p[1] = means3D[3 * (size_t) i + 1], p[2] = means3D[3 * (size_t) i + 2];
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
@@ -137,8 +144,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
                          Tw2v[8] * p[0] + Tw2v[9] * p[1] + Tw2v[10] * p[2] + Tw2v[11]};
     if (pv[2] <= 0.2f) break;
     if (trans_precomp == nullptr) {
-      const float2 s = scales[i];
-      transmat(W, H, p, s.x, s.y, rotations[i], Tw2c, Tw2v, M, nrm);
+      transmat(W, H, p, own_scale.x, own_scale.y, own_rot, Tw2c, Tw2v, M, nrm);
     } else {
 #pragma unroll
       for (int k = 0; k < 9; ++k) M[k] = trans_precomp[9 * (size_t) i + k];
@@ -194,34 +200,60 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     __syncthreads();
     slot += s_block_slot;
   }
+  if (sh_degree < 0 && valid) rgb[0] = shs[3 * (size_t) i], rgb[1] = shs[3 * (size_t) i + 1], rgb[2] = shs[3 * (size_t) i + 2];
+  const float op = opac;
+  // The rows of 80, 36 and 12 bytes leave through LDS (wave_rows_out): 3M surfels 279 -> 235 us, 300k 39 -> 33, with the
+  // positions and shapes requested before the block waits for the camera.
+  const bool rows = kWave && (((uintptr_t) trans_mat | (uintptr_t) colors) & 15) == 0;
+  if (rows) {
+    const int lane = threadIdx.x & 63;
+    if (records) {
+      float4* r = (float4*) s_wave_rows;
+      wave_lds_sync();
+      r[5 * lane]     = ok ? make_float4(M[0], M[1], M[2], M[3]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      r[5 * lane + 1] = ok ? make_float4(M[4], M[5], M[6], M[7]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      r[5 * lane + 2] = ok ? make_float4(M[8], c2[0], c2[1], op) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      r[5 * lane + 3] = ok ? make_float4(nrm[0], nrm[1], nrm[2], rgb[0]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      r[5 * lane + 4] = ok ? make_float4(rgb[1], rgb[2], __int_as_float(f2i_sat(radius)), __int_as_float(view.slot_offsets ? slot : -1))
+                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      wave_lds_sync();
+      wave_rows_out<20>(s_wave_rows, wave_base, P, (float*) records);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 9; ++k) s_wave_rows[9 * lane + k] = ok ? M[k] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s_wave_rows[576 + 3 * lane + k] = rgb[k];
+    wave_lds_sync();
+    if (trans_precomp == nullptr) wave_rows_out<9>(s_wave_rows, wave_base, P, trans_mat);
+    wave_rows_out<3>(s_wave_rows + 576, wave_base, P, colors);
+  }
   if (!valid) return;
 
   if (view.slot_offsets) view.slot_offsets[i] = slot;
   if (view.visible) view.visible[i] = ok && f2i_sat(radius) > 0;
-  if (trans_precomp == nullptr) {
+  if (!rows && trans_precomp == nullptr) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) trans_mat[9 * (size_t) i + k] = ok ? M[k] : 0.0f;
   }
-  if (sh_degree >= 0) {
+  if (!rows && sh_degree >= 0) {
     colors[3 * (size_t) i] = rgb[0], colors[3 * (size_t) i + 1] = rgb[1], colors[3 * (size_t) i + 2] = rgb[2];
   }
   depths[i]        = depth;
   radii[i]         = ok ? f2i_sat(radius) : 0;
   tiles_touched[i] = ok ? area : 0;
   if (ok || !means2D_preserve) means2D[i] = ok ? make_float2(c2[0], c2[1]) : make_float2(0.0f, 0.0f);
-  normal_opacity[i] = ok ? make_float4(nrm[0], nrm[1], nrm[2], opacities[i]) : make_float4(0, 0, 0, 0);
-  if (records) {
+  normal_opacity[i] = ok ? make_float4(nrm[0], nrm[1], nrm[2], op) : make_float4(0, 0, 0, 0);
+  if (records && !rows) {
     // The blend kernels' 80-byte record (layout of pack_records_kernel), written here while every field is in
     // registers. Surfels that are not rendered never enter a tile list; their records are zeros.
-    const float* col = sh_degree >= 0 ? rgb : shs + 3 * (size_t) i;
-    const float op   = opacities[i];
-    float4* r        = records + 5 * (size_t) i;
+    float4* r = records + 5 * (size_t) i;
     if (ok) {
       r[0] = make_float4(M[0], M[1], M[2], M[3]);
       r[1] = make_float4(M[4], M[5], M[6], M[7]);
       r[2] = make_float4(M[8], c2[0], c2[1], op);
-      r[3] = make_float4(nrm[0], nrm[1], nrm[2], col[0]);
-      r[4] = make_float4(col[1], col[2], __int_as_float(f2i_sat(radius)), __int_as_float(view.slot_offsets ? slot : -1));  // -1: not known yet
+      r[3] = make_float4(nrm[0], nrm[1], nrm[2], rgb[0]);
+      r[4] = make_float4(rgb[1], rgb[2], __int_as_float(f2i_sat(radius)), __int_as_float(view.slot_offsets ? slot : -1));  // -1: not known yet
     } else {
 #pragma unroll
       for (int k = 0; k < 5; ++k) r[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -237,7 +269,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       const TileRect r = tile_rect(c2[0], c2[1], f2i_sat(radius), gx, gy);
       const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
       if (w * h <= kCullMaskTiles) {
-        const CullBounds cb = cull_bounds(M, c2[0], c2[1], opacities[i]);
+        const CullBounds cb = cull_bounds(M, c2[0], c2[1], op);
         m = 0u;
         int e = 0;
         for (int y = 0; y < h; ++y)

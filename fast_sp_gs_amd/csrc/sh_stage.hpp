@@ -176,6 +176,19 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Writes a wavefront's rows of kFloats floats from LDS, where they lie without gaps as they will in memory, to dst (on a 16-byte
+// boundary; a wavefront's rows then start on one, too). With its own stores a lane touches lines that it shares with its
+// neighbours' stores of the same kind, an instruction as many lines as its 64 rows cover, for each of its pieces.
+template <int kFloats>
+__device__ __forceinline__ void wave_rows_out(const float* __restrict__ s_rows, int wave_base, int P, float* __restrict__ dst) {
+  const int all = max(min(64, P - wave_base), 0) * kFloats, whole = all >> 2, lane = (int) __lane_id();
+  float* row = dst + (size_t) wave_base * kFloats;
+#pragma unroll
+  for (int k = 0; k < (16 * kFloats + 63) / 64; ++k)
+    if (k * 64 + lane < whole) ((ShPiece*) row)[k * 64 + lane] = ((const ShPiece*) s_rows)[k * 64 + lane];
+  if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = s_rows[4 * whole + lane];
+}
+
 // Which rows of a preprocess kernel move this way: 48 (one tensor), 45 (the first coefficient apart) or 0 (every other
 // degree, number of coefficients or alignment: stage_sh_rows, or the lane's own walk). The gradients' tensors, where there
 // are any, have to be aligned like the coefficients'.

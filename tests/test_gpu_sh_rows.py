@@ -86,3 +86,36 @@ def test_renders(P, path, split, device):
 
     for a, b in zip(both(torch.clone), both(off_boundary)):
         close(a, b, (P, path, split))
+
+
+@pytest.mark.parametrize('P', SIZES)
+@pytest.mark.parametrize('path', ['surfel', 'fast', 'gauss'])
+@pytest.mark.parametrize('split', [False, True])
+def test_preprocess_rows(P, path, split, device):
+    """Every output row of the preprocess operators, those that leave a wavefront together and those that a lane stores itself,
+    and, as the outputs are allocated uninitialised, the rows of what is not rendered."""
+    from fast_sp_gs_amd import scenes
+    from fast_sp_gs_amd._C import get_C_function
+    print(f'[preprocess rows] {path} P={P} split={split}', flush=True)
+    g = torch.Generator(device=device).manual_seed(P)
+    normal = lambda *s: torch.randn(*s, generator=g, device=device)
+    cam = scenes.pinhole(100, 75, 50.0, torch.tensor([0.0, 0.0, 2.0])).to(device)
+    shape = [normal(P, 3) * 1.5, torch.exp(normal(P, 3 if path == 'gauss' else 2) * 0.5 - 3.0),
+             torch.nn.functional.normalize(normal(P, 4), dim=-1), torch.sigmoid(normal(P, 1))]
+    sh = normal(P, 16, 3) * 0.3
+
+    def outputs(move):
+        rows = [sh[:, :1].contiguous(), move(sh[:, 1:].contiguous())] if split else [move(sh), None]
+        view = [cam.Tw2v, cam.Tv2c]
+        if path == 'surfel':
+            return get_C_function('gs_2d_preprocess_forward')(100, 75, 3, False, *shape, *rows, *view, cam.campos,
+                                                              return_records=True, return_masks=True)
+        if path == 'fast':
+            return get_C_function('gs_2d_fast_preprocess_forward')(100, 75, 3, False, *shape, *rows, *view, cam.Tv2s, cam.campos)
+        return get_C_function('gs_preprocess_forward')(100, 75, 3, False, *shape, *rows, *view, cam.campos, (0.5, 0.4))
+
+    for k, (a, b) in enumerate(zip(outputs(torch.clone), outputs(off_boundary))):
+        if path == 'surfel' and k == 7:  # the records: 18 numbers, then the radius and the first slot as integers
+            close(a[:, 18:].contiguous().view(torch.int32), b[:, 18:].contiguous().view(torch.int32), (path, k))
+            a, b = a[:, :18], b[:, :18]
+        close(a, b, (path, k))
