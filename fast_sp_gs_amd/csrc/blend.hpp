@@ -316,7 +316,7 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
     const int k       = atomicAdd(&s_count[r][length_bucket(len)], 1);
     if (k < kBalanceRounds * kCusPerXcd) {
       s_tile[r][k] = t;
-      s_len[r][k]  = (int) (len > 0x7fffffff ? 0x7fffffff : len);
+      s_len[r][k]  = (int) min(len, (int64_t) (1 << 25) - 1);
     } else {
       tile_order[position(r, k)] = t;
     }
@@ -328,7 +328,7 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
   {
     const int lane = threadIdx.x & 63, r = threadIdx.x >> 6;
     if (r < kOrderRegions && lane < kCusPerXcd) {
-      unsigned long long key = (unsigned long long) lane;  // (load << 8) | cu
+      unsigned key = (unsigned) lane;  // (load << 5) | cu, loads up to 2^27 - 1: four lists of 2^25 - 1 at most
       const int n = s_total[r];
       for (int j = 0; j < kBalanceRounds && j * kCusPerXcd < n; ++j) {
         const int k = j * kCusPerXcd + lane;
@@ -336,17 +336,18 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
           if (k < n) tile_order[position(r, k)] = s_tile[r][k];
           break;
         }
+        if (j > 0)  // every load is zero before the first round
 #pragma unroll
-        for (int size = 2; size <= kCusPerXcd; size <<= 1)
+          for (int size = 2; size <= kCusPerXcd; size <<= 1)
 #pragma unroll
-          for (int d = size >> 1; d > 0; d >>= 1) {
-            const unsigned long long other = __shfl_xor(key, d, kCusPerXcd);
-            const bool up = (lane & size) == 0, low = (lane & d) == 0;
-            key = (low == up) ? (key < other ? key : other) : (key < other ? other : key);
-          }
-        const int cu = (int) (key & 0xffull);
+            for (int d = size >> 1; d > 0; d >>= 1) {
+              const unsigned other = (unsigned) __shfl_xor((int) key, d, kCusPerXcd);
+              const bool up = (lane & size) == 0, low = (lane & d) == 0;
+              key = (low == up) ? min(key, other) : max(key, other);
+            }
+        const int cu = (int) (key & (kCusPerXcd - 1));
         tile_order[position(r, j * kCusPerXcd + cu)] = s_tile[r][k];
-        key += (unsigned long long) (unsigned) s_len[r][k] << 8;
+        key += (unsigned) s_len[r][k] << 5;
       }
     }
   }
