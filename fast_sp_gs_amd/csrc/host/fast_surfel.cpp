@@ -192,8 +192,8 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
     if (s.epilogue) {
       if (g.size() > 6) g_flow = g[6];
       if (g[2].defined() || g[3].defined() || g[4].defined() || g[5].defined()) {
-        g_extras = empty({8, H, W}, points);
-        check(fsgs_gs_2d_view_epilogue_backward(W, H, 8, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
+        g_extras = empty({6, H, W}, points);  // the channels that the blend has a gradient for
+        check(fsgs_gs_2d_view_epilogue_backward(W, H, 6, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
                                                 nullptr, f32(g[2]), nullptr, f32(g[3]), f32(g[4]), f32(g[5]), nullptr,
                                                 nullptr, f32(g_extras), nullptr, stream),
               "gs_2d_epilogue_backward");

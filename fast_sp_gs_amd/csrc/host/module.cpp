@@ -90,7 +90,6 @@ PYBIND11_MODULE(_host, m) {
   m.def("deform_apply", &deform_apply, released);
   m.def("mlp_pack", &mlp_pack, released);
   m.def("image_loss", &image_loss, released);
-  m.def("adam_masked", &adam_masked, released);
   m.def("adam_masked_step", &adam_masked_step, released);
   m.def("adam_dense", &adam_dense, released);
 }

@@ -210,9 +210,9 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
       const bool composite = background.defined() && g_image.defined();
       if (composite || g_normals.defined() || g_depths.defined() || g_surf_depth.defined() || g_surf_normal.defined() ||
           g_dist.defined()) {
-        g_extras = empty({9, H, W}, points);
+        g_extras = empty({6, H, W}, points);  // the channels that the blend has a gradient for
         Tensor g_total = composite || !g_opacity.defined() ? empty({H, W}, points) : Tensor();
-        check(fsgs_gs_2d_view_epilogue_backward(W, H, 9, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
+        check(fsgs_gs_2d_view_epilogue_backward(W, H, 6, s.depth_ratio, f32(Tw2v), f32(Tv2c), f32(extras), f32(opacity),
                                                 f32(background), f32(g_normals), f32(g_depths), f32(g_surf_depth),
                                                 f32(g_surf_normal), f32(g_dist), composite ? f32(g_image) : nullptr,
                                                 f32(g_opacity), f32(g_extras), f32(g_total), stream),
