@@ -541,7 +541,7 @@ __global__ void __launch_bounds__(kBlendThreads)
   if (inside) {
     dLp0 = dL_dpix[pix], dLp1 = dL_dpix[pix + HW], dLp2 = dL_dpix[pix + 2 * HW];
     if (kAux) {
-      dL_daccum  = dL_dopacity[pix];
+      dL_daccum  = dL_dopacity ? dL_dopacity[pix] : 0.0f;
       dL_ddepth  = dL_dextras[pix + 0 * HW];
       dLn0       = dL_dextras[pix + 1 * HW];
       dLn1       = dL_dextras[pix + 2 * HW];
@@ -552,7 +552,7 @@ __global__ void __launch_bounds__(kBlendThreads)
       final_D  = out_extras[pix + 6 * HW];
       final_D2 = out_extras[pix + 7 * HW];
     } else if (kPerSplat) {
-      dL_daccum = dL_dopacity[pix];
+      dL_daccum = dL_dopacity ? dL_dopacity[pix] : 0.0f;
     }
     if (kFlow) {
       const float2 gf = dL_dflow[pix];
@@ -1049,7 +1049,7 @@ int fast_render_backward(int P, int W, int H, double near_n, double far_n, int p
     const uint32_t* keep_masks, const uint32_t* hit_blocks, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "GS_2D_fast_render_backward: bad sizes");
   if (P == 0) return kOk;
-  FSGS_REQUIRE(means2D && normal_opacity && colors && trans_mat && inverse_m && out_opacity && dL_dpix && dL_dopacity &&
+  FSGS_REQUIRE(means2D && normal_opacity && colors && trans_mat && inverse_m && out_opacity && dL_dpix && (dL_dopacity || hit_blocks) &&
                    ranges && n_contrib && g_colors && g_means2D && g_trans && g_inv && g_normal_opacity,
                "GS_2D_fast_render_backward: null pointer");
   const bool aux  = out_extras && dL_dextras;

@@ -204,7 +204,7 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
     }
     if (!g_extras.defined()) g_flow = Tensor();
     if (!g_image.defined()) g_image = at::zeros({3, H, W}, points.options());
-    if (!g_opacity.defined()) g_opacity = at::zeros({H, W}, points.options());
+    if (!g_opacity.defined() && s.R == 0) g_opacity = at::zeros({H, W}, points.options());  // without notes it has to be there
 
     const bool want_sh = ctx->needs_input_grad(4), has_rest = sh_rest.defined(), rest_used = has_rest && sh_rest.numel() > 0;
     Tensor g_means2D = empty({P, 2}, points);

@@ -363,7 +363,8 @@ int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far
     float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
     const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
     size_t workspace_bytes, const uint32_t* keep_masks, void* stream);
-/* The same with the hit_blocks that fsgs_gs_2d_fast_view_forward left for these lists (nullptr: footprints are bounded again). */
+/* The same with the hit_blocks that fsgs_gs_2d_fast_view_forward left for these lists (nullptr: footprints are bounded again). With
+ * them dL_dopacity may be nullptr: no gradient. */
 int fsgs_gs_2d_fast_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
     const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,

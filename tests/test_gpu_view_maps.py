@@ -51,3 +51,34 @@ def test_view_maps_equal_the_epilogue(kind, ratio, background, W, H, device):
             # of their differences, two pixels (a pixel is 2 tan(22.5 deg) 3.5 / W) at least
             turn = 16 * 2.0 ** -23 * 4 / (2 * 2 * 0.414 * 3.5 / W)
             assert float((a - b).abs().max()) <= turn, (k, float((a - b).abs().max()), turn)
+
+
+@pytest.mark.parametrize('visible', [True, False])
+@pytest.mark.parametrize('kind,maps', [('surfel', ('images',)), ('surfel', ('images', 'normals')), ('fast', ('images',)),
+                                       ('fast', ('images', 'distortion'))])
+def test_absent_opacity_gradient_is_a_zero_one(kind, maps, visible, device):
+    """A loss that does not use the opacity map gives the gradients of one that uses it times zero, bit for bit (the sums are
+    records, added in a fixed order), also for a view that sees nothing."""
+    from fast_sp_gs_amd import scenes
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    from fast_sp_gs_amd.renderer.gs_2d_fast_render import GS_2D_fast_render
+    print(f'[view maps] {kind} {maps} visible={visible}', flush=True)
+    scene, cam = scenes.config0(P=3000, size=100, seed=3)
+    scene, cam = scene.to(device), cam.to(device)
+    centres = scene.means3D if visible else scene.means3D - 100.0 * cam.Tw2v[2, :3]
+    params = [t.clone().requires_grad_(True) for t in (centres, scene.scales, scene.rotations, scene.opacities, scene.shs)]
+    g = torch.Generator(device=device).manual_seed(1)
+    up = {k: torch.randn(n, 100, 100, generator=g, device=device) for k, n in (('images', 3), ('normals', 3), ('distortion', 1))}
+
+    def grads(with_opacity):
+        render, view = (GS_2D_render, (cam.Tw2v, cam.Tv2c)) if kind == 'surfel' else \
+            (GS_2D_fast_render, (cam.Tw2v, cam.Tv2c, cam.Tv2s))
+        out = render(*params[:4], (100, 100), *view, campos=cam.campos, sh_degree=3, sh_features=params[4])
+        assert bool(out['visibility_filter'].any()) == visible
+        used = [out[k] for k in maps] + ([out['opacity']] if with_opacity else [])
+        return torch.autograd.grad(used, params, [up[k] for k in maps] +
+                                   ([torch.zeros_like(out['opacity'])] if with_opacity else []))
+
+    for a, b in zip(grads(False), grads(True)):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+        assert bool(a.any()) == visible
