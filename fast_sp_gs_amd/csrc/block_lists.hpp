@@ -151,8 +151,8 @@ __device__ __forceinline__ unsigned conic_blocks(float x, float y, float a, floa
 // Fills the lists of one wavefront from the masks of the batch's staged entries (lane l holds those of entries
 // l, 64 + l, ...; zero past the last one): list g at
 // lists + g * kEntries, a byte per entry, padded with `kEntries` -- the number of a record that no pixel blends -- to its
-// full length. Blocks without a lane in `lanes` get an empty list. Returns the longest list's length. The LDS serves a
-// wavefront's accesses in order, so no barrier is needed before the lists are read.
+// full length. Blocks without a lane in `lanes` get an empty list. Returns the longest list's length. One wavefront writes and
+// reads its lists: wave_lds_sync() orders its lanes, no barrier is needed.
 template <int kLanes, int kEntries>
 __device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lists, const unsigned (&masks)[kEntries / kWave], int wave,
                                                  unsigned long long lanes) {
@@ -163,6 +163,7 @@ __device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lis
   uint2* fill = (uint2*) lists;
 #pragma unroll
   for (int e = 0; e < kPerWave * kEntries / 8; e += kWave) fill[e + lane] = make_uint2(kFill, kFill);
+  wave_lds_sync();
   unsigned m[kEntries / kWave];
 #pragma unroll
   for (int c = 0; c < kEntries / kWave; ++c) m[c] = masks[c] >> (kPerWave * wave);
@@ -181,6 +182,7 @@ __device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lis
     }
     longest = max(longest, n);
   }
+  wave_lds_sync();
   return longest;
 }
 
@@ -276,6 +278,7 @@ __device__ __forceinline__ int build_row_lists(unsigned char* __restrict__ lists
   const int lane = __lane_id();
   constexpr unsigned kFill = 0x01010101u * (unsigned) kRowBatch;
   ((uint2*) lists)[lane] = make_uint2(kFill, kFill);
+  wave_lds_sync();
   const unsigned m[2] = {masks[0] >> (4 * wave), masks[1] >> (4 * wave)};
   int longest = 0;
 #pragma unroll
@@ -294,6 +297,7 @@ __device__ __forceinline__ int build_row_lists(unsigned char* __restrict__ lists
     start += count;
     longest = max(longest, count);
   }
+  wave_lds_sync();
   return longest;
 }
 

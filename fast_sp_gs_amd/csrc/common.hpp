@@ -53,6 +53,14 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wavefront's LDS writes before its later LDS reads and writes of what other lanes wrote (no instruction is generated: a
+// wavefront's LDS operations complete in order; this only stops the compiler from moving them across).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Mask of the lanes where `b` holds, straight from the comparison's lane mask: HIP's __ballot takes an int, which makes
 // the compiler materialise the predicate in a register and compare it again.
 __device__ __forceinline__ unsigned long long wave_ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }

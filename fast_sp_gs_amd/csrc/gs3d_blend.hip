@@ -610,6 +610,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
       for (int c = 0; c < kHalf; ++c) s_total[e][h * (kSums / 2) + c] = a[c];
     }
     if (kSlots) __syncthreads();
+    else wave_lds_sync();  // the two lanes of an entry write what the sixteen below read
     if (kSlots && (int) threadIdx.x < n_here) {
       float sums[kSums], a[16];
 #pragma unroll

@@ -3,7 +3,7 @@
 // lines per wavefront alive between touches; moving the block's rows with consecutive lanes on consecutive addresses
 // reads (writes) every line once. Used when the active degree is <= 3 (at most 16 coefficients, 48 floats per row).
 #pragma once
-#include <hip/hip_runtime.h>
+#include "common.hpp"
 
 namespace fsgs {
 
@@ -167,14 +167,6 @@ struct ShWaveRows {
     if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = 0.0f;
   }
 };
-
-// Orders a wavefront's LDS writes before its later LDS reads of other lanes' data (no instruction is generated: a
-// wavefront's LDS operations complete in order; this only stops the compiler from moving them across).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Writes a wavefront's rows of kFloats floats from LDS, where they lie without gaps as they will in memory, to dst (on a 16-byte
 // boundary; a wavefront's rows then start on one, too). With its own stores a lane touches lines that it shares with its
