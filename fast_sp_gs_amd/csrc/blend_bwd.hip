@@ -10,6 +10,11 @@
 // over its pixels with DPP row shifts; per staged batch the sums of a tile's 16 rows are added in row order, and every staged
 // (surfel, tile) instance writes one record at its position in surfel order; slot_reduce_kernel or the preprocess backward
 // sums a surfel's records in a fixed order. (Without scan offsets: one global atomic per surfel, component and tile.)
+// With flow the step is 50 instructions longer. Its channels, and the sum of weights that it is divided by, ride on the recurrence
+// that the image's share, its three quotients take one reciprocal, and the second transforms are loaded when a batch is staged:
+// in 128 registers, four wavefronts per SIMD instead of three. Backward with flow, 300k surfels 800x800: 485 -> 340 us; 5000 surfels
+// over about 4x4 tiles each, 800x800: 784 -> 627; 2000 over about 10x10: 1468 -> 1149 (with a work list per 8x8 quadrant they
+// took 530, 715 and 1280).
 // Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
 // the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
 // 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260
@@ -28,7 +33,6 @@ namespace {
 // The first 16 go through one transposed row reduction; the means2D pair is only non-zero for pixels where the
 // screen-space low-pass filter wins (rho2d < rho3d) and is reduced separately when any lane took that branch.
 constexpr int kGradSlots = 18;
-constexpr int kRowPlaces = 255;  // of a batch: with 36.5 KB of LDS four blocks share a compute unit
 #ifndef FSGS_BWD_WAVES
 #define FSGS_BWD_WAVES 4
 #endif
@@ -50,6 +54,7 @@ blend_backward_kernel(
     if (slots.region) return (stored >= 0 ? stored : (int64_t) slots.offset[id]) + slots.region[slot_region(id)];
     return stored >= 0 ? stored : (id == 0 ? 0 : slots.scan[id - 1]);
   };
+  constexpr int kRowPlaces = kFlow ? 248 : 255;  // of a batch: with 36.5 KB (flow: 40 KB) of LDS four blocks share a compute unit
   using Shape = BlockShape<16>;
   __shared__ Splat s_splat[kRowBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kRowBatch * 9 : 1];
@@ -138,21 +143,18 @@ blend_backward_kernel(
   // The distortion term's per-pixel constants, folded once: with m the normalised depth of a pair,
   //   dL/dweight = (D2 + m^2 A - 2 m D) dL/dreg = D2 dL/dreg + m (m reg_A - reg_2D),
   //   dL/dm      = 2 w (m A - D) dL/dreg        = w (m reg_2A - reg_2D).
-  const float reg_A = (1.0f - T_final) * dL_dreg, reg_2A = 2.0f * reg_A, reg_2D = 2.0f * final_D * dL_dreg,
-              lin_const = final_D2 * dL_dreg + dL_daccum;  // dL/dweight's constant and the opacity map's gradient
-  float dLf0 = 0, dLf1 = 0, dL_dsum_w = 0;
+  const float reg_A = (1.0f - T_final) * dL_dreg, reg_2A = 2.0f * reg_A, reg_2D = 2.0f * final_D * dL_dreg;
+  float lin_const = final_D2 * dL_dreg + dL_daccum;  // dL/dweight's constant and the opacity map's gradient
+  float dLf0 = 0, dLf1 = 0;
   if (kFlow && inside) {
     const float2 g = dL_dflow[pix], o = out_flow[pix];
-    dL_dsum_w = -(g.x * o.x + g.y * o.y) / (sum_w * sum_w);
     dLf0 = g.x / sum_w, dLf1 = g.y / sum_w;
+    lin_const -= (g.x * o.x + g.y * o.y) / (sum_w * sum_w);  // the sum of weights is a channel whose value is 1
   }
 
   float acc_lin = 0;
-  float last_alpha = 0, acc_w = 0;
-  float acc_f0 = 0, acc_f1 = 0, last_f0 = 0, last_f1 = 0;
 
   Splat next;
-  float next_t2[9];
   int next_radius = 0;
   unsigned next_hits = 0u;
   int64_t next_off = 0;
@@ -163,9 +165,6 @@ blend_backward_kernel(
     SplatExtra ex;
     if (hit_blocks) next_hits = hit_blocks[r0 + (n_todo - 1 - done - e)];
     next = gather_splat(point_list[r0 + (n_todo - 1 - done - e)], means2D, colors, normal_opacity, trans_mat, records, &ex);
-    if (kFlow)
-#pragma unroll
-      for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
     if (kSlots) {
       // a record carries the surfel's radius (-1 if it was packed without radii) and, once the binning's scan has
       // stored it, its offset (-1 until then)
@@ -183,9 +182,9 @@ blend_backward_kernel(
       if (e < n_staged) {
         s_splat[e] = next;
         mask = hit_blocks ? pair_blocks(next_hits) : surfel_blocks<16>(next.hot, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
-        if (kFlow)
+        if (kFlow)  // not requested ahead: nine registers more would be spilled, and the spill would wait for them
 #pragma unroll
-          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
         if (kSlots) {
           // position of this instance in the surfel-ordered key list: the binning emits a surfel's tiles row-major
           // over its rectangle, starting at the surfel's prefix-scan offset (gaussian_prepare.cu:47-83)
@@ -210,12 +209,13 @@ blend_backward_kernel(
                                       before, n_here);
     const int my_first = behind - last_contrib, my_median = behind - median_contrib;
     // ---- order-bound part of one (pixel, entry) pair: advances the pixel's back-to-front state -------------------------
-    // All channels that enter the image linearly (colour, depth, opacity, normal) share one recurrence: with
+    // All channels that enter the image linearly (colour, depth, opacity, normal, flow) share one recurrence: with
     // c = <upstream gradient, channel values of this surfel>, the reference's per-channel accumulators
     // acc_x = last_alpha * last_x + (1 - last_alpha) * acc_x contract to a single scalar, updated at the end of the
-    // pair that supplies alpha and x. Leaves the blend weight w, dL/dalpha and dL/ddepth of the pair; call under `hit`
-    // only.
-    auto advance_pixel = [&](const SplatCold& cold, int j, const Hit& h, float& w, float& dL_dalpha, float& dL_dz) {
+    // pair that supplies alpha and x. Leaves the blend weight w, dL/dalpha and dL/ddepth of the pair, and the flow's part of
+    // dL/d(intersection); call under `hit` only.
+    auto advance_pixel = [&](const SplatCold& cold, int j, const Hit& h, float& w, float& dL_dalpha, float& dL_dz, float& fsx,
+                             float& fsy) {
       const float keep = 1.0f - h.alpha;
       T = T * __builtin_amdgcn_rcpf(keep);
       w = h.alpha * T;
@@ -237,6 +237,21 @@ blend_backward_kernel(
         c_lin = 0.0f;
       }
       c_lin = fmaf(cold.r, dLp0, fmaf(cold.g, dLp1, fmaf(cold.b, dLp2, c_lin)));
+      if (kFlow) {
+        const float* Q = &s_t2[j * 9];
+        const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
+        const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
+        float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
+        w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
+        float rw = __builtin_amdgcn_rcpf(w2);
+        rw = fmaf(fmaf(-w2, rw, 1.0f), rw, rw);  // a Newton step: as good as a division
+        // flow u2 / w2 - x as (u2 - x w2) / w2: one rounding in the difference of two nearly equal numbers
+        const float fu = fmaf(-pxf, w2, u2) * rw, fv = fmaf(-pyf, w2, v2) * rw;
+        c_lin = fmaf(fu, dLf0, fmaf(fv, dLf1, c_lin));
+        const float wr = w * rw, gu = wr * dLf0, gv = wr * dLf1, gw = -wr * fmaf(fu + pxf, dLf0, (fv + pyf) * dLf1);
+        fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
+        fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
+      }
       // acc_lin: what the pairs behind this one accumulated, alpha_j c_j weighted by the transmittance between
       dL_dalpha = c_lin - acc_lin;
       acc_lin   = fmaf(keep, acc_lin, h.alpha * c_lin);
@@ -250,27 +265,10 @@ blend_backward_kernel(
                                float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
        if (hit) {
-         advance_pixel(cold, j, h, w, dL_dalpha, dL_dz);
-         if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
-         if (kFlow) {
-           const float* Q = &s_t2[j * 9];
-           const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
-           const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
-           float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
-           w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-           acc_f0 = last_alpha * last_f0 + (1.0f - last_alpha) * acc_f0;
-           acc_f1 = last_alpha * last_f1 + (1.0f - last_alpha) * acc_f1;
-           last_f0 = u2 / w2 - pxf, last_f1 = v2 / w2 - pyf;
-           dL_dalpha += (last_f0 - acc_f0) * dLf0 + (last_f1 - acc_f1) * dLf1;
-           const float gu = w / w2 * dLf0, gv = w / w2 * dLf1;
-           const float gw = -w / (w2 * w2) * (u2 * dLf0 + v2 * dLf1);
-           dsx += Q[0] * gu + Q[3] * gv + Q[6] * gw;
-           dsy += Q[1] * gu + Q[4] * gv + Q[7] * gw;
-           acc_w = last_alpha + (1.0f - last_alpha) * acc_w;
-           dL_dalpha += (1.0f - acc_w) * dL_dsum_w;
-         }
+         advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, dsx, dsy);
+         if (kFlow) dsx += dL_dz * hot.m[6], dsy += dL_dz * hot.m[7];
+         else if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
          GdA = dL_dalpha * T * h.G;
-         last_alpha = h.alpha;
          // the Gaussian's own part of d/ds: only the intersection case uses it (times 1 / p_z below)
          oG = hot.opacity * GdA;
          dsx -= oG * h.sx, dsy -= oG * h.sy;
