@@ -12,9 +12,9 @@
 // sums a surfel's records in a fixed order. (Without scan offsets: one global atomic per surfel, component and tile.)
 // With flow the step is 50 instructions longer. Its channels, and the sum of weights that it is divided by, ride on the recurrence
 // that the image's share, its three quotients take one reciprocal, and the second transforms are loaded when a batch is staged:
-// in 128 registers, four wavefronts per SIMD instead of three. Backward with flow, 300k surfels 800x800: 485 -> 340 us; 5000 surfels
-// over about 4x4 tiles each, 800x800: 784 -> 627; 2000 over about 10x10: 1468 -> 1149 (with a work list per 8x8 quadrant they
-// took 530, 715 and 1280).
+// in 128 registers, four wavefronts per SIMD instead of three. Backward with flow, 300k surfels 800x800:
+// 485 -> 340 us; 5000 surfels with deviations of about 43 pixels 784 -> 627, 2000 of about 128 pixels 1468 -> 1149 (with a work
+// list per 8x8 quadrant they took 530, 715 and 1280).
 // Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
 // the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
 // 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260

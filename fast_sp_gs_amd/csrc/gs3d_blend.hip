@@ -425,12 +425,16 @@ __device__ __forceinline__ float row_sum9_transposed(const float (&v)[9]) {
 }
 
 // Bound by vector issue. Without extra channels nine sums cross the lanes, not sixteen, and the factor -opacity, the same for
-// every pixel, is applied to the sums; the flush takes sixteen lanes per Gaussian, a component each, whose atomics are three
-// requests (a line per gradient tensor). 300k Gaussians 800x800: 177 -> 140 us with a row of lanes per 4x4 block instead of
+// every pixel, is applied to the sums. 300k Gaussians 800x800: 177 -> 140 us with a row of lanes per 4x4 block instead of
 // a wavefront per 8x8 quadrant, over the blocks that the forward noted.
+// The flush writes a component per lane straight from the rows' sums, so no totals are kept in LDS and four blocks share a compute
+// unit, not three: 300k with four extra channels 278 -> 231 us by atomics, 297 -> 254 by records. Where the forward's notes leave an
+// entry few rows and nine components, two lanes per entry and totals in LDS are the faster flush (139 us, by component 142).
 // kSlots: the per-Gaussian sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
-template <int E, bool kSlots>
-__global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
+// kHits: over the blocks that the forward noted (hit_blocks) instead of a bound of every staged footprint.
+template <int E, bool kSlots, bool kHits>
+__global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(E == 0 ? 5 : 4)))
+gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H,
     const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list, const float2* __restrict__ means2D,
     const float4* __restrict__ conic_opacity, const float* __restrict__ colors, const float* __restrict__ extras,
     const float* __restrict__ out_opacity, const int32_t* __restrict__ n_contrib, const float* __restrict__ dL_dpix,
@@ -446,10 +450,10 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
   __shared__ G3Splat<E> s_splat[kB + 1];  // the last one is what padding names: no pixel blends it
   __shared__ __attribute__((aligned(16))) unsigned char s_list[16 * kB + 16];
   __shared__ float s_sum[kRowPlaces + 1][kSums];
-  __shared__ float s_total[kB][kSums + (kNine ? 0 : 1)];  // over the tile, written and read by the same wavefront
+  __shared__ float s_total[kNine && kHits ? kB : 1][kSums];  // over the tile, written and read by the same wavefront
   // What the flush of a batch reads is kept twice, by batch parity: the next batch is staged while others still flush.
   __shared__ uint4 s_place[2][kB];  // where each of the 16 rows stores its sums of each staged Gaussian
-  __shared__ float2 s_tag[2][kB];   // its number and opacity
+  __shared__ float2 s_tag[2][kB];   // its record (kSlots) or number, and its opacity
   __shared__ unsigned s_mask[kB];   // which 4x4 blocks of the tile it can reach
   __shared__ int s_max_contrib;
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
@@ -505,13 +509,12 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
   unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
-  size_t slot = 0;  // record position of the entry this lane staged (the same lane flushes it)
   // entry e of the batch that starts behind `done` entries, counted from the back of the list
   auto gather = [&](int done) {
     const int e = (int) threadIdx.x;
     if (e >= min(kB, n_todo - done)) return;
     const int64_t at = r0 + (n_todo - 1 - done - e);
-    if (hit_blocks) next_hits = hit_blocks[at];
+    if (kHits) next_hits = hit_blocks[at];
     next = gather_splat3<E>(point_list[at], means2D, conic_opacity, colors, extras);
     if (kSlots) next_radius = radii[next.id], next_off = next.id == 0 ? 0 : point_offsets[next.id - 1];
   };
@@ -522,17 +525,17 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
       const int e = (int) threadIdx.x;
       unsigned mask = 0u;
       if (e < n_staged) {
-        mask = hit_blocks ? pair_blocks(next_hits)
-                          : conic_blocks<16>(next.x, next.y, next.a, next.b, next.c, next.opacity, tile_x * kTile,
-                                             tile_y * kTile, flags);
+        mask = kHits ? pair_blocks(next_hits)
+                     : conic_blocks<16>(next.x, next.y, next.a, next.b, next.c, next.opacity, tile_x * kTile, tile_y * kTile, flags);
         s_splat[e]       = next;
-        s_tag[parity][e] = make_float2(__int_as_float(next.id), next.opacity);
         s_place[parity][e] = no_places(kRowPlaces);
+        int to = next.id;
         if (kSlots) {
           // the binning emits a Gaussian's tiles row-major over its rectangle, from its prefix-scan offset on
           const TileRect r = tile_rect(next.x, next.y, next_radius, gx, gy);
-          slot = (size_t) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
+          to = (int) (next_off + (int64_t) (tile_y - r.y0) * (r.x1 - r.x0) + (tile_x - r.x0));
         }
+        s_tag[parity][e] = make_float2(__int_as_float(to), next.opacity);
       }
       s_mask[e] = mask;
     }
@@ -599,37 +602,46 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
     walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j]; }, entry,
                     [] { return true; });
     __syncthreads();
-    // Two lanes per entry add its rows; a wavefront keeps the totals of its 32 entries for itself.
-    static_assert(kBlendThreads == 2 * kB);
-    if (const int e = (int) threadIdx.x >> 1; e < n_here) {
-      constexpr int kHalf = (kSums + 1) / 2;
-      const int h = (int) threadIdx.x & 1;
-      float a[kHalf];
-      sum_places<kSums>(&s_sum[0][0], s_place[parity][e], h * (kSums / 2), a);
+    // Flush the batch: add the sums of the rows that hold an entry, in row order.
+    if (kSlots && kNine) {
+      // two lanes per entry, half of its record's sixteen floats each; the geometry's part still lacks the factor -opacity
+      static_assert(kBlendThreads == 2 * kB && kG3Slots == 16);
+      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
+        const bool upper = threadIdx.x & 1;
+        float a[5];
+        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], upper ? 4 : 0, a);
+        const float2 tag = s_tag[parity][e];
+        const float no = -tag.y;
+        // lower half: colour, mean x; upper half: mean y, conic, opacity
+        float4* dst = (float4*) (slot_records + (size_t) __float_as_int(tag.x) * kG3Slots) + (upper ? 2 : 0);
+        dst[0] = upper ? make_float4(no * a[0], 0.5f * no * a[1], no * a[2], 0.5f * no * a[3]) : make_float4(a[0], a[1], a[2], 0.0f);
+        dst[1] = upper ? make_float4(a[4], 0.0f, 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, no * a[3]);
+      }
+    } else if (kSlots) {
+      // a lane per component of the record
+      for (int t = (int) threadIdx.x; t < n_here * kG3Slots; t += kBlendThreads) {
+        const int e = t / kG3Slots, c = t % kG3Slots;
+        float a[1];
+        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
+        const float2 tag  = s_tag[parity][e];
+        const float scale = c < kGeom || c > kGeom + 4 ? 1.0f : c == kGeom + 2 || c == kGeom + 4 ? -0.5f * tag.y : -tag.y;
+        slot_records[(size_t) __float_as_int(tag.x) * kG3Slots + c] = scale * a[0];
+      }
+    } else if (kNine && kHits) {
+      // Two lanes per entry add its rows; a wavefront keeps the totals of its 32 entries and adds them to the tensors with
+      // sixteen lanes per entry, a component each: three requests (a line per gradient tensor).
+      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
+        const int h = (int) threadIdx.x & 1;
+        float a[5];
+        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], 4 * h, a);
 #pragma unroll
-      for (int c = 0; c < kHalf; ++c) s_total[e][h * (kSums / 2) + c] = a[c];
-    }
-    if (kSlots) __syncthreads();
-    else wave_lds_sync();  // the two lanes of an entry write what the sixteen below read
-    if (kSlots && (int) threadIdx.x < n_here) {
-      float sums[kSums], a[16];
-#pragma unroll
-      for (int c = 0; c < kSums; ++c) sums[c] = s_total[threadIdx.x][c];
-      const float no = -s_tag[parity][threadIdx.x].y;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) a[c] = c < 3 + E ? sums[c < kGeom ? c : 0] : 0.0f;
-      a[7] = no * sums[kGeom], a[8] = no * sums[kGeom + 1];
-      a[9] = 0.5f * no * sums[kGeom + 2], a[10] = no * sums[kGeom + 3], a[11] = 0.5f * no * sums[kGeom + 4];
-      a[12] = sums[kGeom + 5];
-      float4* dst = (float4*) (slot_records + slot * kG3Slots);
-#pragma unroll
-      for (int c = 0; c < kG3Slots / 4; ++c) dst[c] = make_float4(a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]);
-    }
-    if (!kSlots) {
+        for (int c = 0; c < 5; ++c) s_total[e][4 * h + c] = a[c];
+      }
+      wave_lds_sync();  // the two lanes of an entry write what the sixteen below read
       const int c = (int) threadIdx.x & 15, g = c - kGeom;  // component, and its number among the geometry's six
-      if (c < 3 + E || (g >= 0 && g < 6)) {
-        float* const out = c < 3 ? g_colors + c : c < 3 + E ? g_extras + (c - 3) : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
-        const size_t row = c < 3 ? 3 : c < 3 + E ? E : g < 2 ? 2 : 4;
+      if (c < kSums) {
+        float* const out = c < 3 ? g_colors + c : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
+        const size_t row = c < 3 ? 3 : g < 2 ? 2 : 4;
         for (int k = 0; k < kB / 16; ++k) {
           const int e = wave * (kB / 4) + 4 * k + (lane >> 4);
           if (e >= n_here) break;
@@ -639,6 +651,25 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_backward_kernel(int flags,
           if (g == 2 || g == 4) sum *= 0.5f;
           if (sum != 0.0f) atomicAdd(out + row * (size_t) __float_as_int(tag.x), sum);
         }
+      }
+    } else {
+      // one global atomic per Gaussian and component for this tile, a lane per component
+      constexpr int kUsed = kNine ? kSums : 13;
+      for (int t = (int) threadIdx.x; t < n_here * kUsed; t += kBlendThreads) {
+        const int e = t / kUsed, c = t - e * kUsed, g = c - kGeom;  // g: number among the geometry's six
+        if (c >= 3 + E && g < 0) continue;
+        float a[1];
+        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
+        const float2 tag = s_tag[parity][e];
+        const size_t id  = (size_t) __float_as_int(tag.x);
+        float* const out = c < 3       ? g_colors + 3 * id + c
+                           : c < 3 + E ? g_extras + E * id + (c - 3)
+                           : g < 2     ? g_means2D + 2 * id + g
+                                       : g_conic_opacity + 4 * id + (g - 2);
+        float sum = a[0];
+        if (g >= 0 && g < 5) sum *= -tag.y;
+        if (g == 2 || g == 4) sum *= 0.5f;
+        if (sum != 0.0f) atomicAdd(out, sum);
       }
     }
     done += n_here;
@@ -1172,18 +1203,20 @@ int rasterize_backward(int P, int W, int H, int E, const float* means2D,
   const int* tile_order = nullptr;
   const int flags = launch_tile_order(gx, gy, ranges, s, &tile_order);
   const dim3 grid(gx * gy), block(kBlendThreads);
-#define FSGS_G3_BWD(EE, SL)                                                                                         \
-  hipLaunchKernelGGL((gs3d_backward_kernel<EE, SL>), grid, block, 0, s, flags, tile_order, W, H, ranges, point_list, \
+#define FSGS_G3_BWD(EE, SL, HT)                                                                                     \
+  hipLaunchKernelGGL((gs3d_backward_kernel<EE, SL, HT>), grid, block, 0, s, flags, tile_order, W, H, ranges, point_list, \
                      (const float2*) means2D, (const float4*) conic_opacity, colors, extras, out_opacity, n_contrib, \
                      dL_dpix, dL_dout_extras, dL_dout_opacity, g_means2D, g_conic_opacity, g_colors, g_extras,      \
                      point_offsets, radii, ws.records, hit_blocks)
 #define FSGS_G3_BWD_E(EE)                                                                                           \
   do {                                                                                                              \
     if (slots) {                                                                                                    \
-      FSGS_G3_BWD(EE, true);                                                                                        \
+      FSGS_G3_BWD(EE, true, false);                                                                                 \
       launch_slot_sum<kG3Slots>(P, point_offsets, ws, G3Scatter<EE>{g_means2D, g_conic_opacity, g_colors, g_extras}, s); \
+    } else if (hit_blocks) {                                                                                        \
+      FSGS_G3_BWD(EE, false, true);                                                                                 \
     } else {                                                                                                        \
-      FSGS_G3_BWD(EE, false);                                                                                       \
+      FSGS_G3_BWD(EE, false, false);                                                                                \
     }                                                                                                               \
   } while (0)
   switch (E) {

@@ -12,7 +12,7 @@ CSRC = Path(__file__).resolve().parents[1] / 'fast_sp_gs_amd' / 'csrc'
     ('block_lists.hpp', 'int build_block_lists(', 'if (on) lists[', 'return longest'),
     ('block_lists.hpp', 'int build_row_lists(', '((uint2*) lists)[lane] =', 'if (on) lists['),
     ('block_lists.hpp', 'int build_row_lists(', 'if (on) lists[', 'return longest'),
-    ('gs3d_blend.hip', 'gs3d_backward_kernel(', 's_total[e][h * (kSums / 2) + c] =', 'float sum = s_total[e][c]'),
+    ('gs3d_blend.hip', 'gs3d_backward_kernel(', 's_total[e][4 * h + c] =', 'float sum = s_total[e][c]'),
 ])
 def test_lanes_exchange_in_order(source, start, write, read):
     text = (CSRC / source).read_text()
