@@ -54,6 +54,8 @@ blend_backward_kernel(
     if (slots.region) return (stored >= 0 ? stored : (int64_t) slots.offset[id]) + slots.region[slot_region(id)];
     return stored >= 0 ? stored : (id == 0 ? 0 : slots.scan[id - 1]);
   };
+  constexpr bool kRewalk = kFlow || !kSlots;  // several batches per staging (kRewalkBelow); a view's entries come as notes and
+                                              // rarely fill their tile: with it 781 -> 787 us at 3M surfels
   constexpr int kRowPlaces = kFlow ? 248 : 255;  // of a batch: with 36.5 KB (flow: 40 KB) of LDS four blocks share a compute unit
   using Shape = BlockShape<16>;
   __shared__ Splat s_splat[kRowBatch + 1];  // the last one is what padding names: no pixel blends it
@@ -94,7 +96,7 @@ blend_backward_kernel(
   if (threadIdx.x < kGradSlots) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
   if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kRowBatch])[threadIdx.x] = 0u;
   __syncthreads();
-  const int n_todo = min(s_max_contrib, (int) (r1 - r0));  // positions [0, n_todo) of the tile's list, walked from n_todo-1 down to 0
+  const int n_todo = __builtin_amdgcn_readfirstlane(min(s_max_contrib, (int) (r1 - r0)));  // positions [0, n_todo) of the tile's list, walked from n_todo-1 down to 0
   // No zero fill of the records: the instances behind the tile's deepest contributor are never staged, their records
   // are cleared here; every staged instance writes its record at the flush, zeros included
   if (kSlots) {
@@ -158,7 +160,7 @@ blend_backward_kernel(
   int next_radius = 0;
   unsigned next_hits = 0u;
   int64_t next_off = 0;
-  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  // entry e of the 128 staged behind `done` entries, counted from the back of the list
   auto gather = [&](int done) {
     const int e = (int) threadIdx.x;
     if (e >= min(kRowBatch, n_todo - done)) return;
@@ -198,166 +200,175 @@ blend_backward_kernel(
       s_mask[e] = mask;
     }
     __syncthreads();
-    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
-    int start, before[4];
-    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
-    gather(done + n_here);
-    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
-    const int behind = n_todo - done;
-    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
-    const int steps = build_row_lists(&s_list[4 * kRowBatch * wave], (unsigned char*) s_place[parity], masks, wave, first, start,
-                                      before, n_here);
-    const int my_first = behind - last_contrib, my_median = behind - median_contrib;
-    // ---- order-bound part of one (pixel, entry) pair: advances the pixel's back-to-front state -------------------------
-    // All channels that enter the image linearly (colour, depth, opacity, normal, flow) share one recurrence: with
-    // c = <upstream gradient, channel values of this surfel>, the reference's per-channel accumulators
-    // acc_x = last_alpha * last_x + (1 - last_alpha) * acc_x contract to a single scalar, updated at the end of the
-    // pair that supplies alpha and x. Leaves the blend weight w, dL/dalpha and dL/ddepth of the pair, and the flow's part of
-    // dL/d(intersection); call under `hit` only.
-    auto advance_pixel = [&](const SplatCold& cold, int j, const Hit& h, float& w, float& dL_dalpha, float& dL_dz, float& fsx,
-                             float& fsy) {
-      const float keep = 1.0f - h.alpha;
-      T = T * __builtin_amdgcn_rcpf(keep);
-      w = h.alpha * T;
-      // one chain of fused multiply-adds; the per-pixel constant of the distortion term sits in lin_const
-      float c_lin;
-      if (kAux) {
-        const float rd     = __builtin_amdgcn_rcpf(h.depth);
-        const float m_d    = fmaf(-far_near, rd, far_scale);
-        const float dmd_dd = far_near * rd * rd;
-        // dL/dweight of the distortion enters dL/dalpha exactly as a linear channel does (its own value minus what the
-        // pairs behind it accumulated, with the same weights), so it rides on the shared recurrence
-        c_lin = fmaf(h.depth, dL_ddepth, lin_const);
-        c_lin = fmaf(m_d, fmaf(m_d, reg_A, -reg_2D), c_lin);
-        c_lin = fmaf(cold.nx, dLn0, fmaf(cold.ny, dLn1, fmaf(cold.nz, dLn2, c_lin)));
-        // dL/ddepth: through the distortion's normalised depth, the depth map, and the median depth
-        const float per_w = fmaf(fmaf(m_d, reg_2A, -reg_2D), dmd_dd, dL_ddepth);
-        dL_dz = fmaf(w, per_w, j == my_median ? dL_dmedian : 0.0f);
+    unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    const RowCounts counts(masks, wave);
+    int base = 0;  // staged entries of the batches before
+    for (bool more = true; more;) {
+      int start, before[4];
+      const int end = row_batch<kRowPlaces>(counts, base, n_staged, start);
+      if (kRewalk) masks[0] = s_mask[lane], masks[1] = s_mask[kWave + lane];  // read again rather than kept through the walk
+      more = kRewalk && end - base < kRewalkBelow && end < n_staged;
+      if (!more) gather(done + end);
+      // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+      const int behind = n_todo - done;
+      int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+      if (kRewalk) for (int& f : first) f = max(f, base);
+      const int steps = build_row_lists(&s_list[4 * kRowBatch * wave], (unsigned char*) s_place[parity], masks, wave, first, start,
+                                        before, end);
+      const int my_first = behind - last_contrib, my_median = behind - median_contrib;
+      // ---- order-bound part of one (pixel, entry) pair: advances the pixel's back-to-front state -------------------------
+      // All channels that enter the image linearly (colour, depth, opacity, normal, flow) share one recurrence: with
+      // c = <upstream gradient, channel values of this surfel>, the reference's per-channel accumulators
+      // acc_x = last_alpha * last_x + (1 - last_alpha) * acc_x contract to a single scalar, updated at the end of the
+      // pair that supplies alpha and x. Leaves the blend weight w, dL/dalpha and dL/ddepth of the pair, and the flow's part of
+      // dL/d(intersection); call under `hit` only.
+      auto advance_pixel = [&](const SplatCold& cold, int j, const Hit& h, float& w, float& dL_dalpha, float& dL_dz, float& fsx,
+                               float& fsy) {
+        const float keep = 1.0f - h.alpha;
+        T = T * __builtin_amdgcn_rcpf(keep);
+        w = h.alpha * T;
+        // one chain of fused multiply-adds; the per-pixel constant of the distortion term sits in lin_const
+        float c_lin;
+        if (kAux) {
+          const float rd     = __builtin_amdgcn_rcpf(h.depth);
+          const float m_d    = fmaf(-far_near, rd, far_scale);
+          const float dmd_dd = far_near * rd * rd;
+          // dL/dweight of the distortion enters dL/dalpha exactly as a linear channel does (its own value minus what the
+          // pairs behind it accumulated, with the same weights), so it rides on the shared recurrence
+          c_lin = fmaf(h.depth, dL_ddepth, lin_const);
+          c_lin = fmaf(m_d, fmaf(m_d, reg_A, -reg_2D), c_lin);
+          c_lin = fmaf(cold.nx, dLn0, fmaf(cold.ny, dLn1, fmaf(cold.nz, dLn2, c_lin)));
+          // dL/ddepth: through the distortion's normalised depth, the depth map, and the median depth
+          const float per_w = fmaf(fmaf(m_d, reg_2A, -reg_2D), dmd_dd, dL_ddepth);
+          dL_dz = fmaf(w, per_w, j == my_median ? dL_dmedian : 0.0f);
+        } else {
+          c_lin = 0.0f;
+        }
+        c_lin = fmaf(cold.r, dLp0, fmaf(cold.g, dLp1, fmaf(cold.b, dLp2, c_lin)));
+        if (kFlow) {
+          const float* Q = &s_t2[j * 9];
+          const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
+          const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
+          float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
+          w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
+          float rw = __builtin_amdgcn_rcpf(w2);
+          rw = fmaf(fmaf(-w2, rw, 1.0f), rw, rw);  // a Newton step: as good as a division
+          // flow u2 / w2 - x as (u2 - x w2) / w2: one rounding in the difference of two nearly equal numbers
+          const float fu = fmaf(-pxf, w2, u2) * rw, fv = fmaf(-pyf, w2, v2) * rw;
+          c_lin = fmaf(fu, dLf0, fmaf(fv, dLf1, c_lin));
+          const float wr = w * rw, gu = wr * dLf0, gv = wr * dLf1, gw = -wr * fmaf(fu + pxf, dLf0, (fv + pyf) * dLf1);
+          fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
+          fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
+        }
+        // acc_lin: what the pairs behind this one accumulated, alpha_j c_j weighted by the transmittance between
+        dL_dalpha = c_lin - acc_lin;
+        acc_lin   = fmaf(keep, acc_lin, h.alpha * c_lin);
+      };
+       // Gradient terms of one (pixel, entry) pair. The part under `hit` leaves
+       // a few factors (zero for a lane whose pixel does not blend the entry); the 16 + 2 per-surfel components are
+       // products of those factors with quantities that are finite in every lane, formed by all lanes alike, so no
+       // component needs a zero of its own and the two ways a surfel is met (ray-splat intersection / projected centre)
+       // share one instruction stream.
+       auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, const Hit& h, bool hit,
+                                 float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
+         float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
+         if (hit) {
+           advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, dsx, dsy);
+           if (kFlow) dsx += dL_dz * hot.m[6], dsy += dL_dz * hot.m[7];
+           else if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
+           GdA = dL_dalpha * T * h.G;
+           // the Gaussian's own part of d/ds: only the intersection case uses it (times 1 / p_z below)
+           oG = hot.opacity * GdA;
+           dsx -= oG * h.sx, dsy -= oG * h.sy;
+           // s is not finite in a lane whose plane pair degenerates (p_z == 0), and such a lane never blends: every use
+           // of s sits on this side
+           s_ds = dsx * h.sx + dsy * h.sy;
+           z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
+         }
+         const bool by_ray   = h.rho3d <= h.rho2d;
+         const bool filtered = hit && !by_ray;
+         filtered_lanes      = ~wave_ballot(by_ray);  // taken where the comparison is made: its own lane mask, no instruction
+         // d/dp of the homogeneous intersection point p = k x l, negated (the components below are minus the plane
+         // gradients): p_xy = s p_z, so dp_xy = ds / p_z and dp_z = -<ds, s> / p_z
+         const float rz  = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
+         const float npx = -(dsx * rz), npy = -(dsy * rz), npz = s_ds * rz;
+         const float nkx = h.ly * npz - h.lz * npy, nky = h.lz * npx - h.lx * npz, nkz = h.lx * npy - h.ly * npx;
+         const float nlx = npy * h.kz - npz * h.ky, nly = npz * h.kx - npx * h.kz, nlz = npx * h.ky - npy * h.kx;
+         g[0] = w * dLp0, g[1] = w * dLp1, g[2] = w * dLp2;
+         g[3] = nkx, g[4] = nky, g[5] = nkz;
+         g[6] = nlx, g[7] = nly, g[8] = nlz;
+         g[9]  = z_sx - (pxf * nkx + pyf * nlx);
+         g[10] = z_sy - (pxf * nky + pyf * nly);
+         g[11] = dL_dz - (pxf * nkz + pyf * nlz);
+         if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
+         else      g[12] = g[13] = g[14] = 0.0f;
+         g[15] = GdA;
+         const float to_centre = filtered ? -2.0f * oG : 0.0f;
+         g2x = to_centre * h.dx, g2y = to_centre * h.dy;
+       };
+       const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+       float* const sums   = &s_sum[place][lane & 15];               // component lane & 15 of the row's first place
+       float* const centre = &s_sum[place][16 + (lane >> 3 & 1)];  // the row's lanes 0 and 8: means2D
+       auto backward_entry = [&](const SplatHot& hot, int j, int i) {
+        const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+        __builtin_amdgcn_sched_barrier(0);
+        Hit h;
+        unsigned long long pass, filtered = 0ull;
+        intersect_flat(hot, pxf, pyf, near_n, h, &pass);
+        pass &= wave_ballot(j >= my_first);
+        float tot = 0.0f, mid = 0.0f;
+        if (pass != 0ull) {
+          float g[16], g2x, g2y;
+          pair_gradients(hot, cold, j, h, __builtin_amdgcn_inverse_ballot_w64(pass), g, g2x, g2y, filtered);
+          tot = row_sum16_transposed(g);
+          if ((pass & filtered) != 0ull) {  // some lane met the surfel by its projected centre
+            g2x += dpp_shift_zero<0x128, 0xf, 0xf>(g2x), g2y += dpp_shift_zero<0x128, 0xf, 0xf>(g2y);  // row_ror:8
+            mid = (lane & 8) ? g2y : g2x;
+            mid += dpp_shift_zero<0x104, 0xf, 0xf>(mid);  // row_shl:4, 2, 1: totals in lanes 0 and 8
+            mid += dpp_shift_zero<0x102, 0xf, 0xf>(mid);
+            mid += dpp_shift_zero<0x101, 0xf, 0xf>(mid);
+          }
+        }
+        if (j != kRowBatch) {  // not a padding step; zeros, too, have their place
+          sums[i * kGradSlots] = tot;
+          if ((lane & 7) == 0) centre[i * kGradSlots] = mid;
+        }
+       };
+      if (kRewalk && base > 0) __syncthreads();  // the sums of the batch before have been read
+       walk_block_list(&s_list[(4 * wave + row) * kRowBatch], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
+                       [] { return true; });
+      __syncthreads();
+      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      if (kSlots) {
+        // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order, nine components per lane; the
+        // per-surfel sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that
+        // are never staged were cleared at the start), so nobody has to clear the buffer beforehand.
+        static_assert(kBlendThreads == 2 * kRowBatch);
+        if (const int e = base + ((int) threadIdx.x >> 1); e < end) {
+          constexpr int kHalf = kGradSlots / 2;
+          const int h = (int) threadIdx.x & 1;
+          float a[kHalf];
+          sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], h * kHalf, a);
+          float* dst = slot_grads + (size_t) s_slot[parity][e] * kGradSlots + h * kHalf;
+#pragma unroll
+          for (int k = 0; k < kHalf; ++k) dst[k] = a[k];
+        }
       } else {
-        c_lin = 0.0f;
-      }
-      c_lin = fmaf(cold.r, dLp0, fmaf(cold.g, dLp1, fmaf(cold.b, dLp2, c_lin)));
-      if (kFlow) {
-        const float* Q = &s_t2[j * 9];
-        const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
-        const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
-        float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
-        w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-        float rw = __builtin_amdgcn_rcpf(w2);
-        rw = fmaf(fmaf(-w2, rw, 1.0f), rw, rw);  // a Newton step: as good as a division
-        // flow u2 / w2 - x as (u2 - x w2) / w2: one rounding in the difference of two nearly equal numbers
-        const float fu = fmaf(-pxf, w2, u2) * rw, fv = fmaf(-pyf, w2, v2) * rw;
-        c_lin = fmaf(fu, dLf0, fmaf(fv, dLf1, c_lin));
-        const float wr = w * rw, gu = wr * dLf0, gv = wr * dLf1, gw = -wr * fmaf(fu + pxf, dLf0, (fv + pyf) * dLf1);
-        fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
-        fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
-      }
-      // acc_lin: what the pairs behind this one accumulated, alpha_j c_j weighted by the transmittance between
-      dL_dalpha = c_lin - acc_lin;
-      acc_lin   = fmaf(keep, acc_lin, h.alpha * c_lin);
-    };
-     // Gradient terms of one (pixel, entry) pair. The part under `hit` leaves
-     // a few factors (zero for a lane whose pixel does not blend the entry); the 16 + 2 per-surfel components are
-     // products of those factors with quantities that are finite in every lane, formed by all lanes alike, so no
-     // component needs a zero of its own and the two ways a surfel is met (ray-splat intersection / projected centre)
-     // share one instruction stream.
-     auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, const Hit& h, bool hit,
-                               float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
-       float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
-       if (hit) {
-         advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, dsx, dsy);
-         if (kFlow) dsx += dL_dz * hot.m[6], dsy += dL_dz * hot.m[7];
-         else if (kAux) dsx = dL_dz * hot.m[6], dsy = dL_dz * hot.m[7];
-         GdA = dL_dalpha * T * h.G;
-         // the Gaussian's own part of d/ds: only the intersection case uses it (times 1 / p_z below)
-         oG = hot.opacity * GdA;
-         dsx -= oG * h.sx, dsy -= oG * h.sy;
-         // s is not finite in a lane whose plane pair degenerates (p_z == 0), and such a lane never blends: every use
-         // of s sits on this side
-         s_ds = dsx * h.sx + dsy * h.sy;
-         z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
-       }
-       const bool by_ray   = h.rho3d <= h.rho2d;
-       const bool filtered = hit && !by_ray;
-       filtered_lanes      = ~wave_ballot(by_ray);  // taken where the comparison is made: its own lane mask, no instruction
-       // d/dp of the homogeneous intersection point p = k x l, negated (the components below are minus the plane
-       // gradients): p_xy = s p_z, so dp_xy = ds / p_z and dp_z = -<ds, s> / p_z
-       const float rz  = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
-       const float npx = -(dsx * rz), npy = -(dsy * rz), npz = s_ds * rz;
-       const float nkx = h.ly * npz - h.lz * npy, nky = h.lz * npx - h.lx * npz, nkz = h.lx * npy - h.ly * npx;
-       const float nlx = npy * h.kz - npz * h.ky, nly = npz * h.kx - npx * h.kz, nlz = npx * h.ky - npy * h.kx;
-       g[0] = w * dLp0, g[1] = w * dLp1, g[2] = w * dLp2;
-       g[3] = nkx, g[4] = nky, g[5] = nkz;
-       g[6] = nlx, g[7] = nly, g[8] = nlz;
-       g[9]  = z_sx - (pxf * nkx + pyf * nlx);
-       g[10] = z_sy - (pxf * nky + pyf * nly);
-       g[11] = dL_dz - (pxf * nkz + pyf * nlz);
-       if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
-       else      g[12] = g[13] = g[14] = 0.0f;
-       g[15] = GdA;
-       const float to_centre = filtered ? -2.0f * oG : 0.0f;
-       g2x = to_centre * h.dx, g2y = to_centre * h.dy;
-     };
-     const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
-     float* const sums   = &s_sum[place][lane & 15];               // component lane & 15 of the row's first place
-     float* const centre = &s_sum[place][16 + (lane >> 3 & 1)];  // the row's lanes 0 and 8: means2D
-     auto backward_entry = [&](const SplatHot& hot, int j, int i) {
-      const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
-      __builtin_amdgcn_sched_barrier(0);
-      Hit h;
-      unsigned long long pass, filtered = 0ull;
-      intersect_flat(hot, pxf, pyf, near_n, h, &pass);
-      pass &= wave_ballot(j >= my_first);
-      float tot = 0.0f, mid = 0.0f;
-      if (pass != 0ull) {
-        float g[16], g2x, g2y;
-        pair_gradients(hot, cold, j, h, __builtin_amdgcn_inverse_ballot_w64(pass), g, g2x, g2y, filtered);
-        tot = row_sum16_transposed(g);
-        if ((pass & filtered) != 0ull) {  // some lane met the surfel by its projected centre
-          g2x += dpp_shift_zero<0x128, 0xf, 0xf>(g2x), g2y += dpp_shift_zero<0x128, 0xf, 0xf>(g2y);  // row_ror:8
-          mid = (lane & 8) ? g2y : g2x;
-          mid += dpp_shift_zero<0x104, 0xf, 0xf>(mid);  // row_shl:4, 2, 1: totals in lanes 0 and 8
-          mid += dpp_shift_zero<0x102, 0xf, 0xf>(mid);
-          mid += dpp_shift_zero<0x101, 0xf, 0xf>(mid);
+        // one global atomic per surfel and component for this tile, a lane per component: a surfel's are a few requests
+        for (int t = (int) threadIdx.x; t < (end - base) * kGradSlots; t += kBlendThreads) {
+          const int q = t / kGradSlots, c = t - q * kGradSlots, e = base + q, id = s_slot[parity][e];
+          float a[1];
+          sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
+          float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
+                             : c < 12 ? g_trans + 9 * (size_t) id + (c - 3)
+                             : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
+                                      : g_means2D + 2 * (size_t) id + (c - 16);
+          if (a[0] != 0.0f) atomicAdd(out, a[0]);
         }
       }
-      if (j != kRowBatch) {  // not a padding step; zeros, too, have their place
-        sums[i * kGradSlots] = tot;
-        if ((lane & 7) == 0) centre[i * kGradSlots] = mid;
-      }
-     };
-     walk_block_list(&s_list[(4 * wave + row) * kRowBatch], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
-                     [] { return true; });
-    __syncthreads();
-    // Flush the batch: add the sums of the rows that hold an entry, in row order.
-    if (kSlots) {
-      // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order, nine components per lane; the
-      // per-surfel sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that
-      // are never staged were cleared at the start), so nobody has to clear the buffer beforehand.
-      static_assert(kBlendThreads == 2 * kRowBatch);
-      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
-        constexpr int kHalf = kGradSlots / 2;
-        const int h = (int) threadIdx.x & 1;
-        float a[kHalf];
-        sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], h * kHalf, a);
-        float* dst = slot_grads + (size_t) s_slot[parity][e] * kGradSlots + h * kHalf;
-#pragma unroll
-        for (int k = 0; k < kHalf; ++k) dst[k] = a[k];
-      }
-    } else {
-      // one global atomic per surfel and component for this tile, a lane per component: a surfel's are a few requests
-      for (int t = (int) threadIdx.x; t < n_here * kGradSlots; t += kBlendThreads) {
-        const int e = t / kGradSlots, c = t - e * kGradSlots, id = s_slot[parity][e];
-        float a[1];
-        sum_places<kGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
-        float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
-                           : c < 12 ? g_trans + 9 * (size_t) id + (c - 3)
-                           : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
-                                    : g_means2D + 2 * (size_t) id + (c - 16);
-        if (a[0] != 0.0f) atomicAdd(out, a[0]);
-      }
+      base = end;
     }
-    done += n_here;
+    done += base;
     // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
     // records, which nobody reads before, and the other copy of what the flush reads.
   }

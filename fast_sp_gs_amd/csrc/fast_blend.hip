@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(kBlendThreads)
   if (threadIdx.x < kFastGradSlots) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
   if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kB])[threadIdx.x] = 0u;
   __syncthreads();
-  const int n_todo = min(s_max_contrib, (int) (r1 - r0));
+  const int n_todo = __builtin_amdgcn_readfirstlane(min(s_max_contrib, (int) (r1 - r0)));
   // No zero fill of the record buffer: every staged instance writes its record at the flush, zeros included, and the
   // instances behind the tile's deepest contributor, which are never staged, are cleared here.
   if (kSlots) {
@@ -578,7 +578,7 @@ __global__ void __launch_bounds__(kBlendThreads)
   unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
-  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  // entry e of the 128 staged behind `done` entries, counted from the back of the list
   auto gather = [&](int done) {
     const int e = (int) threadIdx.x;
     if (e >= min(kB, n_todo - done)) return;
@@ -621,149 +621,158 @@ __global__ void __launch_bounds__(kBlendThreads)
       s_mask[e] = mask;
     }
     __syncthreads();
-    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
-    int start, before[4];
-    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
-    gather(done + n_here);
-    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
-    const int behind = n_todo - done;
-    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
-    const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
-                                      n_here);
-    const int my_first = behind - last_contrib, my_median = behind - median_contrib;
+    unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    const RowCounts counts(masks, wave);
+    int base = 0;  // staged entries of the batches before
+    for (bool more = true; more;) {
+      int start, before[4];
+      const int end = row_batch<kRowPlaces>(counts, base, n_staged, start);
+      masks[0] = s_mask[lane], masks[1] = s_mask[kWave + lane];  // read again rather than kept through the walk
+      more = end - base < kRewalkBelow && end < n_staged;
+      if (!more) gather(done + end);
+      // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+      const int behind = n_todo - done;
+      int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+      for (int& f : first) f = max(f, base);
+      const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
+                                        end);
+      const int my_first = behind - last_contrib, my_median = behind - median_contrib;
 
-    // The part of a pair that is bound to the list's order: advances the pixel's back-to-front state and leaves the
-    // pair's weight, dL/dalpha (times the transmittance in front of the pair), dL/d(depth along the ray) and, with a
-    // second set of transforms, dL/d(intersection) through it. Only entered by lanes whose pixel blends the entry.
-    auto advance_pixel = [&](const SplatCold& cold, int j, const FastHit& h, float& w, float& dL_dalpha,
-                             float& dL_dz, float& fsx, float& fsy) {
-      T = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
-      w = h.alpha * T;
-      // one back-to-front recurrence for every channel that enters the image linearly: c = <upstream gradient,
-      // channel values of this surfel> replaces the reference's per-channel accumulators
-      float c_lin = cold.r * dLp0 + cold.g * dLp1 + cold.b * dLp2;
-      if (kAux) {
-        const float rd     = __builtin_amdgcn_rcpf(h.depth);
-        const float m_d    = far_scale - far_near * rd;
-        const float dmd_dd = far_near * rd * rd;
-        if (j == my_median) dL_dz += dL_dmedian;
-        if (!kPerSplat) {
-          // dL/dweight of the distortion enters dL/dalpha as a linear channel does (its value minus what the pairs
-          // behind it accumulated, with the same weights): it rides on the shared recurrence
-          c_lin += reg_D2 + m_d * (m_d * reg_A - reg_2D);
-          dL_dz += w * (m_d * reg_2A - reg_2D) * dmd_dd;
-        } else {
-          c_lin += m_d * dL_dM1 + (m_d * m_d) * dL_dM2;
-          dL_dz += dmd_dd * (2.0f * m_d * w * dL_dM2);
-        }
-        c_lin += h.depth * dL_ddepth + cold.nx * dLn0 + cold.ny * dLn1 + cold.nz * dLn2;
-        dL_dz += w * dL_ddepth;
-      }
-      if (kAux || kPerSplat) c_lin += dL_daccum;
-      if (kFlow) {
-        const float* Q = &s_t2[j * 9];
-        const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
-        const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
-        float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
-        w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-        const float rw = 1.0f / w2;
-        c_lin += (u2 * rw - pxf) * dLf0 + (v2 * rw - pyf) * dLf1;
-        const float gu = w * rw * dLf0, gv = w * rw * dLf1;
-        const float gw = -w * rw * rw * (u2 * dLf0 + v2 * dLf1);
-        fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
-        fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
-      }
-      dL_dalpha = c_lin - acc_lin;
-      acc_lin   = fmaf(1.0f - h.alpha, acc_lin, h.alpha * c_lin);
-      dL_dalpha *= T;
-    };
-
-    const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
-    float* const sums  = &s_sum[place][lane & 15];  // component lane & 15 of the row's first place
-    float* const sums2 = &s_sum[place][16 + ((lane & 2) ? 4 : (lane >> 2 & 1) * 2 + (lane >> 3 & 1))];
-    auto blend_entry = [&](const FastHot& hot, int j, int i) {
-        const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
-        __builtin_amdgcn_sched_barrier(0);
-        FastHit h;
-        unsigned long long pass;
-        fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass);
-        pass &= wave_ballot(j >= my_first);
-        if (pass == 0ull) {
-          if (j != kB) {  // not a padding step; zeros, too, have their place
-            sums[i * kFastGradSlots] = 0.0f;
-            if ((lane & 1) == 0) sums2[i * kFastGradSlots] = 0.0f;
+      // The part of a pair that is bound to the list's order: advances the pixel's back-to-front state and leaves the
+      // pair's weight, dL/dalpha (times the transmittance in front of the pair), dL/d(depth along the ray) and, with a
+      // second set of transforms, dL/d(intersection) through it. Only entered by lanes whose pixel blends the entry.
+      auto advance_pixel = [&](const SplatCold& cold, int j, const FastHit& h, float& w, float& dL_dalpha,
+                               float& dL_dz, float& fsx, float& fsy) {
+        T = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
+        w = h.alpha * T;
+        // one back-to-front recurrence for every channel that enters the image linearly: c = <upstream gradient,
+        // channel values of this surfel> replaces the reference's per-channel accumulators
+        float c_lin = cold.r * dLp0 + cold.g * dLp1 + cold.b * dLp2;
+        if (kAux) {
+          const float rd     = __builtin_amdgcn_rcpf(h.depth);
+          const float m_d    = far_scale - far_near * rd;
+          const float dmd_dd = far_near * rd * rd;
+          if (j == my_median) dL_dz += dL_dmedian;
+          if (!kPerSplat) {
+            // dL/dweight of the distortion enters dL/dalpha as a linear channel does (its value minus what the pairs
+            // behind it accumulated, with the same weights): it rides on the shared recurrence
+            c_lin += reg_D2 + m_d * (m_d * reg_A - reg_2D);
+            dL_dz += w * (m_d * reg_2A - reg_2D) * dmd_dd;
+          } else {
+            c_lin += m_d * dL_dM1 + (m_d * m_d) * dL_dM2;
+            dL_dz += dmd_dd * (2.0f * m_d * w * dL_dM2);
           }
-          return;
+          c_lin += h.depth * dL_ddepth + cold.nx * dLn0 + cold.ny * dLn1 + cold.nz * dLn2;
+          dL_dz += w * dL_ddepth;
         }
-        const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
-        float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, fsx = 0.0f, fsy = 0.0f;
-        // The part under `hit` leaves a few factors (zero in a lane whose pixel does not blend the entry); the components are
-        // products of those factors with quantities that are finite in every lane, formed by all lanes alike: no
-        // component needs a zero of its own, and the projected-centre case is the intersection case with a zero in
-        // place of 1 / p_z.
-        float g[16], g5[5];
-        float GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
-        if (hit) {
-          advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, fsx, fsy);
-          // d/ds of the intersection case (times 1 / p_z below); s is not finite in a lane whose p_z is 0, and such a
-          // lane never blends: every use of s sits on this side
-          GdA  = dL_dalpha * h.G;
-          oG   = hot.opacity * GdA;
-          dsx  = fsx - oG * h.sx, dsy = fsy - oG * h.sy;
-          if (kAux) dsx += dL_dz * hot.tw0, dsy += dL_dz * hot.tw1;
-          s_ds = dsx * h.sx + dsy * h.sy;
-          z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
+        if (kAux || kPerSplat) c_lin += dL_daccum;
+        if (kFlow) {
+          const float* Q = &s_t2[j * 9];
+          const float u2 = Q[0] * h.sx + Q[1] * h.sy + Q[2];
+          const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
+          float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
+          w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
+          const float rw = 1.0f / w2;
+          c_lin += (u2 * rw - pxf) * dLf0 + (v2 * rw - pyf) * dLf1;
+          const float gu = w * rw * dLf0, gv = w * rw * dLf1;
+          const float gw = -w * rw * rw * (u2 * dLf0 + v2 * dLf1);
+          fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
+          fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
         }
-        const bool by_ray   = h.rho3d <= h.rho2d;
-        const bool filtered = hit && !by_ray;
-        const float rz = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
-        const float da = dsx * rz, db = dsy * rz, dc = -(s_ds * rz);
-        g[0] = w * dLp0, g[1] = w * dLp1, g[2] = w * dLp2;
-        g[3] = da * pxf, g[4] = da * pyf, g[5] = da;
-        g[6] = db * pxf, g[7] = db * pyf, g[8] = db;
-        g[9] = dc * pxf, g[10] = dc * pyf, g[11] = dc;
-        if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
-        else      g[12] = g[13] = g[14] = 0.0f;
-        g[15] = GdA;
-        const float to_centre = filtered ? -2.0f * oG : 0.0f;
-        g5[0] = z_sx, g5[1] = z_sy, g5[2] = dL_dz;
-        g5[3] = to_centre * h.dx, g5[4] = to_centre * h.dy;
-        const float tot = row_sum16_transposed(g), tot5 = row_sum5_transposed(g5);
-        if (j != kB) {
-          sums[i * kFastGradSlots] = tot;
-          if ((lane & 1) == 0) sums2[i * kFastGradSlots] = tot5;
-        }
-    };
-    walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
-                    [] { return true; });
-    __syncthreads();
-    // Flush the batch: add the sums of the rows that hold an entry, in row order.
-    if (kSlots) {
-      // two lanes per entry, eleven of the record's floats each (component 10 is summed by both)
-      static_assert(kBlendThreads == 2 * kB && kFastGradSlots == 21 && kFastRecordSlots == 22);
-      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
-        const int h = (int) threadIdx.x & 1;
-        float a[11];
-        sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], 10 * h, a);
-        float* dst = slot_records + (size_t) s_slot[parity][e] * kFastRecordSlots + 11 * h;
+        dL_dalpha = c_lin - acc_lin;
+        acc_lin   = fmaf(1.0f - h.alpha, acc_lin, h.alpha * c_lin);
+        dL_dalpha *= T;
+      };
+
+      const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+      float* const sums  = &s_sum[place][lane & 15];  // component lane & 15 of the row's first place
+      float* const sums2 = &s_sum[place][16 + ((lane & 2) ? 4 : (lane >> 2 & 1) * 2 + (lane >> 3 & 1))];
+      auto blend_entry = [&](const FastHot& hot, int j, int i) {
+          const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
+          __builtin_amdgcn_sched_barrier(0);
+          FastHit h;
+          unsigned long long pass;
+          fast_intersect_flat(hot, pxf, pyf, near_n, h, &pass);
+          pass &= wave_ballot(j >= my_first);
+          if (pass == 0ull) {
+            if (j != kB) {  // not a padding step; zeros, too, have their place
+              sums[i * kFastGradSlots] = 0.0f;
+              if ((lane & 1) == 0) sums2[i * kFastGradSlots] = 0.0f;
+            }
+            return;
+          }
+          const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
+          float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, fsx = 0.0f, fsy = 0.0f;
+          // The part under `hit` leaves a few factors (zero in a lane whose pixel does not blend the entry); the components are
+          // products of those factors with quantities that are finite in every lane, formed by all lanes alike: no
+          // component needs a zero of its own, and the projected-centre case is the intersection case with a zero in
+          // place of 1 / p_z.
+          float g[16], g5[5];
+          float GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
+          if (hit) {
+            advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, fsx, fsy);
+            // d/ds of the intersection case (times 1 / p_z below); s is not finite in a lane whose p_z is 0, and such a
+            // lane never blends: every use of s sits on this side
+            GdA  = dL_dalpha * h.G;
+            oG   = hot.opacity * GdA;
+            dsx  = fsx - oG * h.sx, dsy = fsy - oG * h.sy;
+            if (kAux) dsx += dL_dz * hot.tw0, dsy += dL_dz * hot.tw1;
+            s_ds = dsx * h.sx + dsy * h.sy;
+            z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
+          }
+          const bool by_ray   = h.rho3d <= h.rho2d;
+          const bool filtered = hit && !by_ray;
+          const float rz = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
+          const float da = dsx * rz, db = dsy * rz, dc = -(s_ds * rz);
+          g[0] = w * dLp0, g[1] = w * dLp1, g[2] = w * dLp2;
+          g[3] = da * pxf, g[4] = da * pyf, g[5] = da;
+          g[6] = db * pxf, g[7] = db * pyf, g[8] = db;
+          g[9] = dc * pxf, g[10] = dc * pyf, g[11] = dc;
+          if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
+          else      g[12] = g[13] = g[14] = 0.0f;
+          g[15] = GdA;
+          const float to_centre = filtered ? -2.0f * oG : 0.0f;
+          g5[0] = z_sx, g5[1] = z_sy, g5[2] = dL_dz;
+          g5[3] = to_centre * h.dx, g5[4] = to_centre * h.dy;
+          const float tot = row_sum16_transposed(g), tot5 = row_sum5_transposed(g5);
+          if (j != kB) {
+            sums[i * kFastGradSlots] = tot;
+            if ((lane & 1) == 0) sums2[i * kFastGradSlots] = tot5;
+          }
+      };
+      if (base > 0) __syncthreads();  // the sums of the batch before have been read
+      walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
+                      [] { return true; });
+      __syncthreads();
+      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      if (kSlots) {
+        // two lanes per entry, eleven of the record's floats each (component 10 is summed by both)
+        static_assert(kBlendThreads == 2 * kB && kFastGradSlots == 21 && kFastRecordSlots == 22);
+        if (const int e = base + ((int) threadIdx.x >> 1); e < end) {
+          const int h = (int) threadIdx.x & 1;
+          float a[11];
+          sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], 10 * h, a);
+          float* dst = slot_records + (size_t) s_slot[parity][e] * kFastRecordSlots + 11 * h;
 #pragma unroll
-        for (int c = 0; c < 11; ++c) dst[c] = h == 0 ? a[c] : c < 10 ? a[c < 10 ? c + 1 : 0] : 0.0f;
+          for (int c = 0; c < 11; ++c) dst[c] = h == 0 ? a[c] : c < 10 ? a[c < 10 ? c + 1 : 0] : 0.0f;
+        }
+      } else {
+        // one global atomic per surfel and component for this tile, a lane per component
+        for (int t = (int) threadIdx.x; t < (end - base) * kFastGradSlots; t += kBlendThreads) {
+          const int q = t / kFastGradSlots, c = t - q * kFastGradSlots, e = base + q, id = s_slot[parity][e];
+          float a[1];
+          sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
+          float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
+                             : c < 12 ? g_inv + 9 * (size_t) id + (c - 3)
+                             : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
+                             : c < 19 ? g_trans + 9 * (size_t) id + 6 + (c - 16)
+                                      : g_means2D + 2 * (size_t) id + (c - 19);
+          if (a[0] != 0.0f) atomicAdd(out, a[0]);
+        }
       }
-    } else {
-      // one global atomic per surfel and component for this tile, a lane per component
-      for (int t = (int) threadIdx.x; t < n_here * kFastGradSlots; t += kBlendThreads) {
-        const int e = t / kFastGradSlots, c = t - e * kFastGradSlots, id = s_slot[parity][e];
-        float a[1];
-        sum_places<kFastGradSlots>(&s_sum[0][0], s_place[parity][e], c, a);
-        float* const out = c < 3    ? g_colors + 3 * (size_t) id + c
-                           : c < 12 ? g_inv + 9 * (size_t) id + (c - 3)
-                           : c < 16 ? g_normal_opacity + 4 * (size_t) id + (c - 12)
-                           : c < 19 ? g_trans + 9 * (size_t) id + 6 + (c - 16)
-                                    : g_means2D + 2 * (size_t) id + (c - 19);
-        if (a[0] != 0.0f) atomicAdd(out, a[0]);
-      }
+      base = end;
     }
-    done += n_here;
+    done += base;
     // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
     // records, which nobody reads before, and the other copy of what the flush reads.
   }

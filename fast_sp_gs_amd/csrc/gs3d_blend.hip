@@ -443,6 +443,7 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
     float* __restrict__ g_extras, const int64_t* __restrict__ point_offsets, const int32_t* __restrict__ radii,
     float* __restrict__ slot_records, const uint32_t* __restrict__ hit_blocks) {
   constexpr int kB = kRowBatch, kRowPlaces = 255;
+  constexpr bool kRewalk = !kHits;  // several batches per staging (kRewalkBelow); with the notes 300k Gaussians take 2 % more by it
   using Shape = BlockShape<16>;
   // components that cross the lanes: 0-2 colour | 3-6 extras | 7-8 mean2D | 9-11 conic | 12 opacity, without extras close up
   constexpr bool kNine = E == 0;
@@ -480,7 +481,7 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
   if (threadIdx.x < 4) ((unsigned*) &s_list[16 * kB])[threadIdx.x] = 0u;
   if (threadIdx.x < kSums) s_sum[kRowPlaces][threadIdx.x] = 0.0f;
   __syncthreads();
-  const int n_todo = min(s_max_contrib, (int) (r1 - r0));
+  const int n_todo = __builtin_amdgcn_readfirstlane(min(s_max_contrib, (int) (r1 - r0)));
   // No zero fill of the record buffer: every staged instance writes its record at the flush, zeros included, and the
   // instances behind the tile's deepest contributor, which are never staged, are cleared here.
   if (kSlots) {
@@ -509,7 +510,7 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
   unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
-  // entry e of the batch that starts behind `done` entries, counted from the back of the list
+  // entry e of the 128 staged behind `done` entries, counted from the back of the list
   auto gather = [&](int done) {
     const int e = (int) threadIdx.x;
     if (e >= min(kB, n_todo - done)) return;
@@ -540,139 +541,149 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
       s_mask[e] = mask;
     }
     __syncthreads();
-    const unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
-    int start, before[4];
-    const int n_here = row_batch<kRowPlaces>(masks, n_staged, wave, start);
-    gather(done + n_here);
-    // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
-    const int behind = n_todo - done;
-    const int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
-    const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
-                                      n_here);
-    const int my_first = behind - last_contrib;
-    // component that this lane stores, and its place of step 0
-    const int my_part = !kNine ? lane & 15 : (lane & 1) ? 8 : (lane >> 3 & 1) * 4 + (lane >> 2 & 1) * 2 + (lane >> 1 & 1);
-    const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
-    float* const sums = &s_sum[place][my_part];
-    auto entry = [&](const G3Splat<E>& splat, int j, int i) {
-      G3Hit h;
-      unsigned long long pass;
-      conic_alpha_flat(splat, pxf, pyf, h, &pass);
-      pass &= wave_ballot(j >= my_first);
-      if (pass == 0ull) {
-        if (j != kB) sums[i * kSums] = 0.0f;  // not a padding step; zeros, too, have their place
-        return;
-      }
-      const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
-      // Under `hit`: the pixel's back-to-front state and two factors (zero in a lane that does not blend the entry). The
-      // components are their products with quantities that are finite in every lane, formed by all lanes alike, so none
-      // needs a zero of its own.
-      float g[kSums];
-      float dch = 0.0f, GdA = 0.0f;
-      if (hit) {
-        T   = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
-        dch = h.alpha * T;
-        float dL_dalpha = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 3 + E; ++k) {
-          const float v = splat.feat[k];
-          dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
-          accum[k] += v * dch;
+    unsigned masks[2] = {s_mask[lane], s_mask[kWave + lane]};
+    const RowCounts counts(masks, wave);
+    int base = 0;  // staged entries of the batches before
+    for (bool more = true; more;) {
+      int start, before[4];
+      const int end = row_batch<kRowPlaces>(counts, base, n_staged, start);
+      if (kRewalk) masks[0] = s_mask[lane], masks[1] = s_mask[kWave + lane];  // read again rather than kept through the walk
+      more = kRewalk && end - base < kRewalkBelow && end < n_staged;
+      if (!more) gather(done + end);
+      // Entry j of the batch is position n_todo - 1 - done - j of the list; a pixel takes part from its deepest contributor on.
+      const int behind = n_todo - done;
+      int first[4] = {behind - row_last[0], behind - row_last[1], behind - row_last[2], behind - row_last[3]};
+      if (kRewalk) for (int& f : first) f = max(f, base);
+      const int steps = build_row_lists(&s_list[4 * kB * wave], (unsigned char*) s_place[parity], masks, wave, first, start, before,
+                                        end);
+      const int my_first = behind - last_contrib;
+      // component that this lane stores, and its place of step 0
+      const int my_part = !kNine ? lane & 15 : (lane & 1) ? 8 : (lane >> 3 & 1) * 4 + (lane >> 2 & 1) * 2 + (lane >> 1 & 1);
+      const int row = lane >> 4, place = row == 0 ? before[0] : row == 1 ? before[1] : row == 2 ? before[2] : before[3];
+      float* const sums = &s_sum[place][my_part];
+      auto entry = [&](const G3Splat<E>& splat, int j, int i) {
+        G3Hit h;
+        unsigned long long pass;
+        conic_alpha_flat(splat, pxf, pyf, h, &pass);
+        pass &= wave_ballot(j >= my_first);
+        if (pass == 0ull) {
+          if (j != kB) sums[i * kSums] = 0.0f;  // not a padding step; zeros, too, have their place
+          return;
         }
-        GdA = (dL_dalpha - T_final * dL_dT) * __builtin_amdgcn_rcpf(1.0f - h.alpha) * h.G;
-      }
-      if (!kNine) {
+        const bool hit = __builtin_amdgcn_inverse_ballot_w64(pass);
+        // Under `hit`: the pixel's back-to-front state and two factors (zero in a lane that does not blend the entry). The
+        // components are their products with quantities that are finite in every lane, formed by all lanes alike, so none
+        // needs a zero of its own.
+        float g[kSums];
+        float dch = 0.0f, GdA = 0.0f;
+        if (hit) {
+          T   = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
+          dch = h.alpha * T;
+          float dL_dalpha = 0.0f;
 #pragma unroll
-        for (int c = 0; c < kSums; ++c) g[c] = 0.0f;
-      }
+          for (int k = 0; k < 3 + E; ++k) {
+            const float v = splat.feat[k];
+            dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
+            accum[k] += v * dch;
+          }
+          GdA = (dL_dalpha - T_final * dL_dT) * __builtin_amdgcn_rcpf(1.0f - h.alpha) * h.G;
+        }
+        if (!kNine) {
 #pragma unroll
-      for (int k = 0; k < 3 + E; ++k) g[k] = dch * g_out[k];
-      // the geometry's part without the factor -opacity
-      g[kGeom]     = GdA * (splat.a * h.dx + splat.b * h.dy);
-      g[kGeom + 1] = GdA * (splat.c * h.dy + splat.b * h.dx);
-      g[kGeom + 2] = h.dx * h.dx * GdA;
-      g[kGeom + 3] = h.dx * h.dy * GdA;
-      g[kGeom + 4] = h.dy * h.dy * GdA;
-      g[kGeom + 5] = GdA;
-      float tot;
-      if constexpr (kNine) tot = row_sum9_transposed(g);
-      else tot = row_sum16_transposed(g);
-      if (j != kB) sums[i * kSums] = tot;
-    };
-    walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j]; }, entry,
-                    [] { return true; });
-    __syncthreads();
-    // Flush the batch: add the sums of the rows that hold an entry, in row order.
-    if (kSlots && kNine) {
-      // two lanes per entry, half of its record's sixteen floats each; the geometry's part still lacks the factor -opacity
-      static_assert(kBlendThreads == 2 * kB && kG3Slots == 16);
-      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
-        const bool upper = threadIdx.x & 1;
-        float a[5];
-        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], upper ? 4 : 0, a);
-        const float2 tag = s_tag[parity][e];
-        const float no = -tag.y;
-        // lower half: colour, mean x; upper half: mean y, conic, opacity
-        float4* dst = (float4*) (slot_records + (size_t) __float_as_int(tag.x) * kG3Slots) + (upper ? 2 : 0);
-        dst[0] = upper ? make_float4(no * a[0], 0.5f * no * a[1], no * a[2], 0.5f * no * a[3]) : make_float4(a[0], a[1], a[2], 0.0f);
-        dst[1] = upper ? make_float4(a[4], 0.0f, 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, no * a[3]);
-      }
-    } else if (kSlots) {
-      // a lane per component of the record
-      for (int t = (int) threadIdx.x; t < n_here * kG3Slots; t += kBlendThreads) {
-        const int e = t / kG3Slots, c = t % kG3Slots;
-        float a[1];
-        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
-        const float2 tag  = s_tag[parity][e];
-        const float scale = c < kGeom || c > kGeom + 4 ? 1.0f : c == kGeom + 2 || c == kGeom + 4 ? -0.5f * tag.y : -tag.y;
-        slot_records[(size_t) __float_as_int(tag.x) * kG3Slots + c] = scale * a[0];
-      }
-    } else if (kNine && kHits) {
-      // Two lanes per entry add its rows; a wavefront keeps the totals of its 32 entries and adds them to the tensors with
-      // sixteen lanes per entry, a component each: three requests (a line per gradient tensor).
-      if (const int e = (int) threadIdx.x >> 1; e < n_here) {
-        const int h = (int) threadIdx.x & 1;
-        float a[5];
-        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], 4 * h, a);
+          for (int c = 0; c < kSums; ++c) g[c] = 0.0f;
+        }
 #pragma unroll
-        for (int c = 0; c < 5; ++c) s_total[e][4 * h + c] = a[c];
-      }
-      wave_lds_sync();  // the two lanes of an entry write what the sixteen below read
-      const int c = (int) threadIdx.x & 15, g = c - kGeom;  // component, and its number among the geometry's six
-      if (c < kSums) {
-        float* const out = c < 3 ? g_colors + c : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
-        const size_t row = c < 3 ? 3 : g < 2 ? 2 : 4;
-        for (int k = 0; k < kB / 16; ++k) {
-          const int e = wave * (kB / 4) + 4 * k + (lane >> 4);
-          if (e >= n_here) break;
-          float sum = s_total[e][c];
+        for (int k = 0; k < 3 + E; ++k) g[k] = dch * g_out[k];
+        // the geometry's part without the factor -opacity
+        g[kGeom]     = GdA * (splat.a * h.dx + splat.b * h.dy);
+        g[kGeom + 1] = GdA * (splat.c * h.dy + splat.b * h.dx);
+        g[kGeom + 2] = h.dx * h.dx * GdA;
+        g[kGeom + 3] = h.dx * h.dy * GdA;
+        g[kGeom + 4] = h.dy * h.dy * GdA;
+        g[kGeom + 5] = GdA;
+        float tot;
+        if constexpr (kNine) tot = row_sum9_transposed(g);
+        else tot = row_sum16_transposed(g);
+        if (j != kB) sums[i * kSums] = tot;
+      };
+      if (kRewalk && base > 0) __syncthreads();  // the sums of the batch before have been read
+      walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j]; }, entry,
+                      [] { return true; });
+      __syncthreads();
+      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      if (kSlots && kNine) {
+        // two lanes per entry, half of its record's sixteen floats each; the geometry's part still lacks the factor -opacity
+        static_assert(kBlendThreads == 2 * kB && kG3Slots == 16);
+        if (const int e = base + ((int) threadIdx.x >> 1); e < end) {
+          const bool upper = threadIdx.x & 1;
+          float a[5];
+          sum_places<kSums>(&s_sum[0][0], s_place[parity][e], upper ? 4 : 0, a);
           const float2 tag = s_tag[parity][e];
+          const float no = -tag.y;
+          // lower half: colour, mean x; upper half: mean y, conic, opacity
+          float4* dst = (float4*) (slot_records + (size_t) __float_as_int(tag.x) * kG3Slots) + (upper ? 2 : 0);
+          dst[0] = upper ? make_float4(no * a[0], 0.5f * no * a[1], no * a[2], 0.5f * no * a[3]) : make_float4(a[0], a[1], a[2], 0.0f);
+          dst[1] = upper ? make_float4(a[4], 0.0f, 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, no * a[3]);
+        }
+      } else if (kSlots) {
+        // a lane per component of the record
+        for (int t = (int) threadIdx.x; t < (end - base) * kG3Slots; t += kBlendThreads) {
+          const int e = base + t / kG3Slots, c = t % kG3Slots;
+          float a[1];
+          sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
+          const float2 tag  = s_tag[parity][e];
+          const float scale = c < kGeom || c > kGeom + 4 ? 1.0f : c == kGeom + 2 || c == kGeom + 4 ? -0.5f * tag.y : -tag.y;
+          slot_records[(size_t) __float_as_int(tag.x) * kG3Slots + c] = scale * a[0];
+        }
+      } else if (kNine && kHits) {
+        // One batch per staging: base is 0. Two lanes per entry add its rows; a wavefront keeps the totals of its 32 entries
+        // and adds them to the tensors with sixteen lanes per entry, a component each: three requests (a line per gradient
+        // tensor).
+        if (const int e = (int) threadIdx.x >> 1; e < end) {
+          const int h = (int) threadIdx.x & 1;
+          float a[5];
+          sum_places<kSums>(&s_sum[0][0], s_place[parity][e], 4 * h, a);
+#pragma unroll
+          for (int c = 0; c < 5; ++c) s_total[e][4 * h + c] = a[c];
+        }
+        wave_lds_sync();  // the two lanes of an entry write what the sixteen below read
+        const int c = (int) threadIdx.x & 15, g = c - kGeom;  // component, and its number among the geometry's six
+        if (c < kSums) {
+          float* const out = c < 3 ? g_colors + c : g < 2 ? g_means2D + g : g_conic_opacity + (g - 2);
+          const size_t row = c < 3 ? 3 : g < 2 ? 2 : 4;
+          for (int k = 0; k < kB / 16; ++k) {
+            const int e = wave * (kB / 4) + 4 * k + (lane >> 4);
+            if (e >= end) break;
+            float sum = s_total[e][c];
+            const float2 tag = s_tag[parity][e];
+            if (g >= 0 && g < 5) sum *= -tag.y;
+            if (g == 2 || g == 4) sum *= 0.5f;
+            if (sum != 0.0f) atomicAdd(out + row * (size_t) __float_as_int(tag.x), sum);
+          }
+        }
+      } else {
+        // one global atomic per Gaussian and component for this tile, a lane per component
+        constexpr int kUsed = kNine ? kSums : 13;
+        for (int t = (int) threadIdx.x; t < (end - base) * kUsed; t += kBlendThreads) {
+          const int q = t / kUsed, c = t - q * kUsed, e = base + q, g = c - kGeom;  // g: number among the geometry's six
+          if (c >= 3 + E && g < 0) continue;
+          float a[1];
+          sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
+          const float2 tag = s_tag[parity][e];
+          const size_t id  = (size_t) __float_as_int(tag.x);
+          float* const out = c < 3       ? g_colors + 3 * id + c
+                             : c < 3 + E ? g_extras + E * id + (c - 3)
+                             : g < 2     ? g_means2D + 2 * id + g
+                                         : g_conic_opacity + 4 * id + (g - 2);
+          float sum = a[0];
           if (g >= 0 && g < 5) sum *= -tag.y;
           if (g == 2 || g == 4) sum *= 0.5f;
-          if (sum != 0.0f) atomicAdd(out + row * (size_t) __float_as_int(tag.x), sum);
+          if (sum != 0.0f) atomicAdd(out, sum);
         }
       }
-    } else {
-      // one global atomic per Gaussian and component for this tile, a lane per component
-      constexpr int kUsed = kNine ? kSums : 13;
-      for (int t = (int) threadIdx.x; t < n_here * kUsed; t += kBlendThreads) {
-        const int e = t / kUsed, c = t - e * kUsed, g = c - kGeom;  // g: number among the geometry's six
-        if (c >= 3 + E && g < 0) continue;
-        float a[1];
-        sum_places<kSums>(&s_sum[0][0], s_place[parity][e], c, a);
-        const float2 tag = s_tag[parity][e];
-        const size_t id  = (size_t) __float_as_int(tag.x);
-        float* const out = c < 3       ? g_colors + 3 * id + c
-                           : c < 3 + E ? g_extras + E * id + (c - 3)
-                           : g < 2     ? g_means2D + 2 * id + g
-                                       : g_conic_opacity + 4 * id + (g - 2);
-        float sum = a[0];
-        if (g >= 0 && g < 5) sum *= -tag.y;
-        if (g == 2 || g == 4) sum *= 0.5f;
-        if (sum != 0.0f) atomicAdd(out, sum);
-      }
+      base = end;
     }
-    done += n_here;
+    done += base;
     // No barrier needed here: until the barrier behind the next batch's staging, a wavefront that has flushed touches the
     // Gaussians, which nobody reads before, and the other copy of what the flush reads.
   }
