@@ -807,13 +807,16 @@ __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned*
 // LDS round trips and five barriers, whatever n is, where the network takes 33 rounds and 7 barriers for 2048 entries: against
 // the network (merging up to 256 entries), 400k surfels 3840x2160 153 -> 41 us, 3M 1352x1014 62 -> 18, 300k 800x800 24 -> 7.6,
 // 300k Gaussians 29 -> 7.9, 150k 1001x667 9.2 -> 4.6, 10k 256x256 5.1 -> 3.7. With depths in two thin shells, which take the
-// second cut, 1100 entries a tile in 2500 tiles: 140 -> 94..124 us for the whole binning, 200 entries a tile: alike.
+// second cut, 1100 entries a tile in 2500 tiles: 140 -> 87..116 us for the whole binning, 200 entries a tile: alike. With one depth for
+// all, or one of two, 1100 a tile: 67 -> 19 and 25 us, 80 a tile: 7.1 and 8.0, as by merging (a count of all in one counter, twice, and
+// the network behind it took 89 and 81, 10.5 and 9.8).
 // The buckets cut the span of the
 // segment's depth bits into equal parts, so they are in order among themselves; an entry's place is its bucket's start plus the
 // number of smaller entries in the bucket (all 64 bits compared), a few when the depths spread. When some bucket holds more
 // than kBucketLimit entries (surfaces at a few depths, a far outlier), every bucket is cut once more into as many parts as it
-// has entries. False, with nothing written and the keys in `key`, when that leaves too many together as well (equal depths):
-// the comparing sorts take such a segment.
+// has entries, by its depths, or, if it holds a single one, by the surfels' numbers, which decide among equal depths. (To find those
+// buckets costs segments without one about 2 us of the 116.) False, with nothing written and the keys in `key`, when that leaves too
+// many together as well (numbers in clumps, half a bucket at one depth): the comparing sorts take such a segment.
 template <int kPer>
 __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, const uint64_t* __restrict__ entries,
                                             uint64_t (&key)[kPer], uint64_t* s_e, int32_t* __restrict__ point_list,
@@ -845,11 +848,15 @@ __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, cons
     if (keys_out) keys_out[start + to] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
   };
   unsigned rank[kPer];
+  const bool one_depth = __builtin_amdgcn_readfirstlane(hi - lo) == 0 && n > kBucketLimit;  // every entry would wait for the one counter, to no end
+  if (!one_depth) {
 #pragma unroll
-  for (int q = 0; q < kPer; ++q)
-    if ((int) threadIdx.x + 256 * q < n) rank[q] = atomicAdd(&s_count[bucket(key[q])], 1u);
+    for (int q = 0; q < kPer; ++q)
+      if ((int) threadIdx.x + 256 * q < n) rank[q] = atomicAdd(&s_count[bucket(key[q])], 1u);
+  }
   __syncthreads();
-  if (prefix_counters<kOwn, 1>(s_count, s_wave) <= (unsigned) kBucketLimit) {
+  const unsigned most = one_depth ? (unsigned) n : prefix_counters<kOwn, 1>(s_count, s_wave);
+  if (__builtin_amdgcn_readfirstlane(most) <= (unsigned) kBucketLimit) {
 #pragma unroll
     for (int q = 0; q < kPer; ++q)
       if ((int) threadIdx.x + 256 * q < n) s_e[s_count[bucket(key[q])] + rank[q]] = key[q];
@@ -866,14 +873,40 @@ __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, cons
     }
     return true;
   }
-  // part `fine` of n, 16-bit counters in the same words
+  // A bucket is cut by its depths, or, if it holds one depth only, by the surfels' numbers, which come next in the order: over the
+  // span of the segment's numbers. Any entry of a bucket names its depth, an entry with another one marks the bucket.
+  unsigned* s_depth = s_wave + 16;
+  unsigned* s_mixed = s_depth + kBuckets;
+  unsigned id_lo = 0u, id_hi = 0u;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) id_lo = max(id_lo, ~(unsigned) key[q]), id_hi = max(id_hi, (unsigned) key[q]);
+  id_lo = wave_max_to_last(id_lo), id_hi = wave_max_to_last(id_hi);
+  if ((threadIdx.x & 63) == 63) s_wave[8 + 2 * wave] = id_lo, s_wave[9 + 2 * wave] = id_hi;
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) s_mixed[kOwn * threadIdx.x + c] = 0u;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) s_depth[bucket(key[q])] = (unsigned) (key[q] >> 32);
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) id_lo = max(id_lo, s_wave[8 + 2 * w]), id_hi = max(id_hi, s_wave[9 + 2 * w]);
+  id_lo = ~id_lo;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int b = bucket(key[q]);
+    if (s_depth[b] != (unsigned) (key[q] >> 32)) s_mixed[b] = 1u;
+  }
+  __syncthreads();
+  const float id_scale = __builtin_amdgcn_rcpf((float) (id_hi - id_lo) + 1.0f);
+  // part `fine` of n, 16-bit counters in the counters' words
   constexpr int kOwnFine = kPer == 1 ? 1 : kPer / 2;
   uint16_t* s_fine = (uint16_t*) s_count;
   int fine[kPer];
 #pragma unroll
   for (int q = 0; q < kPer; ++q) {
-    const int b = bucket(key[q]), first = s_count[b], held = (b + 1 < kBuckets ? (int) s_count[b + 1] : n) - first;
-    fine[q] = first + min((int) ((place(key[q]) - (float) b) * (float) held), max(held - 1, 0));
+    const int b = bucket(key[q]), first = one_depth ? 0 : (int) s_count[b];
+    const int held = (one_depth || b + 1 == kBuckets ? n : (int) s_count[b + 1]) - first;
+    const float part = s_mixed[b] ? place(key[q]) - (float) b : (float) ((unsigned) key[q] - id_lo) * id_scale;
+    fine[q] = first + min((int) (part * (float) held), max(held - 1, 0));
   }
   __syncthreads();
 #pragma unroll

@@ -46,3 +46,31 @@ def test_list_of_one_tile_by_buckets(n, depths, device, oracle_mod):
                                                     touched.to(device), False, return_keys=True)[:3]
     want_ranges, want_pl, want_keys = oracle_mod.prepare(16, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
     assert np.array_equal(npy(ranges), want_ranges) and np.array_equal(npy(pl), want_pl) and np.array_equal(npy(keys), want_keys)
+
+
+@pytest.mark.parametrize('n', [2, 33, 200, 256, 257, 700, 1025, 2048])
+@pytest.mark.parametrize('depths', ['one', 'two', 'one of many', 'shells'])
+def test_equal_depths_in_one_of_two_tiles(n, depths, device, oracle_mod):
+    """Equal depths are put in order by the surfels' numbers: spread over the tile's span of numbers, or in two clumps of it (the
+    cut by numbers then fills a few parts only). `one of many`: one bucket of many depths holds one depth a hundred times;
+    `shells`: buckets of several depths beside buckets of one."""
+    from fast_sp_gs_amd._C import get_C_function
+    print(f'[tile sort] n={n} equal depths: {depths}', flush=True)
+    g = torch.Generator().manual_seed(n)
+    for clumped in (False, True):
+        P = 20 * n
+        here = torch.zeros(P, dtype=torch.bool)
+        here[torch.cat([torch.arange(n // 2), P - 1 - torch.arange(n - n // 2)]) if clumped else torch.randperm(P, generator=g)[:n]] = True
+        r = torch.rand(P, generator=g)
+        dep = {'one': torch.full((P,), 3.0), 'two': torch.randint(3, 5, (P,), generator=g).float(),
+               'one of many': torch.where(r < 0.3, torch.full((P,), 2.0), 1.0 + 4.0 * r),
+               'shells': torch.where(r < 0.5, torch.full((P,), 3.0), 4.0 + 1e-4 * r)}[depths]
+        m2 = torch.stack([torch.where(here, 8.0, 24.0), torch.full((P,), 8.0)], 1).contiguous()
+        keep = here | (torch.rand(P, generator=g) < 0.02)  # a few in the other tile
+        radii, touched = torch.where(keep, 3, 0).int(), keep.int()
+        ranges, pl, keys = get_C_function('GS_prepare')(32, 16, m2.to(device), dep.to(device), radii.to(device),
+                                                        touched.to(device), False, return_keys=True)[:3]
+        want = oracle_mod.prepare(32, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
+        assert want[0][0, 1] - want[0][0, 0] == n
+        for a, b in zip((ranges, pl, keys), want):
+            assert np.array_equal(npy(a), b)
