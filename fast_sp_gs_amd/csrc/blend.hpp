@@ -219,21 +219,15 @@ __device__ __forceinline__ unsigned quadrant_mask(const SplatHot& h, int tile_px
 // The table is kMaxOrderedTiles ints in a file-scope device array of the library (no allocation), one slot per
 // (device, stream) that bins or blends: calls on one stream are ordered by the stream, calls on different streams use
 // different tables, and a stream that finds every slot taken runs without a table.
-#ifndef FSGS_ORDER_FRAC_BITS
-#define FSGS_ORDER_FRAC_BITS 4
-#endif
-#ifndef FSGS_ORDER_BALANCE_ROUNDS
-#define FSGS_ORDER_BALANCE_ROUNDS 4
-#endif
 constexpr int kMaxOrderedTiles = 1 << 16;
-constexpr int kOrderFracBits   = FSGS_ORDER_FRAC_BITS;  // buckets per octave of list length = 2^this
+constexpr int kOrderFracBits   = 4;  // buckets per octave of list length = 2^this
 constexpr int kOrderFrac       = 1 << kOrderFracBits;
 constexpr int kOrderBuckets    = 32 * kOrderFrac;
 constexpr int kOrderRegions    = 8;
 constexpr int kCusPerXcd       = 32;  // compute units behind one region's table positions
 // rounds of a region's list whose tiles are dealt by CU load: the blocks of the blend backward that fit on a CU (4,
 // bounded by its 128 registers per lane); measured best among 3, 4, 5, 6, 8, 16
-constexpr int kBalanceRounds   = FSGS_ORDER_BALANCE_ROUNDS;
+constexpr int kBalanceRounds   = 4;
 
 // (tile_order_table, tile_order_invalidate and tile_order_release are declared in common.hpp.)
 
@@ -248,16 +242,14 @@ __device__ __forceinline__ int length_bucket(int64_t len64) {
   return 1 + m * kOrderFrac + frac;  // <= 31 * kOrderFrac
 }
 
-#ifndef FSGS_TILE_GROUP
-#define FSGS_TILE_GROUP 2
-#endif
-// Groups of FSGS_TILE_GROUP x FSGS_TILE_GROUP tiles are dealt to the 8 regions in a skewed pattern, so every region is a
+constexpr int kTileGroup = 2;
+// Groups of kTileGroup x kTileGroup tiles are dealt to the 8 regions in a skewed pattern, so every region is a
 // fine-grained sample of the whole image (equal load whatever the scene's layout) while direct neighbours mostly share
 // a region.
 __device__ __forceinline__ int tile_region(int t, int gx, int gy) {
   const int tx = t % gx, ty = t / gx;
   (void) gy;
-  return ((tx / FSGS_TILE_GROUP) + 3 * (ty / FSGS_TILE_GROUP)) & (kOrderRegions - 1);
+  return ((tx / kTileGroup) + 3 * (ty / kTileGroup)) & (kOrderRegions - 1);
 }
 
 // LDS of one block that builds a table (24.6 KB)
@@ -458,18 +450,12 @@ __device__ __forceinline__ void argmax_run_step(ArgmaxRun& a, float w, int id, i
 // same for the halves. Written as inline assembly because the compiler's builtin for these instructions returns the
 // first result twice; the s_nop cover the VALU-write -> swap-read wait states the compiler would insert itself.
 __device__ __forceinline__ float cross_row_sum(float z) {
-#ifdef FSGS_NO_PERMLANE_SWAP
-  z += __shfl_xor(z, 16, kWave);
-  z += __shfl_xor(z, 32, kWave);
-  return z;
-#else
   float a = z, b = z;
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
   z = a + b;
   a = z, b = z;
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
   return a + b;
-#endif
 }
 
 // Sums 16 per-lane values over each 16-lane row at once ("transposed" butterfly): every step halves the number of live

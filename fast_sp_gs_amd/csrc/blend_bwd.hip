@@ -33,12 +33,9 @@ namespace {
 // The first 16 go through one transposed row reduction; the means2D pair is only non-zero for pixels where the
 // screen-space low-pass filter wins (rho2d < rho3d) and is reduced separately when any lane took that branch.
 constexpr int kGradSlots = 18;
-#ifndef FSGS_BWD_WAVES
-#define FSGS_BWD_WAVES 4
-#endif
 
 template <bool kAux, bool kFlow, bool kSlots>
-__global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(FSGS_BWD_WAVES, FSGS_BWD_WAVES)))
+__global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 blend_backward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
     const int32_t* __restrict__ n_contrib, const float2* __restrict__ means2D,

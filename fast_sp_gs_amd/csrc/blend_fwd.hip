@@ -22,14 +22,8 @@
 namespace fsgs {
 namespace {
 
-#ifndef FSGS_FWD_BATCH
-#define FSGS_FWD_BATCH 192
-#endif
-#ifndef FSGS_FWD_LANES
-#define FSGS_FWD_LANES 8
-#endif
-constexpr int kFwdLanes = FSGS_FWD_LANES;  // lanes (pixels) that share a work list
-constexpr int kFwdBatch = FSGS_FWD_BATCH;  // surfels staged per round (<= block size)
+constexpr int kFwdLanes = 8;    // lanes (pixels) that share a work list
+constexpr int kFwdBatch = 192;  // surfels staged per round (<= block size)
 
 // kAccum: 0 = no side outputs, 1 = accum_max_count only (what the reference's training loop passes on every step),
 // 2 = accum_weights_p and / or accum_weights_count as well.
@@ -45,6 +39,7 @@ blend_forward_kernel(
     float2* __restrict__ out_flow, int32_t* __restrict__ accum_max_count, float* __restrict__ accum_weights_p,
     int32_t* __restrict__ accum_weights_count, uint32_t* __restrict__ hit_blocks, ViewMaps maps) {
   using Shape = BlockShape<kFwdLanes>;
+  static_assert(!kHits || kFwdLanes == kHitLanes);
   __shared__ Splat s_splat[kFwdBatch + 1];  // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kFwdBatch * 9 : 1];
   __shared__ unsigned s_mask[kFwdBatch];  // which blocks of the tile each staged surfel can reach

@@ -224,6 +224,9 @@ __device__ __forceinline__ void walk_block_list(const unsigned char* __restrict_
 // A forward kernel (2x4 blocks) can note, per staged entry, the blocks with a pixel that blended it, a byte per block; the
 // backward then walks exactly these instead of bounding every footprint again. Block b's byte is b ^ 3: the product below
 // gathers the low bits of four bytes, the last byte's first.
+constexpr int kHitLanes = 8;  // of a noted block: 32 blocks a tile, which pair_blocks joins to the backward's 4x4
+static_assert(BlockShape<kHitLanes>::kPerTile == 32);
+
 __device__ __forceinline__ unsigned hit_bits(const uint4& lo, const uint4& hi) {
   const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
   unsigned m = 0u;

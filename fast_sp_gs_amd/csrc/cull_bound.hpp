@@ -5,10 +5,7 @@
 
 namespace fsgs {
 
-#ifndef FSGS_CULL_PAD
-#define FSGS_CULL_PAD 0.125f
-#endif
-constexpr float kCullPad = FSGS_CULL_PAD;  // pixels added around the footprint box against rounding
+constexpr float kCullPad = 0.125f;  // pixels added around the footprint box against rounding
 
 // A pixel can only blend a surfel where alpha = min(0.99, o exp(-rho / 2)) >= 1/255, i.e. inside the perspective image of
 // the ellipse u^2 + v^2 <= tau = 2 ln(255 o) of the surfel's tangent plane, or inside the screen-space disc of the

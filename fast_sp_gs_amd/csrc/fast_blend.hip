@@ -148,6 +148,7 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
   // With snapshots the lists end at the buckets of 32 entries, two of which are staged at a time.
   constexpr int kLanes = 8, kB = kSnap ? 64 : 128;
   using Shape = BlockShape<kLanes>;
+  static_assert(!kHits || kLanes == kHitLanes);
   __shared__ FastRecord s_splat[kB + 1];      // the last one is what padding names: no pixel blends it
   __shared__ float s_t2[kFlow ? kB * 9 : 1];  // second-time-step transforms of the staged surfels
   __shared__ unsigned s_mask[kB];             // which blocks of the tile each staged surfel can reach

@@ -135,6 +135,7 @@ __global__ void __launch_bounds__(kBlendThreads) gs3d_forward_kernel(int flags, 
   // With snapshots the lists end at the buckets of 32 entries, two of which are staged at a time.
   constexpr int kLanes = 8, kB = kSnap ? 64 : 192;
   using Shape = BlockShape<kLanes>;
+  static_assert(!kHits || kLanes == kHitLanes);
   __shared__ G3Splat<E> s_splat[kB + 1];  // the last one is what padding names: no pixel blends it
   __shared__ unsigned s_mask[kB];         // which blocks of the tile each staged Gaussian can reach
   __shared__ __attribute__((aligned(16))) unsigned char s_list[Shape::kPerTile * kB + 16];
