@@ -553,25 +553,8 @@ FSGS_API int fsgs_gs_2d_render_backward_culled(int P, int W, int H, double near_
                          workspace_bytes, records, keep_masks, nullptr, stream);
 }
 
-// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp): the records stay in the
-// workspace, the preprocess backward sums them.
-FSGS_API int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
-    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
-    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
-    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
-    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
-    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
-    size_t workspace_bytes, const float* records, void* stream) {
-  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && records),
-               "gs_2d_view_backward: record slots and packed records are required");
-  return render_backward(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2, out_opacity,
-                         out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges, point_list, n_contrib,
-                         nullptr, nullptr, nullptr, nullptr, R,
-                         SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
-                         workspace_bytes, records, nullptr, nullptr, stream);
-}
-
-// The same over the blocks that blended an entry, as the forward noted them (nullptr: bounded here).
+// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp), over the blocks that blended an
+// entry as the forward noted them (nullptr: bounded here): the records stay in the workspace, the preprocess backward sums them.
 FSGS_API int fsgs_gs_2d_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
     const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
@@ -586,4 +569,17 @@ FSGS_API int fsgs_gs_2d_view_backward_hits(int P, int W, int H, double near_n, d
                          nullptr, nullptr, nullptr, nullptr, R,
                          SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
                          workspace_bytes, records, nullptr, hit_blocks, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* trans_mat_t2,
+    const float* out_opacity, const float* out_extras, const float* out_flow, const float* dL_dpix,
+    const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow, const int64_t* ranges,
+    const int32_t* point_list, const int32_t* n_contrib, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const float* records, void* stream) {
+  return fsgs_gs_2d_view_backward_hits(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, trans_mat_t2,
+                                       out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow, ranges,
+                                       point_list, n_contrib, R, slot_offsets, slot_regions, tiles_touched, radii, workspace,
+                                       workspace_bytes, records, nullptr, stream);
 }

@@ -1120,25 +1120,8 @@ FSGS_API int fsgs_gs_2d_fast_render_backward(int P, int W, int H, double near_n,
                               SlotSource{point_offsets}, radii, workspace, workspace_bytes, keep_masks, nullptr, stream);
 }
 
-// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp).
-FSGS_API int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
-    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
-    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
-    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
-    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
-    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
-    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
-    size_t workspace_bytes, const uint32_t* keep_masks, void* stream) {
-  FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched),
-               "gs_2d_fast_view_backward: record slots are required");
-  return fast_render_backward(P, W, H, near_n, far_n, 0, means2D, normal_opacity, colors, trans_mat, inverse_m,
-                              trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras, dL_dflow,
-                              ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
-                              SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
-                              workspace_bytes, keep_masks, nullptr, stream);
-}
-
-// The same over the blocks that blended an entry, as the forward noted them (nullptr: bounded here).
+// The same for views whose preprocess handed out the record slots by regions (instance_slots.hpp), over the blocks that blended an
+// entry as the forward noted them (nullptr: bounded here).
 FSGS_API int fsgs_gs_2d_fast_view_backward_hits(int P, int W, int H, double near_n, double far_n, const float* means2D,
     const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
     const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
@@ -1154,6 +1137,21 @@ FSGS_API int fsgs_gs_2d_fast_view_backward_hits(int P, int W, int H, double near
                               ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv, g_normal_opacity, R,
                               SlotSource{nullptr, slot_offsets, slot_regions, tiles_touched}, radii, workspace,
                               workspace_bytes, keep_masks, hit_blocks, stream);
+}
+
+FSGS_API int fsgs_gs_2d_fast_view_backward(int P, int W, int H, double near_n, double far_n, const float* means2D,
+    const float* normal_opacity, const float* colors, const float* trans_mat, const float* inverse_m,
+    const float* trans_mat_t2, const float* out_opacity, const float* out_extras, const float* out_flow,
+    const float* dL_dpix, const float* dL_dopacity, const float* dL_dextras, const float* dL_dflow,
+    const int64_t* ranges, const int32_t* point_list, const int32_t* n_contrib, float* g_colors, float* g_means2D,
+    float* g_trans, float* g_inv, float* g_normal_opacity, int64_t R, const int32_t* slot_offsets,
+    const int32_t* slot_regions, const int32_t* tiles_touched, const int32_t* radii, void* workspace,
+    size_t workspace_bytes, const uint32_t* keep_masks, void* stream) {
+  return fsgs_gs_2d_fast_view_backward_hits(P, W, H, near_n, far_n, means2D, normal_opacity, colors, trans_mat, inverse_m,
+                                            trans_mat_t2, out_opacity, out_extras, out_flow, dL_dpix, dL_dopacity, dL_dextras,
+                                            dL_dflow, ranges, point_list, n_contrib, g_colors, g_means2D, g_trans, g_inv,
+                                            g_normal_opacity, R, slot_offsets, slot_regions, tiles_touched, radii, workspace,
+                                            workspace_bytes, keep_masks, nullptr, stream);
 }
 
 // The per-splat decomposition itself (fast_bucket_backward_kernel), for callers that want the reference's second
