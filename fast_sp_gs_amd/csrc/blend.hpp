@@ -411,6 +411,12 @@ __device__ __forceinline__ unsigned wave_max_to_last(unsigned v) {
   return v;
 }
 
+// 1 / v by one Newton step behind the hardware's approximation: as good as the division, in three instructions.
+__device__ __forceinline__ float newton_rcp(float v) {
+  const float r = __builtin_amdgcn_rcpf(v);
+  return fmaf(fmaf(-v, r, 1.0f), r, r);
+}
+
 // Sum over each aligned group of 8 or 16 lanes; the total is valid in the group's last lane only.
 template <int kLanes>
 __device__ __forceinline__ float block_sum_to_last(float v) {

@@ -248,8 +248,7 @@ blend_backward_kernel(
           const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
           float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
           w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-          float rw = __builtin_amdgcn_rcpf(w2);
-          rw = fmaf(fmaf(-w2, rw, 1.0f), rw, rw);  // a Newton step: as good as a division
+          const float rw = newton_rcp(w2);
           // flow u2 / w2 - x as (u2 - x w2) / w2: one rounding in the difference of two nearly equal numbers
           const float fu = fmaf(-pxf, w2, u2) * rw, fv = fmaf(-pyf, w2, v2) * rw;
           c_lin = fmaf(fu, dLf0, fmaf(fv, dLf1, c_lin));

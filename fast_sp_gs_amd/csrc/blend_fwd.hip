@@ -14,7 +14,9 @@
 // next batch's gather is issued before the current batch is blended so its HBM latency overlaps the arithmetic.
 // Bound by vector issue (60 instructions a step, three of them transcendental). 300k surfels 800x800: 147 us with one list
 // per quadrant, 107 with lists per 4x4 block, 94 per 2x4 block; 3M 1352x1014: 506, 333, 282; 400k 3840x2160: 930, 845, 849;
-// 10k 256x256: 28, 19, 18. Batches of 64 / 128 / 192 surfels (a list's length varies less over a long batch), 2x4: 113 / 97 /
+// 10k 256x256: 28, 19, 18. With flow the second transforms are loaded when a batch is staged (requested ahead they hold nine
+// registers) and the quotient takes a reciprocal instead of two divisions: 300k 164 -> 142 us, 2000 surfels with deviations of
+// 128 pixels 592 -> 501. Batches of 64 / 128 / 192 surfels (a list's length varies less over a long batch), 2x4: 113 / 97 /
 // 94 us at 300k, 346 / 297 / 282 at 3M.
 #include "block_lists.hpp"
 #include "view_maps.hpp"
@@ -96,13 +98,8 @@ blend_forward_kernel(
   if (kAccum == 2 && threadIdx.x < kFwdBatch) s_accw[threadIdx.x] = 0.0f, s_accn[threadIdx.x] = 0;
 
   Splat next;
-  float next_t2[9];
-  if ((int) threadIdx.x < min(n_todo, kFwdBatch)) {
+  if ((int) threadIdx.x < min(n_todo, kFwdBatch))
     next = gather_splat(point_list[r0 + threadIdx.x], means2D, colors, normal_opacity, trans_mat, records);
-    if (kFlow)
-#pragma unroll
-      for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
-  }
 
   int b = 0;
   for (; b < rounds; ++b) {
@@ -118,18 +115,14 @@ blend_forward_kernel(
         mask = surfel_blocks<kFwdLanes>(next.hot, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
         if (kFlow)
 #pragma unroll
-          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
       }
       s_mask[threadIdx.x] = mask;
     }
     __syncthreads();
     const int nxt = (b + 1) * kFwdBatch + threadIdx.x;
-    if ((int) threadIdx.x < kFwdBatch && nxt < n_todo) {
+    if ((int) threadIdx.x < kFwdBatch && nxt < n_todo)
       next = gather_splat(point_list[r0 + nxt], means2D, colors, normal_opacity, trans_mat, records);
-      if (kFlow)
-#pragma unroll
-        for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
-    }
 
     // One list entry per block of the wavefront. The intersection runs without early exits and yields one predicate; the
     // blend is one divergent region.
@@ -178,8 +171,9 @@ blend_forward_kernel(
               const float v2 = fmaf(Q[3], h.sx, fmaf(Q[4], h.sy, Q[5]));
               float w2       = fmaf(Q[6], h.sx, fmaf(Q[7], h.sy, Q[8]));
               w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-              f0 = fmaf(u2 / w2 - pxf, w, f0);
-              f1 = fmaf(v2 / w2 - pyf, w, f1);
+              const float rw = newton_rcp(w2);
+              f0 = fmaf(fmaf(-pxf, w2, u2) * rw, w, f0);  // u2 / w2 - x: one rounding in the difference
+              f1 = fmaf(fmaf(-pyf, w2, v2) * rw, w, f1);
             }
             wsum += w;
           }

@@ -133,9 +133,12 @@ __device__ __forceinline__ float row_sum5_transposed(const float (&v)[5]) {
 
 // Bound by vector issue. 150k surfels 1001x667: 62 -> 57 us with lists per 2x4 block instead of 8x8 quadrant,
 // noting the blocks (batches of 192 surfels instead of 128: 58; held to five wavefronts per SIMD, which spills: 62).
+// With flow or weights held to four, with flow as in the other forward (transforms loaded at the staging, a reciprocal): 300k
+// 800x800 88 -> 75 us, with snapshots 129 -> 94; 2000 surfels with deviations of 128 pixels 530 -> 436 and 555 -> 436.
 // kHits: notes which blocks blended an entry (hit_blocks), for the backward.
 template <bool kAux, bool kSnap, bool kAccum, bool kFlow, bool kHits>
-__global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
+__global__ void __launch_bounds__(kBlendThreads) __attribute__((amdgpu_waves_per_eu(kFlow || kAccum ? 4 : 1)))
+fast_blend_forward_kernel(
     int ordered, const int* __restrict__ tile_order, int W, int H, float near_n, float far_n, const int64_t* __restrict__ ranges, const int32_t* __restrict__ point_list,
     const float2* __restrict__ means2D, const float* __restrict__ colors, const float* __restrict__ trans_mat,
     const float* __restrict__ inverse_m, const float4* __restrict__ normal_opacity,
@@ -215,15 +218,10 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
   unsigned char* const lists  = &s_list[Shape::kPerWave * wave * kB];
 
   FastSplat next;
-  float next_t2[9];
   auto gather = [&](int at) {
     if ((int) threadIdx.x >= kB || at >= n_todo) return;
     const int id = point_list[r0 + at];
     next = gather_fast(id, means2D, colors, normal_opacity, trans_mat, inverse_m);
-    if (kFlow) {
-#pragma unroll
-      for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) id + k];
-    }
   };
   gather((int) threadIdx.x);
 
@@ -239,7 +237,7 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
         mask = fast_blocks<kLanes>(next, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
         if (kFlow) {
 #pragma unroll
-          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[threadIdx.x * 9 + k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
         }
       }
       s_mask[threadIdx.x] = mask;
@@ -287,8 +285,9 @@ __global__ void __launch_bounds__(kBlendThreads) fast_blend_forward_kernel(
             const float v2 = fmaf(Q[3], h.sx, fmaf(Q[4], h.sy, Q[5]));
             float w2       = fmaf(Q[6], h.sx, fmaf(Q[7], h.sy, Q[8]));
             w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-            f0 = fmaf(u2 / w2 - pxf, w, f0);
-            f1 = fmaf(v2 / w2 - pyf, w, f1);
+            const float rw = newton_rcp(w2);
+            f0 = fmaf(fmaf(-pxf, w2, u2) * rw, w, f0);  // u2 / w2 - x: one rounding in the difference
+            f1 = fmaf(fmaf(-pyf, w2, v2) * rw, w, f1);
           }
         }
         C0 = fmaf(cold.r, w, C0), C1 = fmaf(cold.g, w, C1), C2 = fmaf(cold.b, w, C2);
@@ -465,7 +464,7 @@ __global__ void __launch_bounds__(256) fast_slot_sum_kernel(int P, int gx, int g
 
 // Bound by vector issue and, like every launch here, by its longest tile; four blocks per compute unit. 150k surfels 1001x667:
 // 165 -> 132 us with a row of lanes per 4x4 block, over the blocks that the forward noted, instead of a wavefront per 8x8 quadrant
-// that queued its blended pairs.
+// that queued its blended pairs; 130 with several batches per staging.
 // kSlots: the per-surfel sums go through per-instance records (ordered_sums.hpp) instead of device-scope atomics.
 template <bool kAux, bool kPerSplat, bool kFlow, bool kSlots>
 __global__ void __launch_bounds__(kBlendThreads)
@@ -575,7 +574,6 @@ __global__ void __launch_bounds__(kBlendThreads)
   float acc_lin = 0;  // what the pairs behind the current one accumulated: alpha_j c_j weighted by the transmittance between
 
   FastSplat next;
-  float next_t2[9];
   unsigned next_hits = 0u;
   int next_radius = 0;
   int64_t next_off = 0;
@@ -587,10 +585,6 @@ __global__ void __launch_bounds__(kBlendThreads)
     if (hit_blocks) next_hits = hit_blocks[at];
     const int id = point_list[at];
     next = gather_fast(id, means2D, colors, normal_opacity, trans_mat, inverse_m);
-    if (kFlow) {
-#pragma unroll
-      for (int k = 0; k < 9; ++k) next_t2[k] = trans_mat_t2[9 * (size_t) id + k];
-    }
     if (kSlots) next_radius = radii[id], next_off = slot_first(slots, id);
   };
   gather(0);
@@ -606,7 +600,7 @@ __global__ void __launch_bounds__(kBlendThreads)
                           : fast_blocks<16>(next, keep_local(tile_x) * kTile, keep_local(tile_y) * kTile, ordered);
         if (kFlow) {
 #pragma unroll
-          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = next_t2[k];
+          for (int k = 0; k < 9; ++k) s_t2[e * 9 + k] = trans_mat_t2[9 * (size_t) next.cold.id + k];
         }
         if (kSlots) {
           // The fused binning reserves one key position per tile of the surfel's rectangle, from its prefix-scan offset
@@ -673,10 +667,10 @@ __global__ void __launch_bounds__(kBlendThreads)
           const float v2 = Q[3] * h.sx + Q[4] * h.sy + Q[5];
           float w2       = Q[6] * h.sx + Q[7] * h.sy + Q[8];
           w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
-          const float rw = 1.0f / w2;
-          c_lin += (u2 * rw - pxf) * dLf0 + (v2 * rw - pyf) * dLf1;
-          const float gu = w * rw * dLf0, gv = w * rw * dLf1;
-          const float gw = -w * rw * rw * (u2 * dLf0 + v2 * dLf1);
+          const float rw = newton_rcp(w2);
+          const float fu = fmaf(-pxf, w2, u2) * rw, fv = fmaf(-pyf, w2, v2) * rw;  // u2 / w2 - x: one rounding in the difference
+          c_lin = fmaf(fu, dLf0, fmaf(fv, dLf1, c_lin));
+          const float wr = w * rw, gu = wr * dLf0, gv = wr * dLf1, gw = -wr * fmaf(fu + pxf, dLf0, (fv + pyf) * dLf1);
           fsx = Q[0] * gu + Q[3] * gv + Q[6] * gw;
           fsy = Q[1] * gu + Q[4] * gv + Q[7] * gw;
         }
