@@ -7,7 +7,7 @@
 //
 // Where the reference issues 18-21 global float atomics per (pixel, surfel) pair, a 16-lane row of a wavefront owns a 4x4
 // block of pixels, walks its own list of the staged surfels that reach it (block_lists.hpp) and sums an entry's components
-// over its pixels with DPP row shifts; per staged batch the sums of a tile's 16 rows are added in row order, and every staged
+// over its pixels with DPP row shifts; per staged batch the sums of a tile's 16 rows are added in a fixed order, and every staged
 // (surfel, tile) instance writes one record at its position in surfel order; slot_reduce_kernel or the preprocess backward
 // sums a surfel's records in a fixed order. (Without scan offsets: one global atomic per surfel, component and tile.)
 // With flow the step is 50 instructions longer. Its channels, and the sum of weights that it is divided by, ride on the recurrence
@@ -334,7 +334,7 @@ blend_backward_kernel(
        walk_block_list(&s_list[(4 * wave + row) * kRowBatch], steps, [&](int j) { return s_splat[j].hot; }, backward_entry,
                        [] { return true; });
       __syncthreads();
-      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      // Flush the batch: add the sums of the rows that hold an entry, in a fixed order.
       if (kSlots) {
         // One 72-byte record per (surfel, tile) instance at the instance's position in surfel order, nine components per lane; the
         // per-surfel sums are taken afterwards. Every staged instance writes its record, zeros included (the instances that

@@ -739,7 +739,7 @@ __global__ void __launch_bounds__(kBlendThreads)
       walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
                       [] { return true; });
       __syncthreads();
-      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      // Flush the batch: add the sums of the rows that hold an entry, in a fixed order.
       if (kSlots) {
         // two lanes per entry, eleven of the record's floats each (component 10 is summed by both)
         static_assert(kBlendThreads == 2 * kB && kFastGradSlots == 21 && kFastRecordSlots == 22);

@@ -12,7 +12,7 @@
 // next batch's gather in flight, a work list per small block of pixels from an exact bound of the alpha >= 1/255 ellipse
 // (block_lists.hpp), longest lists scheduled first. Where the reference issues 9 + E global float atomics per (pixel,
 // Gaussian) pair, the backward sums the 9 + E gradient components over a 4x4 block with DPP row shifts, adds the tile's rows
-// in row order and flushes one global atomic per Gaussian, component and tile. (The top-k, per-Gaussian and wide-feature kernels
+// in a fixed order and flushes one global atomic per Gaussian, component and tile. (The top-k, per-Gaussian and wide-feature kernels
 // below keep one list per 8x8 quadrant.)
 #include "block_lists.hpp"
 #include "ordered_sums.hpp"
@@ -611,7 +611,7 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
       walk_block_list(&s_list[(4 * wave + row) * kB], steps, [&](int j) { return s_splat[j]; }, entry,
                       [] { return true; });
       __syncthreads();
-      // Flush the batch: add the sums of the rows that hold an entry, in row order.
+      // Flush the batch: add the sums of the rows that hold an entry, in a fixed order.
       if (kSlots && kNine) {
         // two lanes per entry, half of its record's sixteen floats each; the geometry's part still lacks the factor -opacity
         static_assert(kBlendThreads == 2 * kB && kG3Slots == 16);
