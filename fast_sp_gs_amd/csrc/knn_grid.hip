@@ -9,15 +9,17 @@
 //      distance does not exceed U, in ascending index order. A block builds the list of one of 8 x 8 x 8 coarse cells and
 //      refines it for the (G / 8)^3 cells inside.
 //   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 35 entries for 2048 control
-//      points and G = 32). The walk only keeps the K + 1 smallest keys -- the distance's bits with the low seven replaced
-//      by the list position -- in a sorted register list, one v_med3_u32 per slot; the K exact distances and indices are
-//      looked up afterwards. Queries whose keys cannot separate two neighbours (distances equal in their upper 25 bits),
+//      points and G = 32). The walk only keeps the K + 1 smallest keys -- the distance in 2^-20 parts of
+//      the cell's bound, then the control point's number -- in a sorted register list, one v_med3_u32 per slot; the K exact
+//      distances are formed again afterwards. Queries whose keys cannot separate two neighbours (distances in the same part),
 //      whose cell has more than 128 candidates, or that lie outside the grid are taken by the whole wavefront one at a
 //      time (64 control points per step), or all together by the search over all control points when they are many.
+//      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
+//      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.29 ms a call this way
-// (traced: lists 0.044, queries 0.272; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
-// the address path of the vector memory (TA busy 0.82 of the time: every lane reads its own list lines); vector issue 0.70.
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.24 ms a call this way
+// (traced: lists 0.043, queries 0.223; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
+// vector issue (2340 instructions per 64 queries); the LDS and the address path of the vector memory are busy half the time.
 // 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
 
@@ -26,17 +28,16 @@
 namespace fsgs {
 namespace {
 
-constexpr int kListCap   = 128;   // candidates per cell: seven position bits
+constexpr int kListCap   = 128;   // candidates per cell
 constexpr int kCoarse    = 8;     // coarse cells per axis
 constexpr int kMaxPoints = 2560;  // control points a block keeps in LDS, 16 bytes each (41 of the list kernel's 72 KB at G = 32, of its 51 KB at G = 16)
 constexpr int kMaxK      = 8;
 constexpr int kOctantCap = 1024;  // candidates of an octant of a coarse cell
 constexpr int kAhead = 4;
-// list entries are byte offsets of the control points in a block's LDS copy
-constexpr int kEntryScale = 16;
-static_assert((kMaxPoints + 8) * kEntryScale < 65536, "an entry has 16 bits");
+constexpr uint32_t kNumberBits = 0xfff;  // of a key: the control point's number, 20 bits of distance above it
+static_assert(kMaxPoints + 8 <= (int) kNumberBits, "the numbers behind the last point, too");
 constexpr int kBuildThreads = 512, kQueryThreads = 512;
-constexpr uint16_t kLongList = 0xffff;
+constexpr uint32_t kLongList = 0xffff;
 constexpr int kFewQueries = 16384;
 
 enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
@@ -54,17 +55,22 @@ Scheme knn_scheme(int N, int M, int D, int K) {
   return M > 640 || N >= 1000000 ? kGrid32 : kGrid16;
 }
 
+// A cell: how many candidates its list holds (or kLongList), and what takes a squared distance to 2^32 at the cell's bound.
+struct Cell {
+  uint32_t length;
+  float scale;
+};
 struct GridLayout {
   int G;
-  size_t planes, lengths, lists, bytes;
+  size_t planes, cells, lists, bytes;
 };
 GridLayout grid_layout(Scheme scheme) {
   GridLayout l{scheme == kGrid32 ? 32 : scheme == kGrid16 ? 16 : 0, 0, 0, 0, 0};
   if (l.G == 0) return l;
   const size_t cells = (size_t) l.G * l.G * l.G;
   l.planes  = 0;
-  l.lengths = align_up(3 * (size_t) (l.G + 1) * 4, 256);
-  l.lists   = align_up(l.lengths + cells * 2, 256);
+  l.cells   = align_up(3 * (size_t) (l.G + 1) * 4, 256);
+  l.lists   = align_up(l.cells + cells * sizeof(Cell), 256);
   l.bytes   = l.lists + cells * kListCap * 2;
   return l;
 }
@@ -202,10 +208,10 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
   __syncthreads();
 }
 
-// The members of `sub` within `limit` of a box, appended to `out` (times `scale`) in index order by one wavefront; stops
+// The members of `sub` within `limit` of a box, appended to `out` in index order by one wavefront; stops
 // once there are more than `cap`. Returns how many there are, or a number above cap.
 __device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* sub, int n_sub, const float* lo,
-                                            const float* hi, float limit, int cap, int scale, uint16_t* out) {
+                                            const float* hi, float limit, int cap, uint16_t* out) {
   const int lane = threadIdx.x & 63;
   int n = 0;
   for (int i0 = 0; i0 < n_sub && n <= cap; i0 += kAhead * kWave) {  // the LDS reads of kAhead steps are in flight together
@@ -220,7 +226,7 @@ __device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* s
     for (int u = 0; u < kAhead; ++u) {
       const unsigned long long m = wave_ballot(in[u]);
       const int pos = n + lanes_below(m);
-      if (in[u] && pos < cap) out[pos] = (uint16_t) (i[u] * scale);
+      if (in[u] && pos < cap) out[pos] = (uint16_t) i[u];
       n += (int) __popcll(m);
     }
   }
@@ -232,7 +238,7 @@ __device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* s
 // directly: the coarse lists at the rim of the cloud hold nearly everything.
 template <int kG>
 __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
-    float* __restrict__ planes, uint16_t* __restrict__ lengths, uint16_t* __restrict__ lists) {
+    float* __restrict__ planes, Cell* __restrict__ cells, uint16_t* __restrict__ lists) {
   constexpr int kWaves = kBuildThreads / kWave;
   static_assert(kWaves == 8, "a wavefront per octant");
   __shared__ float4 s_y[kMaxPoints];
@@ -305,7 +311,7 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
 #pragma unroll
     for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][corner[a]], hi[a] = s.plane[a][corner[a] + kIn];
     uint16_t* mine = s_octant[wave];
-    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, bound_of(s_sub, n_sub), kOctantCap, 1, mine);
+    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, bound_of(s_sub, n_sub), kOctantCap, mine);
     from   = mine;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -318,11 +324,16 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     const int cell = (g[2] * kG + g[1]) * kG + g[0];
     uint16_t* list = lists + (size_t) cell * kListCap;
     int n = kListCap + 1;  // an octant with too many candidates: its cells have long lists too
-    if (kG == 16 || n_from <= kOctantCap)
-      n = collect_near(s_y, from, n_from, lo, hi, bound_of(from, n_from), kListCap, kEntryScale, list);
+    float limit = 0.0f;
+    if (kG == 16 || n_from <= kOctantCap) {
+      limit = bound_of(from, n_from);
+      n     = collect_near(s_y, from, n_from, lo, hi, limit, kListCap, list);
+      if (!(limit < 3e38f)) n = kListCap + 1;
+    }
     // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
-    if (n <= kListCap && lane < 8 && n + lane < (n + 7) / 8 * 8) list[n + lane] = (uint16_t) (M * kEntryScale);
-    if (lane == 0) lengths[cell] = n <= kListCap ? (uint16_t) n : kLongList;
+    if (n <= kListCap && lane < 8 && n + lane < (n + 7) / 8 * 8) list[n + lane] = (uint16_t) M;
+    // the K nearest of any query of the cell are nearer than `limit`: their parts stay below 2^32, the others' may saturate
+    if (lane == 0) cells[cell] = Cell{n <= kListCap ? (uint32_t) n : kLongList, fminf(4294967296.0f / limit, 3e38f)};
   }
 }
 
@@ -334,7 +345,14 @@ __device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c)
 
 __device__ __forceinline__ uint32_t and_or_b32(uint32_t a, uint32_t mask, uint32_t b) {
   uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(mask), "s"(b));
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(b));
+  return r;
+}
+
+// v >= 0 cut to a whole number, 2^32 - 1 from 2^32 on (the conversion in C++ is undefined there)
+__device__ __forceinline__ uint32_t saturated_u32(float v) {
+  uint32_t r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
   return r;
 }
 
@@ -363,7 +381,7 @@ __device__ __forceinline__ void store_result(float* __restrict__ dist2, int64_t*
 template <int kK, int kG>
 __global__ void __launch_bounds__(kQueryThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
 knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
-    const float* __restrict__ y, const float* __restrict__ planes, const uint16_t* __restrict__ lengths,
+    const float* __restrict__ y, const float* __restrict__ planes, const Cell* __restrict__ cells,
     const uint16_t* __restrict__ lists, float* __restrict__ dist2, int64_t* __restrict__ index) {
   // a query alone costs a wavefront about 20 M / 64 + 300 instructions, the all-pairs walk about 20 M for all 64
   const int max_alone = 20 * M / (20 * M / 64 + 300);
@@ -374,7 +392,11 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
   __shared__ float s_cand_d[kWaves][kWave];
   __shared__ int s_cand_i[kWaves][kWave];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int i = t; i < M; i += kQueryThreads) s_y[i] = make_float4(y[3 * i], y[3 * i + 1], y[3 * i + 2], 0.0f);
+  // one with a NaN, which is nobody's neighbour, lies at infinity: the keys order no NaN
+  for (int i = t; i < M; i += kQueryThreads) {
+    const float a = y[3 * i], b = y[3 * i + 1], c = y[3 * i + 2];
+    s_y[i] = make_float4(a == a && b == b && c == c ? a : __builtin_inff(), b, c, 0.0f);
+  }
   if (t < 8) s_y[M + t] = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
   if (kG > 0)
     for (int e = t; e < 3 * (kG + 1); e += kQueryThreads) (&s_plane[0][0])[e] = planes[e];
@@ -475,11 +497,10 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         inside = inside && q[a] >= s_plane[a][0] && q[a] < s_plane[a][kG];  // false for NaN
         cell   = cell * kG + i;
       }
-      const int len   = inside ? (int) lengths[cell] : (int) kLongList;
-      bool slow       = live && len == (int) kLongList;
-      const int n_list = len == (int) kLongList ? 0 : len;
+      const Cell here = inside ? cells[cell] : Cell{kLongList, 0.0f};
+      bool unknown    = here.length == kLongList;
+      const int n_list = here.length == kLongList ? 0 : (int) here.length;
       const uint16_t* list = lists + (size_t) cell * kListCap;
-      const uint32_t key_mask = ~(uint32_t) (kListCap - 1);
       uint32_t key[kK + 1];
 #pragma unroll
       for (int k = 0; k <= kK; ++k) key[k] = 0xffffffffu;
@@ -491,30 +512,29 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const uint32_t i = (j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu);
-          const float d = distance2(q[0], q[1], q[2], *(const float4*) (s_dyn + i));
-          const uint32_t nk = and_or_b32(__float_as_uint(d), key_mask, (uint32_t) (c + j));
+          const float d = distance2(q[0], q[1], q[2], s_y[i]);
+          const uint32_t nk = and_or_b32(saturated_u32(d * here.scale), ~kNumberBits, i);
 #pragma unroll
           for (int k = kK; k >= 1; --k) key[k] = med3_u32(key[k - 1], nk, key[k]);
           key[0] = min(key[0], nk);
         }
       }
-      // neighbours that agree in all the bits a key keeps are not in a known order
-      constexpr uint32_t kInfinite = 0x7f800000u;
+      // neighbours in the same part are not in a known order; where the parts saturate (there are not K points at a finite
+      // distance, or the bound is next to nothing) nothing is known
 #pragma unroll
       for (int k = 0; k < kK; ++k)
-        if (key[k] < kInfinite && (key[k] ^ key[k + 1]) < (uint32_t) kListCap) slow = live;
+        if ((key[k] ^ key[k + 1]) <= kNumberBits) unknown = true;
+      if (key[kK - 1] >= ~kNumberBits) unknown = true;
       float bd[kK];
       int bi[kK];
 #pragma unroll
       for (int k = 0; k < kK; ++k) {
-        const bool found = !slow && key[k] < kInfinite;
-        bi[k] = found ? (int) list[key[k] & (uint32_t) (kListCap - 1)] / kEntryScale : M;
+        bi[k] = unknown ? M : (int) (key[k] & kNumberBits);
         bd[k] = distance2(q[0], q[1], q[2], s_y[bi[k]]);
-        if (!found) bi[k] = -1, bd[k] = -1.0f;
       }
-      if (live && !slow) store_result<kK>(dist2, index, n, bd, bi);
+      if (live && !unknown) store_result<kK>(dist2, index, n, bd, bi);
 
-      unsigned long long rest = wave_ballot(slow), together = 0ull;
+      unsigned long long rest = wave_ballot(live && unknown), together = 0ull;
       if (__popcll(rest) > max_alone) together = rest, rest = 0ull;
       while (rest) {
         const int l = __builtin_ctzll(rest);
@@ -538,7 +558,7 @@ void launch_query(int N, int M, const float* x, const float* y, const GridLayout
   const int per_block = kG > 0 ? kQueryThreads : kQueryThreads / kWave;
   const int blocks = std::min(div_up(N, per_block), 256 * 8);
   hipLaunchKernelGGL((knn_cell_query_kernel<kK, kG>), dim3(blocks), dim3(kQueryThreads), lds, s, N, M, x, y,
-                     (const float*) (ws + l.planes), (const uint16_t*) (ws + l.lengths), (const uint16_t*) (ws + l.lists),
+                     (const float*) (ws + l.planes), (const Cell*) (ws + l.cells), (const uint16_t*) (ws + l.lists),
                      dist2, index);
 }
 
@@ -550,11 +570,11 @@ int launch_grid_knn(Scheme scheme, int N, int M, const float* x, const float* y,
     launch_query<kK, 0>(N, M, x, y, l, ws, dist2, index, s);
   } else if (scheme == kGrid16) {
     hipLaunchKernelGGL(knn_cell_lists_kernel<16>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
-                       (float*) (ws + l.planes), (uint16_t*) (ws + l.lengths), (uint16_t*) (ws + l.lists));
+                       (float*) (ws + l.planes), (Cell*) (ws + l.cells), (uint16_t*) (ws + l.lists));
     launch_query<kK, 16>(N, M, x, y, l, ws, dist2, index, s);
   } else {
     hipLaunchKernelGGL(knn_cell_lists_kernel<32>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
-                       (float*) (ws + l.planes), (uint16_t*) (ws + l.lengths), (uint16_t*) (ws + l.lists));
+                       (float*) (ws + l.planes), (Cell*) (ws + l.cells), (uint16_t*) (ws + l.lists));
     launch_query<kK, 32>(N, M, x, y, l, ws, dist2, index, s);
   }
   return check_launch("knn_topk");
