@@ -17,9 +17,9 @@
 //      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
 //      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.24 ms a call this way
-// (traced: lists 0.043, queries 0.223; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
-// vector issue (2340 instructions per 64 queries); the LDS and the address path of the vector memory are busy half the time.
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.22 ms a call this way (mean of 30 inputs)
+// (traced: lists 0.033, queries 0.201; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
+// vector issue (2080 instructions per 64 queries); the LDS and the address path of the vector memory are busy half the time.
 // 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
 
@@ -128,19 +128,40 @@ __device__ __forceinline__ float from_ordered_bits(uint32_t b) {
 
 template <int kG>
 struct PlaneLds {
-  static constexpr int kSamples = 8 * kG;
+  static constexpr int kSamples = 128;
   uint32_t key[3][kSamples];
   float sorted[3][kSamples], along[3][kSamples];
   float plane[3][kG + 1];
+  uint32_t least[3][8], most[3][8];  // of all control points, per wavefront
 };
 
-// The grid planes, from 8 G sampled control points per axis: sorted by counting ranks, inner planes at equal steps of the
-// accumulated square root of the gaps (cells shrink with density, but slower than quantiles would), one plane a tenth of
-// the extent beyond the sample on either side. Every block computes them for itself (3 us) instead of waiting for another launch.
+// The grid planes, from 128 sampled control points per axis (256 cost 6 us more and make the lists no shorter): sorted by counting ranks, inner planes at equal steps of the
+// accumulated square root of the gaps (cells shrink with density, but slower than quantiles would). The outermost planes lie a
+// twentieth of the sample's extent beyond all control points, and at least 0.15 of it beyond the sample: a query outside costs
+// as much as 30 inside, and with planes a tenth beyond the sample there was one in every wavefront (3M normal queries, 2048 normal
+// control points). Where there are planes to spare (G = 32), two more on either side divide that margin, which a sample's
+// gaps know nothing of: its cells would have lists of more than 128. Every block computes the planes for itself (3 us) instead of
+// waiting for another launch.
 template <int kG>
 __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<kG>& s) {
-  constexpr int S = PlaneLds<kG>::kSamples;
+  constexpr int S = PlaneLds<kG>::kSamples, kSpare = kG > 16 ? 2 : 0;
   const int t = threadIdx.x;
+  {
+    uint32_t lo[3] = {~0u, ~0u, ~0u}, hi[3] = {0u, 0u, 0u};
+    for (int i = t; i < M; i += kBuildThreads) {
+      const float4 p      = s_y[i];
+      const uint32_t b[3] = {ordered_bits(p.x), ordered_bits(p.y), ordered_bits(p.z)};
+#pragma unroll
+      for (int c = 0; c < 3; ++c) lo[c] = min(lo[c], b[c]), hi[c] = max(hi[c], b[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1)
+        lo[c] = min(lo[c], (uint32_t) __shfl_xor((int) lo[c], d, kWave)), hi[c] = max(hi[c], (uint32_t) __shfl_xor((int) hi[c], d, kWave));
+      if ((t & 63) == 0) s.least[c][t >> 6] = lo[c], s.most[c][t >> 6] = hi[c];
+    }
+  }
   for (int e = t; e < 3 * S; e += kBuildThreads) {
     const int a = e / S, j = e - a * S;
     const float4 p = s_y[(int) ((int64_t) j * M / S)];
@@ -181,13 +202,20 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
   __syncthreads();
   if (a < 3) {
     const float lo = s.sorted[a][0], hi = s.sorted[a][S - 1], ext = hi - lo;
+    uint32_t least = s.least[a][0], most = s.most[a][0];
+#pragma unroll
+    for (int w = 1; w < kBuildThreads / kWave; ++w) least = min(least, s.least[a][w]), most = max(most, s.most[a][w]);
+    const float first = fminf(from_ordered_bits(least), lo - 0.1f * ext) - 0.05f * ext;
+    const float last  = fmaxf(from_ordered_bits(most), hi + 0.1f * ext) + 0.05f * ext;
     float v = -3e38f;
     if (lane <= kG) {
       const int i = lane;
-      if (i == 0) v = lo - 0.1f * ext;
-      else if (i == kG) v = hi + 0.1f * ext;
+      if (i == 0) v = first;
+      else if (i == kG) v = last;
+      else if (i < 1 + kSpare) v = lo + (i == 1 ? 0.55f : 0.25f) * (first - lo);
+      else if (i > kG - 1 - kSpare) v = hi + (i == kG - 1 ? 0.55f : 0.25f) * (last - hi);
       else {
-        const float target = s.along[a][S - 1] * ((float) (i - 1) / (float) (kG - 2));
+        const float target = s.along[a][S - 1] * ((float) (i - 1 - kSpare) / (float) (kG - 2 - 2 * kSpare));
         int j = 0;  // last sample whose accumulated step does not exceed the target
 #pragma unroll
         for (int step = S / 2; step >= 1; step >>= 1)
@@ -235,7 +263,9 @@ __device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* s
 
 // One block per coarse cell, one wavefront per octant of it: with G = 16 an octant is a cell, with G = 32 it is narrowed
 // down once more for its eight cells. 26 M vector instructions (98 us) when the cells were taken from the coarse list
-// directly: the coarse lists at the rim of the cloud hold nearly everything.
+// directly: the coarse lists at the rim of the cloud hold nearly everything. A wavefront forms the lists of its cells side by
+// side: a candidate is read once for all of them, its distances to their faces are formed once per axis and half of the octant,
+// and nothing waits in a chain of eight (cells one after the other: 25 us of the kernel's 51).
 template <int kG>
 __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
     float* __restrict__ planes, Cell* __restrict__ cells, uint16_t* __restrict__ lists) {
@@ -293,47 +323,96 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
   constexpr int kIn = kSub / 2;  // cells per axis inside an octant
   const int corner[3] = {cc[0] * kSub + (wave & 1) * kIn, cc[1] * kSub + ((wave >> 1) & 1) * kIn,
                          cc[2] * kSub + (wave >> 2) * kIn};
-  auto bound_of = [&](const uint16_t* sub, int n) {
-    float nearest = __builtin_inff();
-    for (int i0 = lane; i0 < n; i0 += kAhead * kWave) {
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        const int i    = i0 + u * kWave;
-        const float d2 = box_far2(s_y[sub[min(i, n - 1)]], lo, hi);
-        nearest        = fminf(nearest, i < n ? d2 : __builtin_inff());
-      }
-    }
-    return widened(wave_kth_bound(nearest, K));
-  };
   const uint16_t* from = s_sub;
   int n_from = n_sub;
   if constexpr (kG > 16) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][corner[a]], hi[a] = s.plane[a][corner[a] + kIn];
+    float nearest = __builtin_inff();
+    for (int i0 = lane; i0 < n_sub; i0 += kAhead * kWave) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int i    = i0 + u * kWave;
+        const float d2 = box_far2(s_y[s_sub[min(i, n_sub - 1)]], lo, hi);
+        nearest        = fminf(nearest, i < n_sub ? d2 : __builtin_inff());
+      }
+    }
     uint16_t* mine = s_octant[wave];
-    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, bound_of(s_sub, n_sub), kOctantCap, mine);
+    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, widened(wave_kth_bound(nearest, K)), kOctantCap, mine);
     from   = mine;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  for (int c = 0; c < kIn * kIn * kIn; ++c) {
-    const int g[3] = {corner[0] + c % kIn, corner[1] + c / kIn % kIn, corner[2] + c / (kIn * kIn)};
+  constexpr int kCells = kIn * kIn * kIn;  // c: half of the octant along x in bit 0, along y in bit 1, along z in bit 2
+  float edge[3][kIn + 1];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][g[a]], hi[a] = s.plane[a][g[a] + 1];
-    const int cell = (g[2] * kG + g[1]) * kG + g[0];
-    uint16_t* list = lists + (size_t) cell * kListCap;
-    int n = kListCap + 1;  // an octant with too many candidates: its cells have long lists too
-    float limit = 0.0f;
-    if (kG == 16 || n_from <= kOctantCap) {
-      limit = bound_of(from, n_from);
-      n     = collect_near(s_y, from, n_from, lo, hi, limit, kListCap, list);
-      if (!(limit < 3e38f)) n = kListCap + 1;
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int h = 0; h <= kIn; ++h) edge[a][h] = s.plane[a][corner[a] + h];
+  // an octant with too many candidates: its cells have long lists, too
+  const bool too_many = kG > 16 && n_from > kOctantCap;
+  if (too_many) n_from = 0;
+  float reach[kCells];
+  {
+    float least_far[kCells];
+#pragma unroll
+    for (int c = 0; c < kCells; ++c) least_far[c] = __builtin_inff();
+#pragma unroll 2
+    for (int i0 = 0; i0 < n_from; i0 += kWave) {
+      const float4 p    = s_y[from[min(i0 + lane, n_from - 1)]];
+      const float at[3] = {p.x, p.y, p.z};
+      float f[3][kIn];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int h = 0; h < kIn; ++h) {
+          const float d = fmaxf(fabsf(at[a] - edge[a][h]), fabsf(at[a] - edge[a][h + 1]));
+          f[a][h] = i0 + lane < n_from ? d * d : __builtin_inff();
+        }
+#pragma unroll
+      for (int c = 0; c < kCells; ++c)
+        least_far[c] = fminf(least_far[c], (f[0][c % kIn] + f[1][c / kIn % kIn]) + f[2][c / (kIn * kIn)]);
     }
+#pragma unroll
+    for (int c = 0; c < kCells; ++c) reach[c] = widened(wave_kth_bound(least_far[c], K));
+  }
+  int n[kCells];
+  uint16_t* list[kCells];
+#pragma unroll
+  for (int c = 0; c < kCells; ++c) {
+    n[c] = 0;
+    list[c] = lists + (size_t) (((corner[2] + c / (kIn * kIn)) * kG + corner[1] + c / kIn % kIn) * kG + corner[0] + c % kIn) * kListCap;
+  }
+#pragma unroll 2
+  for (int i0 = 0; i0 < n_from; i0 += kWave) {
+    const int i       = from[min(i0 + lane, n_from - 1)];
+    const float4 p    = s_y[i];
+    const float at[3] = {p.x, p.y, p.z};
+    float f[3][kIn];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int h = 0; h < kIn; ++h) {
+        const float d = fmaxf(fmaxf(edge[a][h] - at[a], at[a] - edge[a][h + 1]), 0.0f);
+        f[a][h] = d * d;
+      }
+    const unsigned long long there = wave_ballot(i0 + lane < n_from);
+#pragma unroll
+    for (int c = 0; c < kCells; ++c) {
+      const unsigned long long m = there & wave_ballot((f[0][c % kIn] + f[1][c / kIn % kIn]) + f[2][c / (kIn * kIn)] <= reach[c]);
+      const int pos = n[c] + lanes_below(m);
+      if ((m >> lane & 1ull) && pos < kListCap) list[c][pos] = (uint16_t) i;
+      n[c] += (int) __popcll(m);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < kCells; ++c) {
+    const bool fits = !too_many && n[c] <= kListCap && reach[c] < 3e38f;
     // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
-    if (n <= kListCap && lane < 8 && n + lane < (n + 7) / 8 * 8) list[n + lane] = (uint16_t) M;
-    // the K nearest of any query of the cell are nearer than `limit`: their parts stay below 2^32, the others' may saturate
-    if (lane == 0) cells[cell] = Cell{n <= kListCap ? (uint32_t) n : kLongList, fminf(4294967296.0f / limit, 3e38f)};
+    if (fits && lane < 8 && n[c] + lane < (n[c] + 7) / 8 * 8) list[c][n[c] + lane] = (uint16_t) M;
+    // the K nearest of any query of the cell are nearer than `reach`: their parts stay below 2^32, the others' may saturate
+    if (lane == 0) cells[(list[c] - lists) / kListCap] = Cell{fits ? (uint32_t) n[c] : kLongList, fminf(4294967296.0f / reach[c], 3e38f)};
   }
 }
 
