@@ -40,6 +40,10 @@ constexpr int kBuildThreads = 512, kQueryThreads = 512;
 constexpr uint32_t kLongList = 0xffff;
 constexpr int kFewQueries = 16384;
 
+// Lists that the wavefront takes one by one once no more than so many of its lanes have candidates left: a lane's eight more cost
+// the wavefront 180 instructions, what is left of a list about 80. A third of the candidates' steps is walked for a few lanes else.
+constexpr int kFewLists = 4;
+
 enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 
 // Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
@@ -132,21 +136,20 @@ struct PlaneLds {
   uint32_t key[3][kSamples];
   float sorted[3][kSamples], along[3][kSamples];
   float plane[3][kG + 1];
-  uint32_t least[3][8], most[3][8];  // of all control points, per wavefront
+  uint32_t least[kG > 16 ? 3 : 1][8], most[kG > 16 ? 3 : 1][8];  // of all control points, per wavefront
 };
 
-// The grid planes, from 128 sampled control points per axis (256 cost 6 us more and make the lists no shorter): sorted by counting ranks, inner planes at equal steps of the
-// accumulated square root of the gaps (cells shrink with density, but slower than quantiles would). The outermost planes lie a
-// twentieth of the sample's extent beyond all control points, and at least 0.15 of it beyond the sample: a query outside costs
-// as much as 30 inside, and with planes a tenth beyond the sample there was one in every wavefront (3M normal queries, 2048 normal
-// control points). Where there are planes to spare (G = 32), two more on either side divide that margin, which a sample's
-// gaps know nothing of: its cells would have lists of more than 128. Every block computes the planes for itself (3 us) instead of
-// waiting for another launch.
+// The grid planes, from 128 sampled control points per axis (256 cost 6 us more and make the lists no shorter): sorted by
+// counting ranks, inner planes at equal steps of the accumulated square root of the gaps (cells shrink with density, but slower
+// than quantiles would). The outermost planes lie a tenth of the sample's extent beyond it. With many queries (G = 32) they lie beyond all control points, too: a query outside the
+// grid costs as much as 30 inside, and there was one in every wavefront (3M normal queries, 2048 normal control points); two more
+// planes on either side divide that margin, which a sample's gaps know nothing of: its cells would have lists of more than 128.
+// Every block computes the planes for itself (3 us) instead of waiting for another launch.
 template <int kG>
 __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<kG>& s) {
   constexpr int S = PlaneLds<kG>::kSamples, kSpare = kG > 16 ? 2 : 0;
   const int t = threadIdx.x;
-  {
+  if constexpr (kSpare > 0) {
     uint32_t lo[3] = {~0u, ~0u, ~0u}, hi[3] = {0u, 0u, 0u};
     for (int i = t; i < M; i += kBuildThreads) {
       const float4 p      = s_y[i];
@@ -202,11 +205,13 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
   __syncthreads();
   if (a < 3) {
     const float lo = s.sorted[a][0], hi = s.sorted[a][S - 1], ext = hi - lo;
-    uint32_t least = s.least[a][0], most = s.most[a][0];
+    float first = lo - 0.1f * ext, last = hi + 0.1f * ext;
+    if constexpr (kSpare > 0) {
+      uint32_t least = s.least[a][0], most = s.most[a][0];
 #pragma unroll
-    for (int w = 1; w < kBuildThreads / kWave; ++w) least = min(least, s.least[a][w]), most = max(most, s.most[a][w]);
-    const float first = fminf(from_ordered_bits(least), lo - 0.1f * ext) - 0.05f * ext;
-    const float last  = fmaxf(from_ordered_bits(most), hi + 0.1f * ext) + 0.05f * ext;
+      for (int w = 1; w < kBuildThreads / kWave; ++w) least = min(least, s.least[a][w]), most = max(most, s.most[a][w]);
+      first = fminf(from_ordered_bits(least), first) - 0.05f * ext, last = fmaxf(from_ordered_bits(most), last) + 0.05f * ext;
+    }
     float v = -3e38f;
     if (lane <= kG) {
       const int i = lane;
@@ -344,6 +349,7 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
+  constexpr int kTogether = kIn > 1 ? 2 : kAhead;
   constexpr int kCells = kIn * kIn * kIn;  // c: half of the octant along x in bit 0, along y in bit 1, along z in bit 2
   float edge[3][kIn + 1];
 #pragma unroll
@@ -358,7 +364,7 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     float least_far[kCells];
 #pragma unroll
     for (int c = 0; c < kCells; ++c) least_far[c] = __builtin_inff();
-#pragma unroll 2
+#pragma unroll kTogether
     for (int i0 = 0; i0 < n_from; i0 += kWave) {
       const float4 p    = s_y[from[min(i0 + lane, n_from - 1)]];
       const float at[3] = {p.x, p.y, p.z};
@@ -384,7 +390,6 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     n[c] = 0;
     list[c] = lists + (size_t) (((corner[2] + c / (kIn * kIn)) * kG + corner[1] + c / kIn % kIn) * kG + corner[0] + c % kIn) * kListCap;
   }
-#pragma unroll 2
   for (int i0 = 0; i0 < n_from; i0 += kWave) {
     const int i       = from[min(i0 + lane, n_from - 1)];
     const float4 p    = s_y[i];
@@ -583,19 +588,44 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
       uint32_t key[kK + 1];
 #pragma unroll
       for (int k = 0; k <= kK; ++k) key[k] = 0xffffffffu;
+      auto insert = [&](uint32_t nk) {
+#pragma unroll
+        for (int k = kK; k >= 1; --k) key[k] = med3_u32(key[k - 1], nk, key[k]);
+        key[0] = min(key[0], nk);
+      };
+      auto key_of = [&](uint32_t i, float qx, float qy, float qz, float scale) {
+        return and_or_b32(saturated_u32(distance2(qx, qy, qz, s_y[i]) * scale), ~kNumberBits, i);
+      };
       uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
-      for (int c = 0; c < n_list; c += 8) {  // c is the same in every lane still in the loop
-        const uint4 now = next;
-        if (c + 8 < n_list) next = *(const uint4*) (list + c + 8);
-        const uint32_t w[4] = {now.x, now.y, now.z, now.w};
+      int c = 0;
+      unsigned long long longer;
+      for (;; c += 8) {
+        longer = wave_ballot(c < n_list);
+        if (__popcll(longer) <= kFewLists) break;
+        if (c < n_list) {
+          const uint4 now = next;
+          if (c + 8 < n_list) next = *(const uint4*) (list + c + 8);
+          const uint32_t w[4] = {now.x, now.y, now.z, now.w};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t i = (j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu);
-          const float d = distance2(q[0], q[1], q[2], s_y[i]);
-          const uint32_t nk = and_or_b32(saturated_u32(d * here.scale), ~kNumberBits, i);
-#pragma unroll
-          for (int k = kK; k >= 1; --k) key[k] = med3_u32(key[k - 1], nk, key[k]);
-          key[0] = min(key[0], nk);
+          for (int j = 0; j < 8; ++j)
+            insert(key_of((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu), q[0], q[1], q[2], here.scale));
+        }
+      }
+      while (longer) {  // what is left of a few long lists: the whole wavefront on one, a candidate per lane
+        const int l = __builtin_ctzll(longer);
+        longer &= longer - 1;
+        const int count = __builtin_amdgcn_readlane(n_list, l), its_cell = __builtin_amdgcn_readlane(cell, l);
+        const uint16_t* its_list = lists + (size_t) its_cell * kListCap;
+        auto its = [&](float v) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l)); };
+        const float qx = its(q[0]), qy = its(q[1]), qz = its(q[2]), scale = its(here.scale);
+        for (int e = c; e < count; e += kWave) {
+          const uint32_t nk = key_of(its_list[min(e + lane, count - 1)], qx, qy, qz, scale);
+          unsigned long long nearer = wave_ballot(e + lane < count) & wave_ballot(nk < (uint32_t) __builtin_amdgcn_readlane(key[kK], l));
+          while (nearer) {
+            const uint32_t v = __builtin_amdgcn_readlane(nk, __builtin_ctzll(nearer));
+            nearer &= nearer - 1;
+            insert(lane == l ? v : ~0u);
+          }
         }
       }
       // neighbours in the same part are not in a known order; where the parts saturate (there are not K points at a finite
