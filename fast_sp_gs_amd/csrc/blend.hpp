@@ -213,9 +213,11 @@ __device__ __forceinline__ unsigned quadrant_mask(const SplatHot& h, int tile_px
 // An XCD places the first blocks it receives on its CUs in turn, and as many rounds of 32 as blocks fit on a CU stay
 // there together for most of the launch: CU c works on the region's tiles number c, 32 + c, 64 + c, ... In plain
 // descending order CU 0 would get the longest tile of every round and CU 31 the shortest (15 % above the mean for the
-// chord-length profile of a ball of surfels), and the launch lasts as long as its busiest CU. Inside each of the first
-// rounds the tiles are therefore dealt by load: the CU with the least work so far gets the round's longest tile.
-// Later rounds go wherever a slot frees up; for them descending order is what balances.
+// chord-length profile of a ball of surfels), and the launch lasts as long as its busiest CU. The first rounds are therefore
+// dealt back and forth, every second one in ascending order. (Sorting the CUs by the load they hold so far before each round
+// deals no better, blends of 300k surfels 800x800 99 + 229 us against 97 + 226, and the 45 exchanges of its networks held up
+// the scatter, whose extra block builds the table: 15.7 -> 12.8 us.) Later rounds go wherever a slot frees up; for them
+// descending order is what balances.
 // The table is kMaxOrderedTiles ints in a file-scope device array of the library (no allocation), one slot per
 // (device, stream) that bins or blends: calls on one stream are ordered by the stream, calls on different streams use
 // different tables, and a stream that finds every slot taken runs without a table.
@@ -225,8 +227,8 @@ constexpr int kOrderFrac       = 1 << kOrderFracBits;
 constexpr int kOrderBuckets    = 32 * kOrderFrac;
 constexpr int kOrderRegions    = 8;
 constexpr int kCusPerXcd       = 32;  // compute units behind one region's table positions
-// rounds of a region's list whose tiles are dealt by CU load: the blocks of the blend backward that fit on a CU (4,
-// bounded by its 128 registers per lane); measured best among 3, 4, 5, 6, 8, 16
+// rounds of a region's list that are dealt back and forth: the blocks of the blend backward that fit on a CU (4, bounded by its
+// 128 registers per lane)
 constexpr int kBalanceRounds   = 4;
 
 // (tile_order_table, tile_order_invalidate and tile_order_release are declared in common.hpp.)
@@ -252,14 +254,13 @@ __device__ __forceinline__ int tile_region(int t, int gx, int gy) {
   return ((tx / kTileGroup) + 3 * (ty / kTileGroup)) & (kOrderRegions - 1);
 }
 
-// LDS of one block that builds a table (24.6 KB)
+// LDS of one block that builds a table (16.4 KB)
 struct TileOrderLds {
   int count[kOrderRegions][kOrderBuckets];
   int total[kOrderRegions];
-  int tile[kOrderRegions][kBalanceRounds * kCusPerXcd], len[kOrderRegions][kBalanceRounds * kCusPerXcd];
 };
 
-// The work of one whole block (any size that is a multiple of 64 with at least 8 wavefronts): either a launch of its
+// The work of one whole block (any number of wavefronts): either a launch of its
 // own (tile_order_kernel) or one extra block of a kernel that has nothing to do with it but runs at the right time --
 // the binning's scatter, whose other blocks keep the chip busy while this one orders 2 500 numbers (a single-block
 // launch of its own holds up the stream for 10 us).
@@ -267,32 +268,24 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
                                                  int* __restrict__ tile_order, TileOrderLds& lds) {
   auto& s_count = lds.count;
   auto& s_total = lds.total;
-  auto& s_tile  = lds.tile;
-  auto& s_len   = lds.len;
   const int T = gx * gy;
   for (int b = threadIdx.x; b < kOrderRegions * kOrderBuckets; b += blockDim.x) (&s_count[0][0])[b] = 0;
   __syncthreads();
   for (int t = threadIdx.x; t < T; t += blockDim.x)
     atomicAdd(&s_count[tile_region(t, gx, gy)][length_bucket(ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t])], 1);
   __syncthreads();
-  {  // exclusive prefix from the longest bucket down, one wavefront per region
-    const int lane = threadIdx.x & 63, r = threadIdx.x >> 6;
+  // exclusive prefix from the longest bucket down, a wavefront per region
+  for (int r = threadIdx.x >> 6; r < kOrderRegions; r += blockDim.x >> 6) {
+    const int lane = threadIdx.x & 63;
     constexpr int kPer = kOrderBuckets / 64;
-    if (r < kOrderRegions) {
-      int c[kPer], sum = 0;
+    int c[kPer], sum = 0;
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) c[i] = s_count[r][kOrderBuckets - 1 - (lane * kPer + i)], sum += c[i];
-      int inc = sum;
+    for (int i = 0; i < kPer; ++i) c[i] = s_count[r][kOrderBuckets - 1 - (lane * kPer + i)], sum += c[i];
+    const int inc = wave_scan(sum);
+    int run = inc - sum;
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += up;
-      }
-      int run = inc - sum;
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) s_count[r][kOrderBuckets - 1 - (lane * kPer + i)] = run, run += c[i];
-      if (lane == 63) s_total[r] = inc;
-    }
+    for (int i = 0; i < kPer; ++i) s_count[r][kOrderBuckets - 1 - (lane * kPer + i)] = run, run += c[i];
+    if (lane == 63) s_total[r] = inc;
   }
   __syncthreads();
   // position of the k-th tile of region r when the regions are dealt round-robin, skipping exhausted ones
@@ -305,43 +298,10 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
   for (int t = threadIdx.x; t < T; t += blockDim.x) {
     const int r       = tile_region(t, gx, gy);
     const int64_t len = ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t];
-    const int k       = atomicAdd(&s_count[r][length_bucket(len)], 1);
-    if (k < kBalanceRounds * kCusPerXcd) {
-      s_tile[r][k] = t;
-      s_len[r][k]  = (int) min(len, (int64_t) (1 << 25) - 1);
-    } else {
-      tile_order[position(r, k)] = t;
-    }
-  }
-  __syncthreads();
-  // The first rounds of a region, one wavefront per region, lane c = the c-th longest tile of the round: the CUs are
-  // sorted by the work they hold so far (bitonic network over the lanes) and the c-th longest tile goes to the CU with
-  // the c-th smallest load. Round 0 keeps its order, round 1 comes out reversed, later rounds even out what is left.
-  {
-    const int lane = threadIdx.x & 63, r = threadIdx.x >> 6;
-    if (r < kOrderRegions && lane < kCusPerXcd) {
-      unsigned key = (unsigned) lane;  // (load << 5) | cu, loads up to 2^27 - 1: four lists of 2^25 - 1 at most
-      const int n = s_total[r];
-      for (int j = 0; j < kBalanceRounds && j * kCusPerXcd < n; ++j) {
-        const int k = j * kCusPerXcd + lane;
-        if ((j + 1) * kCusPerXcd > n) {  // a partial last round keeps its order
-          if (k < n) tile_order[position(r, k)] = s_tile[r][k];
-          break;
-        }
-        if (j > 0)  // every load is zero before the first round
-#pragma unroll
-          for (int size = 2; size <= kCusPerXcd; size <<= 1)
-#pragma unroll
-            for (int d = size >> 1; d > 0; d >>= 1) {
-              const unsigned other = (unsigned) __shfl_xor((int) key, d, kCusPerXcd);
-              const bool up = (lane & size) == 0, low = (lane & d) == 0;
-              key = (low == up) ? min(key, other) : max(key, other);
-            }
-        const int cu = (int) (key & (kCusPerXcd - 1));
-        tile_order[position(r, j * kCusPerXcd + cu)] = s_tile[r][k];
-        key += (unsigned) s_len[r][k] << 5;
-      }
-    }
+    int k             = atomicAdd(&s_count[r][length_bucket(len)], 1);
+    const int round   = k / kCusPerXcd;
+    if ((round & 1) && round < kBalanceRounds && (round + 1) * kCusPerXcd <= s_total[r]) k = (2 * round + 1) * kCusPerXcd - 1 - k;
+    tile_order[position(r, k)] = t;
   }
 }
 
@@ -390,16 +350,6 @@ template <int kCtrl, int kRowMask, int kBankMask>
 __device__ __forceinline__ float dpp_shift_zero(float v) {
   return __builtin_bit_cast(
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, kRowMask, kBankMask, true));
-}
-
-// Inclusive prefix sums over the 64 lanes.
-template <int kCtrl, int kRows>
-__device__ __forceinline__ int scan_step(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, true);
-}
-__device__ __forceinline__ int wave_scan(int v) {
-  v = scan_step<0x111, 0xf>(v), v = scan_step<0x112, 0xf>(v), v = scan_step<0x114, 0xf>(v), v = scan_step<0x118, 0xf>(v);
-  return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
 }
 
 // Largest of the 64 lanes' values; valid in lane 63 only.

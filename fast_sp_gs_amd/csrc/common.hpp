@@ -65,6 +65,16 @@ __device__ __forceinline__ void wave_lds_sync() {
 // the compiler materialise the predicate in a register and compare it again.
 __device__ __forceinline__ unsigned long long wave_ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 
+// Inclusive prefix sums over the 64 lanes.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int scan_step(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, true);
+}
+__device__ __forceinline__ int wave_scan(int v) {
+  v = scan_step<0x111, 0xf>(v), v = scan_step<0x112, 0xf>(v), v = scan_step<0x114, 0xf>(v), v = scan_step<0x118, 0xf>(v);
+  return scan_step<0x143, 0xc>(scan_step<0x142, 0xa>(v));
+}
+
 // Makes a value opaque at this point of a loop, so that what is computed from it is not hoisted out: a long inner loop
 // beside it keeps the registers that the hoisted values would hold.
 __device__ __forceinline__ int keep_local(int v) {
