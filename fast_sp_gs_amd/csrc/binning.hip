@@ -312,6 +312,7 @@ __global__ void __launch_bounds__(256) cull_mask_kernel(int P, int gx, int gy, c
 // Layout of the `bins` buffer of the bucket binning: the queue length of the long segments in front of the B x T matrix
 // of per-(walk block, tile) instance counts.
 constexpr int kPrefixTiles = 64, kPrefixWaves = 16, kPrefixChunk = 32;  // walk blocks <= kPrefixWaves * kPrefixChunk
+constexpr size_t kBinsExceeds = 8;  // behind queue length and instance count: there is no room for them
 constexpr size_t kBinsSums = 256;  // behind the queue length: the instances of every 64 tiles
 constexpr size_t kBinsHeader = 4096;
 static_assert(kBinsSums + (kMaxLdsTiles / kPrefixTiles) * sizeof(uint32_t) <= kBinsHeader, "the sums fit the header");
@@ -353,6 +354,7 @@ __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, i
   __shared__ unsigned s_count[kTiles];
   // first of all, so that the instance count reaches the host while the rest of the counting is still running
   if (publish.counters && blockIdx.x == 0 && threadIdx.x < kWave) publish_slot_regions(publish);
+  if (!publish.counters && publish.exceeds && blockIdx.x == 0 && threadIdx.x == 0) *publish.exceeds = 0;
   const int T = gx * gy;
   for (int t = threadIdx.x; t < T; t += blockDim.x) s_count[t] = 0u;
   __syncthreads();
@@ -463,13 +465,19 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
 // With `sums` (the instances of every 64 tiles) block b scans the tiles from 4096 b on and adds what lies in front of them
 // itself; without, one block walks all tiles.
 // ends = false: ranges[t] = (start, start), for a scatter that advances ranges[t].y; ends = true: (start, end).
+// exceeds (optional): set when there is no room for the instances; all ranges are empty then.
 __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long long* __restrict__ ranges,
                                                          const uint32_t* __restrict__ sums, int* __restrict__ large_count,
-                                                         bool ends) {
+                                                         bool ends, const int* __restrict__ exceeds) {
   __shared__ unsigned long long s_wave[16];
   const int lane = __lane_id(), wave = threadIdx.x / kWave;
   unsigned long long carry = 0;
   const int first = sums ? blockIdx.x * 4096 : 0, last = sums ? min(T, first + 4096) : T;
+  if (exceeds && *exceeds) {
+    for (int t = first + (int) threadIdx.x; t < last; t += blockDim.x) ranges[2 * (size_t) t] = 0, ranges[2 * (size_t) t + 1] = 0;
+    if (threadIdx.x == 0 && last == T) large_count[0] = 0, large_count[1] = 0;
+    return;
+  }
   if (first > 0) {
     unsigned long long before = 0;
     for (int b = threadIdx.x; b < first / kPrefixTiles; b += blockDim.x) before += sums[b];
@@ -513,8 +521,9 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
 constexpr int kColumn = 64;
 
 __global__ void __launch_bounds__(1024) tile_prefix_scan_kernel(int T, int B, uint32_t* __restrict__ hist,
-    unsigned long long* __restrict__ ranges, int* __restrict__ large_count) {
+    unsigned long long* __restrict__ ranges, int* __restrict__ large_count, const int* __restrict__ exceeds) {
   __shared__ uint32_t s_wave[16];
+  const bool room = !exceeds || *exceeds == 0;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   uint32_t c[kColumn], sum = 0;
 #pragma unroll
@@ -548,7 +557,7 @@ __global__ void __launch_bounds__(1024) tile_prefix_scan_kernel(int T, int B, ui
   }
   if (t < T) {
     const uint32_t start = before + inc - sum;
-    ranges[2 * (size_t) t] = start, ranges[2 * (size_t) t + 1] = start + sum;
+    ranges[2 * (size_t) t] = room ? start : 0, ranges[2 * (size_t) t + 1] = room ? start + sum : 0;
     uint32_t run = 0;
 #pragma unroll
     for (int i = 0; i < kColumn; ++i) {
@@ -1243,12 +1252,14 @@ namespace {
 
 // First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
 // (start, end); the header of `bins` is set (length of the long-segment queue: 0 | instances in all tiles).
+// With publish.capacity the ranges stay empty when there are more instances than that.
 int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in, int64_t* ranges,
-               void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
+               void* bins, hipStream_t s, SlotPublish publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
   int* header = (int*) bins;
+  if (publish.capacity > 0) publish.exceeds = (int*) ((char*) bins + kBinsExceeds);
   const BinsLayout bl = bins_layout(P, T);
   if (bl.blocks > 0) {
     uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
@@ -1259,11 +1270,13 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
                          hist, publish);
     });
     if (T <= 1024 && bl.blocks <= kColumn) {
-      hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header);
+      hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header,
+                         (const int*) publish.exceeds);
     } else {
       hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
                          bl.blocks, hist, rng, sums);
-      hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
+      hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true,
+                         (const int*) publish.exceeds);
     }
     // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
     // sorts) is built from them by an extra block of the scatter, in the second part.
@@ -1275,7 +1288,8 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
       FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, false>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx,
                                                gy, (int64_t) 0, (const float2*) means2D, (const float*) nullptr, radii, in,
                                                rng, (uint64_t*) nullptr));
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, (const uint32_t*) nullptr, header, false);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, (const uint32_t*) nullptr, header, false,
+                       (const int*) nullptr);
   }
   return check_launch("gs_prepare_count");
 }
@@ -1550,6 +1564,52 @@ FSGS_API int fsgs_gs_2d_fast_view_fill(int P, int W, int H, const float* means2D
     return fail(kWorkspaceSmall, "gs_2d_fast_view_fill: workspace %zu < %zu or bins %zu < %zu bytes", workspace_bytes,
                 sort_workspace_bytes(R), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
   return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{inverse_m, opacities, keep_masks}, R, ranges, point_list,
+                   nullptr, workspace, bins, false, (hipStream_t) stream);
+}
+
+// What the views call: both parts, for either kind of surfels (inverse_m and opacities: the fast ones) and Gaussians.
+namespace {
+WalkInputs view_inputs(const float* inverse_m, const float* opacities, const uint32_t* keep_masks) {
+  return inverse_m ? WalkInputs{inverse_m, opacities, keep_masks}
+                   : WalkInputs{nullptr, nullptr, culling_enabled() ? keep_masks : nullptr};
+}
+}  // namespace
+
+FSGS_API size_t fsgs_gs_view_fill_workspace_bytes(int64_t R) {
+  return sort_layout(R).keys1 + align_up((size_t) (R / kSmallSegment + 1) * sizeof(int), 256);  // entries, queue of long segments
+}
+
+FSGS_API int fsgs_gs_view_tally(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
+                                const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters,
+                                int32_t* slot_regions, int64_t* num_rendered_host, int64_t capacity, int64_t* ranges, void* bins,
+                                size_t bins_bytes, void* stream) {
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins && capacity >= 0, "gs_view_tally: bad arguments");
+  FSGS_REQUIRE(means2D && radii && !slot_counters == !num_rendered_host && (!inverse_m || (opacities && keep_masks)),
+               "gs_view_tally: null pointer");
+  if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
+    return fail(kWorkspaceSmall, "gs_view_tally: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+  tile_order_invalidate((hipStream_t) stream);
+  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  return fill_count(P, W, H, means2D, radii, view_inputs(inverse_m, opacities, keep_masks), ranges, bins, (hipStream_t) stream,
+                    SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host, std::max<int64_t>(capacity, 1)});
+}
+
+FSGS_API int fsgs_gs_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                               const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity,
+                               int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && capacity >= 0 && ranges && bins, "gs_view_fill: bad arguments");
+  FSGS_REQUIRE(capacity < (int64_t) 0x7fffffff, "gs_view_fill: %lld instances exceed the 2^31-1 limit", (long long) capacity);
+  FSGS_REQUIRE(means2D && depths && radii && (capacity == 0 || (point_list && workspace)) &&
+                   (!inverse_m || (opacities && keep_masks)), "gs_view_fill: null pointer");
+  if (capacity == 0) {
+    launch_zero_ranges(((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile), ranges, (hipStream_t) stream);
+    return check_launch("gs_view_fill");
+  }
+  if (workspace_bytes < fsgs_gs_view_fill_workspace_bytes(capacity) || bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
+    return fail(kWorkspaceSmall, "gs_view_fill: workspace %zu < %zu or bins %zu < %zu bytes", workspace_bytes,
+                fsgs_gs_view_fill_workspace_bytes(capacity), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+  return fill_sort(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, point_list,
                    nullptr, workspace, bins, false, (hipStream_t) stream);
 }
 

@@ -148,6 +148,19 @@ int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t*
                        uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges,
                        void* bins, size_t bins_bytes, void* stream);
 int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream);
+/* Both parts as the views run them, for surfels and 3D Gaussians (inverse_m and opacities nullptr; keep_masks optional) and for the
+ * "fast" surfels (all three given). `ranges` is complete once fsgs_gs_view_fill has run, and not before; point_list[capacity]
+ * behind the kept instances is not written. `capacity` (the same for both) is the instance count, or a guess made before it is
+ * known, so that the fill and the blend can be queued without waiting: if there are more instances all ranges are left empty, and
+ * both are called again with the count, the tally without slot_counters, slot_regions and num_rendered_host (they were
+ * served by the first). */
+size_t fsgs_gs_view_fill_workspace_bytes(int64_t capacity);
+int fsgs_gs_view_tally(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
+                       const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
+                       int64_t* num_rendered_host, int64_t capacity, int64_t* ranges, void* bins, size_t bins_bytes, void* stream);
+int fsgs_gs_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                      const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity, int64_t* ranges,
+                      int32_t* point_list, void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes, void* stream);
 /* The two parts for the "fast" surfels (tiles that pass the corner test; keep_masks of the preprocess). Unlike
  * fsgs_gs_2d_fast_prepare_fill no padding entries are written behind the kept instances. */
 int fsgs_gs_2d_fast_view_count(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
