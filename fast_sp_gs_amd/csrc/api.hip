@@ -19,13 +19,13 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
-// blockIdx -> tile tables of the blend kernels (see blend.hpp): kTableSlots tables of kMaxOrderedTiles ints each in a
+// blockIdx -> tile tables of the blend kernels (see blend.hpp): kTableSlots tables of kTableInts ints each in a
 // file-scope device array, so the library never calls hipMalloc. A (device, stream) pair takes a free slot on its first
 // binning or blend call and keeps it until fsgs_stream_release or the end of the process; when every slot of a device
 // is taken, further streams get no table and their blocks map to tiles directly (same results, no longest-first order).
 // Slots are never taken away from a stream behind its back: a kernel of that stream may still be reading the table.
 constexpr int kTableSlots   = 8;
-constexpr int kTableInts    = 1 << 16;  // == kMaxOrderedTiles
+constexpr int kTableInts    = kMaxOrderedTiles + kScheduleInts;
 constexpr int kMaxDevices   = 64;
 static __device__ __align__(256) int g_tile_order_tables[kTableSlots][kTableInts];
 

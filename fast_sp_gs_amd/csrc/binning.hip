@@ -437,7 +437,8 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
   // final, nothing in this kernel reads the table, and the per-tile sorts and the blend kernels that follow do.
   if (order_table && blockIdx.x == gridDim.x - 1) {
     static_assert(sizeof(TileOrderLds) <= sizeof(s_cursor), "the schedule's LDS fits the cursor array");
-    build_tile_order(gx, gy, (const int64_t*) ranges, order_table, *reinterpret_cast<TileOrderLds*>(s_cursor));
+    build_tile_order(gx, gy, (const int64_t*) ranges, order_table, order_table + kMaxOrderedTiles,
+                     *reinterpret_cast<TileOrderLds*>(s_cursor));
     return;
   }
   const int T = gx * gy;

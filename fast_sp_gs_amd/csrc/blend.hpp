@@ -218,10 +218,9 @@ __device__ __forceinline__ unsigned quadrant_mask(const SplatHot& h, int tile_px
 // deals no better, blends of 300k surfels 800x800 99 + 229 us against 97 + 226, and the 45 exchanges of its networks held up
 // the scatter, whose extra block builds the table: 15.7 -> 12.8 us.) Later rounds go wherever a slot frees up; for them
 // descending order is what balances.
-// The table is kMaxOrderedTiles ints in a file-scope device array of the library (no allocation), one slot per
+// The table is kMaxOrderedTiles ints, and two of ScheduleInt, in a file-scope device array of the library (no allocation), one slot per
 // (device, stream) that bins or blends: calls on one stream are ordered by the stream, calls on different streams use
 // different tables, and a stream that finds every slot taken runs without a table.
-constexpr int kMaxOrderedTiles = 1 << 16;
 constexpr int kOrderFracBits   = 4;  // buckets per octave of list length = 2^this
 constexpr int kOrderFrac       = 1 << kOrderFracBits;
 constexpr int kOrderBuckets    = 32 * kOrderFrac;
@@ -232,6 +231,11 @@ constexpr int kCusPerXcd       = 32;  // compute units behind one region's table
 constexpr int kBalanceRounds   = 4;
 
 // (tile_order_table, tile_order_invalidate and tile_order_release are declared in common.hpp.)
+
+// What a table says beside the order: the list entries per slot, of which the card has kCus * 4 (blocks of the blend backward
+// that run at a time), and the number of heavy tiles, those of more than an eighth of that.
+enum ScheduleInt : int { kShare = 0, kHeavyTiles = 1 };
+constexpr int kCus = kOrderRegions * kCusPerXcd;
 
 namespace {
 
@@ -258,22 +262,33 @@ __device__ __forceinline__ int tile_region(int t, int gx, int gy) {
 struct TileOrderLds {
   int count[kOrderRegions][kOrderBuckets];
   int total[kOrderRegions];
+  unsigned entries;
+  int heavy[kOrderRegions];
 };
 
 // The work of one whole block (any number of wavefronts): either a launch of its
 // own (tile_order_kernel) or one extra block of a kernel that has nothing to do with it but runs at the right time --
 // the binning's scatter, whose other blocks keep the chip busy while this one orders 2 500 numbers (a single-block
 // launch of its own holds up the stream for 10 us).
+// `schedule` (optional) receives the ints behind the table.
 __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* __restrict__ ranges,
-                                                 int* __restrict__ tile_order, TileOrderLds& lds) {
+                                                 int* __restrict__ tile_order, int* __restrict__ schedule, TileOrderLds& lds) {
   auto& s_count = lds.count;
   auto& s_total = lds.total;
   const int T = gx * gy;
   for (int b = threadIdx.x; b < kOrderRegions * kOrderBuckets; b += blockDim.x) (&s_count[0][0])[b] = 0;
+  if (threadIdx.x == 0) lds.entries = 0u;
   __syncthreads();
-  for (int t = threadIdx.x; t < T; t += blockDim.x)
-    atomicAdd(&s_count[tile_region(t, gx, gy)][length_bucket(ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t])], 1);
+  int entries = 0;
+  for (int t = threadIdx.x; t < T; t += blockDim.x) {
+    const int64_t len = ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t];
+    atomicAdd(&s_count[tile_region(t, gx, gy)][length_bucket(len)], 1);
+    entries += (int) len;
+  }
+  entries = wave_scan(entries);
+  if ((threadIdx.x & 63) == 63 && entries != 0) atomicAdd(&lds.entries, (unsigned) entries);
   __syncthreads();
+  const int share = (int) (lds.entries / (4 * kCus)), light = length_bucket(share / 8);
   // exclusive prefix from the longest bucket down, a wavefront per region
   for (int r = threadIdx.x >> 6; r < kOrderRegions; r += blockDim.x >> 6) {
     const int lane = threadIdx.x & 63;
@@ -284,7 +299,12 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
     const int inc = wave_scan(sum);
     int run = inc - sum;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) s_count[r][kOrderBuckets - 1 - (lane * kPer + i)] = run, run += c[i];
+    for (int i = 0; i < kPer; ++i) {
+      const int b = kOrderBuckets - 1 - (lane * kPer + i);
+      s_count[r][b] = run;
+      if (b == light) lds.heavy[r] = run;  // tiles of longer buckets
+      run += c[i];
+    }
     if (lane == 63) s_total[r] = inc;
   }
   __syncthreads();
@@ -295,6 +315,11 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
     for (int q = 0; q < kOrderRegions; ++q) pos += min(s_total[q], k) + ((q < r && s_total[q] > k) ? 1 : 0);
     return pos;
   };
+  if (schedule && threadIdx.x == 0) {
+    int heavy = 0;
+    for (int r = 0; r < kOrderRegions; ++r) heavy += lds.heavy[r];
+    schedule[kShare] = share, schedule[kHeavyTiles] = heavy;
+  }
   for (int t = threadIdx.x; t < T; t += blockDim.x) {
     const int r       = tile_region(t, gx, gy);
     const int64_t len = ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t];
@@ -306,9 +331,9 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
 }
 
 __global__ void __launch_bounds__(1024) tile_order_kernel(int gx, int gy, const int64_t* __restrict__ ranges,
-                                                          int* __restrict__ tile_order) {
+                                                          int* __restrict__ tile_order, int* __restrict__ schedule) {
   __shared__ TileOrderLds lds;
-  build_tile_order(gx, gy, ranges, tile_order, lds);
+  build_tile_order(gx, gy, ranges, tile_order, schedule, lds);
 }
 
 // Launch flags of the blend kernels: bit 0 = the tile table was built for this launch (T small enough; otherwise blocks
@@ -320,7 +345,8 @@ inline int launch_tile_order(int gx, int gy, const int64_t* ranges, hipStream_t 
   bool rebuild = false;
   int* t = tile_order_table(s, ranges, gx, gy, &rebuild);
   if (!t) return flags;
-  if (rebuild) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, gx, gy, ranges, t);
+  if (rebuild) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, gx, gy, ranges, t,
+                                  t + kMaxOrderedTiles);
   *table = t;
   return flags | kFlagOrdered;
 }
@@ -342,6 +368,33 @@ inline int defer_tile_order(int gx, int gy, const int64_t* ranges, hipStream_t s
 __device__ __forceinline__ int scheduled_tile(int flags, const int* __restrict__ tile_order) {
   return (flags & kFlagOrdered) ? tile_order[blockIdx.x] : (int) blockIdx.x;
 }
+
+// Priority of a backward block's wavefronts among those on its compute unit: the more entries a block has left, the higher.
+// Left to itself the hardware serves the wavefronts that came first, those of the longest lists; but a long list is often cut
+// short, where its pixels saturate, and then a list of half its length is the one that the launch waits for. With priorities
+// the blocks that share a compute unit end together.
+// Only if all heavy tiles start at once (at most kPerCu blocks per compute unit): then what remains is to end together. With
+// more of them, blocks that end together leave the next ones to start together, on a card that was idle meanwhile.
+// 300k surfels, backward, us without -> with priorities: 700x700 217 -> 208, 800x800 226 -> 206 (930 heavy tiles), 850x850 243
+// -> 246, 900x900 266 -> 277, 950x950 279 -> 302; 300k Gaussians (five blocks per compute unit) 800x800 138 -> 118, 900x900 153
+// -> 135, 1000x700 171 -> 169. Without the condition 1M surfels 1352x900 269 -> 283. Priorities in the forwards, whose blocks do not
+// know how far down their lists they will get: 300k surfels equal, 3M 309 -> 320.
+template <int kPerCu>
+struct BlockPriority {
+  int share;  // list entries per slot; 0: no priorities
+  __device__ __forceinline__ BlockPriority(int flags, const int* __restrict__ tile_order) : share(0) {
+    if (!(flags & kFlagOrdered)) return;
+    const int* schedule = tile_order + kMaxOrderedTiles;
+    if (schedule[kHeavyTiles] <= kPerCu * kCus) share = schedule[kShare];
+  }
+  __device__ __forceinline__ void set(int remaining) const {
+    if (share == 0) return;
+    if (remaining > share / 3) __builtin_amdgcn_s_setprio(3);
+    else if (remaining > share / 6) __builtin_amdgcn_s_setprio(2);
+    else if (remaining > share / 12) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+  }
+};
 
 }  // namespace
 

@@ -20,7 +20,8 @@
 // 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260
 // instructions less per staged wavefront, for 7 us more in the forward) 245, 805 and 36; with batches of up to 128 entries
 // whose rows share out one pool of places, instead of 96 with 24 places a row, and a flush that waits for no entry's rows one by
-// one, 230, 782 and 37. One tile of 1800 entries alone, which the launch cannot be shorter than: 179 -> 127.
+// one, 230, 782 and 37; with priorities (BlockPriority) 206 at 300k. One tile of 1800 entries alone, which the launch cannot be
+// shorter than: 179 -> 127.
 #include <algorithm>
 
 #include "block_lists.hpp"
@@ -173,7 +174,9 @@ blend_backward_kernel(
   };
   gather(0);
 
+  const BlockPriority<4> priority(ordered, tile_order);
   for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    priority.set(n_todo - done);
     const int n_staged = min(kRowBatch, n_todo - done);
     if ((int) threadIdx.x < kRowBatch) {
       const int e = (int) threadIdx.x;

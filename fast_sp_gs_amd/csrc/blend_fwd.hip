@@ -327,7 +327,8 @@ FSGS_API int fsgs_debug_tile_order(int gx, int gy, const int64_t* ranges, int32_
   using namespace fsgs;
   FSGS_REQUIRE(gx > 0 && gy > 0 && (int64_t) gx * gy <= kMaxOrderedTiles && ranges && table,
                "debug_tile_order: bad arguments (at most %d tiles)", kMaxOrderedTiles);
-  hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, (hipStream_t) stream, gx, gy, ranges, table);
+  hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, (hipStream_t) stream, gx, gy, ranges, table,
+                     (int*) nullptr);
   return check_launch("debug_tile_order");
 }
 

@@ -119,6 +119,9 @@ __device__ __forceinline__ TileRect tile_rect(float px, float py, int r, int gx,
 // top-k, extra channels) reuse it. A ranges buffer rewritten behind the library's back (or binned on another stream)
 // keeps an older frame's order: still a permutation of the same tile grid, so every tile is processed exactly once --
 // only the longest-first order is stale. All three functions take the same lock.
+// Behind a table's kMaxOrderedTiles entries stand kScheduleInts ints: the lists' work (see ScheduleInt in blend.hpp).
+constexpr int kMaxOrderedTiles = 1 << 16;
+constexpr int kScheduleInts    = 64;
 int* tile_order_table(hipStream_t stream, const int64_t* ranges, int gx, int gy, bool* rebuild);
 void tile_order_invalidate(hipStream_t stream);
 void tile_order_release(hipStream_t stream);

@@ -589,7 +589,9 @@ __global__ void __launch_bounds__(kBlendThreads)
   };
   gather(0);
 
+  const BlockPriority<4> priority(ordered, tile_order);
   for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    priority.set(n_todo - done);
     const int n_staged = min(kB, n_todo - done);
     if ((int) threadIdx.x < kB) {
       const int e = (int) threadIdx.x;

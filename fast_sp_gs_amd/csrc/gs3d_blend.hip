@@ -521,7 +521,9 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
     if (kSlots) next_radius = radii[next.id], next_off = next.id == 0 ? 0 : point_offsets[next.id - 1];
   };
   gather(0);
+  const BlockPriority<E == 0 ? 5 : 4> priority(flags, tile_order);
   for (int done = 0, parity = 0; done < n_todo; parity ^= 1) {
+    priority.set(n_todo - done);
     const int n_staged = min(kB, n_todo - done);
     if ((int) threadIdx.x < kB) {
       const int e = (int) threadIdx.x;
