@@ -328,65 +328,93 @@ constexpr int kGradFloats = 18;  // 0-2 colours | 3-11 transform | 12-14 normal 
 constexpr int kSumStride  = 19;
 
 // Sums of the records of the wavefront's 64 surfels, in position order, to s_sums[64][kSumStride] (rows of surfels that
-// were not rendered stay as they are). Nine lanes of a surfel read a record's 72 bytes; rendered surfels are taken seven at
-// a time and three such groups together, four kept positions of each surfel in flight, so the wavefront pays a handful of
-// trips to memory for all of its surfels. `vis`: this lane's surfel was rendered.
+// were not rendered stay as they are), with kSumScratch floats of scratch behind them. `vis`: this lane's surfel was rendered.
 // `first`, `count` and `mask` are its span and keep mask (any values where it was not).
+// Spans that a mask word covers: nine lanes of a surfel read a record's 72 bytes; surfels are taken seven at
+// a time and three such groups together, four kept positions of each surfel in flight, so the wavefront pays a handful of
+// trips to memory for all of them.
+// A longer span is complete, 72 bytes a position without gaps: the wavefront fetches 64 positions at a time, the next ones while it
+// adds the present ones from LDS, a component per lane. Four positions a trip, a surfel near the camera with hundreds of tiles
+// kept its wavefront, and with it the launch, for a hundred trips. Kernel, us: 300k surfels 800x800 64 -> 51, 3M 1352x1014
+// 393 -> 370, 1M 1352x900 182 -> 131, 30k 1000x1000 33 -> 16.5, 10k 256x256 11.4 -> 11.0; six positions in flight 50, 367 and 11.6.
+constexpr int kSumChunk = kWave, kSumScratch = kSumChunk * kGradFloats;
+constexpr int kSumFloats = kWave * kSumStride + kSumScratch;  // of a wavefront
+
 __device__ __forceinline__ void wave_record_sums(const ViewRecords& in, int first, int count, uint32_t mask, bool vis,
                                                  float* __restrict__ s_sums) {
   static_assert(kCullMaskTiles == 32, "a mask word holds a small rectangle's positions");
   constexpr int kLanes = kGradFloats / 2, kPerPass = 7, kGroups = 3, kDepth = 4;
   const int lane = (int) __lane_id(), sub = lane / kLanes, k = lane - sub * kLanes;
-  const unsigned long long live_mask = __ballot(vis);
+  const bool small = vis && count <= kCullMaskTiles;
+  if (count < kCullMaskTiles) mask &= (1u << max(count, 0)) - 1u;
+  const unsigned long long live_mask = wave_ballot(small);
   const int live = __popcll(live_mask);
-  // lane r of the first `live` lanes learns which lane holds the r-th rendered surfel
+  // lane r of the first `live` lanes learns which lane holds the r-th of them
   const int before = __popcll(live_mask & ((1ull << lane) - 1ull));
-  const int holder = __builtin_amdgcn_ds_permute((vis ? before : live + lane - before) * 4, lane);
+  const int holder = __builtin_amdgcn_ds_permute((small ? before : live + lane - before) * 4, lane);
   for (int r0 = 0; r0 < live; r0 += kGroups * kPerPass) {
     const float2* src[kGroups];
-    int who[kGroups], cnt[kGroups], most = 0;
-    uint32_t keep[kGroups];
+    int who[kGroups];
+    uint32_t bits[kGroups];
     float2 acc[kGroups];
 #pragma unroll
     for (int q = 0; q < kGroups; ++q) {
       const int r   = r0 + q * kPerPass + sub;
       const bool on = sub < kPerPass && r < live;
       who[q] = __shfl(holder, on ? r : 0, 64);
-      const int e = __shfl(first, who[q], 64), c = __shfl(count, who[q], 64);
-      keep[q] = __shfl(mask, who[q], 64);
-      cnt[q]  = on ? c : 0;
-      who[q]  = on ? who[q] : -1;
+      const int e = __shfl(first, who[q], 64);
+      bits[q] = __shfl(mask, who[q], 64);
+      if (!on) who[q] = -1, bits[q] = 0u;
       src[q]  = (const float2*) in.records + (size_t) e * kLanes + k;
       acc[q]  = make_float2(0.0f, 0.0f);
-      most    = max(most, cnt[q]);
     }
-    for (int base = 0; __ballot(base < most) != 0ull; base += 32) {
-      uint32_t bits[kGroups];
+    while (wave_ballot((bits[0] | bits[1] | bits[2]) != 0u) != 0ull) {
+      float2 v[kGroups][kDepth];
 #pragma unroll
-      for (int q = 0; q < kGroups; ++q) {
-        const int left = cnt[q] - base;
-        bits[q] = left <= 0 ? 0u : left >= 32 ? 0xffffffffu : (1u << left) - 1u;
-        if (cnt[q] <= kCullMaskTiles) bits[q] &= keep[q];
-      }
-      while (__ballot((bits[0] | bits[1] | bits[2]) != 0u) != 0ull) {
-        float2 v[kGroups][kDepth];
+      for (int q = 0; q < kGroups; ++q)
 #pragma unroll
-        for (int q = 0; q < kGroups; ++q)
+        for (int j = 0; j < kDepth; ++j) {
+          v[q][j] = make_float2(0.0f, 0.0f);
+          if (bits[q]) v[q][j] = src[q][(size_t) __builtin_ctz(bits[q]) * kLanes];
+          bits[q] &= bits[q] - 1u;
+        }
 #pragma unroll
-          for (int j = 0; j < kDepth; ++j) {
-            v[q][j] = make_float2(0.0f, 0.0f);
-            if (bits[q]) v[q][j] = src[q][(size_t) (base + __builtin_ctz(bits[q])) * kLanes];
-            bits[q] &= bits[q] - 1u;
-          }
+      for (int q = 0; q < kGroups; ++q)
 #pragma unroll
-        for (int q = 0; q < kGroups; ++q)
-#pragma unroll
-          for (int j = 0; j < kDepth; ++j) acc[q].x += v[q][j].x, acc[q].y += v[q][j].y;
-      }
+        for (int j = 0; j < kDepth; ++j) acc[q].x += v[q][j].x, acc[q].y += v[q][j].y;
     }
 #pragma unroll
     for (int q = 0; q < kGroups; ++q)
       if (who[q] >= 0) s_sums[who[q] * kSumStride + 2 * k] = acc[q].x, s_sums[who[q] * kSumStride + 2 * k + 1] = acc[q].y;
+  }
+  float2* const s_chunk = (float2*) (s_sums + kWave * kSumStride);
+  for (unsigned long long todo = wave_ballot(vis && !small); todo != 0ull; todo &= todo - 1ull) {
+    const int holds = (int) __builtin_ctzll(todo);
+    const int e = __builtin_amdgcn_readlane(first, holds), c = __builtin_amdgcn_readlane(count, holds);
+    const float2* span = (const float2*) in.records + (size_t) e * kLanes;
+    float2 v[kLanes];
+    auto fetch = [&](int base) {
+#pragma unroll
+      for (int j = 0; j < kLanes; ++j) {
+        const int at = j * kWave + lane;  // of the chunk's kSumChunk * kLanes pieces
+        v[j] = at < (c - base) * kLanes ? span[(size_t) base * kLanes + at] : make_float2(0.0f, 0.0f);
+      }
+    };
+    float acc = 0.0f;
+    fetch(0);
+    for (int base = 0; base < c; base += kSumChunk) {
+      wave_lds_sync();
+#pragma unroll
+      for (int j = 0; j < kLanes; ++j) s_chunk[j * kWave + lane] = v[j];
+      wave_lds_sync();
+      if (base + kSumChunk < c) fetch(base + kSumChunk);
+      if (lane < kGradFloats) {
+        const float* s = (const float*) s_chunk + lane;
+#pragma unroll 16
+        for (int r = 0; r < kSumChunk; ++r) acc += s[r * kGradFloats];  // zeros behind the span's end
+      }
+    }
+    if (lane < kGradFloats) s_sums[holds * kSumStride + lane] = acc;
   }
 }
 
@@ -407,7 +435,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : kRecords ? kShStageRows * kSumStride : 1];
+  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : kRecords ? 4 * kSumFloats : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
@@ -447,7 +475,8 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       for (int k = 0; k < 3; ++k) col[k] = colors[3 * (size_t) i + k];
   }
   if (kRecords) {  // the rows of coefficients and the above are on their way meanwhile
-    float* s_sums = &s_rows[(threadIdx.x & ~63) * (kStage ? kStride : kSumStride)];
+    static_assert(!kStage || 64 * kStride >= kSumFloats, "the sums fit where the rows will be");
+    float* s_sums = &s_rows[kStage ? (threadIdx.x & ~63) * kStride : (threadIdx.x >> 6) * kSumFloats];
     wave_record_sums(view, first, count, mask, vis, s_sums);
     wave_lds_sync();
     if (vis) {
