@@ -380,18 +380,26 @@ fast_blend_forward_kernel(
 constexpr int kFastGradSlots  = 21;
 constexpr int kFastRecordSlots = 22;  // a record of the ordered-sum path: the 21 slots + one float of padding
 
-// Where slot_sum_kernel puts component c of surfel i: 0-2 colours | 3-11 inverse transform | 12-15 normal, opacity |
+// Where the sums of a surfel go: 0-2 colours | 3-11 inverse transform | 12-15 normal, opacity |
 // 16-18 third row of the transform (the other two rows get no gradient from the blend: zeros) | 19-20 means2D.
 struct FastScatter {
   float *g_means2D, *g_normal_opacity, *g_colors, *g_trans, *g_inv;
-  __device__ __forceinline__ void operator()(int i, int c, float v) const {
-    if (c < 3) g_colors[3 * (size_t) i + c] = v;
-    else if (c < 12) g_inv[9 * (size_t) i + (c - 3)] = v;
-    else if (c < 16) g_normal_opacity[4 * (size_t) i + (c - 12)] = v;
-    else if (c < 19) {
-      g_trans[9 * (size_t) i + 6 + (c - 16)] = v;
-      g_trans[9 * (size_t) i + 2 * (c - 16)] = 0.0f, g_trans[9 * (size_t) i + 2 * (c - 16) + 1] = 0.0f;
-    } else if (c < 21) g_means2D[2 * (size_t) i + (c - 19)] = v;
+  // Rows of n surfels from i0 on, by a wavefront: consecutive lanes write consecutive addresses.
+  template <int kSurfels, int kStride>
+  __device__ __forceinline__ void rows(const float* __restrict__ s_sums, int i0, int n) const {
+    auto table = [&](auto width, float* g, auto value) {
+      constexpr int kWidth = decltype(width)::value;
+#pragma unroll
+      for (int t0 = 0; t0 < kSurfels * kWidth; t0 += kWave) {
+        const int t = t0 + (int) __lane_id(), r = t / kWidth, c = t - r * kWidth;
+        if (t < n * kWidth) g[(size_t) kWidth * i0 + t] = value(s_sums + r * kStride, c);
+      }
+    };
+    table(std::integral_constant<int, 3>(), g_colors, [](const float* s, int c) { return s[c]; });
+    table(std::integral_constant<int, 9>(), g_inv, [](const float* s, int c) { return s[3 + c]; });
+    table(std::integral_constant<int, 4>(), g_normal_opacity, [](const float* s, int c) { return s[12 + c]; });
+    table(std::integral_constant<int, 9>(), g_trans, [](const float* s, int c) { return c < 6 ? 0.0f : s[10 + c]; });
+    table(std::integral_constant<int, 2>(), g_means2D, [](const float* s, int c) { return s[19 + c]; });
   }
 };
 
@@ -399,67 +407,130 @@ struct FastScatter {
 // only the tiles that pass the binning's corner test are in a tile list, and only those positions were written by the
 // blend (a list entry's record by the flush of its batch, or zeros by its tile's block if the entry lies behind the
 // deepest contributor). The test is repeated here, with the binning's own arithmetic, so the other positions are
-// neither cleared nor read. 11 lanes per surfel, each owning one float2 of the 88-byte record: a step covers 11
-// positions of the span -- lane k tests position base + k, the 11 verdicts are shared through a ballot, and the
-// records of the positions that passed are requested together.
-// `keep_masks` (optional, what the preprocess kernel left): the verdicts for rectangles of at most 32 tiles, bit = position
-// in the span; a wavefront none of whose surfels has a larger rectangle then reads neither the adjugates nor the opacity
-// and does not set the test up.
+// neither cleared nor read. `keep_masks` (optional, what the preprocess kernel left): the verdicts for rectangles of at most
+// 32 tiles, bit = position in the span.
+// A wavefront takes 20 surfels. Spans of up to 32 positions: 11 lanes of a surfel read a record's 88 bytes, five surfels beside each
+// other and four such groups together, four written positions of each surfel in flight. Longer ones by the whole wavefront, 64
+// positions tested and their records requested while the last ones are added from LDS, a component per lane. (With five surfels a
+// wavefront, and 11 positions of every span a step, nearly all of the launch was a row of trips to memory, and as many steps as the
+// largest surfel asked for; each component was stored on its own.) 150k surfels 1001x667 24 -> 16.7 us, 300k 1000x700 44 -> 32,
+// 30k 1000x1000 12.3 -> 8.2, 10k 256x256 4.3 -> 4.5.
+constexpr int kFastSumSurfels = 20;
+
 __global__ void __launch_bounds__(256) fast_slot_sum_kernel(int P, int gx, int gy,
     const SlotSource slots, const int32_t* __restrict__ radii, const float2* __restrict__ means2D,
     const float* __restrict__ inverse_m, const float4* __restrict__ normal_opacity,
     const uint32_t* __restrict__ keep_masks, const float* __restrict__ records, FastScatter out) {
-  constexpr int kLanes = kFastRecordSlots / 2, kPerWave = 64 / kLanes;
-  const int lane = threadIdx.x & 63;
-  const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  constexpr int kLanes = kFastRecordSlots / 2, kPerPass = 64 / kLanes, kGroups = 4, kDepth = 4;
+  static_assert(kFastSumSurfels == kPerPass * kGroups);
+  __shared__ float2 s_records[4][kWave * kLanes];
+  __shared__ int s_positions[4][kWave];
+  __shared__ float2 s_sums[4][kFastSumSurfels * kLanes];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane / kLanes, k = lane - sub * kLanes;
-  const int i = wave * kPerWave + sub;
-  const bool active = sub < kPerWave && i < P;
-  const int radius = active ? radii[i] : 0;
-  int count = 0, h = 1, x0 = 0, y0 = 0;
-  float IM[9], opacity = 1.0f;
-#pragma unroll
-  for (int q = 0; q < 9; ++q) IM[q] = 0.0f;
-  const float2* src = (const float2*) records;
-  uint32_t mask = 0u;
-  bool masked = false;  // this surfel's verdicts come from its mask
+  const int i0 = ((int) blockIdx.x * 4 + wave) * kFastSumSurfels, i = i0 + lane;
+  const float2* const src = (const float2*) records;
+  // lanes 0 to 19: a surfel's span and what was written of it
+  int count = 0, h = 1, x0 = 0, y0 = 0, first = 0;
+  uint32_t bits = 0u;
+  const int radius = lane < kFastSumSurfels && i < P ? radii[i] : 0;
   if (radius > 0) {
-    const float2 c   = means2D[i];
+    const float2 c = means2D[i];
+    if (keep_masks) bits = keep_masks[i];
+    first = (int) slot_first(slots, i);  // the number of instances is below 2^31
     const TileRect r = tile_rect(c.x, c.y, radius, gx, gy);
     h = max(r.y1 - r.y0, 1), count = max(r.x1 - r.x0, 0) * max(r.y1 - r.y0, 0), x0 = r.x0, y0 = r.y0;
-    masked = keep_masks != nullptr && count <= 32;
-    if (masked) mask = keep_masks[i];
-    src += (size_t) slot_first(slots, i) * kLanes + k;
   }
-  const bool tested     = radius > 0 && !masked;
-  const bool any_tested = wave_ballot(tested) != 0ull;  // wave-uniform
-  if (tested) {
+  auto corner_test = [&](int id) {
+    float IM[9];
 #pragma unroll
-    for (int q = 0; q < 9; ++q) IM[q] = inverse_m[9 * (size_t) i + q];
-    opacity = normal_opacity[i].w;
+    for (int q = 0; q < 9; ++q) IM[q] = inverse_m[9 * (size_t) id + q];
+    return CornerTest(IM, normal_opacity[id].w);
+  };
+  const bool large = count > 32;
+  if (large) bits = 0u;
+  else if (keep_masks) bits &= count == 32 ? 0xffffffffu : (1u << count) - 1u;
+  else if (count > 0) {
+    const CornerTest ct = corner_test(i);
+    for (int p = 0; p < count; ++p) {
+      const int x = p / h;
+      if (ct.tile(x0 + x, y0 + (p - x * h))) bits |= 1u << p;
+    }
   }
-  CornerTest ct;
-  if (any_tested) ct = CornerTest(IM, opacity);
-  float2 acc = make_float2(0.0f, 0.0f);
-  // the wavefront's surfels step together (the ballot needs every lane): as many steps as its largest rectangle asks
-  int steps = (count + kLanes - 1) / kLanes;
+  {
+    uint32_t left[kGroups];
+    int at[kGroups];
+    float2 acc[kGroups];
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) steps = max(steps, __shfl_xor(steps, d, kWave));
-  for (int st = 0; st < steps; ++st) {
-    const int base = st * kLanes, p = base + k, x = p / h, y = p - x * h;  // x-major over the rectangle
-    bool on = masked && p < count && ((mask >> (p & 31)) & 1u) != 0u;
-    if (any_tested) on = on || (tested && p < count && ct.tile(x0 + x, y0 + y));
-    const unsigned bits = (unsigned) (wave_ballot(on) >> (sub * kLanes)) & ((1u << kLanes) - 1u);
+    for (int q = 0; q < kGroups; ++q) {
+      const int holds = min(q * kPerPass + sub, kFastSumSurfels - 1);
+      left[q] = (uint32_t) __shfl((int) bits, holds, kWave), at[q] = __shfl(first, holds, kWave);
+      if (sub >= kPerPass) left[q] = 0u;
+      acc[q] = make_float2(0.0f, 0.0f);
+    }
+    while (wave_ballot((left[0] | left[1] | left[2] | left[3]) != 0u) != 0ull) {
+      float2 v[kGroups][kDepth];
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q)
+#pragma unroll
+        for (int j = 0; j < kDepth; ++j) {
+          v[q][j] = make_float2(0.0f, 0.0f);
+          if (left[q]) v[q][j] = src[(size_t) (at[q] + __builtin_ctz(left[q])) * kLanes + k];
+          left[q] &= left[q] - 1u;
+        }
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q)
+#pragma unroll
+        for (int j = 0; j < kDepth; ++j) acc[q].x += v[q][j].x, acc[q].y += v[q][j].y;
+    }
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+      const int holds = q * kPerPass + sub;
+      if (sub < kPerPass) s_sums[wave][holds * kLanes + k] = acc[q];
+    }
+  }
+  wave_lds_sync();
+  for (unsigned long long todo = wave_ballot(large); todo != 0ull; todo &= todo - 1ull) {
+    const int holds = (int) __builtin_ctzll(todo), id = i0 + holds;
+    const int s_first = __builtin_amdgcn_readlane(first, holds), s_count = __builtin_amdgcn_readlane(count, holds);
+    const int s_h = __builtin_amdgcn_readlane(h, holds), s_x0 = __builtin_amdgcn_readlane(x0, holds), s_y0 = __builtin_amdgcn_readlane(y0, holds);
+    const CornerTest ct = corner_test(id);
     float2 v[kLanes];
+    auto fetch = [&](int base) {  // how many of the 64 positions from `base` on were written
+      const int p = base + lane, x = p / s_h;
+      const bool on = p < s_count && ct.tile(s_x0 + x, s_y0 + (p - x * s_h));
+      const unsigned long long who = wave_ballot(on);
+      const int n = (int) __popcll(who);
+      wave_lds_sync();
+      if (on) s_positions[wave][__builtin_amdgcn_mbcnt_hi((unsigned) (who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned) who, 0))] = p;
+      wave_lds_sync();
 #pragma unroll
-    for (int j = 0; j < kLanes; ++j)
-      v[j] = ((bits >> j) & 1u) ? src[(size_t) (base + j) * kLanes] : make_float2(0.0f, 0.0f);
+      for (int j = 0; j < kLanes; ++j) {
+        const int t = j * kWave + lane, r = t / kLanes;
+        v[j] = make_float2(0.0f, 0.0f);
+        if (r < n) v[j] = src[(size_t) (s_first + s_positions[wave][r]) * kLanes + (t - r * kLanes)];
+      }
+      return n;
+    };
+    float acc = 0.0f;
+    int n = fetch(0);
+    for (int base = 0; base < s_count; base += kWave) {
+      wave_lds_sync();
 #pragma unroll
-    for (int j = 0; j < kLanes; ++j) acc.x += v[j].x, acc.y += v[j].y;
+      for (int j = 0; j < kLanes; ++j) s_records[wave][j * kWave + lane] = v[j];
+      wave_lds_sync();
+      const int here = n;
+      if (base + kWave < s_count) n = fetch(base + kWave);
+      if (lane < kFastRecordSlots) {
+        const float* f = (const float*) s_records[wave] + lane;
+#pragma unroll 4
+        for (int r = 0; r < here; ++r) acc += f[r * kFastRecordSlots];
+      }
+    }
+    if (lane < kFastRecordSlots) ((float*) s_sums[wave])[holds * kFastRecordSlots + lane] = acc;
   }
-  if (!active) return;
-  out(i, 2 * k, acc.x);
-  out(i, 2 * k + 1, acc.y);
+  wave_lds_sync();
+  out.rows<kFastSumSurfels, kFastRecordSlots>((const float*) s_sums[wave], i0, min(kFastSumSurfels, P - i0));
 }
 
 // Bound by vector issue and, like every launch here, by its longest tile; four blocks per compute unit. 150k surfels 1001x667:
@@ -953,9 +1024,7 @@ __global__ void __launch_bounds__(64) fast_bucket_backward_kernel(int W, int H, 
 void launch_fast_slot_sum(int P, int gx, int gy, const SlotSource& slots, const int32_t* radii,
                           const float* means2D, const float* inverse_m, const float* normal_opacity,
                           const uint32_t* keep_masks, const SlotWorkspace& ws, FastScatter out, hipStream_t s) {
-  constexpr int kPerWave = 64 / (kFastRecordSlots / 2);
-  const int64_t waves = div_up(P, kPerWave);
-  hipLaunchKernelGGL(fast_slot_sum_kernel, dim3((unsigned) div_up(waves * 64, 256)), dim3(256), 0, s, P, gx, gy,
+  hipLaunchKernelGGL(fast_slot_sum_kernel, dim3((unsigned) div_up(P, 4 * kFastSumSurfels)), dim3(256), 0, s, P, gx, gy,
                      slots, radii, (const float2*) means2D, inverse_m, (const float4*) normal_opacity,
                      keep_masks, ws.records, out);
 }
