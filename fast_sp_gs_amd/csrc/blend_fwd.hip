@@ -17,7 +17,7 @@
 // 10k 256x256: 28, 19, 18. With flow the second transforms are loaded when a batch is staged (requested ahead they hold nine
 // registers) and the quotient takes a reciprocal instead of two divisions: 300k 164 -> 142 us, 2000 surfels with deviations of
 // 128 pixels 592 -> 501. Batches of 64 / 128 / 192 surfels (a list's length varies less over a long batch), 2x4: 113 / 97 /
-// 94 us at 300k, 346 / 297 / 282 at 3M.
+// 94 us at 300k, 346 / 297 / 282 at 3M. An entry is intersected beside the blend of the one before (walk_block_list_ahead).
 #include "block_lists.hpp"
 #include "view_maps.hpp"
 
@@ -124,28 +124,44 @@ blend_forward_kernel(
     if ((int) threadIdx.x < kFwdBatch && nxt < n_todo)
       next = gather_splat(point_list[r0 + nxt], means2D, colors, normal_opacity, trans_mat, records);
 
-    // One list entry per block of the wavefront. The intersection runs without early exits and yields one predicate; the
-    // blend is one divergent region.
+    // One list entry per block of the wavefront. The intersection runs without early exits and yields one predicate; what the
+    // pixel's sums take of the entry is one divergent region.
     unsigned char* const lists = &s_list[Shape::kPerWave * wave * kFwdBatch];
     unsigned masks[kFwdBatch / kWave];
 #pragma unroll
     for (int c = 0; c < kFwdBatch / kWave; ++c) masks[c] = s_mask[c * kWave + lane];
     const int steps = build_block_lists<kFwdLanes, kFwdBatch>(lists, masks, wave, live_lanes);
-    auto blend_entry = [&](const SplatHot& hot, int j, int) {
+    struct Eval {
+      float alpha, depth, sx, sy;
+      unsigned long long pass;
+    };
+    auto eval_entry = [&](const SplatHot& hot) {
+      Hit h;
+      Eval e;
+      intersect_flat(hot, pxf, pyf, near_n, h, &e.pass);
+      e.alpha = h.alpha, e.depth = h.depth, e.sx = h.sx, e.sy = h.sy;
+      return e;
+    };
+    auto cold_of = [&](int j) {  // used only if a pixel blends the surfel, but then without waiting
+      const SplatCold cold = s_splat[j].cold;
+      __builtin_amdgcn_sched_barrier(0);
+      return cold;
+    };
+    auto blend_entry = [&](const Eval& e, const SplatCold& cold, int j, int) {
 #pragma clang fp contract(off)  // several copies of this body exist (alternating registers): they must round alike
-        const SplatCold cold = s_splat[j].cold;  // used only if a pixel blends the surfel, but then without waiting
-        __builtin_amdgcn_sched_barrier(0);
-        Hit h;
-        unsigned long long pass;
-        intersect_flat(hot, pxf, pyf, near_n, h, &pass);
-        pass &= live_lanes;
-        if (pass == 0ull) return;
-        const float test_T = T * (1.0f - h.alpha);
+        const unsigned long long pass = e.pass & live_lanes;
+        const float test_T = T * (1.0f - e.alpha);
         const unsigned long long sat = pass & wave_ballot(test_T < 0.0001f);
         live_lanes &= ~sat;
         const unsigned long long blends = pass & ~sat;
+        const float w = e.alpha * T;
+        // by all lanes, beside the next entry's intersection; where a lane does not blend, nothing of it is kept (the asm keeps it here)
+        float m  = fmaf(-far_near, __builtin_amdgcn_rcpf(e.depth), far_scale);
+        float mm = m * m;
+        float spread = fmaf(-2.0f * m, M1, fmaf(mm, 1.0f - T, M2));
+        if (kAux) asm volatile("" : "+v"(m), "+v"(mm), "+v"(spread));
+        if (blends == 0ull) return;
         const bool blend = __builtin_amdgcn_inverse_ballot_w64(blends);
-        const float w      = h.alpha * T;
         if (kAccum == 2) {
           const int n = (int) __popcll(blends >> (lane & -kFwdLanes) & ((1ull << kFwdLanes) - 1ull));
           const float sum = block_sum_to_last<kFwdLanes>(blend ? w : 0.0f);
@@ -155,21 +171,18 @@ blend_forward_kernel(
           if (kHits) my_hit[j * 32] = 1;
           const int contributor = b * kFwdBatch + j + 1;
           if (kAux) {
-            const float A  = 1.0f - T;
-            const float m  = fmaf(-far_near, __builtin_amdgcn_rcpf(h.depth), far_scale);
-            const float mm = m * m;
-            dist = fmaf(fmaf(-2.0f * m, M1, fmaf(mm, A, M2)), w, dist);
-            D    = fmaf(h.depth, w, D);
+            dist = fmaf(spread, w, dist);
+            D    = fmaf(e.depth, w, D);
             M1   = fmaf(m, w, M1);
             M2   = fmaf(mm, w, M2);
-            if (T > 0.5f) median = h.depth, median_c = contributor;
+            if (T > 0.5f) median = e.depth, median_c = contributor;
             N0 = fmaf(cold.nx, w, N0), N1 = fmaf(cold.ny, w, N1), N2 = fmaf(cold.nz, w, N2);
             if (kAccum != 0) argmax_run_step(argmax, w, cold.id, accum_max_count);
             if (kFlow) {
               const float* Q = &s_t2[j * 9];
-              const float u2 = fmaf(Q[0], h.sx, fmaf(Q[1], h.sy, Q[2]));
-              const float v2 = fmaf(Q[3], h.sx, fmaf(Q[4], h.sy, Q[5]));
-              float w2       = fmaf(Q[6], h.sx, fmaf(Q[7], h.sy, Q[8]));
+              const float u2 = fmaf(Q[0], e.sx, fmaf(Q[1], e.sy, Q[2]));
+              const float v2 = fmaf(Q[3], e.sx, fmaf(Q[4], e.sy, Q[5]));
+              float w2       = fmaf(Q[6], e.sx, fmaf(Q[7], e.sy, Q[8]));
               w2             = fabsf(w2) < 1e-5f ? 1e-5f : w2;
               const float rw = newton_rcp(w2);
               f0 = fmaf(fmaf(-pxf, w2, u2) * rw, w, f0);  // u2 / w2 - x: one rounding in the difference
@@ -182,8 +195,9 @@ blend_forward_kernel(
           last = contributor;
         }
       };
-    walk_block_list(lists + lane / kFwdLanes * kFwdBatch, steps, [&](int j) { return s_splat[j].hot; }, blend_entry,
-                    [&]() { return live_lanes != 0ull; });
+    walk_block_list_ahead(lists + lane / kFwdLanes * kFwdBatch, steps, [&](int j) { return s_splat[j].hot; }, cold_of, eval_entry,
+                          blend_entry,
+                          [&]() { return live_lanes != 0ull; });
   }
 
   if (kAccum != 0) argmax_run_flush(argmax, accum_max_count);

@@ -219,6 +219,55 @@ __device__ __forceinline__ void walk_block_list(const unsigned char* __restrict_
   }
 }
 
+// The same, one step further ahead: `eval(record, j)` forms of an entry what does not depend on the pixel's state, while `work` still
+// deals with the entry before it; `late(j)` requests the rest of what `work` reads. Two chains of dependent instructions then
+// stand beside each other. Surfel forward, us: 300k 800x800 99.5 -> 95.5, 3M 1352x1014 307 -> 302, 400k 3840x2160 850 -> 832; the 3D
+// Gaussians' and the fast path's, whose entries have less in front of the blend, took 1 % longer this way. The record's LDS offset
+// kept for both requests instead of formed twice: 96.9, 307, 843.
+template <typename Load, typename Late, typename Eval, typename Work, typename More>
+__device__ __forceinline__ void walk_block_list_ahead(const unsigned char* __restrict__ list, int steps, Load load, Late late,
+                                                      Eval eval, Work work, More more) {
+  if (steps == 0) return;
+  const unsigned* four = (const unsigned*) list;
+  unsigned now = four[0];
+  auto rec = load((int) (now & 255u));
+  auto a   = eval(rec), b = a;
+  rec      = load((int) (now >> 8 & 255u));
+  for (int i = 0;; i += 4) {
+    const unsigned next = four[(i >> 2) + 1];
+    const int j0 = (int) (now & 255u), j1 = (int) (now >> 8 & 255u), j2 = (int) (now >> 16 & 255u), j3 = (int) (now >> 24);
+    {
+      const auto l = late(j0);
+      b   = eval(rec);
+      rec = load(j2);
+      work(a, l, j0, i);
+      if (i + 1 >= steps || !more()) return;
+    }
+    {
+      const auto l = late(j1);
+      a   = eval(rec);
+      rec = load(j3);
+      work(b, l, j1, i + 1);
+      if (i + 2 >= steps || !more()) return;
+    }
+    {
+      const auto l = late(j2);
+      b   = eval(rec);
+      rec = load((int) (next & 255u));
+      work(a, l, j2, i + 2);
+      if (i + 3 >= steps || !more()) return;
+    }
+    {
+      const auto l = late(j3);
+      a   = eval(rec);
+      rec = load((int) (next >> 8 & 255u));
+      work(b, l, j3, i + 3);
+      if (i + 4 >= steps || !more()) return;
+    }
+    now = next;
+  }
+}
+
 // ---- which blocks blended an entry ---------------------------------------------------------------------------------------
 // A forward kernel (2x4 blocks) can note, per staged entry, the blocks with a pixel that blended it, a byte per block; the
 // backward then walks exactly these instead of bounding every footprint again. Block b's byte is b ^ 3: the product below
