@@ -675,10 +675,12 @@ __global__ void __launch_bounds__(256) adam_masked_multi_kernel(AdamTable t, int
     if (row >= N) row = N - 1;  // only past the last element of the tensor, which e + k < total excludes
   }
   if (!(on[0] | on[1] | on[2] | on[3])) return;
+  // gradients and moments pass the memory-side cache by, the parameters stay in it for the next pass: the dynamic iteration of 200k
+  // points 645 -> 638 us
   float g[4], mm[4], vv[4], pp[4];
-  *(float4*) g  = *(const float4*) (grad + e);
-  *(float4*) mm = *(const float4*) (m + e);
-  *(float4*) vv = *(const float4*) (v + e);
+  *(ShPiece*) g  = __builtin_nontemporal_load((const ShPiece*) (grad + e));
+  *(ShPiece*) mm = __builtin_nontemporal_load((const ShPiece*) (m + e));
+  *(ShPiece*) vv = __builtin_nontemporal_load((const ShPiece*) (v + e));
   *(float4*) pp = *(const float4*) (param + e);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -688,8 +690,8 @@ __global__ void __launch_bounds__(256) adam_masked_multi_kernel(AdamTable t, int
     mm[k] = on[k] ? m1 : mm[k], vv[k] = on[k] ? v1 : vv[k], pp[k] = on[k] ? p1 : pp[k];
   }
   *(float4*) (param + e) = *(float4*) pp;  // elements of masked rows are written back as they were
-  *(float4*) (m + e)     = *(float4*) mm;
-  *(float4*) (v + e)     = *(float4*) vv;
+  __builtin_nontemporal_store(*(ShPiece*) mm, (ShPiece*) (m + e));
+  __builtin_nontemporal_store(*(ShPiece*) vv, (ShPiece*) (v + e));
 }
 
 }  // namespace

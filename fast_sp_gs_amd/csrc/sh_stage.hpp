@@ -87,6 +87,11 @@ __device__ __forceinline__ void unstage_sh_grads(const float* __restrict__ s_row
 // 72 MB of its 150): 127 us through stage_sh_rows (4-byte loads behind a block barrier), 64 us this way.
 // In LDS a row has an odd stride, so lanes that read their own rows hit different banks: rows of odd length lie as they
 // do in memory (a piece is one 16-byte LDS write), rows of even length get one float more.
+// The rows are most of what a pass moves, and each is read once and written once in it: they pass the 256 MB memory-side cache by
+// (non-temporal stores, and loads with kStream), which then holds the records, the lists and the model's other tensors from kernel to
+// kernel. Preprocess forward and backward, us: 3M 1352x1014 238 + 369 -> 216 + 330; 1M 1352x900 96 + 131 -> 85 + 119; 300k 800x800
+// 34 + 51 -> 34 + 45. The SH operators' backward reads the coefficients that their forward has read: there the loads are ordinary
+// ones, 1M rows of coefficients 53 + 82 -> 33 + 76 us (with kStream 36 + 77).
 using ShPiece = float __attribute__((ext_vector_type(4)));
 
 template <int kFloats>
@@ -103,6 +108,7 @@ struct ShWaveRows {
 
   // `flags` has bit r set for the rows that are needed (all of them existing rows); a piece of other rows re-reads the
   // first needed row's instead of branching. flags must not be 0.
+  template <bool kStream = false>
   __device__ __forceinline__ void fetch(unsigned long long flags, int wave_base, int P, const float* __restrict__ src) {
     const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
     const int first  = (__builtin_ctzll(flags) * kFloats) >> 2;
@@ -112,7 +118,8 @@ struct ShWaveRows {
       const int e = k * 64 + lane;
       const int r0 = (4 * e) / kFloats, r1 = (4 * e + 3) / kFloats;
       const bool on = e < whole && (((flags >> (r0 & 63)) | (flags >> (r1 & 63))) & 1ull);
-      v[k] = ((const ShPiece*) row)[on ? e : first];
+      const ShPiece* q = (const ShPiece*) row + (on ? e : first);
+      v[k] = kStream ? __builtin_nontemporal_load(q) : *q;
     }
     if (kFloats % 4 != 0) {  // up to three floats behind the last piece of the last wavefront
       tail = 0.0f;
@@ -148,11 +155,11 @@ struct ShWaveRows {
     for (int k = 0; k < kVecs; ++k) {
       const int e = k * 64 + lane;
       if (kFloats % 2 == 1) {
-        if (e < whole) ((ShPiece*) row)[e] = *(const ShPiece*) (s_wave_rows + 4 * e);
+        if (e < whole) __builtin_nontemporal_store(*(const ShPiece*) (s_wave_rows + 4 * e), (ShPiece*) row + e);
       } else if (e < whole) {
         const int r = (4 * e) / kFloats;
         const float* s = s_wave_rows + r * kStride + (4 * e - r * kFloats);
-        ((float4*) row)[e] = make_float4(s[0], s[1], s[2], s[3]);
+        __builtin_nontemporal_store(ShPiece{s[0], s[1], s[2], s[3]}, (ShPiece*) row + e);
       }
     }
     if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = s_wave_rows[4 * whole + lane];
@@ -163,7 +170,7 @@ struct ShWaveRows {
     float* row = dst + (size_t) wave_base * kFloats;
 #pragma unroll
     for (int k = 0; k < kVecs; ++k)
-      if (k * 64 + lane < whole) ((float4*) row)[k * 64 + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (k * 64 + lane < whole) __builtin_nontemporal_store(ShPiece{0.0f, 0.0f, 0.0f, 0.0f}, (ShPiece*) row + k * 64 + lane);
     if (kFloats % 4 != 0 && lane < (all & 3)) row[4 * whole + lane] = 0.0f;
   }
 };
