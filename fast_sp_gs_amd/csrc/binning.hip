@@ -474,11 +474,7 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
   const int lane = __lane_id(), wave = threadIdx.x / kWave;
   unsigned long long carry = 0;
   const int first = sums ? blockIdx.x * 4096 : 0, last = sums ? min(T, first + 4096) : T;
-  if (exceeds && *exceeds) {
-    for (int t = first + (int) threadIdx.x; t < last; t += blockDim.x) ranges[2 * (size_t) t] = 0, ranges[2 * (size_t) t + 1] = 0;
-    if (threadIdx.x == 0 && last == T) large_count[0] = 0, large_count[1] = 0;
-    return;
-  }
+  const bool room = !exceeds || *exceeds == 0;  // on its way while the counts are
   if (first > 0) {
     unsigned long long before = 0;
     for (int b = threadIdx.x; b < first / kPrefixTiles; b += blockDim.x) before += sums[b];
@@ -508,7 +504,7 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
     unsigned long long run = carry + base + inc - sum;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (t0 + k < T) ranges[2 * (size_t) (t0 + k)] = run, ranges[2 * (size_t) (t0 + k) + 1] = ends ? run + c[k] : run;
+      if (t0 + k < T) ranges[2 * (size_t) (t0 + k)] = room ? run : 0, ranges[2 * (size_t) (t0 + k) + 1] = !room ? 0 : ends ? run + c[k] : run;
       run += c[k];
     }
     carry += total;
@@ -1260,7 +1256,7 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
   int* header = (int*) bins;
-  if (publish.capacity > 0) publish.exceeds = (int*) ((char*) bins + kBinsExceeds);
+  if (publish.capacity > 0 && publish.capacity < INT64_MAX) publish.exceeds = (int*) ((char*) bins + kBinsExceeds);
   const BinsLayout bl = bins_layout(P, T);
   if (bl.blocks > 0) {
     uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);

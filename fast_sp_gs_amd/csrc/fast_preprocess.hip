@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     bool maybe = valid && !(culling && culling[i]);
     maybe = maybe && !((Tw2v[8] * p[0] + Tw2v[9] * p[1] + Tw2v[10] * p[2] + Tw2v[11]) <= 0.2f);
     wanted = __ballot(maybe);
-    if (wanted) sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
     if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   }
   do {
@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
       return;
     }
     ShWaveRows<kWave ? kRow : 48> sh_regs;
-    sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
     sh_regs.to_lds(s_wave_rows, wave_base, P);
     wave_lds_sync();
     if (!vis) {

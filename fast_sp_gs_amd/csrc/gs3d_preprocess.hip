@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   float dc[3] = {0, 0, 0};
   if (kWave) {  // the fetch of the rows is in flight during the geometry
     wanted = __ballot(valid && !(culling && culling[i]));
-    if (wanted) sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
     if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   }
   do {
@@ -424,7 +424,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
     const unsigned long long wanted = __ballot(vis);
     if (wanted) {
       ShWaveRows<kWave ? kRow : 48> sh_regs;
-      sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+      sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
       sh_regs.to_lds(s_wave_rows, wave_base, P);
     }
     wave_lds_sync();

@@ -131,7 +131,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     bool maybe = valid && !(culling && culling[i]);
     maybe = maybe && !((s_Tw2v[8] * p[0] + s_Tw2v[9] * p[1] + s_Tw2v[10] * p[2] + s_Tw2v[11]) <= 0.2f);
     wanted = __ballot(maybe);
-    if (wanted) sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
     if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   }
   do {
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   const unsigned long long wanted = kWave ? __ballot(vis) : 0ull;
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   float up[kRecords ? kGradFloats : 1];
-  if (kWave && wanted) sh_regs.template fetch<true>(wanted, wave_base, P, kSplit ? sh_rest : shs);
+  if (kWave && wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
   // what the geometry reads of the surfel
   float M[9], p[3] = {0, 0, 0}, col[3] = {0, 0, 0};
   float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);

@@ -88,16 +88,21 @@ __device__ __forceinline__ void unstage_sh_grads(const float* __restrict__ s_row
 // In LDS a row has an odd stride, so lanes that read their own rows hit different banks: rows of odd length lie as they
 // do in memory (a piece is one 16-byte LDS write), rows of even length get one float more.
 // The rows are most of what a pass moves, and each is read once and written once in it: they pass the 256 MB memory-side cache by
-// (non-temporal stores, and loads with kStream), which then holds the records, the lists and the model's other tensors from kernel to
+// (non-temporal stores, and loads where the rows are 48 MB or more), which then holds the records, the lists and the model's other tensors from kernel to
 // kernel. Preprocess forward and backward, us: 3M 1352x1014 238 + 369 -> 216 + 330; 1M 1352x900 96 + 131 -> 85 + 119; 300k 800x800
 // 34 + 51 -> 34 + 45. The SH operators' backward reads the coefficients that their forward has read: there the loads are ordinary
-// ones, 1M rows of coefficients 53 + 82 -> 33 + 76 us (with kStream 36 + 77).
+// ones, 1M rows of coefficients 53 + 82 -> 33 + 76 us (with streaming loads
+// 36 + 77). Smaller tables stay in the cache from pass to pass: view of 98k surfels 170x120, preprocess 14 us and 16 with streaming
+// loads; 200k 22.3 and 23.5; 300k (58 MB) 36.4 and 35.2; 400k 58 and 52.
 using ShPiece = float __attribute__((ext_vector_type(4)));
+
+constexpr size_t kStreamBytes = 48u << 20;
 
 template <int kFloats>
 struct ShWaveRows {
   static_assert(kFloats % 2 == 1 || kFloats % 4 == 0, "a piece lies in one row or rows are stored without a gap");
   static constexpr int kStride = kFloats | 1;
+  static __device__ __forceinline__ bool large(int P) { return (size_t) P * kFloats * 4 >= kStreamBytes; }
   static constexpr int kPieces = 16 * kFloats;          // of 64 rows
   static constexpr int kVecs   = (kPieces + 63) / 64;   // of a lane
   ShPiece v[kVecs];
@@ -108,18 +113,24 @@ struct ShWaveRows {
 
   // `flags` has bit r set for the rows that are needed (all of them existing rows); a piece of other rows re-reads the
   // first needed row's instead of branching. flags must not be 0.
-  template <bool kStream = false>
-  __device__ __forceinline__ void fetch(unsigned long long flags, int wave_base, int P, const float* __restrict__ src) {
+  // stream (uniform): the pieces pass the memory-side cache by.
+  __device__ __forceinline__ void fetch(unsigned long long flags, int wave_base, int P, const float* __restrict__ src,
+                                        bool stream = false) {
     const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
     const int first  = (__builtin_ctzll(flags) * kFloats) >> 2;
     const float* row = src + (size_t) wave_base * kFloats;
-#pragma unroll
-    for (int k = 0; k < kVecs; ++k) {
+    auto piece = [&](int k) {
       const int e = k * 64 + lane;
       const int r0 = (4 * e) / kFloats, r1 = (4 * e + 3) / kFloats;
       const bool on = e < whole && (((flags >> (r0 & 63)) | (flags >> (r1 & 63))) & 1ull);
-      const ShPiece* q = (const ShPiece*) row + (on ? e : first);
-      v[k] = kStream ? __builtin_nontemporal_load(q) : *q;
+      return (const ShPiece*) row + (on ? e : first);
+    };
+    if (stream) {
+#pragma unroll
+      for (int k = 0; k < kVecs; ++k) v[k] = __builtin_nontemporal_load(piece(k));
+    } else {
+#pragma unroll
+      for (int k = 0; k < kVecs; ++k) v[k] = *piece(k);
     }
     if (kFloats % 4 != 0) {  // up to three floats behind the last piece of the last wavefront
       tail = 0.0f;
