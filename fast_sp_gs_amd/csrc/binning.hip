@@ -775,9 +775,9 @@ __device__ __forceinline__ void merge_sort_lds(uint64_t* e, int n) {
 constexpr int kSortBuckets = kSmallSegment / 2;  // their counters fill the LDS that the network's empty slots take
 constexpr int kBucketLimit = 32;                 // entries of one bucket that are put in order by counting
 
-// Exclusive prefix over the counters of a 256-lane block, in place, and the largest one: a lane owns kOwn neighbouring words of
+// Exclusive prefix over the counters of a block of kWaves wavefronts, in place, and the largest one: a lane owns kOwn neighbouring words of
 // kHalves counters (32 or 16 bits). s_wave: two words a wavefront. Two barriers; one more before the counters are read.
-template <int kOwn, int kHalves>
+template <int kOwn, int kHalves, int kWaves = 4>
 __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned* s_wave) {
   constexpr unsigned kMask = kHalves == 2 ? 0xffffu : ~0u;
   const int wave = threadIdx.x >> 6;
@@ -795,7 +795,7 @@ __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned*
   unsigned at = inc - sum;
   most = 0;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < kWaves; ++w) {
     if (w < wave) at += s_wave[2 * w];
     most = max(most, s_wave[2 * w + 1]);
   }
@@ -999,12 +999,127 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) t
   else sort(std::integral_constant<int, 8>());
 }
 
-// A few blocks walk the queue of long segments: up to kLargeSegment entries in LDS, beyond that the same network on the
-// global array (slow, but such a segment means tens of thousands of surfels over one 16x16 tile).
+// The first cut of bucket_sort for the n <= 1024 * kPer entries of a long segment, by a 1024-lane block. False, with nothing written,
+// when a bucket holds more than 4 * kBucketLimit entries (16 times in longer segments, whose network works in global memory).
+constexpr int kLargeBuckets = 4096;
+
+template <int kPer>
+__device__ __forceinline__ bool bucket_sort_large(int tile, int64_t start, int n, const uint64_t* __restrict__ entries, uint64_t* s_e,
+                                                  unsigned* s_count, unsigned* s_wave, int32_t* __restrict__ point_list,
+                                                  int64_t* __restrict__ keys_out) {
+  constexpr int kThreads = 1024, kWaves = kThreads / kWave, kOwn = kLargeBuckets / kThreads;
+  const int wave = threadIdx.x >> 6;
+  uint64_t key[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) key[q] = entries[start + min((int) threadIdx.x + kThreads * q, n - 1)];
+  unsigned lo = ~0u, hi = 0u;
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) s_count[kOwn * threadIdx.x + c] = 0u;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) lo = min(lo, (unsigned) (key[q] >> 32)), hi = max(hi, (unsigned) (key[q] >> 32));
+  lo = wave_max_to_last(~lo), hi = wave_max_to_last(hi);
+  if ((threadIdx.x & 63) == 63) s_wave[2 * wave] = lo, s_wave[2 * wave + 1] = hi;
+  __syncthreads();
+  lo = s_wave[0], hi = s_wave[1];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) lo = max(lo, s_wave[2 * w]), hi = max(hi, s_wave[2 * w + 1]);
+  lo = ~lo;
+  if (lo == hi) return false;  // one depth: every entry would wait for the one counter
+  const float scale = (float) kLargeBuckets * __builtin_amdgcn_rcpf((float) (hi - lo) + 1.0f);
+  auto bucket = [&](uint64_t k) { return min((int) ((float) ((unsigned) (k >> 32) - lo) * scale), kLargeBuckets - 1); };
+  unsigned rank[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + kThreads * q < n) rank[q] = atomicAdd(&s_count[bucket(key[q])], 1u);
+  __syncthreads();
+  if (prefix_counters<kOwn, 1, kWaves>(s_count, s_wave) > 4u * kBucketLimit) return false;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if ((int) threadIdx.x + kThreads * q < n) s_e[s_count[bucket(key[q])] + rank[q]] = key[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int p = threadIdx.x + kThreads * q;
+    if (p < n) {
+      const uint64_t e = s_e[p];
+      const int b = bucket(e), first = (int) s_count[b], end = b + 1 < kLargeBuckets ? (int) s_count[b + 1] : n;
+      int to = first;
+      for (int i = first; i < end; ++i) to += s_e[i] < e;
+      point_list[start + to] = (int32_t) (uint32_t) e;
+      if (keys_out) keys_out[start + to] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
+    }
+  }
+  return true;
+}
+
+// A segment that does not fit the LDS, the same way, as many buckets at a time as hold at most kLargeSegment entries: the segment is read
+// once to count and once for every such group.
+__device__ __forceinline__ bool bucket_sort_huge(int tile, int64_t start, int64_t len, const uint64_t* __restrict__ entries, uint64_t* s_e,
+                                                 unsigned* s_count, unsigned* s_wave, int32_t* __restrict__ point_list,
+                                                 int64_t* __restrict__ keys_out) {
+  constexpr int kThreads = 1024, kWaves = kThreads / kWave, kOwn = kLargeBuckets / kThreads;
+  constexpr unsigned kLimit = 16 * kBucketLimit;
+  const int wave = threadIdx.x >> 6, n = (int) len;
+  unsigned lo = 0u, hi = 0u;  // lo: of the complement
+  for (int p = threadIdx.x; p < n; p += kThreads) {
+    const unsigned d = (unsigned) (entries[start + p] >> 32);
+    lo = max(lo, ~d), hi = max(hi, d);
+  }
+#pragma unroll
+  for (int c = 0; c < kOwn; ++c) s_count[kOwn * threadIdx.x + c] = 0u;
+  lo = wave_max_to_last(lo), hi = wave_max_to_last(hi);
+  if ((threadIdx.x & 63) == 63) s_wave[2 * wave] = lo, s_wave[2 * wave + 1] = hi;
+  __syncthreads();
+  lo = s_wave[0], hi = s_wave[1];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) lo = max(lo, s_wave[2 * w]), hi = max(hi, s_wave[2 * w + 1]);
+  lo = ~lo;
+  if (lo == hi) return false;
+  const float scale = (float) kLargeBuckets * __builtin_amdgcn_rcpf((float) (hi - lo) + 1.0f);
+  auto bucket = [&](uint64_t k) { return min((int) ((float) ((unsigned) (k >> 32) - lo) * scale), kLargeBuckets - 1); };
+  for (int p = threadIdx.x; p < n; p += kThreads) atomicAdd(&s_count[bucket(entries[start + p])], 1u);
+  __syncthreads();
+  if (prefix_counters<kOwn, 1, kWaves>(s_count, s_wave) > kLimit) return false;
+  // s_count[b]: where bucket b starts; once its group has been placed, where it ends, which is where b + 1 starts
+  for (int b0 = 0, base = 0; b0 < kLargeBuckets;) {
+    int b1 = kLargeBuckets;  // the last bucket whose end is still within the LDS, and one more
+    for (int step = kLargeBuckets, at = b0; step >= 1; step >>= 1) {
+      if (at + step < kLargeBuckets && (int) s_count[at + step] - base <= kLargeSegment) at += step;
+      b1 = at;
+    }
+    if (n - base <= kLargeSegment) b1 = kLargeBuckets;
+    const int end = b1 < kLargeBuckets ? (int) s_count[b1] : n;
+    __syncthreads();
+    for (int p = threadIdx.x; p < n; p += kThreads) {
+      const uint64_t e = entries[start + p];
+      const int b = bucket(e);
+      if (b >= b0 && b < b1) s_e[atomicAdd(&s_count[b], 1u) - base] = e;
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < end - base; p += kThreads) {
+      const uint64_t e = s_e[p];
+      const int b = bucket(e), first = b > 0 ? (int) s_count[b - 1] : 0, last = (int) s_count[b];
+      int to = first;
+      for (int i = first; i < last; ++i) to += s_e[i - base] < e;
+      point_list[start + to] = (int32_t) (uint32_t) e;
+      if (keys_out) keys_out[start + to] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
+    }
+    __syncthreads();
+    b0 = b1, base = end;
+  }
+  return true;
+}
+
+// A few blocks walk the queue of long segments: up to kLargeSegment entries in LDS, by buckets or, where their depths lie too close
+// together, by the sorting network; longer ones by groups of buckets, or by the network on the global array.
+// Against the network, us a launch: 98k surfels 170x120 (lists of 3 to 6 thousand) 52 -> 8, 577k 228x227 108 -> 14, 2M 600x500 96 -> 15;
+// lists above 16 384, 2M 160x110: 1760 (the network) -> 258.
 __global__ void __launch_bounds__(1024) tile_sort_large_kernel(const int64_t* __restrict__ ranges,
     uint64_t* __restrict__ entries, int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out,
     const int* __restrict__ large_count, const int* __restrict__ large_list) {
   __shared__ uint64_t s_e[kLargeSegment];
+  __shared__ unsigned s_count[kLargeBuckets];
+  __shared__ unsigned s_wave[2 * 1024 / kWave];
   const int n_large = *large_count;
   for (int q = blockIdx.x; q < n_large; q += gridDim.x) {
     const int tile = large_list[q];
@@ -1012,6 +1127,13 @@ __global__ void __launch_bounds__(1024) tile_sort_large_kernel(const int64_t* __
     const int64_t len   = ranges[2 * (size_t) tile + 1] - start;
     if (len <= kLargeSegment) {
       const int n = (int) len;
+      __syncthreads();  // the counters and the entries of the segment before have been read
+      bool sorted;
+      if (n <= 4096) sorted = bucket_sort_large<4>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
+      else if (n <= 8192) sorted = bucket_sort_large<8>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
+      else sorted = bucket_sort_large<16>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
+      if (sorted) continue;
+      __syncthreads();
       const int m = padded_length(n);
       for (int k = threadIdx.x; k < m; k += 1024) s_e[k] = k < n ? entries[start + k] : ~0ull;
       __syncthreads();
@@ -1019,6 +1141,8 @@ __global__ void __launch_bounds__(1024) tile_sort_large_kernel(const int64_t* __
       tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
       __syncthreads();
     } else {
+      __syncthreads();
+      if (bucket_sort_huge(tile, start, len, entries, s_e, s_count, s_wave, point_list, keys_out)) continue;
       uint64_t* e = entries + start;
       bitonic_sort<int64_t>(e, len, 1024, [] {
         __threadfence_block();

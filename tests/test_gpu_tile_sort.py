@@ -74,3 +74,25 @@ def test_equal_depths_in_one_of_two_tiles(n, depths, device, oracle_mod):
         assert want[0][0, 1] - want[0][0, 0] == n
         for a, b in zip((ranges, pl, keys), want):
             assert np.array_equal(npy(a), b)
+
+
+@pytest.mark.parametrize('n', [2049, 4095, 4096, 4097, 8192, 8193, 16383, 16384, 16385, 32769, 50_000])
+@pytest.mark.parametrize('depths', ['random', 'equal', 'ties', 'shells', 'outlier', 'signs'])
+def test_long_list_of_one_tile(n, depths, device, oracle_mod):
+    """Lists that the 1024-lane blocks sort: by buckets in LDS, by groups of buckets above 16 384 entries, and by the network where
+    too many entries share a bucket (`equal`, `outlier`, and `shells` at the larger sizes)."""
+    from fast_sp_gs_amd._C import get_C_function
+    print(f'[tile sort] n={n} {depths}', flush=True)
+    g = torch.Generator().manual_seed(n)
+    r = torch.rand(n, generator=g)
+    far = r + 1.0
+    far[n // 2] = 3e38
+    dep = {'random': r * 10.0 + 0.5, 'equal': torch.ones(n), 'ties': (r * n / 4).floor() + 1.0,
+           'shells': torch.randint(1, 3, (n,), generator=g).float() + 1e-3 * r, 'outlier': far,
+           'signs': torch.randn(n, generator=g) * 10.0 ** torch.randint(-30, 30, (n,), generator=g)}[depths].float()
+    m2 = torch.full((n, 2), 8.0)
+    radii, touched = torch.full((n,), 3, dtype=torch.int32), torch.ones(n, dtype=torch.int32)
+    ranges, pl, keys = get_C_function('GS_prepare')(16, 16, m2.to(device), dep.to(device), radii.to(device),
+                                                    touched.to(device), False, return_keys=True)[:3]
+    want_ranges, want_pl, want_keys = oracle_mod.prepare(16, 16, npy(m2), npy(dep), npy(radii), npy(touched), return_keys=True)
+    assert np.array_equal(npy(ranges), want_ranges) and np.array_equal(npy(pl), want_pl) and np.array_equal(npy(keys), want_keys)
