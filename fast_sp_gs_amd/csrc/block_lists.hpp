@@ -188,8 +188,8 @@ __device__ __forceinline__ int build_block_lists(unsigned char* __restrict__ lis
 // Walks the lists of a wavefront: `load(j)` requests the record of entry j, `work(record, j)` evaluates it and `more()`
 // says whether any lane still blends. A wavefront walks alone, so what it would wait for sits on the tile's critical path: the
 // record of the next entry is requested before the present one is evaluated, into alternating registers, and the entry
-// numbers four at a time one step of four ahead. `work` also gets the step's number. (Reads up to four bytes past the list: numbers of another list, or the
-// padding behind the last one; they are loaded but never evaluated.)
+// numbers four at a time one step of four ahead. `work` also gets the step's number. (Reads up to four bytes past the list:
+// numbers of another list, or the padding behind the last one; they are loaded but never evaluated.)
 template <typename Load, typename Work, typename More>
 __device__ __forceinline__ void walk_block_list(const unsigned char* __restrict__ list, int steps, Load load, Work work,
                                                 More more) {
@@ -219,11 +219,12 @@ __device__ __forceinline__ void walk_block_list(const unsigned char* __restrict_
   }
 }
 
-// The same, one step further ahead: `eval(record, j)` forms of an entry what does not depend on the pixel's state, while `work` still
-// deals with the entry before it; `late(j)` requests the rest of what `work` reads. Two chains of dependent instructions then
-// stand beside each other. Surfel forward, us: 300k 800x800 99.5 -> 95.5, 3M 1352x1014 307 -> 302, 400k 3840x2160 850 -> 832; the 3D
-// Gaussians' and the fast path's, whose entries have less in front of the blend, took 1 % longer this way. The record's LDS offset
-// kept for both requests instead of formed twice: 96.9, 307, 843.
+// The same, one step further ahead (past the list as there: loaded, at most intersected, never blended): `eval(record)`
+// forms of an entry what does not depend on the pixel's state, while `work` still deals with the entry before it; `late(j)`
+// requests the rest of what `work` reads. Two chains of dependent instructions then stand beside each other. Surfel
+// forward, us: 300k 800x800 99.5 -> 95.5, 3M 1352x1014 307 -> 302, 400k 3840x2160 850 -> 832; the 3D Gaussians' and the
+// fast path's, whose entries have less in front of the blend, took 1 % longer this way. The record's LDS offset kept for
+// both requests instead of formed twice: 96.9, 307, 843.
 template <typename Load, typename Late, typename Eval, typename Work, typename More>
 __device__ __forceinline__ void walk_block_list_ahead(const unsigned char* __restrict__ list, int steps, Load load, Late late,
                                                       Eval eval, Work work, More more) {
