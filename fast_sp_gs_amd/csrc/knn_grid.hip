@@ -85,6 +85,14 @@ __device__ __forceinline__ float distance2(float qx, float qy, float qz, const f
   return (dx * dx + dy * dy) + dz * dz;
 }
 
+// A control point as the searches take it. One with a NaN is nobody's neighbour: it lies at infinity along every axis, so that
+// its distance is infinite and not a NaN, which the keys would order in front of everything (the conversion makes it 0).
+__device__ __forceinline__ float4 control_point(const float* __restrict__ y, int i) {
+  const float a = y[3 * i], b = y[3 * i + 1], c = y[3 * i + 2];
+  const bool known = a == a && b == b && c == c;
+  return known ? make_float4(a, b, c, 0.0f) : make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
+}
+
 // Upper bound on the K-th smallest of the 64 lanes' non-negative values: the value's upper bits by bisection on lane masks
 // (scalar work), the lower `kDrop` bits rounded up (19: at most 1/16 above the value; 0: the value itself). Infinity when
 // fewer than K lanes hold a finite value.
@@ -283,7 +291,7 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
   __shared__ float s_bound[kWaves];
   __shared__ int s_count[kWaves];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int i = t; i < M; i += kBuildThreads) s_y[i] = make_float4(y[3 * i], y[3 * i + 1], y[3 * i + 2], 0.0f);
+  for (int i = t; i < M; i += kBuildThreads) s_y[i] = control_point(y, i);
   __syncthreads();
   make_planes<kG>(s_y, M, s);
   if (blockIdx.x == 0)
@@ -476,11 +484,7 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
   __shared__ float s_cand_d[kWaves][kWave];
   __shared__ int s_cand_i[kWaves][kWave];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  // one with a NaN, which is nobody's neighbour, lies at infinity: the keys order no NaN
-  for (int i = t; i < M; i += kQueryThreads) {
-    const float a = y[3 * i], b = y[3 * i + 1], c = y[3 * i + 2];
-    s_y[i] = make_float4(a == a && b == b && c == c ? a : __builtin_inff(), b, c, 0.0f);
-  }
+  for (int i = t; i < M; i += kQueryThreads) s_y[i] = control_point(y, i);
   if (t < 8) s_y[M + t] = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
   if (kG > 0)
     for (int e = t; e < 3 * (kG + 1); e += kQueryThreads) (&s_plane[0][0])[e] = planes[e];

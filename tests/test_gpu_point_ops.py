@@ -263,6 +263,34 @@ def test_knn_candidate_lists(N, M, K, kind, device, oracle_mod):
     assert np.array_equal(npy(idx), ri) and np.array_equal(npy(d2), rd)
 
 
+def _all_pairs_knn(pts, ctrl, K, device):
+    """The search over all control points by its own entry point."""
+    from fast_sp_gs_amd import lib as L
+    x, y = pts.to(device), ctrl.to(device)
+    d2 = torch.empty(len(x), K, device=device)
+    idx = torch.empty(len(x), K, device=device, dtype=torch.int64)
+    L.check(L.load().fsgs_knn_topk(len(x), len(y), 3, K, L.ptr(x), L.ptr(y), L.ptr(d2), L.ptr(idx), L.current_stream()), 'knn')
+    return d2, idx
+
+
+# A control point with a NaN in any coordinate is nobody's neighbour, by every search: a wavefront per query, both grids. One
+# such point by itself, too: the keys of several in one cell collide, and the exact search takes over.
+@pytest.mark.parametrize('N,M,K', [(500, 640, 4), (17000, 640, 4), (17000, 2560, 8), (17000, 641, 1)])
+@pytest.mark.parametrize('axes', [(0,), (1,), (2,), (1, 2), (0, 1, 2)])
+@pytest.mark.parametrize('count', [1, 9])
+def test_knn_control_points_with_nan(N, M, K, axes, count, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N + M + count)
+    pts, ctrl = torch.randn(N, 3, generator=g), torch.randn(M, 3, generator=g)
+    gone = torch.randperm(M, generator=g)[:count]
+    for a in axes:
+        ctrl[gone, a] = float('nan')
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert not torch.isin(want_i, gone.to(device)).any() and bool(torch.isfinite(want_d).all())
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+
+
 LBS_CASES = [  # (warp method with a local rotation | None without one, weight method)
     (None, 'weighted_kernel'),   # the reference's default configuration: translations only, kernel weights
     (None, 'dist'), ('LBS', 'dist'), ('LBS_c', 'dist'), ('LBS_c', 'weighted_kernel'), ('LBS', 'kernel'),
