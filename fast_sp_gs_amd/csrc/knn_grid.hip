@@ -138,41 +138,34 @@ __device__ __forceinline__ float from_ordered_bits(uint32_t b) {
   return __uint_as_float((b & 0x80000000u) ? b & 0x7fffffffu : ~b);
 }
 
+constexpr float kRim = 0.5f;  // parts of the sample's extent
+
 template <int kG>
 struct PlaneLds {
   static constexpr int kSamples = 128;
   uint32_t key[3][kSamples];
   float sorted[3][kSamples], along[3][kSamples];
   float plane[3][kG + 1];
-  uint32_t least[kG > 16 ? 3 : 1][8], most[kG > 16 ? 3 : 1][8];  // of all control points, per wavefront
+  float least[kG > 16 ? 3 : 1][8], most[kG > 16 ? 3 : 1][8];  // of the control points near the sample, per wavefront
 };
 
 // The grid planes, from 128 sampled control points per axis (256 cost 6 us more and make the lists no shorter): sorted by
 // counting ranks, inner planes at equal steps of the accumulated square root of the gaps (cells shrink with density, but slower
-// than quantiles would). The outermost planes lie a tenth of the sample's extent beyond it. With many queries (G = 32) they lie beyond all control points, too: a query outside the
-// grid costs as much as 30 inside, and there was one in every wavefront (3M normal queries, 2048 normal control points); two more
-// planes on either side divide that margin, which a sample's gaps know nothing of: its cells would have lists of more than 128.
+// than quantiles would). Coordinates far outside the others are moved in first, for a gap of a thousand times the others' extent
+// would take three quarters of the planes: to half the extent of the sample without its eight outermost on either side, or, where
+// most of it lies in one spot (a flat scene), to the extent without the outermost one. The outermost planes lie a tenth of the
+// sample's extent beyond it. With many queries (G = 32) they lie beyond all control points within half of its extent, too: a
+// query outside the grid costs as much as 30 inside, and there was one in every wavefront (3M normal queries, 2048 normal
+// control points); two more planes on either side divide that margin, which a sample's gaps know nothing of: its cells would have
+// lists of more than 128. Control points still farther out are left to the far search: the cells in front of the gap would have
+// such lists, for every query at the rim. 3M x 2048, K = 8, us, with planes beyond all control points and nothing moved in -> so:
+// no outlier 219 -> 219, one at 10 (1000) times the deviation 295 -> 219 (534 -> 220), in the sample 2775 -> 224; normal points
+// times exp(normal) 1786 -> 930; points nine tenths of which lie in a plane 324 -> 315.
 // Every block computes the planes for itself (3 us) instead of waiting for another launch.
 template <int kG>
 __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<kG>& s) {
   constexpr int S = PlaneLds<kG>::kSamples, kSpare = kG > 16 ? 2 : 0;
   const int t = threadIdx.x;
-  if constexpr (kSpare > 0) {
-    uint32_t lo[3] = {~0u, ~0u, ~0u}, hi[3] = {0u, 0u, 0u};
-    for (int i = t; i < M; i += kBuildThreads) {
-      const float4 p      = s_y[i];
-      const uint32_t b[3] = {ordered_bits(p.x), ordered_bits(p.y), ordered_bits(p.z)};
-#pragma unroll
-      for (int c = 0; c < 3; ++c) lo[c] = min(lo[c], b[c]), hi[c] = max(hi[c], b[c]);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1)
-        lo[c] = min(lo[c], (uint32_t) __shfl_xor((int) lo[c], d, kWave)), hi[c] = max(hi[c], (uint32_t) __shfl_xor((int) hi[c], d, kWave));
-      if ((t & 63) == 0) s.least[c][t >> 6] = lo[c], s.most[c][t >> 6] = hi[c];
-    }
-  }
   for (int e = t; e < 3 * S; e += kBuildThreads) {
     const int a = e / S, j = e - a * S;
     const float4 p = s_y[(int) ((int64_t) j * M / S)];
@@ -188,9 +181,41 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
       const uint4 k = *(const uint4*) &s.key[a][i];
       rank += (k.x < mine) + (k.y < mine) + (k.z < mine) + (k.w < mine);
     }
-    s.sorted[a][rank] = from_ordered_bits(mine & ~(uint32_t) (S - 1));
+    s.along[a][rank] = from_ordered_bits(mine & ~(uint32_t) (S - 1));
   }
   __syncthreads();
+  for (int e = t; e < 3 * S; e += kBuildThreads) {
+    const int a = e / S, j = e - a * S;
+    const float* all  = s.along[a];
+    const float inner = all[S - 9] - all[8], outer = all[S - 2] - all[1];
+    const bool even   = inner > 0.125f * outer;
+    const float rim   = even ? kRim * inner : outer > 0.0f ? outer : __builtin_inff();
+    s.sorted[a][j]    = fminf(fmaxf(all[j], all[even ? 8 : 1] - rim), all[even ? S - 9 : S - 2] + rim);
+  }
+  __syncthreads();
+  if constexpr (kSpare > 0) {
+    float lo[3], hi[3], least[3], most[3];  // the sample's extent and kRim of it on either side
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float rim = kRim * (s.sorted[c][S - 1] - s.sorted[c][0]);
+      lo[c] = s.sorted[c][0] - rim, hi[c] = s.sorted[c][S - 1] + rim;
+      least[c] = __builtin_inff(), most[c] = -__builtin_inff();
+    }
+    for (int i = t; i < M; i += kBuildThreads) {
+      const float4 p    = s_y[i];
+      const float at[3] = {p.x, p.y, p.z};
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        if (at[c] >= lo[c] && at[c] <= hi[c]) least[c] = fminf(least[c], at[c]), most[c] = fmaxf(most[c], at[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1)
+        least[c] = fminf(least[c], __shfl_xor(least[c], d, kWave)), most[c] = fmaxf(most[c], __shfl_xor(most[c], d, kWave));
+      if ((t & 63) == 0) s.least[c][t >> 6] = least[c], s.most[c][t >> 6] = most[c];
+    }
+  }
   const int a = t >> 6, lane = t & 63;  // a wavefront per axis
   if (a < 3) {
     constexpr int kPer = S / 64;
@@ -215,10 +240,10 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
     const float lo = s.sorted[a][0], hi = s.sorted[a][S - 1], ext = hi - lo;
     float first = lo - 0.1f * ext, last = hi + 0.1f * ext;
     if constexpr (kSpare > 0) {
-      uint32_t least = s.least[a][0], most = s.most[a][0];
+      float least = s.least[a][0], most = s.most[a][0];
 #pragma unroll
-      for (int w = 1; w < kBuildThreads / kWave; ++w) least = min(least, s.least[a][w]), most = max(most, s.most[a][w]);
-      first = fminf(from_ordered_bits(least), first) - 0.05f * ext, last = fmaxf(from_ordered_bits(most), last) + 0.05f * ext;
+      for (int w = 1; w < kBuildThreads / kWave; ++w) least = fminf(least, s.least[a][w]), most = fmaxf(most, s.most[a][w]);
+      first = fminf(least, first) - 0.05f * ext, last = fmaxf(most, last) + 0.05f * ext;
     }
     float v = -3e38f;
     if (lane <= kG) {

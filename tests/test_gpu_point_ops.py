@@ -291,6 +291,37 @@ def test_knn_control_points_with_nan(N, M, K, axes, count, device):
     assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
 
 
+def _knn_time(pts, ctrl, K):
+    """Microseconds a call: the best of five times 20."""
+    from fast_sp_gs_amd._C import get_C_function
+    knn, best = get_C_function('knn_topk'), float('inf')
+    for _ in range(6):  # the first one warms up
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(20):
+            knn(pts, ctrl, K)
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) * 1000 / 20)
+    return best
+
+
+# One control point far from all others, of those the grid's planes are taken from (number 0) or not: the others' cells keep
+# short lists. The call took 2.4 and 13 times as long as without it when the planes followed it.
+@pytest.mark.parametrize('which', [0, 1025])
+def test_knn_one_far_control_point(which, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(which)
+    N, M, K = 1_000_000, 2048, 8
+    pts, ctrl = torch.randn(N, 3, generator=g).to(device), torch.randn(M, 3, generator=g).to(device)
+    without = _knn_time(pts, ctrl, K)
+    ctrl[which] = torch.tensor([2500.0, 50.0, -3500.0])
+    d2, idx = get_C_function('knn_topk')(pts, ctrl, K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+    assert _knn_time(pts, ctrl, K) < 1.6 * without
+
+
 LBS_CASES = [  # (warp method with a local rotation | None without one, weight method)
     (None, 'weighted_kernel'),   # the reference's default configuration: translations only, kernel weights
     (None, 'dist'), ('LBS', 'dist'), ('LBS_c', 'dist'), ('LBS_c', 'weighted_kernel'), ('LBS', 'kernel'),
