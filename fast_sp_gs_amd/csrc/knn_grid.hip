@@ -11,7 +11,8 @@
 //   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 35 entries for 2048 control
 //      points and G = 32). The walk only keeps the K + 1 smallest keys -- the distance in 2^-20 parts of
 //      the cell's bound, then the control point's number -- in a sorted register list, one v_med3_u32 per slot; the K exact
-//      distances are formed again afterwards. Queries whose keys cannot separate two neighbours (distances in the same part),
+//      distances are formed again afterwards. Queries whose keys cannot separate two neighbours (distances in the same part)
+//      walk again with parts of another kind if that can help (kCoarseParts); the others of these, those
 //      whose cell has more than 128 candidates, or that lie outside the grid are taken by the whole wavefront one at a
 //      time (64 control points per step), or all together by the search over all control points when they are many.
 //      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
@@ -22,6 +23,7 @@
 // vector issue (2080 instructions per 64 queries); the LDS and the address path of the vector memory are busy half the time.
 // 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -36,6 +38,17 @@ constexpr int kOctantCap = 1024;  // candidates of an octant of a coarse cell
 constexpr int kAhead = 4;
 constexpr uint32_t kNumberBits = 0xfff;  // of a key: the control point's number, 20 bits of distance above it
 static_assert(kMaxPoints + 8 <= (int) kNumberBits, "the numbers behind the last point, too");
+// The distances of a key are equal parts of the cell's bound at first (coarse); where control points sit in clusters much tighter
+// than their cells, all of a query's neighbours fall into the same few parts. Queries with two neighbours in one part, and that
+// below this one (of 2^20), walk their list again with fine parts, which are at least four times as many there; above, equal
+// distances are the rule (points on a lattice). A wavefront with kMostLanes queries in cells of kCrowded control points or more
+// takes fine parts at once: they cost an instruction more per candidate, and without clusters one query in 700 would need the
+// exact search. 128 clusters of 16 among 2048 control points, queries around them, 3M, K = 8, radius 0.01 / 0.001 / 0.0001, us:
+// 267 / 2860 / 3150 with coarse parts only, 214 / 263 / 306 with the second walk, 204 / 209 / 207 so; a key of the float's upper
+// 25 bits and the list position: 225 / 220 / 221.
+constexpr uint32_t kCoarseParts = (1u << 13) * (kNumberBits + 1);
+constexpr uint32_t kCrowdedBit = 0x10000;  // of a cell's length
+constexpr int kCrowded = 8, kMostLanes = 16;
 constexpr int kBuildThreads = 512, kQueryThreads = 512;
 constexpr uint32_t kLongList = 0xffff;
 constexpr int kFewQueries = 16384;
@@ -59,7 +72,7 @@ Scheme knn_scheme(int N, int M, int D, int K) {
   return M > 640 || N >= 1000000 ? kGrid32 : kGrid16;
 }
 
-// A cell: how many candidates its list holds (or kLongList), and what takes a squared distance to 2^32 at the cell's bound.
+// A cell: how many candidates its list holds (or kLongList) and kCrowdedBit, and what takes a squared distance to 2^32 at the cell's bound.
 struct Cell {
   uint32_t length;
   float scale;
@@ -416,11 +429,11 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
 #pragma unroll
     for (int c = 0; c < kCells; ++c) reach[c] = widened(wave_kth_bound(least_far[c], K));
   }
-  int n[kCells];
+  int n[kCells], inside[kCells];  // candidates, and how many of them lie in the cell itself
   uint16_t* list[kCells];
 #pragma unroll
   for (int c = 0; c < kCells; ++c) {
-    n[c] = 0;
+    n[c] = 0, inside[c] = 0;
     list[c] = lists + (size_t) (((corner[2] + c / (kIn * kIn)) * kG + corner[1] + c / kIn % kIn) * kG + corner[0] + c % kIn) * kListCap;
   }
   for (int i0 = 0; i0 < n_from; i0 += kWave) {
@@ -436,9 +449,16 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
         f[a][h] = d * d;
       }
     const unsigned long long there = wave_ballot(i0 + lane < n_from);
+    float d2[kCells], nearest = __builtin_inff();
+#pragma unroll
+    for (int c = 0; c < kCells; ++c) d2[c] = (f[0][c % kIn] + f[1][c / kIn % kIn]) + f[2][c / (kIn * kIn)], nearest = fminf(nearest, d2[c]);
+    if (there & wave_ballot(nearest == 0.0f)) {
+#pragma unroll
+      for (int c = 0; c < kCells; ++c) inside[c] += (int) __popcll(there & wave_ballot(d2[c] == 0.0f));
+    }
 #pragma unroll
     for (int c = 0; c < kCells; ++c) {
-      const unsigned long long m = there & wave_ballot((f[0][c % kIn] + f[1][c / kIn % kIn]) + f[2][c / (kIn * kIn)] <= reach[c]);
+      const unsigned long long m = there & wave_ballot(d2[c] <= reach[c]);
       const int pos = n[c] + lanes_below(m);
       if ((m >> lane & 1ull) && pos < kListCap) list[c][pos] = (uint16_t) i;
       n[c] += (int) __popcll(m);
@@ -450,7 +470,9 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
     if (fits && lane < 8 && n[c] + lane < (n[c] + 7) / 8 * 8) list[c][n[c] + lane] = (uint16_t) M;
     // the K nearest of any query of the cell are nearer than `reach`: their parts stay below 2^32, the others' may saturate
-    if (lane == 0) cells[(list[c] - lists) / kListCap] = Cell{fits ? (uint32_t) n[c] : kLongList, fminf(4294967296.0f / reach[c], 3e38f)};
+    if (lane == 0)
+      cells[(list[c] - lists) / kListCap] = Cell{fits ? (uint32_t) n[c] | (inside[c] >= kCrowded ? kCrowdedBit : 0u) : kLongList,
+                                                 fminf(4294967296.0f / reach[c], 3e38f)};
   }
 }
 
@@ -471,6 +493,15 @@ __device__ __forceinline__ uint32_t saturated_u32(float v) {
   uint32_t r;
   asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
   return r;
+}
+
+// The upper 20 bits of a key, with anything below them: of a squared distance times the cell's scale. Coarse: equal parts of the
+// cell's bound. Fine: an exponent of five bits and 15 bits behind it, for neighbours that are much nearer than the bound.
+template <bool kFine>
+__device__ __forceinline__ uint32_t distance_part(float scaled) {
+  if constexpr (!kFine) return saturated_u32(scaled);
+  constexpr float kBelow = 4294967040.0f;  // the largest float below 2^32
+  return (__float_as_uint(__builtin_amdgcn_fmed3f(scaled, 1.0f, kBelow)) << 4) - (0x3f800000u << 4);
 }
 
 template <int kK>
@@ -610,59 +641,79 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         inside = inside && q[a] >= s_plane[a][0] && q[a] < s_plane[a][kG];  // false for NaN
         cell   = cell * kG + i;
       }
-      const Cell here = inside ? cells[cell] : Cell{kLongList, 0.0f};
-      bool unknown    = here.length == kLongList;
-      const int n_list = here.length == kLongList ? 0 : (int) here.length;
+      const Cell here  = inside ? cells[cell] : Cell{kLongList, 0.0f};
+      const bool listed = here.length != kLongList;
       const uint16_t* list = lists + (size_t) cell * kListCap;
       uint32_t key[kK + 1];
-#pragma unroll
-      for (int k = 0; k <= kK; ++k) key[k] = 0xffffffffu;
       auto insert = [&](uint32_t nk) {
 #pragma unroll
         for (int k = kK; k >= 1; --k) key[k] = med3_u32(key[k - 1], nk, key[k]);
         key[0] = min(key[0], nk);
       };
-      auto key_of = [&](uint32_t i, float qx, float qy, float qz, float scale) {
-        return and_or_b32(saturated_u32(distance2(qx, qy, qz, s_y[i]) * scale), ~kNumberBits, i);
-      };
-      uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
-      int c = 0;
-      unsigned long long longer;
-      for (;; c += 8) {
-        longer = wave_ballot(c < n_list);
-        if (__popcll(longer) <= kFewLists) break;
-        if (c < n_list) {
-          const uint4 now = next;
-          if (c + 8 < n_list) next = *(const uint4*) (list + c + 8);
-          const uint32_t w[4] = {now.x, now.y, now.z, now.w};
+      // The smallest keys of the first n_list candidates and of those that are there already.
+      auto walk = [&](auto fine, int n_list) {
+        auto key_of = [&](uint32_t i, float qx, float qy, float qz, float scale) {
+          return and_or_b32(distance_part<decltype(fine)::value>(distance2(qx, qy, qz, s_y[i]) * scale), ~kNumberBits, i);
+        };
+        uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
+        int c = 0;
+        unsigned long long longer;
+        for (;; c += 8) {
+          longer = wave_ballot(c < n_list);
+          if (__popcll(longer) <= kFewLists) break;
+          if (c < n_list) {
+            const uint4 now = next;
+            if (c + 8 < n_list) next = *(const uint4*) (list + c + 8);
+            const uint32_t w[4] = {now.x, now.y, now.z, now.w};
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            insert(key_of((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu), q[0], q[1], q[2], here.scale));
-        }
-      }
-      while (longer) {  // what is left of a few long lists: the whole wavefront on one, a candidate per lane
-        const int l = __builtin_ctzll(longer);
-        longer &= longer - 1;
-        const int count = __builtin_amdgcn_readlane(n_list, l), its_cell = __builtin_amdgcn_readlane(cell, l);
-        const uint16_t* its_list = lists + (size_t) its_cell * kListCap;
-        auto its = [&](float v) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l)); };
-        const float qx = its(q[0]), qy = its(q[1]), qz = its(q[2]), scale = its(here.scale);
-        for (int e = c; e < count; e += kWave) {
-          const uint32_t nk = key_of(its_list[min(e + lane, count - 1)], qx, qy, qz, scale);
-          unsigned long long nearer = wave_ballot(e + lane < count) & wave_ballot(nk < (uint32_t) __builtin_amdgcn_readlane(key[kK], l));
-          while (nearer) {
-            const uint32_t v = __builtin_amdgcn_readlane(nk, __builtin_ctzll(nearer));
-            nearer &= nearer - 1;
-            insert(lane == l ? v : ~0u);
+            for (int j = 0; j < 8; ++j)
+              insert(key_of((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu), q[0], q[1], q[2], here.scale));
           }
         }
-      }
+        while (longer) {  // what is left of a few long lists: the whole wavefront on one, a candidate per lane
+          const int l = __builtin_ctzll(longer);
+          longer &= longer - 1;
+          const int count = __builtin_amdgcn_readlane(n_list, l), its_cell = __builtin_amdgcn_readlane(cell, l);
+          const uint16_t* its_list = lists + (size_t) its_cell * kListCap;
+          auto its = [&](float v) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l)); };
+          const float qx = its(q[0]), qy = its(q[1]), qz = its(q[2]), scale = its(here.scale);
+          for (int e = c; e < count; e += kWave) {
+            const uint32_t nk = key_of(its_list[min(e + lane, count - 1)], qx, qy, qz, scale);
+            unsigned long long nearer = wave_ballot(e + lane < count) & wave_ballot(nk < (uint32_t) __builtin_amdgcn_readlane(key[kK], l));
+            while (nearer) {
+              const uint32_t v = __builtin_amdgcn_readlane(nk, __builtin_ctzll(nearer));
+              nearer &= nearer - 1;
+              insert(lane == l ? v : ~0u);
+            }
+          }
+        }
+      };
+#pragma unroll
+      for (int k = 0; k <= kK; ++k) key[k] = 0xffffffffu;
+      const int n_list = listed ? (int) (here.length & 0xffu) : 0;
+      // most queries in cells with many control points: fine parts at once
+      const bool fine_first = __popcll(wave_ballot(listed && (here.length & kCrowdedBit))) >= kMostLanes;
+      if (fine_first) walk(std::true_type(), n_list);
+      else walk(std::false_type(), n_list);
       // neighbours in the same part are not in a known order; where the parts saturate (there are not K points at a finite
       // distance, or the bound is next to nothing) nothing is known
+      auto same_part = [&](uint32_t below) {
+        bool same = false;
 #pragma unroll
-      for (int k = 0; k < kK; ++k)
-        if ((key[k] ^ key[k + 1]) <= kNumberBits) unknown = true;
-      if (key[kK - 1] >= ~kNumberBits) unknown = true;
+        for (int k = 0; k < kK; ++k) same |= (key[k] ^ key[k + 1]) <= kNumberBits && key[k] < below;
+        return same;
+      };
+      bool same = same_part(~0u);
+      if (!fine_first && wave_ballot(same)) {
+        const bool again = listed && same_part(kCoarseParts);
+        if (wave_ballot(again)) {
+#pragma unroll
+          for (int k = 0; k <= kK; ++k) key[k] = again ? 0xffffffffu : key[k];
+          walk(std::true_type(), again ? n_list : 0);
+          same = same_part(~0u);
+        }
+      }
+      const bool unknown = !listed || same || key[kK - 1] >= ~kNumberBits;
       float bd[kK];
       int bi[kK];
 #pragma unroll

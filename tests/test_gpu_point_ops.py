@@ -322,6 +322,39 @@ def test_knn_one_far_control_point(which, device):
     assert _knn_time(pts, ctrl, K) < 1.6 * without
 
 
+def _clusters(N, M, radius, g):
+    """M control points in clusters of 16, queries around them."""
+    ctrl = (torch.randn(M // 16, 1, 3, generator=g) + radius * torch.randn(M // 16, 16, 3, generator=g)).reshape(-1, 3)
+    return ctrl[torch.randint(M, (N,), generator=g)] + radius * torch.randn(N, 3, generator=g), ctrl
+
+
+# Neighbours much nearer than their cell's bound: the keys' coarse parts do not tell them apart, the fine ones do; below 2^-32 of
+# the bound, and for coinciding control points, neither does.
+@pytest.mark.parametrize('N,M,K', [(17000, 640, 4), (17001, 2560, 8), (40000, 1024, 1), (17000, 192, 7)])
+@pytest.mark.parametrize('radius', [1e-1, 1e-2, 1e-3, 1e-4, 1e-6])
+@pytest.mark.parametrize('mixed', [False, True])
+def test_knn_clusters(N, M, K, radius, mixed, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N + M + K)
+    pts, ctrl = _clusters(N, M, radius, g)
+    if mixed:  # a quarter of the queries between the clusters, control points of a cluster that coincide
+        pts[::4] = torch.randn(len(pts[::4]), 3, generator=g)
+        ctrl[32:40] = ctrl[32]
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+
+
+def test_knn_clusters_keep_to_the_lists(device):
+    """With the keys' coarse parts alone, tight clusters sent every query to the exact search: thirteen times the time."""
+    g = torch.Generator().manual_seed(7)
+    N, M, K = 1_000_000, 2048, 8
+    loose = _knn_time(torch.randn(N, 3, generator=g).to(device), torch.randn(M, 3, generator=g).to(device), K)
+    for radius in (1e-2, 1e-3, 1e-4):
+        pts, ctrl = _clusters(N, M, radius, g)
+        assert _knn_time(pts.to(device), ctrl.to(device), K) < 1.6 * loose
+
+
 LBS_CASES = [  # (warp method with a local rotation | None without one, weight method)
     (None, 'weighted_kernel'),   # the reference's default configuration: translations only, kernel weights
     (None, 'dist'), ('LBS', 'dist'), ('LBS_c', 'dist'), ('LBS_c', 'weighted_kernel'), ('LBS', 'kernel'),
