@@ -312,7 +312,6 @@ __global__ void __launch_bounds__(256) cull_mask_kernel(int P, int gx, int gy, c
 // Layout of the `bins` buffer of the bucket binning: the queue length of the long segments in front of the B x T matrix
 // of per-(walk block, tile) instance counts.
 constexpr int kPrefixTiles = 64, kPrefixWaves = 16, kPrefixChunk = 32;  // walk blocks <= kPrefixWaves * kPrefixChunk
-constexpr size_t kBinsExceeds = 8;  // behind queue length and instance count: there is no room for them
 constexpr size_t kBinsSums = 256;  // behind the queue length: the instances of every 64 tiles
 constexpr size_t kBinsHeader = 4096;
 static_assert(kBinsSums + (kMaxLdsTiles / kPrefixTiles) * sizeof(uint32_t) <= kBinsHeader, "the sums fit the header");
@@ -354,7 +353,6 @@ __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, i
   __shared__ unsigned s_count[kTiles];
   // first of all, so that the instance count reaches the host while the rest of the counting is still running
   if (publish.counters && blockIdx.x == 0 && threadIdx.x < kWave) publish_slot_regions(publish);
-  if (!publish.counters && publish.exceeds && blockIdx.x == 0 && threadIdx.x == 0) *publish.exceeds = 0;
   const int T = gx * gy;
   for (int t = threadIdx.x; t < T; t += blockDim.x) s_count[t] = 0u;
   __syncthreads();
@@ -442,6 +440,7 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
     return;
   }
   const int T = gx * gy;
+  if ((int64_t) ranges[2 * (size_t) T - 1] > R) return;  // the last tile's end: R was a guess, and too small (see gs_view_scatter)
   const uint32_t* row = hist + (size_t) walk_row(blockIdx.x, (P + per_block - 1) / per_block) * T;
   for (int t = threadIdx.x; t < T; t += blockDim.x) s_cursor[t] = (unsigned) ranges[2 * (size_t) t] + row[t];
   __syncthreads();
@@ -466,15 +465,13 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
 // With `sums` (the instances of every 64 tiles) block b scans the tiles from 4096 b on and adds what lies in front of them
 // itself; without, one block walks all tiles.
 // ends = false: ranges[t] = (start, start), for a scatter that advances ranges[t].y; ends = true: (start, end).
-// exceeds (optional): set when there is no room for the instances; all ranges are empty then.
 __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long long* __restrict__ ranges,
                                                          const uint32_t* __restrict__ sums, int* __restrict__ large_count,
-                                                         bool ends, const int* __restrict__ exceeds) {
+                                                         bool ends) {
   __shared__ unsigned long long s_wave[16];
   const int lane = __lane_id(), wave = threadIdx.x / kWave;
   unsigned long long carry = 0;
   const int first = sums ? blockIdx.x * 4096 : 0, last = sums ? min(T, first + 4096) : T;
-  const bool room = !exceeds || *exceeds == 0;  // on its way while the counts are
   if (first > 0) {
     unsigned long long before = 0;
     for (int b = threadIdx.x; b < first / kPrefixTiles; b += blockDim.x) before += sums[b];
@@ -504,7 +501,7 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
     unsigned long long run = carry + base + inc - sum;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (t0 + k < T) ranges[2 * (size_t) (t0 + k)] = room ? run : 0, ranges[2 * (size_t) (t0 + k) + 1] = !room ? 0 : ends ? run + c[k] : run;
+      if (t0 + k < T) ranges[2 * (size_t) (t0 + k)] = run, ranges[2 * (size_t) (t0 + k) + 1] = ends ? run + c[k] : run;
       run += c[k];
     }
     carry += total;
@@ -518,9 +515,8 @@ __global__ void __launch_bounds__(1024) tile_scan_kernel(int T, unsigned long lo
 constexpr int kColumn = 64;
 
 __global__ void __launch_bounds__(1024) tile_prefix_scan_kernel(int T, int B, uint32_t* __restrict__ hist,
-    unsigned long long* __restrict__ ranges, int* __restrict__ large_count, const int* __restrict__ exceeds) {
+    unsigned long long* __restrict__ ranges, int* __restrict__ large_count) {
   __shared__ uint32_t s_wave[16];
-  const bool room = !exceeds || *exceeds == 0;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   uint32_t c[kColumn], sum = 0;
 #pragma unroll
@@ -554,7 +550,7 @@ __global__ void __launch_bounds__(1024) tile_prefix_scan_kernel(int T, int B, ui
   }
   if (t < T) {
     const uint32_t start = before + inc - sum;
-    ranges[2 * (size_t) t] = room ? start : 0, ranges[2 * (size_t) t + 1] = room ? start + sum : 0;
+    ranges[2 * (size_t) t] = start, ranges[2 * (size_t) t + 1] = start + sum;
     uint32_t run = 0;
 #pragma unroll
     for (int i = 0; i < kColumn; ++i) {
@@ -1373,14 +1369,12 @@ namespace {
 
 // First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
 // (start, end); the header of `bins` is set (length of the long-segment queue: 0 | instances in all tiles).
-// With publish.capacity the ranges stay empty when there are more instances than that.
 int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in, int64_t* ranges,
-               void* bins, hipStream_t s, SlotPublish publish = SlotPublish{}) {
+               void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
   int* header = (int*) bins;
-  if (publish.capacity > 0 && publish.capacity < INT64_MAX) publish.exceeds = (int*) ((char*) bins + kBinsExceeds);
   const BinsLayout bl = bins_layout(P, T);
   if (bl.blocks > 0) {
     uint32_t* hist = (uint32_t*) ((char*) bins + kBinsHeader);
@@ -1391,13 +1385,11 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
                          hist, publish);
     });
     if (T <= 1024 && bl.blocks <= kColumn) {
-      hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header,
-                         (const int*) publish.exceeds);
+      hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header);
     } else {
       hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
                          bl.blocks, hist, rng, sums);
-      hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true,
-                         (const int*) publish.exceeds);
+      hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
     }
     // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
     // sorts) is built from them by an extra block of the scatter, in the second part.
@@ -1409,30 +1401,24 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
       FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, false>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx,
                                                gy, (int64_t) 0, (const float2*) means2D, (const float*) nullptr, radii, in,
                                                rng, (uint64_t*) nullptr));
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, (const uint32_t*) nullptr, header, false,
-                       (const int*) nullptr);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, s, T, rng, (const uint32_t*) nullptr, header, false);
   }
   return check_launch("gs_prepare_count");
 }
 
-// Second part: scatter (depth bits << 32 | surfel) into the tile segments and sort every segment. pad: the list positions
-// behind the kept instances get the fast path's padding entries.
-int fill_sort(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
-              int64_t R, int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace, void* bins,
-              bool pad, hipStream_t s) {
+// Second part: scatter (depth bits << 32 | surfel) into the tile segments. R: what there is room for; `entries` is left as it is
+// where the instances are more (tile grids within kMaxLdsTiles, whose ranges are final).
+void fill_scatter(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
+                  int64_t R, int64_t* ranges, void* workspace, void* bins, hipStream_t s) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
-  int* header             = (int*) bins;
   uint64_t* entries       = sort_keys_in(R, workspace);
-  // queue of long segments: at most R / kSmallSegment tiles, kept behind the entries in the workspace
-  int* large_list = (int*) ((char*) workspace + sort_layout(R).keys1);
   const BinsLayout bl = bins_layout(P, T);
-  // The schedule table: built by one extra block of the scatter (the ranges are final since the counting part), or by a
-  // launch of its own on the global-atomic path, whose ranges only become final with the scatter.
-  const int* order = nullptr;
   if (bl.blocks > 0) {
-    int* build = nullptr;
+    // The schedule table is built by one extra block of the scatter (the ranges are final since the counting part).
+    const int* order = nullptr;
+    int* build       = nullptr;
     (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
     // Entries that do not fit the dies' L2s (4 MB each) leave them in pieces, the smaller the more blocks write at once: LDS that
     // nobody uses keeps a second block off the compute unit. 3M surfels 1352x1014, 6M entries: 71 -> 56 us; 300k 800x800, 1.4M: 12.8 -> 13.9.
@@ -1446,8 +1432,23 @@ int fill_sort(int P, int W, int H, const float* means2D, const float* depths, co
   } else {
     FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, true>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy,
                                              R, (const float2*) means2D, depths, radii, in, rng, entries));
-    (void) launch_tile_order(gx, gy, ranges, s, &order);
   }
+}
+
+// Third part: sort every segment. `R` and `workspace` as for the scatter. pad: the list positions behind the kept instances get the
+// fast path's padding entries.
+void fill_sort(int P, int W, int H, int64_t R, int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace,
+               void* bins, bool pad, hipStream_t s) {
+  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
+  const int T  = gx * gy;
+  int* header       = (int*) bins;
+  uint64_t* entries = sort_keys_in(R, workspace);
+  // queue of long segments: at most R / kSmallSegment tiles, kept behind the entries in the workspace
+  int* large_list = (int*) ((char*) workspace + sort_layout(R).keys1);
+  // The schedule table: the scatter's, or a launch of its own on the global-atomic path, whose ranges only become final with the
+  // scatter.
+  const int* order = nullptr;
+  (void) launch_tile_order(gx, gy, ranges, s, &order);
   // with padding, 256 blocks more than tiles: they write the entries behind the kept instances
   hipLaunchKernelGGL(tile_sort_small_kernel, dim3(T + (pad ? 256 : 0)), dim3(256), 0, s, ranges, entries, point_list,
                      sorted_keys_out, header, large_list, order, T, R, (const int*) (header + 1),
@@ -1455,6 +1456,13 @@ int fill_sort(int P, int W, int H, const float* means2D, const float* depths, co
   if (P > kSmallSegment)  // a surfel is in a tile's list once
     hipLaunchKernelGGL(tile_sort_large_kernel, dim3(256), dim3(1024), 0, s, ranges, entries, point_list, sorted_keys_out,
                        header, large_list);
+}
+
+int fill_lists(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
+               int64_t R, int64_t* ranges, int32_t* point_list, int64_t* sorted_keys_out, void* workspace, void* bins,
+               bool pad, hipStream_t s) {
+  fill_scatter(P, W, H, means2D, depths, radii, in, R, ranges, workspace, bins, s);
+  fill_sort(P, W, H, R, ranges, point_list, sorted_keys_out, workspace, bins, pad, s);
   return check_launch("gs_prepare_fill");
 }
 }  // namespace
@@ -1465,7 +1473,7 @@ int fast_bucket_fill(int P, int W, int H, const float* means2D, const float* inv
                      hipStream_t s) {
   const WalkInputs in{inverse_m, opacities, keep_masks};
   if (int rc = fill_count(P, W, H, means2D, radii, in, ranges, bins, s)) return rc;
-  return fill_sort(P, W, H, means2D, depths, radii, in, R, ranges, point_list, sorted_keys_out, workspace, bins, true, s);
+  return fill_lists(P, W, H, means2D, depths, radii, in, R, ranges, point_list, sorted_keys_out, workspace, bins, true, s);
 }
 
 }  // namespace fsgs
@@ -1571,7 +1579,7 @@ FSGS_API int fsgs_gs_prepare_fill_counted(int P, int W, int H, const float* mean
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_prepare_fill: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
+  return fill_lists(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
                    false, (hipStream_t) stream);
 }
 
@@ -1634,61 +1642,12 @@ FSGS_API int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const floa
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
     return fail(kWorkspaceSmall, "gs_prepare_fill_culled: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? masks : nullptr}, R,
+  return fill_lists(P, W, H, means2D, depths, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? masks : nullptr}, R,
                    ranges, point_list, sorted_keys_out, workspace, bins, false, (hipStream_t) stream);
 }
 
-// The counting part for views whose preprocess handed out the record slots (instance_slots.hpp).
-namespace {
-int view_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in,
-               uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges, void* bins,
-               size_t bins_bytes, void* stream) {
-  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins, "gs_view_count: bad arguments");
-  FSGS_REQUIRE(means2D && radii && slot_counters && num_rendered_host, "gs_view_count: null pointer");
-  if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
-    return fail(kWorkspaceSmall, "gs_view_count: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
-  tile_order_invalidate((hipStream_t) stream);
-  __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
-  return fill_count(P, W, H, means2D, radii, in, ranges, bins, (hipStream_t) stream,
-                    SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
-}
-}  // namespace
-
-FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii,
-                                const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
-                                int64_t* num_rendered_host, int64_t* ranges, void* bins, size_t bins_bytes,
-                                void* stream) {
-  return view_count(P, W, H, means2D, radii, WalkInputs{nullptr, nullptr, culling_enabled() ? keep_masks : nullptr},
-                    slot_counters, slot_regions, num_rendered_host, ranges, bins, bins_bytes, stream);
-}
-
-FSGS_API int fsgs_gs_2d_fast_view_count(int P, int W, int H, const float* means2D, const float* inverse_m,
-                                        const float* opacities, const int32_t* radii, const uint32_t* keep_masks,
-                                        uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host,
-                                        int64_t* ranges, void* bins, size_t bins_bytes, void* stream) {
-  FSGS_REQUIRE(inverse_m && opacities && keep_masks, "gs_2d_fast_view_count: null pointer");
-  return view_count(P, W, H, means2D, radii, WalkInputs{inverse_m, opacities, keep_masks}, slot_counters, slot_regions,
-                    num_rendered_host, ranges, bins, bins_bytes, stream);
-}
-
-FSGS_API int fsgs_gs_2d_fast_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m,
-                                       const float* depths, const float* opacities, const int32_t* radii,
-                                       const uint32_t* keep_masks, int64_t R, int64_t* ranges, int32_t* point_list,
-                                       void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes,
-                                       void* stream) {
-  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && R >= 0 && ranges && bins, "gs_2d_fast_view_fill: bad arguments");
-  FSGS_REQUIRE(R < (int64_t) 0x7fffffff, "gs_2d_fast_view_fill: %lld instances exceed the 2^31-1 limit", (long long) R);
-  if (R == 0) return kOk;
-  FSGS_REQUIRE(means2D && inverse_m && depths && opacities && radii && keep_masks && point_list && workspace,
-               "gs_2d_fast_view_fill: null pointer");
-  if (workspace_bytes < sort_workspace_bytes(R) || bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
-    return fail(kWorkspaceSmall, "gs_2d_fast_view_fill: workspace %zu < %zu or bins %zu < %zu bytes", workspace_bytes,
-                sort_workspace_bytes(R), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{inverse_m, opacities, keep_masks}, R, ranges, point_list,
-                   nullptr, workspace, bins, false, (hipStream_t) stream);
-}
-
-// What the views call: both parts, for either kind of surfels (inverse_m and opacities: the fast ones) and Gaussians.
+// What the views call, for either kind of surfels (inverse_m and opacities: the fast ones) and Gaussians: the counting part, for
+// views whose preprocess handed out the record slots (instance_slots.hpp), the scatter and the sort.
 namespace {
 WalkInputs view_inputs(const float* inverse_m, const float* opacities, const uint32_t* keep_masks) {
   return inverse_m ? WalkInputs{inverse_m, opacities, keep_masks}
@@ -1696,42 +1655,74 @@ WalkInputs view_inputs(const float* inverse_m, const float* opacities, const uin
 }
 }  // namespace
 
-FSGS_API size_t fsgs_gs_view_fill_workspace_bytes(int64_t R) {
-  return sort_layout(R).keys1 + align_up((size_t) (R / kSmallSegment + 1) * sizeof(int), 256);  // entries, queue of long segments
-}
-
-FSGS_API int fsgs_gs_view_tally(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
+FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
                                 const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters,
-                                int32_t* slot_regions, int64_t* num_rendered_host, int64_t capacity, int64_t* ranges, void* bins,
+                                int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges, void* bins,
                                 size_t bins_bytes, void* stream) {
-  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins && capacity >= 0, "gs_view_tally: bad arguments");
-  FSGS_REQUIRE(means2D && radii && !slot_counters == !num_rendered_host && (!inverse_m || (opacities && keep_masks)),
-               "gs_view_tally: null pointer");
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && ranges && bins, "gs_view_count: bad arguments");
+  FSGS_REQUIRE(means2D && radii && slot_counters && num_rendered_host && (!inverse_m || (opacities && keep_masks)),
+               "gs_view_count: null pointer");
   if (bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
-    return fail(kWorkspaceSmall, "gs_view_tally: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+    return fail(kWorkspaceSmall, "gs_view_count: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
   tile_order_invalidate((hipStream_t) stream);
-  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
   return fill_count(P, W, H, means2D, radii, view_inputs(inverse_m, opacities, keep_masks), ranges, bins, (hipStream_t) stream,
-                    SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host, std::max<int64_t>(capacity, 1)});
+                    SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
 }
 
-FSGS_API int fsgs_gs_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
-                               const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity,
-                               int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
-                               size_t workspace_bytes, void* stream) {
-  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && capacity >= 0 && ranges && bins, "gs_view_fill: bad arguments");
-  FSGS_REQUIRE(capacity < (int64_t) 0x7fffffff, "gs_view_fill: %lld instances exceed the 2^31-1 limit", (long long) capacity);
-  FSGS_REQUIRE(means2D && depths && radii && (capacity == 0 || (point_list && workspace)) &&
-                   (!inverse_m || (opacities && keep_masks)), "gs_view_fill: null pointer");
-  if (capacity == 0) {
-    launch_zero_ranges(((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile), ranges, (hipStream_t) stream);
-    return check_launch("gs_view_fill");
+FSGS_API size_t fsgs_gs_view_lists_workspace_bytes(int64_t capacity) {
+  return sort_layout(capacity).keys1 + align_up((size_t) (capacity / kSmallSegment + 1) * sizeof(int), 256);  // entries, queue of long segments
+}
+
+namespace {
+int check_view_lists(const char* what, int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                     const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity,
+                     const int64_t* ranges, const void* bins, size_t bins_bytes, const void* workspace, size_t workspace_bytes) {
+  FSGS_REQUIRE(P > 0 && W > 0 && H > 0 && capacity > 0 && ranges && bins && workspace, "%s: bad arguments", what);
+  FSGS_REQUIRE(capacity < (int64_t) 0x7fffffff, "%s: %lld instances exceed the 2^31-1 limit", what, (long long) capacity);
+  FSGS_REQUIRE(means2D && depths && radii && (!inverse_m || (opacities && keep_masks)), "%s: null pointer", what);
+  if (workspace_bytes < fsgs_gs_view_lists_workspace_bytes(capacity) || bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
+    return fail(kWorkspaceSmall, "%s: workspace %zu < %zu or bins %zu < %zu bytes", what, workspace_bytes,
+                fsgs_gs_view_lists_workspace_bytes(capacity), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
+  return kOk;
+}
+bool ranges_final_before_scatter(int W, int H) {
+  return (int64_t) ((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile) <= kMaxLdsTiles;
+}
+}  // namespace
+
+// Tile grids beyond kMaxLdsTiles are scattered by cursors in the ranges, which allow it once: with the sort, for the count.
+FSGS_API int fsgs_gs_view_scatter(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                                  const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity,
+                                  int64_t* ranges, void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+  if (int rc = check_view_lists("gs_view_scatter", P, W, H, means2D, inverse_m, depths, opacities, radii, keep_masks, capacity,
+                                ranges, bins, bins_bytes, workspace, workspace_bytes))
+    return rc;
+  if (!ranges_final_before_scatter(W, H)) return kOk;
+  fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins,
+               (hipStream_t) stream);
+  return check_launch("gs_view_scatter");
+}
+
+FSGS_API int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                               const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R,
+                               int64_t capacity, int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  hipStream_t s = (hipStream_t) stream;
+  if (R == 0 && P > 0 && W > 0 && H > 0 && ranges) {
+    launch_zero_ranges(((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile), ranges, s);
+    return check_launch("gs_view_sort");
   }
-  if (workspace_bytes < fsgs_gs_view_fill_workspace_bytes(capacity) || bins_bytes < fsgs_gs_prepare_bins_bytes(P, W, H))
-    return fail(kWorkspaceSmall, "gs_view_fill: workspace %zu < %zu or bins %zu < %zu bytes", workspace_bytes,
-                fsgs_gs_view_fill_workspace_bytes(capacity), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
-  return fill_sort(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, point_list,
-                   nullptr, workspace, bins, false, (hipStream_t) stream);
+  FSGS_REQUIRE(R > 0 && R <= capacity && point_list, "gs_view_sort: bad arguments (%lld instances, room for %lld)", (long long) R,
+               (long long) capacity);
+  if (int rc = check_view_lists("gs_view_sort", P, W, H, means2D, inverse_m, depths, opacities, radii, keep_masks, capacity, ranges,
+                                bins, bins_bytes, workspace, workspace_bytes))
+    return rc;
+  if (!ranges_final_before_scatter(W, H))
+    fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins, s);
+  fill_sort(P, W, H, capacity, ranges, point_list, nullptr, workspace, bins, false, s);
+  return check_launch("gs_view_sort");
 }
 
 // Waits until the count has been written. Reading the word is all it takes as long as the stream works; a stream that
@@ -1773,6 +1764,6 @@ FSGS_API int fsgs_gs_prepare_fill(int P, int W, int H, const float* means2D, con
     return fail(kWorkspaceSmall, "gs_prepare_fill: bins %zu < %zu bytes", bins_bytes,
                 fsgs_gs_prepare_bins_bytes(P, W, H));
   if (int rc = fill_count(P, W, H, means2D, radii, WalkInputs{}, ranges, bins, s)) return rc;
-  return fill_sort(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
+  return fill_lists(P, W, H, means2D, depths, radii, WalkInputs{}, R, ranges, point_list, sorted_keys_out, workspace, bins,
                    false, s);
 }

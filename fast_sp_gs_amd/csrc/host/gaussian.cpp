@@ -77,15 +77,6 @@ Buffers forward_view(const GaussianView& v, bool train) {
     b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.n_contrib = empty({H, W}, like, at::kInt);
     if (has(v.extras)) b.extras = empty({E, H, W}, like);
   };
-  auto blend_lists = [&] {
-    if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);
-    check(fsgs_gaussian_view_forward((int) P, W, H, E, f32(v.means2D), f32(b.conic_opacity), colors,
-                                     E ? f32(*v.extras) : nullptr, i32(b.point_list), i64(b.ranges),
-                                     i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
-                                     i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity),
-                                     E ? f32(b.extras) : nullptr, i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), stream),
-          blend);
-  };
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
@@ -98,47 +89,35 @@ Buffers forward_view(const GaussianView& v, bool train) {
                                   i32(b.radii), data<uint8_t>(b.visible), counters.data(),
                                   has(v.cov3D) ? nullptr : b.keep.at<float>(s.cov3D), f32(b.conic_opacity), masks, stream),
           what);
-    auto tally = [&](uint64_t* slots, int32_t* regions, int64_t* word, int64_t positions) {
-      check(fsgs_gs_view_tally((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, slots, regions, word, positions,
-                               i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
-            "GS_prepare");
-    };
-    // fill the lists and blend them
-    auto second_half = [&](int64_t positions) {
-      b.point_list = empty({positions}, like, at::kInt);
-      const size_t fill_bytes = fsgs_gs_view_fill_workspace_bytes(positions);
-      const Tensor fill = empty({(int64_t) fill_bytes}, like, at::kByte);
-      check(fsgs_gs_view_fill((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks, positions,
-                              i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes, fill.data_ptr(), fill_bytes,
-                              stream),
-            "GS_prepare");
-      blend_lists();
-    };
-    const int64_t guess = positions_to_guess(P, T);
-    tally(counters.data(), nullptr, count, guess > 0 ? guess : INT64_MAX);
+    check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
+                             nullptr, count, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
+          "GS_prepare");
     PendingCount pending(count, stream);
     counters.give_back();
-    blend_maps();  // what does not depend on the count is allocated while the device gets there
-    const bool guessed = guess > 0 && !pending.arrived();
-    if (guessed) second_half(guess);
-    const int64_t R = pending.wait("GS_prepare");
-    if (guess > 0 && R > guess) {  // the lists have been left empty
-      tally(nullptr, nullptr, nullptr, R);
-      second_half(R);
-    } else if (!guessed) {
-      second_half(R);
-    } else {
-      at::AutoDispatchBelowADInplaceOrView plain;  // what the view hands out are no views of the longer lists
-      b.point_list = b.point_list.narrow(0, 0, R);
-      if (train) b.hit_blocks = b.hit_blocks.narrow(0, 0, R);
-    }
+    const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
+      check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii),
+                                 masks, to.room, i64(b.ranges), scratch.at<void>(bins), bins_bytes, to.space.data_ptr(),
+                                 to.space.numel(), stream),
+            "GS_prepare");
+    }, blend_maps);
+    b.point_list = empty({in.count}, like, at::kInt);
+    check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks,
+                            in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes,
+                            data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
+          "GS_prepare");
   } else {
     blend_maps();
     b.point_list = empty({0}, like, at::kInt);
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
-    blend_lists();
   }
+  if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);
+  check(fsgs_gaussian_view_forward((int) P, W, H, E, f32(v.means2D), f32(b.conic_opacity), colors,
+                                   E ? f32(*v.extras) : nullptr, i32(b.point_list), i64(b.ranges),
+                                   i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
+                                   i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity),
+                                   E ? f32(b.extras) : nullptr, i32(b.n_contrib), (uint32_t*) i32(b.hit_blocks), stream),
+        blend);
   return b;
 }
 

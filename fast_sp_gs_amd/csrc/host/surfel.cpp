@@ -89,22 +89,6 @@ Buffers forward_view(const SurfelView& v, bool train) {
       b.surf_normal = empty({3, H, W}, like);
     }
   };
-  auto blend_lists = [&] {
-    if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);
-    const bool composite = v.epilogue && has(v.background);
-    check(fsgs_gs_2d_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, f32(b.normal_opacity),
-                                    f32(b.trans_mat), i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
-                                    i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
-                                    i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
-                                    f32(b.flow), i32(b.n_contrib), records, (uint32_t*) i32(b.hit_blocks), v.depth_ratio,
-                                    f32(v.Tw2v), composite ? f32(*v.background) : nullptr, f32(b.normals), f32(b.depths),
-                                    f32(b.surf_depth), f32(b.distortion), stream),
-          blend);
-    if (v.epilogue)
-      check(fsgs_gs_2d_view_surf_normal(W, H, f32(v.Tw2v), f32(v.Tv2c), f32(b.surf_depth), f32(b.opacity), f32(b.surf_normal),
-                                        stream),
-            "gs_2d_epilogue_forward");
-  };
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
@@ -118,47 +102,44 @@ Buffers forward_view(const SurfelView& v, bool train) {
                                      train ? b.keep.at<int32_t>(s.offsets) : nullptr, counters.data(), records, masks,
                                      stream),
           what);
-    auto tally = [&](uint64_t* slots, int32_t* regions, int64_t* word, int64_t positions) {
-      check(fsgs_gs_view_tally((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, slots, regions, word, positions,
-                               i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
-            "GS_prepare");
-    };
-    // fill the lists and blend them
-    auto second_half = [&](int64_t positions) {
-      b.point_list = empty({positions}, like, at::kInt);
-      const size_t fill_bytes = fsgs_gs_view_fill_workspace_bytes(positions);
-      const Tensor fill = empty({(int64_t) fill_bytes}, like, at::kByte);
-      check(fsgs_gs_view_fill((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks, positions,
-                              i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes, fill.data_ptr(), fill_bytes,
-                              stream),
-            "GS_prepare");
-      blend_lists();
-    };
-    const int64_t guess = positions_to_guess(P, T);
-    tally(counters.data(), train ? b.keep.at<int32_t>(s.regions) : nullptr, count, guess > 0 ? guess : INT64_MAX);
+    check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
+                             train ? b.keep.at<int32_t>(s.regions) : nullptr, count, i64(b.ranges), scratch.at<void>(bins),
+                             bins_bytes, stream),
+          "GS_prepare");
     PendingCount pending(count, stream);
     counters.give_back();
-    blend_maps();  // what does not depend on the count is allocated while the device gets there
-    const bool guessed = guess > 0 && !pending.arrived();
-    if (guessed) second_half(guess);
-    s.R = pending.wait("GS_prepare");
-    if (guess > 0 && s.R > guess) {  // the lists have been left empty
-      tally(nullptr, nullptr, nullptr, s.R);
-      second_half(s.R);
-    } else if (!guessed) {
-      second_half(s.R);
-    } else {
-      at::AutoDispatchBelowADInplaceOrView plain;  // what the view hands out are no views of the longer lists
-      b.point_list = b.point_list.narrow(0, 0, s.R);
-      if (train) b.hit_blocks = b.hit_blocks.narrow(0, 0, s.R);
-    }
+    const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
+      check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii),
+                                 masks, to.room, i64(b.ranges), scratch.at<void>(bins), bins_bytes, to.space.data_ptr(),
+                                 to.space.numel(), stream),
+            "GS_prepare");
+    }, blend_maps);
+    s.R = in.count;
+    b.point_list = empty({in.count}, like, at::kInt);
+    check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks,
+                            in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes,
+                            data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
+          "GS_prepare");
   } else {
     blend_maps();
     b.point_list = empty({0}, like, at::kInt);
     check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
           "GS_prepare");
-    blend_lists();
   }
+  if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);
+  const bool composite = v.epilogue && has(v.background);
+  check(fsgs_gs_2d_view_forward((int) P, W, H, v.near_n, v.far_n, f32(v.means2D), colors, f32(b.normal_opacity),
+                                  f32(b.trans_mat), i32(b.point_list), i64(b.ranges), f32(opt(v.trans_mat_t2)),
+                                  i32(opt(v.accum_max_count)), f32(opt(v.accum_weights_p)),
+                                  i32(opt(v.accum_weights_count)), f32(b.image), f32(b.opacity), f32(b.extras),
+                                  f32(b.flow), i32(b.n_contrib), records, (uint32_t*) i32(b.hit_blocks), v.depth_ratio,
+                                  f32(v.Tw2v), composite ? f32(*v.background) : nullptr, f32(b.normals), f32(b.depths),
+                                  f32(b.surf_depth), f32(b.distortion), stream),
+        blend);
+  if (v.epilogue)
+    check(fsgs_gs_2d_view_surf_normal(W, H, f32(v.Tw2v), f32(v.Tv2c), f32(b.surf_depth), f32(b.opacity), f32(b.surf_normal),
+                                      stream),
+          "gs_2d_epilogue_forward");
   return b;
 }
 

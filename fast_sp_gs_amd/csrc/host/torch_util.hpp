@@ -134,14 +134,49 @@ class PendingCount {
   bool known_ = false;
 };
 
-// List positions to queue a view's second half for before its count is known; 0: wait for the count. A surfel has at most one
-// position per tile, and on average fewer than 16 unless the surfels are large (2 to 8 in ordinary scenes); beyond 2^18 surfels a
-// view keeps the device busy for longer than the host needs for the rest of its launches.
-// With the wait in front of them (the device runs dry until the host has queued the rest): 10k surfels 256x256 60.5 -> 54.5 us, 25k
-// Gaussians 639x361 56 -> 53, a dynamic frame of 50k 128.5 -> 125.5, a dynamic iteration of 200k 735 -> 710.
-inline int64_t positions_to_guess(int64_t P, int64_t T) {
+// Room for the instances of a view whose count is not known yet; 0: wait for the count. A surfel has at most one instance per tile,
+// and on average fewer than 16 unless the surfels are large (2 to 8 in ordinary scenes); beyond 2^18 surfels the device is busy
+// with the counting for longer than the host needs to wait and go on.
+inline int64_t instances_to_guess(int64_t P, int64_t T) {
   if (P > (1 << 18) || T > (1 << 14)) return 0;
   return std::min(P * T, std::max<int64_t>(16 * P, 1 << 16));
+}
+
+// A view's instances, scattered into its tiles' segments, and their number.
+struct Instances {
+  Tensor space;      // fsgs_gs_view_lists_workspace_bytes(room) bytes
+  int64_t room = 0;  // for that many
+  int64_t count = 0;
+};
+
+// The scatter is queued for a guess, so that the device has something to do until the host has seen the count and launched the
+// sort; only what lives no longer than the view is sized by the guess. A guess that was too small, or that memory does not suffice
+// for, costs an empty launch, and the scatter is queued again for the count.
+// Six processes each in turn, with the wait in front of the scatter -> so, fastest and median us: view of 10k surfels 256x256 50.7 and
+// 57.4 -> 49.4 and 55.7, of 25k Gaussians 639x361 51.1 and 55.4 -> 50.4 and 54.6; dynamic frame of 50k and iteration of 200k equal
+// within what the runs of one side differ. Counts above the guess (5000 surfels of 43 pixels 800x800, 1.7M instances): 426, 442
+// with the wait and a larger workspace.
+// `scatter(instances)` queues the kernel, `meanwhile()` allocates what does not depend on the count (before
+// the guess, which can do without).
+template <typename Scatter, typename Meanwhile>
+Instances scatter_instances(const char* what, PendingCount& pending, int64_t guess, const Tensor& like, Scatter scatter,
+                            Meanwhile meanwhile) {
+  Instances in;
+  auto queue = [&](int64_t room) {
+    in.space = empty({(int64_t) fsgs_gs_view_lists_workspace_bytes(room)}, like, at::kByte);
+    in.room  = room;
+    scatter(in);
+  };
+  meanwhile();
+  if (guess > 0 && !pending.arrived()) {
+    try {
+      queue(guess);
+    } catch (const c10::OutOfMemoryError&) {
+    }
+  }
+  in.count = pending.wait(what);
+  if (in.count > in.room) queue(in.count);
+  return in;
 }
 
 // 64 zeroed counters on the tensor's device for one view on its current stream. They go back to a list of that stream

@@ -80,8 +80,6 @@ struct SlotPublish {
   unsigned long long* counters = nullptr;  // [64], zeroed again
   int32_t* region = nullptr;               // [64] or nullptr
   int64_t* host_count = nullptr;           // pinned host memory
-  int64_t capacity = 0;                    // of the lists, and where it is noted that the instances exceed it
-  int* exceeds = nullptr;
 };
 
 // One wavefront.
@@ -96,7 +94,6 @@ __device__ __forceinline__ void publish_slot_regions(const SlotPublish& p) {
   }
   if (p.region) p.region[lane] = (int32_t) (inc - mine);
   p.counters[lane] = 0ull;
-  if (lane == kWave - 1 && p.exceeds) *p.exceeds = (int64_t) inc > p.capacity;
   if (lane == kWave - 1) __hip_atomic_store(p.host_count, (int64_t) inc, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

@@ -140,37 +140,29 @@ int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const float* means2
                                         int32_t* point_list, int64_t* sorted_keys_out, void* bins, size_t bins_bytes,
                                         void* workspace, size_t workspace_bytes, void* stream);
 
-/* The counting part of the binning (as fsgs_gs_prepare_count, or _culled with keep_masks) for a view preprocessed by
- * fsgs_gs_*_view_preprocess; P > 0. Its first block writes slot_regions[64] (optional), zeroes slot_counters and stores
+/* The binning of a view preprocessed by fsgs_gs_*_view_preprocess, in the parts that a view runs it in; P > 0. For surfels and 3D
+ * Gaussians (inverse_m and opacities nullptr, keep_masks optional) and for the "fast" surfels (tiles that pass the corner test; all
+ * three given).
+ * fsgs_gs_view_count: per-tile counts. Its first block writes slot_regions[64] (optional), zeroes slot_counters and stores
  * the instance count to num_rendered_host (pinned memory, set to -1 here); fsgs_gs_view_wait returns once it is there.
- * fsgs_gs_prepare_fill_counted(_culled) follows. */
-int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const int32_t* radii, const uint32_t* keep_masks,
-                       uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges,
-                       void* bins, size_t bins_bytes, void* stream);
-int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream);
-/* Both parts as the views run them, for surfels and 3D Gaussians (inverse_m and opacities nullptr; keep_masks optional) and for the
- * "fast" surfels (all three given). `ranges` is complete once fsgs_gs_view_fill has run, and not before; point_list[capacity]
- * behind the kept instances is not written. `capacity` (the same for both) is the instance count, or a guess made before it is
- * known, so that the fill and the blend can be queued without waiting: if there are more instances all ranges are left empty, and
- * both are called again with the count, the tally without slot_counters, slot_regions and num_rendered_host (they were
- * served by the first). */
-size_t fsgs_gs_view_fill_workspace_bytes(int64_t capacity);
-int fsgs_gs_view_tally(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
+ * fsgs_gs_view_scatter puts the instances into `workspace` (fsgs_gs_view_lists_workspace_bytes(capacity) bytes), which has room for
+ * `capacity` of them: the count, or a guess made before it is known, so that the device is busy while the host waits. If there
+ * are more instances than that it writes nothing, and is called again with the count.
+ * fsgs_gs_view_sort takes the workspace and the capacity of the last scatter and the count R <= capacity, and writes point_list[R]
+ * (unlike fsgs_gs_2d_fast_prepare_fill no padding entries) and what is still missing of `ranges`; R == 0: ranges only. The blend
+ * needs nothing but the lists, so point_list and what is sized like it can be allocated for the count. */
+int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
                        const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters, int32_t* slot_regions,
-                       int64_t* num_rendered_host, int64_t capacity, int64_t* ranges, void* bins, size_t bins_bytes, void* stream);
-int fsgs_gs_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
-                      const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity, int64_t* ranges,
-                      int32_t* point_list, void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes, void* stream);
-/* The two parts for the "fast" surfels (tiles that pass the corner test; keep_masks of the preprocess). Unlike
- * fsgs_gs_2d_fast_prepare_fill no padding entries are written behind the kept instances. */
-int fsgs_gs_2d_fast_view_count(int P, int W, int H, const float* means2D, const float* inverse_m, const float* opacities,
-                               const int32_t* radii, const uint32_t* keep_masks, uint64_t* slot_counters,
-                               int32_t* slot_regions, int64_t* num_rendered_host, int64_t* ranges, void* bins,
-                               size_t bins_bytes, void* stream);
-int fsgs_gs_2d_fast_view_fill(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
-                              const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R,
-                              int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
-                              size_t workspace_bytes, void* stream);
+                       int64_t* num_rendered_host, int64_t* ranges, void* bins, size_t bins_bytes, void* stream);
+int fsgs_gs_view_wait(const int64_t* num_rendered_host, void* stream);
+size_t fsgs_gs_view_lists_workspace_bytes(int64_t capacity);
+int fsgs_gs_view_scatter(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                         const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t capacity,
+                         int64_t* ranges, void* bins, size_t bins_bytes, void* workspace, size_t workspace_bytes, void* stream);
+int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const float* inverse_m, const float* depths,
+                      const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R, int64_t capacity,
+                      int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
+                      size_t workspace_bytes, void* stream);
 
 /* ---- per-tile alpha blend ------------------------------------------------------------------------------------- */
 

@@ -1,6 +1,7 @@
-"""Views are queued for a guessed number of list positions before their instance count is known (positions_to_guess in
+"""A view's instances are scattered for a guessed count before the count is known (instances_to_guess in
 csrc/host/torch_util.hpp: 16 per surfel, 65 536 at least, one per surfel and tile at most). Scenes with more instances than that
-take their second half again: the same maps, lists, counts and gradients as by the operators, which wait for the count."""
+are scattered again: the same maps, lists, counts and gradients as by the operators, which wait for the count. Nothing that a
+view hands out or keeps is sized by the guess."""
 import pytest
 import torch
 
@@ -33,3 +34,89 @@ def test_more_instances_than_guessed(which, P, W, H, more, device, monkeypatch):
         views.test_fast_surfel_view_equals_operators(P, W, H, 'sh', device)
     else:
         views.test_gaussian_view_equals_operators(P, W, H, 'sh', device)
+
+
+def _view(s, cam):
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    with torch.no_grad():
+        return GS_2D_render(s.means3D, s.scales, s.rotations, s.opacities, (cam.W, cam.H), cam.Tw2v, cam.Tv2c,
+                            campos=cam.campos, sh_degree=3, sh_features=s.shs)
+
+
+def _time(f):
+    """Microseconds a call: the best of five times 10."""
+    best = float('inf')
+    for _ in range(6):  # the first one warms up
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(10):
+            f()
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) * 1000 / 10)
+    return best
+
+
+@pytest.mark.parametrize('P,W,H', [(900, 480, 288), (5000, 200, 200), (1, 480, 288)])
+@pytest.mark.parametrize('train', [False, True])
+def test_lists_are_no_longer_than_the_count(P, W, H, train, device):
+    """Kept, or saved to a file, a list takes the memory of its entries."""
+    from fast_sp_gs_amd.renderer import GS_2D_render
+    s, cam, _ = _large_surfels(P, W, H, P)
+    s, cam = s.to(device), cam.to(device)
+    out = GS_2D_render(s.means3D.requires_grad_(train), s.scales, s.rotations, s.opacities, (W, H), cam.Tw2v, cam.Tv2c,
+                       campos=cam.campos, sh_degree=3, sh_features=s.shs)
+    point_list = out['buffer'].point_list
+    assert point_list.untyped_storage().nbytes() == point_list.nbytes == 4 * out['buffer'].R
+
+
+def test_exceeded_guess_costs_an_empty_launch(device):
+    """The same 900 large surfels with as many small ones behind the camera as raise the guess above the count: without them the
+    counting, and all behind it, ran twice (1.5 times the time)."""
+    s, cam, g = _large_surfels(900, 480, 288, 901)
+    more = type(s)(*(torch.cat([t, t[torch.randint(900, (30_000,), generator=g)]])
+                     for t in (s.means3D, s.scales, s.rotations, s.opacities, s.shs)), s.sh_degree)
+    more.means3D[900:, 2] = 50.0
+    s, more, cam = s.to(device), more.to(device), cam.to(device)
+    a, b = _view(s, cam), _view(more, cam)
+    assert 65_536 < a['buffer'].R <= 16 * 30_900 and a['buffer'].R == b['buffer'].R and torch.equal(a['images'], b['images'])
+    assert _time(lambda: _view(s, cam)) < 1.25 * _time(lambda: _view(more, cam))
+
+
+def test_guess_that_memory_does_not_suffice_for(device):
+    """A view for whose guess there is no memory waits for its count: it needs no more than that."""
+    g = torch.Generator().manual_seed(3)
+    from fast_sp_gs_amd import scenes
+    s = scenes._surfels(g, 262_144, 'cube', -9.0, 0.1, -1.0, 1.0).to(device)
+    cam = scenes.pinhole(256, 256, 50.0, torch.tensor([0.0, 0.0, 4.0])).to(device)
+    want, total = _view(s, cam)['images'], torch.cuda.get_device_properties(device).total_memory
+    busy = torch.ones(2 ** 28, device=device)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    base, tried, filled = torch.cuda.memory_reserved(), False, []
+    try:
+        torch.cuda.set_per_process_memory_fraction(base / total)
+        for size in (2 ** 28, 2 ** 26, 2 ** 24, 2 ** 22, 2 ** 20 + 1):  # what other tests have left free between their tensors
+            try:
+                while True:
+                    filled.append(torch.empty(size, dtype=torch.uint8, device=device))
+            except torch.OutOfMemoryError:
+                pass
+        for room in range(160, 0, -4):  # MB
+            torch.cuda.set_per_process_memory_fraction((base + room * 2 ** 20) / total)
+            failed = torch.cuda.memory_stats().get('num_ooms', 0)
+            for _ in range(30):  # some milliseconds: the count is not there before the guess
+                busy.mul_(1.0)
+            try:
+                got = _view(s, cam)['images']
+            except torch.OutOfMemoryError:
+                break
+            finally:
+                torch.cuda.synchronize()
+                torch.cuda.empty_cache()
+            assert torch.equal(got, want)
+            tried |= torch.cuda.memory_stats().get('num_ooms', 0) > failed
+            del got
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert tried
