@@ -57,13 +57,14 @@ def _time(f):
     return best
 
 
-@pytest.mark.parametrize('P,W,H', [(900, 480, 288), (5000, 200, 200), (1, 480, 288)])
+@pytest.mark.parametrize('P,W,H,log_scale', [(20_000, 256, 256, -4.6), (900, 480, 288, 0.3), (1, 480, 288, -3.0)])
 @pytest.mark.parametrize('train', [False, True])
-def test_lists_are_no_longer_than_the_count(P, W, H, train, device):
+def test_lists_are_no_longer_than_the_count(P, W, H, log_scale, train, device):
     """Kept, or saved to a file, a list takes the memory of its entries."""
+    from fast_sp_gs_amd import scenes
     from fast_sp_gs_amd.renderer import GS_2D_render
-    s, cam, _ = _large_surfels(P, W, H, P)
-    s, cam = s.to(device), cam.to(device)
+    s = scenes._surfels(torch.Generator().manual_seed(P), P, 'cube', log_scale, 0.3, -1.0, 1.0).to(device)
+    cam = scenes.pinhole(W, H, 50.0, torch.tensor([0.3, 0.2, 4.0])).to(device)
     out = GS_2D_render(s.means3D.requires_grad_(train), s.scales, s.rotations, s.opacities, (W, H), cam.Tw2v, cam.Tv2c,
                        campos=cam.campos, sh_degree=3, sh_features=s.shs)
     point_list = out['buffer'].point_list
