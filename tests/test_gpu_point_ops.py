@@ -355,6 +355,25 @@ def test_knn_clusters_keep_to_the_lists(device):
         assert _knn_time(pts.to(device), ctrl.to(device), K) < 1.6 * loose
 
 
+# 2^22 elements, from where gradients and moments are streamed, and just below; rows that a 16-byte piece straddles
+@pytest.mark.parametrize('N', [2 ** 20 // 13 - 1, 2 ** 20 // 13 + 1, 2 ** 17])
+def test_multi_tensor_adam_around_the_streaming_limit(N, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N)
+    shapes = [(N, 3), (N, 15, 3), (N, 4)]  # 52 elements a row
+    assert (52 * N >= 2 ** 22) == (N > 2 ** 20 // 13)
+    rand = lambda s: torch.randn(s, generator=g).to(device)
+    params, grads, vis = [rand(s) for s in shapes], [rand(s) for s in shapes], (torch.rand(N, generator=g) < 0.6).to(device)
+    moments = [(rand(s) * 0.1, rand(s).square()) for s in shapes]
+    p1, m1, v1 = [p.clone() for p in params], [m.clone() for m, _ in moments], [v.clone() for _, v in moments]
+    get_C_function('AdamMasksedUpdatedMulti')(p1, grads, m1, v1, vis, [1e-2, 1e-3, 1e-4], 0.9, 0.999, [1e-15] * 3, N)
+    for k, s in enumerate(shapes):
+        p2, (m2, v2) = params[k], moments[k]
+        get_C_function('AdamMasksedUpdated')(p2, grads[k], m2, v2, vis, [1e-2, 1e-3, 1e-4][k], 0.9, 0.999, 1e-15, N,
+                                             p2.numel() // N)
+        assert torch.equal(p1[k], p2) and torch.equal(m1[k], m2) and torch.equal(v1[k], v2)
+
+
 LBS_CASES = [  # (warp method with a local rotation | None without one, weight method)
     (None, 'weighted_kernel'),   # the reference's default configuration: translations only, kernel weights
     (None, 'dist'), ('LBS', 'dist'), ('LBS_c', 'dist'), ('LBS_c', 'weighted_kernel'), ('LBS', 'kernel'),
