@@ -19,9 +19,10 @@
 //      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
 // short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.22 ms a call this way (mean of 30 inputs)
-// (traced: lists 0.033, queries 0.201; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
-// vector issue (2080 instructions per 64 queries); the LDS and the address path of the vector memory are busy half the time.
-// 200 000 x 512, K = 4: 57 -> 23 us, 50 000 x 512, K = 3: 37 -> 18 us, 5 000 x 512, K = 4: 36 -> 10 us.
+// (traced: lists 0.037, queries 0.200; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
+// vector issue (2120 instructions per 64 queries, 0.88 of the issue slots); the address path of the vector memory is busy three
+// quarters of the time, the LDS half of it.
+// 200 000 x 512, K = 4: 57 -> 26 us, 50 000 x 512, K = 3: 37 -> 19 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -61,10 +62,10 @@ enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 
 // Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
 // alone) and N * M / 4e12 s when they fill the chip; a wavefront per query 0.8 (M = 512) to 2.0 ns (M = 2048) a query;
-// building the lists 10 us (G = 16, 512 control points) to 48 us (G = 32, 2048). With G = 16 the lists of more than 640
+// building the lists 11 us (G = 16, 512 control points) to 37 us (G = 32, 2048). With G = 16 the lists of more than 640
 // control points outgrow their 128 entries; below that the finer grid pays from a million queries on. Behind the limits
-// the walk over all pairs takes over at its own price: 3M queries, K = 4: 232 us for 2560 control points, 1597 for 2561; 2048
-// control points, K = 8: 313 us, K = 9: 5908. 200 000 queries, K = 4: 90 and 204 us.
+// the walk over all pairs takes over at its own price: 3M queries, K = 4: 164 us for 2560 control points, 1481 for 2561; 2048
+// control points, K = 8: 214 us, K = 9: 5897. 200 000 queries, K = 4: 60 and 187 us.
 Scheme knn_scheme(int N, int M, int D, int K) {
   if (D != 3 || K > kMaxK || M > kMaxPoints || M < 96) return kAllPairs;
   if (N <= kFewQueries) return kAlone;

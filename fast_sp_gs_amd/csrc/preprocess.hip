@@ -337,6 +337,8 @@ constexpr int kSumStride  = 19;
 // adds the present ones from LDS, a component per lane. Four positions a trip, a surfel near the camera with hundreds of tiles
 // kept its wavefront, and with it the launch, for a hundred trips. Kernel, us: 300k surfels 800x800 64 -> 51, 3M 1352x1014
 // 393 -> 370, 1M 1352x900 182 -> 131, 30k 1000x1000 33 -> 16.5, 10k 256x256 11.4 -> 11.0; six positions in flight 50, 367 and 11.6.
+// 1000 surfels of 12 / 25 / 40 pixels 800x800 70 -> 51, 237 -> 150, 548 -> 287; 900 that all cover half of 480x288, in 15 wavefronts, 311
+// -> 331: the wavefront drains between spans.
 constexpr int kSumChunk = kWave, kSumScratch = kSumChunk * kGradFloats;
 constexpr int kSumFloats = kWave * kSumStride + kSumScratch;  // of a wavefront
 
