@@ -105,8 +105,8 @@ def test_blocking_entry_points_match_the_operator(device):
 def test_blend_schedule_is_a_permutation_longest_first(device, gx, gy, kind):
     """The blockIdx -> tile table of the blend kernels (fsgs_debug_tile_order): every tile exactly once, for grids from one
     tile to the 65 536-tile limit, with empty and equal lists; inside each of the 8 interleaved position classes (one
-    XCD each) the list lengths fall from round to round of 32 positions (inside a round the tiles are dealt by the load of
-    the compute units, in any order), up to the resolution of the length buckets (sixteen per octave)."""
+    XCD each) the list lengths fall from round to round of 32 positions (inside a round the tiles may come in
+    any order), up to the resolution of the length buckets (sixteen per octave)."""
     from fast_sp_gs_amd import lib as L
     T = gx * gy
     rng = np.random.default_rng(gx * 1000 + gy)

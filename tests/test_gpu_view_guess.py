@@ -121,3 +121,45 @@ def test_guess_that_memory_does_not_suffice_for(device):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert tried
+
+
+# grids whose ranges one block forms, several do, and beyond the tiles that LDS counters serve
+@pytest.mark.parametrize('gx,gy,P', [(30, 18, 3000), (64, 64, 3000), (17, 2410, 300)])
+def test_scatter_without_room_writes_nothing(gx, gy, P, device):
+    """The C entries with a guess that is too small: nothing is written, and the scatter for the count leaves the lists of
+    `GS_prepare`."""
+    from fast_sp_gs_amd import lib as L, scenes
+    from fast_sp_gs_amd._C import get_C_function
+    lib, stream = L.load(), L.current_stream()
+    W, H = 16 * gx - 3, 16 * gy - 5
+    scene, _ = scenes.config0(P=P, size=max(W, H), seed=4)
+    scene.scales = scene.scales * 20.0
+    s, cam = scene.to(device), scenes.pinhole(W, H, 50.0, torch.tensor([0.0, 0.0, 4.0])).to(device)
+    print(f'[scatter without room] {gx}x{gy} tiles, P={P}', flush=True)
+    m2, _, _, _, depths, radii, touched = get_C_function('gs_2d_preprocess_forward')(
+        W, H, 3, False, s.means3D, s.scales, s.rotations, s.opacities, s.shs, None, cam.Tw2v, cam.Tv2c, cam.campos, None, None, None)
+    want_ranges, want_list = get_C_function('GS_prepare')(W, H, m2, depths, radii, touched, False)[:2]
+    R = int(touched.sum())
+    assert R == want_list.numel() > P
+    counters = torch.zeros(64, dtype=torch.int64, device=device)
+    counters[5], counters[63] = R - 7, 7
+    word = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    ranges = torch.full((gx * gy, 2), -1, dtype=torch.int64, device=device)
+    bins = torch.full((lib.fsgs_gs_prepare_bins_bytes(P, W, H),), 0xff, dtype=torch.uint8, device=device)
+    L.check(lib.fsgs_gs_view_count(P, W, H, L.ptr(m2), None, None, L.ptr(radii), None, L.ptr(counters), None, word.data_ptr(),
+                                   L.ptr(ranges), L.ptr(bins), bins.numel(), stream), 'count')
+    L.check(lib.fsgs_gs_view_wait(word.data_ptr(), stream), 'wait')
+    assert int(word[0]) == R and not counters.any()
+    point_list = torch.full((R,), -5, dtype=torch.int32, device=device)
+    for room in (1, R // 2, R - 1, R):
+        size = lib.fsgs_gs_view_lists_workspace_bytes(room)
+        space = torch.full((size + 4096,), 0xab, dtype=torch.uint8, device=device)
+        args = (P, W, H, L.ptr(m2), None, L.ptr(depths), None, L.ptr(radii), None)
+        L.check(lib.fsgs_gs_view_scatter(*args, room, L.ptr(ranges), L.ptr(bins), bins.numel(), L.ptr(space), size, stream), 'scatter')
+        torch.cuda.synchronize()
+        assert (room == R and gx * gy <= 40_960) != bool((space == 0xab).all()) and bool((space[size:] == 0xab).all())
+        rc = lib.fsgs_gs_view_sort(*args, R, room, L.ptr(ranges), L.ptr(point_list), L.ptr(bins), bins.numel(), L.ptr(space),
+                                   size, stream)
+        assert (rc == 0) == (room == R)
+    torch.cuda.synchronize()
+    assert torch.equal(ranges, want_ranges) and torch.equal(point_list, want_list) and bool((space[size:] == 0xab).all())
