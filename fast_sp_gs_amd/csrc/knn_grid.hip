@@ -6,10 +6,10 @@
 // ruled out for a whole cell of a grid over the control points at once:
 //   1. knn_cell_lists_kernel: the cells of a G x G x G grid. U = a bound on the K-th nearest distance of ANY point of the
 //      cell (the K-th smallest of 64 far-corner distances); the cell's list holds the control points whose nearest-corner
-//      distance does not exceed U, in ascending index order. A block builds the list of one of 8 x 8 x 8 coarse cells and
-//      refines it for the (G / 8)^3 cells inside.
-//   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 35 entries for 2048 control
-//      points and G = 32). The walk only keeps the K + 1 smallest keys -- the distance in 2^-20 parts of
+//      distance does not exceed U, with many queries in the order of the distances from the cell's centre (kOrderFrom), else of the
+//      indices. A block builds the list of one of 8 x 8 x 8 coarse cells and refines it for the (G / 8)^3 cells inside.
+//   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 38 entries for 2048 control
+//      points and G = 32; in order, about 20 of them: what follows is farther from the centre than the K-th neighbour can be). The walk only keeps the K + 1 smallest keys -- the distance in 2^-20 parts of
 //      the cell's bound, then the control point's number -- in a sorted register list, one v_med3_u32 per slot; the K exact
 //      distances are formed again afterwards. Queries whose keys cannot separate two neighbours (distances in the same part)
 //      walk again with parts of another kind if that can help (kCoarseParts); the others of these, those
@@ -18,11 +18,12 @@
 //      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
 //      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.22 ms a call this way (mean of 30 inputs)
-// (traced: lists 0.037, queries 0.200; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by
-// vector issue (2120 instructions per 64 queries, 0.88 of the issue slots); the address path of the vector memory is busy three
-// quarters of the time, the LDS half of it.
-// 200 000 x 512, K = 4: 57 -> 26 us, 50 000 x 512, K = 3: 37 -> 19 us, 5 000 x 512, K = 4: 36 -> 10 us.
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.17 ms a call this way
+// (traced: lists 0.047, queries 0.118; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by vector issue (1090
+// instructions per 64 queries, 0.82 of the issue slots). With lists in index order and a row of results stored by each lane for itself
+// it took 0.202 ms and 2180 instructions; in order alone 0.169, its memory path busy with stores of 16 bytes each; results through LDS in
+// runs of 512 and 1024 bytes 0.152, and past the caches, which then keep the lists (8 MB), 0.118.
+// 200 000 x 512, K = 4: 57 -> 24 us, 50 000 x 512, K = 3: 37 -> 19 us, 5 000 x 512, K = 4: 36 -> 10 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -48,10 +49,10 @@ static_assert(kMaxPoints + 8 <= (int) kNumberBits, "the numbers behind the last 
 // 267 / 2860 / 3150 with coarse parts only, 214 / 263 / 306 with the second walk, 204 / 209 / 207 so; a key of the float's upper
 // 25 bits and the list position: 225 / 220 / 221.
 constexpr uint32_t kCoarseParts = (1u << 13) * (kNumberBits + 1);
-constexpr uint32_t kCrowdedBit = 0x10000;  // of a cell's length
+constexpr uint32_t kCrowdedBit = 0x100;  // of a cell's length
 constexpr int kCrowded = 8, kMostLanes = 16;
 constexpr int kBuildThreads = 512, kQueryThreads = 512;
-constexpr uint32_t kLongList = 0xffff;
+constexpr uint32_t kLongList = 0xff;
 constexpr int kFewQueries = 16384;
 
 // Lists that the wavefront takes one by one once no more than so many of its lanes have candidates left: a lane's eight more cost
@@ -65,7 +66,7 @@ enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 // building the lists 11 us (G = 16, 512 control points) to 37 us (G = 32, 2048). With G = 16 the lists of more than 640
 // control points outgrow their 128 entries; below that the finer grid pays from a million queries on. Behind the limits
 // the walk over all pairs takes over at its own price: 3M queries, K = 4: 164 us for 2560 control points, 1481 for 2561; 2048
-// control points, K = 8: 214 us, K = 9: 5897. 200 000 queries, K = 4: 60 and 187 us.
+// control points, K = 8: 171 us, K = 9: 5897. 200 000 queries, K = 4: 60 and 187 us.
 Scheme knn_scheme(int N, int M, int D, int K) {
   if (D != 3 || K > kMaxK || M > kMaxPoints || M < 96) return kAllPairs;
   if (N <= kFewQueries) return kAlone;
@@ -73,10 +74,22 @@ Scheme knn_scheme(int N, int M, int D, int K) {
   return M > 640 || N >= 1000000 ? kGrid32 : kGrid16;
 }
 
-// A cell: how many candidates its list holds (or kLongList) and kCrowdedBit, and what takes a squared distance to 2^32 at the cell's bound.
-struct Cell {
-  uint32_t length;
+// Whether the lists are put in the order of the distances from their cell's centre, so that a query's walk is over after half of its
+// list (below). It costs 10 us with G = 32, whatever the number of queries, and saves 9 ns a thousand queries at K = 8, 1 at K = 1; with G = 16 it
+// costs less than 1 us. M = 2048, us in index order -> in this one: K = 8, N = 500 000 73.6 -> 78.6, 1M 93.4 -> 89.5, 3M 193 -> 167; K = 4, 500 000
+// 63.1 -> 69.5, 1.5M 86.6 -> 85.0, 3M 145 -> 132; K = 1, 3M 111.5 -> 107.9, M = 1024 83.7 -> 86.8. M = 600 (G = 16), 200 000: K = 8 47.7 -> 45.1, K = 1
+// 34.3 -> 33.3; M = 200, 50 000: K = 4 24.2 -> 24.2, K = 1 21.1 -> 22.1.
+template <int kK, int kG>
+constexpr int64_t kOrderFrom = kG == 16 ? (kK >= 3 ? 0 : 400000) : kK == 1 ? INT64_MAX : 10000000 / (kK + 2);  // queries
+
+// A cell. `length`: how many candidates its list holds (or kLongList) and kCrowdedBit, and the first bound; `scale`: what takes a squared
+// distance to 2^32 at the cell's bound. Where the list is in the order of the distances from the cell's centre, byte g - 1 of the bounds
+// is a lower bound, in cell_step's, on the distances from the 8 g-th entry on; else they are 0. (The last one counts for what is behind it, too.)
+constexpr int kBounds = 10;
+struct __attribute__((aligned(16))) Cell {
+  uint32_t length;  // bounds 0 and 1 in the upper half
   float scale;
+  uint32_t bounds[2];
 };
 struct GridLayout {
   int G;
@@ -137,6 +150,11 @@ __device__ __forceinline__ float box_near2(const float4& p, const float* lo, con
 // near the underflow threshold, by an absolute amount), so that a point left out is strictly farther in single precision
 // than K points of the list, whatever the query.
 __device__ __forceinline__ float widened(float bound2) { return bound2 * 1.00002f + 1e-36f; }
+
+// The unit of a cell's bounds: no entry of its list is farther from its centre than twice the root of 2^32 / scale.
+__device__ __forceinline__ float cell_step(float scale) { return __builtin_amdgcn_rsqf(scale) * (2.0f * 65536.0f / 255.0f); }
+__device__ __forceinline__ float cell_centre(float lo, float hi) { return 0.5f * (lo + hi); }
+__device__ __forceinline__ float centre_distance(float x, float y, float z) { return __builtin_amdgcn_sqrtf(fmaf(x, x, fmaf(y, y, z * z))); }
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
   return (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) mask, 0u));
@@ -313,12 +331,61 @@ __device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* s
   return n;
 }
 
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, kCtrl, 0xf, 0xf, true);
+}
+// The lane's value across the 16-lane (32-lane) rows beside each other: lane l ^ 16 (l ^ 32).
+__device__ __forceinline__ uint32_t across16(uint32_t v, bool odd) {
+  uint32_t a = v, b = v;  // after the swap: rows 0 0 2 2, and 1 1 3 3 (s_nop: the wait states that the compiler does not count in here)
+  asm("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return odd ? a : b;
+}
+__device__ __forceinline__ uint32_t across32(uint32_t v, bool odd) {
+  uint32_t a = v, b = v;
+  asm("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return odd ? a : b;
+}
+// Bitonic networks over the 64 lanes' values, every merge begun with the mirror image so that all of it ascends.
+struct WaveSort {
+  bool b1, b2, b4, b8, b16, b32;
+  __device__ __forceinline__ WaveSort() {
+    const int lane = __lane_id();
+    b1 = lane & 1, b2 = lane & 2, b4 = lane & 4, b8 = lane & 8, b16 = lane & 16, b32 = lane & 32;
+  }
+  static constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kXor3 = 0x1b, kXor7 = 0x141, kXor8 = 0x128, kXor15 = 0x140;  // quad_perm, mirrors, row_ror:8
+  static __device__ __forceinline__ uint32_t xor4(uint32_t x) { return dpp_u32<kXor3>(dpp_u32<kXor7>(x)); }
+  static __device__ __forceinline__ void keep(uint32_t& v, uint32_t other, bool upper) {
+    const uint32_t lo = min(v, other), hi = max(v, other);
+    v = upper ? hi : lo;
+  }
+  __device__ __forceinline__ uint32_t mirrored(uint32_t v) const { return dpp_u32<kXor15>(across16(across32(v, b32), b16)); }
+  __device__ __forceinline__ void below4(uint32_t& v) const { keep(v, dpp_u32<kXor2>(v), b2), keep(v, dpp_u32<kXor1>(v), b1); }
+  __device__ __forceinline__ void below16(uint32_t& v) const { keep(v, dpp_u32<kXor8>(v), b8), keep(v, xor4(v), b4), below4(v); }
+  __device__ __forceinline__ void below64(uint32_t& v) const { keep(v, across32(v, b32), b32), keep(v, across16(v, b16), b16), below16(v); }
+  __device__ __forceinline__ void ascending(uint32_t& v) const {
+    keep(v, dpp_u32<kXor1>(v), b1);
+    keep(v, dpp_u32<kXor3>(v), b2), keep(v, dpp_u32<kXor1>(v), b1);
+    keep(v, dpp_u32<kXor7>(v), b4), below4(v);
+    keep(v, dpp_u32<kXor15>(v), b8), keep(v, xor4(v), b4), below4(v);
+    keep(v, dpp_u32<kXor15>(across16(v, b16)), b16), below16(v);
+    keep(v, mirrored(v), b32), keep(v, across16(v, b16), b16), below16(v);
+  }
+  // of 128 values, the lower ones to v
+  __device__ __forceinline__ void ascending(uint32_t& v, uint32_t& w) const {
+    ascending(v), ascending(w);
+    const uint32_t m = mirrored(w);
+    w = max(v, m), v = min(v, m);
+    below64(v), below64(w);
+  }
+};
+
 // One block per coarse cell, one wavefront per octant of it: with G = 16 an octant is a cell, with G = 32 it is narrowed
 // down once more for its eight cells. 26 M vector instructions (98 us) when the cells were taken from the coarse list
 // directly: the coarse lists at the rim of the cloud hold nearly everything. A wavefront forms the lists of its cells side by
 // side: a candidate is read once for all of them, its distances to their faces are formed once per axis and half of the octant,
 // and nothing waits in a chain of eight (cells one after the other: 25 us of the kernel's 51).
-template <int kG>
+template <int kG, bool kOrder>
 __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
     float* __restrict__ planes, Cell* __restrict__ cells, uint16_t* __restrict__ lists) {
   constexpr int kWaves = kBuildThreads / kWave;
@@ -465,16 +532,57 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
       n[c] += (int) __popcll(m);
     }
   }
+  // The lists again, to be put in order (ranks counted over LDS instead of the networks: 24 us instead of 10): an entry or two per lane, all of them on their way together.
+  constexpr int kEntries = kOrder ? kListCap / kWave : 1;
+  uint32_t held[kCells][kEntries];
+  if constexpr (kOrder) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+#pragma unroll
+    for (int c = 0; c < kCells; ++c)
+#pragma unroll
+      for (int h = 0; h < kEntries; ++h) held[c][h] = kWave * h + lane < min(n[c], kListCap) ? list[c][kWave * h + lane] : 0u;
+  }
+  // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
+  Cell cell[kCells];
+  const WaveSort sort;
 #pragma unroll
   for (int c = 0; c < kCells; ++c) {
     const bool fits = !too_many && n[c] <= kListCap && reach[c] < 3e38f;
-    // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
     if (fits && lane < 8 && n[c] + lane < (n[c] + 7) / 8 * 8) list[c][n[c] + lane] = (uint16_t) M;
     // the K nearest of any query of the cell are nearer than `reach`: their parts stay below 2^32, the others' may saturate
-    if (lane == 0)
-      cells[(list[c] - lists) / kListCap] = Cell{fits ? (uint32_t) n[c] | (inside[c] >= kCrowded ? kCrowdedBit : 0u) : kLongList,
-                                                 fminf(4294967296.0f / reach[c], 3e38f)};
+    cell[c] = Cell{fits ? (uint32_t) n[c] | (inside[c] >= kCrowded ? kCrowdedBit : 0u) : kLongList, fminf(4294967296.0f / reach[c], 3e38f), {}};
+    if constexpr (kOrder) {
+      if (!fits || n[c] <= 8) continue;
+      uint32_t key[kEntries];
+#pragma unroll
+      for (int h = 0; h < kEntries; ++h) {
+        const float4 p = s_y[held[c][h]];
+        const float d  = centre_distance(p.x - cell_centre(edge[0][c % kIn], edge[0][c % kIn + 1]),
+                                         p.y - cell_centre(edge[1][c / kIn % kIn], edge[1][c / kIn % kIn + 1]),
+                                         p.z - cell_centre(edge[2][c / (kIn * kIn)], edge[2][c / (kIn * kIn) + 1]));
+        key[h] = kWave * h + lane < n[c] ? (__float_as_uint(d) & ~kNumberBits) | held[c][h] : ~0u;
+      }
+      if (n[c] > kWave) sort.ascending(key[0], key[1]);
+      else sort.ascending(key[0]);
+      const float per_step = 0.9999f * __builtin_amdgcn_rcpf(cell_step(cell[c].scale));  // rounded down, by far more than either side's rounding
+      uint32_t bound[kEntries];
+#pragma unroll
+      for (int h = 0; h < kEntries; ++h) {
+        if (kWave * h + lane < n[c]) list[c][kWave * h + lane] = (uint16_t) (key[h] & kNumberBits);
+        bound[h] = (uint32_t) fminf(__uint_as_float(key[h] & ~kNumberBits) * per_step, 255.0f);  // (of a place past the end: a NaN, 255)
+      }
+      auto at = [&](int g) { return (uint32_t) __builtin_amdgcn_readlane(bound[8 * g / kWave], 8 * g % kWave); };
+#pragma unroll
+      for (int g = 1; g <= kBounds; ++g) {
+        uint32_t& word = g <= 2 ? cell[c].length : cell[c].bounds[(g - 3) / 4];
+        word |= at(g) << (g <= 2 ? 8 * g + 8 : (g - 3) % 4 * 8);
+      }
+    }
   }
+#pragma unroll
+  for (int c = 0; c < kCells; ++c)
+    if (lane == 0) cells[(list[c] - lists) / kListCap] = cell[c];
 }
 
 __device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
@@ -526,21 +634,59 @@ __device__ __forceinline__ void store_result(float* __restrict__ dist2, int64_t*
   }
 }
 
-// kG == 0: no grid, a wavefront per query.
-template <int kK, int kG>
+// The same for 64 queries from n0 on, a lane each, through `lds` (128 words of the wavefront's): rows of 16 to 64 bytes a lane apart make
+// a store of every 64 bytes they lie in, whole runs of 512 and 1024 bytes do not. kStream: past the caches.
+template <int kK, bool kStream>
+__device__ __forceinline__ void store_results(float* __restrict__ dist2, int64_t* __restrict__ index, int n0,
+                                              const float (&d)[kK], const int (&i)[kK], float* lds) {
+  typedef float Distances __attribute__((ext_vector_type(2)));
+  typedef int64_t Numbers __attribute__((ext_vector_type(2)));
+  constexpr int kQueries = kK > 4 ? 16 : 32, kPairs = kQueries * kK / 2;
+  static_assert(kPairs <= kWave);
+  const int lane = __lane_id();
+#pragma unroll
+  for (int c = 0; c < kWave / kQueries; ++c) {
+    const size_t at = ((size_t) n0 + c * kQueries) * kK + 2 * lane;
+    const bool mine = lane / kQueries == c, stores = lane < kPairs;
+    float* const to = lds + lane % kQueries * kK;
+    wave_lds_sync();
+    if (mine)
+#pragma unroll
+      for (int k = 0; k < kK; ++k) to[k] = d[k];
+    wave_lds_sync();
+    const Distances v = ((const Distances*) lds)[lane];
+    if constexpr (kStream) { if (stores) __builtin_nontemporal_store(v, (Distances*) (dist2 + at)); }
+    else if (stores) *(Distances*) (dist2 + at) = v;
+    wave_lds_sync();
+    if (mine)
+#pragma unroll
+      for (int k = 0; k < kK; ++k) to[k] = __int_as_float(i[k]);
+    wave_lds_sync();
+    const int2 w = ((const int2*) lds)[lane];
+    if constexpr (kStream) { if (stores) __builtin_nontemporal_store(Numbers{w.x, w.y}, (Numbers*) (index + at)); }
+    else if (stores) *(Numbers*) (index + at) = Numbers{w.x, w.y};
+  }
+  wave_lds_sync();
+}
+
+// kG == 0: no grid, a wavefront per query. kOrder: the lists are in the order of their cells' centre distances.
+template <int kK, int kG, bool kOrder>
 __global__ void __launch_bounds__(kQueryThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
 knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
     const float* __restrict__ y, const float* __restrict__ planes, const Cell* __restrict__ cells,
     const uint16_t* __restrict__ lists, float* __restrict__ dist2, int64_t* __restrict__ index) {
+  // 60 MB of results and more would push the lists out of the caches; fewer are left there for whoever asked
+  constexpr bool kStream = kOrder && kG > 16;
   // a query alone costs a wavefront about 20 M / 64 + 300 instructions, the all-pairs walk about 20 M for all 64
   const int max_alone = 20 * M / (20 * M / 64 + 300);
   constexpr int kWaves = kQueryThreads / kWave;
   extern __shared__ __attribute__((aligned(16))) char s_dyn[];
   float4* s_y = (float4*) s_dyn;  // [M + 8], the last eight at infinity
   __shared__ float s_plane[3][kG + 1];
-  __shared__ float s_cand_d[kWaves][kWave];
-  __shared__ int s_cand_i[kWaves][kWave];
+  __shared__ __attribute__((aligned(16))) float s_cand[kWaves][2 * kWave];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  float* const s_cand_d = s_cand[wave];  // distances and numbers of a query's candidates, or results on their way out
+  int* const s_cand_i   = (int*) &s_cand[wave][kWave];
   for (int i = t; i < M; i += kQueryThreads) s_y[i] = control_point(y, i);
   if (t < 8) s_y[M + t] = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
   if (kG > 0)
@@ -559,7 +705,7 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         const float d = distance2(qx, qy, qz, s_y[i]);
         const unsigned long long m = wave_ballot(i < M) & wave_ballot(d <= bound) & wave_ballot(d < __builtin_inff());
         const int pos = count + lanes_below(m);
-        if (((m >> lane) & 1ull) && pos < kWave) s_cand_d[wave][pos] = d, s_cand_i[wave][pos] = i;
+        if (((m >> lane) & 1ull) && pos < kWave) s_cand_d[pos] = d, s_cand_i[pos] = i;
         count += (int) __popcll(m);
       }
       return count;
@@ -570,11 +716,11 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const float d = lane < count ? s_cand_d[wave][lane] : __builtin_inff();
-    const int i   = lane < count ? s_cand_i[wave][lane] : -1;
+    const float d = lane < count ? s_cand_d[lane] : __builtin_inff();
+    const int i   = lane < count ? s_cand_i[lane] : -1;
     int rank = 0;
     for (int c = 0; c < count; ++c) {
-      const float o = s_cand_d[wave][c];
+      const float o = s_cand_d[c];
       rank += (int) (o < d) | ((int) (o == d) & (int) (c < lane));
     }
     if (lane >= count) rank = lane;  // slots nobody fills
@@ -633,6 +779,7 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
       const float q[3] = {x[at], x[at + 1], x[at + 2]};
       bool inside = live;
       int cell = 0;
+      float off[3];  // from the cell's centre
 #pragma unroll
       for (int a = 2; a >= 0; --a) {
         int i = 0;
@@ -641,9 +788,15 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
           if (s_plane[a][i + step] <= q[a]) i += step;
         inside = inside && q[a] >= s_plane[a][0] && q[a] < s_plane[a][kG];  // false for NaN
         cell   = cell * kG + i;
+        off[a] = q[a] - cell_centre(s_plane[a][i], s_plane[a][i + 1]);
       }
-      const Cell here  = inside ? cells[cell] : Cell{kLongList, 0.0f};
-      const bool listed = here.length != kLongList;
+      Cell here{kLongList, 0.0f, {}};
+      if (inside) {
+        if constexpr (kOrder) here = cells[cell];
+        else here.length = cells[cell].length, here.scale = cells[cell].scale;
+      }
+      const float far_off = kOrder ? 1.0001f * centre_distance(off[0], off[1], off[2]) : 0.0f, step = kOrder ? cell_step(here.scale) : 0.0f;
+      const bool listed = (here.length & 0xffu) != kLongList;
       const uint16_t* list = lists + (size_t) cell * kListCap;
       uint32_t key[kK + 1];
       auto insert = [&](uint32_t nk) {
@@ -659,7 +812,18 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
         int c = 0;
         unsigned long long longer;
+        uint32_t now_bounds = here.length >> 16, next_bounds = here.bounds[0], last_bounds = here.bounds[1];
         for (;; c += 8) {
+          // An entry at distance d from the centre is at least d - far_off away: past the last one that can be among the smallest
+          // keys the list is over.
+          if (kOrder && c > 0) {
+            const float least = fmaxf(fmaf((float) (now_bounds & 255u), step, -far_off), 0.0f);
+            const uint32_t part = distance_part<decltype(fine)::value>(least * least * here.scale);
+            if (part > (key[kK] | kNumberBits)) n_list = min(n_list, c);
+            if (c == 16) now_bounds = next_bounds;
+            else if (c == 48) now_bounds = last_bounds;
+            else if (c < 8 * kBounds) now_bounds >>= 8;
+          }
           longer = wave_ballot(c < n_list);
           if (__popcll(longer) <= kFewLists) break;
           if (c < n_list) {
@@ -722,7 +886,11 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         bi[k] = unknown ? M : (int) (key[k] & kNumberBits);
         bd[k] = distance2(q[0], q[1], q[2], s_y[bi[k]]);
       }
-      if (live && !unknown) store_result<kK>(dist2, index, n, bd, bi);
+      if (kK > 2 && wave_ballot(live && !unknown) == ~0ull) {
+        if constexpr (kK > 2) store_results<kK, kStream>(dist2, index, n0, bd, bi, s_cand_d);
+      } else if (live && !unknown) {
+        store_result<kK>(dist2, index, n, bd, bi);
+      }
 
       unsigned long long rest = wave_ballot(live && unknown), together = 0ull;
       if (__popcll(rest) > max_alone) together = rest, rest = 0ull;
@@ -739,7 +907,7 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
   }
 }
 
-template <int kK, int kG>
+template <int kK, int kG, bool kOrder>
 void launch_query(int N, int M, const float* x, const float* y, const GridLayout& l, char* ws, float* dist2,
                   int64_t* index, hipStream_t s) {
   const size_t lds = 16 * (size_t) (M + 8);
@@ -747,7 +915,7 @@ void launch_query(int N, int M, const float* x, const float* y, const GridLayout
   // blocks that fit on a compute unit (one round 259 us, two 248, four and more 248 at 3M x 2048)
   const int per_block = kG > 0 ? kQueryThreads : kQueryThreads / kWave;
   const int blocks = std::min(div_up(N, per_block), 256 * 8);
-  hipLaunchKernelGGL((knn_cell_query_kernel<kK, kG>), dim3(blocks), dim3(kQueryThreads), lds, s, N, M, x, y,
+  hipLaunchKernelGGL((knn_cell_query_kernel<kK, kG, kOrder>), dim3(blocks), dim3(kQueryThreads), lds, s, N, M, x, y,
                      (const float*) (ws + l.planes), (const Cell*) (ws + l.cells), (const uint16_t*) (ws + l.lists),
                      dist2, index);
 }
@@ -756,17 +924,23 @@ template <int kK>
 int launch_grid_knn(Scheme scheme, int N, int M, const float* x, const float* y, float* dist2, int64_t* index, char* ws,
                     hipStream_t s) {
   const GridLayout l = grid_layout(scheme);
-  if (scheme == kAlone) {
-    launch_query<kK, 0>(N, M, x, y, l, ws, dist2, index, s);
-  } else if (scheme == kGrid16) {
-    hipLaunchKernelGGL(knn_cell_lists_kernel<16>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
+  auto launch = [&](auto grid, auto order) {
+    constexpr int kG = decltype(grid)::value;
+    constexpr bool kOrder = decltype(order)::value;
+    hipLaunchKernelGGL((knn_cell_lists_kernel<kG, kOrder>), dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
                        (float*) (ws + l.planes), (Cell*) (ws + l.cells), (uint16_t*) (ws + l.lists));
-    launch_query<kK, 16>(N, M, x, y, l, ws, dist2, index, s);
-  } else {
-    hipLaunchKernelGGL(knn_cell_lists_kernel<32>, dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
-                       (float*) (ws + l.planes), (Cell*) (ws + l.cells), (uint16_t*) (ws + l.lists));
-    launch_query<kK, 32>(N, M, x, y, l, ws, dist2, index, s);
-  }
+    launch_query<kK, kG, kOrder>(N, M, x, y, l, ws, dist2, index, s);
+  };
+  auto launch_grid = [&](auto grid) {
+    constexpr int64_t kFrom = kOrderFrom<kK, decltype(grid)::value>;
+    if constexpr (kFrom == 0) launch(grid, std::true_type());
+    else if constexpr (kFrom == INT64_MAX) launch(grid, std::false_type());
+    else if (N >= kFrom) launch(grid, std::true_type());
+    else launch(grid, std::false_type());
+  };
+  if (scheme == kAlone) launch_query<kK, 0, false>(N, M, x, y, l, ws, dist2, index, s);
+  else if (scheme == kGrid16) launch_grid(std::integral_constant<int, 16>());
+  else launch_grid(std::integral_constant<int, 32>());
   return check_launch("knn_topk");
 }
 

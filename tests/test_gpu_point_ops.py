@@ -345,6 +345,29 @@ def test_knn_clusters(N, M, K, radius, mixed, device):
     assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
 
 
+# Lists in the order of their cells' centre distances (32^3 cells from 10M / (K + 2) queries on, 16^3 from K = 3 or 400 000), where a query's
+# walk ends before its list does; the last wavefront is not full. Far from the origin a cell's extent is a few roundings of its coordinates.
+@pytest.mark.parametrize('N,M,K', [(1_000_001, 2560, 8), (1_428_573, 641, 5), (2_500_007, 700, 2), (400_001, 640, 1), (16_449, 192, 3)])
+@pytest.mark.parametrize('kind', ['normal', 'lattice', 'clusters', 'far', 'heavy tails', 'flat'])
+def test_knn_ordered_lists(N, M, K, kind, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N + M + K)
+    pts, ctrl = torch.randn(N, 3, generator=g), torch.randn(M, 3, generator=g)
+    if kind == 'lattice':
+        pts, ctrl = (pts * 4).round() / 4, (ctrl * 4).round() / 4
+    elif kind == 'clusters':
+        pts, ctrl = _clusters(N, M // 16 * 16, 1e-2, g)
+    elif kind == 'far':
+        pts, ctrl = pts * 1e-2 + 3e3, ctrl * 1e-2 + 3e3
+    elif kind == 'heavy tails':
+        pts, ctrl = pts * torch.randn(N, 1, generator=g).exp(), ctrl * torch.randn(M, 1, generator=g).exp()
+    elif kind == 'flat':
+        pts[:, 1], ctrl[:, 1] = 0.5, 0.5
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+
+
 def test_knn_clusters_keep_to_the_lists(device):
     """With the keys' coarse parts alone, tight clusters sent every query to the exact search: thirteen times the time."""
     g = torch.Generator().manual_seed(7)
