@@ -142,7 +142,8 @@ constexpr int kNarrowTiles = 16384, kMaxLdsTiles = 40960;
 
 // Which tiles of a surfel's rectangle are visited: all of them (the reference's lists), those that pass the fast path's
 // corner test (CornerTest, from the surfel's adjugate and opacity), or those whose bit is set in the surfel's keep mask
-// (cull_mask_kernel: the tiles some pixel of which can blend the surfel; rectangles above 32 tiles are kept whole).
+// (cull_mask_kernel: the tiles some pixel of which can blend the surfel; for rectangles above 32 tiles a window of them,
+// cull_window, or all).
 // kWalkCornerMask is the corner test with its verdicts for rectangles of at most 32 tiles taken from a mask the
 // preprocess kernel left (bit x * h + y: x-major, the order of the fast path's key span), so that the test's set-up (a
 // double-precision logarithm among it) runs once per surfel and view instead of once per walk; larger rectangles are
@@ -170,7 +171,10 @@ constexpr int kWalkGroup = 4;
 // With the depth loaded by each visit, every entry of a surfel cost the scatter a round trip to memory: 3M surfels
 // 1352x1014 104 -> 91 us, 25k Gaussians 639x361 10.8 -> 7.4, 10k surfels 256x256 5.6 -> 4.5. What bounds it at many entries is
 // the rate at which the L2s take single stores, 100 to 140 G/s: 4-byte entries (the sort gathering the depths) took 3840x2160 from
-// 152 to 145 us, parts of the picture one after the other, each within the L2s, to 140.
+// 152 to 145 us, parts of the picture one after the other, each within the L2s, to 140. So fewer entries is what helps: windows
+// of the large rectangles (cull_window) took that view's 10.7M entries to 6.0M, the scatter from 161 to 100 us, the sort from 46
+// to 37 and the blend from 950 to 870, with the count at 34 as before (41 with each window worked out by the whole wavefront in
+// its turn, 59 with the tiles' columns and rows by division too).
 template <int kMode, typename Visit>
 __device__ __forceinline__ void for_each_instance(int i, int P, int gx, int gy, const float2* __restrict__ means2D,
                                                   const int32_t* __restrict__ radii, const float* __restrict__ depths,
@@ -226,19 +230,44 @@ __device__ __forceinline__ void for_each_instance(int i, int P, int gx, int gy, 
     }
   }
   unsigned long long big = __ballot(count > kCoopThreshold);
+  // Large rectangles with a window: its columns and rows, without those of their tiles that lie outside its diagonals. Each
+  // lane works out its own surfel's window, in tiles of the grid, and the wavefront then reads one lane's after the other.
+  TileWindow v = {0, 0, 0, 0, 0, 0, 0, 0};
+  unsigned inv_width = 0u;
+  if (kMode == kWalkMask && big) {
+    v = tile_window(keep_mask, w, h);
+    v.x0 += x0, v.x1 += x0, v.y0 += y0, v.y1 += y0, v.s0 += x0 + y0, v.s1 += x0 + y0;
+    v.d0 += x0 - y0 - (h - 1), v.d1 += x0 - y0 - (h - 1);
+    big = __ballot(count > kCoopThreshold && v.x0 <= v.x1);
+    inv_width = (unsigned) (65536.0f * __builtin_amdgcn_rcpf((float) max(v.x1 - v.x0 + 1, 1))) + 1u;  // e / width = e * this >> 16 for e <= 64
+  }
   while (big) {
     const int src = __ffsll((long long) big) - 1;
     big &= big - 1;
-    const int sx0 = __shfl(x0, src, kWave), sy0 = __shfl(y0, src, kWave), sw = __shfl(w, src, kWave);
-    const int scount = __shfl(count, src, kWave), sid = __shfl(i, src, kWave);
-    const uint32_t sdepth = (uint32_t) __shfl((int) depth, src, kWave);
-    float sIM[kCorner ? 9 : 1];
+    auto of = [src](int value) { return __builtin_amdgcn_readlane(value, src); };
+    const int sx0 = of(x0), sy0 = of(y0), sw = of(w), sid = of(i);
+    const uint32_t sdepth = (uint32_t) of((int) depth);
+    if (kMode == kWalkMask) {
+      // a lane goes on by 64 tiles, `down` rows and `right` columns, so that nothing is divided on the way
+      const int left = of(v.x0), end = of(v.x1), bottom = of(v.y1), width = end - left + 1;
+      const int s0 = of(v.s0), s1 = of(v.s1), d0 = of(v.d0), d1 = of(v.d1);
+      const unsigned inv = (unsigned) of((int) inv_width);
+      const int down = (int) (kWave * inv >> 16), right = kWave - down * width, first = (int) (lane * inv >> 16);
+      for (int y = of(v.y0) + first, x = left + lane - first * width; y <= bottom; y += down) {
+        if (x + y >= s0 && x + y <= s1 && x - y >= d0 && x - y <= d1) visit_one(y * gx + x, sid, sdepth);
+        x += right;
+        if (x > end) x -= width, ++y;
+      }
+    } else {
+      const int scount = of(count);
+      float sIM[kCorner ? 9 : 1];
 #pragma unroll
-    for (int k = 0; k < (kCorner ? 9 : 1); ++k) sIM[k] = kCorner ? __shfl(IM[k], src, kWave) : 0.0f;
-    const CornerTest ct(sIM, kCorner ? __shfl(opacity, src, kWave) : 1.0f);
-    for (int e = lane; e < scount; e += kWave) {
-      const int y = e / sw, x = e - y * sw;
-      if (!kCorner || ct.tile(sx0 + x, sy0 + y)) visit_one((sy0 + y) * gx + (sx0 + x), sid, sdepth);
+      for (int k = 0; k < (kCorner ? 9 : 1); ++k) sIM[k] = kCorner ? __shfl(IM[k], src, kWave) : 0.0f;
+      const CornerTest ct(sIM, kCorner ? __shfl(opacity, src, kWave) : 1.0f);
+      for (int e = lane; e < scount; e += kWave) {
+        const int y = e / sw, x = e - y * sw;
+        if (!kCorner || ct.tile(sx0 + x, sy0 + y)) visit_one((sy0 + y) * gx + (sx0 + x), sid, sdepth);
+      }
     }
   }
 }

@@ -110,7 +110,45 @@ __device__ __forceinline__ bool cull_keeps_tile(const CullBounds& c, float ox, f
 }
 
 // Which tiles of a surfel's rectangle the binning keeps, as a bit per tile in row-major order (bit (ty - y0) * w +
-// (tx - x0)); rectangles of more than 32 tiles are kept whole (all bits set).
+// (tx - x0)). The word of a rectangle of more than kCullMaskTiles tiles says the same in coarser form, as a window: all bits
+// set keeps it whole, as the sums of gradient records expect it; a view without a backward stores cull_window.
 constexpr int kCullMaskTiles = 32;
+
+// The window of a large rectangle: cull_keeps_tile in whole tiles is four intervals, of the tile's column, its row and its two
+// diagonals (x + y, x - y) in the rectangle, each of which is kept in sixteenths of the n values it can take: four bits for
+// 15 less the sixteenth of its first value, four for that of its last. Up to 16 columns or rows (17 tiles a diagonal) a
+// sixteenth holds one value at most and nothing is lost. 0: no tile; all bits set: all.
+// A 3840x2160 view of 400k surfels has 64 % of its instances in rectangles above 32 tiles, two thirds of which no pixel can
+// blend; a bit per group of tiles instead (32 groups) drops half of them.
+struct TileWindow {
+  int x0, x1, y0, y1, s0, s1, d0, d1;  // inclusive; column, row, column + row, column - row + h - 1
+};
+
+__device__ __forceinline__ TileWindow tile_window(uint32_t word, int w, int h) {
+  auto first = [&](int shift, int n) { return ((15 - (int) (word >> shift & 15u)) * n + 15) >> 4; };
+  auto last  = [&](int shift, int n) { return ((((int) (word >> shift & 15u) + 1) * n + 15) >> 4) - 1; };
+  const int n = w + h - 1;
+  return {first(0, w), last(4, w), first(8, h), last(12, h), first(16, n), last(20, n), first(24, n), last(28, n)};
+}
+
+__device__ __forceinline__ uint32_t cull_window(const CullBounds& c, float ox, float oy, const TileRect& r) {
+  if (c.state != 2) return c.state == 1 ? 0xffffffffu : 0u;
+  const int w = r.x1 - r.x0, h = r.y1 - r.y0;
+  const float side = (float) (kTile - 1);
+  uint32_t word = 0u;
+  bool some = true;
+  // the values k of 0 .. n - 1 with low <= kTile (k + base) <= high, in pixels; what is no number bounds nothing
+  auto interval = [&](int shift, float low, float high, int base, int n) {
+    const int a = (int) fminf(fmaxf(ceilf(low * (1.0f / kTile)) - (float) base, 0.0f), (float) n);
+    const int b = (int) fmaxf(fminf(floorf(high * (1.0f / kTile)) - (float) base, (float) (n - 1)), -1.0f);
+    some &= a <= b;
+    if (some) word |= (15u - (unsigned) a * 16u / (unsigned) n | (unsigned) b * 16u / (unsigned) n << 4) << shift;
+  };
+  interval(0, c.x0 + ox - side, c.x1 + ox, r.x0, w);
+  interval(8, c.y0 + oy - side, c.y1 + oy, r.y0, h);
+  interval(16, c.a0 + (ox + oy) - 2.0f * side, c.a1 + (ox + oy), r.x0 + r.y0, w + h - 1);
+  interval(24, c.b0 + (ox - oy) - side, c.b1 + (ox - oy) + side, r.x0 - r.y0 - (h - 1), w + h - 1);
+  return some ? word : 0u;
+}
 
 }  // namespace fsgs

@@ -261,20 +261,27 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   }
   if (keep_masks) {
     // Which tiles of the surfel's rectangle some pixel of which can blend it (the culled binning's input): a bit per
-    // tile, row-major; rectangles above kCullMaskTiles tiles keep every bit. Evaluated here, where transform, centre
+    // tile, row-major, or for rectangles above kCullMaskTiles tiles a window of them. With record slots the backward sums
+    // every position of a large rectangle, so there all bits are set. Evaluated here, where transform, centre
     // and radius are in registers and the vector units wait for memory anyway.
+    const bool windows = view.counters && !view.slot_offsets;
     uint32_t m = 0xffffffffu;
     if (ok) {
       const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
       const TileRect r = tile_rect(c2[0], c2[1], f2i_sat(radius), gx, gy);
       const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
-      if (w * h <= kCullMaskTiles) {
+      const bool small = w * h <= kCullMaskTiles;
+      if (small || windows) {
         const CullBounds cb = cull_bounds(M, c2[0], c2[1], op);
         m = 0u;
         int e = 0;
-        for (int y = 0; y < h; ++y)
-          for (int x = 0; x < w; ++x, ++e)
-            if (cull_keeps_tile(cb, c2[0], c2[1], r.x0 + x, r.y0 + y)) m |= 1u << e;
+        if (small) {
+          for (int y = 0; y < h; ++y)
+            for (int x = 0; x < w; ++x, ++e)
+              if (cull_keeps_tile(cb, c2[0], c2[1], r.x0 + x, r.y0 + y)) m |= 1u << e;
+        } else {
+          m = cull_window(cb, c2[0], c2[1], r);
+        }
       }
     }
     keep_masks[i] = m;

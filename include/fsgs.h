@@ -52,7 +52,8 @@ int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, 
 /* A whole view without a prefix scan (no counterpart in the reference): the preprocess hands out the gradient records'
  * slots itself. slot_counters[64] are zero before the call and again after fsgs_gs_view_count; a surfel's slots start at
  * slot_offsets[i] + slot_regions[(i / 256) % 64] and are tiles_touched[i] many. visible[P] (0 / 1), slot_offsets, records
- * and keep_masks are optional. Every row of the outputs is written. */
+ * and keep_masks are optional. Without slot_offsets there will be no backward, and keep_masks of surfels with rectangles above 32
+ * tiles, which have all bits set otherwise, narrow those rectangles too (the binning knows how). Every row of the outputs is written. */
 int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
     const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
