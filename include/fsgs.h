@@ -10,7 +10,7 @@
  *    caller (the *_workspace_bytes functions size them). Outputs need not be zero-initialised unless stated. What the
  *    library keeps of its own is in file-scope device arrays that exist once per GPU from the moment the library is
  *    loaded: eight blockIdx -> tile schedule tables of 256 KiB (one per stream that bins or blends, see
- *    fsgs_stream_release) and the 512 KiB of fsgs_image_loss_forward_static.
+ *    fsgs_stream_release) and the 2.5 MiB of fsgs_image_loss_forward_static.
  *  - Return value 0 = success; otherwise fsgs_last_error() describes the failure (thread local).
  *  - `file:line` citations name the reference interface each entry point replaces (relative to the reference root).
  */

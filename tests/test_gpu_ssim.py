@@ -124,3 +124,40 @@ def test_fused_image_loss(shape, lam, device, oracle_mod):
     assert rel_err(npy(x.grad), npy(y.grad)) < 1e-5
     # no gradient wanted: the same number
     assert float(l1_dssim_loss(img1.to(device), t, lam)) == float(loss)
+
+
+@pytest.mark.parametrize("shape,shift", [((1, 1, 1, 1), 0), ((1, 2, 6, 53), 0), ((2, 5, 7, 54), 0), ((1, 3, 8, 55), 0),
+                                         ((1, 4, 15, 108), 1), ((1, 1, 64, 1), 0), ((3, 1, 2, 163), 0), ((1, 3, 71, 866), 0)])
+def test_ssim_tile_edges(shape, shift, device, oracle_mod):
+    """Tiles of 54 x 7 outputs: sizes around one and two of them, single rows and columns, more channels than a block has
+    wavefronts, odd widths and planes off a multiple of 8 bytes (whole rows instead of pairs), more than eight tiles; the loss
+    form's gradient and sums against the map form's. Tolerances as above."""
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.ssim import l1_dssim_loss
+    O = oracle_mod
+    B, CH, H, W = shape
+    g = torch.Generator().manual_seed(H * W + CH)
+    n = B * CH * H * W
+    place = lambda t: torch.cat([torch.zeros(shift), t.flatten()]).to(device)[shift:].view(shape)
+    img1, img2 = torch.rand(*shape, generator=g), torch.rand(*shape, generator=g)
+    img2[..., : W // 2] = img1[..., : W // 2] * 0.9
+    gmap = torch.randn(*shape, generator=g)
+    x, y = place(img1), place(img2)
+    m, d1, d2, d3 = get_C_function('fusedssim')(0.01 ** 2, 0.03 ** 2, x, y, True)
+    a, b = npy(img1), npy(img2)
+    rm, r1, r2, r3, rg, rl = (np.zeros_like(a) for _ in range(6))
+    assert O.call("fusedssim_forward_f32", B, CH, H, W, 0.01 ** 2, 0.03 ** 2, a, b, rm, r1, r2, r3) == 0
+    assert abs_err(npy(m), rm) < 5e-6
+    for u, r, name in ((d1, r1, 'dm_dmu1'), (d2, r2, 'dm_dsigma1_sq'), (d3, r3, 'dm_dsigma12')):
+        assert rel_err(npy(u), r) < 1e-4, name
+    grad = get_C_function('fusedssim_backward')(0.01 ** 2, 0.03 ** 2, x, y, place(gmap), d1, d2, d3)
+    assert O.call("fusedssim_backward_f32", B, CH, H, W, a, b, npy(gmap), npy(d1), npy(d2), npy(d3), rg) == 0
+    assert rel_err(npy(grad), rg) < 1e-4
+    leaf = x.detach().requires_grad_(True)
+    loss, terms = l1_dssim_loss(leaf, y, 0.3, return_terms=True)
+    loss.backward()
+    assert abs(float(terms[0]) - np.abs(a.astype(np.float64) - b).mean()) < 2e-6
+    assert abs(float(terms[1]) - float(m.double().mean())) < 2e-6
+    assert O.call("fusedssim_backward_f32", B, CH, H, W, a, b, np.full_like(a, -0.3 / n), npy(d1), npy(d2), npy(d3), rl) == 0
+    want = rl.astype(np.float64) + 0.7 / n * np.sign(a.astype(np.float64) - b)
+    assert rel_err(npy(leaf.grad), want.astype(np.float32)) < 1e-4
