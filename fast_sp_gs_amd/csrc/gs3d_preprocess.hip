@@ -293,11 +293,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
   float dc[3] = {0, 0, 0};
-  if (kWave) {  // the fetch of the rows is in flight during the geometry
-    wanted = __ballot(valid && !(culling && culling[i]));
-    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
-    if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
-  }
+  if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   do {
     if (!valid || (culling && culling[i])) break;
     float Tw2v[16], Tv2c[16];
@@ -316,10 +312,33 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
                          cov2D_precomp ? cov2D_precomp + 3 * (size_t) i : nullptr, fx, fy, tanx, tany, Tw2v, sc);
   } while (false);
 
+  if (kWave) {
+    // as in the surfels' kernel only the rows of what is on the screen; the mask is found while they are on their way. 300k
+    // Gaussians 31.2 -> 29.1 us, 25k 12.7 -> 12.4
+    wanted = __ballot(ok);
+    if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
+  }
   if (view.counters) {  // how many instances the view has
     int total;
     (void) slots_in_block(ok ? sc.area : 0, s_wave_slots, total);
     if (threadIdx.x == 0) atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+  }
+  uint32_t keep = 0xffffffffu;
+  if (keep_masks) {
+    // which tiles of the rectangle some pixel of which can blend the Gaussian (as conic_cull_mask_kernel finds it), here
+    // where centre and conic are in registers
+    if (ok) {
+      const TileRect r = tile_rect(sc.px, sc.py, f2i_sat(sc.radius), gx, gy);
+      const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
+      if (w * h <= kCullMaskTiles) {
+        const CullBounds cb = conic_cull_bounds(sc.conic[0], sc.conic[1], sc.conic[2], opacity);
+        keep = 0u;
+        int e = 0;
+        for (int y = 0; y < h; ++y)
+          for (int x = 0; x < w; ++x, ++e)
+            if (cull_keeps_tile(cb, sc.px, sc.py, r.x0 + x, r.y0 + y)) keep |= 1u << e;
+      }
+    }
   }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
@@ -372,24 +391,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   if (view.visible) view.visible[i] = ok && f2i_sat(sc.radius) > 0;
   if (ok || !means2D_preserve) means2D[i] = ok ? make_float2(sc.px, sc.py) : make_float2(0.0f, 0.0f);
   conic_opacity[i] = ok ? make_float4(sc.conic[0], sc.conic[1], sc.conic[2], opacity) : make_float4(0, 0, 0, 0);
-  if (keep_masks) {
-    // which tiles of the rectangle some pixel of which can blend the Gaussian (as conic_cull_mask_kernel finds it), here
-    // where centre and conic are in registers
-    uint32_t m = 0xffffffffu;
-    if (ok) {
-      const TileRect r = tile_rect(sc.px, sc.py, f2i_sat(sc.radius), gx, gy);
-      const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
-      if (w * h <= kCullMaskTiles) {
-        const CullBounds cb = conic_cull_bounds(sc.conic[0], sc.conic[1], sc.conic[2], opacity);
-        m = 0u;
-        int e = 0;
-        for (int y = 0; y < h; ++y)
-          for (int x = 0; x < w; ++x, ++e)
-            if (cull_keeps_tile(cb, sc.px, sc.py, r.x0 + x, r.y0 + y)) m |= 1u << e;
-      }
-    }
-    keep_masks[i] = m;
-  }
+  if (keep_masks) keep_masks[i] = keep;
 }
 
 template <int kSh, int kRow>
