@@ -15,7 +15,7 @@
 // in 128 registers, four wavefronts per SIMD instead of three. Backward with flow, 300k surfels 800x800:
 // 485 -> 340 us; 5000 surfels with deviations of about 43 pixels 784 -> 627, 2000 of about 128 pixels 1468 -> 1149 (with a work
 // list per 8x8 quadrant they took 530, 715 and 1280).
-// Bound by vector issue (166 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
+// Bound by vector issue (152 instructions a step) and by the waits between batches. Against a work list per 8x8 quadrant with
 // the blended pairs queued and their components formed 64 pairs at a time: 300k surfels 800x800 311 -> 289 us, 3M 1352x1014
 // 1170 -> 950, 10k 256x256 58 -> 40; with the forward's hit_blocks in place of a bound per footprint (a tenth fewer steps, 260
 // instructions less per staged wavefront, for 7 us more in the forward) 245, 805 and 36; with batches of up to 128 entries
@@ -270,7 +270,7 @@ blend_backward_kernel(
        // share one instruction stream.
        auto pair_gradients = [&](const SplatHot& hot, const SplatCold& cold, int j, const Hit& h, bool hit,
                                  float (&g)[16], float& g2x, float& g2y, unsigned long long& filtered_lanes) {
-         float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, s_ds = 0.0f, z_sx = 0.0f, z_sy = 0.0f;
+         float w = 0.0f, dL_dalpha = 0.0f, dL_dz = 0.0f, GdA = 0.0f, oG = 0.0f, dsx = 0.0f, dsy = 0.0f, sx = 0.0f, sy = 0.0f;
          if (hit) {
            advance_pixel(cold, j, h, w, dL_dalpha, dL_dz, dsx, dsy);
            if (kFlow) dsx += dL_dz * hot.m[6], dsy += dL_dz * hot.m[7];
@@ -279,26 +279,24 @@ blend_backward_kernel(
            // the Gaussian's own part of d/ds: only the intersection case uses it (times 1 / p_z below)
            oG = hot.opacity * GdA;
            dsx -= oG * h.sx, dsy -= oG * h.sy;
-           // s is not finite in a lane whose plane pair degenerates (p_z == 0), and such a lane never blends: every use
-           // of s sits on this side
-           s_ds = dsx * h.sx + dsy * h.sy;
-           z_sx = dL_dz * h.sx, z_sy = dL_dz * h.sy;
+           // s is not finite in a lane whose plane pair degenerates (p_z == 0), and such a lane never blends: what is used of
+           // it is zero there
+           sx = h.sx, sy = h.sy;
          }
          const bool by_ray   = h.rho3d <= h.rho2d;
          const bool filtered = hit && !by_ray;
          filtered_lanes      = ~wave_ballot(by_ray);  // taken where the comparison is made: its own lane mask, no instruction
-         // d/dp of the homogeneous intersection point p = k x l, negated (the components below are minus the plane
-         // gradients): p_xy = s p_z, so dp_xy = ds / p_z and dp_z = -<ds, s> / p_z
+         // s = (s, 1) solves k s = l s = 0, so with dk_z and dl_z from the 2x2 system of its first two components (whose
+         // determinant is p_z) the gradients of the planes are dk = dk_z (s, 1) and dl = dl_z (s, 1), those of the
+         // transform's rows -dk, -dl and, with the depth <row 2, (s, 1)>, x dk + y dl + dL/dz (s, 1). As l x dp and dp x k, dp the
+         // gradient of p = k x l, they were 14 instructions more: 300k 215 -> 205 us, 3M 843 -> 805, and less exact.
          const float rz  = (hit && by_ray) ? __builtin_amdgcn_rcpf(h.pz) : 0.0f;
-         const float npx = -(dsx * rz), npy = -(dsy * rz), npz = s_ds * rz;
-         const float nkx = h.ly * npz - h.lz * npy, nky = h.lz * npx - h.lx * npz, nkz = h.lx * npy - h.ly * npx;
-         const float nlx = npy * h.kz - npz * h.ky, nly = npz * h.kx - npx * h.kz, nlz = npx * h.ky - npy * h.kx;
+         const float ax = dsx * rz, ay = dsy * rz;
+         const float nk = h.ly * ax - h.lx * ay, nl = h.kx * ay - h.ky * ax, nw = dL_dz - (pxf * nk + pyf * nl);
          g[0] = w * dLp0, g[1] = w * dLp1, g[2] = w * dLp2;
-         g[3] = nkx, g[4] = nky, g[5] = nkz;
-         g[6] = nlx, g[7] = nly, g[8] = nlz;
-         g[9]  = z_sx - (pxf * nkx + pyf * nlx);
-         g[10] = z_sy - (pxf * nky + pyf * nly);
-         g[11] = dL_dz - (pxf * nkz + pyf * nlz);
+         g[3] = nk * sx, g[4] = nk * sy, g[5] = nk;
+         g[6] = nl * sx, g[7] = nl * sy, g[8] = nl;
+         g[9] = nw * sx, g[10] = nw * sy, g[11] = nw;
          if (kAux) g[12] = w * dLn0, g[13] = w * dLn1, g[14] = w * dLn2;
          else      g[12] = g[13] = g[14] = 0.0f;
          g[15] = GdA;
