@@ -500,12 +500,15 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
   const float T_final = inside ? 1.0f - out_opacity[pix] : 0.0f;
   float T = T_final;
   const float dL_dT = inside ? -dL_dout_opacity[pix] : 0.0f;
-  float g_out[3 + (E > 0 ? E : 1)], accum[3 + (E > 0 ? E : 1)];
+  float g_out[3 + (E > 0 ? E : 1)];
 #pragma unroll
-  for (int k = 0; k < 3 + E; ++k) {
-    accum[k] = 0.0f;
-    g_out[k] = !inside ? 0.0f : (k < 3 ? dL_dpix[k * HW + pix] : dL_dout_extras[(k - 3) * HW + pix]);
-  }
+  for (int k = 0; k < 3 + E; ++k) g_out[k] = !inside ? 0.0f : (k < 3 ? dL_dpix[k * HW + pix] : dL_dout_extras[(k - 3) * HW + pix]);
+  // All channels share one recurrence: with c = <upstream gradient, channels of the Gaussian> the pairs behind a pair have left
+  // sum c w in `behind_sum`, and what the background's transmittance takes, the same for every pair, starts it. Ten instructions
+  // of about 95 less than an accumulator per channel, and the registers of two: 300k Gaussians 125 -> 116 us. Errors of the
+  // gradients against 64 bits, upstream gradients at random: centres 2.8e-7 -> 2.8e-7 to 4.6e-7 -> 4.4e-7, conics 2.8e-7 -> 2.8e-7
+  // to 5.7e-7 -> 5.5e-7 (typical row); the same for every pixel and channel: 2.3e-7 -> 2.3e-7 to 4.0e-7 -> 4.2e-7.
+  float behind_sum = T_final * dL_dT;
 
   G3Splat<E> next;
   unsigned next_hits = 0u;
@@ -580,16 +583,14 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
         float g[kSums];
         float dch = 0.0f, GdA = 0.0f;
         if (hit) {
-          T   = T * __builtin_amdgcn_rcpf(1.0f - h.alpha);
-          dch = h.alpha * T;
-          float dL_dalpha = 0.0f;
+          const float r = __builtin_amdgcn_rcpf(1.0f - h.alpha);
+          float c = splat.feat[0] * g_out[0];
 #pragma unroll
-          for (int k = 0; k < 3 + E; ++k) {
-            const float v = splat.feat[k];
-            dL_dalpha += (v * T * (1.0f - h.alpha) - accum[k]) * g_out[k];
-            accum[k] += v * dch;
-          }
-          GdA = (dL_dalpha - T_final * dL_dT) * __builtin_amdgcn_rcpf(1.0f - h.alpha) * h.G;
+          for (int k = 1; k < 3 + E; ++k) c = fmaf(splat.feat[k], g_out[k], c);
+          GdA = fmaf(c, T, -behind_sum) * r * h.G;  // T: behind the pair
+          T   = T * r;
+          dch = h.alpha * T;
+          behind_sum = fmaf(c, dch, behind_sum);
         }
         if (!kNine) {
 #pragma unroll
@@ -600,9 +601,9 @@ gs3d_backward_kernel(int flags, const int* __restrict__ tile_order, int W, int H
         // the geometry's part without the factor -opacity
         g[kGeom]     = GdA * (splat.a * h.dx + splat.b * h.dy);
         g[kGeom + 1] = GdA * (splat.c * h.dy + splat.b * h.dx);
-        g[kGeom + 2] = h.dx * h.dx * GdA;
-        g[kGeom + 3] = h.dx * h.dy * GdA;
-        g[kGeom + 4] = h.dy * h.dy * GdA;
+        g[kGeom + 2] = h.dx * (h.dx * GdA);
+        g[kGeom + 3] = h.dy * (h.dx * GdA);
+        g[kGeom + 4] = h.dy * (h.dy * GdA);
         g[kGeom + 5] = GdA;
         float tot;
         if constexpr (kNine) tot = row_sum9_transposed(g);
