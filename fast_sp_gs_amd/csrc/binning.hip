@@ -339,7 +339,7 @@ __global__ void __launch_bounds__(256) cull_mask_kernel(int P, int gx, int gy, c
 }
 
 // Layout of the `bins` buffer of the bucket binning: the queue length of the long segments in front of the B x T matrix
-// of per-(walk block, tile) instance counts.
+// of per-(walk block, tile) instance counts, whose last row holds the tiles' totals.
 constexpr int kPrefixTiles = 64, kPrefixWaves = 16, kPrefixChunk = 32;  // walk blocks <= kPrefixWaves * kPrefixChunk
 constexpr size_t kBinsSums = 256;  // behind the queue length: the instances of every 64 tiles
 constexpr size_t kBinsHeader = 4096;
@@ -357,7 +357,7 @@ inline BinsLayout bins_layout(int P, int T) {
   const int most = T > kNarrowTiles ? kPrefixWaves * kPrefixChunk / 2 : kPrefixWaves * kPrefixChunk;
   l.per_block = 1024 * std::max(1, div_up(P, 1024 * most));
   l.blocks    = div_up(P, l.per_block);
-  l.bytes     = kBinsHeader + align_up((size_t) l.blocks * T * sizeof(uint32_t), 256);
+  l.bytes     = kBinsHeader + align_up((size_t) (l.blocks + 1) * T * sizeof(uint32_t), 256);
   return l;
 }
 
@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
       if (i < chunk && b < B) hist[(size_t) b * T + t] = run;
       run += c[i];
     }
-    if (wave == 0) ranges[2 * (size_t) t + 1] = total;
+    if (wave == 0) ranges[2 * (size_t) t + 1] = total, hist[(size_t) B * T + t] = (uint32_t) total;
   }
   if (wave == 0) {
     uint32_t all = t < T ? total : 0u;
@@ -454,24 +454,65 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
 
 // Step 3: the walk of step 1 again; a block's cursor of a tile starts at the tile's start plus the instances of the
 // blocks in front of it, so the placement needs no global atomics either.
+// scan_header: the tiles' totals have not been scanned yet. Every block does that for itself (up to kScanTiles, four a lane) and the
+// first one leaves ranges and header for the kernels behind: what tile_scan_kernel does, without a launch on the way. Its 4.2 us
+// and the gap behind it against 1.2 to 2.4 us more here: 300k surfels 800x800 420.9 -> 417.7 us a pass, 300k Gaussians 270.3 -> 265.9,
+// fast surfels 150k 1001x667 288 -> 284. Where one block does prefix and scan it is 1.5 us more than that block saves (10k 256x256,
+// 25k 639x361), and beyond kScanTiles every block would scan in several steps.
+constexpr int kScanTiles = 4096;
+
 template <int kMode, int kTiles>
 __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block, int gx, int gy, int64_t R,
     const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
-    WalkInputs in, const uint32_t* __restrict__ hist, const unsigned long long* __restrict__ ranges,
-    uint64_t* __restrict__ entries, int* __restrict__ order_table) {
+    WalkInputs in, const uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges,
+    uint64_t* __restrict__ entries, int* __restrict__ order_table, int* __restrict__ scan_header) {
   __shared__ unsigned s_cursor[kTiles];
+  const int T = gx * gy, B = (P + per_block - 1) / per_block;
+  const uint32_t* totals = hist + (size_t) B * T;
   // One block more than the walk needs, when the frame's blockIdx -> tile schedule is still to be built: the ranges are
   // final, nothing in this kernel reads the table, and the per-tile sorts and the blend kernels that follow do.
   if (order_table && blockIdx.x == gridDim.x - 1) {
     static_assert(sizeof(TileOrderLds) <= sizeof(s_cursor), "the schedule's LDS fits the cursor array");
-    build_tile_order(gx, gy, (const int64_t*) ranges, order_table, order_table + kMaxOrderedTiles,
-                     *reinterpret_cast<TileOrderLds*>(s_cursor));
+    TileOrderLds& lds = *reinterpret_cast<TileOrderLds*>(s_cursor);
+    if (scan_header) build_tile_order(gx, gy, [&](int t) { return (int64_t) totals[t]; }, order_table, order_table + kMaxOrderedTiles, lds);
+    else build_tile_order(gx, gy, [&](int t) { return (int64_t) (ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t]); }, order_table,
+                          order_table + kMaxOrderedTiles, lds);
     return;
   }
-  const int T = gx * gy;
-  if ((int64_t) ranges[2 * (size_t) T - 1] > R) return;  // the last tile's end: R was a guess, and too small (see gs_view_scatter)
-  const uint32_t* row = hist + (size_t) walk_row(blockIdx.x, (P + per_block - 1) / per_block) * T;
-  for (int t = threadIdx.x; t < T; t += blockDim.x) s_cursor[t] = (unsigned) ranges[2 * (size_t) t] + row[t];
+  const uint32_t* row = hist + (size_t) walk_row(blockIdx.x, B) * T;
+  if (scan_header) {
+    unsigned long long* s_wave = (unsigned long long*) &s_cursor[kTiles - 32];  // behind the cursors of kScanTiles tiles
+    const int lane = __lane_id(), wave = threadIdx.x / kWave, t0 = threadIdx.x * 4;
+    unsigned c[4], mine[4];
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = t0 + k < T ? totals[t0 + k] : 0u, mine[k] = t0 + k < T ? row[t0 + k] : 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum += c[k];
+    const unsigned long long inc = wave_inclusive_scan(sum);
+    if (lane == kWave - 1) s_wave[wave] = inc;
+    __syncthreads();
+    unsigned long long run = inc - sum, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const unsigned long long v = s_wave[w];
+      if (w < wave) run += v;
+      all += v;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (t0 + k < T) {
+        s_cursor[t0 + k] = (unsigned) run + mine[k];
+        if (blockIdx.x == 0) ranges[2 * (size_t) (t0 + k)] = run, ranges[2 * (size_t) (t0 + k) + 1] = run + c[k];
+      }
+      run += c[k];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) scan_header[0] = 0, scan_header[1] = (int) all;  // queue length | instances in all tiles
+    if ((int64_t) all > R) return;  // R was a guess, and too small (see gs_view_scatter)
+  } else {
+    if ((int64_t) ranges[2 * (size_t) T - 1] > R) return;  // the last tile's end
+    for (int t = threadIdx.x; t < T; t += blockDim.x) s_cursor[t] = (unsigned) ranges[2 * (size_t) t] + row[t];
+  }
   __syncthreads();
   const int first = blockIdx.x * per_block, last = min(P, first + per_block);
   const int rounds = (last - first + (int) blockDim.x - 1) / (int) blockDim.x;
@@ -1396,10 +1437,15 @@ namespace {
     }                                                                   \
   } while (0)
 
+// Who forms the tile ranges: the prefix kernel itself, the scatter (of a view), or tile_scan_kernel.
+bool scan_in_prefix(int T, int blocks) { return T <= 1024 && blocks <= kColumn; }
+bool scan_in_scatter(int T, int blocks) { return !scan_in_prefix(T, blocks) && T <= kScanTiles; }
+
 // First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
 // (start, end); the header of `bins` is set (length of the long-segment queue: 0 | instances in all tiles).
+// for_scatter: the scan may be left to the scatter (scan_in_scatter).
 int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in, int64_t* ranges,
-               void* bins, hipStream_t s, const SlotPublish& publish = SlotPublish{}) {
+               void* bins, hipStream_t s, bool for_scatter = false, const SlotPublish& publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
@@ -1413,12 +1459,13 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
       hipLaunchKernelGGL(kernel, dim3(bl.blocks), dim3(1024), 0, s, P, bl.per_block, gx, gy, (const float2*) means2D, radii, in,
                          hist, publish);
     });
-    if (T <= 1024 && bl.blocks <= kColumn) {
+    if (scan_in_prefix(T, bl.blocks)) {
       hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header);
     } else {
       hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
                          bl.blocks, hist, rng, sums);
-      hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
+      if (!for_scatter || !scan_in_scatter(T, bl.blocks))
+        hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
     }
     // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
     // sorts) is built from them by an extra block of the scatter, in the second part.
@@ -1438,7 +1485,7 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
 // Second part: scatter (depth bits << 32 | surfel) into the tile segments. R: what there is room for; `entries` is left as it is
 // where the instances are more (tile grids within kMaxLdsTiles, whose ranges are final).
 void fill_scatter(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
-                  int64_t R, int64_t* ranges, void* workspace, void* bins, hipStream_t s) {
+                  int64_t R, int64_t* ranges, void* workspace, void* bins, hipStream_t s, bool of_view = false) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   const int T  = gx * gy;
   unsigned long long* rng = (unsigned long long*) ranges;
@@ -1456,7 +1503,7 @@ void fill_scatter(int P, int W, int H, const float* means2D, const float* depths
       auto kernel = T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles> : tile_scatter_kernel<kMode, kNarrowTiles>;
       hipLaunchKernelGGL(kernel, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), alone, s, P, bl.per_block, gx, gy, R,
                          (const float2*) means2D, depths, radii, in, (const uint32_t*) ((const char*) bins + kBinsHeader), rng,
-                         entries, build);
+                         entries, build, of_view && scan_in_scatter(T, bl.blocks) ? (int*) bins : nullptr);
     });
   } else {
     FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, true>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy,
@@ -1695,7 +1742,7 @@ FSGS_API int fsgs_gs_view_count(int P, int W, int H, const float* means2D, const
     return fail(kWorkspaceSmall, "gs_view_count: bins %zu < %zu bytes", bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
   tile_order_invalidate((hipStream_t) stream);
   __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
-  return fill_count(P, W, H, means2D, radii, view_inputs(inverse_m, opacities, keep_masks), ranges, bins, (hipStream_t) stream,
+  return fill_count(P, W, H, means2D, radii, view_inputs(inverse_m, opacities, keep_masks), ranges, bins, (hipStream_t) stream, true,
                     SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
 }
 
@@ -1730,7 +1777,7 @@ FSGS_API int fsgs_gs_view_scatter(int P, int W, int H, const float* means2D, con
     return rc;
   if (!ranges_final_before_scatter(W, H)) return kOk;
   fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins,
-               (hipStream_t) stream);
+               (hipStream_t) stream, true);
   return check_launch("gs_view_scatter");
 }
 

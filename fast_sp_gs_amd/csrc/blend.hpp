@@ -270,9 +270,10 @@ struct TileOrderLds {
 // own (tile_order_kernel) or one extra block of a kernel that has nothing to do with it but runs at the right time --
 // the binning's scatter, whose other blocks keep the chip busy while this one orders 2 500 numbers (a single-block
 // launch of its own holds up the stream for 10 us).
-// `schedule` (optional) receives the ints behind the table.
-__device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* __restrict__ ranges,
-                                                 int* __restrict__ tile_order, int* __restrict__ schedule, TileOrderLds& lds) {
+// `length(t)`: entries of tile t. `schedule` (optional) receives the ints behind the table.
+template <typename Length>
+__device__ __forceinline__ void build_tile_order(int gx, int gy, Length length, int* __restrict__ tile_order,
+                                                 int* __restrict__ schedule, TileOrderLds& lds) {
   auto& s_count = lds.count;
   auto& s_total = lds.total;
   const int T = gx * gy;
@@ -281,7 +282,7 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
   __syncthreads();
   int entries = 0;
   for (int t = threadIdx.x; t < T; t += blockDim.x) {
-    const int64_t len = ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t];
+    const int64_t len = length(t);
     atomicAdd(&s_count[tile_region(t, gx, gy)][length_bucket(len)], 1);
     entries += (int) len;
   }
@@ -322,7 +323,7 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
   }
   for (int t = threadIdx.x; t < T; t += blockDim.x) {
     const int r       = tile_region(t, gx, gy);
-    const int64_t len = ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t];
+    const int64_t len = length(t);
     int k             = atomicAdd(&s_count[r][length_bucket(len)], 1);
     const int round   = k / kCusPerXcd;
     if ((round & 1) && round < kBalanceRounds && (round + 1) * kCusPerXcd <= s_total[r]) k = (2 * round + 1) * kCusPerXcd - 1 - k;
@@ -333,7 +334,7 @@ __device__ __forceinline__ void build_tile_order(int gx, int gy, const int64_t* 
 __global__ void __launch_bounds__(1024) tile_order_kernel(int gx, int gy, const int64_t* __restrict__ ranges,
                                                           int* __restrict__ tile_order, int* __restrict__ schedule) {
   __shared__ TileOrderLds lds;
-  build_tile_order(gx, gy, ranges, tile_order, schedule, lds);
+  build_tile_order(gx, gy, [&](int t) { return ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t]; }, tile_order, schedule, lds);
 }
 
 // Launch flags of the blend kernels: bit 0 = the tile table was built for this launch (T small enough; otherwise blocks

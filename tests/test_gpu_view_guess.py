@@ -163,3 +163,24 @@ def test_scatter_without_room_writes_nothing(gx, gy, P, device):
         assert (rc == 0) == (room == R)
     torch.cuda.synchronize()
     assert torch.equal(ranges, want_ranges) and torch.equal(point_list, want_list) and bool((space[size:] == 0xab).all())
+
+
+# around the grids whose ranges one block forms (1024 tiles, 65 536 surfels), the scatter itself, and a kernel of its own (from
+# 4097 tiles on); the last tile of a lane's four, and grids that end inside them
+@pytest.mark.parametrize('gx,gy,P', [(32, 32, 65_536), (32, 32, 65_537), (25, 41, 900), (61, 67, 2000), (64, 64, 2000), (17, 241, 2000)])
+def test_lists_of_a_view_are_the_operators(gx, gy, P, device, monkeypatch):
+    from fast_sp_gs_amd import scenes
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.renderer import gs_2d_render as m
+    W, H = 16 * gx - 3, 16 * gy - 5
+    s = scenes._surfels(torch.Generator().manual_seed(P), P, 'cube', -3.5 if P < 10_000 else -4.5, 0.7, 0.0, 1.5).to(device)
+    cam = scenes.pinhole(W, H, 50.0, torch.tensor([0.0, 0.0, 4.0])).to(device)
+    monkeypatch.setattr(m, 'CULL_LISTS', False)
+    m2, _, _, _, depths, radii, touched = get_C_function('gs_2d_preprocess_forward')(
+        W, H, 3, False, s.means3D, s.scales, s.rotations, s.opacities, s.shs, None, cam.Tw2v, cam.Tv2c, cam.campos, None, None, None)
+    want_ranges, want_list = get_C_function('GS_prepare')(W, H, m2, depths, radii, touched, False)[:2]
+    with torch.no_grad():
+        for _ in range(2):  # the second view's room is guessed
+            b = m.GS_2D_render(s.means3D, s.scales, s.rotations, s.opacities, (W, H), cam.Tw2v, cam.Tv2c, campos=cam.campos,
+                               sh_degree=3, near=0.2, far=100.0, sh_features=s.shs)['buffer']
+            assert torch.equal(b.tile_ranges, want_ranges) and torch.equal(b.point_list, want_list)
