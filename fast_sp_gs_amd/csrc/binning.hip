@@ -454,18 +454,18 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
 
 // Step 3: the walk of step 1 again; a block's cursor of a tile starts at the tile's start plus the instances of the
 // blocks in front of it, so the placement needs no global atomics either.
-// scan_header: the tiles' totals have not been scanned yet. Every block does that for itself (up to kScanTiles, four a lane) and the
+// kScan: the tiles' totals have not been scanned yet. Every block does that for itself (up to kScanTiles, four a lane) and the
 // first one leaves ranges and header for the kernels behind: what tile_scan_kernel does, without a launch on the way. Its 4.2 us
 // and the gap behind it against 1.2 to 2.4 us more here: 300k surfels 800x800 420.9 -> 417.7 us a pass, 300k Gaussians 270.3 -> 265.9,
 // fast surfels 150k 1001x667 288 -> 284. Where one block does prefix and scan it is 1.5 us more than that block saves (10k 256x256,
 // 25k 639x361), and beyond kScanTiles every block would scan in several steps.
 constexpr int kScanTiles = 4096;
 
-template <int kMode, int kTiles>
+template <int kMode, int kTiles, bool kScan>
 __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block, int gx, int gy, int64_t R,
     const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
     WalkInputs in, const uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges,
-    uint64_t* __restrict__ entries, int* __restrict__ order_table, int* __restrict__ scan_header) {
+    uint64_t* __restrict__ entries, int* __restrict__ order_table, int* __restrict__ header) {
   __shared__ unsigned s_cursor[kTiles];
   const int T = gx * gy, B = (P + per_block - 1) / per_block;
   const uint32_t* totals = hist + (size_t) B * T;
@@ -474,13 +474,13 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
   if (order_table && blockIdx.x == gridDim.x - 1) {
     static_assert(sizeof(TileOrderLds) <= sizeof(s_cursor), "the schedule's LDS fits the cursor array");
     TileOrderLds& lds = *reinterpret_cast<TileOrderLds*>(s_cursor);
-    if (scan_header) build_tile_order(gx, gy, [&](int t) { return (int64_t) totals[t]; }, order_table, order_table + kMaxOrderedTiles, lds);
+    if (kScan) build_tile_order(gx, gy, [&](int t) { return (int64_t) totals[t]; }, order_table, order_table + kMaxOrderedTiles, lds);
     else build_tile_order(gx, gy, [&](int t) { return (int64_t) (ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t]); }, order_table,
                           order_table + kMaxOrderedTiles, lds);
     return;
   }
   const uint32_t* row = hist + (size_t) walk_row(blockIdx.x, B) * T;
-  if (scan_header) {
+  if (kScan) {
     unsigned long long* s_wave = (unsigned long long*) &s_cursor[kTiles - 32];  // behind the cursors of kScanTiles tiles
     const int lane = __lane_id(), wave = threadIdx.x / kWave, t0 = threadIdx.x * 4;
     unsigned c[4], mine[4];
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
       }
       run += c[k];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) scan_header[0] = 0, scan_header[1] = (int) all;  // queue length | instances in all tiles
+    if (blockIdx.x == 0 && threadIdx.x == 0) header[0] = 0, header[1] = (int) all;  // queue length | instances in all tiles
     if ((int64_t) all > R) return;  // R was a guess, and too small (see gs_view_scatter)
   } else {
     if ((int64_t) ranges[2 * (size_t) T - 1] > R) return;  // the last tile's end
@@ -1498,12 +1498,14 @@ void fill_scatter(int P, int W, int H, const float* means2D, const float* depths
     (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
     // Entries that do not fit the dies' L2s (4 MB each) leave them in pieces, the smaller the more blocks write at once: LDS that
     // nobody uses keeps a second block off the compute unit. 3M surfels 1352x1014, 6M entries: 71 -> 56 us; 300k 800x800, 1.4M: 12.8 -> 13.9.
+    const bool scan = of_view && scan_in_scatter(T, bl.blocks);
     const size_t alone = T <= kNarrowTiles && R > (int64_t) 4 << 20 ? 32768 : 0;
     FSGS_BY_WALK_MODE(in, {
-      auto kernel = T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles> : tile_scatter_kernel<kMode, kNarrowTiles>;
+      auto kernel = scan ? tile_scatter_kernel<kMode, kNarrowTiles, true>
+                    : T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles, false> : tile_scatter_kernel<kMode, kNarrowTiles, false>;
       hipLaunchKernelGGL(kernel, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), alone, s, P, bl.per_block, gx, gy, R,
                          (const float2*) means2D, depths, radii, in, (const uint32_t*) ((const char*) bins + kBinsHeader), rng,
-                         entries, build, of_view && scan_in_scatter(T, bl.blocks) ? (int*) bins : nullptr);
+                         entries, build, (int*) bins);
     });
   } else {
     FSGS_BY_WALK_MODE(in, hipLaunchKernelGGL((tile_emit_kernel<kMode, true>), dim3(div_up(P, 256)), dim3(256), 0, s, P, gx, gy,
