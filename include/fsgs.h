@@ -758,7 +758,7 @@ int fsgs_image_loss_backward(int B, int CH, int H, int W, double lambda_dssim, c
 /* fsgs_image_loss_forward for callers that cannot allocate device memory or carry a workspace (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). It has no counterpart in the reference. Same inputs,
  * outputs and results as fsgs_image_loss_forward; the per-block partial sums go into a device array built into the
- * library (512 KiB per GPU, held until the process ends) instead of a workspace, so the call allocates nothing. Limit:
+ * library (2.5 MiB per GPU, held until the process ends) instead of a workspace, so the call allocates nothing. Limit:
  * B * ceil(W / 32) * ceil(H / 32) <= fsgs_image_loss_static_max_blocks() (65536: one 8192 x 8192 image); larger inputs
  * are rejected with an error. All calls on one GPU share that array: calls that overlap on one GPU (two streams, two
  * host threads) race; calls on one stream are ordered. Nothing in the array has to be cleared between calls. */
