@@ -20,7 +20,7 @@
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
 // short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.17 ms a call this way
 // (traced: lists 0.047, queries 0.118; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by vector issue (1090
-// instructions per 64 queries, 0.82 of the issue slots). With lists in index order and a row of results stored by each lane for itself
+// instructions per 64 queries, 0.7 of the issue slots) and LDS (half of the time, a fifth in bank conflicts). With lists in index order and a row of results stored by each lane for itself
 // it took 0.202 ms and 2180 instructions; in order alone 0.169, its memory path busy with stores of 16 bytes each; results through LDS in
 // runs of 512 and 1024 bytes 0.152, and past the caches, which then keep the lists (8 MB), 0.118.
 // 200 000 x 512, K = 4: 57 -> 24 us, 50 000 x 512, K = 3: 37 -> 19 us, 5 000 x 512, K = 4: 36 -> 10 us.
