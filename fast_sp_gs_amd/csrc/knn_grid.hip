@@ -155,6 +155,9 @@ __device__ __forceinline__ float widened(float bound2) { return bound2 * 1.00002
 __device__ __forceinline__ float cell_step(float scale) { return __builtin_amdgcn_rsqf(scale) * (2.0f * 65536.0f / 255.0f); }
 __device__ __forceinline__ float cell_centre(float lo, float hi) { return 0.5f * (lo + hi); }
 __device__ __forceinline__ float centre_distance(float x, float y, float z) { return __builtin_amdgcn_sqrtf(fmaf(x, x, fmaf(y, y, z * z))); }
+// Infinite where its square exceeds the floats, from 1.844e19 on: an entry of a list whose K nearest are still in reach may lie there.
+// As a lower bound it then says no more than this.
+constexpr float kFarthest = 1.84e19f;
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
   return (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) mask, 0u));
@@ -570,7 +573,8 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
 #pragma unroll
       for (int h = 0; h < kEntries; ++h) {
         if (kWave * h + lane < n[c]) list[c][kWave * h + lane] = (uint16_t) (key[h] & kNumberBits);
-        bound[h] = (uint32_t) fminf(__uint_as_float(key[h] & ~kNumberBits) * per_step, 255.0f);  // (of a place past the end: a NaN, 255)
+        // (of a place past the end, a NaN, any)
+        bound[h] = (uint32_t) fminf(fminf(__uint_as_float(key[h] & ~kNumberBits), kFarthest) * per_step, 255.0f);
       }
       auto at = [&](int g) { return (uint32_t) __builtin_amdgcn_readlane(bound[8 * g / kWave], 8 * g % kWave); };
 #pragma unroll

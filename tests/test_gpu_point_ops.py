@@ -368,6 +368,20 @@ def test_knn_ordered_lists(N, M, K, kind, device):
     assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
 
 
+# Coordinates so large that squared distances from a cell's centre exceed the floats while those of a query's neighbours do not: an
+# entry that lies infinitely far from the centre by its square may be a neighbour all the same.
+@pytest.mark.parametrize('N,M,K', [(200_003, 600, 3), (1_000_001, 700, 8)])
+@pytest.mark.parametrize('spread,scale', [('normal', 2e19), ('normal', 3e19), ('uniform', 5e19)])
+def test_knn_ordered_lists_of_huge_cells(N, M, K, spread, scale, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(N + M + K)
+    draw = (lambda n: torch.randn(n, 3, generator=g)) if spread == 'normal' else (lambda n: torch.rand(n, 3, generator=g) * 2 - 1)
+    pts, ctrl = draw(N) * scale, draw(M) * scale
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+
+
 def test_knn_clusters_keep_to_the_lists(device):
     """With the keys' coarse parts alone, tight clusters sent every query to the exact search: thirteen times the time."""
     g = torch.Generator().manual_seed(7)
