@@ -82,12 +82,19 @@ Scheme knn_scheme(int N, int M, int D, int K) {
 template <int kK, int kG>
 constexpr int64_t kOrderFrom = kG == 16 ? (kK >= 3 ? 0 : 400000) : kK == 1 ? INT64_MAX : 10000000 / (kK + 2);  // queries
 
-// A cell. `length`: how many candidates its list holds (or kLongList) and kCrowdedBit, and the first bound; `scale`: what takes a squared
-// distance to 2^32 at the cell's bound. Where the list is in the order of the distances from the cell's centre, byte g - 1 of the bounds
-// is a lower bound, in cell_step's, on the distances from the 8 g-th entry on; else they are 0. (The last one counts for what is behind it, too.)
+// A cell. `length`: how many candidates its list holds (or kLongList) and kCrowdedBit; `scale`: what takes a squared distance to 2^32 at
+// the cell's bound. Where the list is in the order of the distances from the cell's centre, byte g - 1 of the bounds, the first two of
+// which are the upper half of `length`, is a lower bound, in cell_step's, on the distances from the 8 g-th entry on (the last one counts
+// for what is behind it, too).
 constexpr int kBounds = 10;
-struct __attribute__((aligned(16))) Cell {
-  uint32_t length;  // bounds 0 and 1 in the upper half
+template <bool kOrder>
+struct Cell {
+  uint32_t length;
+  float scale;
+};
+template <>
+struct __attribute__((aligned(16))) Cell<true> {
+  uint32_t length;
   float scale;
   uint32_t bounds[2];
 };
@@ -101,7 +108,7 @@ GridLayout grid_layout(Scheme scheme) {
   const size_t cells = (size_t) l.G * l.G * l.G;
   l.planes  = 0;
   l.cells   = align_up(3 * (size_t) (l.G + 1) * 4, 256);
-  l.lists   = align_up(l.cells + cells * sizeof(Cell), 256);
+  l.lists   = align_up(l.cells + cells * sizeof(Cell<true>), 256);
   l.bytes   = l.lists + cells * kListCap * 2;
   return l;
 }
@@ -390,7 +397,7 @@ struct WaveSort {
 // and nothing waits in a chain of eight (cells one after the other: 25 us of the kernel's 51).
 template <int kG, bool kOrder>
 __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
-    float* __restrict__ planes, Cell* __restrict__ cells, uint16_t* __restrict__ lists) {
+    float* __restrict__ planes, Cell<kOrder>* __restrict__ cells, uint16_t* __restrict__ lists) {
   constexpr int kWaves = kBuildThreads / kWave;
   static_assert(kWaves == 8, "a wavefront per octant");
   __shared__ float4 s_y[kMaxPoints];
@@ -547,14 +554,14 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
       for (int h = 0; h < kEntries; ++h) held[c][h] = kWave * h + lane < min(n[c], kListCap) ? list[c][kWave * h + lane] : 0u;
   }
   // the walk takes eight entries at a time: the rest of the last eight is the point at infinity, number M
-  Cell cell[kCells];
+  Cell<kOrder> cell[kCells];
   const WaveSort sort;
 #pragma unroll
   for (int c = 0; c < kCells; ++c) {
     const bool fits = !too_many && n[c] <= kListCap && reach[c] < 3e38f;
     if (fits && lane < 8 && n[c] + lane < (n[c] + 7) / 8 * 8) list[c][n[c] + lane] = (uint16_t) M;
     // the K nearest of any query of the cell are nearer than `reach`: their parts stay below 2^32, the others' may saturate
-    cell[c] = Cell{fits ? (uint32_t) n[c] | (inside[c] >= kCrowded ? kCrowdedBit : 0u) : kLongList, fminf(4294967296.0f / reach[c], 3e38f), {}};
+    cell[c] = Cell<kOrder>{fits ? (uint32_t) n[c] | (inside[c] >= kCrowded ? kCrowdedBit : 0u) : kLongList, fminf(4294967296.0f / reach[c], 3e38f)};
     if constexpr (kOrder) {
       if (!fits || n[c] <= 8) continue;
       uint32_t key[kEntries];
@@ -677,7 +684,7 @@ __device__ __forceinline__ void store_results(float* __restrict__ dist2, int64_t
 template <int kK, int kG, bool kOrder>
 __global__ void __launch_bounds__(kQueryThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
 knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
-    const float* __restrict__ y, const float* __restrict__ planes, const Cell* __restrict__ cells,
+    const float* __restrict__ y, const float* __restrict__ planes, const Cell<kOrder>* __restrict__ cells,
     const uint16_t* __restrict__ lists, float* __restrict__ dist2, int64_t* __restrict__ index) {
   // 60 MB of results and more would push the lists out of the caches; fewer are left there for whoever asked
   constexpr bool kStream = kOrder && kG > 16;
@@ -794,11 +801,7 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         cell   = cell * kG + i;
         off[a] = q[a] - cell_centre(s_plane[a][i], s_plane[a][i + 1]);
       }
-      Cell here{kLongList, 0.0f, {}};
-      if (inside) {
-        if constexpr (kOrder) here = cells[cell];
-        else here.length = cells[cell].length, here.scale = cells[cell].scale;
-      }
+      const Cell<kOrder> here = inside ? cells[cell] : Cell<kOrder>{kLongList, 0.0f};
       const float far_off = kOrder ? 1.0001f * centre_distance(off[0], off[1], off[2]) : 0.0f, step = kOrder ? cell_step(here.scale) : 0.0f;
       const bool listed = (here.length & 0xffu) != kLongList;
       const uint16_t* list = lists + (size_t) cell * kListCap;
@@ -816,7 +819,8 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         uint4 next = n_list > 0 ? *(const uint4*) list : make_uint4(0, 0, 0, 0);
         int c = 0;
         unsigned long long longer;
-        uint32_t now_bounds = here.length >> 16, next_bounds = here.bounds[0], last_bounds = here.bounds[1];
+        uint32_t now_bounds = here.length >> 16, next_bounds = 0u, last_bounds = 0u;
+        if constexpr (kOrder) next_bounds = here.bounds[0], last_bounds = here.bounds[1];
         for (;; c += 8) {
           // An entry at distance d from the centre is at least d - far_off away: past the last one that can be among the smallest
           // keys the list is over.
@@ -920,7 +924,7 @@ void launch_query(int N, int M, const float* x, const float* y, const GridLayout
   const int per_block = kG > 0 ? kQueryThreads : kQueryThreads / kWave;
   const int blocks = std::min(div_up(N, per_block), 256 * 8);
   hipLaunchKernelGGL((knn_cell_query_kernel<kK, kG, kOrder>), dim3(blocks), dim3(kQueryThreads), lds, s, N, M, x, y,
-                     (const float*) (ws + l.planes), (const Cell*) (ws + l.cells), (const uint16_t*) (ws + l.lists),
+                     (const float*) (ws + l.planes), (const Cell<kOrder>*) (ws + l.cells), (const uint16_t*) (ws + l.lists),
                      dist2, index);
 }
 
@@ -932,7 +936,7 @@ int launch_grid_knn(Scheme scheme, int N, int M, const float* x, const float* y,
     constexpr int kG = decltype(grid)::value;
     constexpr bool kOrder = decltype(order)::value;
     hipLaunchKernelGGL((knn_cell_lists_kernel<kG, kOrder>), dim3(kCoarse * kCoarse * kCoarse), dim3(kBuildThreads), 0, s, M, kK, y,
-                       (float*) (ws + l.planes), (Cell*) (ws + l.cells), (uint16_t*) (ws + l.lists));
+                       (float*) (ws + l.planes), (Cell<kOrder>*) (ws + l.cells), (uint16_t*) (ws + l.lists));
     launch_query<kK, kG, kOrder>(N, M, x, y, l, ws, dist2, index, s);
   };
   auto launch_grid = [&](auto grid) {
