@@ -75,12 +75,28 @@ Scheme knn_scheme(int N, int M, int D, int K) {
 }
 
 // Whether the lists are put in the order of the distances from their cell's centre, so that a query's walk is over after half of its
-// list (below). It costs 10 us with G = 32, whatever the number of queries, and saves 9 ns a thousand queries at K = 8, 1 at K = 1; with G = 16 it
-// costs less than 1 us. M = 2048, us in index order -> in this one: K = 8, N = 500 000 73.6 -> 78.6, 1M 93.4 -> 89.5, 3M 193 -> 167; K = 4, 500 000
-// 63.1 -> 69.5, 1.5M 86.6 -> 85.0, 3M 145 -> 132; K = 1, 3M 111.5 -> 107.9, M = 1024 83.7 -> 86.8. M = 600 (G = 16), 200 000: K = 8 47.7 -> 45.1, K = 1
-// 34.3 -> 33.3; M = 200, 50 000: K = 4 24.2 -> 24.2, K = 1 21.1 -> 22.1.
+// list (below). With G = 32 that costs 4 to 8 us whatever the number of queries, with G = 16 1 us; what it saves grows with the queries,
+// with K and with the length of the lists, that is, with M. Past about 200 MB of results the stores past the caches, which come with
+// the order (kStream), outweigh that. us a call in index order -> in this one, queries in a ball | normal (what two runs differ by: 1 to 3):
+//   G = 32, K = 8, M = 2048:  500 000 59 -> 59 | 79 -> 82;  1M 81 -> 76 | 104 -> 100;  3M 183 -> 131 | 204 -> 154
+//           K = 8, M = 256:   1.7M 75 -> 77 | 86 -> 89;  2.5M 124 -> 99 | 136 -> 114
+//           K = 4, M = 400 (640): 1.7M 58.1 -> 59.7 | 68.7 -> 67.9 (62.5 -> 61.9 | 72.5 -> 71.4)
+//           K = 3, M = 640 (1024): 2.1M 65.2 -> 67.4 | 78.6 -> 78.2 (70.2 -> 69.2 | 82.4 -> 81.2)
+//           K = 2, 2.5M: M = 640 64.6 -> 69.6 | 76.5 -> 80.1;  1400 71.4 -> 75.3 | 89.3 -> 87.9;  2048 80.1 -> 77.3 | 100 -> 93
+//           K = 1, 3M: M = 1024 67.4 -> 69.1 | 79.6 -> 81.3;  2048 78.5 -> 78.7 | 102.5 -> 97.9
+//   G = 16, K = 3, M = 512: 50 000 17.8 -> 17.2 | 27.8 -> 27.1;  K = 1: 50 000 16.4 -> 16.2 | 23.2 -> 22.8;  400 000 22.0 -> 20.6 | 29.9 -> 27.7;
+//           K = 1, M = 256: 120 000 15.2 -> 15.4 | 21.5 -> 21.8;  400 000 20.1 -> 19.2 | 26.7 -> 26.1
 template <int kK, int kG>
-constexpr int64_t kOrderFrom = kG == 16 ? (kK >= 3 ? 0 : 400000) : kK == 1 ? INT64_MAX : 10000000 / (kK + 2);  // queries
+constexpr bool kAlwaysOrdered = kG == 16 && kK >= 3;
+template <int kK, int kG>
+constexpr bool kNeverOrdered = kG == 32 && kK == 1;
+template <int kK, int kG>
+bool lists_in_order(int64_t N, int M) {
+  if (kG == 16) return N >= 400000;
+  const int64_t results = N * (kK + 2), entries = M * (kK + 2);
+  if (kK == 2) return results >= 10000000 && M >= 1400;
+  return results >= (entries >= 3800 ? 10000000 : 20000000);
+}
 
 // A cell. `length`: how many candidates its list holds (or kLongList) and kCrowdedBit; `scale`: what takes a squared distance to 2^32 at
 // the cell's bound. Where the list is in the order of the distances from the cell's centre, byte g - 1 of the bounds, the first two of
@@ -940,10 +956,10 @@ int launch_grid_knn(Scheme scheme, int N, int M, const float* x, const float* y,
     launch_query<kK, kG, kOrder>(N, M, x, y, l, ws, dist2, index, s);
   };
   auto launch_grid = [&](auto grid) {
-    constexpr int64_t kFrom = kOrderFrom<kK, decltype(grid)::value>;
-    if constexpr (kFrom == 0) launch(grid, std::true_type());
-    else if constexpr (kFrom == INT64_MAX) launch(grid, std::false_type());
-    else if (N >= kFrom) launch(grid, std::true_type());
+    constexpr int kG = decltype(grid)::value;
+    if constexpr (kAlwaysOrdered<kK, kG>) launch(grid, std::true_type());
+    else if constexpr (kNeverOrdered<kK, kG>) launch(grid, std::false_type());
+    else if (lists_in_order<kK, kG>(N, M)) launch(grid, std::true_type());
     else launch(grid, std::false_type());
   };
   if (scheme == kAlone) launch_query<kK, 0, false>(N, M, x, y, l, ws, dist2, index, s);
