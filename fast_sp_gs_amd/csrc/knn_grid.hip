@@ -704,6 +704,9 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
     const uint16_t* __restrict__ lists, float* __restrict__ dist2, int64_t* __restrict__ index) {
   // 60 MB of results and more would push the lists out of the caches; fewer are left there for whoever asked
   constexpr bool kStream = kOrder && kG > 16;
+  // Short rows behind long walks are stored by their lanes: by way of LDS, lists in index order, K = 3 took 1.2 % longer (1M x 1024
+  // 47.5 -> 48.9 us), K = 4 as long; K = 8 3 % less (800 000 x 700 59.9 -> 56.6).
+  constexpr bool kRuns = kK > (kOrder ? 2 : 4);
   // a query alone costs a wavefront about 20 M / 64 + 300 instructions, the all-pairs walk about 20 M for all 64
   const int max_alone = 20 * M / (20 * M / 64 + 300);
   constexpr int kWaves = kQueryThreads / kWave;
@@ -910,8 +913,8 @@ knn_cell_query_kernel(int N, int M, const float* __restrict__ x,
         bi[k] = unknown ? M : (int) (key[k] & kNumberBits);
         bd[k] = distance2(q[0], q[1], q[2], s_y[bi[k]]);
       }
-      if (kK > 2 && wave_ballot(live && !unknown) == ~0ull) {
-        if constexpr (kK > 2) store_results<kK, kStream>(dist2, index, n0, bd, bi, s_cand_d);
+      if (kRuns && wave_ballot(live && !unknown) == ~0ull) {
+        if constexpr (kRuns) store_results<kK, kStream>(dist2, index, n0, bd, bi, s_cand_d);
       } else if (live && !unknown) {
         store_result<kK>(dist2, index, n, bd, bi);
       }
