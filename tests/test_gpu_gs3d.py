@@ -142,6 +142,35 @@ def test_gs3d_rasterize(P, W, H, E, device):
         assert not a[_binned.radii <= 0].any()
 
 
+@pytest.mark.parametrize("E,seed,conic,opacity", [(0, 31, 1.35, 1.5), (0, 32, 1.35, 1.5), (4, 31, 1.1, 1.2)])
+def test_gs3d_backward_error_of_uniform_gradients(E, seed, conic, opacity, device):
+    """What rounding leaves in the gradients of conics and opacities when the upstream gradient is the same for every pixel and
+    channel: a rounding that depends on the Gaussian alone then repeats in all its pixels and averages out nowhere. The
+    yardstick is the oracle's recurrence per channel in single precision, with true divisions, against double precision
+    (geometric mean of the rows' relative errors). An accumulator per channel: 1.24 to 1.25 and 1.33 to 1.36 times the oracle's (1.00 and
+    1.05 with E = 4); one sum over the channels of a Gaussian, whose rounding repeats: 1.46 to 1.48 and 1.65 to 1.68 (1.13, 1.27)."""
+    from fast_sp_gs_amd._C import get_C_function
+    P, W, H = 20000, 128, 128
+    m2, col, co, ranges, pl = _binned(P, W, H, seed, device)
+    g = torch.Generator().manual_seed(seed)
+    ex = torch.randn(P, E, generator=g).to(device) if E else None
+    _, oo, _, nc = get_C_function('gaussian_rasterize_forward')(W, H, m2, co, col, ex, pl, ranges, None, None, None)
+    gi, go = torch.ones(3, H, W, device=device), torch.zeros(H, W, device=device)
+    ge = torch.ones(E, H, W, device=device) if E else None
+    got = npy(get_C_function('gaussian_rasterize_backward')(m2, co, col, ex, oo, gi, go, ge, ranges, pl, nc, _binned.offsets,
+                                                            _binned.radii)[3])
+    n = lambda t, dt: None if t is None else npy(t).astype(dt) if t.is_floating_point() else npy(t)
+    single, double = (O.gs3d_render_backward(W, H, *[n(t, dt) for t in (m2, co, col, ex, oo, nc, gi, ge, go, pl, ranges)])[3]
+                      for dt in (np.float32, np.float64))
+
+    def error(v, c):
+        norm = np.linalg.norm(double[:, c], axis=1)
+        rel = np.linalg.norm(v[:, c].astype(np.float64) - double[:, c], axis=1)[norm > 0] / norm[norm > 0]
+        return np.exp(np.log(np.maximum(rel, 1e-10)).mean())
+    for c, most in ((slice(0, 3), conic), (slice(3, 4), opacity)):
+        assert error(got, c) < most * error(single, c), (c, error(got, c) / error(single, c))
+
+
 @pytest.mark.parametrize("K", [1, 4, 7, 16])
 def test_gs3d_topk_weights(K, device):
     from fast_sp_gs_amd._C import get_C_function
