@@ -212,16 +212,17 @@ ssim_forward_kernel(int H, int W, int CH, int tiles_x, bool pairs, float C1, flo
     for (int q = 0; q < kLaneOut; ++q) {
 #pragma clang fp contract(off)  // the same numbers in all forms of the kernel
       const float m1 = mu1[q], m2 = mu2[q];
-      const float mu_sq = fmaf(m1, m1, m2 * m2), sigma_sq = fmaf(-m1, m1, e11[q]) + fmaf(-m2, m2, e22[q]);
+      const float mu_sq = m1 * m1 + m2 * m2, sigma_sq = fmaf(-m1, m1, e11[q]) + fmaf(-m2, m2, e22[q]);
       const float C = fmaf(2.0f, m1 * m2, C1), D = fmaf(2.0f, fmaf(-m1, m2, e12[q]), C2);
       const float A = mu_sq + C1, B = sigma_sq + C2;
-      // SSIM = CD / (AB); its derivatives over the one quotient: 1 / B = A / (AB), 1 / B - 1 / A = (A - B) / (AB)
-      const float r = 1.0f / (A * B);
-      map[q] = C * D * r;
+      // SSIM = CD / (AB) as one rounded quotient: of images that are alike exactly 1, and finite where 1 / (AB) is not. The derivatives
+      // with reciprocals of either factor for the same reason, and 1 / B - 1 / A = (A - B) / (AB).
+      map[q] = (C * D) / (A * B);
       if (kTrain) {
-        by_mu1[q] = 2.0f * r * fmaf(m2, D - C, m1 * ((A - B) * map[q]));
-        by_var[q] = -map[q] * (A * r);
-        by_cov[q] = 2.0f * C * r;
+        const float rA = __builtin_amdgcn_rcpf(A), rB = __builtin_amdgcn_rcpf(B);
+        by_mu1[q] = 2.0f * fmaf(m2, D - C, m1 * ((A - B) * map[q])) * rA * rB;
+        by_var[q] = -map[q] * rB;
+        by_cov[q] = 2.0f * C * rA * rB;
       }
       if (kLoss && t.writes && t.x0 + t.first + q < W) sum_ssim += map[q];
     }

@@ -161,3 +161,32 @@ def test_ssim_tile_edges(shape, shift, device, oracle_mod):
     assert O.call("fusedssim_backward_f32", B, CH, H, W, a, b, np.full_like(a, -0.3 / n), npy(d1), npy(d2), npy(d3), rl) == 0
     want = rl.astype(np.float64) + 0.7 / n * np.sign(a.astype(np.float64) - b)
     assert rel_err(npy(leaf.grad), want.astype(np.float32)) < 1e-4
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 71, 130), (2, 1, 40, 55)])
+def test_ssim_of_images_that_are_alike(shape, device):
+    """Numerator and denominator of an image with itself are the same number: the map is 1 everywhere, in every form, and the loss 0."""
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.ssim import l1_dssim_loss
+    g = torch.Generator().manual_seed(shape[2])
+    for image in (torch.rand(*shape, generator=g), torch.full(shape, 0.3), torch.zeros(shape)):
+        x = image.to(device)
+        for train in (False, True):
+            assert bool((get_C_function('fusedssim')(0.01 ** 2, 0.03 ** 2, x, x.clone(), train)[0] == 1).all())
+        # 1 - (sum of n ones) * (1 / n), where 1 / n is rounded
+        assert abs(float(l1_dssim_loss(x, x.clone(), 1.0))) <= 2.0 ** -23
+
+
+@pytest.mark.parametrize("scale,tol", [(3e-10, 1e-3), (1e-9, 1e-5), (1e-8, 1e-5), (1e4, 1e-5), (1e9, 1e-5)])
+def test_ssim_scales_with_its_images(scale, tol, device):
+    """SSIM does not change when images are multiplied by s and the constants by s^2, its derivatives go with 1 / s and 1 / s^2: also where
+    the reciprocal of the denominator, which goes with s^4, is out of the floats' range. There the denominator itself, 1e-3 s^4 and more
+    (the filter's corners), is a subnormal number of 2^-149 parts: 1.7e-4 of it twice. Elsewhere some tens of roundings."""
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(3)
+    a, b = torch.rand(1, 3, 64, 80, generator=g).to(device), torch.rand(1, 3, 64, 80, generator=g).to(device)
+    call = lambda s: get_C_function('fusedssim')(0.01 ** 2 * s * s, 0.03 ** 2 * s * s, a * s, b * s, True)
+    want, got = call(1.0), call(scale)
+    for k, power in enumerate((0, 1, 2, 2)):
+        w, v = want[k].double(), got[k].double() * scale ** power
+        assert bool(torch.isfinite(v).all()) and float((v - w).abs().max()) < tol * float(w.abs().max()), k
