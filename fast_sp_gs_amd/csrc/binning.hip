@@ -341,7 +341,8 @@ __global__ void __launch_bounds__(256) cull_mask_kernel(int P, int gx, int gy, c
 // Layout of the `bins` buffer of the bucket binning: the queue length of the long segments in front of the B x T matrix
 // of per-(walk block, tile) instance counts, whose last row holds the tiles' totals.
 constexpr int kPrefixTiles = 64, kPrefixWaves = 16, kPrefixChunk = 32;  // walk blocks <= kPrefixWaves * kPrefixChunk
-constexpr size_t kBinsSums = 256;  // behind the queue length: the instances of every 64 tiles
+constexpr int kUnscanned   = 2;    // in front of it, behind the queue's length and the instances in all tiles (see tile_prefix_kernel)
+constexpr size_t kBinsSums = 256;  // the instances of every 64 tiles
 constexpr size_t kBinsHeader = 4096;
 static_assert(kBinsSums + (kMaxLdsTiles / kPrefixTiles) * sizeof(uint32_t) <= kBinsHeader, "the sums fit the header");
 struct BinsLayout {
@@ -402,11 +403,14 @@ __global__ void __launch_bounds__(1024) tile_hist_kernel(int P, int per_block, i
   for (int t = threadIdx.x; t < T; t += blockDim.x) row[t] = s_count[t];
 }
 
-// Step 2: per tile, the exclusive prefix of its column over the walk blocks (in place) and the column total, which goes
-// to ranges[t].y for tile_scan_kernel, and the sum over the block's tiles to sums[blockIdx.x]. 64 tiles per block, lane = tile, the 16 wavefronts share the walk blocks in
-// contiguous chunks so that a wavefront's loads are all in flight at once.
+// Step 2: per tile, the exclusive prefix of its column over the walk blocks (in place), the column total, which goes to the row
+// behind the blocks' and to ranges[t] (an empty range there) for tile_scan_kernel, and the sum over the block's tiles to
+// sums[blockIdx.x]. header[kUnscanned]: whether the scan of the totals is left to the scatter. 64 tiles per block, lane = tile, the
+// 16 wavefronts share the walk blocks in contiguous chunks so that a wavefront's loads are all in flight at once.
 __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kernel(int T, int B,
-    uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges, uint32_t* __restrict__ sums) {
+    uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges, uint32_t* __restrict__ sums, int* __restrict__ header,
+    bool unscanned) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) header[kUnscanned] = unscanned;
   __shared__ uint32_t s_sum[kPrefixWaves][kPrefixTiles];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = blockIdx.x * kPrefixTiles + lane;
@@ -442,7 +446,7 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
       if (i < chunk && b < B) hist[(size_t) b * T + t] = run;
       run += c[i];
     }
-    if (wave == 0) ranges[2 * (size_t) t + 1] = total, hist[(size_t) B * T + t] = (uint32_t) total;
+    if (wave == 0) ranges[2 * (size_t) t] = ranges[2 * (size_t) t + 1] = total, hist[(size_t) B * T + t] = total;
   }
   if (wave == 0) {
     uint32_t all = t < T ? total : 0u;
@@ -454,14 +458,16 @@ __global__ void __launch_bounds__(kPrefixTiles * kPrefixWaves) tile_prefix_kerne
 
 // Step 3: the walk of step 1 again; a block's cursor of a tile starts at the tile's start plus the instances of the
 // blocks in front of it, so the placement needs no global atomics either.
-// kScan: the tiles' totals have not been scanned yet. Every block does that for itself (up to kScanTiles, four a lane) and the
-// first one leaves ranges and header for the kernels behind: what tile_scan_kernel does, without a launch on the way. Its 4.2 us
-// and the gap behind it against 1.2 to 2.4 us more here: 300k surfels 800x800 420.9 -> 417.7 us a pass, 300k Gaussians 270.3 -> 265.9,
+// kScan: whether the tiles' totals have still to be scanned, always, never, or where the header says so (a binning begun by the count
+// of a view and ended by the operators; asking takes 0.4 us, 300k surfels with whole lists 16.9 -> 17.3). Every block does that for
+// itself (up to kScanTiles, four a lane) and the first one leaves ranges and header for the kernels behind: what tile_scan_kernel does,
+// without a launch on the way. Its 4.2 us and the gap behind it against 1.2 to 2.4 us more here: 300k surfels 800x800 420.9 -> 417.7 us a pass, 300k Gaussians 270.3 -> 265.9,
 // fast surfels 150k 1001x667 288 -> 284. Where one block does prefix and scan it is 1.5 us more than that block saves (10k 256x256,
 // 25k 639x361), and beyond kScanTiles every block would scan in several steps.
 constexpr int kScanTiles = 4096;
+enum ScanInScatter { kScanned, kToScan, kAskHeader };
 
-template <int kMode, int kTiles, bool kScan>
+template <int kMode, int kTiles, ScanInScatter kScan>
 __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block, int gx, int gy, int64_t R,
     const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
     WalkInputs in, const uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges,
@@ -469,18 +475,26 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
   __shared__ unsigned s_cursor[kTiles];
   const int T = gx * gy, B = (P + per_block - 1) / per_block;
   const uint32_t* totals = hist + (size_t) B * T;
-  // One block more than the walk needs, when the frame's blockIdx -> tile schedule is still to be built: the ranges are
+  // One block more than the walk needs, when the frame's blockIdx -> tile schedule is still to be built: the tiles' totals are
   // final, nothing in this kernel reads the table, and the per-tile sorts and the blend kernels that follow do.
   if (order_table && blockIdx.x == gridDim.x - 1) {
     static_assert(sizeof(TileOrderLds) <= sizeof(s_cursor), "the schedule's LDS fits the cursor array");
     TileOrderLds& lds = *reinterpret_cast<TileOrderLds*>(s_cursor);
-    if (kScan) build_tile_order(gx, gy, [&](int t) { return (int64_t) totals[t]; }, order_table, order_table + kMaxOrderedTiles, lds);
+    if (kScan != kScanned) build_tile_order(gx, gy, [&](int t) { return (int64_t) totals[t]; }, order_table, order_table + kMaxOrderedTiles, lds);
     else build_tile_order(gx, gy, [&](int t) { return (int64_t) (ranges[2 * (size_t) t + 1] - ranges[2 * (size_t) t]); }, order_table,
                           order_table + kMaxOrderedTiles, lds);
     return;
   }
   const uint32_t* row = hist + (size_t) walk_row(blockIdx.x, B) * T;
-  if (kScan) {
+  bool scan = kScan == kToScan;
+  if (kScan != kToScan) {
+    // on its way with the cursors of the other case. Not cleared in here: other blocks read it, and the next count sets it
+    if (kScan == kAskHeader) scan = header[kUnscanned] != 0;
+    if ((int64_t) ranges[2 * (size_t) T - 1] > R && !scan) return;  // the last tile's end
+    for (int t = threadIdx.x; t < T; t += blockDim.x) s_cursor[t] = (unsigned) ranges[2 * (size_t) t] + row[t];
+    __syncthreads();
+  }
+  if (scan) {
     unsigned long long* s_wave = (unsigned long long*) &s_cursor[kTiles - 32];  // behind the cursors of kScanTiles tiles
     const int lane = __lane_id(), wave = threadIdx.x / kWave, t0 = threadIdx.x * 4;
     unsigned c[4], mine[4];
@@ -509,11 +523,8 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) header[0] = 0, header[1] = (int) all;  // queue length | instances in all tiles
     if ((int64_t) all > R) return;  // R was a guess, and too small (see gs_view_scatter)
-  } else {
-    if ((int64_t) ranges[2 * (size_t) T - 1] > R) return;  // the last tile's end
-    for (int t = threadIdx.x; t < T; t += blockDim.x) s_cursor[t] = (unsigned) ranges[2 * (size_t) t] + row[t];
+    __syncthreads();
   }
-  __syncthreads();
   const int first = blockIdx.x * per_block, last = min(P, first + per_block);
   const int rounds = (last - first + (int) blockDim.x - 1) / (int) blockDim.x;
   for (int r = 0; r < rounds; ++r) {
@@ -1437,13 +1448,13 @@ namespace {
     }                                                                   \
   } while (0)
 
-// Who forms the tile ranges: the prefix kernel itself, the scatter (of a view), or tile_scan_kernel.
+// Who forms the tile ranges: the prefix kernel itself, the scatter (behind the count of a view), or tile_scan_kernel.
 bool scan_in_prefix(int T, int blocks) { return T <= 1024 && blocks <= kColumn; }
 bool scan_in_scatter(int T, int blocks) { return !scan_in_prefix(T, blocks) && T <= kScanTiles; }
 
 // First part of the bucket binning, independent of the instance count: per-tile instance counts and the tile ranges
 // (start, end); the header of `bins` is set (length of the long-segment queue: 0 | instances in all tiles).
-// for_scatter: the scan may be left to the scatter (scan_in_scatter).
+// for_scatter: the scan, and with it ranges and header, may be left to the scatter (scan_in_scatter); the ranges are empty till then.
 int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, const WalkInputs& in, int64_t* ranges,
                void* bins, hipStream_t s, bool for_scatter = false, const SlotPublish& publish = SlotPublish{}) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
@@ -1462,12 +1473,13 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
     if (scan_in_prefix(T, bl.blocks)) {
       hipLaunchKernelGGL(tile_prefix_scan_kernel, dim3(1), dim3(1024), 0, s, T, bl.blocks, hist, rng, header);
     } else {
+      const bool unscanned = for_scatter && scan_in_scatter(T, bl.blocks);
       hipLaunchKernelGGL(tile_prefix_kernel, dim3(div_up(T, kPrefixTiles)), dim3(kPrefixTiles * kPrefixWaves), 0, s, T,
-                         bl.blocks, hist, rng, sums);
-      if (!for_scatter || !scan_in_scatter(T, bl.blocks))
+                         bl.blocks, hist, rng, sums, header, unscanned);
+      if (!unscanned)
         hipLaunchKernelGGL(tile_scan_kernel, dim3(div_up(T, 4096)), dim3(1024), 0, s, T, rng, sums, header, true);
     }
-    // The ranges are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
+    // The tiles' totals are final here; the schedule table the blend kernels of this frame are going to use (and the per-tile
     // sorts) is built from them by an extra block of the scatter, in the second part.
   } else {
     // no room for one LDS counter per tile (or no surfels): count straight into ranges[t].y, then scan to (start, start)
@@ -1483,7 +1495,7 @@ int fill_count(int P, int W, int H, const float* means2D, const int32_t* radii, 
 }
 
 // Second part: scatter (depth bits << 32 | surfel) into the tile segments. R: what there is room for; `entries` is left as it is
-// where the instances are more (tile grids within kMaxLdsTiles, whose ranges are final).
+// where the instances are more (tile grids within kMaxLdsTiles, whose cursors are not the ranges).
 void fill_scatter(int P, int W, int H, const float* means2D, const float* depths, const int32_t* radii, const WalkInputs& in,
                   int64_t R, int64_t* ranges, void* workspace, void* bins, hipStream_t s, bool of_view = false) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
@@ -1492,17 +1504,18 @@ void fill_scatter(int P, int W, int H, const float* means2D, const float* depths
   uint64_t* entries       = sort_keys_in(R, workspace);
   const BinsLayout bl = bins_layout(P, T);
   if (bl.blocks > 0) {
-    // The schedule table is built by one extra block of the scatter (the ranges are final since the counting part).
+    // The schedule table is built by one extra block of the scatter (the tiles' totals are final since the counting part).
     const int* order = nullptr;
     int* build       = nullptr;
     (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
     // Entries that do not fit the dies' L2s (4 MB each) leave them in pieces, the smaller the more blocks write at once: LDS that
     // nobody uses keeps a second block off the compute unit. 3M surfels 1352x1014, 6M entries: 71 -> 56 us; 300k 800x800, 1.4M: 12.8 -> 13.9.
-    const bool scan = of_view && scan_in_scatter(T, bl.blocks);
+    const ScanInScatter scan = !scan_in_scatter(T, bl.blocks) ? kScanned : of_view ? kToScan : kAskHeader;
     const size_t alone = T <= kNarrowTiles && R > (int64_t) 4 << 20 ? 32768 : 0;
     FSGS_BY_WALK_MODE(in, {
-      auto kernel = scan ? tile_scatter_kernel<kMode, kNarrowTiles, true>
-                    : T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles, false> : tile_scatter_kernel<kMode, kNarrowTiles, false>;
+      auto kernel = scan == kToScan ? tile_scatter_kernel<kMode, kNarrowTiles, kToScan>
+                    : scan == kAskHeader ? tile_scatter_kernel<kMode, kNarrowTiles, kAskHeader>
+                    : T > kNarrowTiles ? tile_scatter_kernel<kMode, kMaxLdsTiles, kScanned> : tile_scatter_kernel<kMode, kNarrowTiles, kScanned>;
       hipLaunchKernelGGL(kernel, dim3(bl.blocks + (build ? 1 : 0)), dim3(1024), alone, s, P, bl.per_block, gx, gy, R,
                          (const float2*) means2D, depths, radii, in, (const uint32_t*) ((const char*) bins + kBinsHeader), rng,
                          entries, build, (int*) bins);
@@ -1764,7 +1777,7 @@ int check_view_lists(const char* what, int P, int W, int H, const float* means2D
                 fsgs_gs_view_lists_workspace_bytes(capacity), bins_bytes, fsgs_gs_prepare_bins_bytes(P, W, H));
   return kOk;
 }
-bool ranges_final_before_scatter(int W, int H) {
+bool scatter_can_repeat(int W, int H) {
   return (int64_t) ((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile) <= kMaxLdsTiles;
 }
 }  // namespace
@@ -1777,7 +1790,7 @@ FSGS_API int fsgs_gs_view_scatter(int P, int W, int H, const float* means2D, con
   if (int rc = check_view_lists("gs_view_scatter", P, W, H, means2D, inverse_m, depths, opacities, radii, keep_masks, capacity,
                                 ranges, bins, bins_bytes, workspace, workspace_bytes))
     return rc;
-  if (!ranges_final_before_scatter(W, H)) return kOk;
+  if (!scatter_can_repeat(W, H)) return kOk;
   fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins,
                (hipStream_t) stream, true);
   return check_launch("gs_view_scatter");
@@ -1797,7 +1810,7 @@ FSGS_API int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const 
   if (int rc = check_view_lists("gs_view_sort", P, W, H, means2D, inverse_m, depths, opacities, radii, keep_masks, capacity, ranges,
                                 bins, bins_bytes, workspace, workspace_bytes))
     return rc;
-  if (!ranges_final_before_scatter(W, H))
+  if (!scatter_can_repeat(W, H))
     fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins, s);
   fill_sort(P, W, H, capacity, ranges, point_list, nullptr, workspace, bins, false, s);
   return check_launch("gs_view_sort");

@@ -145,7 +145,9 @@ int fsgs_gs_prepare_fill_counted_culled(int P, int W, int H, const float* means2
  * Gaussians (inverse_m and opacities nullptr, keep_masks optional) and for the "fast" surfels (tiles that pass the corner test; all
  * three given).
  * fsgs_gs_view_count: per-tile counts. Its first block writes slot_regions[64] (optional), zeroes slot_counters and stores
- * the instance count to num_rendered_host (pinned memory, set to -1 here); fsgs_gs_view_wait returns once it is there.
+ * the instance count to num_rendered_host (pinned memory, set to -1 here); fsgs_gs_view_wait returns once it is there. `ranges` holds
+ * empty ranges or the final ones, by the size of the tile grid; what comes next fills them in: fsgs_gs_view_scatter, or one of the
+ * fsgs_gs_prepare_fill_counted calls.
  * fsgs_gs_view_scatter puts the instances into `workspace` (fsgs_gs_view_lists_workspace_bytes(capacity) bytes), which has room for
  * `capacity` of them: the count, or a guess made before it is known, so that the device is busy while the host waits. If there
  * are more instances than that it writes nothing, and is called again with the count.

@@ -184,3 +184,39 @@ def test_lists_of_a_view_are_the_operators(gx, gy, P, device, monkeypatch):
             b = m.GS_2D_render(s.means3D, s.scales, s.rotations, s.opacities, (W, H), cam.Tw2v, cam.Tv2c, campos=cam.campos,
                                sh_degree=3, near=0.2, far=100.0, sh_features=s.shs)['buffer']
             assert torch.equal(b.tile_ranges, want_ranges) and torch.equal(b.point_list, want_list)
+
+
+# the same sides of those lines
+@pytest.mark.parametrize('gx,gy,P', [(32, 32, 65_536), (32, 32, 65_537), (25, 41, 900), (61, 67, 2000), (64, 64, 2000), (17, 241, 2000)])
+def test_operators_end_what_the_count_of_a_view_began(gx, gy, P, device):
+    """The C entries: `fsgs_gs_view_count`, then `fsgs_gs_prepare_fill_counted` instead of scatter and sort of a view, twice. The count
+    leaves empty ranges where the scatter forms them, which is all there is to do for a view without instances."""
+    from fast_sp_gs_amd import lib as L, scenes
+    from fast_sp_gs_amd._C import get_C_function
+    lib, stream = L.load(), L.current_stream()
+    W, H = 16 * gx - 3, 16 * gy - 5
+    s = scenes._surfels(torch.Generator().manual_seed(P), P, 'cube', -3.5 if P < 10_000 else -4.5, 0.7, 0.0, 1.5).to(device)
+    cam = scenes.pinhole(W, H, 50.0, torch.tensor([0.0, 0.0, 4.0])).to(device)
+    m2, _, _, _, depths, radii, touched = get_C_function('gs_2d_preprocess_forward')(
+        W, H, 3, False, s.means3D, s.scales, s.rotations, s.opacities, s.shs, None, cam.Tw2v, cam.Tv2c, cam.campos, None, None, None)
+    want_ranges, want_list = get_C_function('GS_prepare')(W, H, m2, depths, radii, touched, False)[:2]
+    bins = torch.full((lib.fsgs_gs_prepare_bins_bytes(P, W, H),), 0xff, dtype=torch.uint8, device=device)
+    word = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    for seen in (radii, torch.zeros_like(radii)):
+        R = int(touched.sum()) if seen is radii else 0
+        counters = torch.zeros(64, dtype=torch.int64, device=device)
+        counters[7] = R
+        ranges = torch.full((gx * gy, 2), -1, dtype=torch.int64, device=device)
+        L.check(lib.fsgs_gs_view_count(P, W, H, L.ptr(m2), None, None, L.ptr(seen), None, L.ptr(counters), None, word.data_ptr(),
+                                       L.ptr(ranges), L.ptr(bins), bins.numel(), stream), 'count')
+        L.check(lib.fsgs_gs_view_wait(word.data_ptr(), stream), 'wait')
+        assert int(word[0]) == R and bool((ranges[:, 0] <= ranges[:, 1]).all())
+        space = torch.empty(max(lib.fsgs_gs_prepare_fill_workspace_bytes(R), 1), dtype=torch.uint8, device=device)
+        for _ in range(2):
+            point_list = torch.full((R,), -5, dtype=torch.int32, device=device)
+            L.check(lib.fsgs_gs_prepare_fill_counted(P, W, H, L.ptr(m2), L.ptr(depths), L.ptr(seen), R, L.ptr(ranges), L.ptr(point_list),
+                                                     None, L.ptr(bins), bins.numel(), L.ptr(space), space.numel(), stream), 'fill')
+            if R:
+                assert torch.equal(ranges, want_ranges) and torch.equal(point_list, want_list)
+        if not R:
+            assert bool((ranges[:, 0] == ranges[:, 1]).all())
