@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(1024) tile_scatter_kernel(int P, int per_block
     const float2* __restrict__ means2D, const float* __restrict__ depths, const int32_t* __restrict__ radii,
     WalkInputs in, const uint32_t* __restrict__ hist, unsigned long long* __restrict__ ranges,
     uint64_t* __restrict__ entries, int* __restrict__ order_table, int* __restrict__ header) {
-  __shared__ unsigned s_cursor[kTiles];
+  __shared__ __attribute__((aligned(8))) unsigned s_cursor[kTiles];  // (64-bit words in it below)
   const int T = gx * gy, B = (P + per_block - 1) / per_block;
   const uint32_t* totals = hist + (size_t) B * T;
   // One block more than the walk needs, when the frame's blockIdx -> tile schedule is still to be built: the tiles' totals are
