@@ -92,16 +92,17 @@ Buffers forward_view(const SurfelView& v, bool train) {
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
-    check(fsgs_gs_2d_view_preprocess((int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations),
-                                     f32(v.opacities), f32(v.shs),
-                                     has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr, f32(v.Tw2v),
-                                     f32(v.Tv2c), f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
-                                     v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), f32(b.trans_mat),
-                                     f32(b.normal_opacity), scratch.at<float>(depths), i32(b.radii),
-                                     data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles),
-                                     train ? b.keep.at<int32_t>(s.offsets) : nullptr, counters.data(), records, masks,
-                                     stream),
-          what);
+    auto preprocess = [&](auto entry, auto... slot_offsets) {
+      check(entry((int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations), f32(v.opacities), f32(v.shs),
+                  has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr, f32(v.Tw2v), f32(v.Tv2c),
+                  f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
+                  v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), f32(b.trans_mat), f32(b.normal_opacity),
+                  scratch.at<float>(depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles),
+                  slot_offsets..., counters.data(), records, masks, stream),
+            what);
+    };
+    if (train) preprocess(fsgs_gs_2d_view_preprocess, b.keep.at<int32_t>(s.offsets));
+    else preprocess(fsgs_gs_2d_view_preprocess_no_backward);
     check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
                              train ? b.keep.at<int32_t>(s.regions) : nullptr, count, i64(b.ranges), scratch.at<void>(bins),
                              bins_bytes, stream),

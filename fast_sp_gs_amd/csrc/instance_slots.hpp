@@ -73,6 +73,7 @@ struct ViewOutputs {
   unsigned long long* counters = nullptr;
   int32_t* slot_offsets = nullptr;
   uint8_t* visible = nullptr;
+  bool windows = false;  // no backward follows: keep masks of large rectangles may be windows (cull_window)
 };
 
 // What the kernel behind the preprocess hands on: see above. `counters` nullptr: nothing to do.

@@ -261,17 +261,16 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   }
   if (keep_masks) {
     // Which tiles of the surfel's rectangle some pixel of which can blend it (the culled binning's input): a bit per
-    // tile, row-major, or for rectangles above kCullMaskTiles tiles a window of them. With record slots the backward sums
-    // every position of a large rectangle, so there all bits are set. Evaluated here, where transform, centre and radius are
+    // tile, row-major, or for rectangles above kCullMaskTiles tiles a window of them. A backward sums
+    // every position of a large rectangle, so where one may follow all bits are set. Evaluated here, where transform, centre and radius are
     // in registers and the vector units wait for memory anyway (in the flight of the rows instead: 3M 209 -> 204 us, but
     // 300k 34.0 -> 34.8, 400k at 3840x2160 53.7 -> 55.7).
     uint32_t keep = 0xffffffffu;
-    const bool windows = view.counters && !view.slot_offsets;
     if (ok) {
       const TileRect r = tile_rect(c2[0], c2[1], f2i_sat(radius), gx, gy);
       const int w = max(r.x1 - r.x0, 0), h = max(r.y1 - r.y0, 0);
       const bool small = w * h <= kCullMaskTiles;
-      if (small || windows) {
+      if (small || view.windows) {
         const CullBounds cb = cull_bounds(M, c2[0], c2[1], op);
         keep = 0u;
         int e = 0;
@@ -707,6 +706,18 @@ FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int 
                             campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
                             tiles_touched, records, keep_masks,
                             ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
+  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
+                            tiles_touched, records, keep_masks,
+                            ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, true}, stream);
 }
 
 namespace {

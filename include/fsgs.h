@@ -52,13 +52,19 @@ int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, 
 /* A whole view without a prefix scan (no counterpart in the reference): the preprocess hands out the gradient records'
  * slots itself. slot_counters[64] are zero before the call and again after fsgs_gs_view_count; a surfel's slots start at
  * slot_offsets[i] + slot_regions[(i / 256) % 64] and are tiles_touched[i] many. visible[P] (0 / 1), slot_offsets, records
- * and keep_masks are optional. Without slot_offsets there will be no backward, and keep_masks of surfels with rectangles above 32
- * tiles, which have all bits set otherwise, narrow those rectangles too (the binning knows how). Every row of the outputs is written. */
+ * and keep_masks are optional. Every row of the outputs is written.
+ * _no_backward: the same for a view that is not back-propagated. keep_masks of surfels with rectangles above 32 tiles, which have all
+ * bits set otherwise, narrow those rectangles too: the binning knows how, the sums of a backward do not. */
 int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
     const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
     float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
     int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream);
+int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
+    const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
+    float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream);
 
 /* gs_2d_preprocess_backward -- gs_2d_preprocess.cu:423-499 (kernel :268-329). Every row of g_* is ASSIGNED: the
  * gradient for surfels with radii > 0, zeros for the others and for SH coefficients above the active degree (the

@@ -56,3 +56,33 @@ def test_windows_change_no_map(P, W, H, scale, thin, device):
         if name == 'whole':
             want = ids
     assert torch.equal(ids, want)
+
+
+def test_only_views_without_a_backward_get_windows(device):
+    """The C entries: without record slots, too, the masks of large rectangles have all bits set, as the sums of
+    `fsgs_gs_2d_render_backward_culled` expect them; with `_no_backward` they are windows, the others' masks are the same."""
+    from fast_sp_gs_amd import lib as L, scenes
+    lib, stream = L.load(), L.current_stream()
+    P, W, H = 400, 640, 353
+    g = torch.Generator().manual_seed(7)
+    s = scenes._surfels(g, P, 'cube', -1.4, 0.7, 0.0, 1.5).to(device)
+    cam = scenes.pinhole(W, H, 50.0, torch.tensor([0.3, 0.2, 4.0])).to(device)
+
+    def masks(entry, *slots):
+        f = lambda *shape, dtype=torch.float32: torch.empty(shape, dtype=dtype, device=device)
+        means2D, colors, trans, normal_opacity, depths = f(P, 2), f(P, 3), f(P, 3, 3), f(P, 4), f(P)
+        radii, touched, keep = f(P, dtype=torch.int32), f(P, dtype=torch.int32), f(P, dtype=torch.int32)
+        counters = torch.zeros(64, dtype=torch.int64, device=device)
+        L.check(entry(P, W, H, 3, 16, L.ptr(s.means3D), L.ptr(s.scales), L.ptr(s.rotations), L.ptr(s.opacities), L.ptr(s.shs), None,
+                      L.ptr(cam.Tw2v), L.ptr(cam.Tv2c), L.ptr(cam.campos), None, L.ptr(means2D), L.ptr(colors), L.ptr(trans),
+                      L.ptr(normal_opacity), L.ptr(depths), L.ptr(radii), None, L.ptr(touched), *slots, L.ptr(counters), None,
+                      L.ptr(keep), stream), 'preprocess')
+        assert int(counters.sum()) == int(touched.sum())
+        return touched, keep
+    offsets = torch.empty(P, dtype=torch.int32, device=device)
+    touched, kept = masks(lib.fsgs_gs_2d_view_preprocess, L.ptr(offsets))
+    large = touched > 32
+    assert int(large.sum()) > P // 4 and bool((kept[large] == -1).all())
+    assert torch.equal(masks(lib.fsgs_gs_2d_view_preprocess, None)[1], kept)
+    windows = masks(lib.fsgs_gs_2d_view_preprocess_no_backward)[1]
+    assert torch.equal(windows[~large], kept[~large]) and int((windows[large] != -1).sum()) > P // 8
