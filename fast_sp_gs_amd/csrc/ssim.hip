@@ -316,14 +316,20 @@ ssim_backward_kernel(int H, int W, int CH, int tiles_x, bool pairs, const float*
 // The launch of either kernel: a block per tile of an image, a wavefront per channel. Outputs two at a time where rows and planes
 // start at multiples of 8 bytes and seven rows are within a buffer's offsets: 3x800x800 backward 13.5 us against 15.5 by rows
 // through LDS. Elsewhere by rows: 3x667x1001 forward 22 us against 27 with single words from the lanes, which lie 24 bytes apart.
+// By rows, too, once the maps that a call with gradients reads and writes are more than the memory-side cache holds with them: the pairs
+// leave the L2s as parts of lines. us pairs | rows: 3x2160x3840 (map and derivatives 597 MB) 238 | 181, in loss form (498 MB) 200 | 163, backward
+// (697, 597 MB) 197 | 181 and 165 | 149; in loss form 288 MB 113 | 100, 243 MB 70 | 76; backward 310 MB 89 | 83, 292 MB 75 | 69, 270 MB 61 | 68.
+// The map with its derivatives, four maps written: 115 MB 37 | 36, 149 MB 44 | 40, 265 MB 86 | 77. (The map alone: 3x4000x6000 308 | 314.)
+constexpr double kPairsMost = 280e6, kPairsMostOfFour = 120e6;
 struct SsimGrid {
   int tiles_x, tiles;
   dim3 grid, block;
   bool pairs;
-  SsimGrid(int B, int CH, int H, int W, std::initializer_list<const void*> planes) {
+  // planes: those that are written or read a pair at a time; maps: how many the call reads and writes, where it is one with gradients
+  SsimGrid(int B, int CH, int H, int W, std::initializer_list<const void*> planes, int maps, double most = kPairsMost) {
     tiles_x = div_up(W, kOutCols), grid = dim3(tiles_x * div_up(H, kOutRows), 1, B), tiles = grid.x * B;
     block = dim3(kWave * std::min(CH, kSsimWaves));
-    pairs = W % 2 == 0 && W < (1 << 26);
+    pairs = W % 2 == 0 && W < (1 << 26) && 4.0 * maps * B * CH * H * W <= most;
     for (const void* p : planes) pairs &= ((uintptr_t) p & 7) == 0;
   }
 };
@@ -342,7 +348,7 @@ FSGS_API int fsgs_fusedssim_forward(int B, int CH, int H, int W, double C1, doub
   const bool train = dm_dmu1 != nullptr;
   FSGS_REQUIRE(!train || (dm_dsigma1_sq && dm_dsigma12), "fusedssim: the three partial-derivative maps go together");
   FSGS_REQUIRE(B <= 65535, "fusedssim: batch %d exceeds the grid limit", B);
-  const SsimGrid g(B, CH, H, W, {ssim_map, dm_dmu1, dm_dsigma1_sq, dm_dsigma12});
+  const SsimGrid g(B, CH, H, W, {ssim_map, dm_dmu1, dm_dsigma1_sq, dm_dsigma12}, train ? 6 : 0, kPairsMostOfFour);
   hipLaunchKernelGGL((train ? ssim_forward_kernel<true, false> : ssim_forward_kernel<false, false>), g.grid, g.block, 0,
                      (hipStream_t) stream, H, W, CH, g.tiles_x, g.pairs, (float) C1, (float) C2, img1, img2,
                      ssim_map, dm_dmu1, dm_dsigma1_sq, dm_dsigma12, nullptr);
@@ -357,7 +363,7 @@ FSGS_API int fsgs_fusedssim_backward(int B, int CH, int H, int W, const float* i
   FSGS_REQUIRE(img1 && img2 && dL_dmap && dm_dmu1 && dm_dsigma1_sq && dm_dsigma12 && dL_dimg1,
                "fusedssim_backward: null pointer");
   FSGS_REQUIRE(B <= 65535, "fusedssim_backward: batch %d exceeds the grid limit", B);
-  const SsimGrid g(B, CH, H, W, {img1, img2, dL_dimg1});
+  const SsimGrid g(B, CH, H, W, {img1, img2, dL_dimg1}, 7);
   hipLaunchKernelGGL(ssim_backward_kernel<false>, g.grid, g.block, 0, (hipStream_t) stream, H, W, CH, g.tiles_x, g.pairs, img1, img2, dL_dmap, dm_dmu1, dm_dsigma1_sq, dm_dsigma12, dL_dimg1, 0.0f, 0.0f);
   return check_launch("fusedssim_backward");
 }
@@ -377,7 +383,7 @@ FSGS_API int fsgs_image_loss_forward(int B, int CH, int H, int W, double C1, dou
   if (workspace_bytes < fsgs_image_loss_workspace_bytes(B, H, W))
     return fail(kWorkspaceSmall, "image_loss: workspace %zu < %zu bytes", workspace_bytes,
                 fsgs_image_loss_workspace_bytes(B, H, W));
-  const SsimGrid g(B, CH, H, W, {dm_dmu1, dm_dsigma1_sq, dm_dsigma12});
+  const SsimGrid g(B, CH, H, W, {dm_dmu1, dm_dsigma1_sq, dm_dsigma12}, 5);
   hipStream_t s = (hipStream_t) stream;
   float* partials = (float*) workspace;
   hipLaunchKernelGGL((train ? ssim_forward_kernel<true, true> : ssim_forward_kernel<false, true>), g.grid, g.block, 0, s, H, W,
@@ -436,7 +442,7 @@ FSGS_API int fsgs_image_loss_backward(int B, int CH, int H, int W, double lambda
   FSGS_REQUIRE(B > 0 && CH > 0 && H > 0 && W > 0 && B <= 65535, "image_loss_backward: bad sizes");
   FSGS_REQUIRE(img && target && grad_loss && dm_dmu1 && dm_dsigma1_sq && dm_dsigma12 && dL_dimg,
                "image_loss_backward: null pointer");
-  const SsimGrid g(B, CH, H, W, {img, target, dL_dimg});
+  const SsimGrid g(B, CH, H, W, {img, target, dL_dimg}, 6);
   const double n = (double) B * CH * H * W;
   hipLaunchKernelGGL(ssim_backward_kernel<true>, g.grid, g.block, 0, (hipStream_t) stream, H, W, CH, g.tiles_x, g.pairs, img, target, grad_loss, dm_dmu1, dm_dsigma1_sq, dm_dsigma12, dL_dimg,
                      (float) (-lambda_dssim / n), (float) ((1.0 - lambda_dssim) / n));

@@ -190,3 +190,24 @@ def test_ssim_scales_with_its_images(scale, tol, device):
     for k, power in enumerate((0, 1, 2, 2)):
         w, v = want[k].double(), got[k].double() * scale ** power
         assert bool(torch.isfinite(v).all()) and float((v - w).abs().max()) < tol * float(w.abs().max()), k
+
+
+def test_ssim_pairs_and_rows_are_the_same(device):
+    """Maps larger than the memory-side cache are written row by row, smaller ones two pixels a lane, and so are those of odd widths: the
+    numbers are the same to the bit, here those of an image of 290 MB of maps with gradients and of its upper half, away from the cut."""
+    from fast_sp_gs_amd._C import get_C_function
+    from fast_sp_gs_amd.ssim import l1_dssim_loss
+    H, W = 2100, 1920
+    g = torch.Generator(device=device).manual_seed(1)
+    a, b, up = (torch.rand(1, 3, H, W, generator=g, device=device) for _ in range(3))
+    fwd, bwd = get_C_function('fusedssim'), get_C_function('fusedssim_backward')
+    call = lambda x, y, u: (lambda maps: [*maps, bwd(0.01 ** 2, 0.03 ** 2, x, y, u, *maps[1:])])(fwd(0.01 ** 2, 0.03 ** 2, x, y, True))
+    whole, half = call(a, b, up), call(*(t[..., : H // 2, :].contiguous() for t in (a, b, up)))
+    for w, h in zip(whole, half):
+        assert torch.equal(w[..., : H // 2 - 10, :], h[..., : H // 2 - 10, :])
+    x = a.clone().requires_grad_(True)
+    l1_dssim_loss(x, b, 0.2).backward()  # 6 x 48 MB
+    n = 3 * H * W
+    maps = [torch.full_like(a, -0.2 / n), *whole[1:4]]
+    want = bwd(0.01 ** 2, 0.03 ** 2, a, b, *maps) + 0.8 / n * torch.sign(a - b)
+    assert rel_err(npy(x.grad), npy(want)) < 1e-5
