@@ -142,8 +142,8 @@ constexpr int kNarrowTiles = 16384, kMaxLdsTiles = 40960;
 
 // Which tiles of a surfel's rectangle are visited: all of them (the reference's lists), those that pass the fast path's
 // corner test (CornerTest, from the surfel's adjugate and opacity), or those whose bit is set in the surfel's keep mask
-// (cull_mask_kernel: the tiles some pixel of which can blend the surfel; for rectangles above 32 tiles a window of them,
-// cull_window, or all).
+// (cull_mask_kernel, or the preprocess kernels: the tiles some pixel of which can blend the surfel; rectangles above 32 tiles are kept
+// whole, or, by the surfels' preprocess in a view without a backward, as a window of them, cull_window).
 // kWalkCornerMask is the corner test with its verdicts for rectangles of at most 32 tiles taken from a mask the
 // preprocess kernel left (bit x * h + y: x-major, the order of the fast path's key span), so that the test's set-up (a
 // double-precision logarithm among it) runs once per surfel and view instead of once per walk; larger rectangles are

@@ -314,7 +314,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
 
   if (kWave) {
     // as in the surfels' kernel only the rows of what is on the screen; the mask is found while they are on their way. 300k
-    // Gaussians 31.2 -> 29.1 us, 25k 12.7 -> 12.4
+    // Gaussians 29.8 -> 27.4 us, 60k 14.0 -> 13.6, 25k 12.6 -> 12.2 (traced in turn, 60 views of three inputs four times)
     wanted = __ballot(ok);
     if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
   }

@@ -6,7 +6,7 @@
 // ruled out for a whole cell of a grid over the control points at once:
 //   1. knn_cell_lists_kernel: the cells of a G x G x G grid. U = a bound on the K-th nearest distance of ANY point of the
 //      cell (the K-th smallest of 64 far-corner distances); the cell's list holds the control points whose nearest-corner
-//      distance does not exceed U, with many queries in the order of the distances from the cell's centre (kOrderFrom), else of the
+//      distance does not exceed U, with many queries in the order of the distances from the cell's centre (lists_in_order), else of the
 //      indices. A block builds the list of one of 8 x 8 x 8 coarse cells and refines it for the (G / 8)^3 cells inside.
 //   2. knn_cell_query_kernel: a lane finds its query's cell and walks the cell's list (about 38 entries for 2048 control
 //      points and G = 32; in order, about 20 of them: what follows is farther from the centre than the K-th neighbour can be). The walk only keeps the K + 1 smallest keys -- the distance in 2^-20 parts of
@@ -18,12 +18,14 @@
 //      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
 //      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.17 ms a call this way
-// (traced: lists 0.047, queries 0.118; 0.063 ms for the 324 MB of inputs and outputs alone). The query kernel is bound by vector issue (1090
-// instructions per 64 queries, 0.7 of the issue slots) and LDS (half of the time, a fifth in bank conflicts). With lists in index order and a row of results stored by each lane for itself
-// it took 0.202 ms and 2180 instructions; in order alone 0.169, its memory path busy with stores of 16 bytes each; results through LDS in
-// runs of 512 and 1024 bytes 0.152, and past the caches, which then keep the lists (8 MB), 0.118.
-// 200 000 x 512, K = 4: 57 -> 24 us, 50 000 x 512, K = 3: 37 -> 19 us, 5 000 x 512, K = 4: 36 -> 10 us.
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.154 ms a call this way
+// (traced: lists 0.046, queries 0.118 to 0.129; 0.063 ms for the 324 MB of inputs and outputs alone). In the query kernel neither unit is
+// full: the vector units are busy 0.62 of the time (1090 instructions per 64 queries), LDS 0.52, 0.22 in bank conflicts. With lists in
+// index order and a row of results stored by each lane for itself it took 0.202 ms and 2180 instructions; in order alone 0.169, its
+// memory path busy with stores of 16 bytes each; results through LDS in runs of 512 and 1024 bytes 0.152, and past the caches, which then
+// keep the lists (8 MB), 0.118.
+// Over all pairs -> this way, calls in a row, queries in a ball (normal): 200 000 x 512, K = 4 57 -> 21 (31) us, 50 000 x 512, K = 3 37 -> 18 (28),
+// 5 000 x 512, K = 4 36 -> 6.2 (6.3).
 #include <algorithm>
 #include <type_traits>
 
@@ -63,10 +65,10 @@ enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 
 // Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
 // alone) and N * M / 4e12 s when they fill the chip; a wavefront per query 0.8 (M = 512) to 2.0 ns (M = 2048) a query;
-// building the lists 11 us (G = 16, 512 control points) to 37 us (G = 32, 2048). With G = 16 the lists of more than 640
+// building the lists 11 us (G = 16, 512 control points) to 37 us (G = 32, 2048), in order 12 and 46. With G = 16 the lists of more than 640
 // control points outgrow their 128 entries; below that the finer grid pays from a million queries on. Behind the limits
-// the walk over all pairs takes over at its own price: 3M queries, K = 4: 164 us for 2560 control points, 1481 for 2561; 2048
-// control points, K = 8: 171 us, K = 9: 5897. 200 000 queries, K = 4: 60 and 187 us.
+// the walk over all pairs takes over at its own price: 3M normal queries, K = 4: 133 us for 2560 control points, 1550 for 2561; 2048
+// control points, K = 8: 156 us, K = 9: 5940. 200 000 queries, K = 4: 60 and 187 us.
 Scheme knn_scheme(int N, int M, int D, int K) {
   if (D != 3 || K > kMaxK || M > kMaxPoints || M < 96) return kAllPairs;
   if (N <= kFewQueries) return kAlone;

@@ -753,7 +753,7 @@ int fsgs_fusedssim_backward(int B, int CH, int H, int W, const float* img1, cons
  * fast_2d_gs/gaussian_splatting.py:321 / network.py:1027 with losses/ssim.py:24-47, which the reference evaluates as an
  * L1 in torch, the fusedssim map, two means and their autograd. img, target [B,CH,H,W]. loss_out[3] = (loss, L1 mean,
  * SSIM mean). dm_* are NULL (no gradient wanted) or the three [B,CH,H,W] maps the backward reads. The workspace holds
- * two partial sums per 32x32 block, added in a fixed order. The backward reads the upstream gradient of the scalar loss
+ * two partial sums per tile of 54x7 pixels, added in a fixed order. The backward reads the upstream gradient of the scalar loss
  * from device memory (grad_loss[0]) and writes dL_dimg[B,CH,H,W] in full. */
 size_t fsgs_image_loss_workspace_bytes(int B, int H, int W);
 int fsgs_image_loss_forward(int B, int CH, int H, int W, double C1, double C2, double lambda_dssim, const float* img,
