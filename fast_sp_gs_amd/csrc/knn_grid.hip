@@ -78,10 +78,11 @@ Scheme knn_scheme(int N, int M, int D, int K) {
 
 // Whether the lists are put in the order of the distances from their cell's centre, so that a query's walk is over after half of its
 // list (below). With G = 32 that costs 4 to 8 us whatever the number of queries, with G = 16 1 us; what it saves grows with the queries,
-// with K and with the length of the lists, that is, with M. Past about 200 MB of results the stores past the caches, which come with
+// with K and with the length of the lists, that is, with M. Past about 150 MB of results the stores past the caches, which come with
 // the order (kStream), outweigh that. us a call in index order -> in this one, queries in a ball | normal (what two runs differ by: 1 to 3):
 //   G = 32, K = 8, M = 2048:  500 000 59 -> 59 | 79 -> 82;  1M 81 -> 76 | 104 -> 100;  3M 183 -> 131 | 204 -> 154
-//           K = 8, M = 256:   1.7M 75 -> 77 | 86 -> 89;  2.5M 124 -> 99 | 136 -> 114
+//           K = 8, M = 256:   1.5M 72 -> 73 | 79 -> 83;  1.75M 76 -> 76 | 85 -> 89;  2M 84 -> 81 | 100 -> 97;  2.5M 124 -> 99 | 136 -> 114
+//           K = 5, M = 400:   2.2M 71.5 -> 69.8 | 84.8 -> 82.7;  2.5M 77.8 -> 77.0 | 93.8 -> 88.8
 //           K = 4, M = 400 (640): 1.7M 58.1 -> 59.7 | 68.7 -> 67.9 (62.5 -> 61.9 | 72.5 -> 71.4)
 //           K = 3, M = 640 (1024): 2.1M 65.2 -> 67.4 | 78.6 -> 78.2 (70.2 -> 69.2 | 82.4 -> 81.2)
 //           K = 2, 2.5M: M = 640 64.6 -> 69.6 | 76.5 -> 80.1;  1400 71.4 -> 75.3 | 89.3 -> 87.9;  2048 80.1 -> 77.3 | 100 -> 93
@@ -97,7 +98,7 @@ bool lists_in_order(int64_t N, int M) {
   if (kG == 16) return N >= 400000;
   const int64_t results = N * (kK + 2), entries = M * (kK + 2);
   if (kK == 2) return results >= 10000000 && M >= 1400;
-  return results >= (entries >= 3800 ? 10000000 : 20000000);
+  return results >= (entries >= 3800 ? 10000000 : 17500000);
 }
 
 // A cell. `length`: how many candidates its list holds (or kLongList) and kCrowdedBit; `scale`: what takes a squared distance to 2^32 at

@@ -345,11 +345,11 @@ def test_knn_clusters(N, M, K, radius, mixed, device):
     assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
 
 
-# Lists in the order of their cells' centre distances (32^3 cells from 10M / (K + 2) queries on, with few control points from 20M / (K + 2),
+# Lists in the order of their cells' centre distances (32^3 cells from 10M / (K + 2) queries on, with few control points from 17.5M / (K + 2),
 # with K = 2 only with many, with K = 1 never; 16^3 from K = 3 or 400 000), where a query's walk ends before its list does, and lists beside
 # those lines; the last wavefront is not full. Far from the origin a cell's extent is a few roundings of its coordinates.
 @pytest.mark.parametrize('N,M,K', [(1_000_001, 2560, 8), (1_428_573, 641, 5), (2_500_007, 700, 2), (400_001, 640, 1), (16_449, 192, 3),
-                                   (2_500_001, 1400, 2), (2_000_003, 300, 8), (1_999_999, 300, 8)])
+                                   (2_500_001, 1400, 2), (1_750_003, 300, 8), (1_749_999, 300, 8)])
 @pytest.mark.parametrize('kind', ['normal', 'lattice', 'clusters', 'far', 'heavy tails', 'flat'])
 def test_knn_ordered_lists(N, M, K, kind, device):
     from fast_sp_gs_amd._C import get_C_function
