@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
-  float dc[3] = {0, 0, 0};
+  float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
   if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   do {
     if (!valid || (culling && culling[i])) break;
@@ -237,6 +237,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     const float* cr = kWave ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
     for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
     rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+    if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
   }
   if (view.slot_offsets) {
     if (threadIdx.x == 0) s_block_slot = (int) block_slot;
@@ -258,6 +259,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     wave_rows_out<9>(s_adj, wave_base, P, inverse_m);
     wave_rows_out<3>(s_rgb, wave_base, P, colors);
   }
+  if (kWave && view.color_derivs) wave_derivs_out(s_wave_rows, derivs, wave_base, P, view.color_derivs);
   if (!valid) return;
   if (view.slot_offsets) view.slot_offsets[i] = slot;
   if (view.visible) view.visible[i] = ok && f2i_sat(radius) > 0;
@@ -349,7 +351,9 @@ __global__ void __launch_bounds__(256) fast_duplicate_keys_kernel(int P, int gx,
   }
 }
 
-template <int kSh, int kRow>
+// kDerivs: from the colours' derivatives that the forward left, without the rows of coefficients (as the surfels'). 150k surfels
+// 1001x667: 16.4 -> 12.6 us, the forward 17.3 -> 18.4.
+template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -358,16 +362,18 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     float2* __restrict__ grad_mean2D, const float* __restrict__ grad_trans, const float* __restrict__ grad_inv_m,
     const float* __restrict__ grad_colors, const float4* __restrict__ grad_normal_opacity,
     float* __restrict__ g_means3D, float2* __restrict__ g_scales, float4* __restrict__ g_rot,
-    float* __restrict__ g_opac, float* __restrict__ g_shs, float* __restrict__ g_sh_rest) {
+    float* __restrict__ g_opac, float* __restrict__ g_shs, float* __restrict__ g_sh_rest, const float* __restrict__ color_derivs) {
+  static_assert(!kDerivs || kRow != 0);
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
-  __shared__ __align__(16) float s_rows[kWave ? kShStageRows * kStride : 1];
+  constexpr int kWaveRows = kDerivs ? kShHalfRows : 64;  // that pass through the LDS at a time
+  __shared__ __align__(16) float s_rows[kWave ? 4 * kWaveRows * kStride : 1];
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
   const bool vis   = valid && radii[i] > 0;
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
-  float* my_row       = &s_rows[kWave ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveRows * kStride : 0];
+  float* my_row       = &s_rows[kWave && !kDerivs ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
   // Rows of surfels that were not rendered get explicit zeros, so the outputs need no initialisation (the reference
   // leaves them to the caller's zero fill; a caller that zero-fills gets the same result).
   auto zero_geometry = [&]() {
@@ -387,13 +393,15 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
       if (valid) zero_geometry();
       return;
     }
-    ShWaveRows<kWave ? kRow : 48> sh_regs;
-    sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
-    sh_regs.to_lds(s_wave_rows, wave_base, P);
-    wave_lds_sync();
+    if (!kDerivs) {
+      ShWaveRows<kWave ? kRow : 48> sh_regs;
+      sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
+      sh_regs.to_lds(s_wave_rows, wave_base, P);
+      wave_lds_sync();
+    }
     if (!vis) {
 #pragma unroll
-      for (int c = kSplit ? 3 : 0; c < kShStageFloats; ++c) my_row[c] = 0.0f;
+      for (int c = kSplit ? 3 : 0; c < (kDerivs ? 0 : kShStageFloats); ++c) my_row[c] = 0.0f;
       if (kSplit && valid && g_shs)
         g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       if (valid) zero_geometry();
@@ -411,6 +419,9 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     }
     return;
   }
+  float g[3] = {}, Y[kSh];  // the colour's gradient and the basis: their products are the gradients of the coefficients
+#pragma unroll
+  for (int l = 0; l < (kDerivs ? kSh : 0); ++l) Y[l] = 0.0f;
   if (vis) {
   float Tw2v[16], Tv2s[9];
 #pragma unroll
@@ -455,10 +466,12 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
   fast_transmat_backward(s.x, s.y, q, Tw2v, Tv2s, gT, gN, gp, gs, gq);
 
   if (sh_degree >= 0) {
-    float x, y, z, Y[kSh], tl[kSh];
+    float x, y, z, derivs[kColorDerivs];
+    if (kDerivs)
+#pragma unroll
+      for (int k = 0; k < kColorDerivs; ++k) derivs[k] = color_derivs[kColorDerivs * (size_t) i + k];
     const float nn = view_dir(p, campos, x, y, z);
     sh_eval(sh_degree, x, y, z, Y);
-    float g[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) g[c] = grad_colors[3 * (size_t) i + c] * (float) (colors[3 * (size_t) i + c] > 0);
     const int n  = sh_count(sh_degree);
@@ -466,21 +479,19 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     // with kWave the coefficients are read from the lane's staged row and the gradient row is written over them
     const float* c0 = kWave ? my_row : shs + (size_t) i * m1 * 3;
     const float* cr = kWave ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-    float* o0  = kWave && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
-    float* orr = kWave ? my_row
+    float* o0  = kDerivs && !kSplit ? nullptr : kWave && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
+    float* orr = kDerivs ? nullptr : kWave ? my_row
                        : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
     if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
-    tl[0] = 0.0f;
-    for (int l = 1; l < n; ++l) {
-      tl[l] = g[0] * cr[3 * l] + g[1] * cr[3 * l + 1] + g[2] * cr[3 * l + 2];
+    const float dir[3] = {x, y, z};
+    float dx = 0, dy = 0, dz = 0;
+    sh_direction_part<kSh, kDerivs>(sh_degree, dir, g, cr, derivs, dx, dy, dz);  // before the coefficients are written over
+    for (int l = 1; l < n; ++l)
       if (orr) orr[3 * l] = g[0] * Y[l], orr[3 * l + 1] = g[1] * Y[l], orr[3 * l + 2] = g[2] * Y[l];
-    }
     if (!kWave && orr) {  // coefficients above the active degree
       for (int l = n; l < (sh_rest ? n_sh + 1 : n_sh); ++l)
         orr[3 * l] = 0.0f, orr[3 * l + 1] = 0.0f, orr[3 * l + 2] = 0.0f;
     }
-    float dx = 0, dy = 0, dz = 0;
-    sh_grad_accumulate(sh_degree, x, y, z, tl, dx, dy, dz);
     const float vx = p[0] - campos[0], vy = p[1] - campos[1], vz = p[2] - campos[2];
     const float tt = -(vx * dx + vy * dy + vz * dz) * nn * nn * nn;
     gp[0] = gp[0] + (dx * nn + tt * vx);
@@ -494,7 +505,9 @@ __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
   const float depth = m[8];
   grad_mean2D[i] = make_float2(gT[2] * depth * 0.5f * (float) W, gT[5] * depth * 0.5f * (float) H);
   }
-  if (kWave) {
+  if constexpr (kDerivs) {
+    sh_products_to_global<kRow>(s_wave_rows, g, Y, wave_base, P, kSplit ? g_sh_rest : g_shs);
+  } else if (kWave) {
     wave_lds_sync();
     ShWaveRows<kWave ? kRow : 48>::to_global(s_wave_rows, wave_base, P, kSplit ? g_sh_rest : g_shs);
   }
@@ -585,16 +598,28 @@ FSGS_API int fsgs_gs_2d_fast_preprocess_forward(int P, int W, int H, int sh_degr
                                  normal_opacity, depths, radii, tiles_touched, keep_masks, ViewOutputs{}, stream);
 }
 
+FSGS_API int fsgs_gs_2d_fast_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
+    int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, float* color_derivs, void* stream) {
+  FSGS_REQUIRE(!color_derivs || wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0, "gs_2d_fast_view_preprocess: no derivatives of these rows");
+  FSGS_REQUIRE(slot_counters, "gs_2d_fast_view_preprocess: slot_counters are required");
+  return fast_preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
+                                 campos, nullptr, culling, 0, means2D, colors, trans_mat, inverse_m, normal_opacity, depths,
+                                 radii, tiles_touched, keep_masks,
+                                 ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible, false, color_derivs}, stream);
+}
+
 FSGS_API int fsgs_gs_2d_fast_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
     float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
     int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, void* stream) {
-  FSGS_REQUIRE(slot_counters, "gs_2d_fast_view_preprocess: slot_counters are required");
-  return fast_preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
-                                 campos, nullptr, culling, 0, means2D, colors, trans_mat, inverse_m, normal_opacity, depths,
-                                 radii, tiles_touched, keep_masks,
-                                 ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
+  return fsgs_gs_2d_fast_view_preprocess_derivs(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2s,
+                                                campos, culling, means2D, colors, trans_mat, inverse_m, normal_opacity, depths,
+                                                radii, visible, tiles_touched, slot_offsets, slot_counters, keep_masks, nullptr,
+                                                stream);
 }
 
 FSGS_API int fsgs_gs_2d_fast_prepare_sort_bits(int W, int H) {
@@ -648,10 +673,10 @@ FSGS_API int fsgs_gs_2d_fast_prepare_fill(int P, int W, int H, const float* mean
   return check_launch("gs_2d_fast_prepare_fill");
 }
 
-FSGS_API int fsgs_gs_2d_fast_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+FSGS_API int fsgs_gs_2d_fast_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2s, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
-    float* grad_mean2D, const float* grad_trans, const float* grad_inv_m, const float* grad_colors,
+    const float* color_derivs, float* grad_mean2D, const float* grad_trans, const float* grad_inv_m, const float* grad_colors,
     const float* grad_normal_opacity, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
     float* g_sh_rest, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_fast_preprocess_backward: bad sizes");
@@ -664,16 +689,28 @@ FSGS_API int fsgs_gs_2d_fast_preprocess_backward(int P, int W, int H, int sh_deg
   if (P == 0) return kOk;
   float* g_rows  = sh_rest ? g_sh_rest : g_shs;
   const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
-  auto kernel = sh_degree > 3 ? fast_preprocess_backward_kernel<64, 0>
-                : rows == 48  ? fast_preprocess_backward_kernel<16, 48>
-                : rows == 45  ? fast_preprocess_backward_kernel<16, 45>
-                              : fast_preprocess_backward_kernel<16, 0>;
+  auto kernel = sh_degree > 3 ? fast_preprocess_backward_kernel<64, 0, false>
+                : rows == 48  ? (color_derivs ? fast_preprocess_backward_kernel<16, 48, true> : fast_preprocess_backward_kernel<16, 48, false>)
+                : rows == 45  ? (color_derivs ? fast_preprocess_backward_kernel<16, 45, true> : fast_preprocess_backward_kernel<16, 45, false>)
+                              : fast_preprocess_backward_kernel<16, 0, false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh,
                      means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v, Tv2s, campos,
                      trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_inv_m, grad_colors,
                      (const float4*) grad_normal_opacity, g_means3D, (float2*) g_scales, (float4*) g_rot, g_opac, g_shs,
-                     g_sh_rest);
+                     g_sh_rest, color_derivs);
   return check_launch("gs_2d_fast_preprocess_backward");
+}
+
+FSGS_API int fsgs_gs_2d_fast_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2s, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    float* grad_mean2D, const float* grad_trans, const float* grad_inv_m, const float* grad_colors,
+    const float* grad_normal_opacity, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
+    float* g_sh_rest, void* stream) {
+  return fsgs_gs_2d_fast_view_preprocess_backward_derivs(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2s,
+                                                         campos, trans_mat, radii, colors, nullptr, grad_mean2D, grad_trans,
+                                                         grad_inv_m, grad_colors, grad_normal_opacity, g_means3D, g_scales,
+                                                         g_rot, g_opac, g_shs, g_sh_rest, stream);
 }
 
 FSGS_API int fsgs_gs_2d_fast_compute_transmat_forward(int P, const float* means3D, const float* scales,

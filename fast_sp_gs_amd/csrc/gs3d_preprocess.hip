@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
-  float dc[3] = {0, 0, 0};
+  float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
   if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   do {
     if (!valid || (culling && culling[i])) break;
@@ -361,6 +361,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
       float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
       for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
       rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+      if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
     }
   }
   // cov3Ds is absent with a pre-computed 3D covariance: the caller hands that tensor on as the operator's output
@@ -378,6 +379,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
     if (cov3Ds) wave_rows_out<6>(s_cov, wave_base, P, cov3Ds);
     wave_rows_out<3>(s_rgb, wave_base, P, colors);
   }
+  if (kWave && view.color_derivs) wave_derivs_out(s_wave_rows, derivs, wave_base, P, view.color_derivs);
   if (!valid) return;
   if (!rows && cov3Ds)
 #pragma unroll
@@ -394,7 +396,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   if (keep_masks) keep_masks[i] = keep;
 }
 
-template <int kSh, int kRow>
+// kDerivs: from the colours' derivatives that the forward left, without the rows of coefficients (as the surfels'). 300k Gaussians
+// 800x800: 32 -> 22 us, the forward 27.6 -> 30.5.
+template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, int W, int H, int sh_degree, int n_sh,
     int is_opengl, const float* __restrict__ means3D, const float* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -404,12 +408,14 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
     const float* __restrict__ grad_colors,
     const float4* __restrict__ grad_conic, float* __restrict__ g_means3D, float* __restrict__ g_scales,
     float4* __restrict__ g_rot, float* __restrict__ g_opac, float* __restrict__ g_shs, float* __restrict__ g_sh_rest,
-    float* __restrict__ g_cov3D, float* __restrict__ g_Tw2v, float* __restrict__ g_campos) {
+    float* __restrict__ g_cov3D, float* __restrict__ g_Tw2v, float* __restrict__ g_campos, const float* __restrict__ color_derivs) {
+  static_assert(!kDerivs || kRow != 0);
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
   __shared__ float s_Tw2v[16], s_Tv2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
+  constexpr int kWaveRows = kDerivs ? kShHalfRows : 64;  // that pass through the LDS at a time
+  __shared__ __align__(16) float s_rows[kStage ? 4 * kWaveRows * kStride : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   if (threadIdx.x < 16) s_Tw2v[threadIdx.x] = Tw2v_g[threadIdx.x], s_Tv2c[threadIdx.x] = Tv2c_g[threadIdx.x];
   __syncthreads();
@@ -418,11 +424,11 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
   const bool vis   = valid && radii[i] > 0;
   const int n      = sh_degree >= 0 ? sh_count(sh_degree) : 0;
   const int m1     = sh_rest ? 1 : n_sh;
-  float* my_row    = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
+  float* my_row    = &s_rows[kStage && !kDerivs ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
   const float fx = 0.5f * (float) W / tanx, fy = 0.5f * (float) H / tany;
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
-  if (kWave) {
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveRows * kStride : 0];
+  if (kWave && !kDerivs) {
     const unsigned long long wanted = __ballot(vis);
     if (wanted) {
       ShWaveRows<kWave ? kRow : 48> sh_regs;
@@ -430,7 +436,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
       sh_regs.to_lds(s_wave_rows, wave_base, P);
     }
     wave_lds_sync();
-  } else if (kStage && sh_degree >= 0) {
+  } else if (!kWave && kStage && sh_degree >= 0) {
     s_flag[threadIdx.x] = vis;
     __syncthreads();
     stage_sh_rows(s_rows, s_flag, blockIdx.x * blockDim.x, P, n, n_sh, shs, sh_rest);
@@ -441,6 +447,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
 #pragma unroll
   for (int k = 0; k < 15; ++k) cam[k] = 0.0f;
   const int cov_w = cov2Ds ? 3 : 6;  // columns of g_cov3D
+  float g[3] = {}, Y[kSh];  // the colour's gradient and the basis: their products are the gradients of the coefficients
+#pragma unroll
+  for (int l = 0; l < (kDerivs ? kSh : 0); ++l) Y[l] = 0.0f;
   if (vis) {
     float Tw2v[16], Tv2c[16];
 #pragma unroll
@@ -496,29 +505,29 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
 #pragma unroll
       for (int k = 0; k < 6; ++k) g_cov3D[6 * (size_t) i + k] = gcov[k];
     if (sh_degree >= 0) {
-      float x, y, z, Y[kSh], tl[kSh];
+      float x, y, z, derivs[kColorDerivs];
+      if (kDerivs)
+#pragma unroll
+        for (int k = 0; k < kColorDerivs; ++k) derivs[k] = color_derivs[kColorDerivs * (size_t) i + k];
       const float nn = view_dir(p, campos, x, y, z);
       sh_eval(sh_degree, x, y, z, Y);
-      float g[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) g[c] = grad_colors[3 * (size_t) i + c] * (float) (colors[3 * (size_t) i + c] > 0);
       const float* c0 = kStage ? my_row : shs + (size_t) i * m1 * 3;
       const float* cr = kStage ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float* o0  = kStage && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
-      float* orr = kStage ? my_row
+      float* o0  = kDerivs && !kSplit ? nullptr : kStage && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
+      float* orr = kDerivs ? nullptr : kStage ? my_row
                           : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
       if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
-      tl[0] = 0.0f;
-      for (int l = 1; l < n; ++l) {
-        tl[l] = g[0] * cr[3 * l] + g[1] * cr[3 * l + 1] + g[2] * cr[3 * l + 2];
+      const float dir[3] = {x, y, z};
+      float dx = 0, dy = 0, dz = 0;
+      sh_direction_part<kSh, kDerivs>(sh_degree, dir, g, cr, derivs, dx, dy, dz);  // before the coefficients are written over
+      for (int l = 1; l < n; ++l)
         if (orr) orr[3 * l] = g[0] * Y[l], orr[3 * l + 1] = g[1] * Y[l], orr[3 * l + 2] = g[2] * Y[l];
-      }
       if (!kStage && orr) {
         for (int l = n; l < (sh_rest ? n_sh + 1 : n_sh); ++l)
           orr[3 * l] = 0.0f, orr[3 * l + 1] = 0.0f, orr[3 * l + 2] = 0.0f;
       }
-      float dx = 0, dy = 0, dz = 0;
-      sh_grad_accumulate(sh_degree, x, y, z, tl, dx, dy, dz);
       const float vx = p[0] - campos[0], vy = p[1] - campos[1], vz = p[2] - campos[2];
       const float tt = -(vx * dx + vy * dy + vz * dz) * nn * nn * nn;
       const float gd[3] = {dx * nn + tt * vx, dy * nn + tt * vy, dz * nn + tt * vz};
@@ -545,7 +554,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
       for (int k = 0; k < cov_w; ++k) g_cov3D[(size_t) cov_w * i + k] = 0.0f;
     if (sh_degree >= 0) {
       if (kStage) {
-        for (int c = kSplit ? 3 : 0; c < n * 3; ++c) my_row[c] = 0.0f;
+        for (int c = kSplit ? 3 : 0; c < (kDerivs ? 0 : n * 3); ++c) my_row[c] = 0.0f;
         if (kSplit && g_shs)
           g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       } else {
@@ -577,7 +586,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, in
           if (cam[12 + k] != 0.0f) atomicAdd(&g_campos[k], cam[12 + k]);
     }
   }
-  if (kWave) {
+  if constexpr (kDerivs) {
+    sh_products_to_global<kRow>(s_wave_rows, g, Y, wave_base, P, kSplit ? g_sh_rest : g_shs);
+  } else if (kWave) {
     wave_lds_sync();
     ShWaveRows<kWave ? kRow : 48>::to_global(s_wave_rows, wave_base, P, kSplit ? g_sh_rest : g_shs);
   } else if (kStage && sh_degree >= 0 && (g_shs || g_sh_rest)) {
@@ -752,25 +763,38 @@ FSGS_API int fsgs_gs_preprocess_forward(int P, int W, int H, int sh_degree, int 
                                  nullptr, ViewOutputs{}, stream);
 }
 
+FSGS_API int fsgs_gs_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
+    const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
+    float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
+    uint32_t* keep_masks, float* color_derivs, void* stream) {
+  FSGS_REQUIRE(!color_derivs || wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0, "gs_view_preprocess: no derivatives of these rows");
+  FSGS_REQUIRE(slot_counters, "gs_view_preprocess: slot_counters are required");
+  return gs3d_preprocess_forward(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest,
+                                 Tw2v, Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp,
+                                 means2D_preserve, means2D, depths, colors, radii, nullptr, cov3Ds, conic_opacity, keep_masks,
+                                 ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, false, color_derivs}, stream);
+}
+
 FSGS_API int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
     const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
     float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
     uint32_t* keep_masks, void* stream) {
-  FSGS_REQUIRE(slot_counters, "gs_view_preprocess: slot_counters are required");
-  return gs3d_preprocess_forward(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest,
-                                 Tw2v, Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp,
-                                 means2D_preserve, means2D, depths, colors, radii, nullptr, cov3Ds, conic_opacity, keep_masks,
-                                 ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible}, stream);
+  return fsgs_gs_view_preprocess_derivs(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v,
+                                        Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp, means2D_preserve,
+                                        means2D, depths, colors, radii, visible, slot_counters, cov3Ds, conic_opacity, keep_masks,
+                                        nullptr, stream);
 }
 
-FSGS_API int fsgs_gs_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
+FSGS_API int fsgs_gs_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
     const float* means3D, const float* scales, const float* rotations, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const int32_t* radii,
-    const float* colors, const float* cov3Ds, const float* cov2Ds, float* grad_mean2D, const float* grad_colors,
-    const float* grad_conic, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
-    float* g_sh_rest, float* g_cov, float* g_Tw2v, float* g_campos, void* stream) {
+    const float* colors, const float* cov3Ds, const float* cov2Ds, const float* color_derivs, float* grad_mean2D,
+    const float* grad_colors, const float* grad_conic, float* g_means3D, float* g_scales, float* g_rot, float* g_opac,
+    float* g_shs, float* g_sh_rest, float* g_cov, float* g_Tw2v, float* g_campos, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0 && tan_fovx > 0 && tan_fovy > 0, "gs_preprocess_backward: bad sizes");
   FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_preprocess_backward: sh_degree %d > %d not supported", sh_degree,
                kMaxShDegree);
@@ -784,14 +808,26 @@ FSGS_API int fsgs_gs_preprocess_backward(int P, int W, int H, int sh_degree, int
     FSGS_REQUIRE(shs && colors && grad_colors, "gs_preprocess_backward: SH path needs shs, colors and grad_colors");
   float* g_rows  = sh_rest ? g_sh_rest : g_shs;
   const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
-  auto kernel = sh_degree > 3 ? gs3d_preprocess_backward_kernel<64, 0>
-                : rows == 48  ? gs3d_preprocess_backward_kernel<16, 48>
-                : rows == 45  ? gs3d_preprocess_backward_kernel<16, 45>
-                              : gs3d_preprocess_backward_kernel<16, 0>;
+  auto kernel = sh_degree > 3 ? gs3d_preprocess_backward_kernel<64, 0, false>
+                : rows == 48  ? (color_derivs ? gs3d_preprocess_backward_kernel<16, 48, true> : gs3d_preprocess_backward_kernel<16, 48, false>)
+                : rows == 45  ? (color_derivs ? gs3d_preprocess_backward_kernel<16, 45, true> : gs3d_preprocess_backward_kernel<16, 45, false>)
+                              : gs3d_preprocess_backward_kernel<16, 0, false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh,
                      is_opengl, means3D, scales, (const float4*) rotations, shs, sh_rest, Tw2v, Tv2c, campos,
                      (float) tan_fovx, (float) tan_fovy, radii, colors, cov3Ds, cov2Ds, (float2*) grad_mean2D,
                      grad_colors, (const float4*) grad_conic, g_means3D, g_scales, (float4*) g_rot, g_opac, g_shs,
-                     g_sh_rest, g_cov, g_Tw2v, g_campos);
+                     g_sh_rest, g_cov, g_Tw2v, g_campos, color_derivs);
   return check_launch("gs_preprocess_backward");
+}
+
+FSGS_API int fsgs_gs_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,
+    const float* means3D, const float* scales, const float* rotations, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const int32_t* radii,
+    const float* colors, const float* cov3Ds, const float* cov2Ds, float* grad_mean2D, const float* grad_colors,
+    const float* grad_conic, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
+    float* g_sh_rest, float* g_cov, float* g_Tw2v, float* g_campos, void* stream) {
+  return fsgs_gs_view_preprocess_backward_derivs(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c,
+                                                 campos, tan_fovx, tan_fovy, radii, colors, cov3Ds, cov2Ds, nullptr, grad_mean2D,
+                                                 grad_colors, grad_conic, g_means3D, g_scales, g_rot, g_opac, g_shs, g_sh_rest,
+                                                 g_cov, g_Tw2v, g_campos, stream);
 }

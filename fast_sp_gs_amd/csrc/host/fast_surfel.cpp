@@ -13,7 +13,8 @@ struct Saved : torch::CustomClassHolder {  // what the backward reads besides te
   double near_n, far_n, depth_ratio;
   bool epilogue;
   int64_t R = 0;
-  size_t colors, trans_mat, inverse_m, normal_opacity, masks, offsets, regions, tiles;  // places in the slab
+  size_t colors, trans_mat, inverse_m, normal_opacity, masks, offsets, regions, tiles, derivs;  // places in the slab
+  bool has_derivs = false;
 };
 
 struct Buffers {
@@ -69,7 +70,10 @@ Buffers forward_view(const FastSurfelView& v, bool train) {
   s.inverse_m = b.keep.reserve((size_t) P * 36);
   s.masks     = b.keep.reserve((size_t) P * 4);
   s.tiles     = b.keep.reserve((size_t) P * 4);
+  const float* sh_rest = has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr;
   if (train) s.offsets = b.keep.reserve((size_t) P * 4), s.regions = b.keep.reserve(kSlotRegions * 4);
+  s.has_derivs = train && fsgs_view_keeps_color_derivs(v.sh_degree, M, f32(v.shs), sh_rest) != 0;
+  if (s.has_derivs) s.derivs = b.keep.reserve((size_t) P * 36);
   b.keep.allocate(like);
   Slab scratch;
   const size_t depths = scratch.reserve((size_t) P * 4);
@@ -94,14 +98,13 @@ Buffers forward_view(const FastSurfelView& v, bool train) {
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
-    check(fsgs_gs_2d_fast_view_preprocess((int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations),
-                                          f32(v.opacities), f32(v.shs),
-                                          has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr,
-                                          f32(v.Tw2v), f32(v.Tv2s), f32(v.campos), data<uint8_t>(opt(v.culling)),
-                                          f32(v.means2D), v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), trans_mat,
-                                          inverse_m, normal_opacity, scratch.at<float>(depths), i32(b.radii),
-                                          data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles),
-                                          train ? b.keep.at<int32_t>(s.offsets) : nullptr, counters.data(), masks, stream),
+    check(fsgs_gs_2d_fast_view_preprocess_derivs(
+              (int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations), f32(v.opacities), f32(v.shs), sh_rest,
+              f32(v.Tw2v), f32(v.Tv2s), f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
+              v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), trans_mat, inverse_m, normal_opacity,
+              scratch.at<float>(depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles),
+              train ? b.keep.at<int32_t>(s.offsets) : nullptr, counters.data(), masks,
+              s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr, stream),
           what);
     check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), inverse_m, f32(v.opacities), i32(b.radii), masks, counters.data(),
                              train ? b.keep.at<int32_t>(s.regions) : nullptr, count, i64(b.ranges), scratch.at<void>(bins),
@@ -236,13 +239,12 @@ struct FastSurfelRender : public torch::autograd::Function<FastSurfelRender> {
                                           (const int32_t*) keep(s.tiles), i32(radii), scratch.at<void>(ws), ws_bytes,
                                           (const uint32_t*) keep(s.masks), (const uint32_t*) i32(t[20]), stream),
             "GS_2D_fast_render_backward");
-      check(fsgs_gs_2d_fast_preprocess_backward((int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations),
-                                                f32(shs), rest_used ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2s),
-                                                f32(campos), keep(s.trans_mat), i32(radii), colors, f32(g_means2D),
-                                                scratch.at<float>(g_trans), scratch.at<float>(g_inv), g_colors,
-                                                scratch.at<float>(g_no), f32(g_points), f32(g_scales), f32(g_rot),
-                                                f32(g_opac), sh ? f32(g_sh) : nullptr, rest_used ? f32(g_rest) : nullptr,
-                                                stream),
+      check(fsgs_gs_2d_fast_view_preprocess_backward_derivs(
+                (int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations), f32(shs),
+                rest_used ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2s), f32(campos), keep(s.trans_mat), i32(radii), colors,
+                s.has_derivs ? keep(s.derivs) : nullptr, f32(g_means2D), scratch.at<float>(g_trans), scratch.at<float>(g_inv),
+                g_colors, scratch.at<float>(g_no), f32(g_points), f32(g_scales), f32(g_rot), f32(g_opac),
+                sh ? f32(g_sh) : nullptr, rest_used ? f32(g_rest) : nullptr, stream),
             "gs_2d_fast_preprocess_backward");
     }
     return first_order_only(upstream, {points, scales, rotations, opacities, shs, sh_rest, means2D},

@@ -10,7 +10,8 @@ struct Saved : torch::CustomClassHolder {  // what the backward reads besides te
   int W, H, sh_degree, E;
   double tan_x, tan_y;
   bool is_opengl;
-  size_t colors, cov3D;  // places in the slab
+  size_t colors, cov3D, derivs;  // places in the slab
+  bool has_derivs = false;
 };
 
 struct Buffers {
@@ -64,6 +65,9 @@ Buffers forward_view(const GaussianView& v, bool train) {
   s.W = W, s.H = H, s.sh_degree = v.sh_degree, s.E = E, s.tan_x = v.tan_x, s.tan_y = v.tan_y, s.is_opengl = v.is_opengl;
   s.colors = b.keep.reserve((size_t) P * 12);
   s.cov3D  = b.keep.reserve(train || !has(v.cov3D) ? (size_t) P * 24 : 0);
+  const float* sh_rest = has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr;
+  s.has_derivs = train && fsgs_view_keeps_color_derivs(v.sh_degree, M, f32(v.shs), sh_rest) != 0;
+  if (s.has_derivs) s.derivs = b.keep.reserve((size_t) P * 36);
   b.keep.allocate(like);
   Slab scratch;
   const size_t depths = scratch.reserve((size_t) P * 4), masks_at = scratch.reserve((size_t) P * 4);
@@ -80,14 +84,14 @@ Buffers forward_view(const GaussianView& v, bool train) {
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
-    check(fsgs_gs_view_preprocess((int) P, W, H, v.sh_degree, M, v.is_opengl, f32(v.points), f32(v.scales),
-                                  f32(v.rotations), f32(v.opacities), f32(v.shs),
-                                  has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr, f32(v.Tw2v),
-                                  f32(v.Tv2c), f32(v.campos), v.tan_x, v.tan_y, data<uint8_t>(opt(v.culling)),
-                                  f32(opt(v.cov3D)), f32(opt(v.cov2D)), v.preserve, f32(v.means2D),
-                                  scratch.at<float>(depths), v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors),
-                                  i32(b.radii), data<uint8_t>(b.visible), counters.data(),
-                                  has(v.cov3D) ? nullptr : b.keep.at<float>(s.cov3D), f32(b.conic_opacity), masks, stream),
+    check(fsgs_gs_view_preprocess_derivs((int) P, W, H, v.sh_degree, M, v.is_opengl, f32(v.points), f32(v.scales),
+                                         f32(v.rotations), f32(v.opacities), f32(v.shs), sh_rest, f32(v.Tw2v), f32(v.Tv2c),
+                                         f32(v.campos), v.tan_x, v.tan_y, data<uint8_t>(opt(v.culling)), f32(opt(v.cov3D)),
+                                         f32(opt(v.cov2D)), v.preserve, f32(v.means2D), scratch.at<float>(depths),
+                                         v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), i32(b.radii),
+                                         data<uint8_t>(b.visible), counters.data(),
+                                         has(v.cov3D) ? nullptr : b.keep.at<float>(s.cov3D), f32(b.conic_opacity), masks,
+                                         s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr, stream),
           what);
     check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
                              nullptr, count, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
@@ -202,13 +206,14 @@ struct GaussianRender : public torch::autograd::Function<GaussianRender> {
             "gaussian_rasterize_backward");
       if (g[2].defined()) g_means2D.add_(g[2]);
       if (g[3].defined()) g_conic.add_(g[3]);
-      check(fsgs_gs_preprocess_backward((int) P, W, H, s.sh_degree, M, s.is_opengl, f32(points), f32(scales), f32(rotations),
-                                        f32(shs), rest_used ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2c), f32(campos),
-                                        s.tan_x, s.tan_y, i32(radii), colors, cov3D.defined() ? f32(cov3D) : keep(s.cov3D),
-                                        f32(cov2D), f32(g_means2D), f32(g_colors), f32(g_conic), f32(g_points),
-                                        f32(g_scales), f32(g_rot), f32(g_opac), f32(g_sh),
-                                        rest_used ? f32(g_rest) : nullptr, f32(cov2D.defined() ? g_cov2D : g_cov3D), nullptr,
-                                        nullptr, stream),
+      check(fsgs_gs_view_preprocess_backward_derivs((int) P, W, H, s.sh_degree, M, s.is_opengl, f32(points), f32(scales),
+                                                    f32(rotations), f32(shs), rest_used ? f32(sh_rest) : nullptr, f32(Tw2v),
+                                                    f32(Tv2c), f32(campos), s.tan_x, s.tan_y, i32(radii), colors,
+                                                    cov3D.defined() ? f32(cov3D) : keep(s.cov3D), f32(cov2D),
+                                                    s.has_derivs ? keep(s.derivs) : nullptr, f32(g_means2D), f32(g_colors),
+                                                    f32(g_conic), f32(g_points), f32(g_scales), f32(g_rot), f32(g_opac),
+                                                    f32(g_sh), rest_used ? f32(g_rest) : nullptr,
+                                                    f32(cov2D.defined() ? g_cov2D : g_cov3D), nullptr, nullptr, stream),
             "gs_preprocess_backward");
     }
     if (!sh && want_sh) g_sh = g_colors;  // pre-computed colours: the blend's sums are their gradient

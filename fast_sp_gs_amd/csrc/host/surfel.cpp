@@ -10,7 +10,8 @@ struct Saved {  // what the backward reads besides tensors
   double near_n, far_n, depth_ratio;
   bool epilogue;
   int64_t R;
-  size_t colors, records, masks, offsets, regions, tiles;  // places in the slab
+  size_t colors, records, masks, offsets, regions, tiles, derivs;  // places in the slab
+  bool has_derivs;
 };
 
 struct Buffers {
@@ -62,12 +63,17 @@ Buffers forward_view(const SurfelView& v, bool train) {
   b.radii = empty({P}, like, at::kInt), b.visible = empty({P}, like, at::kBool);
   b.ranges = empty({T, 2}, like, at::kLong);
   Saved& s = b.saved;
-  s = Saved{W, H, v.sh_degree, v.near_n, v.far_n, v.depth_ratio, v.epilogue, 0, 0, 0, 0, 0, 0, 0};
+  s = Saved{W, H, v.sh_degree, v.near_n, v.far_n, v.depth_ratio, v.epilogue, 0, 0, 0, 0, 0, 0, 0, 0, false};
   s.records = b.keep.reserve((size_t) P * 80);
   s.colors  = b.keep.reserve((size_t) P * 12);
   s.masks   = b.keep.reserve((size_t) P * 4);
   s.tiles   = b.keep.reserve((size_t) P * 4);
-  if (train) s.offsets = b.keep.reserve((size_t) P * 4), s.regions = b.keep.reserve(kSlotRegions * 4);
+  const float* sh_rest = has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr;
+  if (train) {
+    s.offsets = b.keep.reserve((size_t) P * 4), s.regions = b.keep.reserve(kSlotRegions * 4);
+    s.has_derivs = fsgs_view_keeps_color_derivs(v.sh_degree, M, f32(v.shs), sh_rest) != 0;
+    if (s.has_derivs) s.derivs = b.keep.reserve((size_t) P * 36);
+  }
   b.keep.allocate(like);
   Slab scratch;
   const size_t depths = scratch.reserve((size_t) P * 4);
@@ -92,17 +98,18 @@ Buffers forward_view(const SurfelView& v, bool train) {
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
-    auto preprocess = [&](auto entry, auto... slot_offsets) {
+    auto preprocess = [&](auto entry, auto... outputs) {
       check(entry((int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations), f32(v.opacities), f32(v.shs),
-                  has(v.sh_rest) && v.sh_rest->numel() > 0 ? f32(*v.sh_rest) : nullptr, f32(v.Tw2v), f32(v.Tv2c),
-                  f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
+                  sh_rest, f32(v.Tw2v), f32(v.Tv2c), f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
                   v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), f32(b.trans_mat), f32(b.normal_opacity),
-                  scratch.at<float>(depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles),
-                  slot_offsets..., counters.data(), records, masks, stream),
+                  scratch.at<float>(depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles), outputs...,
+                  stream),
             what);
     };
-    if (train) preprocess(fsgs_gs_2d_view_preprocess, b.keep.at<int32_t>(s.offsets));
-    else preprocess(fsgs_gs_2d_view_preprocess_no_backward);
+    if (train)
+      preprocess(fsgs_gs_2d_view_preprocess_derivs, b.keep.at<int32_t>(s.offsets), counters.data(), records, masks,
+                 s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr);
+    else preprocess(fsgs_gs_2d_view_preprocess_no_backward, counters.data(), records, masks);
     check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
                              train ? b.keep.at<int32_t>(s.regions) : nullptr, count, i64(b.ranges), scratch.at<void>(bins),
                              bins_bytes, stream),
@@ -251,12 +258,12 @@ struct SurfelRender : public torch::autograd::Function<SurfelRender> {
                                      (const int32_t*) keep(s.tiles), i32(radii), scratch.at<void>(ws), ws_bytes,
                                      (const float*) keep(s.records), (const uint32_t*) i32(t[22]), stream),
             "GS_2D_render_backward");
-      check(fsgs_gs_2d_view_preprocess_backward(
+      check(fsgs_gs_2d_view_preprocess_backward_derivs(
                 (int) P, W, H, s.sh_degree, M, f32(points), f32(scales), f32(rotations), f32(shs),
                 has_rest && sh_rest.numel() > 0 ? f32(sh_rest) : nullptr, f32(Tw2v), f32(Tv2c), f32(campos),
                 f32(trans_mat), i32(radii), colors, (const int32_t*) keep(s.offsets), (const int32_t*) keep(s.regions),
                 (const int32_t*) keep(s.tiles), holder->cull ? (const uint32_t*) keep(s.masks) : nullptr,
-                scratch.at<const float>(ws), f32(g_means2D), f32(g_points), f32(g_scales), f32(g_rot), f32(g_opac),
+                scratch.at<const float>(ws), s.has_derivs ? (const float*) keep(s.derivs) : nullptr, f32(g_means2D), f32(g_points), f32(g_scales), f32(g_rot), f32(g_opac),
                 s.sh_degree >= 0 ? f32(g_sh) : nullptr, has_rest && sh_rest.numel() > 0 ? f32(g_rest) : nullptr, stream),
             "gs_2d_preprocess_backward");
     }

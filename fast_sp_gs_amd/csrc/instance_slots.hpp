@@ -74,6 +74,7 @@ struct ViewOutputs {
   int32_t* slot_offsets = nullptr;
   uint8_t* visible = nullptr;
   bool windows = false;  // no backward follows: keep masks of large rectangles may be windows (cull_window)
+  float* color_derivs = nullptr;  // [P, 9], for the backward; only where the coefficients' rows are complete (wave_row_floats)
 };
 
 // What the kernel behind the preprocess hands on: see above. `counters` nullptr: nothing to do.

@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
-  float dc[3] = {0, 0, 0};
+  float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
   if (kSplit && valid) dc[0] = shs[3 * (size_t) i], dc[1] = shs[3 * (size_t) i + 1], dc[2] = shs[3 * (size_t) i + 2];
   do {
     if (!valid || (culling && culling[i])) break;
@@ -193,6 +193,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
       for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
       rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+      if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
     }
   }
   if (view.slot_offsets) {
@@ -228,6 +229,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     if (trans_precomp == nullptr) wave_rows_out<9>(s_wave_rows, wave_base, P, trans_mat);
     wave_rows_out<3>(s_wave_rows + 576, wave_base, P, colors);
   }
+  if (kWave && view.color_derivs) wave_derivs_out(s_wave_rows, derivs, wave_base, P, view.color_derivs);
   if (!valid) return;
 
   if (view.slot_offsets) view.slot_offsets[i] = slot;
@@ -429,7 +431,12 @@ __device__ __forceinline__ void wave_record_sums(const ViewRecords& in, int firs
 // kRecords: the upstream gradients are the sums of the view's records, taken here: summed by a kernel of its own they went
 // through memory once more (72 bytes per surfel out and in), and that kernel waited for three dependent loads per seven
 // surfels and wavefront. 3M surfels 1352x1014: sum 244 + preprocess 325 us -> 376 us; 300k 800x800: 34 + 36 -> 65 us.
-template <int kSh, int kRow, bool kRecords>
+// kDerivs: the forward left the colours' derivatives (36 bytes a surfel), and the rows of coefficients (192 bytes) are not read again. Bound
+// by memory at 3M surfels (about 1.4 GB at 5.2 TB/s); with fewer, by the trips to the records. Kernel, us, 3M 1352x1014 / 300k 800x800 /
+// 10k 256x256: 331 / 47 / 11.3 with the coefficients, 302 / 41 / 10.4 with the derivatives and LDS for 64 rows a wavefront (three of
+// them per SIMD), 266 / 40 / 9.6 with half of the rows at a time (sh_products_to_global: four). For that the forward takes 217, 36 and
+// 10.5 instead of 198, 33 and 9.7.
+template <int kSh, int kRow, bool kRecords, bool kDerivs>
 __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
     const float4* __restrict__ rotations, const float* __restrict__ shs, const float* __restrict__ sh_rest,
@@ -438,12 +445,15 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     float2* __restrict__ grad_mean2D, const float* __restrict__ grad_trans, const float* __restrict__ grad_colors,
     const float4* __restrict__ grad_normal_opacity, float* __restrict__ g_means3D, float2* __restrict__ g_scales,
     float4* __restrict__ g_rot, float* __restrict__ g_opac, float* __restrict__ g_shs,
-    float* __restrict__ g_sh_rest, ViewRecords view) {
+    float* __restrict__ g_sh_rest, ViewRecords view, const float* __restrict__ color_derivs) {
+  static_assert(!kDerivs || kRow != 0);
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : kRecords ? 4 * kSumFloats : 1];
+  constexpr int kWaveFloats = kDerivs ? kSumFloats : 64 * kStride;  // of LDS
+  static_assert(!kDerivs || kSumFloats >= kShHalfRows * kStride);
+  __shared__ __align__(16) float s_rows[kStage ? 4 * kWaveFloats : kRecords ? 4 * kSumFloats : 1];
   __shared__ unsigned char s_flag[kShStageRows];
   load_camera(Tw2v_g, Tv2c_g, s_Tw2v, s_Tw2c);
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
@@ -459,15 +469,16 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
   const bool vis   = valid && radii[i] > 0;
   const int n      = sh_degree >= 0 ? sh_count(sh_degree) : 0;
   const int m1     = sh_rest ? 1 : n_sh;
-  float* my_row    = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
+  float* my_row    = &s_rows[kStage && !kDerivs ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveFloats : 0];
   const unsigned long long wanted = kWave ? __ballot(vis) : 0ull;
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   float up[kRecords ? kGradFloats : 1];
-  if (kWave && wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
+  if (kWave && !kDerivs && wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
   // what the geometry reads of the surfel
   float M[9], p[3] = {0, 0, 0}, col[3] = {0, 0, 0};
+  float derivs[kColorDerivs] = {};
   float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float2 s = make_float2(0.0f, 0.0f);
 #pragma unroll
@@ -481,10 +492,13 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     if (sh_degree >= 0)
 #pragma unroll
       for (int k = 0; k < 3; ++k) col[k] = colors[3 * (size_t) i + k];
+    if (kDerivs)
+#pragma unroll
+      for (int k = 0; k < kColorDerivs; ++k) derivs[k] = color_derivs[kColorDerivs * (size_t) i + k];
   }
   if (kRecords) {  // the rows of coefficients and the above are on their way meanwhile
     static_assert(!kStage || 64 * kStride >= kSumFloats, "the sums fit where the rows will be");
-    float* s_sums = &s_rows[kStage ? (threadIdx.x & ~63) * kStride : (threadIdx.x >> 6) * kSumFloats];
+    float* s_sums = &s_rows[(threadIdx.x >> 6) * (kStage ? kWaveFloats : kSumFloats)];
     wave_record_sums(view, first, count, mask, vis, s_sums);
     wave_lds_sync();
     if (vis) {
@@ -510,8 +524,10 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       }
       return;
     }
-    sh_regs.to_lds(s_wave_rows, wave_base, P);
-    wave_lds_sync();
+    if (!kDerivs) {
+      sh_regs.to_lds(s_wave_rows, wave_base, P);
+      wave_lds_sync();
+    }
   } else if (kStage && sh_degree >= 0) {
     s_flag[threadIdx.x] = vis;
     __syncthreads();
@@ -519,6 +535,9 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     __syncthreads();
   }
 
+  float g[3] = {}, Y[kSh];  // the colour's gradient and the basis: their products are the gradients of the coefficients
+#pragma unroll
+  for (int l = 0; l < (kDerivs ? kSh : 0); ++l) Y[l] = 0.0f;
   if (vis) {
     float Tw2v[16], Tw2c[16];
 #pragma unroll
@@ -548,31 +567,28 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     transmat_backward(W, H, s.x, s.y, q, Tw2c, Tw2v, gM, gN, gp, gs, gq);
 
     if (sh_degree >= 0) {
-      float x, y, z, Y[kSh], tl[kSh];
+      float x, y, z;
       const float nn = view_dir(p, campos, x, y, z);
       sh_eval(sh_degree, x, y, z, Y);
-      float g[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) g[c] = (kRecords ? up[c * kUp] : grad_colors[3 * (size_t) i + c]) * (float) (col[c] > 0);
       // coefficient rows are read from LDS when staged, and each gradient row is written over the coefficients it
       // was computed from (a lane only ever touches its own row)
       const float* c0 = kStage ? my_row : shs + (size_t) i * m1 * 3;
       const float* cr = kStage ? my_row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float* o0  = kStage && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
-      float* orr = kStage ? my_row
+      float* o0  = kDerivs && !kSplit ? nullptr : kStage && !kSplit ? my_row : (g_shs ? g_shs + (size_t) i * m1 * 3 : nullptr);
+      float* orr = kDerivs ? nullptr : kStage ? my_row
                           : (sh_rest ? (g_sh_rest ? g_sh_rest + (size_t) i * n_sh * 3 - 3 : nullptr) : o0);
       if (o0) o0[0] = g[0] * Y[0], o0[1] = g[1] * Y[0], o0[2] = g[2] * Y[0];
-      tl[0] = 0.0f;
-      for (int l = 1; l < n; ++l) {
-        tl[l] = g[0] * cr[3 * l] + g[1] * cr[3 * l + 1] + g[2] * cr[3 * l + 2];
+      const float dir[3] = {x, y, z};
+      float dx = 0, dy = 0, dz = 0;
+      sh_direction_part<kSh, kDerivs>(sh_degree, dir, g, cr, derivs, dx, dy, dz);  // before the coefficients are written over
+      for (int l = 1; l < n; ++l)
         if (orr) orr[3 * l] = g[0] * Y[l], orr[3 * l + 1] = g[1] * Y[l], orr[3 * l + 2] = g[2] * Y[l];
-      }
       if (!kStage && orr) {  // coefficients above the active degree
         for (int l = n; l < (sh_rest ? n_sh + 1 : n_sh); ++l)
           orr[3 * l] = 0.0f, orr[3 * l + 1] = 0.0f, orr[3 * l + 2] = 0.0f;
       }
-      float dx = 0, dy = 0, dz = 0;
-      sh_grad_accumulate(sh_degree, x, y, z, tl, dx, dy, dz);
       const float vx = p[0] - campos[0], vy = p[1] - campos[1], vz = p[2] - campos[2];
       const float tt = -(vx * dx + vy * dy + vz * dz) * nn * nn * nn;
       gp[0] = gp[0] + (dx * nn + tt * vx);
@@ -593,7 +609,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     g_rot[i]    = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (sh_degree >= 0) {
       if (kStage) {
-        for (int c = kSplit ? 3 : 0; c < n * 3; ++c) my_row[c] = 0.0f;
+        for (int c = kSplit ? 3 : 0; c < (kDerivs ? 0 : n * 3); ++c) my_row[c] = 0.0f;
         if (kSplit && g_shs)
           g_shs[3 * (size_t) i] = 0.0f, g_shs[3 * (size_t) i + 1] = 0.0f, g_shs[3 * (size_t) i + 2] = 0.0f;
       } else {
@@ -604,7 +620,9 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
       }
     }
   }
-  if (kWave) {
+  if constexpr (kDerivs) {
+    sh_products_to_global<kRow>(s_wave_rows, g, Y, wave_base, P, kSplit ? g_sh_rest : g_shs);
+  } else if (kWave) {
     wave_lds_sync();
     ShWaveRows<kWave ? kRow : 48>::to_global(s_wave_rows, wave_base, P, kSplit ? g_sh_rest : g_shs);
   } else if (kStage && sh_degree >= 0 && (g_shs || g_sh_rest)) {
@@ -656,6 +674,10 @@ __global__ void __launch_bounds__(256) transmat_backward_kernel(int P, int W, in
 
 using namespace fsgs;
 
+FSGS_API int fsgs_view_keeps_color_derivs(int sh_degree, int n_sh, const float* shs, const float* sh_rest) {
+  return wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0;
+}
+
 namespace {
 int preprocess_forward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
@@ -696,16 +718,27 @@ FSGS_API int fsgs_gs_2d_preprocess_forward(int P, int W, int H, int sh_degree, i
                             depths, radii, tiles_touched, records, keep_masks, ViewOutputs{}, stream);
 }
 
+FSGS_API int fsgs_gs_2d_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
+  FSGS_REQUIRE(!color_derivs || wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0, "gs_2d_view_preprocess: no derivatives of these rows");
+  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
+                            tiles_touched, records, keep_masks,
+                            ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible, false, color_derivs}, stream);
+}
+
 FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
     float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
     int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream) {
-  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
-  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
-                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
-                            tiles_touched, records, keep_masks,
-                            ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible}, stream);
+  return fsgs_gs_2d_view_preprocess_derivs(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                                           campos, culling, means2D, colors, trans_mat, normal_opacity, depths, radii, visible,
+                                           tiles_touched, slot_offsets, slot_counters, records, keep_masks, nullptr, stream);
 }
 
 FSGS_API int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
@@ -726,7 +759,8 @@ int preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const floa
     const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v, const float* Tv2c,
     const float* campos, const float* trans_mat, const int32_t* radii, const float* colors, float* grad_mean2D,
     const float* grad_trans, const float* grad_colors, const float* grad_normal_opacity, float* g_means3D,
-    float* g_scales, float* g_rot, float* g_opac, float* g_shs, float* g_sh_rest, const ViewRecords& view, void* stream) {
+    float* g_scales, float* g_rot, float* g_opac, float* g_shs, float* g_sh_rest, const ViewRecords& view,
+    const float* color_derivs, void* stream) {
   FSGS_REQUIRE(P >= 0 && W > 0 && H > 0, "gs_2d_preprocess_backward: bad sizes");
   FSGS_REQUIRE(sh_degree <= kMaxShDegree, "gs_2d_preprocess_backward: sh_degree %d > %d not supported", sh_degree,
                kMaxShDegree);
@@ -739,14 +773,15 @@ int preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const floa
   if (P == 0) return kOk;
   float* g_rows  = sh_rest ? g_sh_rest : g_shs;
   const int rows = g_rows ? wave_row_floats(sh_degree, n_sh, shs, sh_rest, g_rows) : 0;
-  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, 0, kRecords>
-                : rows == 48  ? preprocess_backward_kernel<16, 48, kRecords>
-                : rows == 45  ? preprocess_backward_kernel<16, 45, kRecords>
-                              : preprocess_backward_kernel<16, 0, kRecords>;
+  const bool derivs = kRecords && color_derivs;
+  auto kernel = sh_degree > 3 ? preprocess_backward_kernel<64, 0, kRecords, false>
+                : rows == 48  ? (derivs ? preprocess_backward_kernel<16, 48, kRecords, kRecords> : preprocess_backward_kernel<16, 48, kRecords, false>)
+                : rows == 45  ? (derivs ? preprocess_backward_kernel<16, 45, kRecords, kRecords> : preprocess_backward_kernel<16, 45, kRecords, false>)
+                              : preprocess_backward_kernel<16, 0, kRecords, false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, W, H, sh_degree, n_sh, means3D, (const float2*) scales, (const float4*) rotations, shs, sh_rest, Tw2v,
                      Tv2c, campos, trans_mat, radii, colors, (float2*) grad_mean2D, grad_trans, grad_colors,
                      (const float4*) grad_normal_opacity, g_means3D, (float2*) g_scales, (float4*) g_rot, g_opac,
-                     g_shs, g_sh_rest, view);
+                     g_shs, g_sh_rest, view, color_derivs);
   return check_launch("gs_2d_preprocess_backward");
 }
 }  // namespace
@@ -758,15 +793,15 @@ FSGS_API int fsgs_gs_2d_preprocess_backward(int P, int W, int H, int sh_degree, 
     float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs, float* g_sh_rest, void* stream) {
   return preprocess_backward<false>(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c, campos,
                                     trans_mat, radii, colors, grad_mean2D, grad_trans, grad_colors, grad_normal_opacity,
-                                    g_means3D, g_scales, g_rot, g_opac, g_shs, g_sh_rest, ViewRecords{}, stream);
+                                    g_means3D, g_scales, g_rot, g_opac, g_shs, g_sh_rest, ViewRecords{}, nullptr, stream);
 }
 
-FSGS_API int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+FSGS_API int fsgs_gs_2d_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
     const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
     const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
-    const float* slot_grads, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
-    float* g_sh_rest, void* stream) {
+    const float* slot_grads, const float* color_derivs, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot,
+    float* g_opac, float* g_shs, float* g_sh_rest, void* stream) {
   FSGS_REQUIRE(P == 0 || (slot_offsets && slot_regions && tiles_touched && slot_grads),
                "gs_2d_view_preprocess_backward: record slots and records are required");
   ViewRecords view;
@@ -775,7 +810,19 @@ FSGS_API int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_deg
   view.records = slot_grads;
   return preprocess_backward<true>(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c, campos,
                                    trans_mat, radii, colors, g_means2D, nullptr, nullptr, nullptr, g_means3D, g_scales,
-                                   g_rot, g_opac, g_shs, g_sh_rest, view, stream);
+                                   g_rot, g_opac, g_shs, g_sh_rest, view, color_derivs, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
+    const float* slot_grads, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
+    float* g_sh_rest, void* stream) {
+  return fsgs_gs_2d_view_preprocess_backward_derivs(P, W, H, sh_degree, n_sh, means3D, scales, rotations, shs, sh_rest, Tw2v, Tv2c,
+                                                    campos, trans_mat, radii, colors, slot_offsets, slot_regions, tiles_touched,
+                                                    keep_masks, slot_grads, nullptr, g_means2D, g_means3D, g_scales, g_rot,
+                                                    g_opac, g_shs, g_sh_rest, stream);
 }
 
 FSGS_API int fsgs_gs_2d_compute_transmat_forward(int P, int W, int H, const float* means3D, const float* scales,

@@ -80,6 +80,53 @@ __device__ __forceinline__ void sh_grad_accumulate(int degree, T x, T y, T z, co
   if constexpr (kN > 16) sh_grad_accumulate_high(degree, x, y, z, t, dx, dy, dz);
 }
 
+// Derivatives of a colour's three channels by the unit direction, degree <= 3: j[3 c + k] = d colour_c / d direction_k, from the
+// coefficients `coef(l, c)`. A view's forward keeps them (36 bytes a point) where its backward would read the coefficients again
+// (192); every other backward forms them here, in the same operations, so that both round alike.
+template <typename Coef>
+__device__ __forceinline__ void sh_color_derivatives(int degree, float x, float y, float z, Coef coef, float (&j)[9]) {
+#pragma clang fp contract(off)
+  if (degree < 1) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) j[k] = 0.0f;
+    return;
+  }
+  constexpr float k1 = 0.48860251190291992f, k4 = 1.0925484305920792f, k10 = 2.8906114426405538f, k15 = 1.7701307697799304f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) j[3 * c] = -k1 * coef(3, c), j[3 * c + 1] = -k1 * coef(1, c), j[3 * c + 2] = k1 * coef(2, c);
+  if (degree < 2) return;
+  const float x4 = k4 * x, y4 = k4 * y, z4 = k4 * z, z6 = 1.8923493915151202f * z;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    float &jx = j[3 * c], &jy = j[3 * c + 1], &jz = j[3 * c + 2];
+    const float c4 = coef(4, c), c5 = coef(5, c), c7 = coef(7, c), c8 = coef(8, c);
+    jx = fmaf(c4, y4, jx), jx = fmaf(-c7, z4, jx), jx = fmaf(c8, x4, jx);
+    jy = fmaf(c4, x4, jy), jy = fmaf(-c5, z4, jy), jy = fmaf(-c8, y4, jy);
+    jz = fmaf(-c5, y4, jz), jz = fmaf(coef(6, c), z6, jz), jz = fmaf(-c7, x4, jz);
+  }
+  if (degree < 3) return;
+  const float xx = x * x, yy = y * y, zz = z * z, xy = x * y, yz = y * z, xz = x * z;
+  const float xy9 = 2.0f * k15 * xy, d9 = k15 * (yy - xx), xy10 = k10 * xy, xz10 = k10 * xz, yz10 = k10 * yz;
+  const float z11 = fmaf(-2.2852289973223288f, zz, 0.45704579946446572f), xz11 = 4.5704579946446566f * xz, yz11 = 4.5704579946446566f * yz;
+  const float z12 = fmaf(5.597644988851731f, zz, -1.1195289977703462f), d14 = 1.4453057213202769f * (xx - yy);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    float &jx = j[3 * c], &jy = j[3 * c + 1], &jz = j[3 * c + 2];
+    const float c9 = coef(9, c), c10 = coef(10, c), c11 = coef(11, c), c13 = coef(13, c), c14 = coef(14, c), c15 = coef(15, c);
+    jx = fmaf(-c9, xy9, jx), jx = fmaf(c10, yz10, jx), jx = fmaf(c13, z11, jx), jx = fmaf(c14, xz10, jx), jx = fmaf(c15, d9, jx);
+    jy = fmaf(c9, d9, jy), jy = fmaf(c10, xz10, jy), jy = fmaf(c11, z11, jy), jy = fmaf(-c14, yz10, jy), jy = fmaf(c15, xy9, jy);
+    jz = fmaf(c10, xy10, jz), jz = fmaf(-c11, yz11, jz), jz = fmaf(coef(12, c), z12, jz), jz = fmaf(-c13, xz11, jz), jz = fmaf(c14, d14, jz);
+  }
+}
+
+// The upstream gradient of the direction from that of the colour.
+__device__ __forceinline__ void sh_direction_gradient(const float (&g)[3], const float (&j)[9], float& dx, float& dy, float& dz) {
+#pragma clang fp contract(off)
+  dx = fmaf(g[2], j[6], fmaf(g[1], j[3], g[0] * j[0]));
+  dy = fmaf(g[2], j[7], fmaf(g[1], j[4], g[0] * j[1]));
+  dz = fmaf(g[2], j[8], fmaf(g[1], j[5], g[0] * j[2]));
+}
+
 // ---- the bare encoder on half tensors, degree <= 3 -----------------------------------------------------------------------
 // With scalar_t = at::Half the reference keeps its monomials (xy, xz, yz, x2, y2, z2) and, in the backward, the three
 // running sums in half: a product of two halves is formed in float and rounded to half (shencoder.cu:31-33, 190-193),

@@ -4,6 +4,7 @@
 // reads (writes) every line once. Used when the active degree is <= 3 (at most 16 coefficients, 48 floats per row).
 #pragma once
 #include "common.hpp"
+#include "sh.hpp"
 
 namespace fsgs {
 
@@ -110,8 +111,9 @@ struct ShWaveRows {
   ShPiece v[kVecs];
   float tail;
 
-  // floats and complete pieces of the wavefront's existing rows
-  static __device__ __forceinline__ int floats(int wave_base, int P) { return max(min(64, P - wave_base), 0) * kFloats; }
+  // floats of the wavefront's existing rows
+  template <int kRows = 64>
+  static __device__ __forceinline__ int floats(int wave_base, int P) { return max(min(kRows, P - wave_base), 0) * kFloats; }
 
   // `flags` has bit r set for the rows that are needed (all of them existing rows); a piece of other rows re-reads the
   // first needed row's instead of branching. flags must not be 0.
@@ -159,13 +161,14 @@ struct ShWaveRows {
     }
   }
 
-  // Writes the wavefront's staged rows (every existing row) to dst.
+  // Writes the wavefront's staged rows (every existing row; kRows at most, from wave_base on) to dst.
+  template <int kRows = 64>
   static __device__ __forceinline__ void to_global(const float* __restrict__ s_wave_rows, int wave_base, int P,
                                                    float* __restrict__ dst) {
-    const int all = floats(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
+    const int all = floats<kRows>(wave_base, P), whole = all >> 2, lane = (int) __lane_id();
     float* row = dst + (size_t) wave_base * kFloats;
 #pragma unroll
-    for (int k = 0; k < kVecs; ++k) {
+    for (int k = 0; k < (kRows * kFloats / 4 + 63) / 64; ++k) {
       const int e = k * 64 + lane;
       if (kFloats % 2 == 1) {
         if (e < whole) __builtin_nontemporal_store(*(const ShPiece*) (s_wave_rows + 4 * e), (ShPiece*) row + e);
@@ -208,6 +211,63 @@ inline int wave_row_floats(int sh_degree, int n_sh, const float* shs, const floa
   if (sh_degree != 3 || n_sh != (sh_rest ? 15 : 16)) return 0;
   if ((((uintptr_t) (sh_rest ? sh_rest : shs) | (uintptr_t) g_rows) & 15) != 0) return 0;
   return sh_rest ? 45 : 48;
+}
+
+// The derivatives of the colours by the direction (sh_color_derivatives) that a view's forward leaves for its backward: a row of
+// nine floats per point.
+constexpr int kColorDerivs = 9;
+
+// Leaves a wavefront's rows of them (`derivs`, of every lane; aligned as wave_rows_out asks) by way of the LDS that held its rows.
+__device__ __forceinline__ void wave_derivs_out(float* __restrict__ s_wave_rows, const float (&derivs)[kColorDerivs], int wave_base,
+                                                int P, float* __restrict__ dst) {
+  const int lane = (int) __lane_id();
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < kColorDerivs; ++k) s_wave_rows[kColorDerivs * lane + k] = derivs[k];
+  wave_lds_sync();
+  wave_rows_out<kColorDerivs>(s_wave_rows, wave_base, P, dst);
+}
+
+// The gradients of a wavefront's rows of kRow coefficients (48, or 45 with the first coefficient apart) where nothing is read from
+// them: the products of a lane's colour gradient `g` and basis `Y` (zeros where there is no gradient). Half of the rows at a time
+// pass through the LDS, so that it holds 32 rows of a wavefront, and more of them share a compute unit than with room for all 64.
+constexpr int kShHalfRows = 32;
+template <int kRow>
+__device__ __forceinline__ void sh_products_to_global(float* __restrict__ s_half_rows, const float (&g)[3], const float (&Y)[16],
+                                                      int wave_base, int P, float* __restrict__ dst) {
+  static_assert(kShHalfRows * kRow % 4 == 0);
+  constexpr int kStride = kRow | 1, kFirst = (48 - kRow) / 3;
+  const int lane = (int) __lane_id();
+  float* row = s_half_rows + (lane & (kShHalfRows - 1)) * kStride;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    wave_lds_sync();
+    if (lane / kShHalfRows == h) {
+#pragma unroll
+      for (int l = kFirst; l < 16; ++l)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) row[3 * (l - kFirst) + c] = g[c] * Y[l];
+    }
+    wave_lds_sync();
+    ShWaveRows<kRow>::template to_global<kShHalfRows>(s_half_rows, wave_base + h * kShHalfRows, P, dst);
+  }
+}
+
+// A backward's gradient of the view direction `dir`: from the forward's derivatives (kDerivs), or from the coefficients (`rows`:
+// coefficient l of channel c at 3 l + c).
+template <int kSh, bool kDerivs>
+__device__ __forceinline__ void sh_direction_part(int degree, const float (&dir)[3], const float (&g)[3], const float* rows,
+                                                  float (&derivs)[kColorDerivs], float& dx, float& dy, float& dz) {
+  if constexpr (kSh == 16) {
+    if (!kDerivs) sh_color_derivatives(degree, dir[0], dir[1], dir[2], [&](int l, int c) { return rows[3 * l + c]; }, derivs);
+    sh_direction_gradient(g, derivs, dx, dy, dz);
+  } else {
+    const int n = sh_count(degree);
+    float tl[kSh];
+    tl[0] = 0.0f;
+    for (int l = 1; l < n; ++l) tl[l] = g[0] * rows[3 * l] + g[1] * rows[3 * l + 1] + g[2] * rows[3 * l + 2];
+    sh_grad_accumulate(degree, dir[0], dir[1], dir[2], tl, dx, dy, dz);
+  }
 }
 
 }  // namespace fsgs

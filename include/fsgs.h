@@ -66,6 +66,17 @@ int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, i
     float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
     uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream);
 
+/* _derivs, of the surfels' preprocess and of the other two kinds' below: leaves the colours' derivatives by the view direction, too, nine
+ * floats per point (channel-major; on a 16-byte boundary, zeros for points that are not rendered; nullptr: none), which the _derivs form
+ * of the backward reads instead of the coefficients. Only for the rows of coefficients that fsgs_view_keeps_color_derivs accepts (all
+ * of degree 3, on a 16-byte boundary). */
+int fsgs_view_keeps_color_derivs(int sh_degree, int n_sh, const float* shs, const float* sh_rest);
+int fsgs_gs_2d_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
+    const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
+    float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, void* stream);
+
 /* gs_2d_preprocess_backward -- gs_2d_preprocess.cu:423-499 (kernel :268-329). Every row of g_* is ASSIGNED: the
  * gradient for surfels with radii > 0, zeros for the others and for SH coefficients above the active degree (the
  * reference relies on its caller's zero-fill for those), so the outputs need no initialisation. grad_mean2D[P,2] is
@@ -266,6 +277,12 @@ int fsgs_gs_2d_view_preprocess_backward(int P, int W, int H, int sh_degree, int 
     const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
     const float* slot_grads, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot, float* g_opac,
     float* g_shs, float* g_sh_rest, void* stream);
+int fsgs_gs_2d_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    const int32_t* slot_offsets, const int32_t* slot_regions, const int32_t* tiles_touched, const uint32_t* keep_masks,
+    const float* slot_grads, const float* color_derivs, float* g_means2D, float* g_means3D, float* g_scales, float* g_rot,
+    float* g_opac, float* g_shs, float* g_sh_rest, void* stream);
 
 /* ---- "fast" surfel path: transform through camera intrinsics Tv2s[3,3], adjugate-based intersection, fused
  * corner-test binning. Optical flow (trans_mat_t2) is carried by the two blend entry points below. ---- */
@@ -289,6 +306,11 @@ int fsgs_gs_2d_fast_view_preprocess(int P, int W, int H, int sh_degree, int n_sh
     const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
     float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
     int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, void* stream);
+int fsgs_gs_2d_fast_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2s, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* inverse_m, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible,
+    int32_t* tiles_touched, int32_t* slot_offsets, uint64_t* slot_counters, uint32_t* keep_masks, float* color_derivs, void* stream);
 
 /* Binning half of gs_2d_fast_preprocess_forward -- gs_2d_fast_preprocess.cu:264-327 (duplicateWithKeys with the
  * per-tile corner test, x-major, unused slots padded with key = T << 32 / value = -1), :711-778 (sort on
@@ -311,6 +333,12 @@ int fsgs_gs_2d_fast_preprocess_backward(int P, int W, int H, int sh_degree, int 
     const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2s, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
     float* grad_mean2D, const float* grad_trans, const float* grad_inv_m, const float* grad_colors,
+    const float* grad_normal_opacity, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
+    float* g_sh_rest, void* stream);
+int fsgs_gs_2d_fast_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2s, const float* campos, const float* trans_mat, const int32_t* radii, const float* colors,
+    const float* color_derivs, float* grad_mean2D, const float* grad_trans, const float* grad_inv_m, const float* grad_colors,
     const float* grad_normal_opacity, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
     float* g_sh_rest, void* stream);
 
@@ -574,6 +602,12 @@ int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, int is
     const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
     float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
     uint32_t* keep_masks, void* stream);
+int fsgs_gs_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
+    const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
+    float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
+    uint32_t* keep_masks, float* color_derivs, void* stream);
 
 /* gs_preprocess_backward -- gaussian_preprocess.cu:567-636 (kernel :246-372, with gaussian_compute_cov2D.cu:64-186 and
  * gaussian_compute_cov3D.cu:76-118). grad_mean2D[P,2] is rewritten in place as (0.5 W g.x, +-0.5 H g.y) as in the
@@ -588,6 +622,12 @@ int fsgs_gs_preprocess_backward(int P, int W, int H, int sh_degree, int n_sh, in
     const float* colors, const float* cov3Ds, const float* cov2Ds, float* grad_mean2D, const float* grad_colors,
     const float* grad_conic, float* g_means3D, float* g_scales, float* g_rot, float* g_opac, float* g_shs,
     float* g_sh_rest, float* g_cov, float* g_Tw2v, float* g_campos, void* stream);
+int fsgs_gs_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
+    const float* scales, const float* rotations, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const int32_t* radii,
+    const float* colors, const float* cov3Ds, const float* cov2Ds, const float* color_derivs, float* grad_mean2D,
+    const float* grad_colors, const float* grad_conic, float* g_means3D, float* g_scales, float* g_rot, float* g_opac,
+    float* g_shs, float* g_sh_rest, float* g_cov, float* g_Tw2v, float* g_campos, void* stream);
 
 /* gaussian_topk_weights -- fast_2d_gs/_C/src/gaussian_splatting/gaussian_topk.cu:212-228 (kernel :12-93): per pixel
  * the topk (<= 16) largest blend weights of the 3D-Gaussian rasteriser and their Gaussian ids, descending;
