@@ -19,7 +19,7 @@ OBJ_DIR = PKG_DIR / "build"
 LIB_PATH = PKG_DIR / "libfsgs_hip.so"
 HOST_SRC = CSRC / "host"
 HOST_PATH = PKG_DIR / "_host.so"
-HOST_SOURCES = ["torch_util.cpp", "surfel.cpp", "fast_surfel.cpp", "gaussian.cpp", "deform.cpp", "module.cpp"]
+HOST_SOURCES = ["torch_util.cpp", "surfel.cpp", "fast_surfel.cpp", "gaussian.cpp", "deform.cpp", "encode.cpp", "module.cpp"]
 SOURCES = ["api.hip", "preprocess.hip", "binning.hip", "blend_fwd.hip", "blend_bwd.hip", "blend_topk.hip", "fast_preprocess.hip",
            "fast_blend.hip", "point_ops.hip", "knn_grid.hip", "lbs_bwd.hip", "ssim.hip", "epilogue.hip", "simple_knn.hip", "compaction.hip", "gs3d_preprocess.hip", "gs3d_blend.hip", "mlp.hip"]
 HIPCC_FLAGS = [

@@ -2,6 +2,7 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include "deform.hpp"
+#include "encode.hpp"
 #include "fast_surfel.hpp"
 #include "gaussian.hpp"
 #include "surfel.hpp"
@@ -87,6 +88,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("deform_mlp", &deform_mlp_py);
   const auto released = py::call_guard<py::gil_scoped_release>();
   m.def("knn_points", &knn_points, released);
+  m.def("sh_encode", &sh_encode, released);
+  m.def("sh_to_rgb", &sh_to_rgb, released);
   m.def("deform_apply", &deform_apply, released);
   m.def("mlp_pack", &mlp_pack, released);
   m.def("image_loss", &image_loss, released);

@@ -13,9 +13,18 @@ import math
 import torch
 from torch import Tensor, nn
 
+from fast_sp_gs_amd import lib as L
+from fast_sp_gs_amd._C import _ops
 from fast_sp_gs_amd.autograd import KernelPair
 
 __all__ = ['sh_encode', 'SH_to_RGB', 'freq_encode', 'FreqEncoder', 'cdist_top']
+
+
+def _native(degree, *tensors) -> bool:
+    """Whether a call may go to the host layer's node: plain tensors (the layer looks at their type, device and shape itself and
+    answers None for what is not its own, which the operator pair then takes or refuses), and nobody times the operators."""
+    return (type(degree) is int and _ops.STAGE_EVENTS is None and all(type(t) in (Tensor, nn.Parameter) for t in tensors)
+            and not torch.compiler.is_compiling())
 
 
 # ---- SH basis of unit directions: [B, D >= 3] -> [B, (degree + 1)^2] ---------------------------------------------------
@@ -39,6 +48,10 @@ _sh_pair = KernelPair('sh_encode_forward', 'sh_encode_backward', _sh_launch, _sh
 
 def sh_encode(dirs: Tensor, degree: int) -> Tensor:
     """Real SH basis up to `degree` of the directions in the last dimension; leading dimensions are kept."""
+    if _native(degree, dirs):
+        basis = L.host.sh_encode(dirs, degree)
+        if basis is not None:
+            return basis
     lead = dirs.shape[:-1]
     return _sh_pair(dirs.reshape(-1, dirs.shape[-1]), degree).reshape(*lead, -1)
 
@@ -67,6 +80,10 @@ _rgb_pair = KernelPair('SH_to_RGB_forward', 'SH_to_RGB_backward', _rgb_launch, _
 def SH_to_RGB(sh: Tensor, dirs: Tensor, campos: Tensor = None, degree: int = 0, clamp: bool = True) -> Tensor:
     """rgb = max(0, sum_k basis_k(dir) sh_k + 0.5) (clamp optional); with `campos`, `dirs` are positions and the
     direction is normalize(position - campos)."""
+    if _native(degree, sh, dirs) and (campos is None or type(campos) in (Tensor, nn.Parameter)):
+        rgb = L.host.sh_to_rgb(sh, dirs, campos, degree, bool(clamp))
+        if rgb is not None:
+            return rgb
     return _rgb_pair(sh, dirs, campos, degree, clamp)
 
 
