@@ -1,6 +1,7 @@
 // The spherical-harmonic operators. Forward and backward of both over 1M points are 137 us of kernels in four launches, for which the
 // Python nodes needed 108 us of host time on the fastest core of a machine and 185 on others: the device waited. Both operators forward
-// and backward, us, Python nodes -> these: 2k points 111 -> 60 and 188 -> 92; 400k 108 -> 61 and 185 -> 92; 1M 136 -> 134 and 189 -> 135.
+// and backward, us, Python nodes -> these: 2k points 111 -> 60 and 188 -> 92; 400k 108 -> 61 and 185 -> 92; 1M 136 -> 134 and 189 -> 135
+(109 with the colours' derivatives kept, 113 us of kernels).
 #include "encode.hpp"
 
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -55,29 +56,35 @@ struct Encode : public torch::autograd::Function<Encode> {
   }
 };
 
-Tensor rgb_forward(const Tensor& sh, const Tensor& dirs, const OptTensor& campos, int64_t degree, bool clamp) {
+// derivs: where it is defined, it gets the colours' derivatives by the direction
+Tensor rgb_forward(const Tensor& sh, const Tensor& dirs, const OptTensor& campos, int64_t degree, bool clamp, const Tensor& derivs) {
   Tensor rgb = empty({dirs.size(0), 3}, dirs);
-  check(fsgs_sh_to_rgb_forward((int) dirs.size(0), (int) sh.size(1), (int) degree, clamp, f32(dirs), f32(opt(campos)), f32(sh), f32(rgb),
-                               stream_of(dirs)),
+  check(fsgs_sh_to_rgb_forward_derivs((int) dirs.size(0), (int) sh.size(1), (int) degree, clamp, f32(dirs), f32(opt(campos)), f32(sh),
+                                      f32(rgb), f32(derivs), stream_of(dirs)),
         "SH_to_RGB_forward");
   return rgb;
 }
 
 struct Rgb : public torch::autograd::Function<Rgb> {
   static Tensor forward(AutogradContext* ctx, const Tensor& sh, const Tensor& dirs, const OptTensor& campos, int64_t degree, bool clamp) {
-    Tensor rgb = rgb_forward(sh, dirs, campos, degree, clamp);
-    ctx->save_for_backward({sh, dirs, opt(campos), rgb});
+    Tensor derivs;  // for a gradient of the direction, where the rows of coefficients allow it
+    if ((dirs.requires_grad() || (has(campos) && campos->requires_grad())) &&
+        fsgs_view_keeps_color_derivs((int) degree, (int) sh.size(1), f32(sh), nullptr))
+      derivs = empty({dirs.size(0), 9}, dirs);
+    Tensor rgb = rgb_forward(sh, dirs, campos, degree, clamp, derivs);
+    ctx->save_for_backward({sh, dirs, opt(campos), rgb, derivs});
     ctx->saved_data["degree"] = degree, ctx->saved_data["clamp"] = clamp;
     return rgb;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto t = ctx->get_saved_variables();
-    const Tensor &sh = t[0], &dirs = t[1], &campos = t[2], &rgb = t[3];
+    const Tensor &sh = t[0], &dirs = t[1], &campos = t[2], &rgb = t[3], &derivs = t[4];
     at::AutoDispatchBelowADInplaceOrView no_graph;
     const char* what = "SH_to_RGB_backward";
     const Tensor g_rgb = contiguous(g[0]);
     require(what, "sh_features", sh, at::kFloat), require(what, "dir_or_pos", dirs, at::kFloat);
     require(what, "rgb", rgb, at::kFloat), require(what, "grad_rgb", g_rgb, at::kFloat);
+    if (derivs.defined()) require(what, "derivs", derivs, at::kFloat);
     const int64_t degree = ctx->saved_data["degree"].toInt();
     // the operator writes whole rows of the directions and the coefficients of its degree, and adds to the camera centre's
     const bool whole = sh.size(1) == (degree + 1) * (degree + 1);
@@ -85,8 +92,9 @@ struct Rgb : public torch::autograd::Function<Rgb> {
     if (ctx->needs_input_grad(0)) g_sh = whole ? at::empty_like(sh) : at::zeros_like(sh);
     if (ctx->needs_input_grad(1)) g_dirs = at::empty_like(dirs);
     if (campos.defined() && ctx->needs_input_grad(2)) g_campos = at::zeros_like(campos);
-    check(fsgs_sh_to_rgb_backward((int) dirs.size(0), (int) sh.size(1), (int) degree, ctx->saved_data["clamp"].toBool(), f32(dirs),
-                                  f32(campos), f32(sh), f32(rgb), f32(g_rgb), f32(g_dirs), f32(g_campos), f32(g_sh), stream_of(dirs)),
+    check(fsgs_sh_to_rgb_backward_derivs((int) dirs.size(0), (int) sh.size(1), (int) degree, ctx->saved_data["clamp"].toBool(),
+                                         f32(dirs), f32(campos), f32(sh), f32(rgb), f32(g_rgb), f32(derivs), f32(g_dirs),
+                                         f32(g_campos), f32(g_sh), stream_of(dirs)),
           what);
     return first_order_only(g, {sh, dirs, campos}, {g_sh, g_dirs, g_campos, Tensor(), Tensor()});
   }
@@ -109,7 +117,7 @@ OptTensor sh_to_rgb(const Tensor& sh, const Tensor& dirs, const OptTensor& campo
       (degree + 1) * (degree + 1) > sh.size(1) || (int64_t) 1 << degree > sh.size(1))
     return std::nullopt;
   if (records(sh) || records(dirs) || (has(campos) && records(*campos))) return Rgb::apply(sh, dirs, campos, degree, clamp);
-  return rgb_forward(sh, dirs, campos, degree, clamp);
+  return rgb_forward(sh, dirs, campos, degree, clamp, Tensor());
 }
 
 }  // namespace fsgs_host

@@ -29,41 +29,54 @@ namespace {
 // A lane that walks its own row touches one 128-byte line per load instruction (920 GB/s measured at 1M points); each
 // wavefront therefore moves its 64 rows as 16-byte pieces, 1 KB of consecutive addresses per instruction, through its own
 // slice of LDS, and every lane then reads its row there (the scheme of the preprocess kernels, sh_stage.hpp). 0: other rows.
-template <int kSh, int kRow>
+// kDerivs: the derivatives of the colours by the direction (36 bytes a point) are left for the backward, which then reads them instead of
+// the coefficients (192). Both kernels are bound by what they move. Forward + backward, us, with the coefficients read again -> with the
+// derivatives: 20k points 4.2 + 6.4 -> 4.7 + 4.9; 150k 7.9 + 10.4 -> 9.4 + 8.8; 400k 16.4 + 33 -> 19.9 + 20.5; 1M 33.2 + 76 ->
+// 41.6 + 44 (252 MB and 276 MB: 6.1 and 6.3 TB/s); 3M 119 + 239 -> 128 + 148.
+// Coefficients that are read once in a pass are worth nothing in the memory-side cache (256 MB), but stay there from pass to pass where they
+// fit beside the rest: by ordinary and by streaming loads 400k (77 MB) 40.4 and 41.0, 700k (134 MB) 61.7 and 62.4, 1M (192 MB) 93.3 and
+// 85.6, 3M 287 and 276.
+constexpr size_t kStreamCoefficients = (size_t) 160 << 20;
+template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) sh_to_rgb_forward_kernel(int P, int F, int degree, int clamp,
     const float* __restrict__ pos, const float* __restrict__ campos, const float* __restrict__ sh,
-    float* __restrict__ rgb) {
+    float* __restrict__ rgb, float* __restrict__ derivs) {
   constexpr bool kRows  = kRow != 0;
   using Rows            = ShWaveRows<kRows ? kRow : 48>;
   constexpr int kStride = Rows::kStride;
+  static_assert(!kDerivs || kRow == 48);
   __shared__ __align__(16) float s_rows[kRows ? 4 * kWave * kStride : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
   float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kStride : 0);
   if (kRows) {
     const unsigned long long live = __ballot(i < P);
     if (live != 0ull) {
-      const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
       Rows regs;
-      regs.fetch(live, wave_base, P, sh);
+      regs.fetch(live, wave_base, P, sh, kDerivs && (size_t) P * kRow * 4 >= kStreamCoefficients);
       regs.to_lds(my_rows, wave_base, P);
       wave_lds_sync();
     }
   }
-  if (i >= P) return;
-  float x = pos[3 * (size_t) i], y = pos[3 * (size_t) i + 1], z = pos[3 * (size_t) i + 2];
-  if (campos) {
-    const float p[3] = {x, y, z};
-    view_dir(p, campos, x, y, z);
+  float j[kColorDerivs] = {};
+  if (i < P) {
+    float x = pos[3 * (size_t) i], y = pos[3 * (size_t) i + 1], z = pos[3 * (size_t) i + 2];
+    if (campos) {
+      const float p[3] = {x, y, z};
+      view_dir(p, campos, x, y, z);
+    }
+    float Y[kSh];
+    sh_eval(degree, x, y, z, Y);
+    const int n    = sh_count(degree);
+    const float* c = kRows ? my_rows + (threadIdx.x & 63) * kStride : sh + (size_t) i * F * 3;
+    float r = c[0] * Y[0], g = c[1] * Y[0], b = c[2] * Y[0];
+    for (int l = 1; l < n; ++l) r += c[3 * l] * Y[l], g += c[3 * l + 1] * Y[l], b += c[3 * l + 2] * Y[l];
+    r += 0.5f, g += 0.5f, b += 0.5f;
+    if (clamp) r = fmaxf(0.0f, r), g = fmaxf(0.0f, g), b = fmaxf(0.0f, b);
+    rgb[3 * (size_t) i] = r, rgb[3 * (size_t) i + 1] = g, rgb[3 * (size_t) i + 2] = b;
+    if constexpr (kDerivs) sh_color_derivatives(degree, x, y, z, [&](int l, int ch) { return c[3 * l + ch]; }, j);
   }
-  float Y[kSh];
-  sh_eval(degree, x, y, z, Y);
-  const int n    = sh_count(degree);
-  const float* c = kRows ? my_rows + (threadIdx.x & 63) * kStride : sh + (size_t) i * F * 3;
-  float r = c[0] * Y[0], g = c[1] * Y[0], b = c[2] * Y[0];
-  for (int l = 1; l < n; ++l) r += c[3 * l] * Y[l], g += c[3 * l + 1] * Y[l], b += c[3 * l + 2] * Y[l];
-  r += 0.5f, g += 0.5f, b += 0.5f;
-  if (clamp) r = fmaxf(0.0f, r), g = fmaxf(0.0f, g), b = fmaxf(0.0f, b);
-  rgb[3 * (size_t) i] = r, rgb[3 * (size_t) i + 1] = g, rgb[3 * (size_t) i + 2] = b;
+  if constexpr (kDerivs) wave_derivs_out(my_rows, j, wave_base, P, derivs);
 }
 
 __device__ __forceinline__ float wave_sum_xor(float v) {
@@ -72,20 +85,24 @@ __device__ __forceinline__ float wave_sum_xor(float v) {
   return v;
 }
 
-template <int kSh, int kRow>
+// kDerivs: nothing is read of the coefficients, and half of a wavefront's gradient rows at a time pass through the LDS; `derivs` are the
+// forward's, or nullptr where no gradient of the direction is asked for.
+template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, int degree, int clamp,
     const float* __restrict__ pos, const float* __restrict__ campos, const float* __restrict__ sh,
-    const float* __restrict__ rgb, const float* __restrict__ grad_rgb, float* __restrict__ grad_dir,
-    float* __restrict__ grad_campos, float* __restrict__ grad_sh) {
+    const float* __restrict__ rgb, const float* __restrict__ grad_rgb, const float* __restrict__ derivs,
+    float* __restrict__ grad_dir, float* __restrict__ grad_campos, float* __restrict__ grad_sh) {
   __shared__ float s_cam[4][3];
   constexpr bool kRows  = kRow != 0;
   using Rows            = ShWaveRows<kRows ? kRow : 48>;
   constexpr int kStride = Rows::kStride;
-  __shared__ __align__(16) float s_rows[kRows ? 4 * kWave * kStride : 1];
+  static_assert(!kDerivs || kRow == 48);
+  constexpr int kWaveRows = kDerivs ? kShHalfRows : kWave;
+  __shared__ __align__(16) float s_rows[kRows ? 4 * kWaveRows * kStride : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
-  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kStride : 0);
-  if (kRows) {  // coefficient rows in through LDS; the gradient rows leave the same way (a lane overwrites its own row)
+  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWaveRows * kStride : 0);
+  if (kRows && !kDerivs) {  // coefficient rows in through LDS; the gradient rows leave the same way (a lane overwrites its own row)
     const unsigned long long live = __ballot(i < P);
     if (live != 0ull) {
       Rows regs;
@@ -94,31 +111,33 @@ __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, i
       wave_lds_sync();
     }
   }
-  float dx = 0, dy = 0, dz = 0;
+  float dx = 0, dy = 0, dz = 0, g[3] = {}, Y[kSh];
+  if constexpr (kDerivs) {
+#pragma unroll
+    for (int l = 0; l < kSh; ++l) Y[l] = 0.0f;
+  }
   if (i < P) {
     const float p[3] = {pos[3 * (size_t) i], pos[3 * (size_t) i + 1], pos[3 * (size_t) i + 2]};
-    float x = p[0], y = p[1], z = p[2], nn = 1.0f;
-    if (campos) nn = view_dir(p, campos, x, y, z);
-    float g[3];
+    float j[kColorDerivs] = {};
+    if constexpr (kDerivs) {
+      if (derivs) {
+#pragma unroll
+        for (int k = 0; k < kColorDerivs; ++k) j[k] = derivs[kColorDerivs * (size_t) i + k];
+      }
+    }
+    float dir[3] = {p[0], p[1], p[2]}, nn = 1.0f;
+    if (campos) nn = view_dir(p, campos, dir[0], dir[1], dir[2]);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       g[c] = grad_rgb[3 * (size_t) i + c];
       if (clamp) g[c] *= (float) (rgb[3 * (size_t) i + c] > 0);
     }
-    float Y[kSh], tl[kSh];
-    sh_eval(degree, x, y, z, Y);
+    sh_eval(degree, dir[0], dir[1], dir[2], Y);
     const int n    = sh_count(degree);
     float* row     = my_rows + (threadIdx.x & 63) * kStride;
     const float* c = kRows ? row : sh + (size_t) i * F * 3;
-    float* o       = kRows ? (grad_sh ? row : nullptr) : (grad_sh ? grad_sh + (size_t) i * F * 3 : nullptr);
-    tl[0] = 0.0f;
-    for (int l = 0; l < n; ++l) {  // a coefficient is read before its slot takes the gradient
-      const float c0 = c[3 * l], c1 = c[3 * l + 1], c2 = c[3 * l + 2];
-      tl[l] = g[0] * c0 + g[1] * c1 + g[2] * c2;
-      if (o) o[3 * l] = g[0] * Y[l], o[3 * l + 1] = g[1] * Y[l], o[3 * l + 2] = g[2] * Y[l];
-    }
     if (grad_dir || grad_campos) {
-      sh_grad_accumulate(degree, x, y, z, tl, dx, dy, dz);
+      sh_direction_part<kSh, kDerivs>(degree, dir, g, c, j, dx, dy, dz);  // before the gradients take the coefficients' place
       if (campos) {
         const float vx = p[0] - campos[0], vy = p[1] - campos[1], vz = p[2] - campos[2];
         const float t  = -(vx * dx + vy * dy + vz * dz) * nn * nn * nn;
@@ -126,8 +145,14 @@ __global__ void __launch_bounds__(256) sh_to_rgb_backward_kernel(int P, int F, i
       }
       if (grad_dir) grad_dir[3 * (size_t) i] = dx, grad_dir[3 * (size_t) i + 1] = dy, grad_dir[3 * (size_t) i + 2] = dz;
     }
+    if (!kDerivs && grad_sh) {
+      float* o = kRows ? row : grad_sh + (size_t) i * F * 3;
+      for (int l = 0; l < n; ++l) o[3 * l] = g[0] * Y[l], o[3 * l + 1] = g[1] * Y[l], o[3 * l + 2] = g[2] * Y[l];
+    }
   }
-  if (kRows && grad_sh) {
+  if constexpr (kDerivs) {
+    if (grad_sh) sh_products_to_global<48>(my_rows, g, Y, wave_base, P, grad_sh);
+  } else if (kRows && grad_sh) {
     wave_lds_sync();
     Rows::to_global(my_rows, wave_base, P, grad_sh);
   }
@@ -816,40 +841,57 @@ FSGS_API int fsgs_adam_masked_update_multi(int n_tensors, int64_t N, const int64
   return check_launch("AdamMasksedUpdated");
 }
 
-FSGS_API int fsgs_sh_to_rgb_forward(int P, int F, int degree, int clamp, const float* pos, const float* campos,
-                                    const float* sh, float* rgb, void* stream) {
+FSGS_API int fsgs_sh_to_rgb_forward_derivs(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+                                           const float* sh, float* rgb, float* derivs, void* stream) {
   FSGS_REQUIRE(P >= 0 && pos && sh && rgb, "SH_to_RGB_forward: bad arguments");
   FSGS_REQUIRE(0 <= degree && degree <= kMaxShDegree && (degree + 1) * (degree + 1) <= F,
                "SH_to_RGB_forward: degree %d unsupported or > features %d", degree, F);
-  if (P == 0) return kOk;
   const int rows = F == (degree + 1) * (degree + 1) && ((uintptr_t) sh & 15) == 0 ? degree : 0;
-  auto kernel = degree > 3  ? sh_to_rgb_forward_kernel<64, 0>
-                : rows == 3 ? sh_to_rgb_forward_kernel<16, 48>
-                : rows == 2 ? sh_to_rgb_forward_kernel<16, 27>
-                : rows == 1 ? sh_to_rgb_forward_kernel<16, 12>
-                            : sh_to_rgb_forward_kernel<16, 0>;
+  FSGS_REQUIRE(!derivs || (rows == 3 && ((uintptr_t) derivs & 15) == 0), "SH_to_RGB_forward: no derivatives of these rows");
+  if (P == 0) return kOk;
+  auto kernel = degree > 3  ? sh_to_rgb_forward_kernel<64, 0, false>
+                : rows == 3 ? (derivs ? sh_to_rgb_forward_kernel<16, 48, true> : sh_to_rgb_forward_kernel<16, 48, false>)
+                : rows == 2 ? sh_to_rgb_forward_kernel<16, 27, false>
+                : rows == 1 ? sh_to_rgb_forward_kernel<16, 12, false>
+                            : sh_to_rgb_forward_kernel<16, 0, false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, F, degree,
-                     clamp, pos, campos, sh, rgb);
+                     clamp, pos, campos, sh, rgb, derivs);
   return check_launch("SH_to_RGB_forward");
 }
 
-FSGS_API int fsgs_sh_to_rgb_backward(int P, int F, int degree, int clamp, const float* pos, const float* campos,
-    const float* sh, const float* rgb, const float* grad_rgb, float* grad_dir, float* grad_campos, float* grad_sh,
-    void* stream) {
+FSGS_API int fsgs_sh_to_rgb_forward(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+                                    const float* sh, float* rgb, void* stream) {
+  return fsgs_sh_to_rgb_forward_derivs(P, F, degree, clamp, pos, campos, sh, rgb, nullptr, stream);
+}
+
+FSGS_API int fsgs_sh_to_rgb_backward_derivs(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+    const float* sh, const float* rgb, const float* grad_rgb, const float* derivs, float* grad_dir, float* grad_campos,
+    float* grad_sh, void* stream) {
   FSGS_REQUIRE(P >= 0 && pos && sh && rgb && grad_rgb, "SH_to_RGB_backward: bad arguments");
   FSGS_REQUIRE(0 <= degree && degree <= kMaxShDegree && (degree + 1) * (degree + 1) <= F,
                "SH_to_RGB_backward: degree %d unsupported or > features %d", degree, F);
   FSGS_REQUIRE(!grad_campos || campos, "SH_to_RGB_backward: grad_campos without campos");
   if (P == 0) return kOk;
-  const int rows = F == (degree + 1) * (degree + 1) && (((uintptr_t) sh | (uintptr_t) grad_sh) & 15) == 0 ? degree : 0;
-  auto kernel = degree > 3  ? sh_to_rgb_backward_kernel<64, 0>
-                : rows == 3 ? sh_to_rgb_backward_kernel<16, 48>
-                : rows == 2 ? sh_to_rgb_backward_kernel<16, 27>
-                : rows == 1 ? sh_to_rgb_backward_kernel<16, 12>
-                            : sh_to_rgb_backward_kernel<16, 0>;
+  const bool full = F == (degree + 1) * (degree + 1);
+  const int rows = full && (((uintptr_t) sh | (uintptr_t) grad_sh) & 15) == 0 ? degree : 0;
+  // The coefficients are read for the direction's gradient alone: not where nobody asks for it, or the forward left its derivatives.
+  const bool unread = degree == 3 && full && ((uintptr_t) grad_sh & 15) == 0 && (derivs || !(grad_dir || grad_campos));
+  auto kernel = degree > 3  ? sh_to_rgb_backward_kernel<64, 0, false>
+                : unread    ? sh_to_rgb_backward_kernel<16, 48, true>
+                : rows == 3 ? sh_to_rgb_backward_kernel<16, 48, false>
+                : rows == 2 ? sh_to_rgb_backward_kernel<16, 27, false>
+                : rows == 1 ? sh_to_rgb_backward_kernel<16, 12, false>
+                            : sh_to_rgb_backward_kernel<16, 0, false>;
   hipLaunchKernelGGL(kernel, dim3(div_up(P, 256)), dim3(256), 0, (hipStream_t) stream, P, F, degree,
-                     clamp, pos, campos, sh, rgb, grad_rgb, grad_dir, grad_campos, grad_sh);
+                     clamp, pos, campos, sh, rgb, grad_rgb, derivs, grad_dir, grad_campos, grad_sh);
   return check_launch("SH_to_RGB_backward");
+}
+
+FSGS_API int fsgs_sh_to_rgb_backward(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+    const float* sh, const float* rgb, const float* grad_rgb, float* grad_dir, float* grad_campos, float* grad_sh,
+    void* stream) {
+  return fsgs_sh_to_rgb_backward_derivs(P, F, degree, clamp, pos, campos, sh, rgb, grad_rgb, nullptr, grad_dir, grad_campos, grad_sh,
+                                        stream);
 }
 
 // ---- encoders and nearest / farthest search: one typed entry each plus the single-precision shorthand -----------------

@@ -93,8 +93,8 @@ __device__ __forceinline__ void unstage_sh_grads(const float* __restrict__ s_row
 // kernel. Preprocess forward and backward, us: 3M 1352x1014 238 + 369 -> 216 + 330; 1M 1352x900 96 + 131 -> 85 + 119; 300k 800x800
 // 34 + 51 -> 34 + 45. Stores by ordinary and by streaming ones, preprocess backward of small scenes: 10k 10.9 and 11.0, 50k 14.6 and
 // 14.2, 100k 19.3 and 18.1, 200k 39.3 and 37.2; colours' backward 10k 6.4 and 6.3, 50k 7.9 and 7.0, 200k 19.0 and 18.0: no size at which
-// ordinary ones are better. The SH operators' backward reads the coefficients that their forward has read: there the loads are ordinary
-// ones, 1M rows of coefficients 53 + 82 -> 33 + 76 us (with streaming loads
+// ordinary ones are better. The SH operators' backward, where it reads the coefficients that their forward has read, uses ordinary
+// loads, 1M rows of coefficients 53 + 82 -> 33 + 76 us (with streaming loads
 // 36 + 77). Smaller tables stay in the cache from pass to pass: view of 98k surfels 170x120, preprocess 14 us and 16 with streaming
 // loads; 200k 22.3 and 23.5; 300k (58 MB) 36.4 and 35.2; 400k 58 and 52.
 using ShPiece = float __attribute__((ext_vector_type(4)));

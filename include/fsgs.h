@@ -449,6 +449,16 @@ int fsgs_sh_to_rgb_backward(int P, int F, int degree, int clamp, const float* po
     const float* sh, const float* rgb, const float* grad_rgb, float* grad_dir, float* grad_campos, float* grad_sh,
     void* stream);
 
+/* _derivs: the forward leaves the colours' derivatives by the direction, too (derivs[P,9], channel-major, on a 16-byte boundary;
+ * nullptr: none), and the backward reads them instead of the coefficients (nullptr: the coefficients). The forward does so only for
+ * rows of coefficients that fsgs_view_keeps_color_derivs(degree, F, sh, nullptr) accepts; the backward reads the coefficients all the
+ * same where grad_sh is not on a 16-byte boundary. */
+int fsgs_sh_to_rgb_forward_derivs(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+    const float* sh, float* rgb, float* derivs, void* stream);
+int fsgs_sh_to_rgb_backward_derivs(int P, int F, int degree, int clamp, const float* pos, const float* campos,
+    const float* sh, const float* rgb, const float* grad_rgb, const float* derivs, float* grad_dir, float* grad_campos,
+    float* grad_sh, void* stream);
+
 /* Element types of the `_typed` entry points below. The reference dispatches these small operators on the tensor's
  * scalar type (AT_DISPATCH_FLOATING_TYPES[_AND_HALF]); a `_typed` entry takes the same buffers as untyped addresses plus
  * this selector. FSGS_DTYPE_F16 is IEEE binary16 storage with single-precision arithmetic. */

@@ -55,3 +55,30 @@ def test_kept_or_formed_again(kind, split, P, device):
             assert (a - b).abs().max() <= 1e-5 * b.abs().max() + 1e-30
         else:
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('P', [1, 31, 33, 64, 255, 257, 1500])
+@pytest.mark.parametrize('camera', [False, True])
+def test_sh_to_rgb_kept_or_formed_again(P, camera, device):
+    """The operator pair on its own: every choice of gradients, from the forward's derivatives (and, without a gradient of the direction,
+    from nothing of the coefficients) against gradients from the coefficients, which rows off a 16-byte boundary are given."""
+    from fast_sp_gs_amd.ops import SH_to_RGB
+    print(f'[colour derivatives] SH_to_RGB P={P} camera={camera}', flush=True)
+    g = torch.Generator().manual_seed(P)
+    normal = lambda *s: torch.randn(*s, generator=g).to(device)
+    sh, pos, cam, up = normal(P, 16, 3) * 0.4, normal(P, 3), normal(3) * 3.0, normal(P, 3)
+    if not camera:
+        pos = torch.nn.functional.normalize(pos, dim=-1)
+    for wants in range(1, 8 if camera else 4):
+        def run(move):
+            p = [move(sh), pos.clone(), cam.clone() if camera else None]
+            wrt = [t.requires_grad_(True) for k, t in enumerate(p) if t is not None and wants >> k & 1]
+            rgb = SH_to_RGB(*p, 3, True)
+            return [rgb, *torch.autograd.grad(rgb, wrt, up)]
+        for k, (a, b) in enumerate(zip(run(torch.clone), run(_move))):
+            if a.shape == (3,):  # the camera's: sums over blocks of 256 points, one atomic each, in any order
+                assert (a - b).abs().max() <= 1e-6 * P ** 0.5 * max(float(b.abs().max()), 1.0)
+            elif k == 0:  # the colours: contraction may differ between the two kernels, 16 terms of at most a few units
+                assert (a - b).abs().max() <= 16 * 2 ** -23
+            else:
+                assert torch.equal(a, b), (wants, k)
