@@ -1,7 +1,7 @@
 // The spherical-harmonic operators. Forward and backward of both over 1M points are 137 us of kernels in four launches, for which the
 // Python nodes needed 108 us of host time on the fastest core of a machine and 185 on others: the device waited. Both operators forward
 // and backward, us, Python nodes -> these: 2k points 111 -> 60 and 188 -> 92; 400k 108 -> 61 and 185 -> 92; 1M 136 -> 134 and 189 -> 135
-(109 with the colours' derivatives kept, 113 us of kernels).
+// (109 with the colours' derivatives kept, 113 us of kernels).
 #include "encode.hpp"
 
 #include <c10/core/impl/LocalDispatchKeySet.h>
