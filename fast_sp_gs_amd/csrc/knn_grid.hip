@@ -18,8 +18,8 @@
 //      (A key of the distance's upper 25 bits and the list position costs three instructions less per candidate, but the
 //      numbers have to be fetched from the list again, eight scattered loads a query: 272 us of queries at 3M x 2048, K = 8.)
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
-// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.154 ms a call this way
-// (traced: lists 0.046, queries 0.118 to 0.129; 0.063 ms for the 324 MB of inputs and outputs alone). In the query kernel neither unit is
+// short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.145 ms a call this way
+// (traced: lists 0.039, queries 0.118 to 0.129; 0.063 ms for the 324 MB of inputs and outputs alone). In the query kernel neither unit is
 // full: the vector units are busy 0.62 of the time (1090 instructions per 64 queries), LDS 0.52, 0.22 in bank conflicts. With lists in
 // index order and a row of results stored by each lane for itself it took 0.202 ms and 2180 instructions; in order alone 0.169, its
 // memory path busy with stores of 16 bytes each; results through LDS in runs of 512 and 1024 bytes 0.152, and past the caches, which then
@@ -65,7 +65,7 @@ enum Scheme { kAllPairs, kAlone, kGrid16, kGrid32 };
 
 // Which search. Measured: an all-pairs walk takes 65 ns per control point however few queries there are (a lane walks
 // alone) and N * M / 4e12 s when they fill the chip; a wavefront per query 0.8 (M = 512) to 2.0 ns (M = 2048) a query;
-// building the lists 11 us (G = 16, 512 control points) to 37 us (G = 32, 2048), in order 12 and 46. With G = 16 the lists of more than 640
+// building the lists 9 us (G = 16, 512 control points, in order or not) to 35 us (G = 32, 2048), in order 39. With G = 16 the lists of more than 640
 // control points outgrow their 128 entries; below that the finer grid pays from a million queries on. Behind the limits
 // the walk over all pairs takes over at its own price: 3M normal queries, K = 4: 133 us for 2560 control points, 1550 for 2561; 2048
 // control points, K = 8: 156 us, K = 9: 5940. 200 000 queries, K = 4: 60 and 187 us.
@@ -77,7 +77,7 @@ Scheme knn_scheme(int N, int M, int D, int K) {
 }
 
 // Whether the lists are put in the order of the distances from their cell's centre, so that a query's walk is over after half of its
-// list (below). With G = 32 that costs 4 to 8 us whatever the number of queries, with G = 16 1 us; what it saves grows with the queries,
+// list (below). With G = 32 that costs 4 us (8 when the limits below were measured) whatever the number of queries, with G = 16 1 us; what it saves grows with the queries,
 // with K and with the length of the lists, that is, with M. Past about 150 MB of results the stores past the caches, which come with
 // the order (kStream), outweigh that. us a call in index order -> in this one, queries in a ball | normal (what two runs differ by: 1 to 3):
 //   G = 32, K = 8, M = 2048:  500 000 59 -> 59 | 79 -> 82;  1M 81 -> 76 | 104 -> 100;  3M 183 -> 131 | 204 -> 154
@@ -199,12 +199,109 @@ __device__ __forceinline__ float from_ordered_bits(uint32_t b) {
   return __uint_as_float((b & 0x80000000u) ? b & 0x7fffffffu : ~b);
 }
 
+__device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, kCtrl, 0xf, 0xf, true);
+}
+constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kXor3 = 0x1b, kXor7 = 0x141, kXor8 = 0x128, kXor15 = 0x140;  // quad_perm, mirrors, row_ror:8
+// The lane's value and that of lane l ^ 16 (l ^ 32), one in a and one in b: after the swap, of the 16-lane (32-lane) rows, a holds the
+// even ones and b the odd ones (s_nop: the wait states that the compiler does not count in here).
+__device__ __forceinline__ void pair16(uint32_t v, uint32_t& a, uint32_t& b) {
+  a = v, b = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void pair32(uint32_t v, uint32_t& a, uint32_t& b) {
+  a = v, b = v;
+  asm("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+// Bitonic network over the 64 lanes' values. A step keeps the smaller or the larger of a lane's value and its partner's: the median of
+// the two and 0 or 2^32 - 1, one instruction behind the partner's value (a minimum, a maximum and a choice between them are three, and
+// a mirror image across rows costs a choice more: the merges of rows run over rows of opposite directions instead).
+struct WaveSort {
+  uint32_t m1, m2, m4, m8, m16, m32;  // all ones in the lanes that have that bit
+  __device__ __forceinline__ WaveSort() {
+    const int lane = __lane_id();
+    auto mask = [&](int bit) { return lane & bit ? ~0u : 0u; };
+    m1 = mask(1), m2 = mask(2), m4 = mask(4), m8 = mask(8), m16 = mask(16), m32 = mask(32);
+  }
+  static __device__ __forceinline__ uint32_t xor4(uint32_t x) { return dpp_u32<kXor3>(dpp_u32<kXor7>(x)); }
+  static __device__ __forceinline__ void keep(uint32_t& v, uint32_t other, uint32_t upper) { v = med3_u32(v, other, upper); }
+  static __device__ __forceinline__ void keep16(uint32_t& v, uint32_t upper) {
+    uint32_t a, b;
+    pair16(v, a, b);
+    v = med3_u32(a, b, upper);
+  }
+  static __device__ __forceinline__ void keep32(uint32_t& v, uint32_t upper) {
+    uint32_t a, b;
+    pair32(v, a, b);
+    v = med3_u32(a, b, upper);
+  }
+  // `down`: all ones in the rows that are to descend
+  __device__ __forceinline__ void below4(uint32_t& v, uint32_t down) const { keep(v, dpp_u32<kXor2>(v), m2 ^ down), keep(v, dpp_u32<kXor1>(v), m1 ^ down); }
+  __device__ __forceinline__ void below16(uint32_t& v, uint32_t down) const {
+    keep(v, dpp_u32<kXor8>(v), m8 ^ down), keep(v, xor4(v), m4 ^ down), below4(v, down);
+  }
+  __device__ __forceinline__ void below64(uint32_t& v) const { keep32(v, m32), keep16(v, m16), below16(v, 0u); }
+  __device__ __forceinline__ void ascending(uint32_t& v) const {
+    keep(v, dpp_u32<kXor1>(v), m1 ^ m16);
+    keep(v, dpp_u32<kXor3>(v), m2 ^ m16), keep(v, dpp_u32<kXor1>(v), m1 ^ m16);
+    keep(v, dpp_u32<kXor7>(v), m4 ^ m16), below4(v, m16);
+    keep(v, dpp_u32<kXor15>(v), m8 ^ m16), keep(v, xor4(v), m4 ^ m16), below4(v, m16);
+    keep16(v, m16 ^ m32), below16(v, m32);
+    below64(v);
+  }
+  // of 128 values, the lower ones to v
+  __device__ __forceinline__ void ascending(uint32_t& v, uint32_t& w) const {
+    w = ~w;
+    ascending(v), ascending(w);
+    const uint32_t down = ~w;  // descending
+    w = max(v, down), v = min(v, down);
+    below64(v), below64(w);
+  }
+};
+
+// Of the 64 lanes: all get the least (largest); a lane gets the sum (the largest) of its own and the lanes' below it.
+template <bool kMost>
+__device__ __forceinline__ float wave_extreme(float v) {
+  auto of = [](float a, float b) { return kMost ? fmaxf(a, b) : fminf(a, b); };
+  auto partner = [&](auto ctrl) { return __uint_as_float(dpp_u32<decltype(ctrl)::value>(__float_as_uint(v))); };
+  v = of(v, partner(std::integral_constant<int, kXor1>())), v = of(v, partner(std::integral_constant<int, kXor2>()));
+  v = of(v, partner(std::integral_constant<int, kXor7>())), v = of(v, partner(std::integral_constant<int, kXor15>()));
+  uint32_t a, b;
+  pair16(__float_as_uint(v), a, b);
+  pair32(__float_as_uint(of(__uint_as_float(a), __uint_as_float(b))), a, b);
+  return of(__uint_as_float(a), __uint_as_float(b));
+}
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ float dpp_or(float v, float otherwise) {  // `otherwise` where no lane of the row (no such row) is read
+  return __uint_as_float((uint32_t) __builtin_amdgcn_update_dpp((int) __float_as_uint(otherwise), (int) __float_as_uint(v), kCtrl, kRows, 0xf, false));
+}
+constexpr int kShiftRow = 0x110, kShiftWave = 0x138, kLastOfRow = 0x142, kLastOfHalf = 0x143;  // row_shr, wave_shr:1, row_bcast:15 and :31
+__device__ __forceinline__ float wave_running_sum(float v) {
+  v += dpp_or<kShiftRow + 1>(v, 0.0f), v += dpp_or<kShiftRow + 2>(v, 0.0f), v += dpp_or<kShiftRow + 4>(v, 0.0f);
+  v += dpp_or<kShiftRow + 8>(v, 0.0f), v += dpp_or<kLastOfRow, 0xa>(v, 0.0f), v += dpp_or<kLastOfHalf, 0xc>(v, 0.0f);
+  return v;
+}
+__device__ __forceinline__ float wave_running_max(float v) {
+  v = fmaxf(v, dpp_or<kShiftRow + 1>(v, v)), v = fmaxf(v, dpp_or<kShiftRow + 2>(v, v)), v = fmaxf(v, dpp_or<kShiftRow + 4>(v, v));
+  v = fmaxf(v, dpp_or<kShiftRow + 8>(v, v)), v = fmaxf(v, dpp_or<kLastOfRow, 0xa>(v, v)), v = fmaxf(v, dpp_or<kLastOfHalf, 0xc>(v, v));
+  return v;
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __uint_as_float((uint32_t) __builtin_amdgcn_readlane((int) __float_as_uint(v), lane));
+}
+
 constexpr float kRim = 0.5f;  // parts of the sample's extent
 
 template <int kG>
 struct PlaneLds {
   static constexpr int kSamples = 128;
-  uint32_t key[3][kSamples];
   float sorted[3][kSamples], along[3][kSamples];
   float plane[3][kG + 1];
   float least[kG > 16 ? 3 : 1][8], most[kG > 16 ? 3 : 1][8];  // of the control points near the sample, per wavefront
@@ -222,39 +319,41 @@ struct PlaneLds {
 // such lists, for every query at the rim. 3M x 2048, K = 8, us, with planes beyond all control points and nothing moved in -> so:
 // no outlier 219 -> 219, one at 10 (1000) times the deviation 295 -> 219 (534 -> 220), in the sample 2775 -> 224; normal points
 // times exp(normal) 1786 -> 930; points nine tenths of which lie in a plane 324 -> 315.
-// Every block computes the planes for itself (3 us) instead of waiting for another launch.
+// Every block computes the planes for itself instead of waiting for another launch: 4.4 us of the list kernel at G = 32, 1.9 at G = 16. A
+// wavefront per axis sorts the samples in its registers and sums over its lanes; ranks counted over LDS by all threads, sums by shuffles
+// and a barrier behind each step took 6.6 and 4.2.
 template <int kG>
 __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<kG>& s) {
   constexpr int S = PlaneLds<kG>::kSamples, kSpare = kG > 16 ? 2 : 0;
-  const int t = threadIdx.x;
-  for (int e = t; e < 3 * S; e += kBuildThreads) {
-    const int a = e / S, j = e - a * S;
-    const float4 p = s_y[(int) ((int64_t) j * M / S)];
-    s.key[a][j] = (ordered_bits(a == 0 ? p.x : a == 1 ? p.y : p.z) & ~(uint32_t) (S - 1)) | (uint32_t) j;
-  }
-  __syncthreads();
-  for (int e = t; e < 3 * S; e += kBuildThreads) {
-    const int a = e / S, j = e - a * S;
-    const uint32_t mine = s.key[a][j];
-    int rank = 0;
-#pragma unroll 4
-    for (int i = 0; i < S; i += 4) {
-      const uint4 k = *(const uint4*) &s.key[a][i];
-      rank += (k.x < mine) + (k.y < mine) + (k.z < mine) + (k.w < mine);
+  static_assert(S == 2 * kWave);
+  const int t = threadIdx.x, a = t >> 6, lane = t & 63;  // a wavefront per axis, two samples to a lane
+  float along = 0.0f;
+  if (a < 3) {
+    const WaveSort sort;
+    uint32_t key[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = h * kWave + lane;
+      const float4 p = s_y[(int) ((int64_t) j * M / S)];
+      key[h] = (ordered_bits(a == 0 ? p.x : a == 1 ? p.y : p.z) & ~(uint32_t) (S - 1)) | (uint32_t) j;
     }
-    s.along[a][rank] = from_ordered_bits(mine & ~(uint32_t) (S - 1));
-  }
-  __syncthreads();
-  for (int e = t; e < 3 * S; e += kBuildThreads) {
-    const int a = e / S, j = e - a * S;
-    const float* all  = s.along[a];
-    const float inner = all[S - 9] - all[8], outer = all[S - 2] - all[1];
+    sort.ascending(key[0], key[1]);
+    float v = from_ordered_bits(key[0] & ~(uint32_t) (S - 1)), w = from_ordered_bits(key[1] & ~(uint32_t) (S - 1));
+    const float low8 = lane_value(v, 8), low1 = lane_value(v, 1), high8 = lane_value(w, kWave - 9), high1 = lane_value(w, kWave - 2);
+    const float inner = high8 - low8, outer = high1 - low1;
     const bool even   = inner > 0.125f * outer;
     const float rim   = even ? kRim * inner : outer > 0.0f ? outer : __builtin_inff();
-    s.sorted[a][j]    = fminf(fmaxf(all[j], all[even ? 8 : 1] - rim), all[even ? S - 9 : S - 2] + rim);
+    const float least = (even ? low8 : low1) - rim, most = (even ? high8 : high1) + rim;
+    v = fminf(fmaxf(v, least), most), w = fminf(fmaxf(w, least), most);
+    s.sorted[a][lane] = v, s.sorted[a][kWave + lane] = w;
+    const float sum  = wave_running_sum(sqrtf(fmaxf(v - dpp_or<kShiftWave>(v, v), 0.0f)));
+    const float half = lane_value(sum, kWave - 1);
+    const float rest = half + wave_running_sum(sqrtf(fmaxf(w - dpp_or<kShiftWave>(w, lane_value(v, kWave - 1)), 0.0f)));
+    s.along[a][lane] = sum, s.along[a][kWave + lane] = rest;
+    along = lane_value(rest, kWave - 1);
   }
-  __syncthreads();
   if constexpr (kSpare > 0) {
+    __syncthreads();
     float lo[3], hi[3], least[3], most[3];  // the sample's extent and kRim of it on either side
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -271,32 +370,13 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1)
-        least[c] = fminf(least[c], __shfl_xor(least[c], d, kWave)), most[c] = fmaxf(most[c], __shfl_xor(most[c], d, kWave));
-      if ((t & 63) == 0) s.least[c][t >> 6] = least[c], s.most[c][t >> 6] = most[c];
+      least[c] = wave_extreme<false>(least[c]), most[c] = wave_extreme<true>(most[c]);
+      if (lane == 0) s.least[c][a] = least[c], s.most[c][a] = most[c];
     }
+    __syncthreads();
+  } else if (a < 3) {
+    wave_lds_sync();
   }
-  const int a = t >> 6, lane = t & 63;  // a wavefront per axis
-  if (a < 3) {
-    constexpr int kPer = S / 64;
-    float part[kPer], sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int j = lane * kPer + i;
-      sum += j > 0 ? sqrtf(fmaxf(s.sorted[a][j] - s.sorted[a][j - 1], 0.0f)) : 0.0f;
-      part[i] = sum;
-    }
-    float inc = sum;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float up = __shfl_up(inc, d, kWave);
-      if (lane >= d) inc += up;
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) s.along[a][lane * kPer + i] = (inc - sum) + part[i];
-  }
-  __syncthreads();
   if (a < 3) {
     const float lo = s.sorted[a][0], hi = s.sorted[a][S - 1], ext = hi - lo;
     float first = lo - 0.1f * ext, last = hi + 0.1f * ext;
@@ -314,7 +394,7 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
       else if (i < 1 + kSpare) v = lo + (i == 1 ? 0.55f : 0.25f) * (first - lo);
       else if (i > kG - 1 - kSpare) v = hi + (i == kG - 1 ? 0.55f : 0.25f) * (last - hi);
       else {
-        const float target = s.along[a][S - 1] * ((float) (i - 1 - kSpare) / (float) (kG - 2 - 2 * kSpare));
+        const float target = along * ((float) (i - 1 - kSpare) / (float) (kG - 2 - 2 * kSpare));
         int j = 0;  // last sample whose accumulated step does not exceed the target
 #pragma unroll
         for (int step = S / 2; step >= 1; step >>= 1)
@@ -324,96 +404,23 @@ __device__ __forceinline__ void make_planes(const float4* s_y, int M, PlaneLds<k
         v = s.sorted[a][j] + (s.sorted[a][n] - s.sorted[a][j]) * (w > 0.0f ? (target - s.along[a][j]) / w : 0.0f);
       }
     }
-    // ascending whatever the roundings did
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float up = __shfl_up(v, d, kWave);
-      if (lane >= d) v = fmaxf(v, up);
-    }
+    v = wave_running_max(v);  // ascending whatever the roundings did
     if (lane <= kG) s.plane[a][lane] = v;
   }
   __syncthreads();
 }
-
-// The members of `sub` within `limit` of a box, appended to `out` in index order by one wavefront; stops
-// once there are more than `cap`. Returns how many there are, or a number above cap.
-__device__ __forceinline__ int collect_near(const float4* s_y, const uint16_t* sub, int n_sub, const float* lo,
-                                            const float* hi, float limit, int cap, uint16_t* out) {
-  const int lane = threadIdx.x & 63;
-  int n = 0;
-  for (int i0 = 0; i0 < n_sub && n <= cap; i0 += kAhead * kWave) {  // the LDS reads of kAhead steps are in flight together
-    int i[kAhead];
-    bool in[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) i[u] = sub[min(i0 + u * kWave + lane, n_sub - 1)];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u)
-      in[u] = (int) (box_near2(s_y[i[u]], lo, hi) <= limit) & (int) (i0 + u * kWave + lane < n_sub);
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const unsigned long long m = wave_ballot(in[u]);
-      const int pos = n + lanes_below(m);
-      if (in[u] && pos < cap) out[pos] = (uint16_t) i[u];
-      n += (int) __popcll(m);
-    }
-  }
-  return n;
-}
-
-template <int kCtrl>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
-  return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, kCtrl, 0xf, 0xf, true);
-}
-// The lane's value across the 16-lane (32-lane) rows beside each other: lane l ^ 16 (l ^ 32).
-__device__ __forceinline__ uint32_t across16(uint32_t v, bool odd) {
-  uint32_t a = v, b = v;  // after the swap: rows 0 0 2 2, and 1 1 3 3 (s_nop: the wait states that the compiler does not count in here)
-  asm("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-  return odd ? a : b;
-}
-__device__ __forceinline__ uint32_t across32(uint32_t v, bool odd) {
-  uint32_t a = v, b = v;
-  asm("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-  return odd ? a : b;
-}
-// Bitonic networks over the 64 lanes' values, every merge begun with the mirror image so that all of it ascends.
-struct WaveSort {
-  bool b1, b2, b4, b8, b16, b32;
-  __device__ __forceinline__ WaveSort() {
-    const int lane = __lane_id();
-    b1 = lane & 1, b2 = lane & 2, b4 = lane & 4, b8 = lane & 8, b16 = lane & 16, b32 = lane & 32;
-  }
-  static constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kXor3 = 0x1b, kXor7 = 0x141, kXor8 = 0x128, kXor15 = 0x140;  // quad_perm, mirrors, row_ror:8
-  static __device__ __forceinline__ uint32_t xor4(uint32_t x) { return dpp_u32<kXor3>(dpp_u32<kXor7>(x)); }
-  static __device__ __forceinline__ void keep(uint32_t& v, uint32_t other, bool upper) {
-    const uint32_t lo = min(v, other), hi = max(v, other);
-    v = upper ? hi : lo;
-  }
-  __device__ __forceinline__ uint32_t mirrored(uint32_t v) const { return dpp_u32<kXor15>(across16(across32(v, b32), b16)); }
-  __device__ __forceinline__ void below4(uint32_t& v) const { keep(v, dpp_u32<kXor2>(v), b2), keep(v, dpp_u32<kXor1>(v), b1); }
-  __device__ __forceinline__ void below16(uint32_t& v) const { keep(v, dpp_u32<kXor8>(v), b8), keep(v, xor4(v), b4), below4(v); }
-  __device__ __forceinline__ void below64(uint32_t& v) const { keep(v, across32(v, b32), b32), keep(v, across16(v, b16), b16), below16(v); }
-  __device__ __forceinline__ void ascending(uint32_t& v) const {
-    keep(v, dpp_u32<kXor1>(v), b1);
-    keep(v, dpp_u32<kXor3>(v), b2), keep(v, dpp_u32<kXor1>(v), b1);
-    keep(v, dpp_u32<kXor7>(v), b4), below4(v);
-    keep(v, dpp_u32<kXor15>(v), b8), keep(v, xor4(v), b4), below4(v);
-    keep(v, dpp_u32<kXor15>(across16(v, b16)), b16), below16(v);
-    keep(v, mirrored(v), b32), keep(v, across16(v, b16), b16), below16(v);
-  }
-  // of 128 values, the lower ones to v
-  __device__ __forceinline__ void ascending(uint32_t& v, uint32_t& w) const {
-    ascending(v), ascending(w);
-    const uint32_t m = mirrored(w);
-    w = max(v, m), v = min(v, m);
-    below64(v), below64(w);
-  }
-};
 
 // One block per coarse cell, one wavefront per octant of it: with G = 16 an octant is a cell, with G = 32 it is narrowed
 // down once more for its eight cells. 26 M vector instructions (98 us) when the cells were taken from the coarse list
 // directly: the coarse lists at the rim of the cloud hold nearly everything. A wavefront forms the lists of its cells side by
 // side: a candidate is read once for all of them, its distances to their faces are formed once per axis and half of the octant,
 // and nothing waits in a chain of eight (cells one after the other: 25 us of the kernel's 51).
+// With G = 32 the octants' lists come from the coarse one the same way: a wavefront looks at an eighth of it for all octants instead of
+// at all of it for its own. Bound by the instructions of four wavefronts per SIMD; a median wavefront and the last one (rim of the
+// cloud, 1300 candidates of 2048 in the coarse list) of 2048 control points, K = 8, in order, us: control points 1.5, planes 4.4 (5.4),
+// coarse list 2.3 (3.4), octants 4.5 (7.8), reach of the cells 2.4 (4.0), lists 2.2 (4.3), order 6.3 (7.5). The kernel, by the steps of
+// the sort from three instructions to one, of the planes and of the octants: 46 -> 43 -> 41 -> 39 us, not in order 39.3 -> 37.1 -> 35.1,
+// G = 16 with 512 control points 11.9 -> 9.3.
 template <int kG, bool kOrder>
 __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, int K, const float* __restrict__ y,
     float* __restrict__ planes, Cell<kOrder>* __restrict__ cells, uint16_t* __restrict__ lists) {
@@ -425,7 +432,10 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
   __shared__ PlaneLds<kG> s;
   __shared__ float s_bound[kWaves];
   __shared__ int s_count[kWaves];
+  __shared__ uint32_t s_far[kG > 16 ? kWaves : 1][kWave];  // an octant's squared distances to control points' farthest corners, the least of each lane
+  __shared__ int s_share[kG > 16 ? kWaves : 1][kWaves];    // what a wavefront has found for each octant
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (kG > 16) s_far[wave][lane] = 0x7f800000u;
   for (int i = t; i < M; i += kBuildThreads) s_y[i] = control_point(y, i);
   __syncthreads();
   make_planes<kG>(s_y, M, s);
@@ -447,11 +457,19 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) limit = fminf(limit, s_bound[w]);
   limit = widened(limit);
+  constexpr int kSteps = kMaxPoints / (kWaves * kWave);  // of 64 control points, a wavefront
+  static_assert(kMaxPoints % (kWaves * kWave) == 0);
   const int per = ((M + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;  // a contiguous share per wavefront: index order
   const int first = wave * per, last = min(M, first + per);
+  unsigned long long near[kSteps];
   int n_mine = 0;
-  for (int i0 = first; i0 < last; i0 += kWave)
-    n_mine += __popcll(wave_ballot(i0 + lane < last && box_near2(s_y[min(i0 + lane, M - 1)], lo, hi) <= limit));
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u) {
+    const int i = first + u * kWave + lane;
+    near[u] = 0ull;
+    if (first + u * kWave < last) near[u] = wave_ballot(i < last) & wave_ballot(box_near2(s_y[min(i, M - 1)], lo, hi) <= limit);
+    n_mine += __popcll(near[u]);
+  }
   if (lane == 0) s_count[wave] = n_mine;
   __syncthreads();
   int at = 0, n_sub = 0;
@@ -460,11 +478,10 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
     if (w < wave) at += s_count[w];
     n_sub += s_count[w];
   }
-  for (int i0 = first; i0 < last; i0 += kWave) {
-    const bool in = i0 + lane < last && box_near2(s_y[min(i0 + lane, M - 1)], lo, hi) <= limit;
-    const unsigned long long m = wave_ballot(in);
-    if (in) s_sub[at + lanes_below(m)] = (uint16_t) (i0 + lane);
-    at += __popcll(m);
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u) {
+    if (near[u] >> lane & 1ull) s_sub[at + lanes_below(near[u])] = (uint16_t) (first + u * kWave + lane);
+    at += __popcll(near[u]);
   }
   __syncthreads();
 
@@ -474,23 +491,101 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
   const uint16_t* from = s_sub;
   int n_from = n_sub;
   if constexpr (kG > 16) {
+    // The octants' lists, from the coarse one: a wavefront looks at its share of that for all eight octants side by side (as for the
+    // cells below), not at all of it for its own.
+    constexpr int kHalves = 2;
+    float face[3][kHalves + 1];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) lo[a] = s.plane[a][corner[a]], hi[a] = s.plane[a][corner[a] + kIn];
-    float nearest = __builtin_inff();
-    for (int i0 = lane; i0 < n_sub; i0 += kAhead * kWave) {
+    for (int a = 0; a < 3; ++a)
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        const int i    = i0 + u * kWave;
-        const float d2 = box_far2(s_y[s_sub[min(i, n_sub - 1)]], lo, hi);
-        nearest        = fminf(nearest, i < n_sub ? d2 : __builtin_inff());
+      for (int h = 0; h <= kHalves; ++h) face[a][h] = s.plane[a][cc[a] * kSub + h * kIn];
+    const int share = ((n_sub + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave, begin = wave * share, end = min(n_sub, begin + share);
+    float least_far[kWaves];
+#pragma unroll
+    for (int c = 0; c < kWaves; ++c) least_far[c] = __builtin_inff();
+    for (int i0 = begin; i0 < end; i0 += kWave) {
+      const float4 p    = s_y[s_sub[min(i0 + lane, end - 1)]];
+      const float at[3] = {p.x, p.y, p.z};
+      float f[3][kHalves];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int h = 0; h < kHalves; ++h) {
+          const float d = fmaxf(fabsf(at[a] - face[a][h]), fabsf(at[a] - face[a][h + 1]));
+          f[a][h] = i0 + lane < end ? d * d : __builtin_inff();
+        }
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c) least_far[c] = fminf(least_far[c], (f[0][c & 1] + f[1][c >> 1 & 1]) + f[2][c >> 2]);
+    }
+    if (begin < end) {
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c) atomicMin(&s_far[c][lane], __float_as_uint(least_far[c]));
+    }
+    __syncthreads();
+    const float mine = widened(wave_kth_bound(__uint_as_float(s_far[wave][lane]), K));
+    if (lane == 0) s_bound[wave] = mine;
+    __syncthreads();
+    float within[kWaves];
+#pragma unroll
+    for (int c = 0; c < kWaves; ++c) within[c] = s_bound[c];
+    uint32_t in[kSteps];  // bit c: within reach of octant c
+    int count[kWaves];
+#pragma unroll
+    for (int c = 0; c < kWaves; ++c) count[c] = 0;
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      const int i0 = begin + u * kWave;
+      in[u] = 0u;
+      if (i0 >= end) continue;
+      const float4 p    = s_y[s_sub[min(i0 + lane, end - 1)]];
+      const float at[3] = {p.x, p.y, p.z};
+      float f[3][kHalves];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int h = 0; h < kHalves; ++h) {
+          const float d = fmaxf(fmaxf(face[a][h] - at[a], at[a] - face[a][h + 1]), 0.0f);
+          f[a][h] = d * d;
+        }
+      const unsigned long long there = wave_ballot(i0 + lane < end);
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c) {
+        const bool near = (f[0][c & 1] + f[1][c >> 1 & 1]) + f[2][c >> 2] <= within[c];
+        in[u] |= near ? 1u << c : 0u;
+        count[c] += (int) __popcll(there & wave_ballot(near));
+      }
+      if (i0 + lane >= end) in[u] = 0u;
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c) s_share[wave][c] = count[c];
+    }
+    __syncthreads();
+    int place[kWaves];
+#pragma unroll
+    for (int c = 0; c < kWaves; ++c) place[c] = 0;
+    n_from = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c)
+        if (w < wave) place[c] += s_share[w][c];
+      n_from += s_share[w][wave];
+    }
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      if (begin + u * kWave >= end) continue;
+      const uint16_t number = s_sub[min(begin + u * kWave + lane, end - 1)];
+#pragma unroll
+      for (int c = 0; c < kWaves; ++c) {
+        const unsigned long long m = wave_ballot((in[u] >> c & 1u) != 0u);
+        const int pos = place[c] + lanes_below(m);
+        if ((in[u] >> c & 1u) && pos < kOctantCap) s_octant[c][pos] = number;
+        place[c] += (int) __popcll(m);
       }
     }
-    uint16_t* mine = s_octant[wave];
-    n_from = collect_near(s_y, s_sub, n_sub, lo, hi, widened(wave_kth_bound(nearest, K)), kOctantCap, mine);
-    from   = mine;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __syncthreads();
+    from = s_octant[wave];
   }
   constexpr int kTogether = kIn > 1 ? 2 : kAhead;
   constexpr int kCells = kIn * kIn * kIn;  // c: half of the octant along x in bit 0, along y in bit 1, along z in bit 2
@@ -561,7 +656,7 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
       n[c] += (int) __popcll(m);
     }
   }
-  // The lists again, to be put in order (ranks counted over LDS instead of the networks: 24 us instead of 10): an entry or two per lane, all of them on their way together.
+  // The lists again, to be put in order (ranks counted over LDS instead of the networks: 14 us more): an entry or two per lane, all of them on their way together.
   constexpr int kEntries = kOrder ? kListCap / kWave : 1;
   uint32_t held[kCells][kEntries];
   if constexpr (kOrder) {
@@ -613,12 +708,6 @@ __global__ void __launch_bounds__(kBuildThreads) knn_cell_lists_kernel(int M, in
 #pragma unroll
   for (int c = 0; c < kCells; ++c)
     if (lane == 0) cells[(list[c] - lists) / kListCap] = cell[c];
-}
-
-__device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
-  uint32_t r;
-  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
 }
 
 __device__ __forceinline__ uint32_t and_or_b32(uint32_t a, uint32_t mask, uint32_t b) {

@@ -291,6 +291,26 @@ def test_knn_control_points_with_nan(N, M, K, axes, count, device):
     assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
 
 
+# A block's wavefronts share its coarse list for all octants: shares of one to five steps of 64, of a few wavefronts and of all; points on
+# a sphere are all in reach of the cells inside it (octants with more candidates than their lists hold), points on a line of few.
+@pytest.mark.parametrize('M', [641, 1023, 1025, 2047, 2560])
+@pytest.mark.parametrize('kind', ['sphere', 'line', 'shrunk'])
+@pytest.mark.parametrize('K', [1, 8])
+def test_knn_octant_shares(M, kind, K, device):
+    from fast_sp_gs_amd._C import get_C_function
+    g = torch.Generator().manual_seed(M + K)
+    pts, ctrl = torch.randn(20_000, 3, generator=g), torch.randn(M, 3, generator=g)
+    if kind == 'sphere':
+        ctrl = torch.nn.functional.normalize(ctrl, dim=1)
+    elif kind == 'line':
+        ctrl[:, 1:] = 0.25
+    else:  # most of them in one coarse cell
+        ctrl[::2] *= 0.02
+    d2, idx = get_C_function('knn_topk')(pts.to(device), ctrl.to(device), K)
+    want_d, want_i = _all_pairs_knn(pts, ctrl, K, device)
+    assert torch.equal(idx, want_i) and torch.equal(d2, want_d)
+
+
 def _knn_time(pts, ctrl, K):
     """Microseconds a call: the best of five times 20."""
     from fast_sp_gs_amd._C import get_C_function
