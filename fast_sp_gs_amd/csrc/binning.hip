@@ -886,7 +886,7 @@ __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned*
   return most;
 }
 
-// Sorts the n <= 256 * kPer entries at `entries` by a 256-lane block and writes list and keys. Bound by its chain of about ten
+// Sorts n <= 256 * kPer entries by a 256-lane block and writes list and keys. Bound by its chain of about ten
 // LDS round trips and five barriers, whatever n is, where the network takes 33 rounds and 7 barriers for 2048 entries: against
 // the network (merging up to 256 entries), 400k surfels 3840x2160 153 -> 41 us, 3M 1352x1014 62 -> 18, 300k 800x800 24 -> 7.6,
 // 300k Gaussians 29 -> 7.9, 150k 1001x667 9.2 -> 4.6, 10k 256x256 5.1 -> 3.7. With depths in two thin shells, which take the
@@ -900,16 +900,17 @@ __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned*
 // has entries, by its depths, or, if it holds a single one, by the surfels' numbers, which decide among equal depths. (To find those
 // buckets costs segments without one about 2 us of the 116.) False, with nothing written and the keys in `key`, when that leaves too
 // many together as well (numbers in clumps, half a bucket at one depth): the comparing sorts take such a segment.
-template <int kPer>
-__device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, const uint64_t* __restrict__ entries,
-                                            uint64_t (&key)[kPer], uint64_t* s_e, int32_t* __restrict__ point_list,
-                                            int64_t* __restrict__ keys_out) {
+// load(i): entry i, from memory, or, kHeld, from s_e itself.
+template <int kPer, bool kHeld, typename Load>
+__device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, Load load, uint64_t (&key)[kPer], uint64_t* s_e,
+                                            int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
   constexpr int kBuckets = kPer == 1 ? kSortBuckets / 2 : kSortBuckets, kOwn = kBuckets / 256;
   unsigned* s_count = (unsigned*) (s_e + kSmallSegment);
   unsigned* s_wave  = (unsigned*) s_e;  // before the entries come
   const int wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) key[q] = entries[start + min((int) threadIdx.x + 256 * q, n - 1)];
+  for (int q = 0; q < kPer; ++q) key[q] = load(min((int) threadIdx.x + 256 * q, n - 1));
+  if (kHeld) __syncthreads();
   unsigned lo = ~0u, hi = 0u;
 #pragma unroll
   for (int c = 0; c < kOwn; ++c) s_count[kOwn * threadIdx.x + c] = 0u;
@@ -1013,6 +1014,37 @@ __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, cons
   return true;
 }
 
+// n <= kSmallSegment entries (see bucket_sort for load and kHeld), by as many a lane as they need; s_e holds kSmallSegment + kSmallSegment / 4.
+template <bool kHeld, typename Load>
+__device__ __forceinline__ void sort_small_segment(int tile, int64_t start, int n, Load load, uint64_t* s_e,
+                                                   int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
+  auto sort = [&](auto per) {  // entries per lane
+    constexpr int kPer = decltype(per)::value;
+    uint64_t key[kPer];
+    if (bucket_sort<kPer, kHeld>(tile, start, n, load, key, s_e, point_list, keys_out)) return;
+    if constexpr (kPer == 1) {
+      s_e[threadIdx.x] = (int) threadIdx.x < n ? key[0] : ~0ull;
+      __syncthreads();
+      merge_sort_lds(s_e, n);
+      tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
+    } else {
+      const int m = padded_length(n);
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int k = threadIdx.x + 256 * q;
+        if (k < m) s_e[lds_slot<true>(k)] = k < n ? key[q] : ~0ull;
+      }
+      __syncthreads();
+      bitonic_sort_lds<true>(s_e, m, 256);
+      tile_sort_output<true>(tile, start, n, s_e, point_list, keys_out);
+    }
+  };
+  if (n <= kMergeSegment) sort(std::integral_constant<int, 1>());
+  else if (n <= 512) sort(std::integral_constant<int, 2>());
+  else if (n <= 1024) sort(std::integral_constant<int, 4>());
+  else sort(std::integral_constant<int, 8>());
+}
+
 // One block per tile: segments up to kSmallSegment entries are sorted in LDS by as many entries per lane as they need (the
 // first loads of all are in flight together), longer ones are queued for
 // tile_sort_large_kernel; empty tiles get the (0, 0) range the reference's zero-initialised output has.
@@ -1048,32 +1080,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) t
     if (threadIdx.x == 0) large_list[atomicAdd(large_count, 1)] = tile;
     return;
   }
-  const int n = (int) len;
-  auto sort = [&](auto per) {  // entries per lane
-    constexpr int kPer = decltype(per)::value;
-    uint64_t key[kPer];
-    if (bucket_sort(tile, start, n, entries, key, s_e, point_list, keys_out)) return;
-    if constexpr (kPer == 1) {
-      s_e[threadIdx.x] = (int) threadIdx.x < n ? key[0] : ~0ull;
-      __syncthreads();
-      merge_sort_lds(s_e, n);
-      tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
-    } else {
-      const int m = padded_length(n);
-#pragma unroll
-      for (int q = 0; q < kPer; ++q) {
-        const int k = threadIdx.x + 256 * q;
-        if (k < m) s_e[lds_slot<true>(k)] = k < n ? key[q] : ~0ull;
-      }
-      __syncthreads();
-      bitonic_sort_lds<true>(s_e, m, 256);
-      tile_sort_output<true>(tile, start, n, s_e, point_list, keys_out);
-    }
-  };
-  if (n <= kMergeSegment) sort(std::integral_constant<int, 1>());
-  else if (n <= 512) sort(std::integral_constant<int, 2>());
-  else if (n <= 1024) sort(std::integral_constant<int, 4>());
-  else sort(std::integral_constant<int, 8>());
+  sort_small_segment<false>(tile, start, (int) len, [&](int i) { return entries[start + i]; }, s_e, point_list, keys_out);
 }
 
 // The first cut of bucket_sort for the n <= 1024 * kPer entries of a long segment, by a 1024-lane block. False, with nothing written,
@@ -1187,46 +1194,247 @@ __device__ __forceinline__ bool bucket_sort_huge(int tile, int64_t start, int64_
   return true;
 }
 
-// A few blocks walk the queue of long segments: up to kLargeSegment entries in LDS, by buckets or, where their depths lie too close
+struct LargeSortLds {
+  uint64_t e[kLargeSegment];
+  unsigned count[kLargeBuckets];
+  unsigned wave[2 * 1024 / kWave];
+};
+
+// A long segment by a block of 1024 lanes: up to kLargeSegment entries in LDS, by buckets or, where their depths lie too close
 // together, by the sorting network; longer ones by groups of buckets, or by the network on the global array.
 // Against the network, us a launch: 98k surfels 170x120 (lists of 3 to 6 thousand) 52 -> 8, 577k 228x227 108 -> 14, 2M 600x500 96 -> 15;
 // lists above 16 384, 2M 160x110: 1760 (the network) -> 258.
+__device__ __forceinline__ void sort_large_segment(int tile, int64_t start, int64_t len, uint64_t* __restrict__ entries, LargeSortLds& s,
+                                                   int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
+  if (len <= kLargeSegment) {
+    const int n = (int) len;
+    __syncthreads();  // the counters and the entries of the segment before have been read
+    bool sorted;
+    if (n <= 4096) sorted = bucket_sort_large<4>(tile, start, n, entries, s.e, s.count, s.wave, point_list, keys_out);
+    else if (n <= 8192) sorted = bucket_sort_large<8>(tile, start, n, entries, s.e, s.count, s.wave, point_list, keys_out);
+    else sorted = bucket_sort_large<16>(tile, start, n, entries, s.e, s.count, s.wave, point_list, keys_out);
+    if (sorted) return;
+    __syncthreads();
+    const int m = padded_length(n);
+    for (int k = threadIdx.x; k < m; k += 1024) s.e[k] = k < n ? entries[start + k] : ~0ull;
+    __syncthreads();
+    bitonic_sort_lds<false>(s.e, m, 1024);
+    tile_sort_output<false>(tile, start, n, s.e, point_list, keys_out);
+    __syncthreads();
+  } else {
+    __syncthreads();
+    if (bucket_sort_huge(tile, start, len, entries, s.e, s.count, s.wave, point_list, keys_out)) return;
+    uint64_t* e = entries + start;
+    bitonic_sort<int64_t>(e, len, 1024, [] {
+      __threadfence_block();
+      __syncthreads();
+    });
+    tile_sort_output<false>(tile, start, (int) len, e, point_list, keys_out);
+  }
+}
+
+// A few blocks walk the queue of long segments.
 __global__ void __launch_bounds__(1024) tile_sort_large_kernel(const int64_t* __restrict__ ranges,
     uint64_t* __restrict__ entries, int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out,
     const int* __restrict__ large_count, const int* __restrict__ large_list) {
-  __shared__ uint64_t s_e[kLargeSegment];
-  __shared__ unsigned s_count[kLargeBuckets];
-  __shared__ unsigned s_wave[2 * 1024 / kWave];
+  __shared__ LargeSortLds s;
   const int n_large = *large_count;
   for (int q = blockIdx.x; q < n_large; q += gridDim.x) {
     const int tile = large_list[q];
     const int64_t start = ranges[2 * (size_t) tile];
-    const int64_t len   = ranges[2 * (size_t) tile + 1] - start;
-    if (len <= kLargeSegment) {
-      const int n = (int) len;
-      __syncthreads();  // the counters and the entries of the segment before have been read
-      bool sorted;
-      if (n <= 4096) sorted = bucket_sort_large<4>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
-      else if (n <= 8192) sorted = bucket_sort_large<8>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
-      else sorted = bucket_sort_large<16>(tile, start, n, entries, s_e, s_count, s_wave, point_list, keys_out);
-      if (sorted) continue;
-      __syncthreads();
-      const int m = padded_length(n);
-      for (int k = threadIdx.x; k < m; k += 1024) s_e[k] = k < n ? entries[start + k] : ~0ull;
-      __syncthreads();
-      bitonic_sort_lds<false>(s_e, m, 1024);
-      tile_sort_output<false>(tile, start, n, s_e, point_list, keys_out);
-      __syncthreads();
-    } else {
-      __syncthreads();
-      if (bucket_sort_huge(tile, start, len, entries, s_e, s_count, s_wave, point_list, keys_out)) continue;
-      uint64_t* e = entries + start;
-      bitonic_sort<int64_t>(e, len, 1024, [] {
-        __threadfence_block();
-        __syncthreads();
-      });
-      tile_sort_output<false>(tile, start, (int) len, e, point_list, keys_out);
+    sort_large_segment(tile, start, ranges[2 * (size_t) tile + 1] - start, entries, s, point_list, keys_out);
+  }
+}
+
+// ---- lists of a small view, tile by tile ------------------------------------------------------------------------------
+// A small view's counting, prefix, scatter and sort are four or five launches of 2 to 7 us each, most of them latency: its lists are
+// formed by the tiles' own blocks instead. A block looks at every surfel's rectangle of tiles (a word each, left by the preprocess kernel:
+// three instructions for whether the tile is in it), checks the keep masks of those that contain it, sorts what remains and
+// leaves it in a place of its own; a second launch moves the lists together. Bound by the latency of its loads and, from some millions of
+// looks on, by its instructions. Kernels, us, count, prefix, scatter and the two sorts -> gather and place: 10k surfels 256x256
+// 3.8 + 4.7 + 4.7 + 3.7 + 1.7 -> 6.7 + 3.5; 25k Gaussians 639x361 4.9 + 5.9 + 6.8 + 4.1 + 1.8 -> 11 + 4.1; 50k surfels 501x403
+// 4.5 + 7.2 + 6.6 + 4.6 + 1.8 -> 17 + 4.5. (Words tested by a ballot each whether or not one was in, held by the block behind barriers, one
+// load ahead: 8.7, 17.6 and 29.)
+// The work grows with surfels times tiles, but the others' prefix is one block's up to 1024 tiles. Views, us, so binned -> gathered:
+// 5k surfels 640x480 (1200 tiles) 50 -> 42.5, 20k 54.5 -> 51.7, 25k 800x600 (1900, 47.5M looks) 62.2 -> 62.3, 30k Gaussians
+// 800x600 (57M) 54.9 -> 56.3; 1024 tiles and fewer: 65k surfels 500x500 90 -> 82, 440x440 91 -> 85, 65k Gaussians 440x440 85 -> 80, one
+// surfel 47 -> 44. With long lists: 8000 surfels 256x256, 1220 entries a tile, 255 -> 235, 40k 160x160, up to 2961, 294 -> 241.
+constexpr int kGatherSide  = 127;    // tiles along either axis: a rectangle is four numbers of seven bits
+constexpr int kGatherTiles = 2040;   // two a lane in the second launch, and eight a block: 255 blocks, and one for the schedule
+constexpr int kGatherChunk = 16 * kWave;  // surfels that a wavefront looks at in one go
+constexpr int kGatherHeld  = 2 * kGatherChunk;  // of them, what a wavefront can hold
+constexpr int kGatherMost  = 65535;  // surfels: their numbers are held in 16 bits
+constexpr int64_t kGatherLooks = 48000000;  // surfels times tiles, above 1024 tiles (see above)
+
+// Bytes of a rectangle's word: first column, 127 - last column, first row, 127 - last row. gather_word(tx, ty) less it has the upper
+// bit of a byte set where the tile is on the rectangle's side of that bound.
+__device__ __forceinline__ uint32_t gather_word(int tx, int ty) {
+  return 0x80808080u | (uint32_t) tx | (uint32_t) (127 - tx) << 8 | (uint32_t) ty << 16 | (uint32_t) (127 - ty) << 24;
+}
+__device__ __forceinline__ bool gather_hit(uint32_t tile, uint32_t rect) { return ((tile - rect) & 0x80808080u) == 0x80808080u; }
+
+// Whether the keep mask of a surfel (its rectangle contains the tile) keeps the tile: what for_each_instance<kWalkMask> visits.
+__device__ __forceinline__ bool gather_keeps(uint32_t rect, uint32_t mask, int tx, int ty) {
+  const int x0 = (int) (rect & 127u), y0 = (int) (rect >> 16 & 127u), w = 128 - (int) (rect >> 8 & 127u) - x0, h = 128 - (int) (rect >> 24) - y0;
+  const int x = tx - x0, y = ty - y0;
+  if (w * h <= kCullMaskTiles) return mask >> (y * w + x) & 1u;
+  const TileWindow v = tile_window(mask, w, h);
+  const int sum = x + y, diff = x - y + h - 1;
+  return x >= v.x0 && x <= v.x1 && y >= v.y0 && y <= v.y1 && sum >= v.s0 && sum <= v.s1 && diff >= v.d0 && diff <= v.d1;
+}
+
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
+  return (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) m, 0u));
+}
+
+// A place behind `at` (LDS) for each lane that is `on`; all lanes of a wavefront together.
+__device__ __forceinline__ int gather_place(bool on, int* at) {
+  const unsigned long long m = __ballot(on);
+  if (m == 0ull) return 0;
+  int base = 0;
+  if (__lane_id() == 0) base = atomicAdd(at, (int) __popcll(m));
+  return __builtin_amdgcn_readfirstlane(base) + lanes_below(m);
+}
+
+__global__ void __launch_bounds__(256) tile_gather_kernel(int P, int gx, const uint32_t* __restrict__ rects,
+    const uint32_t* __restrict__ masks, const float* __restrict__ depths, uint32_t* __restrict__ counts, int32_t* __restrict__ lists,
+    SlotPublish publish) {
+  constexpr int kWaves = 256 / kWave, kQuads = kGatherChunk / (4 * kWave);  // quads: of four words a lane
+  __shared__ __align__(16) uint64_t s_e[kSmallSegment + kSmallSegment / 4];
+  __shared__ uint16_t s_held[kWaves][kGatherHeld];  // surfels whose rectangle contains the tile
+  __shared__ int s_kept;
+  if (blockIdx.x == 0 && threadIdx.x < kWave) publish_slot_regions(publish);
+  const int tile = blockIdx.x, ty = tile / gx, tx = tile - ty * gx, lane = __lane_id(), wave = threadIdx.x / kWave;
+  const uint32_t word = gather_word(tx, ty);
+  uint16_t* const held = s_held[wave];
+  int n_held = 0;
+  // behind the last surfel the rectangles contain no tile up to a multiple of 256, behind that another quad's are read and not looked at
+  auto words = [&](int first, uint4 (&r)[kQuads]) {
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q) {
+      const int at = first + 4 * kWave * q;
+      r[q] = *(const uint4*) (rects + (at < P ? at : 0) + 4 * lane);
     }
+  };
+  constexpr int kStep = kWaves * kGatherChunk;
+  uint4 r[3][kQuads];  // two goes' words are on their way
+  const int begin = __builtin_amdgcn_readfirstlane(wave) * kGatherChunk;
+  words(begin, r[0]), words(begin + kStep, r[1]);
+  if (threadIdx.x == 0) s_kept = 0;
+  __syncthreads();
+  auto keep_held = [&] {  // of the surfels held, those kept, as entries to be sorted
+    wave_lds_sync();
+    for (int e0 = 0; e0 < n_held; e0 += kWave) {
+      const int e = e0 + lane;
+      const int i = held[min(e, n_held - 1)];
+      const uint32_t depth = __float_as_uint(depths[i]);
+      const bool kept = e < n_held && (!masks || gather_keeps(rects[i], masks[i], tx, ty));
+      const int at = gather_place(kept, &s_kept);
+      if (kept && at < kSmallSegment) s_e[at] = (uint64_t) depth << 32 | (uint32_t) i;
+    }
+    wave_lds_sync();
+    n_held = 0;
+  };
+  auto look = [&](int first, const uint4 (&r)[kQuads]) {
+    auto one = [&](uint32_t rect, int i) {
+      const bool hit = gather_hit(word, rect);
+      if (const unsigned long long m = __ballot(hit)) {  // one in five, or fewer
+        if (hit) held[n_held + lanes_below(m)] = (uint16_t) i;
+        n_held += (int) __popcll(m);
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q) {
+      const int at = first + 4 * kWave * q;
+      if (at >= P) break;
+      one(r[q].x, at + 4 * lane), one(r[q].y, at + 4 * lane + 1), one(r[q].z, at + 4 * lane + 2), one(r[q].w, at + 4 * lane + 3);
+    }
+    if (n_held > kGatherHeld - kGatherChunk) keep_held();
+  };
+  for (int first = begin; first < P; first += 3 * kStep) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      if (first + u * kStep >= P) break;
+      words(first + (u + 2) * kStep, r[(u + 2) % 3]);
+      look(first + u * kStep, r[u]);
+    }
+  }
+  keep_held();
+  __syncthreads();
+  const int n = s_kept;
+  if (threadIdx.x == 0) counts[tile] = (uint32_t) n;
+  if (n == 0 || n > kSmallSegment) return;  // a longer list is left to tile_place_kernel
+  sort_small_segment<true>(tile, (int64_t) tile * kSmallSegment, n, [&](int i) { return s_e[i]; }, s_e, lists, nullptr);
+}
+
+// The lists one behind the other, kTiles tiles a block, and the ranges; lists of more than kSmallSegment entries are formed here.
+// One block more than that where the blend kernels' schedule is to be built, the first one: it takes longest. A block takes a compute
+// unit's LDS, so that there are 256 of them at most (257 took 6.2 us instead of 4.5), and no more tiles share one than have to: 65k
+// surfels in 16 tiles, lists of up to 16 817 entries, four a block 961 us a view, one a block 816 (947 by the queue of long segments).
+constexpr int kPlaceBlocks = 255;
+template <int kTiles>
+__global__ void __launch_bounds__(1024) tile_place_kernel(int P, int gx, int gy, int64_t R, const uint32_t* __restrict__ rects,
+    const uint32_t* __restrict__ masks, const float* __restrict__ depths, const uint32_t* __restrict__ counts,
+    const int32_t* __restrict__ lists, int64_t* __restrict__ ranges, int32_t* __restrict__ point_list, uint64_t* __restrict__ entries,
+    int* __restrict__ order_table) {
+  __shared__ LargeSortLds s;
+  constexpr int kLanes = 1024 / kTiles;
+  __shared__ int s_end[2048];  // of the tiles' lists
+  const int T = gx * gy, lane = __lane_id(), wave = threadIdx.x / kWave;
+  if (order_table && blockIdx.x == 0) {
+    static_assert(sizeof(TileOrderLds) <= sizeof(s.e), "the schedule's LDS fits");
+    build_tile_order(gx, gy, [&](int t) { return (int64_t) counts[t]; }, order_table, order_table + kMaxOrderedTiles,
+                     *reinterpret_cast<TileOrderLds*>(s.e));
+    return;
+  }
+  const int t0 = 2 * (int) threadIdx.x, low = t0 < T ? (int) counts[t0] : 0, mine = low + (t0 + 1 < T ? (int) counts[t0 + 1] : 0);
+  const int block = (int) blockIdx.x - (order_table ? 1 : 0), own = kTiles * block + (int) threadIdx.x / kLanes;  // this lane's tile
+  const int k0 = threadIdx.x % kLanes;
+  const int32_t* list = lists + (size_t) min(own, T - 1) * kSmallSegment;
+  const int32_t ahead[2] = {list[k0], list[k0 + kLanes]};  // whatever they are: on their way with the counts
+  const int inc  = wave_scan(mine);
+  if (lane == kWave - 1) s.wave[wave] = (unsigned) inc;
+  __syncthreads();
+  int before = 0;
+#pragma unroll
+  for (int w = 0; w < 1024 / kWave; ++w) before += w < wave ? (int) s.wave[w] : 0;
+  s_end[t0] = before + inc - mine + low, s_end[t0 + 1] = before + inc;
+  __syncthreads();
+  auto start_of = [&](int t) { return t > 0 ? s_end[t - 1] : 0; };
+  int is_long = 0;
+  if (own < T) {
+    const int start = start_of(own), n = s_end[own] - start;
+    if (k0 == 0) ranges[2 * (size_t) own] = n ? start : 0, ranges[2 * (size_t) own + 1] = n ? start + n : 0;
+    if (n <= kSmallSegment) {
+      auto put = [&](int k, int32_t i) {
+        if (k < n && start + k < R) point_list[start + k] = i;
+      };
+      put(k0, ahead[0]), put(k0 + kLanes, ahead[1]);
+      for (int k = k0 + 2 * kLanes; k < n; k += kLanes) put(k, list[k]);
+    } else {
+      is_long = 1;
+    }
+  }
+  if (!__syncthreads_or(is_long)) return;
+  for (int q = 0; q < kTiles; ++q) {
+    const int t = kTiles * block + q;
+    if (t >= T) return;
+    const int start = start_of(t), n = s_end[t] - start, ty = t / gx, tx = t - ty * gx;
+    if (n <= kSmallSegment || (int64_t) start + n > R) continue;
+    const uint32_t word = gather_word(tx, ty);
+    int* at = (int*) s.wave;
+    __syncthreads();
+    if (threadIdx.x == 0) *at = 0;
+    __syncthreads();
+    for (int i0 = 0; i0 < P; i0 += 1024) {
+      const int i = min(i0 + (int) threadIdx.x, P - 1);
+      const uint32_t rect = rects[i];
+      const bool kept = i0 + (int) threadIdx.x < P && gather_hit(word, rect) && (!masks || gather_keeps(rect, masks[i], tx, ty));
+      const int to = gather_place(kept, at);
+      if (kept && to < n) entries[start + to] = (uint64_t) __float_as_uint(depths[i]) << 32 | (uint32_t) i;
+    }
+    __threadfence_block();
+    sort_large_segment(t, start, n, entries, s, point_list, nullptr);
   }
 }
 
@@ -1814,6 +2022,71 @@ FSGS_API int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const 
     fill_scatter(P, W, H, means2D, depths, radii, view_inputs(inverse_m, opacities, keep_masks), capacity, ranges, workspace, bins, s);
   fill_sort(P, W, H, capacity, ranges, point_list, nullptr, workspace, bins, false, s);
   return check_launch("gs_view_sort");
+}
+
+namespace {
+struct GatherLayout {
+  size_t lists, bytes;
+};
+GatherLayout gather_layout(int T) {
+  GatherLayout l;
+  l.lists = align_up((size_t) T * sizeof(uint32_t), 256);
+  l.bytes = l.lists + (size_t) T * kSmallSegment * sizeof(int32_t);
+  return l;
+}
+}  // namespace
+
+FSGS_API int fsgs_gs_view_gathers(int P, int W, int H) {
+  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
+  return P > 0 && P <= kGatherMost && gx > 0 && gy > 0 && gx <= kGatherSide && gy <= kGatherSide && gx * gy <= kGatherTiles &&
+         (gx * gy <= 1024 || (int64_t) P * gx * gy <= kGatherLooks);
+}
+
+FSGS_API size_t fsgs_gs_view_gather_bytes(int W, int H) {
+  return gather_layout(((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile)).bytes;
+}
+
+FSGS_API int fsgs_gs_view_gather(int P, int W, int H, const float* depths, const uint32_t* tile_rects, const uint32_t* keep_masks,
+                                 uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, void* lists,
+                                 size_t lists_bytes, void* stream) {
+  FSGS_REQUIRE(fsgs_gs_view_gathers(P, W, H), "gs_view_gather: not a view for it");
+  FSGS_REQUIRE(depths && tile_rects && ((uintptr_t) tile_rects & 15) == 0 && slot_counters && lists,
+               "gs_view_gather: null pointer, or rectangles off a 16-byte boundary");
+  if (lists_bytes < fsgs_gs_view_gather_bytes(W, H))
+    return fail(kWorkspaceSmall, "gs_view_gather: lists %zu < %zu bytes", lists_bytes, fsgs_gs_view_gather_bytes(W, H));
+  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
+  tile_order_invalidate((hipStream_t) stream);
+  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  hipLaunchKernelGGL(tile_gather_kernel, dim3(gx * gy), dim3(256), 0, (hipStream_t) stream, P, gx, tile_rects,
+                     culling_enabled() ? keep_masks : nullptr, depths, (uint32_t*) lists,
+                     (int32_t*) ((char*) lists + gather_layout(gx * gy).lists),
+                     SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
+  return check_launch("gs_view_gather");
+}
+
+FSGS_API int fsgs_gs_view_place(int P, int W, int H, const float* depths, const uint32_t* tile_rects, const uint32_t* keep_masks,
+                                int64_t R, int64_t* ranges, int32_t* point_list, void* lists, size_t lists_bytes, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  FSGS_REQUIRE(fsgs_gs_view_gathers(P, W, H) && ranges && R >= 0 && R < (int64_t) 0x7fffffff, "gs_view_place: bad arguments");
+  const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
+  hipStream_t s = (hipStream_t) stream;
+  if (R == 0) {
+    launch_zero_ranges(gx * gy, ranges, s);
+    return check_launch("gs_view_place");
+  }
+  FSGS_REQUIRE(depths && tile_rects && point_list && lists && workspace, "gs_view_place: null pointer");
+  if (lists_bytes < fsgs_gs_view_gather_bytes(W, H) || workspace_bytes < (size_t) R * sizeof(uint64_t))
+    return fail(kWorkspaceSmall, "gs_view_place: lists %zu < %zu or workspace %zu < %zu bytes", lists_bytes,
+                fsgs_gs_view_gather_bytes(W, H), workspace_bytes, (size_t) R * sizeof(uint64_t));
+  const int* order = nullptr;
+  int* build       = nullptr;
+  (void) defer_tile_order(gx, gy, ranges, s, &order, &build);
+  const int T = gx * gy, tiles = T <= kPlaceBlocks ? 1 : T <= 2 * kPlaceBlocks ? 2 : T <= 4 * kPlaceBlocks ? 4 : 8;
+  auto kernel = tiles == 1 ? tile_place_kernel<1> : tiles == 2 ? tile_place_kernel<2> : tiles == 4 ? tile_place_kernel<4> : tile_place_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3(div_up(gx * gy, tiles) + (build ? 1 : 0)), dim3(1024), 0, s, P, gx, gy, R, tile_rects,
+                     culling_enabled() ? keep_masks : nullptr, depths, (const uint32_t*) lists,
+                     (const int32_t*) ((const char*) lists + gather_layout(gx * gy).lists), ranges, point_list, (uint64_t*) workspace, build);
+  return check_launch("gs_view_place");
 }
 
 // Waits until the count has been written. Reading the word is all it takes as long as the stream works; a stream that

@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
   if (view.counters) {
     int total;
     slot = slots_in_block(ok ? area : 0, s_wave_slots, total);
-    if (threadIdx.x == 0) block_slot = atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+    if (threadIdx.x == 0) block_slot = add_slots(view, total);
   }
   float adj[9];
 #pragma unroll

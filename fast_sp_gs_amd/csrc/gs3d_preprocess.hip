@@ -318,10 +318,11 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
     wanted = __ballot(ok);
     if (wanted) sh_regs.fetch(wanted, wave_base, P, kSplit ? sh_rest : shs, sh_regs.large(P));
   }
+  int total = 0;
+  unsigned long long added = 0;
   if (view.counters) {  // how many instances the view has
-    int total;
     (void) slots_in_block(ok ? sc.area : 0, s_wave_slots, total);
-    if (threadIdx.x == 0) atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+    if (threadIdx.x == 0) added = add_slots(view, total);
   }
   uint32_t keep = 0xffffffffu;
   if (keep_masks) {
@@ -364,6 +365,8 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
       if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
     }
   }
+  SlotSums sums;
+  if (view.counters && threadIdx.x == 0) sums.add(view, added, total);
   // cov3Ds is absent with a pre-computed 3D covariance: the caller hands that tensor on as the operator's output
   // rows of 24 and 12 bytes leave through LDS (wave_rows_out); with the early requests above 300k Gaussians 32 -> 30 us
   const bool rows = kWave && (((uintptr_t) cov3Ds | (uintptr_t) colors) & 15) == 0;
@@ -380,6 +383,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
     wave_rows_out<3>(s_rgb, wave_base, P, colors);
   }
   if (kWave && view.color_derivs) wave_derivs_out(s_wave_rows, derivs, wave_base, P, view.color_derivs);
+  if (threadIdx.x == 0) sums.publish(view);
+  if (view.tile_rects)  // up to the last block's end
+    view.tile_rects[i] = ok && f2i_sat(sc.radius) > 0 ? tile_rect_word(tile_rect(sc.px, sc.py, f2i_sat(sc.radius), gx, gy)) : kNoTiles;
   if (!valid) return;
   if (!rows && cov3Ds)
 #pragma unroll
@@ -768,13 +774,15 @@ FSGS_API int fsgs_gs_view_preprocess_derivs(int P, int W, int H, int sh_degree, 
     const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
     const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
     float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
-    uint32_t* keep_masks, float* color_derivs, void* stream) {
+    uint32_t* keep_masks, float* color_derivs, uint32_t* tile_rects, int64_t* num_rendered_host, void* stream) {
+  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  FSGS_REQUIRE(!tile_rects || (W <= 127 * kTile && H <= 127 * kTile), "gs_view_preprocess: %dx%d is too large for rectangles in a word", W, H);
   FSGS_REQUIRE(!color_derivs || wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0, "gs_view_preprocess: no derivatives of these rows");
   FSGS_REQUIRE(slot_counters, "gs_view_preprocess: slot_counters are required");
   return gs3d_preprocess_forward(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest,
                                  Tw2v, Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp,
                                  means2D_preserve, means2D, depths, colors, radii, nullptr, cov3Ds, conic_opacity, keep_masks,
-                                 ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, false, color_derivs}, stream);
+                                 ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, false, color_derivs, num_rendered_host, tile_rects}, stream);
 }
 
 FSGS_API int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, int is_opengl, const float* means3D,
@@ -786,7 +794,7 @@ FSGS_API int fsgs_gs_view_preprocess(int P, int W, int H, int sh_degree, int n_s
   return fsgs_gs_view_preprocess_derivs(P, W, H, sh_degree, n_sh, is_opengl, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v,
                                         Tv2c, campos, tan_fovx, tan_fovy, culling, cov3D_precomp, cov2D_precomp, means2D_preserve,
                                         means2D, depths, colors, radii, visible, slot_counters, cov3Ds, conic_opacity, keep_masks,
-                                        nullptr, stream);
+                                        nullptr, nullptr, nullptr, stream);
 }
 
 FSGS_API int fsgs_gs_view_preprocess_backward_derivs(int P, int W, int H, int sh_degree, int n_sh, int is_opengl,

@@ -69,14 +69,10 @@ Buffers forward_view(const GaussianView& v, bool train) {
   s.has_derivs = train && fsgs_view_keeps_color_derivs(v.sh_degree, M, f32(v.shs), sh_rest) != 0;
   if (s.has_derivs) s.derivs = b.keep.reserve((size_t) P * 36);
   b.keep.allocate(like);
-  Slab scratch;
-  const size_t depths = scratch.reserve((size_t) P * 4), masks_at = scratch.reserve((size_t) P * 4);
-  const size_t bins_bytes = fsgs_gs_prepare_bins_bytes((int) P, W, H);
-  const size_t bins = scratch.reserve(bins_bytes);
-  scratch.allocate(like);
+  const ViewScratch scratch(P, W, H, like);
 
   const float* colors = v.sh_degree < 0 ? f32(v.shs) : b.keep.at<float>(s.colors);
-  uint32_t* masks = v.cull ? scratch.at<uint32_t>(masks_at) : nullptr;
+  uint32_t* masks = v.cull ? scratch.at<uint32_t>(scratch.masks) : nullptr;
   auto blend_maps = [&] {
     b.image = empty({3, H, W}, like), b.opacity = empty({H, W}, like), b.n_contrib = empty({H, W}, like, at::kInt);
     if (has(v.extras)) b.extras = empty({E, H, W}, like);
@@ -87,32 +83,37 @@ Buffers forward_view(const GaussianView& v, bool train) {
     check(fsgs_gs_view_preprocess_derivs((int) P, W, H, v.sh_degree, M, v.is_opengl, f32(v.points), f32(v.scales),
                                          f32(v.rotations), f32(v.opacities), f32(v.shs), sh_rest, f32(v.Tw2v), f32(v.Tv2c),
                                          f32(v.campos), v.tan_x, v.tan_y, data<uint8_t>(opt(v.culling)), f32(opt(v.cov3D)),
-                                         f32(opt(v.cov2D)), v.preserve, f32(v.means2D), scratch.at<float>(depths),
+                                         f32(opt(v.cov2D)), v.preserve, f32(v.means2D), scratch.at<float>(scratch.depths),
                                          v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), i32(b.radii),
                                          data<uint8_t>(b.visible), counters.data(),
                                          has(v.cov3D) ? nullptr : b.keep.at<float>(s.cov3D), f32(b.conic_opacity), masks,
-                                         s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr, stream),
+                                         s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr, scratch.small_rects(),
+                                         scratch.small ? count : nullptr, stream),
           what);
-    check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
-                             nullptr, count, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
-          "GS_prepare");
-    PendingCount pending(count, stream);
-    counters.give_back();
-    const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
-      check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii),
-                                 masks, to.room, i64(b.ranges), scratch.at<void>(bins), bins_bytes, to.space.data_ptr(),
-                                 to.space.numel(), stream),
+    if (scratch.small) {
+      b.point_list = small_view_lists(scratch, P, W, H, masks, counters, nullptr, b.ranges, count, stream, blend_maps);
+    } else {
+      check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
+                               nullptr, count, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, stream),
             "GS_prepare");
-    }, blend_maps);
-    b.point_list = empty({in.count}, like, at::kInt);
-    check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks,
-                            in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes,
-                            data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
-          "GS_prepare");
+      PendingCount pending(count, stream);
+      counters.give_back();
+      const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
+        check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(scratch.depths), nullptr, i32(b.radii),
+                                   masks, to.room, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, to.space.data_ptr(),
+                                   to.space.numel(), stream),
+              "GS_prepare");
+      }, blend_maps);
+      b.point_list = empty({in.count}, like, at::kInt);
+      check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(scratch.depths), nullptr, i32(b.radii), masks,
+                              in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(scratch.bins), scratch.bins_bytes,
+                              data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
+            "GS_prepare");
+    }
   } else {
     blend_maps();
     b.point_list = empty({0}, like, at::kInt);
-    check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
+    check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, stream),
           "GS_prepare");
   }
   if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);

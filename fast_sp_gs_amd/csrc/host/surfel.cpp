@@ -75,11 +75,7 @@ Buffers forward_view(const SurfelView& v, bool train) {
     if (s.has_derivs) s.derivs = b.keep.reserve((size_t) P * 36);
   }
   b.keep.allocate(like);
-  Slab scratch;
-  const size_t depths = scratch.reserve((size_t) P * 4);
-  const size_t bins_bytes = fsgs_gs_prepare_bins_bytes((int) P, W, H);
-  const size_t bins = scratch.reserve(bins_bytes);
-  scratch.allocate(like);
+  const ViewScratch scratch(P, W, H, like);
 
   const float* colors = v.sh_degree < 0 ? f32(v.shs) : b.keep.at<float>(s.colors);
   uint32_t* masks = v.cull ? b.keep.at<uint32_t>(s.masks) : nullptr;
@@ -98,40 +94,46 @@ Buffers forward_view(const SurfelView& v, bool train) {
   if (P > 0) {
     SlotCounters counters(like);
     int64_t* count = pinned_count();
+    int64_t* count_of_small = scratch.small ? count : nullptr;
     auto preprocess = [&](auto entry, auto... outputs) {
       check(entry((int) P, W, H, v.sh_degree, M, f32(v.points), f32(v.scales), f32(v.rotations), f32(v.opacities), f32(v.shs),
                   sh_rest, f32(v.Tw2v), f32(v.Tv2c), f32(v.campos), data<uint8_t>(opt(v.culling)), f32(v.means2D),
                   v.sh_degree < 0 ? nullptr : b.keep.at<float>(s.colors), f32(b.trans_mat), f32(b.normal_opacity),
-                  scratch.at<float>(depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles), outputs...,
+                  scratch.at<float>(scratch.depths), i32(b.radii), data<uint8_t>(b.visible), b.keep.at<int32_t>(s.tiles), outputs...,
                   stream),
             what);
     };
     if (train)
       preprocess(fsgs_gs_2d_view_preprocess_derivs, b.keep.at<int32_t>(s.offsets), counters.data(), records, masks,
-                 s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr);
-    else preprocess(fsgs_gs_2d_view_preprocess_no_backward, counters.data(), records, masks);
-    check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
-                             train ? b.keep.at<int32_t>(s.regions) : nullptr, count, i64(b.ranges), scratch.at<void>(bins),
-                             bins_bytes, stream),
-          "GS_prepare");
-    PendingCount pending(count, stream);
-    counters.give_back();
-    const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
-      check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii),
-                                 masks, to.room, i64(b.ranges), scratch.at<void>(bins), bins_bytes, to.space.data_ptr(),
-                                 to.space.numel(), stream),
+                 s.has_derivs ? b.keep.at<float>(s.derivs) : nullptr, scratch.small_rects(), count_of_small);
+    else preprocess(fsgs_gs_2d_view_preprocess_no_backward_rects, counters.data(), records, masks, scratch.small_rects(), count_of_small);
+    int32_t* regions = train ? b.keep.at<int32_t>(s.regions) : nullptr;
+    if (scratch.small) {
+      b.point_list = small_view_lists(scratch, P, W, H, masks, counters, regions, b.ranges, count, stream, blend_maps);
+      s.R = b.point_list.numel();
+    } else {
+      check(fsgs_gs_view_count((int) P, W, H, f32(v.means2D), nullptr, nullptr, i32(b.radii), masks, counters.data(),
+                               regions, count, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, stream),
             "GS_prepare");
-    }, blend_maps);
-    s.R = in.count;
-    b.point_list = empty({in.count}, like, at::kInt);
-    check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(depths), nullptr, i32(b.radii), masks,
-                            in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(bins), bins_bytes,
-                            data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
-          "GS_prepare");
+      PendingCount pending(count, stream);
+      counters.give_back();
+      const Instances in = scatter_instances("GS_prepare", pending, instances_to_guess(P, T), like, [&](const Instances& to) {
+        check(fsgs_gs_view_scatter((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(scratch.depths), nullptr, i32(b.radii),
+                                   masks, to.room, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, to.space.data_ptr(),
+                                   to.space.numel(), stream),
+              "GS_prepare");
+      }, blend_maps);
+      s.R = in.count;
+      b.point_list = empty({in.count}, like, at::kInt);
+      check(fsgs_gs_view_sort((int) P, W, H, f32(v.means2D), nullptr, scratch.at<float>(scratch.depths), nullptr, i32(b.radii), masks,
+                              in.count, in.room, i64(b.ranges), i32(b.point_list), scratch.at<void>(scratch.bins), scratch.bins_bytes,
+                              data<void>(in.space), in.room > 0 ? in.space.numel() : 0, stream),
+            "GS_prepare");
+    }
   } else {
     blend_maps();
     b.point_list = empty({0}, like, at::kInt);
-    check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(bins), bins_bytes, stream),
+    check(fsgs_gs_prepare_count(0, W, H, nullptr, nullptr, i64(b.ranges), scratch.at<void>(scratch.bins), scratch.bins_bytes, stream),
           "GS_prepare");
   }
   if (train) b.hit_blocks = empty({b.point_list.numel()}, like, at::kInt);

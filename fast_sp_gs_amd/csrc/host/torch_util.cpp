@@ -118,7 +118,7 @@ SlotCounters::SlotCounters(const Tensor& like) : key_((int) like.device().index(
       --g_counters_kept;
     }
   }
-  if (!memory_.defined()) memory_ = at::zeros({kSlotRegions}, like.options().dtype(at::kLong));
+  if (!memory_.defined()) memory_ = at::zeros({kSlotRegions + 1}, like.options().dtype(at::kLong));
 }
 
 void SlotCounters::give_back() {

@@ -179,7 +179,40 @@ Instances scatter_instances(const char* what, PendingCount& pending, int64_t gue
   return in;
 }
 
-// 64 zeroed counters on the tensor's device for one view on its current stream. They go back to a list of that stream
+// A view's scratch. A small view (fsgs_gs_view_gathers) has its lists gathered tile by tile, by way of `rects` and `lists`, the others
+// are binned by way of `bins`, and so is a small one for whose lists (8 KB a tile) there is no memory.
+struct ViewScratch {
+  bool small = false;
+  size_t depths = 0, masks = 0, bins = 0, bins_bytes = 0, rects = 0, lists = 0, lists_bytes = 0;
+  Slab slab;
+  ViewScratch(int64_t P, int W, int H, const Tensor& like) {
+    if (fsgs_gs_view_gathers((int) P, W, H)) {
+      try {
+        lay_out(P, W, H, like, true);
+        return;
+      } catch (const c10::OutOfMemoryError&) {
+      }
+    }
+    lay_out(P, W, H, like, false);
+  }
+  template <typename T>
+  T* at(size_t offset) const {
+    return slab.at<T>(offset);
+  }
+  uint32_t* small_rects() const { return small ? slab.at<uint32_t>(rects) : nullptr; }
+
+ private:
+  void lay_out(int64_t P, int W, int H, const Tensor& like, bool as_small) {
+    slab = Slab(), small = as_small;
+    depths = slab.reserve((size_t) P * 4), masks = slab.reserve((size_t) P * 4);
+    lists_bytes = small ? fsgs_gs_view_gather_bytes(W, H) : 0, bins_bytes = small ? 0 : fsgs_gs_prepare_bins_bytes((int) P, W, H);
+    if (small) rects = slab.reserve((size_t) (P + 255) / 256 * 1024), lists = slab.reserve(lists_bytes);
+    else bins = slab.reserve(bins_bytes);
+    slab.allocate(like);
+  }
+};
+
+// 65 zeroed counters on the tensor's device for one view on its current stream. They go back to a list of that stream
 // once the kernel that zeroes them again is queued; a view that fails in between drops them.
 class SlotCounters {
  public:
@@ -191,5 +224,33 @@ class SlotCounters {
   Tensor memory_;
   std::pair<int, void*> key_;
 };
+
+// Both parts of a small view's binning (`regions` optional), behind a preprocess kernel that stores the count to `count`; `meanwhile()`
+// allocates what does not depend on it. Returns the list of as many places as there are instances.
+template <typename Meanwhile>
+Tensor small_view_lists(const ViewScratch& scratch, int64_t P, int W, int H, const uint32_t* masks, SlotCounters& counters,
+                        int32_t* regions, const Tensor& ranges, int64_t* count, void* stream, Meanwhile meanwhile) {
+  const char* what = "GS_prepare";
+  PendingCount pending(count, stream);
+  const float* depths = scratch.at<float>(scratch.depths);
+  check(fsgs_gs_view_gather((int) P, W, H, depths, scratch.small_rects(), masks, counters.data(), regions, nullptr,
+                            scratch.at<void>(scratch.lists), scratch.lists_bytes, stream),
+        what);
+  counters.give_back();
+  meanwhile();
+  // for lists too long to be sorted by their own blocks, as many entries as there may be: nearly always that is enough
+  Tensor space;
+  try {
+    space = empty({16 * P * 8}, ranges, at::kByte);
+  } catch (const c10::OutOfMemoryError&) {
+  }
+  const int64_t R = pending.wait(what);
+  const Tensor list = empty({R}, ranges, at::kInt);
+  if (!space.defined() || 8 * R > space.numel()) space = empty({8 * std::max<int64_t>(R, 1)}, ranges, at::kByte);
+  check(fsgs_gs_view_place((int) P, W, H, depths, scratch.small_rects(), masks, R, i64(ranges), i32(list),
+                           scratch.at<void>(scratch.lists), scratch.lists_bytes, space.data_ptr(), space.numel(), stream),
+        what);
+  return list;
+}
 
 }  // namespace fsgs_host

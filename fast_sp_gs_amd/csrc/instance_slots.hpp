@@ -75,19 +75,56 @@ struct ViewOutputs {
   uint8_t* visible = nullptr;
   bool windows = false;  // no backward follows: keep masks of large rectangles may be windows (cull_window)
   float* color_derivs = nullptr;  // [P, 9], for the backward; only where the coefficients' rows are complete (wave_row_floats)
+  int64_t* host_count = nullptr;  // pinned host memory: the instance count, as soon as it is known; the counters are 65 then
+  uint32_t* tile_rects = nullptr; // [P, up to a multiple of 256] tile_rect_word; grids of at most 127 x 127 tiles
 };
+
+// Thread 0 of a block of the preprocess kernel adds the block's instances to its region's counter (`added`: what was there before, of use
+// much later). With a host_count the counters count the blocks, too, above their sums: the last block of a region adds the region's
+// sum to one counter more, and the last region's block has the instances of the view, while most of the kernel is still to come.
+// A small view's binning is over before the host, told by the next kernel, has launched what needs the count: 10k surfels 256x256
+// 50 -> 47 us a view.
+constexpr int kSlotBlocksShift = 40;
+constexpr unsigned long long kSlotSum = (1ull << kSlotBlocksShift) - 1;
+__device__ __forceinline__ unsigned long long add_slots(const ViewOutputs& view, int total) {
+  return atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)],
+                   (unsigned long long) total + (view.host_count ? 1ull << kSlotBlocksShift : 0ull));
+}
+// In two steps, so that the second counter's answer is not waited for between them.
+struct SlotSums {
+  unsigned long long sum = 0, before = 0;  // sum: of the region, where this is its last block
+  bool last = false;
+  __device__ __forceinline__ void add(const ViewOutputs& view, unsigned long long added, int total) {
+    const int region = blockIdx.x & (kSlotRegions - 1), blocks = ((int) gridDim.x - region + kSlotRegions - 1) / kSlotRegions;
+    last = view.host_count && (int) (added >> kSlotBlocksShift) + 1 == blocks;
+    if (!last) return;
+    sum    = (added & kSlotSum) + (unsigned long long) total;
+    before = atomicAdd(&view.counters[kSlotRegions], sum + (1ull << kSlotBlocksShift));
+  }
+  __device__ __forceinline__ void publish(const ViewOutputs& view) const {
+    if (!last || (int) (before >> kSlotBlocksShift) + 1 != min((int) gridDim.x, kSlotRegions)) return;
+    view.counters[kSlotRegions] = 0ull;
+    __hip_atomic_store(view.host_count, (int64_t) ((before & kSlotSum) + sum), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+
+// A rectangle of tiles as a word (ViewOutputs::tile_rects): first column, 127 - last column, first row, 127 - last row.
+constexpr uint32_t kNoTiles = 0x7f7f7f7fu;
+__device__ __forceinline__ uint32_t tile_rect_word(const TileRect& r) {
+  return (uint32_t) r.x0 | (uint32_t) (128 - r.x1) << 8 | (uint32_t) r.y0 << 16 | (uint32_t) (128 - r.y1) << 24;
+}
 
 // What the kernel behind the preprocess hands on: see above. `counters` nullptr: nothing to do.
 struct SlotPublish {
   unsigned long long* counters = nullptr;  // [64], zeroed again
   int32_t* region = nullptr;               // [64] or nullptr
-  int64_t* host_count = nullptr;           // pinned host memory
+  int64_t* host_count = nullptr;           // pinned host memory, or nullptr
 };
 
 // One wavefront.
 __device__ __forceinline__ void publish_slot_regions(const SlotPublish& p) {
   const int lane = threadIdx.x & 63;
-  const unsigned long long mine = p.counters[lane];
+  const unsigned long long mine = p.counters[lane] & kSlotSum;
   unsigned long long inc = mine;
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -96,7 +133,7 @@ __device__ __forceinline__ void publish_slot_regions(const SlotPublish& p) {
   }
   if (p.region) p.region[lane] = (int32_t) (inc - mine);
   p.counters[lane] = 0ull;
-  if (lane == kWave - 1) __hip_atomic_store(p.host_count, (int64_t) inc, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (p.host_count && lane == kWave - 1) __hip_atomic_store(p.host_count, (int64_t) inc, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace fsgs

@@ -165,12 +165,11 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   }
 
   // the block's record slots: the atomic is on its way while the colours are formed
-  int slot = 0;
+  int slot = 0, total = 0;
   unsigned long long block_slot = 0;
   if (view.counters) {
-    int total;
     slot = slots_in_block(ok ? area : 0, s_wave_slots, total);
-    if (threadIdx.x == 0) block_slot = atomicAdd(&view.counters[blockIdx.x & (kSlotRegions - 1)], (unsigned long long) total);
+    if (threadIdx.x == 0) block_slot = add_slots(view, total);
   }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
@@ -196,6 +195,8 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
     }
   }
+  SlotSums sums;
+  if (view.counters && threadIdx.x == 0) sums.add(view, block_slot, total);
   if (view.slot_offsets) {
     if (threadIdx.x == 0) s_block_slot = (int) block_slot;
     __syncthreads();
@@ -230,6 +231,9 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     wave_rows_out<3>(s_wave_rows + 576, wave_base, P, colors);
   }
   if (kWave && view.color_derivs) wave_derivs_out(s_wave_rows, derivs, wave_base, P, view.color_derivs);
+  if (threadIdx.x == 0) sums.publish(view);
+  if (view.tile_rects)  // up to the last block's end
+    view.tile_rects[i] = ok && f2i_sat(radius) > 0 ? tile_rect_word(tile_rect(c2[0], c2[1], f2i_sat(radius), gx, gy)) : kNoTiles;
   if (!valid) return;
 
   if (view.slot_offsets) view.slot_offsets[i] = slot;
@@ -722,13 +726,16 @@ FSGS_API int fsgs_gs_2d_view_preprocess_derivs(int P, int W, int H, int sh_degre
     const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
     const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
     float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
-    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, void* stream) {
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, uint32_t* tile_rects,
+    int64_t* num_rendered_host, void* stream) {
   FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
+  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  FSGS_REQUIRE(!tile_rects || (W <= 127 * kTile && H <= 127 * kTile), "gs_2d_view_preprocess: %dx%d is too large for rectangles in a word", W, H);
   FSGS_REQUIRE(!color_derivs || wave_row_floats(sh_degree, n_sh, shs, sh_rest) != 0, "gs_2d_view_preprocess: no derivatives of these rows");
   return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
                             campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
                             tiles_touched, records, keep_masks,
-                            ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible, false, color_derivs}, stream);
+                            ViewOutputs{(unsigned long long*) slot_counters, slot_offsets, visible, false, color_derivs, num_rendered_host, tile_rects}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
@@ -738,7 +745,21 @@ FSGS_API int fsgs_gs_2d_view_preprocess(int P, int W, int H, int sh_degree, int 
     int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream) {
   return fsgs_gs_2d_view_preprocess_derivs(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
                                            campos, culling, means2D, colors, trans_mat, normal_opacity, depths, radii, visible,
-                                           tiles_touched, slot_offsets, slot_counters, records, keep_masks, nullptr, stream);
+                                           tiles_touched, slot_offsets, slot_counters, records, keep_masks, nullptr, nullptr, nullptr, stream);
+}
+
+FSGS_API int fsgs_gs_2d_view_preprocess_no_backward_rects(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest,
+    const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
+    float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    uint64_t* slot_counters, float* records, uint32_t* keep_masks, uint32_t* tile_rects, int64_t* num_rendered_host, void* stream) {
+  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
+  if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
+  FSGS_REQUIRE(!tile_rects || (W <= 127 * kTile && H <= 127 * kTile), "gs_2d_view_preprocess: %dx%d is too large for rectangles in a word", W, H);
+  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
+                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
+                            tiles_touched, records, keep_masks,
+                            ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, true, nullptr, num_rendered_host, tile_rects}, stream);
 }
 
 FSGS_API int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
@@ -746,11 +767,10 @@ FSGS_API int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_
     const float* Tw2v, const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors,
     float* trans_mat, float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
     uint64_t* slot_counters, float* records, uint32_t* keep_masks, void* stream) {
-  FSGS_REQUIRE(slot_counters, "gs_2d_view_preprocess: slot_counters are required");
-  return preprocess_forward(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v, Tv2c,
-                            campos, nullptr, culling, 0, means2D, colors, trans_mat, normal_opacity, depths, radii,
-                            tiles_touched, records, keep_masks,
-                            ViewOutputs{(unsigned long long*) slot_counters, nullptr, visible, true}, stream);
+  return fsgs_gs_2d_view_preprocess_no_backward_rects(P, W, H, sh_degree, n_sh, means3D, scales, rotations, opacities, shs, sh_rest, Tw2v,
+                                                      Tv2c, campos, culling, means2D, colors, trans_mat, normal_opacity, depths,
+                                                      radii, visible, tiles_touched, slot_counters, records, keep_masks, nullptr,
+                                                      nullptr, stream);
 }
 
 namespace {

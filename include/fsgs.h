@@ -69,13 +69,21 @@ int fsgs_gs_2d_view_preprocess_no_backward(int P, int W, int H, int sh_degree, i
 /* _derivs, of the surfels' preprocess and of the other two kinds' below: leaves the colours' derivatives by the view direction, too, nine
  * floats per point (channel-major; on a 16-byte boundary, zeros for points that are not rendered; nullptr: none), which the _derivs form
  * of the backward reads instead of the coefficients. Only for the rows of coefficients that fsgs_view_keeps_color_derivs accepts (all
- * of degree 3, on a 16-byte boundary). */
+ * of degree 3, on a 16-byte boundary). tile_rects[P, up to a multiple of 256] (optional, surfels and Gaussians): the rectangle of tiles as fsgs_gs_view_gather
+ * takes it, for pictures of at most 127 x 127 tiles; _no_backward_rects leaves it, too. num_rendered_host (optional, pinned memory, set
+ * to -1 here): gets the instance count before the kernel ends; slot_counters are 65 then, and fsgs_gs_view_gather is called without it. */
 int fsgs_view_keeps_color_derivs(int sh_degree, int n_sh, const float* shs, const float* sh_rest);
 int fsgs_gs_2d_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh, const float* means3D, const float* scales,
     const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
     const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
     float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
-    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, void* stream);
+    int32_t* slot_offsets, uint64_t* slot_counters, float* records, uint32_t* keep_masks, float* color_derivs, uint32_t* tile_rects,
+    int64_t* num_rendered_host, void* stream);
+int fsgs_gs_2d_view_preprocess_no_backward_rects(int P, int W, int H, int sh_degree, int n_sh, const float* means3D,
+    const float* scales, const float* rotations, const float* opacities, const float* shs, const float* sh_rest, const float* Tw2v,
+    const float* Tv2c, const float* campos, const uint8_t* culling, float* means2D, float* colors, float* trans_mat,
+    float* normal_opacity, float* depths, int32_t* radii, uint8_t* visible, int32_t* tiles_touched,
+    uint64_t* slot_counters, float* records, uint32_t* keep_masks, uint32_t* tile_rects, int64_t* num_rendered_host, void* stream);
 
 /* gs_2d_preprocess_backward -- gs_2d_preprocess.cu:423-499 (kernel :268-329). Every row of g_* is ASSIGNED: the
  * gradient for surfels with radii > 0, zeros for the others and for SH coefficients above the active degree (the
@@ -183,6 +191,20 @@ int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const float* in
                       const float* opacities, const int32_t* radii, const uint32_t* keep_masks, int64_t R, int64_t capacity,
                       int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
                       size_t workspace_bytes, void* stream);
+
+/* The same binning for a small view of surfels or 3D Gaussians (fsgs_gs_view_gathers: at most 65 535 of them and 1024 tiles, and not too
+ * many of both), in two parts: fsgs_gs_view_gather takes the place of fsgs_gs_view_count (slot_regions, slot_counters and
+ * num_rendered_host, here optional, as there) and leaves every tile's list in `lists` (fsgs_gs_view_gather_bytes bytes);
+ * fsgs_gs_view_place, with the count R, puts them into point_list[R] and writes ranges. tile_rects (on a 16-byte boundary) and depths
+ * are the preprocess kernels', keep_masks (optional) too; workspace: 8 R bytes. */
+int fsgs_gs_view_gathers(int P, int W, int H);
+size_t fsgs_gs_view_gather_bytes(int W, int H);
+int fsgs_gs_view_gather(int P, int W, int H, const float* depths, const uint32_t* tile_rects, const uint32_t* keep_masks,
+                        uint64_t* slot_counters, int32_t* slot_regions, int64_t* num_rendered_host, void* lists, size_t lists_bytes,
+                        void* stream);
+int fsgs_gs_view_place(int P, int W, int H, const float* depths, const uint32_t* tile_rects, const uint32_t* keep_masks, int64_t R,
+                       int64_t* ranges, int32_t* point_list, void* lists, size_t lists_bytes, void* workspace, size_t workspace_bytes,
+                       void* stream);
 
 /* ---- per-tile alpha blend ------------------------------------------------------------------------------------- */
 
@@ -617,7 +639,7 @@ int fsgs_gs_view_preprocess_derivs(int P, int W, int H, int sh_degree, int n_sh,
     const float* Tw2v, const float* Tv2c, const float* campos, double tan_fovx, double tan_fovy, const uint8_t* culling,
     const float* cov3D_precomp, const float* cov2D_precomp, int means2D_preserve, float* means2D, float* depths,
     float* colors, int32_t* radii, uint8_t* visible, uint64_t* slot_counters, float* cov3Ds, float* conic_opacity,
-    uint32_t* keep_masks, float* color_derivs, void* stream);
+    uint32_t* keep_masks, float* color_derivs, uint32_t* tile_rects, int64_t* num_rendered_host, void* stream);
 
 /* gs_preprocess_backward -- gaussian_preprocess.cu:567-636 (kernel :246-372, with gaussian_compute_cov2D.cu:64-186 and
  * gaussian_compute_cov3D.cu:76-118). grad_mean2D[P,2] is rewritten in place as (0.5 W g.x, +-0.5 H g.y) as in the
