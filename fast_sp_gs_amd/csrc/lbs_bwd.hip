@@ -20,6 +20,7 @@ namespace {
 
 constexpr int kTableFloats  = 36864;  // 144 KB of LDS for the per-block table
 constexpr int kMaxAccBlocks = 256;    // partial tables per launch
+constexpr int kAccPoints    = 512;  // a block, at least: its table has to be cleared, stored and added to the others'
 constexpr int kAccThreads   = 1024;  // 16 wavefronts share one LDS table: the loop is bound by gather latency, not by the atomics
 
 __global__ void __launch_bounds__(256) zero_floats_kernel(size_t n, float* __restrict__ p) {
@@ -178,7 +179,8 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(in
 
 // The same sums without float atomics, for tables of up to kStageTable cells and K <= kBinK neighbours: LDS float
 // atomics retire about one lane every three cycles on this chip, and the 18 per neighbour above are what that kernel's
-// time is made of. A block takes 1024 points at a time. Every lane does its point's own outputs and counts its
+// time is made of. A block takes up to 1024 points at a time, as many as leave every block the same number (with 1024 where there are
+// as many, 200k points were one block's work for 196 of the 256 compute units, 300k two blocks' for 37). Every lane does its point's own outputs and counts its
 // neighbours per control point (integer LDS atomics), the counts are scanned, every (point, neighbour) pair is placed
 // in its control point's bin (weight, kernel-mode factor, owning lane and slot), and then each table cell is summed by
 // one lane over its control point's bin from the points' gradients parked in LDS. Partial tables go out as in mode 1.
@@ -187,13 +189,16 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_accumulate_kernel(in
 // The sums are bound by LDS reads through the bins (a pair's owner, its factor, its features), so a lane sums four columns
 // that share their reads: a row of [dL/dR | dL/dt] from one component of g and (p, 1), the rotation and the scale residuals,
 // the offsets p - y. One column per lane took 46 us at 200k points, 512 control points, K = 4, and 19 us more for the
-// distances' gradient; together they are 33.
+// distances' gradient; together they were 33.
+// kStaged: the table of transforms passes through the LDS that the gradients are parked in afterwards. A lane gathers twenty 16-byte pieces
+// of it, from as many lines in the L1. Both together, 512 control points, K = 4: 20k points 20.3 -> 17.2 us, 60k 23.8 -> 17.5, 200k
+// 31.0 -> 26.6, 300k 47.3 -> 35.4 (unstaged 27.6 and 36.5; four pairs of a sum in flight instead of two 27 and 36).
 constexpr int kBinK = 4;
 // Per point four float4s: (g, -), (p, 1), g_rot, g_scale, at slot ^ (point / 4 % 4): reads of one slot at random points then
 // spread over all banks.
 __device__ __forceinline__ int bin_slot(int point, int slot) { return 4 * point + (slot ^ ((point >> 2) & 3)); }
-template <bool kNearest>
-__global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N, int M, int K, int S, int warp_mode,
+template <bool kNearest, bool kStaged>
+__global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N, int per, int M, int K, int S, int warp_mode,
     int weight_mode, float temperature, const float* __restrict__ points, const float* __restrict__ xf,
     const float* __restrict__ pair_in, const int64_t* __restrict__ index, const float* __restrict__ g_xyz,
     const float* __restrict__ g_rot, const float* __restrict__ g_scale, const float* __restrict__ sp_points,
@@ -209,15 +214,19 @@ __global__ void __launch_bounds__(kAccThreads) lbs_backward_binned_kernel(int N,
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int e = tid; e < cells; e += kAccThreads) s_tab[e] = 0.0f;
   const float inv_t = 1.0f / temperature;
-  for (int n0 = blockIdx.x * kAccThreads; n0 < N; n0 += gridDim.x * kAccThreads) {
+  for (int n0 = blockIdx.x * per; n0 < N; n0 += gridDim.x * per) {
     const int n = n0 + tid;
-    const bool live = n < N;
+    const bool live = tid < per && n < N;
     s_count[tid] = 0;
+    if (kStaged)
+      for (int e = tid; e < M * (kXf / 4); e += kAccThreads) s_feat[e] = ((const float4*) xf)[e];
     __syncthreads();
     LbsPoint<kBinK> P;
+    if (live)
+      lbs_point_backward<kBinK>(n, M, K, S, warp_mode, weight_mode, inv_t, points, kStaged ? (const float*) s_feat : xf, pair_in, index,
+                                g_xyz, g_rot, g_scale, g_points, g_pair, P);
+    if (kStaged) __syncthreads();
     if (live) {
-      lbs_point_backward<kBinK>(n, M, K, S, warp_mode, weight_mode, inv_t, points, xf, pair_in, index, g_xyz, g_rot, g_scale,
-                                g_points, g_pair, P);
       s_feat[bin_slot(tid, 0)] = make_float4(P.g[0], P.g[1], P.g[2], 0.0f);
       s_feat[bin_slot(tid, 1)] = make_float4(P.p[0], P.p[1], P.p[2], 1.0f);
       s_feat[bin_slot(tid, 2)] = make_float4(P.gr[0], P.gr[1], P.gr[2], P.gr[3]);
@@ -437,17 +446,17 @@ struct TablePlan {
   bool lds;
 };
 
-TablePlan plan_table(int N, int cells) {
+TablePlan plan_table(int N, int cells, int points = kAccThreads) {  // points: of a block, at least
   TablePlan p;
   p.lds    = cells <= kTableFloats;
-  p.blocks = std::max(1, std::min(div_up(N, kAccThreads), p.lds ? kMaxAccBlocks : 1024));
+  p.blocks = std::max(1, p.lds ? std::min(div_up(N, points), kMaxAccBlocks) : std::min(div_up(N, kAccThreads), 1024));
   return p;
 }
 
 bool lbs_binned(int M, int K, int cells) { return cells <= kStageTable && M <= kAccThreads && K <= kBinK; }
 
-size_t partial_bytes(int N, int cells) {
-  const TablePlan p = plan_table(N, cells);
+size_t partial_bytes(int N, int cells, int points = kAccThreads) {
+  const TablePlan p = plan_table(N, cells, points);
   return p.lds ? align_up((size_t) p.blocks * cells * 4, 256) : 256;
 }
 
@@ -459,7 +468,7 @@ using namespace fsgs;
 FSGS_API size_t fsgs_lbs_blend_backward_workspace_bytes(int N, int M, int S) {
   if (N < 0 || M <= 0 || S < 0 || S > 4) return 0;
   const int F = 21 + S;  // the widest row: rotation block, kernel-weight columns, the distances' gradient
-  return align_up((size_t) M * kXf * 4, 256) + align_up((size_t) M * F * 4, 256) + partial_bytes(N, M * F);
+  return align_up((size_t) M * kXf * 4, 256) + align_up((size_t) M * F * 4, 256) + partial_bytes(N, M * F, kAccPoints);
 }
 
 namespace {
@@ -488,7 +497,7 @@ int lbs_backward(int N, int M, int K, int warp_mode, int weight_mode, double tem
     return fail(kWorkspaceSmall, "lbs_blend_backward: workspace %zu < %zu bytes", workspace_bytes, need);
   const LbsCols C = lbs_cols(warp_mode, weight_mode, S);
   const int cells = M * (C.F + (nearest ? 3 : 0));
-  const TablePlan plan = plan_table(N, cells);
+  const TablePlan plan = plan_table(N, cells, lbs_binned(M, K, cells) ? kAccPoints : kAccThreads);
   const float* xf = table ? table : (const float*) workspace;
   float* acc     = (float*) ((char*) workspace + align_up((size_t) M * kXf * 4, 256));
   float* partial = (float*) ((char*) acc + align_up((size_t) M * (21 + S) * 4, 256));
@@ -503,8 +512,11 @@ int lbs_backward(int N, int M, int K, int warp_mode, int weight_mode, double tem
   if (N > 0) {
     if (plan.lds) {
       if (lbs_binned(M, K, cells)) {
-        auto kernel = nearest ? lbs_backward_binned_kernel<true> : lbs_backward_binned_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3(plan.blocks), dim3(kAccThreads), 0, s, N, M, K, S, warp_mode, weight_mode,
+        const bool staged = (size_t) M * kXf <= 16 * (size_t) kAccThreads;
+        auto kernel = nearest ? (staged ? lbs_backward_binned_kernel<true, true> : lbs_backward_binned_kernel<true, false>)
+                              : (staged ? lbs_backward_binned_kernel<false, true> : lbs_backward_binned_kernel<false, false>);
+        const int per = 64 * div_up(div_up(N, plan.blocks * div_up(N, plan.blocks * kAccThreads)), 64);  // points a block takes at a time
+        hipLaunchKernelGGL(kernel, dim3(plan.blocks), dim3(kAccThreads), 0, s, N, per, M, K, S, warp_mode, weight_mode,
                            (float) temperature, points, xf, pair_in, index, g_xyz, g_rot, g_scale, sp_points, g_points, g_pair,
                            partial);
       } else {

@@ -1162,3 +1162,14 @@ def test_simple_knn_mixed_density_large(device):
         best = d2.topk(4, dim=1, largest=False).values[:, 1:]
         want = best.mean(1)
         assert float(((want - got[part]).abs() / want.clamp_min(1e-30)).max()) <= 1e-5
+
+
+# binned sums: the last table of transforms that passes through LDS and the first that does not (585 and 586 control points, where the
+# widest rows that are binned allow them), points around a block's share, around what all blocks take at once, and what is left over
+@pytest.mark.parametrize('N,M', [(1, 585), (511, 586), (513, 585), (1025, 586), (131_073, 512), (131_071, 500), (262_145, 512)])
+@pytest.mark.parametrize('warp_method,weight_method', [(None, 'kernel'), ('LBS_c', 'dist')])
+def test_lbs_backward_shares(N, M, warp_method, weight_method, device, oracle_mod):
+    g = torch.Generator().manual_seed(N + M)
+    pts, ctrl = torch.rand(N, 3, generator=g) * 2 - 1, torch.rand(M, 3, generator=g) * 2 - 1
+    _lbs_backward_case(device, pts, ctrl, 0.1 * torch.randn(M, 3, generator=g), 0.2 * torch.randn(M, 4, generator=g),
+                       0.1 * torch.randn(M, 2, generator=g), 4, warp_method, weight_method, seed=N % 97)
