@@ -47,6 +47,7 @@ class DynamicStep:
         # the reference's training render passes `accum_max_count` on every step (network.py:706): per Gaussian, the
         # number of (pixel, blended entry) events at which it was the pixel's strongest contributor so far
         self.accum_max_count = torch.zeros(self.params[0].shape[0], dtype=torch.int32, device=dev)
+        self._one = torch.ones((), device=dev)  # the loss's own gradient, which backward() would fill a new tensor with each time
 
     def forward_loss(self, t: Tensor):
         """-> (loss, render outputs). Differentiable in the Gaussians' parameters, the control points and the network."""
@@ -72,7 +73,7 @@ class DynamicStep:
     def step(self, t: Tensor):
         """One full iteration; returns (loss, visibility mask) as device tensors (nothing is copied to the host)."""
         loss, out = self.forward_loss(t)
-        loss.backward()
+        loss.backward(self._one)
         visible = out['visibility_filter']
         self.opt.set_before_step(visible, self.params[0].shape[0])
         self.opt.step()
