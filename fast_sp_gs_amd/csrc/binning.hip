@@ -648,12 +648,12 @@ __global__ void __launch_bounds__(1024) tile_prefix_scan_kernel(int T, int B, ui
 template <bool kPad>
 __device__ __forceinline__ int lds_slot(int i) { return kPad ? i + (i >> 2) : i; }
 
-template <bool kPad>
+template <bool kPad, typename Number>
 __device__ __forceinline__ void tile_sort_output(int tile, int64_t start, int n, const uint64_t* sorted_local,
-                                                 int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
+                                                 Number* __restrict__ point_list, int64_t* __restrict__ keys_out) {
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     const uint64_t e = sorted_local[lds_slot<kPad>(k)];
-    point_list[start + k] = (int32_t) (uint32_t) e;
+    point_list[start + k] = (Number) (uint32_t) e;
     if (keys_out) keys_out[start + k] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
   }
 }
@@ -901,9 +901,9 @@ __device__ __forceinline__ unsigned prefix_counters(unsigned* s_count, unsigned*
 // buckets costs segments without one about 2 us of the 116.) False, with nothing written and the keys in `key`, when that leaves too
 // many together as well (numbers in clumps, half a bucket at one depth): the comparing sorts take such a segment.
 // load(i): entry i, from memory, or, kHeld, from s_e itself.
-template <int kPer, bool kHeld, typename Load>
+template <int kPer, bool kHeld, typename Load, typename Number>
 __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, Load load, uint64_t (&key)[kPer], uint64_t* s_e,
-                                            int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
+                                            Number* __restrict__ point_list, int64_t* __restrict__ keys_out) {
   constexpr int kBuckets = kPer == 1 ? kSortBuckets / 2 : kSortBuckets, kOwn = kBuckets / 256;
   unsigned* s_count = (unsigned*) (s_e + kSmallSegment);
   unsigned* s_wave  = (unsigned*) s_e;  // before the entries come
@@ -928,7 +928,7 @@ __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, Load
   auto emit   = [&](uint64_t e, int first, int end) {
     int to = first;
     for (int i = first; i < end; ++i) to += s_e[i] < e;
-    point_list[start + to] = (int32_t) (uint32_t) e;
+    point_list[start + to] = (Number) (uint32_t) e;
     if (keys_out) keys_out[start + to] = (int64_t) (((uint64_t) (uint32_t) tile << 32) | (e >> 32));
   };
   unsigned rank[kPer];
@@ -1015,9 +1015,9 @@ __device__ __forceinline__ bool bucket_sort(int tile, int64_t start, int n, Load
 }
 
 // n <= kSmallSegment entries (see bucket_sort for load and kHeld), by as many a lane as they need; s_e holds kSmallSegment + kSmallSegment / 4.
-template <bool kHeld, typename Load>
+template <bool kHeld, typename Load, typename Number>
 __device__ __forceinline__ void sort_small_segment(int tile, int64_t start, int n, Load load, uint64_t* s_e,
-                                                   int32_t* __restrict__ point_list, int64_t* __restrict__ keys_out) {
+                                                   Number* __restrict__ point_list, int64_t* __restrict__ keys_out) {
   auto sort = [&](auto per) {  // entries per lane
     constexpr int kPer = decltype(per)::value;
     uint64_t key[kPer];
@@ -1258,13 +1258,17 @@ __global__ void __launch_bounds__(1024) tile_sort_large_kernel(const int64_t* __
 // The work grows with surfels times tiles, but the others' prefix is one block's up to 1024 tiles. Views, us, so binned -> gathered:
 // 5k surfels 640x480 (1200 tiles) 50 -> 42.5, 20k 54.5 -> 51.7, 25k 800x600 (1900, 47.5M looks) 62.2 -> 62.3, 30k Gaussians
 // 800x600 (57M) 54.9 -> 56.3; 1024 tiles and fewer: 65k surfels 500x500 90 -> 82, 440x440 91 -> 85, 65k Gaussians 440x440 85 -> 80, one
-// surfel 47 -> 44. With long lists: 8000 surfels 256x256, 1220 entries a tile, 255 -> 235, 40k 160x160, up to 2961, 294 -> 241.
+// surfel 47 -> 44. With many surfels on few tiles those are few blocks, their lists are long, and what is longer than 2048 entries is
+// looked for twice: 49 tiles 10k surfels 97.5 -> 93.4, 20k 162 -> 171, 40k 195 -> 228; 100 tiles 20k 91 -> 86, 40k 154 -> 178; 256 tiles
+// 40k 91 -> 89, 65k 121 -> 125. Large surfels, up to that line: 8000 surfels 256x256, 1220 entries a tile, 255 -> 235; 60k
+// 400x400, 1585 a tile and up to 5381, 470 -> 458.
 constexpr int kGatherSide  = 127;    // tiles along either axis: a rectangle is four numbers of seven bits
 constexpr int kGatherTiles = 2040;   // two a lane in the second launch, and eight a block: 255 blocks, and one for the schedule
 constexpr int kGatherChunk = 16 * kWave;  // surfels that a wavefront looks at in one go
 constexpr int kGatherHeld  = 2 * kGatherChunk;  // of them, what a wavefront can hold
 constexpr int kGatherMost  = 65535;  // surfels: their numbers are held in 16 bits
 constexpr int64_t kGatherLooks = 48000000;  // surfels times tiles, above 1024 tiles (see above)
+constexpr int kGatherPerTile   = 200;       // surfels per tile (see above)
 
 // Bytes of a rectangle's word: first column, 127 - last column, first row, 127 - last row. gather_word(tx, ty) less it has the upper
 // bit of a byte set where the tile is on the rectangle's side of that bound.
@@ -1297,7 +1301,7 @@ __device__ __forceinline__ int gather_place(bool on, int* at) {
 }
 
 __global__ void __launch_bounds__(256) tile_gather_kernel(int P, int gx, const uint32_t* __restrict__ rects,
-    const uint32_t* __restrict__ masks, const float* __restrict__ depths, uint32_t* __restrict__ counts, int32_t* __restrict__ lists,
+    const uint32_t* __restrict__ masks, const float* __restrict__ depths, uint32_t* __restrict__ counts, uint16_t* __restrict__ lists,
     SlotPublish publish) {
   constexpr int kWaves = 256 / kWave, kQuads = kGatherChunk / (4 * kWave);  // quads: of four words a lane
   __shared__ __align__(16) uint64_t s_e[kSmallSegment + kSmallSegment / 4];
@@ -1375,7 +1379,7 @@ constexpr int kPlaceBlocks = 255;
 template <int kTiles>
 __global__ void __launch_bounds__(1024) tile_place_kernel(int P, int gx, int gy, int64_t R, const uint32_t* __restrict__ rects,
     const uint32_t* __restrict__ masks, const float* __restrict__ depths, const uint32_t* __restrict__ counts,
-    const int32_t* __restrict__ lists, int64_t* __restrict__ ranges, int32_t* __restrict__ point_list, uint64_t* __restrict__ entries,
+    const uint16_t* __restrict__ lists, int64_t* __restrict__ ranges, int32_t* __restrict__ point_list, uint64_t* __restrict__ entries,
     int* __restrict__ order_table) {
   __shared__ LargeSortLds s;
   constexpr int kLanes = 1024 / kTiles;
@@ -1390,7 +1394,7 @@ __global__ void __launch_bounds__(1024) tile_place_kernel(int P, int gx, int gy,
   const int t0 = 2 * (int) threadIdx.x, low = t0 < T ? (int) counts[t0] : 0, mine = low + (t0 + 1 < T ? (int) counts[t0 + 1] : 0);
   const int block = (int) blockIdx.x - (order_table ? 1 : 0), own = kTiles * block + (int) threadIdx.x / kLanes;  // this lane's tile
   const int k0 = threadIdx.x % kLanes;
-  const int32_t* list = lists + (size_t) min(own, T - 1) * kSmallSegment;
+  const uint16_t* list = lists + (size_t) min(own, T - 1) * kSmallSegment;
   const int32_t ahead[2] = {list[k0], list[k0 + kLanes]};  // whatever they are: on their way with the counts
   const int inc  = wave_scan(mine);
   if (lane == kWave - 1) s.wave[wave] = (unsigned) inc;
@@ -2031,7 +2035,7 @@ struct GatherLayout {
 GatherLayout gather_layout(int T) {
   GatherLayout l;
   l.lists = align_up((size_t) T * sizeof(uint32_t), 256);
-  l.bytes = l.lists + (size_t) T * kSmallSegment * sizeof(int32_t);
+  l.bytes = l.lists + (size_t) T * kSmallSegment * sizeof(uint16_t);
   return l;
 }
 }  // namespace
@@ -2039,7 +2043,7 @@ GatherLayout gather_layout(int T) {
 FSGS_API int fsgs_gs_view_gathers(int P, int W, int H) {
   const int gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
   return P > 0 && P <= kGatherMost && gx > 0 && gy > 0 && gx <= kGatherSide && gy <= kGatherSide && gx * gy <= kGatherTiles &&
-         (gx * gy <= 1024 || (int64_t) P * gx * gy <= kGatherLooks);
+         P <= kGatherPerTile * gx * gy && (gx * gy <= 1024 || (int64_t) P * gx * gy <= kGatherLooks);
 }
 
 FSGS_API size_t fsgs_gs_view_gather_bytes(int W, int H) {
@@ -2059,7 +2063,7 @@ FSGS_API int fsgs_gs_view_gather(int P, int W, int H, const float* depths, const
   if (num_rendered_host) __atomic_store_n(num_rendered_host, (int64_t) -1, __ATOMIC_RELEASE);
   hipLaunchKernelGGL(tile_gather_kernel, dim3(gx * gy), dim3(256), 0, (hipStream_t) stream, P, gx, tile_rects,
                      culling_enabled() ? keep_masks : nullptr, depths, (uint32_t*) lists,
-                     (int32_t*) ((char*) lists + gather_layout(gx * gy).lists),
+                     (uint16_t*) ((char*) lists + gather_layout(gx * gy).lists),
                      SlotPublish{(unsigned long long*) slot_counters, slot_regions, num_rendered_host});
   return check_launch("gs_view_gather");
 }
@@ -2085,7 +2089,7 @@ FSGS_API int fsgs_gs_view_place(int P, int W, int H, const float* depths, const 
   auto kernel = tiles == 1 ? tile_place_kernel<1> : tiles == 2 ? tile_place_kernel<2> : tiles == 4 ? tile_place_kernel<4> : tile_place_kernel<8>;
   hipLaunchKernelGGL(kernel, dim3(div_up(gx * gy, tiles) + (build ? 1 : 0)), dim3(1024), 0, s, P, gx, gy, R, tile_rects,
                      culling_enabled() ? keep_masks : nullptr, depths, (const uint32_t*) lists,
-                     (const int32_t*) ((const char*) lists + gather_layout(gx * gy).lists), ranges, point_list, (uint64_t*) workspace, build);
+                     (const uint16_t*) ((const char*) lists + gather_layout(gx * gy).lists), ranges, point_list, (uint64_t*) workspace, build);
   return check_launch("gs_view_place");
 }
 

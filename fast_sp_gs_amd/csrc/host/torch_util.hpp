@@ -180,7 +180,7 @@ Instances scatter_instances(const char* what, PendingCount& pending, int64_t gue
 }
 
 // A view's scratch. A small view (fsgs_gs_view_gathers) has its lists gathered tile by tile, by way of `rects` and `lists`, the others
-// are binned by way of `bins`, and so is a small one for whose lists (8 KB a tile) there is no memory.
+// are binned by way of `bins`, and so is a small one for whose lists (4 KB a tile) there is no memory.
 struct ViewScratch {
   bool small = false;
   size_t depths = 0, masks = 0, bins = 0, bins_bytes = 0, rects = 0, lists = 0, lists_bytes = 0;

@@ -192,8 +192,8 @@ int fsgs_gs_view_sort(int P, int W, int H, const float* means2D, const float* in
                       int64_t* ranges, int32_t* point_list, void* bins, size_t bins_bytes, void* workspace,
                       size_t workspace_bytes, void* stream);
 
-/* The same binning for a small view of surfels or 3D Gaussians (fsgs_gs_view_gathers: at most 65 535 of them and 1024 tiles, and not too
- * many of both), in two parts: fsgs_gs_view_gather takes the place of fsgs_gs_view_count (slot_regions, slot_counters and
+/* The same binning for a small view of surfels or 3D Gaussians (fsgs_gs_view_gathers: at most 65 535 of them, 200 a tile
+ * and 2040 tiles, above 1024 tiles not too many of both), in two parts: fsgs_gs_view_gather takes the place of fsgs_gs_view_count (slot_regions, slot_counters and
  * num_rendered_host, here optional, as there) and leaves every tile's list in `lists` (fsgs_gs_view_gather_bytes bytes);
  * fsgs_gs_view_place, with the count R, puts them into point_list[R] and writes ranges. tile_rects (on a 16-byte boundary) and depths
  * are the preprocess kernels', keep_masks (optional) too; workspace: 8 R bytes. */

@@ -58,7 +58,7 @@ def _gather(rects, masks, depths, gx, gy, R, device):
 # numbers of surfels around a quad of words, a go of a wavefront and of a block, two of a block and the most; grids of one tile, one row
 # or column as long as a word's bounds allow, and around the tiles per block of the second launch
 @pytest.mark.parametrize('P,gx,gy', [(1, 1, 1), (3, 1, 127), (255, 127, 1), (256, 15, 17), (257, 16, 16), (1023, 30, 17), (1025, 73, 7),
-                                     (4095, 32, 32), (4097, 20, 51), (8193, 1021, 1), (5000, 40, 51), (2049, 127, 16), (65_535, 7, 5)])
+                                     (4095, 32, 32), (4097, 20, 51), (8193, 1021, 1), (5000, 40, 51), (2049, 127, 16), (65_535, 19, 18)])
 @pytest.mark.parametrize('masked', [False, True])
 def test_lists_from_rectangles(P, gx, gy, masked, device):
     print(f'[small view] P={P} {gx}x{gy} masked={masked}', flush=True)
@@ -84,7 +84,8 @@ def test_lists_from_rectangles(P, gx, gy, masked, device):
 
 
 # lists that their own blocks cannot sort: around 2048 entries, above 4096, 8192 and 16 384, beside short ones
-@pytest.mark.parametrize('P,gx,gy', [(2048, 2, 1), (2049, 1, 1), (2500, 16, 16), (5000, 3, 2), (9000, 30, 40), (17_000, 2, 2), (65_535, 1, 1)])
+@pytest.mark.parametrize('P,gx,gy', [(2048, 11, 1), (2049, 1, 11), (2500, 16, 16), (5000, 5, 5), (9000, 30, 40), (17_000, 10, 9), (20_000, 25, 30),
+                                     (65_535, 20, 20)])
 @pytest.mark.parametrize('one_depth', [False, True])
 def test_long_lists(P, gx, gy, one_depth, device):
     print(f'[small view] long lists P={P} {gx}x{gy} one_depth={one_depth}', flush=True)
@@ -93,8 +94,8 @@ def test_long_lists(P, gx, gy, one_depth, device):
     rects = np.stack([tx, ty, tx + 1, ty + 1], 1)
     rects[g.random(P) < 0.97] = (gx // 2, gy // 2, gx // 2 + 1, gy // 2 + 1)  # nearly all in one tile, that and its neighbour
     rects[::2, 2] = np.minimum(gx, rects[::2, 2] + 1)
-    if gx == 2 and gy == 1:
-        rects[:] = (0, 0, 2, 1)
+    if P == 2048:  # as long as a block sorts, twice
+        rects[:] = (3, 0, 5, 1)
     depths = np.full(P, 7.5, np.float32) if one_depth else g.random(P).astype(np.float32) + 0.2
     want, ranges = _host_lists(rects, None, depths, gx, gy)
     got, got_ranges = _gather(rects, None, depths, gx, gy, len(want), device)
@@ -103,7 +104,8 @@ def test_long_lists(P, gx, gy, one_depth, device):
 
 # the last sizes that are gathered and the first that are not: by tiles, by numbers, by both
 @pytest.mark.parametrize('gx,gy,P,small', [(40, 51, 900, True), (41, 50, 900, False), (127, 3, 500, True), (128, 3, 500, False),
-                                           (32, 32, 65_535, True), (32, 32, 65_536, False), (41, 25, 46_829, True), (41, 25, 46_830, False)])
+                                           (32, 32, 65_535, True), (32, 32, 65_536, False), (41, 25, 46_829, True), (41, 25, 46_830, False),
+                                           (5, 7, 7000, True), (5, 7, 7001, False)])
 @pytest.mark.parametrize('cull', [False, True])
 def test_views_at_the_limits(gx, gy, P, small, cull, device, monkeypatch):
     from fast_sp_gs_amd import lib as L, scenes
