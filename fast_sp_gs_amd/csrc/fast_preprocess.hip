@@ -100,6 +100,8 @@ __device__ __forceinline__ void fast_transmat_backward(float sx, float sy, const
 // kRow: floats of a row that each wavefront moves on its own (sh_stage.hpp), 45 with the first coefficient apart; 0: none
 constexpr int kCoopThreshold = 32;  // rectangles with more tiles are walked (and corner-tested) by a whole wavefront
 
+// The rows reach the lanes' registers through LDS for 32 of them, four blocks to a compute unit instead of three: 300k surfels 800x800
+// 33 -> 30 us, 150k 1001x667 18.5 -> 17.6, 30k 500x400 12.7 -> 11.9.
 template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
@@ -111,8 +113,9 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
     int32_t* __restrict__ radii, int32_t* __restrict__ tiles_touched, uint32_t* __restrict__ keep_masks,
     ViewOutputs view) {
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
-  constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
-  __shared__ __align__(16) float s_rows[kWave ? kShStageRows * kStride : 1];
+  constexpr int kWaveFloats = ShWaveRows<kWave ? kRow : 48>::kHalfFloats;
+  static_assert(kWaveFloats >= 64 * 21, "what a wavefront writes passes through the same LDS");
+  __shared__ __align__(16) float s_rows[kWave ? 4 * kWaveFloats : 1];
   const int i0     = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i0 < P;
   __shared__ int s_wave_slots[4];
@@ -132,7 +135,7 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
   for (int k = 0; k < 9; ++k) M[k] = 0.0f;
   const float p[3] = {means3D[3 * (size_t) i], means3D[3 * (size_t) i + 1], means3D[3 * (size_t) i + 2]};
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveFloats : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
   float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
@@ -222,22 +225,25 @@ __global__ void __launch_bounds__(256) fast_preprocess_forward_kernel(
       }
     }
   }
-  if (kWave) {
-    if (wanted) sh_regs.to_lds(s_wave_rows, wave_base, P);
-    wave_lds_sync();
+  float own[kWave ? kRow : 1];
+  if constexpr (kWave) {
+    if (wanted) sh_regs.to_lanes(own, s_wave_rows, wave_base, P);
   }
   if (ok && sh_degree >= 0) {
-    float x, y, z, Y[kSh];
+    float x, y, z;
     view_dir(p, campos, x, y, z);
-    sh_eval(sh_degree, x, y, z, Y);
-    const int n = sh_count(sh_degree);
-    const float* row = &s_rows[kWave ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
-    const float* c0 = kWave ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
-    float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
-    const float* cr = kWave ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-    for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
-    rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
-    if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
+    if constexpr (kWave) {
+      sh_lane_colors(own, dc, sh_degree, x, y, z, view.color_derivs != nullptr, rgb, derivs);
+    } else {
+      float Y[kSh];
+      sh_eval(sh_degree, x, y, z, Y);
+      const int n = sh_count(sh_degree);
+      const float* c0 = shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
+      const float* cr = sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0;  // coefficient l at 3 l
+      float r = c0[0] * Y[0], g = c0[1] * Y[0], b = c0[2] * Y[0];
+      for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
+      rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+    }
   }
   if (view.slot_offsets) {
     if (threadIdx.x == 0) s_block_slot = (int) block_slot;
@@ -352,7 +358,7 @@ __global__ void __launch_bounds__(256) fast_duplicate_keys_kernel(int P, int gx,
 }
 
 // kDerivs: from the colours' derivatives that the forward left, without the rows of coefficients (as the surfels'). 150k surfels
-// 1001x667: 16.4 -> 12.6 us, the forward 17.3 -> 18.4.
+// 1001x667: 16.4 -> 12.6 us, the forward 17.3 -> 18.4 (17.6 since its rows take half of the LDS).
 template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) fast_preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,

@@ -249,6 +249,8 @@ __device__ __forceinline__ bool screen_geometry(int W, int H, int gx, int gy, bo
 }
 
 // kRow: floats of a row that each wavefront moves on its own (sh_stage.hpp), 45 with the first coefficient apart; 0: none
+// The rows reach the lanes' registers through LDS for 32 of them, four blocks to a compute unit instead of three: 300k Gaussians 800x800
+// 30.1 -> 27.4 us, 100k 640x480 16.0 -> 15.0, 25k 639x361 without a backward 13.6 -> 13.0.
 template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int W, int H, int sh_degree, int n_sh,
     int is_opengl, const float* __restrict__ means3D, const float* __restrict__ scales,
@@ -262,10 +264,12 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;
+  constexpr int kWaveFloats = kWave ? ShWaveRows<kWave ? kRow : 48>::kHalfFloats : 64 * kStride;
+  static_assert(!kWave || kWaveFloats >= 64 * 9, "what a wavefront writes passes through the same LDS");
   __shared__ int s_wave_slots[4];
   __shared__ float s_Tw2v[16], s_Tv2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
-  __shared__ unsigned char s_flag[kShStageRows];
+  __shared__ __align__(16) float s_rows[kStage ? 4 * kWaveFloats : 1];
+  __shared__ unsigned char s_flag[kWave ? 1 : kShStageRows];
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < P;
   // the Gaussian's own values are on their way while the block waits for the camera
@@ -289,7 +293,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   float c3[6] = {0, 0, 0, 0, 0, 0}, rgb[3] = {0, 0, 0};
   Screen sc = {};
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveFloats : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
   float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
@@ -343,9 +347,9 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
   }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
-    if (kWave) {
-      if (wanted) sh_regs.to_lds(s_wave_rows, wave_base, P);
-      wave_lds_sync();
+    float own[kWave ? kRow : 1];
+    if constexpr (kWave) {
+      if (wanted) sh_regs.to_lanes(own, s_wave_rows, wave_base, P);
     } else if (kStage) {
       s_flag[threadIdx.x] = ok;
       __syncthreads();
@@ -353,16 +357,20 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
       __syncthreads();
     }
     if (ok) {
-      float x, y, z, Y[kSh];
+      float x, y, z;
       view_dir(p, campos, x, y, z);
-      sh_eval(sh_degree, x, y, z, Y);
-      const float* row = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
-      const float* c0 = kStage ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
-      const float* cr = kStage ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
-      for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
-      rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
-      if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
+      if constexpr (kWave) {
+        sh_lane_colors(own, dc, sh_degree, x, y, z, view.color_derivs != nullptr, rgb, derivs);
+      } else {
+        float Y[kSh];
+        sh_eval(sh_degree, x, y, z, Y);
+        const float* row = &s_rows[kStage ? threadIdx.x * kStride : 0];  // coefficient l at 3 l
+        const float* c0 = kStage ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
+        const float* cr = kStage ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
+        float r = c0[0] * Y[0], g = c0[1] * Y[0], b = c0[2] * Y[0];
+        for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
+        rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+      }
     }
   }
   SlotSums sums;
@@ -403,7 +411,7 @@ __global__ void __launch_bounds__(256) gs3d_preprocess_forward_kernel(int P, int
 }
 
 // kDerivs: from the colours' derivatives that the forward left, without the rows of coefficients (as the surfels'). 300k Gaussians
-// 800x800: 32 -> 22 us, the forward 27.6 -> 30.5.
+// 800x800: 32 -> 22 us, the forward 27.6 -> 30.5 (27.4 since its rows take half of the LDS).
 template <int kSh, int kRow, bool kDerivs>
 __global__ void __launch_bounds__(256) gs3d_preprocess_backward_kernel(int P, int W, int H, int sh_degree, int n_sh,
     int is_opengl, const float* __restrict__ means3D, const float* __restrict__ scales,

@@ -84,6 +84,10 @@ __device__ __forceinline__ void transmat(int W, int H, const float* p, float sx,
 }
 
 // kRow: floats of a row that each wavefront moves on its own (sh_stage.hpp), 45 with the first coefficient apart; 0: none
+// Bound by a chain of trips to memory for few surfels and by 440 bytes a surfel for many, both of which want more wavefronts in
+// flight. The rows reach the lanes' registers through LDS for 32 of them (to_lanes), four blocks to a compute unit; with room for 64 it
+// was three. Training, us: 3M 1352x1014 220 -> 207, 300k 800x800 36 -> 33, 200k 29 -> 22.5, 10k 256x256 12.0 -> 11.2; 400k 3840x2160
+// without a backward 52 -> 47.
 template <int kSh, int kRow>
 __global__ void __launch_bounds__(256) preprocess_forward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
@@ -97,9 +101,11 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   constexpr bool kWave = kRow != 0, kSplit = kRow == 45;
   constexpr int kStride = kWave ? kRow | 1 : kShStageStride;
   constexpr bool kStage = kSh == 16;  // degree <= 3: SH rows travel through LDS, read from HBM line by line
+  constexpr int kWaveFloats = kWave ? ShWaveRows<kWave ? kRow : 48>::kHalfFloats : 64 * kStride;
+  static_assert(!kWave || kWaveFloats >= 64 * 20, "a wavefront's records pass through the same LDS");
   __shared__ float s_Tw2v[16], s_Tw2c[16];
-  __shared__ __align__(16) float s_rows[kStage ? kShStageRows * kStride : 1];
-  __shared__ unsigned char s_flag[kShStageRows];
+  __shared__ __align__(16) float s_rows[kStage ? 4 * kWaveFloats : 1];
+  __shared__ unsigned char s_flag[kWave ? 1 : kShStageRows];
   __shared__ int s_wave_slots[4];
   __shared__ int s_block_slot;
   const int i      = blockIdx.x * blockDim.x + threadIdx.x;
@@ -122,7 +128,7 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
 #pragma unroll
   for (int k = 0; k < 9; ++k) M[k] = 0.0f;
   const int wave_base = blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x & ~63) * kStride : 0];
+  float* s_wave_rows  = &s_rows[kWave ? (threadIdx.x >> 6) * kWaveFloats : 0];
   ShWaveRows<kWave ? kRow : 48> sh_regs;
   unsigned long long wanted = 0;
   float dc[3] = {0, 0, 0}, derivs[kColorDerivs] = {};
@@ -173,9 +179,9 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
   }
   if (sh_degree >= 0) {
     const int n = sh_count(sh_degree);
-    if (kWave) {
-      if (wanted) sh_regs.to_lds(s_wave_rows, wave_base, P);
-      wave_lds_sync();
+    float own[kWave ? kRow : 1];
+    if constexpr (kWave) {
+      if (wanted) sh_regs.to_lanes(own, s_wave_rows, wave_base, P);
     } else if (kStage) {
       s_flag[threadIdx.x] = ok;
       __syncthreads();
@@ -183,16 +189,20 @@ __global__ void __launch_bounds__(256) preprocess_forward_kernel(
       __syncthreads();
     }
     if (ok) {
-      float x, y, z, Y[kSh];
+      float x, y, z;
       view_dir(p, campos, x, y, z);
-      sh_eval(sh_degree, x, y, z, Y);
-      const float* row = &s_rows[kStage ? threadIdx.x * kStride : 0] - (kSplit ? 3 : 0);  // coefficient l at 3 l
-      const float* c0 = kStage ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
-      const float* cr = kStage ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
-      float r = (kSplit ? dc[0] : c0[0]) * Y[0], g = (kSplit ? dc[1] : c0[1]) * Y[0], b = (kSplit ? dc[2] : c0[2]) * Y[0];
-      for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
-      rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
-      if (kWave && view.color_derivs) sh_color_derivatives(sh_degree, x, y, z, [&](int l, int c) { return cr[3 * l + c]; }, derivs);
+      if constexpr (kWave) {
+        sh_lane_colors(own, dc, sh_degree, x, y, z, view.color_derivs != nullptr, rgb, derivs);
+      } else {
+        float Y[kSh];
+        sh_eval(sh_degree, x, y, z, Y);
+        const float* row = &s_rows[kStage ? threadIdx.x * kStride : 0];  // coefficient l at 3 l
+        const float* c0 = kStage ? row : shs + (size_t) i * (sh_rest ? 1 : n_sh) * 3;
+        const float* cr = kStage ? row : (sh_rest ? sh_rest + (size_t) i * n_sh * 3 - 3 : c0);
+        float r = c0[0] * Y[0], g = c0[1] * Y[0], b = c0[2] * Y[0];
+        for (int l = 1; l < n; ++l) r += cr[3 * l] * Y[l], g += cr[3 * l + 1] * Y[l], b += cr[3 * l + 2] * Y[l];
+        rgb[0] = fmaxf(0.0f, r + 0.5f), rgb[1] = fmaxf(0.0f, g + 0.5f), rgb[2] = fmaxf(0.0f, b + 0.5f);
+      }
     }
   }
   SlotSums sums;
@@ -438,8 +448,8 @@ __device__ __forceinline__ void wave_record_sums(const ViewRecords& in, int firs
 // kDerivs: the forward left the colours' derivatives (36 bytes a surfel), and the rows of coefficients (192 bytes) are not read again. Bound
 // by memory at 3M surfels (about 1.4 GB at 5.2 TB/s); with fewer, by the trips to the records. Kernel, us, 3M 1352x1014 / 300k 800x800 /
 // 10k 256x256: 331 / 47 / 11.3 with the coefficients, 302 / 41 / 10.4 with the derivatives and LDS for 64 rows a wavefront (three of
-// them per SIMD), 266 / 40 / 9.6 with half of the rows at a time (sh_products_to_global: four). For that the forward takes 217, 36 and
-// 10.5 instead of 198, 33 and 9.7.
+// them per SIMD), 266 / 40 / 9.6 with half of the rows at a time (sh_products_to_global: four). For that the forward took 217, 36 and
+// 10.5 instead of 198, 33 and 9.7, with room in LDS for 64 rows a wavefront on both sides.
 template <int kSh, int kRow, bool kRecords, bool kDerivs>
 __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     int P, int W, int H, int sh_degree, int n_sh, const float* __restrict__ means3D, const float2* __restrict__ scales,
