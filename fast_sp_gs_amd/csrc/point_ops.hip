@@ -32,7 +32,9 @@ namespace {
 // kDerivs: the derivatives of the colours by the direction (36 bytes a point) are left for the backward, which then reads them instead of
 // the coefficients (192). Both kernels are bound by what they move. Forward + backward, us, with the coefficients read again -> with the
 // derivatives: 20k points 4.2 + 6.4 -> 4.7 + 4.9; 150k 7.9 + 10.4 -> 9.4 + 8.8; 400k 16.4 + 33 -> 19.9 + 20.5; 1M 33.2 + 76 ->
-// 41.6 + 44 (252 MB and 276 MB: 6.1 and 6.3 TB/s); 3M 119 + 239 -> 128 + 148.
+// 41.6 + 44 (252 MB and 276 MB: 6.1 and 6.3 TB/s); 3M 119 + 239 -> 128 + 148. The forward since a wavefront's rows of 48 floats take
+// the LDS of half of them (to_lanes; five blocks to a compute unit instead of three): 20k 4.8 -> 4.3, 150k 9.5 -> 8.5, 200k 12.9 -> 10.6,
+// 1M 41.8 -> 39.9, 3M 123 -> 120.
 // Coefficients that are read once in a pass are worth nothing in the memory-side cache (256 MB), but stay there from pass to pass where they
 // fit beside the rest: by ordinary and by streaming loads 400k (77 MB) 40.4 and 41.0, 700k (134 MB) 61.7 and 62.4, 1M (192 MB) 93.3 and
 // 85.6, 3M 287 and 276.
@@ -45,17 +47,24 @@ __global__ void __launch_bounds__(256) sh_to_rgb_forward_kernel(int P, int F, in
   using Rows            = ShWaveRows<kRows ? kRow : 48>;
   constexpr int kStride = Rows::kStride;
   static_assert(!kDerivs || kRow == 48);
-  __shared__ __align__(16) float s_rows[kRows ? 4 * kWave * kStride : 1];
+  constexpr bool kLanes     = kRow == 48;
+  constexpr int kWaveFloats = kLanes ? Rows::kHalfFloats : kWave * kStride;
+  __shared__ __align__(16) float s_rows[kRows ? 4 * kWaveFloats : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int wave_base = (int) (blockIdx.x * blockDim.x + (threadIdx.x & ~63));
-  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWave * kStride : 0);
+  float* my_rows = s_rows + (kRows ? (threadIdx.x >> 6) * kWaveFloats : 0);
+  float own[kLanes ? kRow : 1];
   if (kRows) {
     const unsigned long long live = __ballot(i < P);
     if (live != 0ull) {
       Rows regs;
       regs.fetch(live, wave_base, P, sh, kDerivs && (size_t) P * kRow * 4 >= kStreamCoefficients);
-      regs.to_lds(my_rows, wave_base, P);
-      wave_lds_sync();
+      if constexpr (kLanes) {
+        regs.to_lanes(own, my_rows, wave_base, P);
+      } else {
+        regs.to_lds(my_rows, wave_base, P);
+        wave_lds_sync();
+      }
     }
   }
   float j[kColorDerivs] = {};
@@ -68,9 +77,14 @@ __global__ void __launch_bounds__(256) sh_to_rgb_forward_kernel(int P, int F, in
     float Y[kSh];
     sh_eval(degree, x, y, z, Y);
     const int n    = sh_count(degree);
-    const float* c = kRows ? my_rows + (threadIdx.x & 63) * kStride : sh + (size_t) i * F * 3;
+    const float* c = kLanes ? own : kRows ? my_rows + (threadIdx.x & 63) * kStride : sh + (size_t) i * F * 3;
     float r = c[0] * Y[0], g = c[1] * Y[0], b = c[2] * Y[0];
-    for (int l = 1; l < n; ++l) r += c[3 * l] * Y[l], g += c[3 * l + 1] * Y[l], b += c[3 * l + 2] * Y[l];
+    if constexpr (kLanes) {
+#pragma unroll
+      for (int l = 1; l < 16; ++l) r = fmaf(own[3 * l], Y[l], r), g = fmaf(own[3 * l + 1], Y[l], g), b = fmaf(own[3 * l + 2], Y[l], b);
+    } else {
+      for (int l = 1; l < n; ++l) r += c[3 * l] * Y[l], g += c[3 * l + 1] * Y[l], b += c[3 * l + 2] * Y[l];
+    }
     r += 0.5f, g += 0.5f, b += 0.5f;
     if (clamp) r = fmaxf(0.0f, r), g = fmaxf(0.0f, g), b = fmaxf(0.0f, b);
     rgb[3 * (size_t) i] = r, rgb[3 * (size_t) i + 1] = g, rgb[3 * (size_t) i + 2] = b;

@@ -57,3 +57,18 @@ def test_colors(P, path, split, device):
         # sixteen terms of at most 2.9 |c| a summand: each is formed and added with a rounding, its direction and basis with some ten more
         bound = 26 * 2.0 ** -24 * ((Y.abs() + 1.0)[:, :, None] * sh.double().abs()).sum(1) + 2.0 ** -23
         assert ((colors.double() - want.clamp_min(0)).abs() <= bound)[seen].all(), name
+
+
+@pytest.mark.parametrize('P', [1, 31, 32, 33, 63, 65, 97, 255, 289])
+@pytest.mark.parametrize('grad', [False, True])
+def test_sh_to_rgb(P, grad, device):
+    from fast_sp_gs_amd.ops import SH_to_RGB
+    print(f'[half rows] SH_to_RGB P={P} grad={grad}', flush=True)
+    g = torch.Generator(device=device).manual_seed(P)
+    sh, points = torch.randn(P, 16, 3, generator=g, device=device), torch.randn(P, 3, generator=g, device=device)
+    campos = torch.tensor([0.3, -0.2, 5.0], device=device)
+    Y = _basis(torch.nn.functional.normalize(points.double() - campos.double(), dim=-1))
+    want = (Y[:, :, None] * sh.double()).sum(1) + 0.5
+    bound = 26 * 2.0 ** -24 * ((Y.abs() + 1.0)[:, :, None] * sh.double().abs()).sum(1) + 2.0 ** -23  # as above
+    got = SH_to_RGB(sh.requires_grad_(grad), points.requires_grad_(grad), campos, 3, True)
+    assert ((got.double() - want.clamp_min(0)).abs() <= bound).all()
