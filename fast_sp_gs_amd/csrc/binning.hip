@@ -10,6 +10,8 @@
 //  * standard path: bucket the instances by tile (count -> scan -> scatter) and sort every tile's segment on its own
 //    (see "binning by tile buckets" below); rectangles above 32 tiles are walked cooperatively by the whole wavefront
 //    so one huge surfel cannot serialise a wave.
+//  * small views (tile_gather_kernel, tile_place_kernel): every tile's block finds its own list among all surfels' rectangles, a
+//    word each, and sorts it: two launches instead of five.
 //  * device-wide radix sort (used by the fused corner-test binning of the fast path, whose padding entries and sort width
 //    follow the reference): 8-bit digits. Per pass: block histograms -> per-digit scan over blocks -> scatter. The
 //    scatter ranks keys with 64-bit ballot match masks (8 ballots per round, popcount of the mask below the lane),

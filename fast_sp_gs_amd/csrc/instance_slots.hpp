@@ -10,6 +10,7 @@
 //    afterwards (publish_slot_regions, run by a block of the next kernel), which also hands the instance count to the
 //    host. Which block comes first inside a region varies from run to run, the sums do not: a surfel's records are always
 //    its own, added in tile order.
+// Where the preprocess kernel itself hands the count to the host (ViewOutputs::host_count), a 65th adds up the regions.
 // 64 counters keep the atomics on one address few (5 at 300k surfels, 180 at 3M); they are served one after the other.
 #pragma once
 #include "common.hpp"
