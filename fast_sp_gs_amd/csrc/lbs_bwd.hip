@@ -460,6 +460,14 @@ size_t partial_bytes(int N, int cells, int points = kAccThreads) {
   return p.lds ? align_up((size_t) p.blocks * cells * 4, 256) : 256;
 }
 
+// Room for the partial tables of every warp and weight mode. Whether a table goes by LDS depends on the mode's columns: 2048 control
+// points with S = 2 do not in the widest mode (23 columns, 47 104 cells), which then asks for no room, but do by distances with a rotation
+// (18 columns, exactly the 36 864 cells), and that is 29 MB at 200k points. So: the most cells that LDS holds, unless not even the narrowest row fits.
+size_t lbs_partial_bytes(int N, int M, int S) {
+  const int64_t least = (int64_t) M * lbs_cols(0, 0, S).F, most = (int64_t) M * (21 + S);
+  return least > kTableFloats ? 256 : partial_bytes(N, (int) std::min<int64_t>(most, kTableFloats), kAccPoints);
+}
+
 }  // namespace
 }  // namespace fsgs
 
@@ -468,7 +476,7 @@ using namespace fsgs;
 FSGS_API size_t fsgs_lbs_blend_backward_workspace_bytes(int N, int M, int S) {
   if (N < 0 || M <= 0 || S < 0 || S > 4) return 0;
   const int F = 21 + S;  // the widest row: rotation block, kernel-weight columns, the distances' gradient
-  return align_up((size_t) M * kXf * 4, 256) + align_up((size_t) M * F * 4, 256) + partial_bytes(N, M * F, kAccPoints);
+  return align_up((size_t) M * kXf * 4, 256) + align_up((size_t) M * F * 4, 256) + lbs_partial_bytes(N, M, S);
 }
 
 namespace {
@@ -501,6 +509,8 @@ int lbs_backward(int N, int M, int K, int warp_mode, int weight_mode, double tem
   const float* xf = table ? table : (const float*) workspace;
   float* acc     = (float*) ((char*) workspace + align_up((size_t) M * kXf * 4, 256));
   float* partial = (float*) ((char*) acc + align_up((size_t) M * (21 + S) * 4, 256));
+  if (N > 0 && plan.lds && (size_t) ((char*) (partial + (size_t) plan.blocks * cells) - (char*) workspace) > workspace_bytes)
+    return fail(kWorkspaceSmall, "lbs_blend_backward: no room for %d tables of %d cells", plan.blocks, cells);
   hipStream_t s = (hipStream_t) stream;
   if (!table)
     hipLaunchKernelGGL(lbs_prepare_kernel, dim3(div_up(M, 256)), dim3(256), 0, s, M, warp_mode, sp_points, sp_t, sp_rot, sp_r,

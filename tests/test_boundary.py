@@ -40,6 +40,26 @@ def test_workspace_queries_are_host_only():
     assert L.fsgs_lbs_blend_workspace_bytes(512) >= 512 * 48
 
 
+def test_lbs_backward_workspace_holds_every_modes_tables():
+    """The workspace is sized by N, M and S alone, the tables that pass through LDS (36 864 cells at most) by the columns of the mode:
+    the transforms (28 floats a row), the sums (the widest row), then a table for each block of 512 points, 256 of them at most (of 1024
+    points, where a table is larger than 11 264 cells)."""
+    from fast_sp_gs_amd import lib
+    L = lib.load()
+    up = lambda n: (n + 255) // 256 * 256
+    least = {S: 7 + S for S in range(5)}
+    for S in range(5):
+        edges = {36_864 // F + d for F in range(7 + S, 22 + S) for d in (-1, 0, 1)} | {1, 3, 512, 585, 1024, 1025, 1700, 2048, 10_000}
+        for M in sorted(edges):
+            for N in (1, 513, 20_000, 200_000, 3_000_000):
+                have = L.fsgs_lbs_blend_backward_workspace_bytes(N, M, S)
+                for columns in {least[S] + rotation + kernel + nearest for rotation in (0, 9) for kernel in (0, 2) for nearest in (0, 3)}:
+                    cells = M * columns
+                    points = 512 if cells <= 11_264 and M <= 1024 else 1024
+                    tables = max(1, min(-(-N // points), 256)) if cells <= 36_864 else 0
+                    assert have >= up(28 * 4 * M) + up((21 + S) * 4 * M) + tables * cells * 4, (N, M, S, columns)
+
+
 def test_operator_namespace_semantics():
     from fast_sp_gs_amd import _C
     for name in REFERENCE_NAMES:

@@ -1173,3 +1173,24 @@ def test_lbs_backward_shares(N, M, warp_method, weight_method, device, oracle_mo
     pts, ctrl = torch.rand(N, 3, generator=g) * 2 - 1, torch.rand(M, 3, generator=g) * 2 - 1
     _lbs_backward_case(device, pts, ctrl, 0.1 * torch.randn(M, 3, generator=g), 0.2 * torch.randn(M, 4, generator=g),
                        0.1 * torch.randn(M, 2, generator=g), 4, warp_method, weight_method, seed=N % 97)
+
+
+# tables that pass through LDS although those of the widest mode with as many control points do not (from 1603 of them on, with two scale
+# columns): inside that range, the last of it by columns (2048 with a rotation, 4096 without) and the first behind it
+@pytest.mark.parametrize('M,warp_method', [(1602, 'LBS_c'), (1603, 'LBS_c'), (1700, 'LBS'), (2048, 'LBS_c'), (2049, 'LBS_c'), (4096, None),
+                                           (4097, None)])
+@pytest.mark.parametrize('N', [700, 30_011])
+def test_lbs_backward_large_tables(N, M, warp_method, device, oracle_mod, monkeypatch):
+    from fast_sp_gs_amd._C import _ops
+    guarded = []
+
+    def workspace(size, on):
+        guarded.append((torch.full((size + 2 ** 16,), 0xab, dtype=torch.uint8, device=on), size))
+        return guarded[-1][0][:size]
+
+    monkeypatch.setattr(_ops, '_workspace', workspace)
+    g = torch.Generator().manual_seed(N + M)
+    pts, ctrl = torch.rand(N, 3, generator=g) * 2 - 1, torch.rand(M, 3, generator=g) * 2 - 1
+    _lbs_backward_case(device, pts, ctrl, 0.1 * torch.randn(M, 3, generator=g), 0.2 * torch.randn(M, 4, generator=g),
+                       0.1 * torch.randn(M, 2, generator=g), 4, warp_method, 'dist', seed=M % 97)
+    assert guarded and all(bool((memory[size:] == 0xab).all()) for memory, size in guarded)
