@@ -78,8 +78,11 @@ struct Rgb : public torch::autograd::Function<Rgb> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto t = ctx->get_saved_variables();
-    const Tensor &sh = t[0], &dirs = t[1], &campos = t[2], &rgb = t[3], &derivs = t[4];
     at::AutoDispatchBelowADInplaceOrView no_graph;
+    // handed back strided by a hook: as the Python pair, taken where no gradient in the same layout is asked for
+    auto input = [&](size_t k) { return ctx->needs_input_grad(k) ? Tensor(t[k]) : contiguous(t[k]); };
+    const Tensor sh = input(0), dirs = input(1);
+    const Tensor &campos = t[2], &rgb = t[3], &derivs = t[4];
     const char* what = "SH_to_RGB_backward";
     const Tensor g_rgb = contiguous(g[0]);
     require(what, "sh_features", sh, at::kFloat), require(what, "dir_or_pos", dirs, at::kFloat);
@@ -96,7 +99,7 @@ struct Rgb : public torch::autograd::Function<Rgb> {
                                          f32(dirs), f32(campos), f32(sh), f32(rgb), f32(g_rgb), f32(derivs), f32(g_dirs),
                                          f32(g_campos), f32(g_sh), stream_of(dirs)),
           what);
-    return first_order_only(g, {sh, dirs, campos}, {g_sh, g_dirs, g_campos, Tensor(), Tensor()});
+    return first_order_only(g, {t[0], t[1], campos}, {g_sh, g_dirs, g_campos, Tensor(), Tensor()});
   }
 };
 

@@ -84,3 +84,28 @@ def test_calls_of_the_pair(device):
             x.mul_(2.0)  # what the backward reads has been edited
         with pytest.raises(RuntimeError, match='modified by an inplace operation'):
             out.sum().backward()
+
+
+@pytest.mark.parametrize('strided', [0, 1])
+@pytest.mark.parametrize('wanted', [0, 1])
+@pytest.mark.parametrize('camera', [False, True])
+def test_saved_inputs_handed_back_strided(camera, wanted, strided, device):
+    """A hook may hand the saved coefficients or positions back in another layout (kept by columns, say): the pair takes them so where
+    their own gradient is not asked for, and the node does what the pair does."""
+    from fast_sp_gs_amd import ops
+    sh, pos, cam, _, up = _inputs(300, 16, device, camera)
+    def run(f):
+        inputs = [sh.clone(), pos.clone()]
+        inputs[wanted].requires_grad_(True)
+        at = inputs[strided].data_ptr()
+        back = lambda s: s[0].transpose(0, 1).contiguous().transpose(0, 1) if s[1] else s[0]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (t, t.data_ptr() == at), back):
+            out = f(*inputs, cam, 3, True)
+        return [out, torch.autograd.grad(out, inputs[wanted], up)[0]]
+    if wanted == strided:
+        for f in (ops.SH_to_RGB, ops._rgb_pair):
+            with pytest.raises(RuntimeError, match='must be contiguous'):
+                run(f)
+    else:
+        for x, y in zip(run(ops.SH_to_RGB), run(ops._rgb_pair)):
+            assert torch.equal(x, y)
