@@ -36,6 +36,16 @@ def test_more_instances_than_guessed(which, P, W, H, more, device, monkeypatch):
         views.test_gaussian_view_equals_operators(P, W, H, 'sh', device)
 
 
+# The surfels' and Gaussians' views of the sizes above are gathered tile by tile and need no guess (their lists' workspace is sized
+# by one, too, and made anew). Beyond those limits: grids of more than 127 columns, 1280 and 512 tiles, and more than 200 points a tile
+@pytest.mark.parametrize('P,W,H,more', [(700, 2048, 160, True), (900, 2048, 64, True), (20_001, 160, 160, True), (1, 2048, 64, False)])
+@pytest.mark.parametrize('which', ['surfel', 'gaussian'])
+def test_more_instances_than_guessed_beyond_small_views(which, P, W, H, more, device, monkeypatch):
+    from fast_sp_gs_amd import lib as L
+    assert not L.load().fsgs_gs_view_gathers(P, W, H)
+    test_more_instances_than_guessed(which, P, W, H, more, device, monkeypatch)
+
+
 def _view(s, cam):
     from fast_sp_gs_amd.renderer import GS_2D_render
     with torch.no_grad():
@@ -57,7 +67,8 @@ def _time(f):
     return best
 
 
-@pytest.mark.parametrize('P,W,H,log_scale', [(20_000, 256, 256, -4.6), (900, 480, 288, 0.3), (1, 480, 288, -3.0)])
+@pytest.mark.parametrize('P,W,H,log_scale', [(20_000, 256, 256, -4.6), (900, 480, 288, 0.3), (1, 480, 288, -3.0),
+                                             (60_000, 272, 272, -4.6), (900, 2048, 64, 0.3), (1, 2048, 64, -3.0)])  # the last three: not gathered
 @pytest.mark.parametrize('train', [False, True])
 def test_lists_are_no_longer_than_the_count(P, W, H, log_scale, train, device):
     """Kept, or saved to a file, a list takes the memory of its entries."""
@@ -73,7 +84,7 @@ def test_lists_are_no_longer_than_the_count(P, W, H, log_scale, train, device):
 
 def test_exceeded_guess_costs_an_empty_launch(device):
     """The same 900 large surfels with as many small ones behind the camera as raise the guess above the count: without them the
-    counting, and all behind it, ran twice (1.5 times the time)."""
+    counting, and all behind it, ran twice (1.5 times the time). Both views are gathered tile by tile; for grids that are not, see below."""
     s, cam, g = _large_surfels(900, 480, 288, 901)
     more = type(s)(*(torch.cat([t, t[torch.randint(900, (30_000,), generator=g)]])
                      for t in (s.means3D, s.scales, s.rotations, s.opacities, s.shs)), s.sh_degree)
@@ -82,6 +93,25 @@ def test_exceeded_guess_costs_an_empty_launch(device):
     a, b = _view(s, cam), _view(more, cam)
     assert 65_536 < a['buffer'].R <= 16 * 30_900 and a['buffer'].R == b['buffer'].R and torch.equal(a['images'], b['images'])
     assert _time(lambda: _view(s, cam)) < 1.25 * _time(lambda: _view(more, cam))
+
+
+def test_exceeded_guess_costs_an_empty_launch_beyond_small_views(device):
+    """As above on a grid that is not gathered, with opacities that leave each surfel a small part of its rectangle (which is what is counted):
+    the time is the binning's, not the blend's."""
+    from fast_sp_gs_amd import lib as L
+    s, cam, g = _large_surfels(900, 2048, 64, 901)
+    s.opacities.fill_(0.0045)
+    more = type(s)(*(torch.cat([t, t[torch.randint(900, (30_000,), generator=g)]])
+                     for t in (s.means3D, s.scales, s.rotations, s.opacities, s.shs)), s.sh_degree)
+    more.means3D[900:, 2] = 50.0
+    assert not L.load().fsgs_gs_view_gathers(900, 2048, 64) and not L.load().fsgs_gs_view_gathers(30_900, 2048, 64)
+    s, more, cam = s.to(device), more.to(device), cam.to(device)
+    a, b = _view(s, cam), _view(more, cam)
+    assert 65_536 < a['buffer'].R <= 16 * 30_900 and a['buffer'].R == b['buffer'].R and torch.equal(a['images'], b['images'])
+    turns = [(_time(lambda: _view(s, cam)), _time(lambda: _view(more, cam))) for _ in range(3)]
+    took, with_room = (min(t) for t in zip(*turns))
+    print(f'[exceeded guess] {took:.1f} us, with room {with_room:.1f}', flush=True)
+    assert took < 1.35 * with_room  # 90 and 77: an empty launch, and one that the host's answer to the count is waited for
 
 
 def test_guess_that_memory_does_not_suffice_for(device):
