@@ -20,7 +20,7 @@
 // The grid planes follow the control points (density to the power 1/2, from a sample), so clusters and far outliers keep
 // short lists. 3M queries x 2048 control points, K = 8: 2.43 ms for the search over all pairs, 0.145 ms a call this way
 // (traced: lists 0.039, queries 0.118 to 0.129; 0.063 ms for the 324 MB of inputs and outputs alone). In the query kernel neither unit is
-// full: the vector units are busy 0.62 of the time (1090 instructions per 64 queries), LDS 0.52, 0.22 in bank conflicts. With lists in
+// full: the vector units are busy 0.74 of the time (1130 instructions per 64 queries), LDS 0.60, 0.24 in bank conflicts. With lists in
 // index order and a row of results stored by each lane for itself it took 0.202 ms and 2180 instructions; in order alone 0.169, its
 // memory path busy with stores of 16 bytes each; results through LDS in runs of 512 and 1024 bytes 0.152, and past the caches, which then
 // keep the lists (8 MB), 0.118.

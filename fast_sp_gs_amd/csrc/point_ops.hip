@@ -35,6 +35,8 @@ namespace {
 // 41.6 + 44 (252 MB and 276 MB: 6.1 and 6.3 TB/s); 3M 119 + 239 -> 128 + 148. The forward since a wavefront's rows of 48 floats take
 // the LDS of half of them (to_lanes; five blocks to a compute unit instead of three): 20k 4.8 -> 4.3, 150k 9.5 -> 8.5, 200k 12.9 -> 10.6,
 // 1M 41.8 -> 39.9, 3M 123 -> 120.
+// Rows of degrees 1 and 2 are read again by the backward (1M 12 + 27 and 20 + 45): 36 bytes written and read are more than a row of
+// degree 1 (48), and would save 36 of the 400 bytes a point that a pass of degree 2 moves.
 // Coefficients that are read once in a pass are worth nothing in the memory-side cache (256 MB), but stay there from pass to pass where they
 // fit beside the rest: by ordinary and by streaming loads 400k (77 MB) 40.4 and 41.0, 700k (134 MB) 61.7 and 62.4, 1M (192 MB) 93.3 and
 // 85.6, 3M 287 and 276.
